@@ -49,174 +49,9 @@ namespace {
 
 using namespace anc_reduce;
 
-// bf16 (round to nearest even) by the hardware conversion, as in the 256-tile kernel
-__device__ __forceinline__ uint32_t hw_bf16(float x) { return anc_pk_bf16(x, 0.0f) & 0xFFFFu; }
-
-template <int EPI>
-__global__ void __launch_bounds__(kGemmThreads, 2) k_ns_gemm(NsGemm p) {
-  __shared__ __attribute__((aligned(16))) uint16_t sA[BM * PITCH];
-  // B tile: [n][k] rows of PITCH for the symmetric products; [k][n] rows of NPITCH (320 bytes:
-  // consecutive rows start 64 bytes apart in the banks) for X = a X + B X, which reads the
-  // iterate (K, N) row-major as it lies in memory and transposes while reading fragments.
-  constexpr int NPITCH = BN + 32;
-  constexpr bool BT = (EPI == EPI_BX);
-  __shared__ __attribute__((aligned(16))) uint16_t sB[BT ? BK * NPITCH : BN * PITCH];
-
-  const int L = xcd_remap((int)blockIdx.x, (int)gridDim.x);
-  const int tiles_per = p.lower ? p.tiles_m * (p.tiles_m + 1) / 2 : p.tiles_m * p.tiles_n;
-  const int e = L / tiles_per;
-  const int t = L % tiles_per;
-  int tm, tn;
-  if (p.lower) {
-    tm = 0;
-    while ((tm + 1) * (tm + 2) / 2 <= t) ++tm;
-    tn = t - tm * (tm + 1) / 2;
-  } else {
-    tm = t / p.tiles_n;
-    tn = t % p.tiles_n;
-  }
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int lrow = tid >> 3, lk = (tid & 7) * 8;     // loader: 8 lanes per 128-byte row
-  const int K = p.K;
-  const int nk = K / BK;
-  const int total = anc_ns_terms(p, e) * nk;
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[bi][bj][r] = 0.0f;
-
-  anc_u32x4 ra[4], rb[4];
-  auto gload = [&](int step) {
-    const int term = step / nk, kt = step - term * nk;
-    const uint16_t *Ap = p.A[term] + (int64_t)e * p.strideA + (int64_t)(tm * BM + lrow) * K + kt * BK + lk;
-    // (k, n) tile: 16 lanes per 256-byte row, 16 rows per pass
-    const uint16_t *Bp = BT ? p.B[term] + (int64_t)e * p.strideB + (int64_t)(kt * BK + (tid >> 4)) * p.N + tn * BN + (tid & 15) * 8
-                            : p.B[term] + (int64_t)e * p.strideB + (int64_t)(tn * BN + lrow) * K + kt * BK + lk;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      ra[i] = *(const anc_u32x4 *)(Ap + (int64_t)(32 * i) * K);
-      rb[i] = BT ? *(const anc_u32x4 *)(Bp + (int64_t)(16 * i) * p.N) : *(const anc_u32x4 *)(Bp + (int64_t)(32 * i) * K);
-    }
-  };
-  auto lstore = [&]() {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      *(anc_u32x4 *)&sA[(lrow + 32 * i) * PITCH + lk] = ra[i];
-      if (BT) *(anc_u32x4 *)&sB[((tid >> 4) + 16 * i) * NPITCH + (tid & 15) * 8] = rb[i];
-      else *(anc_u32x4 *)&sB[(lrow + 32 * i) * PITCH + lk] = rb[i];
-    }
-  };
-
-  gload(0);
-  lstore();
-  __syncthreads();
-  const int arow = (wm * 64 + (lane & 31)) * PITCH + (lane >> 5) * 8;
-  const int brow = (wn * 64 + (lane & 31)) * PITCH + (lane >> 5) * 8;
-  // transposing reads: lane s of each 16-lane group addresses row s/4, columns 4*(s%4)..+3
-  const int btr = (8 * (lane >> 5) + ((lane & 15) >> 2)) * NPITCH + wn * 64 + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  for (int step = 0; step < total; ++step) {
-    const bool more = step + 1 < total;
-    if (more) gload(step + 1);
-#pragma unroll
-    for (int kk = 0; kk < BK / 16; ++kk) {
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int bi = 0; bi < 2; ++bi) a[bi] = *(const bf16x8 *)&sA[arow + bi * 32 * PITCH + kk * 16];
-#pragma unroll
-      for (int bj = 0; bj < 2; ++bj)
-        b[bj] = BT ? anc_lds_tr_frag(&sB[btr + kk * 16 * NPITCH + bj * 32], &sB[btr + (kk * 16 + 4) * NPITCH + bj * 32])
-                   : *(const bf16x8 *)&sB[brow + bj * 32 * PITCH + kk * 16];
-#pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < 2; ++bj)
-          acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
-    }
-    __syncthreads();
-    if (more) {
-      lstore();
-      __syncthreads();
-    }
-  }
-
-  // ---- epilogue. Accumulator element r of block (bi,bj) in lane l is
-  //      row 8*(r/4) + 4*(l/32) + r%4, column l%32 of the 32x32 block.
-  const int M = p.M, N = p.N;
-  const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
-  float sc = 1.0f;
-  if (EPI != EPI_BMAT && p.scale != nullptr) sc = p.scale[e];
-  const float acc_scale = (EPI == EPI_GRAM) ? sc * sc : sc;
-  const bool has_a32 = EPI != EPI_BX && anc_ns_has_a32(p, e);
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi) {
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int gi = tm * BM + wm * 64 + bi * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int gj = tn * BN + wn * 64 + bj * 32 + (lane & 31);
-        const float v = (EPI == EPI_BMAT) ? acc[bi][bj][r] : acc[bi][bj][r] * acc_scale;
-        if (EPI == EPI_GRAM) {
-          const bool diag = gi == gj;
-          const uint16_t fh = diag ? (uint16_t)0 : (uint16_t)hw_bf16(v);
-          if (has_a32) p.A32[mm + (int64_t)gi * M + gj] = v;
-          p.Fh[mm + (int64_t)gi * M + gj] = fh;
-          if (tm != tn) {
-            if (has_a32) p.A32[mm + (int64_t)gj * M + gi] = v;
-            p.Fh[mm + (int64_t)gj * M + gi] = fh;
-          }
-          if (p.Fl != nullptr) {
-            const uint16_t fl =
-                diag ? (uint16_t)0 : (uint16_t)hw_bf16(v - anc_bf16_bits_to_f32(fh));
-            p.Fl[mm + (int64_t)gi * M + gj] = fl;
-            if (tm != tn) p.Fl[mm + (int64_t)gj * M + gi] = fl;
-          }
-          if (diag) p.dA[mv + gi] = v;
-        } else if (EPI == EPI_BMAT) {
-          const float a = has_a32 ? p.A32[mm + (int64_t)gi * M + gj]
-                                  : anc_bf16_bits_to_f32(p.Fh[mm + (int64_t)gi * M + gj]);
-          const float di = p.dA[mv + gi], dj = p.dA[mv + gj];
-          uint16_t bh, bl = 0;
-          if (gi != gj) {
-            const float a2 = v + (di * a + a * dj);   // symmetric in (i,j)
-            const float bv = p.cb * a + p.cc * a2;
-            bh = (uint16_t)hw_bf16(bv);
-            bl = (uint16_t)hw_bf16(bv - anc_bf16_bits_to_f32(bh));
-          } else {
-            const float a2 = v + di * di;
-            p.dB[mv + gi] = p.cb * di + p.cc * a2;
-            bh = 0;
-          }
-          p.Bh[mm + (int64_t)gi * M + gj] = bh;
-          if (tm != tn) p.Bh[mm + (int64_t)gj * M + gi] = bh;
-          if (p.Bl != nullptr) {
-            p.Bl[mm + (int64_t)gi * M + gj] = bl;
-            if (tm != tn) p.Bl[mm + (int64_t)gj * M + gi] = bl;
-          }
-        } else {
-          const int64_t o = mn + (int64_t)gi * N + gj;
-          const float x = (anc_bf16_bits_to_f32(p.Xh[o]) + anc_bf16_bits_to_f32(p.Xl[o])) * sc;
-          const float y = (p.ca + p.dB[mv + gi]) * x + v;
-          if (p.X32 != nullptr) p.X32[o] = y;
-          if (p.Yh != nullptr) {
-            const uint32_t yh = hw_bf16(y);
-            p.Yh[o] = (uint16_t)yh;
-            p.Yl[o] = (uint16_t)hw_bf16(y - anc_bf16_bits_to_f32(yh));
-          }
-        }
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------- fp32 validation GEMM
 // 128x128x16 tiles, v_mfma_f32_32x32x2_f32: every product and every sum in fp32.
+constexpr int BM = 128, BN = 128, kGemmThreads = 256;
 constexpr int FK = 16, FPITCH = 20, FNPITCH = 132;
 
 struct NsGemmF32 {
@@ -320,56 +155,64 @@ k_fro_partials(const float *__restrict__ X, int64_t mn, int nchunks, double *__r
 }
 
 // One block per matrix: lane t adds partials t, t+256, ... in order; butterfly; 4 wavefronts in order.
-// pow2 (pair entries only, else null): a matrix whose sum of squares is below 2^-100 (products of
-// its elements would underflow fp32 in the first A = U U^T) gets pow2[e] = 2^k with 2^k ||U|| in
-// [1, 2), every other matrix 1; k_pair_rescale multiplies the pair by it (exact) and the
-// reciprocal carries 2^-k, so the first step sees the same scale*U as without.
-__global__ void __launch_bounds__(kThreads)
-k_fro_finalize(const double *__restrict__ partials, int nchunks, float eps, float *__restrict__ recip,
-               float *__restrict__ pow2) {
+// Lane 0 returns the sum of squares.
+__device__ __forceinline__ double fro_sum(const double *p, int nchunks) {
   __shared__ double wave_sum[kThreads / 64];
-  const double *p = partials + (int64_t)blockIdx.x * nchunks;
   double acc = 0.0;
   for (int i = threadIdx.x; i < nchunks; i += kThreads) acc = acc + p[i];
   acc = anc_wave_sum_f64(acc);
   if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = acc;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = wave_sum[0];
+  double t = wave_sum[0];
 #pragma unroll
-    for (int w = 1; w < kThreads / 64; ++w) t = t + wave_sum[w];
-    float r = 1.0f / ((float)sqrt(t) + eps);
-    if (pow2 != nullptr) {
-      float sc = 1.0f;
-      if (t > 0.0 && t < 0x1p-100) {
-        const int k = -ilogb(sqrt(t));
-        sc = ldexpf(1.0f, k);
-        r = ldexpf(r, -k);
-      }
-      pow2[blockIdx.x] = sc;
-    }
-    recip[blockIdx.x] = r;
-  }
+  for (int w = 1; w < kThreads / 64; ++w) t = t + wave_sum[w];
+  return t;
+}
+__global__ void __launch_bounds__(kThreads)
+k_fro_finalize(const double *__restrict__ partials, int nchunks, float eps, float *__restrict__ recip) {
+  const double t = fro_sum(partials + (int64_t)blockIdx.x * nchunks, nchunks);
+  if (threadIdx.x == 0) recip[blockIdx.x] = 1.0f / ((float)sqrt(t) + eps);
 }
 
-// Multiply the bf16 pair of every matrix whose pow2 is not 1 by it (exact). One workgroup per
-// matrix: it returns at once unless its matrix is one of the rare tiny ones.
-__global__ void __launch_bounds__(kThreads)
-k_pair_rescale(uint16_t *__restrict__ Uh, uint16_t *__restrict__ Ul, const float *__restrict__ pow2, int64_t mn) {
-  const float sc = pow2[blockIdx.x];
-  if (sc == 1.0f) return;
+// The same for the bf16 pairs of up to kMaxGroups batches in one launch. A matrix whose sum of squares is below
+// 2^-100 (products of its elements would underflow fp32 in the first A = U U^T) is multiplied in place by
+// the power of two 2^k that brings ||U|| into [1, 2), exactly, and its reciprocal carries 2^-k, so the
+// first step sees the same scale*U as without. One launch instead of two per batch: 7 batches of a small model
+// took 52 us of launches here.
+struct NsPrologue {
+  int n;
+  int blocks[kMaxGroups];            // matrices per batch
+  int nchunks[kMaxGroups];
+  const double *partials[kMaxGroups];
+  float *recip[kMaxGroups];
+  uint16_t *Uh[kMaxGroups], *Ul[kMaxGroups];
+  int64_t mn[kMaxGroups];
+};
+__global__ void __launch_bounds__(kThreads) k_pair_prologue(NsPrologue a, float eps) {
+  int e = (int)blockIdx.x, q = 0;
+  while (q + 1 < a.n && e >= a.blocks[q]) { e -= a.blocks[q]; ++q; }
+  const double t = fro_sum(a.partials[q] + (int64_t)e * a.nchunks[q], a.nchunks[q]);
+  float r = 1.0f / ((float)sqrt(t) + eps), sc = 1.0f;
+  if (t > 0.0 && t < 0x1p-100) {
+    const int k = -ilogb(sqrt(t));
+    sc = ldexpf(1.0f, k);
+    r = ldexpf(r, -k);
+  }
+  if (threadIdx.x == 0) a.recip[q][e] = r;
+  if (sc == 1.0f) return;            // (uniform over the block)
+  const int64_t mn = a.mn[q];
   for (int64_t o = (int64_t)threadIdx.x * 8; o < mn; o += (int64_t)kThreads * 8) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      uint16_t *p = (h ? Ul : Uh) + (int64_t)blockIdx.x * mn + o;
+      uint16_t *p = (h ? a.Ul[q] : a.Uh[q]) + (int64_t)e * mn + o;
       anc_u32x4 w = *(const anc_u32x4 *)p;
-      uint32_t q[4] = {w.x, w.y, w.z, w.w};
+      uint32_t u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float lo = __uint_as_float(q[i] << 16) * sc, hi = __uint_as_float(q[i] & 0xFFFF0000u) * sc;
-        q[i] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
+        const float lo = __uint_as_float(u[i] << 16) * sc, hi = __uint_as_float(u[i] & 0xFFFF0000u) * sc;
+        u[i] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
       }
-      *(anc_u32x4 *)p = anc_u32x4{q[0], q[1], q[2], q[3]};
+      *(anc_u32x4 *)p = anc_u32x4{u[0], u[1], u[2], u[3]};
     }
   }
 }
@@ -411,8 +254,10 @@ k_ns_prep(float *__restrict__ X, const float *__restrict__ recip, int64_t mn, in
 // in r directions that are spread over the rows (outlier columns). Read from Fh (bf16, zero
 // diagonal). kCondParts blocks per matrix, each over M*M/kCondParts consecutive elements: lane t
 // takes the 8-element vectors t, t+256, ..., adds their squares left to right in fp32, widens to
-// fp64; butterfly over the wavefront; the 4 wavefront sums in order. The consumers add the
-// kCondParts partial sums in order (anc_ns_terms).
+// fp64; butterfly over the wavefront; the 4 wavefront sums in order. k_ns_colstat and k_ns_classify combine the
+// kCondParts partial sums by the same butterfly (one wavefront, a part per lane); classify leaves the sum for
+// the products to read. (64 parts: a single 1024x1024 matrix in 8 parts took 36 us, latency of a
+// few wavefronts.)
 struct NsCondArgs {
   int n;
   int blocks[kMaxGroups];
@@ -472,22 +317,20 @@ struct WideRule {
 // the cheap gates at 1024x3072, 1e-4 .. 2e-4 with every residual term) or has its mass in directions
 // that are not columns at all (near-duplicate rows: ratio 0.5 .. 0.75).
 constexpr double kColcFrac = 0.85, kBulkShare = 3e-3;
-__device__ __forceinline__ double cond_proxy(const double *c, int N) {
-  double s = c[0];
-#pragma unroll
-  for (int i = 1; i < kCondParts; ++i) s = s + c[i];
-  return s * (double)N;
-}
+// sum of a matrix's partial sums, called by whole wavefronts
+__device__ __forceinline__ double cond_sum(const double *parts) { return anc_wave_sum_f64(parts[threadIdx.x & 63]); }
+static_assert(kCondParts == 64, "a partial sum per lane");
 __device__ __host__ __forceinline__ bool wants_colstat(const WideRule &r, double p) {
   return p >= r.hi || (p > r.near_lo && p <= r.lo);
 }
 struct NsColArgs {
   int n;
   int blocks[kMaxGroups];          // colstat: E * parts, classify: E
+  double *sum[kMaxGroups];         // (E) the proxy's sum, classify's output
   const uint16_t *Xh[kMaxGroups];  // (E, M, N) row-major
-  const double *cond[kMaxGroups];
+  const double *cond[kMaxGroups];  // (E, kCondParts)
   double *part[kMaxGroups];        // (E, parts, 2)
-  int32_t *flag[kMaxGroups];       // (E)
+  int32_t *flag[kMaxGroups];       // (E) or null (no wide gate)
   int M[kMaxGroups], N[kMaxGroups], parts[kMaxGroups];
   WideRule rule[kMaxGroups];
 };
@@ -504,7 +347,7 @@ __global__ void __launch_bounds__(kThreads) k_ns_colstat(NsColArgs a) {
   while (q + 1 < a.n && b >= a.blocks[q]) { b -= a.blocks[q]; ++q; }
   const int e = b / a.parts[q], part = b % a.parts[q];
   const int M = a.M[q], N = a.N[q];
-  if (!wants_colstat(a.rule[q], cond_proxy(a.cond[q] + (int64_t)e * kCondParts, N))) return;
+  if (!wants_colstat(a.rule[q], cond_sum(a.cond[q] + (int64_t)e * kCondParts) * (double)N)) return;
   // lane (rg, cg): columns part*64 + 8*cg .. +7 (one 16-byte load per row), rows 4 rg, 4 (rg + 32), ...
   const int cg = (int)threadIdx.x % kColLanes, rg = (int)threadIdx.x / kColLanes;
   const int j = part * kColBlock + 8 * cg;
@@ -545,12 +388,14 @@ __global__ void __launch_bounds__(kThreads) k_ns_colstat(NsColArgs a) {
 }
 static_assert(kColBlock % 64 == 0 && kColBlock <= kThreads, "k_ns_colstat: whole wavefronts of one lane per column in the final sum");
 __global__ void __launch_bounds__(kThreads) k_ns_classify(NsColArgs a) {
-  int t = (int)(blockIdx.x * kThreads + threadIdx.x), q = 0;
+  int t = (int)(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6)), q = 0;      // one wavefront per matrix
   while (q + 1 < a.n && t >= a.blocks[q]) { t -= a.blocks[q]; ++q; }
   if (t >= a.blocks[q]) return;
   const int e = t, N = a.N[q];
   const WideRule r = a.rule[q];
-  const double p = cond_proxy(a.cond[q] + (int64_t)e * kCondParts, N);
+  const double sum = cond_sum(a.cond[q] + (int64_t)e * kCondParts), p = sum * (double)N;
+  if ((threadIdx.x & 63) == 0) a.sum[q][e] = sum;
+  if (a.flag[q] == nullptr || (threadIdx.x & 63) != 0) return;
   bool wide = p > r.lo && p < r.hi;
   if (!wide && wants_colstat(r, p)) {
     const double *c = a.part[q] + (int64_t)e * a.parts[q] * 2;
@@ -770,8 +615,8 @@ struct Plan {
   uint16_t *Fl, *Bl;
   double *partials;
   float *recip;
-  float *pow2;           // (E) power-of-two pre-scale of tiny inputs, pair entries
-  double *cond;          // (E, kCondParts) conditioning proxy, bf16 modes
+  double *condpart;      // (E, kCondParts) partial sums of the conditioning proxy, bf16 modes
+  double *cond;          // (E) the proxy
   double *colpart;       // (E, col_parts, 2) column statistic, plans with a wide gate
   int32_t *wide_flag;    // (E) the wide gate's decision
   int col_parts;
@@ -792,7 +637,6 @@ Plan make_plan(uint64_t base, int64_t E, int64_t M, int64_t N, int mode, int ste
   pl.split = pl.sp.x_from < steps;
   pl.partials = c.take<double>(E * pl.nchunks);
   pl.recip = c.take<float>(E);
-  pl.pow2 = c.take<float>(E);
   if (mode == ANC_NS_FP32) {
     pl.Af = c.take<float>(E * M * M);
     pl.Bf = c.take<float>(E * M * M);
@@ -811,7 +655,8 @@ Plan make_plan(uint64_t base, int64_t E, int64_t M, int64_t N, int mode, int ste
     }
     pl.dA = c.take<float>(E * M);
     pl.dB = c.take<float>(E * M);
-    pl.cond = c.take<double>(E * kCondParts);
+    pl.condpart = c.take<double>(E * kCondParts);
+    pl.cond = c.take<double>(E);
     if (pl.sp.wide()) {
       pl.col_parts = (int)((N + kColBlock - 1) / kColBlock);
       pl.colpart = c.take<double>(E * pl.col_parts * 2);
@@ -821,6 +666,8 @@ Plan make_plan(uint64_t base, int64_t E, int64_t M, int64_t N, int mode, int ste
   pl.bytes = c.off;
   return pl;
 }
+
+constexpr int kTileFlags = ANC_NS_TILE128 | ANC_NS_FORCE_T64 | ANC_NS_FORCE_T128 | ANC_NS_FORCE_T256;
 
 int check_shape(int64_t E, int64_t M, int64_t N, int mode, const char *who) {
   ANC_REQUIRE(E > 0 && M > 0 && N > 0, "%s: E, M, N must be positive", who);
@@ -836,6 +683,27 @@ int check_shape(int64_t E, int64_t M, int64_t N, int mode, const char *who) {
   return ANC_OK;
 }
 
+void add_prologue(NsPrologue &a, const Plan &pl, uint64_t Uh, uint64_t Ul, uint64_t fro, int64_t n_partials, int64_t E,
+                  int64_t mn) {
+  const int q = a.n++;
+  a.blocks[q] = (int)E;
+  a.nchunks[q] = (int)n_partials;
+  a.partials[q] = (const double *)fro;
+  a.recip[q] = pl.recip;
+  a.Uh[q] = (uint16_t *)Uh;
+  a.Ul[q] = (uint16_t *)Ul;
+  a.mn[q] = mn;
+}
+int launch_prologue(const NsPrologue &a, float eps, hipStream_t s) {
+  int64_t blocks = 0;
+  for (int q = 0; q < a.n; ++q) blocks += a.blocks[q];
+  ANC_REQUIRE(blocks < (1ll << 31), "Newton-Schulz chain: too many matrices");
+  AncProfScope prof(ANC_PROF_NS_FRO, s);
+  hipLaunchKernelGGL(k_pair_prologue, dim3((unsigned)blocks), dim3(kThreads), 0, s, a, eps);
+  ANC_LAUNCH_CHECK();
+  return ANC_OK;
+}
+
 // One problem of a chain launch: a batch of E (M,N) matrices with its workspace plan.
 struct ChainProb {
   Plan pl;
@@ -847,16 +715,40 @@ struct ChainProb {
   const anc_muon_desc_t *upd;  // or: the weights (E entries) the last step updates in its epilogue
 };
 
+// Tiles of a launch, from the tiles each size would give it, weighted by their K against the longest
+// (a launch ends with its longest tiles; short ones fill gaps). A CU takes operand bytes into LDS at one
+// rate whatever the tile, so small tiles finish first while they find idle CUs and lose, by the bytes they
+// fetch more often, once every CU has several. Measured, us per 5 launches on 64 / 128 / 256-wide tiles:
+//   A = X X^T   8 x (512,512) 87 / 120 / 196 (384 tiles of 64), 4 x (1024,1024) 134 / 131 / 195 (640),
+//               8 x (1024,1024) 196 / 182 / 202 (320 of 128), 16 x (1024,1024) 335 / 306 / 237 (640)
+//   X = a X + B X   1 x (1024,3072) 107 / 110 / 142 (768 of 64), 4 x (512,1536) 118 / 120 / 157 (768),
+//               8 x (512,1536) 192 / 164 / 162 (384 of 128), 8 x (1024,2048) 385 / 280 / 247 (1024)
+// hence 64 below 600 (symmetric) or 768 tiles of 64, 128 below 400 tiles of 128.
+int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
+  double longest = 0.0, t64 = 0.0;
+  for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
+  for (int k = 0; k < n; ++k) {
+    const double m = (double)(ps[k].M / 64), d = (double)(ps[k].diag / 64);
+    const double per = epi == EPI_BX ? m * (double)(ps[k].N / 64) : m * (m + d) / 2.0;
+    t64 += (double)Es[k] * per * ((double)ps[k].K / longest);
+  }
+  if (t64 < (epi == EPI_BX ? 768.0 : 600.0)) return 64;
+  return t64 < 1600.0 ? 128 : 256;
+}
+
+// What a mode's tile flags ask for (0: nothing).
+int forced_tile(int flags) {
+  return (flags & ANC_NS_FORCE_T64) ? 64 : (flags & (ANC_NS_FORCE_T128 | ANC_NS_TILE128)) ? 128
+         : (flags & ANC_NS_FORCE_T256) ? 256 : 0;
+}
+
 // steps x { A = X X^T; B = b A + c A A; X = a X + B X } on n problems side by side: every
 // product of a step is ONE launch over all problems (problems in the order given; put the
 // longest K first). First step's output goes to pair `nxt` of each plan, later steps ping-pong;
-// the last step writes the fp32 results. With n == 1 and a shape that is not a multiple of 256
-// (or force_small) the 128x128-tile kernel runs instead.
-int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool force_small, hipStream_t s,
+// the last step writes the fp32 results. `flags`: the tile flags of the mode.
+int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags, hipStream_t s,
                    const NsUpdate *upd = nullptr) {
-  bool big = !force_small;
-  for (int q = 0; q < n; ++q) big = big && (cp[q].M % 256 == 0) && (cp[q].N % 256 == 0);
-  ANC_REQUIRE(big || n == 1, "Newton-Schulz chain: several problems per launch need dims that are multiples of 256");
+  const int force = forced_tile(flags);
   const uint16_t *curH[kMaxGroups], *curL[kMaxGroups];
   int nxt[kMaxGroups];
   int64_t Es[kMaxGroups];
@@ -873,10 +765,12 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool forc
       const int64_t M = cp[q].M, N = cp[q].N, mn = M * N;
       const bool split = k >= pl.sp.x_from;        // X residual terms
       const bool split_fb = k >= pl.sp.fb_from;    // F and Boff residual terms
-      const int tile = big ? 256 : BM;
-      const int tM = (int)(M / tile), tN = (int)(N / tile);
+      // a property of the shape, whatever the tiles: blocks on the diagonal of a symmetric product that are
+      // computed in full, and whether low halves of the iterate may be 8 bits
+      const bool wide256 = !(flags & ANC_NS_TILE128) && M % 256 == 0 && N % 256 == 0;
       NsGemm g{};
       g.M = (int)M; g.N = (int)N;
+      g.diag = wide256 ? 256 : 128;
       g.A32 = pl.A32; g.Fh = pl.Fh; g.dA = pl.dA; g.Bh = pl.Bh; g.dB = pl.dB;
       if (pl.sp.drop_a32) {
         // the first iteration runs before the classification: nobody is flagged yet
@@ -887,11 +781,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool forc
       g.Bl = split_fb ? pl.Bl : nullptr;
       g.ca = coef[3 * k]; g.cb = coef[3 * k + 1]; g.cc = coef[3 * k + 2];
       g.scale = (k == 0) ? cp[q].scale0 : nullptr;
-      // 256-tile kernels: everything the chain itself writes (F, B, every iterate after the input)
-      // is in panel layout; the input pair is row-major as the caller left it
-      g.f_panel = big ? 1 : 0;
-      g.x_panel = (big && k > 0) ? 1 : 0;
-      g.y_panel = big ? 1 : 0;
+      g.x_panel = k > 0 ? 1 : 0;                   // the input pair is row-major as the caller left it
       // the wide gate of this iteration (a band of the proxy; the proxy is N * sum, hence the / N)
       const bool wide_g = pl.sp.wide_gram(k);      // implies !split
       const bool wide_a = pl.sp.wide_all(k);       // implies !split_fb
@@ -919,7 +809,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool forc
         ga[q].Fl = pl.Fl;
         ga[q].lo_gated = 1;
       }
-      ga[q].K = (int)N; ga[q].strideA = mn; ga[q].strideB = mn; ga[q].tiles_m = tM; ga[q].tiles_n = tM; ga[q].lower = 1;
+      ga[q].K = (int)N; ga[q].strideA = mn; ga[q].strideB = mn;
       // B = b A + c A A
       gb[q] = g;
       gb[q].A[0] = pl.Fh; gb[q].B[0] = pl.Fh; gb[q].nterms = 1;
@@ -933,7 +823,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool forc
         gb[q].Bl = pl.Bl;
         gb[q].lo_gated = 1;
       }
-      gb[q].K = (int)M; gb[q].strideA = M * M; gb[q].strideB = M * M; gb[q].tiles_m = tM; gb[q].tiles_n = tM; gb[q].lower = 1;
+      gb[q].K = (int)M; gb[q].strideA = M * M; gb[q].strideB = M * M;
       // X = a X + B X
       gx[q] = g;
       gx[q].A[0] = pl.Bh; gx[q].B[0] = curH[q]; gx[q].nterms = 1;
@@ -950,7 +840,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool forc
         gx[q].A[2] = pl.Bl; gx[q].B[2] = curH[q];
         set_wide(gx[q], 3);
       }
-      gx[q].K = (int)M; gx[q].strideA = M * M; gx[q].strideB = mn; gx[q].tiles_m = tM; gx[q].tiles_n = tN; gx[q].lower = 0;
+      gx[q].K = (int)M; gx[q].strideA = M * M; gx[q].strideB = mn;
       gx[q].Xh = curH[q]; gx[q].Xl = curL[q];
       gx[q].Yh = last ? nullptr : pl.Xh[nxt[q]];
       gx[q].Yl = last ? nullptr : pl.Xl[nxt[q]];
@@ -960,7 +850,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool forc
       // next iteration multiplies: every matrix outside the wide gate if that iteration has no gate,
       // those below its gate if it has one, none if its plan splits X for everybody.
       double l8_next = 0.0;
-      if (big && pl.sp.low8 && !last && pl.sp.any_gate(steps) && k + 1 < pl.sp.x_from)
+      if (wide256 && pl.sp.low8 && !last && pl.sp.any_gate(steps) && k + 1 < pl.sp.x_from)
         l8_next = pl.sp.gated(k + 1) ? (double)pl.sp.gate_tau[k + 1] / (double)N : 1e300;
       gx[q].l8_cond = pl.cond;
       gx[q].l8_wide = pl.sp.wide() ? pl.wide_flag : nullptr;
@@ -968,21 +858,17 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool forc
       gx[q].l8_out = l8_next;
       l8_cur[q] = l8_next;
     }
-    const int tM0 = (int)(cp[0].M / BM), tN0 = (int)(cp[0].N / BN);
-    const unsigned g_sym = (unsigned)(cp[0].E * tM0 * (tM0 + 1) / 2), g_mn = (unsigned)(cp[0].E * tM0 * tN0);
     {
       AncProfScope prof(ANC_PROF_NS_GRAM, s);
-      if (big) { if (int rc = anc_ns_gemm_big_multi(EPI_GRAM, ga, Es, n, s)) return rc; }
-      else hipLaunchKernelGGL(k_ns_gemm<EPI_GRAM>, dim3(g_sym), dim3(kGemmThreads), 0, s, ga[0]);
+      if (int rc = anc_ns_gemm_multi(EPI_GRAM, ga, Es, n, force, s)) return rc;
     }
-    ANC_LAUNCH_CHECK();
     if (k == 0 && want_cond) {
       // the proxy of every problem that gates a later product, from the Fh this launch wrote
       NsCondArgs ca{};
       int blocks = 0;
       for (int q = 0; q < n; ++q) {
         if (!cp[q].pl.sp.any_gate(steps)) continue;
-        ca.Fh[ca.n] = cp[q].pl.Fh; ca.out[ca.n] = cp[q].pl.cond; ca.M[ca.n] = (int)cp[q].M;
+        ca.Fh[ca.n] = cp[q].pl.Fh; ca.out[ca.n] = cp[q].pl.condpart; ca.M[ca.n] = (int)cp[q].M;
         ca.blocks[ca.n] = (int)(cp[q].E * kCondParts);
         blocks += ca.blocks[ca.n];
         ++ca.n;
@@ -992,40 +878,37 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool forc
       ANC_LAUNCH_CHECK();
       // the wide gate's decision per matrix, from the proxy and, where it asks, the column norms
       NsColArgs cs{}, cf{};
-      int cs_blocks = 0, cf_lanes = 0;
+      int cs_blocks = 0, cf_mats = 0;
       for (int q = 0; q < n; ++q) {
         const Plan &pl = cp[q].pl;
-        if (!pl.sp.wide()) continue;
+        if (!pl.sp.any_gate(steps)) continue;
         const int i = cs.n;
-        cs.Xh[i] = cp[q].inH; cs.cond[i] = pl.cond; cs.part[i] = pl.colpart; cs.flag[i] = pl.wide_flag;
+        cs.Xh[i] = cp[q].inH; cs.cond[i] = pl.condpart; cs.sum[i] = pl.cond; cs.part[i] = pl.colpart; cs.flag[i] = pl.wide_flag;
         cs.M[i] = (int)cp[q].M; cs.N[i] = (int)cp[q].N; cs.parts[i] = pl.col_parts;
         cs.rule[i] = WideRule{(double)pl.sp.wide_near, (double)pl.sp.wide_lo, (double)pl.sp.wide_hi,
                               (double)pl.sp.wide_near_diff};
-        cs.blocks[i] = (int)(cp[q].E * pl.col_parts);
+        cs.blocks[i] = (int)(cp[q].E * pl.col_parts);    // 0 without a wide gate
         cs_blocks += cs.blocks[i];
         ++cs.n;
       }
-      if (cs.n > 0) {
-        cf = cs;
-        for (int i = 0; i < cf.n; ++i) { cf.blocks[i] = cs.blocks[i] / cs.parts[i]; cf_lanes += cf.blocks[i]; }
+      cf = cs;
+      for (int i = 0, q = 0; q < n; ++q)
+        if (cp[q].pl.sp.any_gate(steps)) { cf.blocks[i] = (int)cp[q].E; cf_mats += cf.blocks[i]; ++i; }
+      if (cs_blocks > 0) {
         hipLaunchKernelGGL(k_ns_colstat, dim3((unsigned)cs_blocks), dim3(kThreads), 0, s, cs);
         ANC_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_ns_classify, dim3((unsigned)((cf_lanes + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, cf);
-        ANC_LAUNCH_CHECK();
       }
+      hipLaunchKernelGGL(k_ns_classify, dim3((unsigned)((cf_mats + kThreads / 64 - 1) / (kThreads / 64))), dim3(kThreads), 0, s, cf);
+      ANC_LAUNCH_CHECK();
     }
     {
       AncProfScope prof(ANC_PROF_NS_BMAT, s);
-      if (big) { if (int rc = anc_ns_gemm_big_multi(EPI_BMAT, gb, Es, n, s)) return rc; }
-      else hipLaunchKernelGGL(k_ns_gemm<EPI_BMAT>, dim3(g_sym), dim3(kGemmThreads), 0, s, gb[0]);
+      if (int rc = anc_ns_gemm_multi(EPI_BMAT, gb, Es, n, force, s)) return rc;
     }
-    ANC_LAUNCH_CHECK();
     {
       AncProfScope prof(last && upd != nullptr ? ANC_PROF_NS_BX_UPD : ANC_PROF_NS_BX, s);
-      if (big) { if (int rc = anc_ns_gemm_big_multi(EPI_BX, gx, Es, n, s, last ? upd : nullptr)) return rc; }
-      else hipLaunchKernelGGL(k_ns_gemm<EPI_BX>, dim3(g_mn), dim3(kGemmThreads), 0, s, gx[0]);
+      if (int rc = anc_ns_gemm_multi(EPI_BX, gx, Es, n, force, s, last ? upd : nullptr)) return rc;
     }
-    ANC_LAUNCH_CHECK();
     for (int q = 0; q < n; ++q) {
       curH[q] = cp[q].pl.Xh[nxt[q]]; curL[q] = cp[q].pl.Xl[nxt[q]];
       nxt[q] ^= 1;
@@ -1036,8 +919,56 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, bool forc
 
 }  // namespace
 
+int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int force, hipStream_t s,
+                      const NsUpdate *upd) {
+  ANC_REQUIRE(n >= 1 && n <= kMaxGroups, "Newton-Schulz chain: 1..%d problems per launch", kMaxGroups);
+  bool any_upd = false, all_upd = true;
+  for (int k = 0; k < n; ++k) { any_upd = any_upd || ps[k].upd != nullptr; all_upd = all_upd && ps[k].upd != nullptr; }
+  ANC_REQUIRE(any_upd == all_upd && (!any_upd || upd != nullptr),
+              "Newton-Schulz chain: the fused update applies to every problem of a launch or to none");
+  // B is symmetric and stored in full, so X = a X + B X can fetch its tile by rows k (256-byte rows) as
+  // well as by rows m (64-byte row pieces). Measured per 5 launches: 84 x (1024, 3072) 4.12
+  // against 4.27 ms, 208 x (1024, 1024) 3.37 against 3.56 ms, but 64 x (512, 512) 0.238 against
+  // 0.212 ms: by rows k from M = 1024 on. The two ways read the same values except inside the
+  // diagonal blocks of a B that descends from an A = X X^T with residual terms: there
+  // element (i, j) and element (j, i) add the same products in a different order and may differ
+  // in the last bit. So the way of reading is a property of the problem's shape, never of what
+  // it shares a call with: a call with problems of both kinds becomes two launches.
+  // Where 256-wide tiles are the choice, problems whose dims do not allow them get a launch of their own.
+  NsGemm part[kMaxGroups];
+  int64_t pe[kMaxGroups];
+  bool done[2] = {false, false};
+  for (int pass = 0; pass < 4; ++pass) {
+    const bool by_rows = epi == EPI_BX && (pass & 1) == 0, wide = pass < 2;
+    auto collect = [&](bool all) {
+      int m = 0;
+      for (int k = 0; k < n; ++k) {
+        if (epi == EPI_BX ? (ps[k].M >= 1024) != by_rows : (pass & 1) != 0) continue;
+        if (!all && (ps[k].diag == 256) != wide) continue;
+        part[m] = ps[k];
+        pe[m++] = Es[k];
+      }
+      return m;
+    };
+    const auto pick = [&](int m) { return force ? force : pick_tile(epi, part, pe, m); };
+    const NsUpdate *u = any_upd ? upd : nullptr;
+    const int m_wide = collect(false);
+    if (wide) {
+      if (m_wide > 0 && pick(m_wide) == 256) {
+        if (int rc = anc_ns_gemm_big_multi(epi, part, pe, m_wide, s, by_rows, u)) return rc;
+      } else if (const int m = collect(true)) {
+        if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m, s, pick(m) == 64, by_rows, u, false)) return rc;
+        done[pass & 1] = true;
+      }
+    } else if (m_wide > 0 && !done[pass & 1]) {
+      if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m_wide, s, pick(m_wide) == 64, by_rows, u, false)) return rc;
+    }
+  }
+  return ANC_OK;
+}
+
 extern "C" int64_t anc_ns_workspace_bytes(int64_t E, int64_t M, int64_t N, int mode) {
-  mode &= ~ANC_NS_TILE128;
+  mode &= ~kTileFlags;
   if (check_shape(E, M, N, mode, "anc_ns_workspace_bytes")) return -1;
   // sized for any step count: with steps >= 3 every optional buffer of the mode's plan is present
   // (the longer of a long and a 5-step chain's plans, should the two ever differ)
@@ -1061,15 +992,15 @@ static double sym_tile_flops(int64_t M, int64_t N, bool force_small) {
 // `dense` is the textbook steps*(4 M^2 N + 2 M^3) per matrix.
 extern "C" int anc_ns_flops(int64_t E, int64_t M, int64_t N, int steps, int mode,
                             double *executed, double *dense) {
-  const bool force_small = (mode & ANC_NS_TILE128) != 0;
-  mode &= ~ANC_NS_TILE128;
+  const int flags = mode & kTileFlags;
+  mode &= ~kTileFlags;
   if (int rc = check_shape(E, M, N, mode, "anc_ns_flops")) return rc;
   ANC_REQUIRE(executed != nullptr && dense != nullptr && steps >= 0, "anc_ns_flops: bad arguments");
   const double m = (double)M, n = (double)N, e = (double)E;
   *dense = e * steps * (4.0 * m * m * n + 2.0 * m * m * m);
   if (mode == ANC_NS_FP32) { *executed = *dense; return ANC_OK; }
   const SplitPlan sp = split_plan(M, N, mode, steps);
-  const double sym = sym_tile_flops(M, N, force_small);
+  const double sym = sym_tile_flops(M, N, (flags & ANC_NS_TILE128) != 0);
   double ex = 0.0;
   for (int k = 0; k < steps; ++k) {
     const bool sx = k >= sp.x_from, sfb = k >= sp.fb_from;
@@ -1083,8 +1014,8 @@ extern "C" int anc_ns_flops(int64_t E, int64_t M, int64_t N, int steps, int mode
 
 extern "C" int anc_ns_product_flops(int64_t E, int64_t M, int64_t N, int steps, int mode, int k, int product,
                                     double *executed) {
-  const bool force_small = (mode & ANC_NS_TILE128) != 0;
-  mode &= ~ANC_NS_TILE128;
+  const int flags = mode & kTileFlags;
+  mode &= ~kTileFlags;
   if (int rc = check_shape(E, M, N, mode, "anc_ns_product_flops")) return rc;
   ANC_REQUIRE(executed != nullptr && steps > 0 && k >= 0 && k < steps && product >= 0 && product <= 2,
               "anc_ns_product_flops: bad arguments");
@@ -1095,7 +1026,7 @@ extern "C" int anc_ns_product_flops(int64_t E, int64_t M, int64_t N, int steps, 
   }
   const SplitPlan sp = split_plan(M, N, mode, steps);
   const bool sx = k >= sp.x_from, sfb = k >= sp.fb_from;
-  const double sym = sym_tile_flops(M, N, force_small);
+  const double sym = sym_tile_flops(M, N, (flags & ANC_NS_TILE128) != 0);
   double ex;
   if (product == 0)      ex = sym * (sx ? 3 : 1) * n;
   else if (product == 1) ex = sym * (sfb ? 3 : 1) * m;
@@ -1109,8 +1040,8 @@ extern "C" int anc_ns_product_flops(int64_t E, int64_t M, int64_t N, int steps, 
 // Synchronises `stream`, then reads the proxy's partial sums back and takes the kernels' decisions.
 extern "C" int anc_ns_hard_info(uint64_t workspace, int64_t E, int64_t M, int64_t N, int mode, int steps,
                                 int32_t *n_gated, double *extra_flops, uint64_t stream) {
-  const bool force_small = (mode & ANC_NS_TILE128) != 0;
-  mode &= ~ANC_NS_TILE128;
+  const int flags = mode & kTileFlags;
+  mode &= ~kTileFlags;
   if (int rc = check_shape(E, M, N, mode, "anc_ns_hard_info")) return rc;
   ANC_REQUIRE(n_gated != nullptr && extra_flops != nullptr && workspace != 0 && steps >= 0,
               "anc_ns_hard_info: bad arguments");
@@ -1119,25 +1050,24 @@ extern "C" int anc_ns_hard_info(uint64_t workspace, int64_t E, int64_t M, int64_
   if (mode == ANC_NS_FP32) return ANC_OK;
   const Plan pl = make_plan(workspace, E, M, N, mode, steps);
   if (!pl.sp.any_gate(steps)) return ANC_OK;
-  std::vector<double> host((size_t)(E * kCondParts));
+  std::vector<double> host((size_t)E);
   ANC_HIP(hipStreamSynchronize(anc_stream(stream)));
   ANC_HIP(hipMemcpy(host.data(), pl.cond, host.size() * sizeof(double), hipMemcpyDeviceToHost));
-  std::vector<int32_t> flags((size_t)E, 0);
+  std::vector<int32_t> wide((size_t)E, 0);
   if (pl.sp.wide())
-    ANC_HIP(hipMemcpy(flags.data(), pl.wide_flag, flags.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
-  const double gram_extra = 2.0 * sym_tile_flops(M, N, force_small) * (double)N;     // two more terms
+    ANC_HIP(hipMemcpy(wide.data(), pl.wide_flag, wide.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+  const double gram_extra = 2.0 * sym_tile_flops(M, N, (flags & ANC_NS_TILE128) != 0) * (double)N;     // two more terms
   const double bx_extra = 2.0 * (double)M * (double)M * (double)N;                   // one more term
   for (int64_t e = 0; e < E; ++e) {
-    double t = host[(size_t)(e * kCondParts)];
-    for (int i = 1; i < kCondParts; ++i) t = t + host[(size_t)(e * kCondParts + i)];
+    const double t = host[(size_t)e];
     bool any = false;
-    const bool in_band = flags[(size_t)e] != 0;
+    const bool in_band = wide[(size_t)e] != 0;
     for (int k = 0; k < steps; ++k) {
       if (in_band) {                    // the wide gate takes precedence over the others
         const bool sx = k >= pl.sp.x_from;
         if (pl.sp.wide_gram(k)) { *extra_flops += gram_extra; any = true; }
         if (pl.sp.wide_all(k)) {
-          *extra_flops += 2.0 * sym_tile_flops(M, N, force_small) * (double)M + (sx ? 1.0 : 2.0) * bx_extra;
+          *extra_flops += 2.0 * sym_tile_flops(M, N, (flags & ANC_NS_TILE128) != 0) * (double)M + (sx ? 1.0 : 2.0) * bx_extra;
           any = true;
         }
         continue;
@@ -1154,8 +1084,8 @@ extern "C" int anc_ns_hard_info(uint64_t workspace, int64_t E, int64_t M, int64_
 extern "C" int anc_ns_batched(uint64_t X, int64_t E, int64_t M, int64_t N, int steps,
                               const float *coef, float eps, int mode, uint64_t workspace,
                               int64_t workspace_bytes, uint64_t stream) {
-  const bool force_small = (mode & ANC_NS_TILE128) != 0;
-  mode &= ~ANC_NS_TILE128;
+  const int flags = mode & kTileFlags;
+  mode &= ~kTileFlags;
   if (int rc = check_shape(E, M, N, mode, "anc_ns_batched")) return rc;
   ANC_REQUIRE(X != 0 && (X & 15) == 0, "anc_ns_batched: X must be a 16-byte aligned device pointer");
   ANC_REQUIRE(steps >= 0 && steps <= 64 && (steps == 0 || coef != nullptr),
@@ -1173,7 +1103,7 @@ extern "C" int anc_ns_batched(uint64_t X, int64_t E, int64_t M, int64_t N, int s
                      pl.nchunks, pl.partials); }
   ANC_LAUNCH_CHECK();
   { AncProfScope prof(ANC_PROF_NS_FRO, s); hipLaunchKernelGGL(k_fro_finalize, dim3((unsigned)E), dim3(kThreads), 0, s, pl.partials, pl.nchunks,
-                     eps, pl.recip, (float *)nullptr); }
+                     eps, pl.recip); }
   ANC_LAUNCH_CHECK();
   const int64_t total8 = E * mn / 8;
   const unsigned prep_grid = (unsigned)((total8 + kThreads - 1) / kThreads);
@@ -1219,7 +1149,7 @@ extern "C" int anc_ns_batched(uint64_t X, int64_t E, int64_t M, int64_t N, int s
                      pl.Xh[0], pl.Xl[0]); }
   ANC_LAUNCH_CHECK();
   ChainProb cp{pl, pl.Xh[0], pl.Xl[0], 1, nullptr, X32, E, M, N, nullptr};
-  return run_bf16_chain(&cp, 1, steps, coef, force_small, s);
+  return run_bf16_chain(&cp, 1, steps, coef, flags, s);
 }
 
 // The chain on an unnormalised bf16 pair (what anc_muon_momentum_multi_pair leaves) with the
@@ -1229,8 +1159,8 @@ extern "C" int anc_ns_batched_pair(uint64_t Uh, uint64_t Ul, uint64_t fro_partia
                                    uint64_t X32_out, int64_t E, int64_t M, int64_t N, int steps,
                                    const float *coef, float eps, int mode, uint64_t workspace,
                                    int64_t workspace_bytes, uint64_t stream) {
-  const bool force_small = (mode & ANC_NS_TILE128) != 0;
-  mode &= ~ANC_NS_TILE128;
+  const int flags = mode & kTileFlags;
+  mode &= ~kTileFlags;
   if (int rc = check_shape(E, M, N, mode, "anc_ns_batched_pair")) return rc;
   ANC_REQUIRE(mode != ANC_NS_FP32, "anc_ns_batched_pair: the fp32 chain takes fp32 input (anc_ns_batched)");
   ANC_REQUIRE(Uh != 0 && Ul != 0 && ((Uh | Ul) & 15) == 0 && X32_out != 0 && (X32_out & 15) == 0,
@@ -1244,14 +1174,11 @@ extern "C" int anc_ns_batched_pair(uint64_t Uh, uint64_t Ul, uint64_t fro_partia
   ANC_REQUIRE(workspace_bytes >= pl.bytes, "anc_ns_batched_pair: workspace holds %lld bytes, %lld needed",
               (long long)workspace_bytes, (long long)pl.bytes);
   hipStream_t s = anc_stream(stream);
-  { AncProfScope prof(ANC_PROF_NS_FRO, s); hipLaunchKernelGGL(k_fro_finalize, dim3((unsigned)E), dim3(kThreads), 0, s,
-                     (const double *)fro_partials, (int)n_partials, eps, pl.recip, pl.pow2); }
-  ANC_LAUNCH_CHECK();
-  { AncProfScope prof(ANC_PROF_NS_FRO, s); hipLaunchKernelGGL(k_pair_rescale, dim3((unsigned)E), dim3(kThreads), 0, s,
-                     (uint16_t *)Uh, (uint16_t *)Ul, pl.pow2, M * N); }
-  ANC_LAUNCH_CHECK();
+  NsPrologue pro{};
+  add_prologue(pro, pl, Uh, Ul, fro_partials, n_partials, E, M * N);
+  if (int rc = launch_prologue(pro, eps, s)) return rc;
   ChainProb cp{pl, (const uint16_t *)Uh, (const uint16_t *)Ul, 0, pl.recip, (float *)X32_out, E, M, N, nullptr};
-  return run_bf16_chain(&cp, 1, steps, coef, force_small, s);
+  return run_bf16_chain(&cp, 1, steps, coef, flags, s);
 }
 
 // n_probs <= 8 independent batches (the shape groups of one optimizer step) through the chain
@@ -1262,16 +1189,16 @@ static int pair_multi_impl(const char *who, const anc_ns_problem_t *probs, int32
                            const uint64_t *desc_tables, const NsUpdate *upd, int steps, const float *coef,
                            float eps, int mode, uint64_t stream) {
   ANC_REQUIRE(probs != nullptr && n_probs >= 1 && n_probs <= kMaxGroups, "%s: 1..%d problems", who, kMaxGroups);
-  ANC_REQUIRE(mode == ANC_NS_BF16 || mode == ANC_NS_BF16_FAST || mode == ANC_NS_BF16_X3 || mode == ANC_NS_BF16_LATE3,
-              "%s: bf16 modes only", who);
+  ANC_REQUIRE((mode & ~kTileFlags) != ANC_NS_FP32, "%s: bf16 modes only", who);
   ANC_REQUIRE(steps >= 2 && steps <= 64 && coef != nullptr, "%s: steps=%d: 2..64", who, steps);
+  const int flags = mode & kTileFlags;
+  mode &= ~kTileFlags;
   hipStream_t s = anc_stream(stream);
   ChainProb cp[kMaxGroups];
   int order[kMaxGroups];
   for (int q = 0; q < n_probs; ++q) {
     const anc_ns_problem_t &b = probs[q];
     if (int rc = check_shape(b.E, b.M, b.N, mode, who)) return rc;
-    ANC_REQUIRE(b.M % 256 == 0 && b.N % 256 == 0, "%s: dims must be multiples of 256", who);
     ANC_REQUIRE(b.Uh != 0 && b.Ul != 0 && ((b.Uh | b.Ul | b.X32_out) & 15) == 0,
                 "%s: pointers must be 16-byte aligned and non-null", who);
     if (desc_tables == nullptr) ANC_REQUIRE(b.X32_out != 0, "%s: null X32_out", who);
@@ -1287,21 +1214,18 @@ static int pair_multi_impl(const char *who, const anc_ns_problem_t *probs, int32
       const anc_ns_problem_t &x = probs[order[a]], &y = probs[order[c]];
       if (y.N > x.N || (y.N == x.N && y.M > x.M)) { const int t = order[a]; order[a] = order[c]; order[c] = t; }
     }
+  NsPrologue pro{};
   for (int q = 0; q < n_probs; ++q) {
     const anc_ns_problem_t &b = probs[order[q]];
     const Plan pl = make_plan(b.workspace, b.E, b.M, b.N, mode, steps);
     ANC_REQUIRE(b.workspace_bytes >= pl.bytes, "%s: workspace holds %lld bytes, %lld needed", who,
                 (long long)b.workspace_bytes, (long long)pl.bytes);
-    { AncProfScope prof(ANC_PROF_NS_FRO, s); hipLaunchKernelGGL(k_fro_finalize, dim3((unsigned)b.E), dim3(kThreads), 0, s,
-                       (const double *)b.fro_partials, (int)b.n_partials, eps, pl.recip, pl.pow2); }
-    ANC_LAUNCH_CHECK();
-    { AncProfScope prof(ANC_PROF_NS_FRO, s); hipLaunchKernelGGL(k_pair_rescale, dim3((unsigned)b.E), dim3(kThreads), 0, s,
-                       (uint16_t *)b.Uh, (uint16_t *)b.Ul, pl.pow2, b.M * b.N); }
-    ANC_LAUNCH_CHECK();
+    add_prologue(pro, pl, b.Uh, b.Ul, b.fro_partials, b.n_partials, b.E, b.M * b.N);
     cp[q] = ChainProb{pl, (const uint16_t *)b.Uh, (const uint16_t *)b.Ul, 0, pl.recip, (float *)b.X32_out, b.E, b.M, b.N,
                       desc_tables ? (const anc_muon_desc_t *)desc_tables[order[q]] : nullptr};
   }
-  return run_bf16_chain(cp, n_probs, steps, coef, false, s, upd);
+  if (int rc = launch_prologue(pro, eps, s)) return rc;
+  return run_bf16_chain(cp, n_probs, steps, coef, flags, s, upd);
 }
 
 extern "C" int anc_ns_batched_pair_multi(const anc_ns_problem_t *probs, int32_t n_probs, int steps,
@@ -1311,7 +1235,7 @@ extern "C" int anc_ns_batched_pair_multi(const anc_ns_problem_t *probs, int32_t 
 
 // The same chain with the Muon weight update applied by the last step's epilogue: problem q's
 // matrix e is the orthogonalised update of the weight desc_tables[q][e] (p32, p16, K, N,
-// transpose, scale_idx and seed are read; p16t must be 0). Same bits in p32 and p16 as the chain
+// transpose, scale_idx and seed are read; p16t with ANC_MUON_P16T). Same bits in p32 and p16 as the chain
 // followed by anc_muon_update_multi, without the fp32 hand-off in between.
 extern "C" int anc_muon_ns_update_multi(const anc_ns_problem_t *probs, int32_t n_probs,
                                         const uint64_t *desc_tables, int steps, const float *coef, float eps,
@@ -1320,8 +1244,9 @@ extern "C" int anc_muon_ns_update_multi(const anc_ns_problem_t *probs, int32_t n
   ANC_REQUIRE(desc_tables != nullptr && lr_scales != nullptr, "anc_muon_ns_update_multi: null descriptor tables or lr_scales");
   NsUpdate u{};
   for (int k = 0; k < ANC_MUON_MAX_SCALES; ++k) u.lr[k] = lr_scales[k];
-  ANC_REQUIRE(sr == 0 || sr == ANC_SR_ON || sr == (ANC_SR_ON | ANC_SR_STEP_SEED),
-              "anc_muon_ns_update_multi: sr must be 0, ANC_SR_ON or ANC_SR_ON | ANC_SR_STEP_SEED");
+  const int sr_only = sr & ~ANC_MUON_P16T;
+  ANC_REQUIRE(sr_only == 0 || sr_only == ANC_SR_ON || sr_only == (ANC_SR_ON | ANC_SR_STEP_SEED),
+              "anc_muon_ns_update_multi: sr must be 0, ANC_SR_ON or ANC_SR_ON | ANC_SR_STEP_SEED, with or without ANC_MUON_P16T");
   ANC_REQUIRE(!(sr & ANC_SR_STEP_SEED) || ctl != 0, "anc_muon_ns_update_multi: ANC_SR_STEP_SEED needs the control block");
   u.sr = sr;
   u.seed_base = seed_base;

@@ -34,13 +34,11 @@ __device__ __forceinline__ void anc_pk_pair(float a, float b, uint32_t &hi, uint
   lo = anc_pk_bf16(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xFFFF0000u));
 }
 
-constexpr int BM = 128, BN = 128, BK = 64;
-constexpr int kCondParts = 8;            // partial sums per matrix of the conditioning proxy
-constexpr int PITCH = BK + 8;            // bf16 elements per LDS row: 144 bytes
-constexpr int kGemmThreads = 256;
+constexpr int kCondParts = 64;           // partial sums per matrix of the conditioning proxy
 constexpr int kXcds = 8;
 
 enum { EPI_GRAM = 0, EPI_BMAT = 1, EPI_BX = 2 };
+enum { VAR_NONE = 0, VAR_UPDATE = 1, VAR_PLAIN = 2, VAR_UPDATE_T = 3 };   // variants of the EPI_BX epilogue
 
 // Workgroup id -> logical tile id such that logical ids [start(x), start(x+1)) run on XCD x
 // (hardware deals consecutive workgroup ids round-robin over the 8 XCDs).
@@ -63,6 +61,8 @@ struct NsGemm {
   int lower;                 // symmetric output: tiles with tn <= tm only, mirrored
   int plain_sum;             // plain product: 1 = write X32 = (A32, if not null, else 0) + A B and, if Yh is
                              // not null, its bf16 copy (RNE) to Yh; 0 = write X32 = A B
+  int diag;                  // symmetric output: width of the blocks on the diagonal that are computed in full
+                             // (256 or 128); everything below them is mirrored
   int blk_r, blk_c;          // plain product and X = a X + B X: the tile sequence of a matrix runs block by block, blocks of
                              // blk_r x blk_c tiles (rows x columns): (tiles_m, 1) = column panel by column
                              // panel, (1, tiles_n) or 0 = row by row
@@ -71,8 +71,7 @@ struct NsGemm {
   float *A32;                // (E,M,M) fp32 A            GRAM out, BMAT in
   // With a32_gated set the fp32 copy of A exists only for the matrices that a32_flag marks (a null
   // a32_flag marks none): GRAM writes A32 for those alone and BMAT takes the off-diagonal entries
-  // of A from Fh (bf16) for every other matrix. Fh is then read at the output position, which for
-  // the 256-tile kernel means panel layout.
+  // of A from Fh (bf16) for every other matrix.
   int a32_gated;
   const int32_t *a32_flag;   // (E)
   uint16_t *Fh;              // (E,M,M) bf16 off-diag A   GRAM out
@@ -86,7 +85,7 @@ struct NsGemm {
   const anc_muon_desc_t *upd;  // BX, last step only: if set, matrix e is the Newton-Schulz result of the
                              // weight upd[e] and the epilogue applies W -= lr*O to it (p32, p16) instead
                              // of writing X32
-  const double *cond;        // null, or (E, kCondParts) partial sums of the conditioning proxy (see
+  const double *cond;        // null, or (E) the conditioning proxy's sum (see
                              // k_ns_cond): a matrix whose sum exceeds cond_thresh multiplies
                              // nterms_hard terms instead of nterms (its list is a prefix of the hard one)
   double cond_thresh;
@@ -103,19 +102,18 @@ struct NsGemm {
                              // acts on X = scale*U: GRAM multiplies its accumulator by scale^2, BX
                              // multiplies the accumulator and the epilogue's X by scale.
   // Panel layout of a bf16 matrix with R rows: element (r, c) at ((c / 32) * R + r) * 32 + c % 32,
-  // i.e. 32-column panels, each (R, 32) row-major. The K tile of a product is one panel, so the
+  // i.e. 32-column panels, each (R, 32) row-major. The K tile of a product is one or two panels, so the
   // rows a tile fetches are one contiguous block instead of 64-byte pieces of rows that lie a
-  // whole row pitch apart. 256-tile kernel only; R = M for every matrix of the chain.
-  int f_panel;               // Fh, Fl, Bh, Bl are in panel layout (GRAM, BMAT write them so; BMAT, BX read them so)
-  int x_panel;               // the input iterate (operands X of GRAM and BX, Xh/Xl of the BX epilogue)
-  int y_panel;               // the output iterate Yh/Yl of BX
-  // 8-bit low halves (256-tile X = a X + B X, panel layout only). Where the low half of a matrix's
+  // whole row pitch apart. R = M for every matrix of the chain. Everything the chain writes for itself (F, B, every
+  // iterate after the input) is in this layout.
+  int x_panel;               // the input iterate (operands X of GRAM and BX, Xh/Xl of the BX epilogue) is too
+  // 8-bit low halves. Where the low half of a matrix's
   // iterate is never a matrix-core operand it is kept as one byte per element (anc_low8_encode), in the first M*N bytes of the matrix's Xl (Yl) region, panels of
   // (M, 32) bytes: the epilogue then reads and writes 3 instead of 4 bytes per element. A matrix
   // takes the format on the input side if l8_in > 0, it is not flagged in l8_wide and its proxy
   // sum (l8_cond, the units of cond_thresh) does not exceed l8_in; l8_out likewise for the output.
   // The launches that read an iterate must be given the threshold it was written with.
-  const double *l8_cond;     // (E, kCondParts) or null (no matrix takes the format)
+  const double *l8_cond;     // (E) or null (no matrix takes the format)
   const int32_t *l8_wide;    // (E) or null
   double l8_in, l8_out;
 };
@@ -128,17 +126,6 @@ template <typename T> __device__ __forceinline__ T anc_ld_const(const T *p) {
   return *(const __attribute__((address_space(4))) T *)(p);
 }
 
-// Number of accumulation terms of matrix e: p.nterms, or p.nterms_hard for a matrix that the
-// conditioning proxy marks as hard. The partial sums are added in a fixed order, so every
-// workgroup of every launch takes the same decision for a matrix.
-__device__ __forceinline__ double anc_cond_sum(const double *cond, int e) {
-  const double *c = cond + (int64_t)e * kCondParts;
-  double s = anc_ld_const(c);
-#pragma unroll
-  for (int i = 1; i < kCondParts; ++i) s = s + anc_ld_const(c + i);
-  return s;
-}
-__device__ __forceinline__ double anc_ns_proxy(const NsGemm &p, int e) { return anc_cond_sum(p.cond, e); }
 // Did the classification flag matrix e for the second gate?
 __device__ __forceinline__ bool anc_ns_wide(const NsGemm &p, int e) {
   return p.wide_flag != nullptr && anc_ld_const(p.wide_flag + e) != 0;
@@ -152,7 +139,7 @@ __device__ __forceinline__ bool anc_ns_has_a32(const NsGemm &p, int e) {
 __device__ __forceinline__ bool anc_ns_low8(const NsGemm &p, int e, double thresh) {
   if (!(thresh > 0.0) || p.l8_cond == nullptr) return false;
   if (p.l8_wide != nullptr && anc_ld_const(p.l8_wide + e) != 0) return false;
-  return !(anc_cond_sum(p.l8_cond, e) > thresh);
+  return !(anc_ld_const(p.l8_cond + e) > thresh);
 }
 // The 8-bit low half of y next to its high half h = bf16(y), in the integer space of the fp32 bit
 // patterns, where rounding to bf16 is rounding to a multiple of 0x10000: d = bits(y) - (h << 16) lies
@@ -168,10 +155,11 @@ __device__ __forceinline__ uint32_t anc_low8_encode(float y, uint32_t htop) {
 __device__ __forceinline__ float anc_low8_decode(uint32_t htop, int q) {
   return __uint_as_float(htop + ((uint32_t)q << 8));
 }
+// Number of accumulation terms of matrix e: p.nterms, or more for a matrix that a gate marks.
 __device__ __forceinline__ int anc_ns_terms(const NsGemm &p, int e) {
   if (p.nterms_wide > 0 && anc_ns_wide(p, e)) return p.nterms_wide;
   if (p.cond == nullptr) return p.nterms;
-  return anc_ns_proxy(p, e) > p.cond_thresh ? p.nterms_hard : p.nterms;
+  return anc_ld_const(p.cond + e) > p.cond_thresh ? p.nterms_hard : p.nterms;
 }
 
 // Up to 8 independent problems of the same kind (the same product of different shape groups)
@@ -257,13 +245,18 @@ __device__ __forceinline__ void anc_seq_tile(const NsGemmMulti &pm, int bid, int
   L = pos;
 }
 
-// 256x256-tile kernel (ns_gemm_big.hip): same products, same accumulation order and
-// therefore the same bits as the 128x128 kernel; used when M and N are multiples of 256.
-int anc_ns_gemm_big(int epi, const NsGemm &p, int64_t E, hipStream_t s);
-// The same for n <= kMaxGroups problems in one launch (ps[k] with batch size Es[k]).
-// `upd` (may be null) carries the scalars of the fused weight update for problems whose `upd` is set.
-int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s,
-                          const NsUpdate *upd = nullptr);
+// One product of the chain for n <= kMaxGroups problems (ps[k] with batch size Es[k]) on the tiles that suit
+// the launch (ns.hip: the rule), or on tiles of `force` (64, 128, 256; 0: the rule). Every choice gives the
+// same bits. `upd` carries the scalars of the fused weight update for problems whose `upd` is set.
+int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int force, hipStream_t s,
+                      const NsUpdate *upd = nullptr);
+// The kernels behind it. 256x256 tiles for the symmetric products, 128x256 for X = a X + B X
+// (ns_gemm_big.hip; M and N multiples of 256); `by_rows`: X = a X + B X reads its B by rows k.
+int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool by_rows,
+                          const NsUpdate *upd);
+// 64x64 (small) or 128x128 tiles (ns_gemm_tile.hip; M and N multiples of 128); `plain`: the bare product.
+int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool small, bool by_rows,
+                           const NsUpdate *upd, bool plain);
 // Bare fp32 products C[e] = A[e] B[e] on the same K loop (ns_gemm_big.hip); a_transposed: A is
 // given as (K, M) row-major with row pitch ldA (and strideA between matrices), C = A^T B.
 int anc_ns_gemm_big_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool a_transposed = false);

@@ -20,7 +20,7 @@
 // X = a X + B X is the iterate itself, (k, n) row-major: its tile is [k][256 columns], fetched
 // as whole 512-byte rows, and its fragments come from transposing LDS reads
 // (ds_read_b64_tr_b16), so no transposed copy of the iterate exists anywhere.
-// Operands in panel layout (NsGemm::f_panel, x_panel) land in the same LDS positions; only the
+// Operands in panel layout (NsGemm::x_panel) land in the same LDS positions; only the
 // global addresses differ: an [row][k] tile is one contiguous block (rows 64 bytes apart, the
 // next K tile one panel further), a [k][n] tile one 2 KiB block per 32 columns.
 //
@@ -45,18 +45,13 @@
 // 128x128 kernel of ns.hip (terms in order, k ascending, one accumulator).
 #include <type_traits>
 
+#include "lds_dma.h"
 #include "ns_common.h"
 
 // Epilogue store: streaming, the written tile is not read again by this launch.
 template <typename T> __device__ __forceinline__ void epi_st(T *p, T v) { anc_st_stream(p, v); }
 
 namespace {
-
-#define LDS3(p) ((__attribute__((address_space(3))) void *)(p))
-#define GLB1(p) ((const __attribute__((address_space(1))) void *)(p))
-
-// X = a X + B X reads its symmetric B operand by rows k (see AT below).
-constexpr bool kBxReadsBByRows = true;
 
 struct Frags {
   bf16x8 a[4], b[2];
@@ -109,11 +104,10 @@ __device__ __forceinline__ void mfma8(const Frags &f, f32x16 (&acc)[4][2]) {
 // bf16 tile staging through LDS. `v` holds, for the wavefront's 32-row slab, the bf16 values of
 // its 2 column blocks in accumulator layout (element r: row 8*(r/4) + 4*(lane/32) + r%4, column
 // bj*32 + lane%32), packed two per dword: v[bj][i] = elements r = 2i (low half), 2i+1 (high).
-// Row-major output: out[row*ld + col]; transposed: outT[col*ldT + row].
-// With pstride > 0 the output is in panel layout: `out` addresses the slab's first row in its
-// first 32-column panel, rows lie 32 elements apart and the second panel pstride elements further.
+// `out` addresses the slab's first row in its first 32-column panel; the second panel lies pstride
+// elements further. The transposed slab is 64 rows of one panel.
 __device__ __forceinline__ void stage_rows(unsigned char *region, const uint32_t (&v)[2][8], int lane,
-                                           uint16_t *out, int64_t ld, int64_t pstride = 0) {
+                                           uint16_t *out, int64_t pstride) {
   uint16_t *t = (uint16_t *)region;                 // [32][72]
 #pragma unroll
   for (int bj = 0; bj < 2; ++bj)
@@ -127,8 +121,7 @@ __device__ __forceinline__ void stage_rows(unsigned char *region, const uint32_t
   for (int p = 0; p < 4; ++p) {
     const int idx = p * 64 + lane, row = idx >> 3, c8 = (idx & 7) * 8;
     const anc_u32x4 q = *(const anc_u32x4 *)(t + row * 72 + c8);
-    if (pstride > 0) epi_st((anc_u32x4 *)(out + (int64_t)(c8 >> 5) * pstride + row * 32 + (c8 & 31)), q);
-    else epi_st((anc_u32x4 *)(out + (int64_t)row * ld + c8), q);
+    epi_st((anc_u32x4 *)(out + (int64_t)(c8 >> 5) * pstride + row * 32 + (c8 & 31)), q);
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);
   __builtin_amdgcn_wave_barrier();
@@ -136,7 +129,7 @@ __device__ __forceinline__ void stage_rows(unsigned char *region, const uint32_t
 // Transposed: a lane's 4 consecutive rows are 4 consecutive elements of an output row, so they
 // go to LDS as one 8-byte write.
 __device__ __forceinline__ void stage_cols(unsigned char *region, const uint32_t (&v)[2][8], int lane,
-                                           uint16_t *outT, int64_t ldT) {
+                                           uint16_t *outT) {
   uint16_t *t = (uint16_t *)region;                 // [64][40]
 #pragma unroll
   for (int bj = 0; bj < 2; ++bj)
@@ -151,7 +144,7 @@ __device__ __forceinline__ void stage_cols(unsigned char *region, const uint32_t
   for (int p = 0; p < 4; ++p) {
     const int idx = p * 64 + lane, col = idx >> 2, r8 = (idx & 3) * 8;
     const anc_u32x4 q = *(const anc_u32x4 *)(t + col * 40 + r8);
-    epi_st((anc_u32x4 *)(outT + (int64_t)col * ldT + r8), q);
+    epi_st((anc_u32x4 *)(outT + col * 32 + r8), q);
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);
   __builtin_amdgcn_wave_barrier();
@@ -159,40 +152,11 @@ __device__ __forceinline__ void stage_cols(unsigned char *region, const uint32_t
 
 constexpr int kStageRegion = 6144;      // bytes of epilogue staging per wavefront (>= 64*40*2)
 
-// vmcnt(n): wait until at most n vector-memory operations of this wavefront are outstanding
-// (they complete in issue order), leaving lgkmcnt/expcnt alone.
-template <int N> __device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// One LDS-DMA instruction: lane l of the wavefront copies 16 bytes from g (per lane) to LDS byte
-// address lds_base + 16*l (lds_base wavefront-uniform, carried in M0). Written as inline
-// assembly so that the stage ring's explicit vmcnt waits are the only ones: the compiler's own
-// wait insertion is conservative about LDS-DMA writes that it cannot prove distinct from later
-// LDS reads and would drain the ring on every tile.
-__device__ __forceinline__ void dma16(const void *g, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(g)
-               : "memory", "m0");
-}
 __device__ __forceinline__ void dma16_epi(const void *g, uint32_t lds_base) { dma16(g, lds_base); }
-__device__ __forceinline__ uint32_t lds_addr(const void *p) {
-  return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const void *)p);
-}
-
-// Workgroup barrier that orders LDS traffic only: this wavefront's LDS reads and writes have
-// completed (lgkmcnt 0) before it arrives. Unlike __syncthreads() it carries no fence over
-// global memory, so LDS-DMA loads of younger stages stay in flight across it; the caller waits
-// (wait_vm<N>) for the DMA it needs before calling this.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // VAR (X = a X + B X only) selects a variant of the epilogue as its own instantiation, so that
 // the extra registers and branches do not weigh on the other launches: VAR_UPDATE applies the
-// weight update; VAR_PLAIN is the bare product C = A B written as fp32 (no iterate at the output
+// weight update, VAR_UPDATE_T refreshes a transposed bf16 copy of the weight as well; VAR_PLAIN is the bare product C = A B written as fp32 (no iterate at the output
 // position, no row scaling), which the weight-gradient GEMM uses; with `plain_sum` set it writes
 // C = (A32 or 0) + A B and, if Yh is set, the bf16 copy of C.
 // AT (X = a X + B X kernel only): the A operand is read transposed, from a (K, M) row-major matrix
@@ -201,7 +165,6 @@ __device__ __forceinline__ void lds_barrier() {
 // for the activations of a weight-gradient GEMM as they lie (C = x^T dy) and for the chain's
 // own B X, whose B is symmetric (stored in full): B read by rows k is B^T read by rows m, the
 // same values in the same order of summation.
-enum { VAR_NONE = 0, VAR_UPDATE = 1, VAR_PLAIN = 2 };
 template <int EPI, int TM, int TN, int TK, int NS, int MINBLOCKS, int VAR = VAR_NONE, bool AT = false>
 __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_gemm_big(NsGemmMulti pm) {
   constexpr int NWN = TN / 64, NWAVES = (TM / 128) * NWN;
@@ -275,8 +238,8 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   // (rows_of_the_matrix * 64 bytes) apart; a (k, n) tile is one 2 KiB block per 32 columns.
   const int ldA = p.ldA > 0 ? p.ldA : K;
   static_assert(TK == 32, "a K tile is one 32-column panel");
-  const bool a_pan = !PLAINV && (EPI == EPI_GRAM ? p.x_panel != 0 : p.f_panel != 0);
-  const bool b_pan = !PLAINV && (EPI == EPI_BMAT ? p.f_panel != 0 : p.x_panel != 0);
+  const bool a_pan = !PLAINV && (EPI != EPI_GRAM || p.x_panel != 0);
+  const bool b_pan = !PLAINV && (EPI == EPI_BMAT || p.x_panel != 0);
   const int64_t panel = (int64_t)p.M * 64;          // bytes per panel (every matrix of the chain has M rows)
   const int rpA = a_pan ? 64 : ldA * 2;             // bytes between consecutive rows of the A operand
   const int rpB = b_pan ? 64 : K * 2;               // the same for an "NT" B operand
@@ -465,7 +428,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   __syncthreads();
 
   // ---- epilogue
-  if (VAR == VAR_UPDATE && pm.ctl != nullptr && pm.ctl->skip != 0u) return;   // skipped step
+  if ((VAR == VAR_UPDATE || VAR == VAR_UPDATE_T) && pm.ctl != nullptr && pm.ctl->skip != 0u) return;   // skipped step
   const int M = p.M, N = p.N;
   const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
   unsigned char *region = st(wave / WPS) + (wave % WPS) * kStageRegion;
@@ -590,19 +553,21 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     // epilogue reads that block of the fp32 master, subtracts lr*O, writes it back together with
     // its bf16 copy. The master block is requested (8 x 16 bytes per lane) before the wait for
     // the slab's DMA, so that its latency runs under the wait and the arithmetic.
-    constexpr bool fused = (VAR == VAR_UPDATE);
+    constexpr bool fused = (VAR == VAR_UPDATE || VAR == VAR_UPDATE_T);
     constexpr bool plain = PLAINV;
     float *W32 = nullptr;
-    uint16_t *W16 = nullptr;
+    uint16_t *W16 = nullptr, *W16t = nullptr;
     float wlr = 0.0f;
     uint32_t wseed = 0;
-    int wN = 0;
+    int wN = 0, wK = 0;
     bool wtr = false;
     if (fused) {
       const anc_muon_desc_t &d = p.upd[e];
       W32 = (float *)d.p32;
       W16 = (uint16_t *)d.p16;
+      W16t = (uint16_t *)d.p16t;
       wN = d.N;
+      wK = d.K;
       wtr = d.transpose != 0;
       wlr = pm.lr[d.scale_idx & (ANC_MUON_MAX_SCALES - 1)];
       wseed = pm.seed_base + d.seed + ((pm.sr & ANC_SR_STEP_SEED) ? ANC_SR_SEED_STRIDE * pm.ctl->t : 0u);
@@ -787,9 +752,33 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
             }
             const anc_f32x4 po = {pp[0], pp[1], pp[2], pp[3]};
             epi_st((anc_f32x4 *)(W32 + we), po);
-            if (W16 != nullptr) {
-              const anc_u32x2 ho = {(hb[0] & 0xFFFFu) | (hb[1] << 16), (hb[2] & 0xFFFFu) | (hb[3] << 16)};
-              epi_st((anc_u32x2 *)(W16 + we), ho);
+            const anc_u32x2 ho = {(hb[0] & 0xFFFFu) | (hb[1] << 16), (hb[2] & 0xFFFFu) | (hb[3] << 16)};
+            if (W16 != nullptr) epi_st((anc_u32x2 *)(W16 + we), ho);
+            if (VAR == VAR_UPDATE_T) { pv[pz].x = __uint_as_float(ho.x); pv[pz].y = __uint_as_float(ho.y); }
+          }
+          if (VAR == VAR_UPDATE_T && W16t != nullptr) {
+            // The transposed copy: the slab's bf16 values cross the buffer, which O has left, once more. A lane then
+            // holds 32 consecutive rows of one column of W, 64 contiguous bytes of the copy. (These stores
+            // are not in the counts of the waits above, which makes the waits longer, never shorter.)
+            lds_wave_sync();
+            const int pitch = wtr ? 40 : 72;
+            uint16_t *sh = (uint16_t *)b;
+#pragma unroll
+            for (int pz = 0; pz < 8; ++pz) {
+              const int idx = pz * 64 + lane;
+              uint16_t *q = wtr ? sh + (idx >> 3) * pitch + (idx & 7) * 4 : sh + (idx >> 4) * pitch + (idx & 15) * 4;
+              *(anc_u32x2 *)q = anc_u32x2{__float_as_uint(pv[pz].x), __float_as_uint(pv[pz].y)};
+            }
+            lds_wave_sync();
+            const int wc = wtr ? lane & 31 : lane, wr = wtr ? (lane >> 5) * 32 : 0;
+            uint16_t *o = W16t + (int64_t)((wtr ? gi0 : gj0w) + wc) * wK + (wtr ? gj0w : gi0) + wr;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              uint32_t w[4];
+#pragma unroll
+              for (int k4 = 0; k4 < 4; ++k4)
+                w[k4] = (uint32_t)sh[(wr + 8 * i + 2 * k4) * pitch + wc] | ((uint32_t)sh[(wr + 8 * i + 2 * k4 + 1) * pitch + wc] << 16);
+              epi_st((anc_u32x4 *)(o + 8 * i), anc_u32x4{w[0], w[1], w[2], w[3]});
             }
           }
         }
@@ -827,10 +816,8 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         __builtin_amdgcn_s_waitcnt(0xC07F);
         __builtin_amdgcn_wave_barrier();
         // element offset of chunk c (8 columns) of slab row `row` in the output iterate
-        const bool y_pan = p.y_panel != 0;
         auto y_off = [&](int row, int c) -> int64_t {
-          return y_pan ? mn + ((int64_t)(gj0w / 32 + (c >> 2)) * M + gi0 + row) * 32 + (c & 3) * 8
-                       : mn + (int64_t)(gi0 + row) * N + gj0w + c * 8;
+          return mn + ((int64_t)(gj0w / 32 + (c >> 2)) * M + gi0 + row) * 32 + (c & 3) * 8;
         };
 #pragma unroll
         for (int pz = 0; pz < 4; ++pz) {
@@ -975,23 +962,22 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     }
     // Where the slab (rows gi0.., columns gj0w..) and its mirror image (rows gj0w.., columns gi0..:
     // 64 rows of one 32-column panel, a contiguous 4 KiB in panel layout) go in an (M, M) matrix.
-    const bool f_pan = p.f_panel != 0;
-    const int64_t o_rows = f_pan ? mm + ((int64_t)(gj0w / 32) * M + gi0) * 32 : mm + (int64_t)gi0 * M + gj0w;
-    const int64_t o_cols = f_pan ? mm + ((int64_t)(gi0 / 32) * M + gj0w) * 32 : mm + (int64_t)gj0w * M + gi0;
-    const int64_t ps = f_pan ? (int64_t)M * 32 : 0, ldT = f_pan ? 32 : M;
+    const int64_t o_rows = mm + ((int64_t)(gj0w / 32) * M + gi0) * 32;
+    const int64_t o_cols = mm + ((int64_t)(gi0 / 32) * M + gj0w) * 32;
+    const int64_t ps = (int64_t)M * 32;
     if (EPI == EPI_GRAM) {
-      stage_rows(region, hv, lane, p.Fh + o_rows, M, ps);
-      if (mirror) stage_cols(region, hv, lane, p.Fh + o_cols, ldT);
+      stage_rows(region, hv, lane, p.Fh + o_rows, ps);
+      if (mirror) stage_cols(region, hv, lane, p.Fh + o_cols);
       if (write_lo) {
-        stage_rows(region, lv, lane, p.Fl + o_rows, M, ps);
-        if (mirror) stage_cols(region, lv, lane, p.Fl + o_cols, ldT);
+        stage_rows(region, lv, lane, p.Fl + o_rows, ps);
+        if (mirror) stage_cols(region, lv, lane, p.Fl + o_cols);
       }
     } else if (EPI == EPI_BMAT) {
-      stage_rows(region, hv, lane, p.Bh + o_rows, M, ps);
-      if (mirror) stage_cols(region, hv, lane, p.Bh + o_cols, ldT);
+      stage_rows(region, hv, lane, p.Bh + o_rows, ps);
+      if (mirror) stage_cols(region, hv, lane, p.Bh + o_cols);
       if (write_lo) {
-        stage_rows(region, lv, lane, p.Bl + o_rows, M, ps);
-        if (mirror) stage_cols(region, lv, lane, p.Bl + o_cols, ldT);
+        stage_rows(region, lv, lane, p.Bl + o_rows, ps);
+        if (mirror) stage_cols(region, lv, lane, p.Bl + o_cols);
       }
       __builtin_amdgcn_s_waitcnt(0xC07F);
       asm volatile("" ::: "memory");
@@ -1006,9 +992,10 @@ int launch_sym(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s) {
   pm.n = n;
   int64_t grid = 0;
   for (int k = 0; k < n; ++k) {
-    ANC_REQUIRE(!ps[k].a32_gated || ps[k].f_panel, "anc_ns_gemm_big: A taken from Fh needs the panel layout");
+    ANC_REQUIRE(ps[k].diag == 256, "anc_ns_gemm_big: 256-wide blocks on the diagonal");
     pm.g[k] = ps[k];
     pm.g[k].tiles_m = pm.g[k].tiles_n = ps[k].M / 256;
+    pm.g[k].lower = 1;
     const int64_t t = Es[k] * ((int64_t)pm.g[k].tiles_m * (pm.g[k].tiles_m + 1) / 2);
     ANC_REQUIRE(t > 0 && t < (1ll << 30), "anc_ns_gemm_big: grid out of range");
     pm.tiles[k] = (int)t;
@@ -1037,8 +1024,8 @@ int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const N
     pm.g[k].lower = 0;
     ANC_REQUIRE(!(ps[k].l8_in > 0.0) || (ps[k].x_panel && ps[k].Xl != nullptr),
                 "anc_ns_gemm_big: 8-bit low halves of the input need the panel layout");
-    ANC_REQUIRE(!(ps[k].l8_out > 0.0) || (ps[k].y_panel && ps[k].Yl != nullptr),
-                "anc_ns_gemm_big: 8-bit low halves of the output need the panel layout");
+    ANC_REQUIRE(!(ps[k].l8_out > 0.0) || ps[k].Yl != nullptr,
+                "anc_ns_gemm_big: 8-bit low halves without an output for them");
     // A matrix's tiles are walked in blocks of 4 x 2 tiles (512 rows of B, 512 columns of X) instead
     // of row by row: the 64 workgroups an XCD runs together then share 4 row blocks of B and a few
     // column blocks of X per matrix instead of all of X, and its L2 fetches X from HBM about once
@@ -1065,7 +1052,12 @@ int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const N
     pm.seed_base = upd->seed_base;
     pm.ctl = upd->ctl;
   }
-  if (fused) {
+  if (fused && (upd->sr & ANC_MUON_P16T)) {
+    if (by_rows)
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_UPDATE_T, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+    else
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_UPDATE_T, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+  } else if (fused) {
     if (by_rows)
       hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_UPDATE, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
     else
@@ -1084,7 +1076,7 @@ int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const N
 
 // Symmetric products run on 256x256 tiles (lower triangle); X = a X + B X runs on 128x256 tiles
 // (the tile counts of the problems are recomputed here).
-int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s,
+int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool by_rows,
                           const NsUpdate *upd) {
   ANC_REQUIRE(n >= 1 && n <= kMaxGroups, "anc_ns_gemm_big: 1..%d problems per launch", kMaxGroups);
   for (int k = 0; k < n; ++k)
@@ -1092,29 +1084,7 @@ int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, h
                 "anc_ns_gemm_big: dims must be multiples of 256");
   if (epi == EPI_GRAM) return launch_sym<EPI_GRAM>(ps, Es, n, s);
   if (epi == EPI_BMAT) return launch_sym<EPI_BMAT>(ps, Es, n, s);
-  bool any_upd = false, all_upd = true;
-  for (int k = 0; k < n; ++k) { any_upd = any_upd || ps[k].upd != nullptr; all_upd = all_upd && ps[k].upd != nullptr; }
-  ANC_REQUIRE(any_upd == all_upd, "anc_ns_gemm_big: the fused update applies to every problem of a launch or to none");
-  ANC_REQUIRE(!any_upd || upd != nullptr, "anc_ns_gemm_big: fused update without its scalars");
-  // B is symmetric and stored in full, so its tile can be fetched by rows k (256-byte rows) as
-  // well as by rows m (64-byte row pieces). Measured per 5 launches: 84 x (1024, 3072) 4.12
-  // against 4.27 ms, 208 x (1024, 1024) 3.37 against 3.56 ms, but 64 x (512, 512) 0.238 against
-  // 0.212 ms: by rows k from M = 1024 on. The two ways read the same values except inside the
-  // diagonal 256x256 tiles of a B that descends from an A = X X^T with residual terms: there
-  // element (i, j) and element (j, i) add the same products in a different order and may differ
-  // in the last bit. So the way of reading is a property of the problem's shape, never of what
-  // it shares a call with: a call with problems of both kinds becomes two launches.
-  NsGemm part[kMaxGroups];
-  int64_t pe[kMaxGroups];
-  for (int pass = 0; pass < 2; ++pass) {
-    const bool by_rows = pass == 0;
-    int m = 0;
-    for (int k = 0; k < n; ++k)
-      if ((kBxReadsBByRows && ps[k].M >= 1024) == by_rows) { part[m] = ps[k]; pe[m] = Es[k]; ++m; }
-    if (m > 0)
-      if (int rc = launch_bx(part, pe, m, s, upd, by_rows)) return rc;
-  }
-  return ANC_OK;
+  return launch_bx(ps, Es, n, s, upd, by_rows);
 }
 
 // Bare products C[e] = A[e] B[e] (fp32 out, p.X32), A (M, K) with row pitch p.ldA -- or, with
@@ -1175,8 +1145,4 @@ int anc_ns_gemm_big_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_
     hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_PLAIN>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   ANC_LAUNCH_CHECK();
   return ANC_OK;
-}
-
-int anc_ns_gemm_big(int epi, const NsGemm &p, int64_t E, hipStream_t s) {
-  return anc_ns_gemm_big_multi(epi, &p, &E, 1, s, nullptr);
 }

@@ -1,0 +1,488 @@
+// The products of the Newton-Schulz chain (A = X X^T, B = b A + c A A, X = a X + B X with their
+// epilogues; see ns.hip for the arithmetic) on 64x64 and 128x128 tiles, and the bare product of the
+// weight-gradient GEMM on the same tiles: for launches that the 256-wide tiles of ns_gemm_big.hip
+// would leave most of the chip idle, and for dims that are multiples of 128 only.
+//
+// What bounds it. Operand bytes come into LDS at about 24 B per clock and CU whatever the tile, so a
+// product lasts as long as the CU with the most tiles needs for its operands: a single 1024x1024
+// output is 10 tiles of 256x256 (10 CUs at work, 512 K-bytes each step) or 160 of 64x64 (160 CUs,
+// 128), a quarter of the time although the operands are fetched four times as often. Which tile a
+// launch takes is anc_ns_gemm_multi's rule (below).
+//
+// Layout. 4 wavefronts as 2x2, each WB x WB blocks of v_mfma_f32_32x32x16_bf16 (tile 64 WB). A stage is 16 KiB,
+// one half per operand: KP = 2 (64x64) or 1 (128x128) panels of 32 k. Operands arrive in pieces of 16 rows x
+// 64 bytes, one LDS-DMA instruction each, four per wavefront and stage; stages form a ring of four,
+// two workgroups per CU. An operand whose rows are tile rows ("NT") lies in LDS as [panel][row][64 bytes] with the
+// 16-byte chunk index XORed with bits 2..3 of the row; an operand whose rows are k (the iterate in X = a X +
+// B X, its symmetric B from M = 1024 on, activations and output gradients) lies as [32-column block][k][64
+// bytes] without a swizzle: a transposing read touches 4 rows x 64 contiguous bytes, all banks once.
+// In panel layout both are contiguous in memory as well.
+//
+// Epilogue: block by block through a 32x36 fp32 buffer of the wavefront, so that a lane holds 16
+// consecutive columns of a row (or, for mirrored halves, transposed weights and their transposed copies, 16
+// consecutive rows of a column): a 32x32 block in panel layout is 2 KiB contiguous.
+//
+// Same bits as the 256-wide tiles: terms in order, k ascending, one accumulator, and a symmetric product is
+// computed directly inside the 256x256 blocks on the diagonal (128x128 where M is no multiple of 256) and mirrored outside,
+// where residual terms make element (i, j) and element (j, i) differ in the last bit.
+#include <type_traits>
+
+#include "lds_dma.h"
+#include "ns_common.h"
+
+namespace {
+
+constexpr int kRing = 4, kStageBytes = 16384, kIps = 4;   // stages, their size, DMA instructions per wavefront and stage
+constexpr int kSgPitch = 36;                              // floats per row of the epilogue buffer
+
+template <int EPI, int WB, bool AT, int VAR>
+__global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
+  constexpr int TM = 64 * WB, KP = WB == 1 ? 2 : 1, TK = 32 * KP;
+  constexpr bool BT = EPI == EPI_BX, PLAINV = VAR == VAR_PLAIN;
+  constexpr int kHalf = TM * TK * 2;
+  static_assert(2 * kHalf == kStageBytes && kHalf / 1024 == 8, "stage");
+  static_assert(!AT || BT, "A by rows k: X = a X + B X and the plain product only");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing * kStageBytes];
+
+  int gsel, L;
+  if (PLAINV && pm.seq) anc_seq_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
+  else anc_group_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
+  const NsGemm &p = pm.g[gsel];
+  int e, tm, tn;
+  if (p.lower) {
+    // lower triangle of blocks of G x G tiles (G = blk_r), every tile of a block computed
+    const int G = p.blk_r, q = p.tiles_m / G, per = G * G * (q * (q + 1) / 2);
+    e = L / per;
+    const int t = L % per, i = t % (G * G);
+    int b = t / (G * G), bm = 0;
+    while (b > bm) { b -= bm + 1; ++bm; }
+    tm = bm * G + i / G;
+    tn = b * G + i % G;
+  } else {
+    const int per = p.tiles_m * p.tiles_n, bper = p.blk_r * p.blk_c, across = p.tiles_n / p.blk_c;
+    e = L / per;
+    const int t = L % per, b = t / bper, i = t % bper;
+    tm = (b / across) * p.blk_r + i / p.blk_c;
+    tn = (b % across) * p.blk_c + i % p.blk_c;
+  }
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int K = p.K, nk = (K + TK - 1) / TK, total = anc_ns_terms(p, e) * nk;
+  // plain product only: K % 32 == 0, so with two panels per step the last step may hold one
+  const bool half_tail = PLAINV && KP == 2 && (K & 63) != 0;
+
+  // ---- DMA addressing. Bytes between rows and between 32-element panels of an operand.
+  const int M = p.M, N = p.N;
+  const bool a_pan = !PLAINV && (EPI != EPI_GRAM || p.x_panel != 0);
+  const bool b_pan = !PLAINV && (EPI == EPI_BMAT || p.x_panel != 0);
+  const int64_t panel = (int64_t)M * 64;
+  const int64_t rpA = a_pan ? 64 : (int64_t)(p.ldA > 0 ? p.ldA : K) * 2, rpB = b_pan ? 64 : (int64_t)(BT ? N : K) * 2;
+  const int64_t psA = a_pan ? panel : 64, psB = b_pan ? panel : 64;
+  const int dr = lane >> 2, dc = lane & 3;
+  const int64_t voA = (int64_t)dr * rpA + (AT ? dc : dc ^ (dr >> 2)) * 16;
+  const int64_t voB = (int64_t)dr * rpB + (BT ? dc : dc ^ (dr >> 2)) * 16;
+  int64_t offA[2], offB[2], cutA[2], cutB[2];     // this wavefront's two pieces of each operand; cut: see half_tail
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int q = wave * 2 + j;
+    const int pa = AT ? q / (TK / 16) : q / (TM / 16), ra = AT ? q % (TK / 16) : q % (TM / 16);
+    const int pb = BT ? q / (TK / 16) : q / (TM / 16), rb = BT ? q % (TK / 16) : q % (TM / 16);
+    offA[j] = pa * psA + ra * 16 * rpA;
+    offB[j] = pb * psB + rb * 16 * rpB;
+    cutA[j] = AT ? (ra >= 2 ? 32 * rpA : 0) : (pa >= 1 ? psA : 0);
+    cutB[j] = BT ? (rb >= 2 ? 32 * rpB : 0) : (pb >= 1 ? psB : 0);
+  }
+  const int64_t baseA = (int64_t)e * p.strideA * 2 + (AT ? (int64_t)(tm * (TM / 32)) * psA : (int64_t)tm * TM * rpA);
+  const int64_t baseB = (int64_t)e * p.strideB * 2 + (BT ? (int64_t)(tn * (TM / 32)) * psB : (int64_t)tn * TM * rpB);
+  const int64_t advA = AT ? TK * rpA : KP * psA, advB = BT ? TK * rpB : KP * psB;
+  const char *Ab[3], *Bb[3];
+#pragma unroll
+  for (int t3 = 0; t3 < 3; ++t3) {
+    Ab[t3] = (const char *)p.A[t3] + baseA;
+    Bb[t3] = (const char *)p.B[t3] + baseB;
+  }
+  const char *curA = Ab[0], *curB = Bb[0];
+  int is_kt = 0, is_term = 0;
+  auto issue = [&](unsigned char *st) {
+    const bool cut = half_tail && is_kt + 1 == nk;      // (the missing panel's pieces fetch the one that is there)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) dma16(curA + offA[j] - (cut ? cutA[j] : 0) + voA, lds_addr(st + (wave * 2 + j) * 1024));
+#pragma unroll
+    for (int j = 0; j < 2; ++j) dma16(curB + offB[j] - (cut ? cutB[j] : 0) + voB, lds_addr(st + kHalf + (wave * 2 + j) * 1024));
+    curA += advA;
+    curB += advB;
+    if (++is_kt == nk) {
+      is_kt = 0;
+      ++is_term;
+      curA = is_term == 1 ? Ab[1] : Ab[2];
+      curB = is_term == 1 ? Bb[1] : Bb[2];
+    }
+  };
+
+  // ---- fragment addressing: tr = [block][k][64 B] by transposing reads, else [panel][row][64 B]
+  const int l31 = lane & 31, hh = lane >> 5, g16 = lane >> 4, s16 = lane & 15;
+  const int tr_lane = (8 * (g16 >> 1) + (s16 >> 2)) * 64 + 32 * (g16 & 1) + 8 * (s16 & 3);
+  auto frag = [&](auto tr, const unsigned char *half, int blk, int kk) -> bf16x8 {
+    if constexpr (decltype(tr)::value) {
+      const unsigned char *q = half + blk * (TK * 64) + kk * 16 * 64 + tr_lane;
+      return anc_lds_tr_frag(q, q + 4 * 64);
+    } else {
+      return *(const bf16x8 *)(half + (kk >> 1) * (TM * 64) + (blk * 32 + l31) * 64 + ((((kk & 1) * 2 + hh) ^ ((l31 >> 2) & 3)) * 16));
+    }
+  };
+  using TrA = std::bool_constant<AT>;
+  using TrB = std::bool_constant<BT>;
+
+  f32x16 acc[WB][WB];
+#pragma unroll
+  for (int bi = 0; bi < WB; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < WB; ++bj)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[bi][bj][r] = 0.0f;
+
+  // ---- K loop. Step k lives in stage k % 4. At its top a wavefront waits for its own DMA of the step (two younger
+  // ones stay in flight), the workgroup meets, and the DMA of step k + 3 goes out into the stage everybody
+  // has just left.
+#pragma unroll
+  for (int s0 = 0; s0 < kRing - 1; ++s0)
+    if (s0 < total) issue(lds + s0 * kStageBytes);
+  auto body = [&](int step, int s0) {
+    if (step + kRing - 1 <= total) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
+    lds_barrier();
+    if (step + kRing - 1 < total) issue(lds + ((s0 + kRing - 1) % kRing) * kStageBytes);
+    const unsigned char *st = lds + s0 * kStageBytes;
+    const bool cut = half_tail && step + 1 == total;
+#pragma unroll
+    for (int kk = 0; kk < TK / 16; ++kk) {
+      if (PLAINV && kk >= 2 && cut) break;
+      bf16x8 a[WB], b[WB];
+#pragma unroll
+      for (int i = 0; i < WB; ++i) a[i] = frag(TrA{}, st, wm * WB + i, kk);
+#pragma unroll
+      for (int i = 0; i < WB; ++i) b[i] = frag(TrB{}, st + kHalf, wn * WB + i, kk);
+#pragma unroll
+      for (int bi = 0; bi < WB; ++bi)
+#pragma unroll
+        for (int bj = 0; bj < WB; ++bj)      // operands exchanged: a lane ends with runs of 4 columns of one row
+          acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bj], a[bi], acc[bi][bj], 0, 0, 0);
+    }
+  };
+  for (int step = 0; step < total; step += kRing) {
+#pragma unroll
+    for (int s0 = 0; s0 < kRing; ++s0)
+      if (step + s0 < total) body(step + s0, s0);
+  }
+  __syncthreads();
+
+  // ---- epilogue
+  if (VAR == VAR_UPDATE && pm.ctl != nullptr && pm.ctl->skip != 0u) return;   // skipped step
+  const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
+  float *sg = (float *)lds + wave * 32 * kSgPitch;
+  float sc = 1.0f;
+  if (EPI != EPI_BMAT && !PLAINV && p.scale != nullptr) sc = anc_ld_const(p.scale + e);
+  const float acc_scale = (EPI == EPI_GRAM) ? sc * sc : sc;
+  const bool write_lo = (EPI == EPI_GRAM ? p.Fl != nullptr : EPI == EPI_BMAT ? p.Bl != nullptr : false) &&
+                        (p.lo_gated == 0 || anc_ns_wide(p, e));
+  const bool has_a32 = EPI != EPI_BX && anc_ns_has_a32(p, e);
+  const bool in8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_in);
+  const bool out8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_out);
+  const int row = lane >> 1, c0 = (lane & 1) * 16;      // this lane's 16 elements of a block: row `row`, columns c0 ..
+                                                        // (or, reading the block transposed, column `row`, rows c0 ..)
+  float v[16];
+  auto put_rows = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const anc_f32x4 w = {v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+      *(anc_f32x4 *)(sg + row * kSgPitch + c0 + 4 * i) = w;
+    }
+    lds_wave_sync();
+  };
+  auto get_cols = [&]() {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = sg[(c0 + i) * kSgPitch + row];
+  };
+  auto unpack = [&](const anc_u32x4 &w, float *x) {
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { x[2 * i] = __uint_as_float(u[i] << 16); x[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u); }
+  };
+  // 16 floats -> 16 bf16 at out (32 bytes), and the residuals at lo if not null
+  auto put_bf16 = [&](uint16_t *out, uint16_t *lo) {
+    uint32_t h[8], l[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (lo != nullptr) anc_pk_pair(v[2 * i], v[2 * i + 1], h[i], l[i]);
+      else h[i] = anc_pk_bf16(v[2 * i], v[2 * i + 1]);
+    }
+    *(anc_u32x4 *)out = anc_u32x4{h[0], h[1], h[2], h[3]};
+    *(anc_u32x4 *)(out + 8) = anc_u32x4{h[4], h[5], h[6], h[7]};
+    if (lo != nullptr) {
+      *(anc_u32x4 *)lo = anc_u32x4{l[0], l[1], l[2], l[3]};
+      *(anc_u32x4 *)(lo + 8) = anc_u32x4{l[4], l[5], l[6], l[7]};
+    }
+  };
+#pragma unroll
+  for (int bi = 0; bi < WB; ++bi) {
+#pragma unroll
+    for (int bj = 0; bj < WB; ++bj) {
+      const int gi0 = tm * TM + (wm * WB + bi) * 32, gj0 = tn * TM + (wn * WB + bj) * 32;
+      const int gi = gi0 + row, gj = gj0 + c0;
+      // position of this lane's elements in a matrix of M rows in panel layout
+      const int64_t pan = ((int64_t)(gj0 / 32) * M + gi) * 32 + c0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const anc_f32x4 w = {acc[bi][bj][4 * q], acc[bi][bj][4 * q + 1], acc[bi][bj][4 * q + 2], acc[bi][bj][4 * q + 3]};
+        *(anc_f32x4 *)(sg + l31 * kSgPitch + 8 * q + 4 * hh) = w;
+      }
+      lds_wave_sync();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const anc_f32x4 w = *(const anc_f32x4 *)(sg + row * kSgPitch + c0 + 4 * i);
+        v[4 * i] = w.x; v[4 * i + 1] = w.y; v[4 * i + 2] = w.z; v[4 * i + 3] = w.w;
+      }
+      lds_wave_sync();                       // the buffer is free again
+      if constexpr (EPI != EPI_BX) {
+        const bool diag = gi0 == gj0;        // the block on the diagonal: element k = row - c0 of this lane
+        if (EPI == EPI_GRAM) {
+#pragma unroll
+          for (int k = 0; k < 16; ++k) v[k] = v[k] * acc_scale;
+          if (has_a32) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              *(anc_f32x4 *)(p.A32 + mm + (int64_t)gi * M + gj + 4 * i) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+          }
+          if (diag) {
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+              if (row == c0 + k) { p.dA[mv + gi] = v[k]; v[k] = 0.0f; }
+          }
+        } else {
+          float a[16];
+          if (has_a32) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const anc_f32x4 w = *(const anc_f32x4 *)(p.A32 + mm + (int64_t)gi * M + gj + 4 * i);
+              a[4 * i] = w.x; a[4 * i + 1] = w.y; a[4 * i + 2] = w.z; a[4 * i + 3] = w.w;
+            }
+          } else {
+            unpack(*(const anc_u32x4 *)(p.Fh + mm + pan), a);
+            unpack(*(const anc_u32x4 *)(p.Fh + mm + pan + 8), a + 8);
+          }
+          const float di = p.dA[mv + gi];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const anc_f32x4 dj = *(const anc_f32x4 *)(p.dA + mv + gj + 4 * i);
+            const float d[4] = {dj.x, dj.y, dj.z, dj.w};
+#pragma unroll
+            for (int k4 = 0; k4 < 4; ++k4) {
+              const int k = 4 * i + k4;
+              if (diag && row == c0 + k) {
+                const float a2 = v[k] + di * di;
+                p.dB[mv + gi] = p.cb * di + p.cc * a2;
+                v[k] = 0.0f;
+              } else {
+                const float a2 = v[k] + (di * a[k] + a[k] * d[k4]);   // symmetric in (i,j)
+                v[k] = p.cb * a[k] + p.cc * a2;
+              }
+            }
+          }
+        }
+        uint16_t *oh = EPI == EPI_GRAM ? p.Fh : p.Bh, *ol = EPI == EPI_GRAM ? p.Fl : p.Bl;
+        put_bf16(oh + mm + pan, write_lo ? ol + mm + pan : nullptr);
+        if (tm / p.blk_r != tn / p.blk_r) {  // mirror image: rows gj0 .., 32-column panel gi0/32
+          put_rows();
+          get_cols();
+          const int64_t pt = ((int64_t)(gi0 / 32) * M + gj0 + row) * 32 + c0;
+          put_bf16(oh + mm + pt, write_lo ? ol + mm + pt : nullptr);
+          lds_wave_sync();
+        }
+      } else if constexpr (PLAINV) {
+        const int64_t o = mn + (int64_t)gi * N + gj;
+        if (p.plain_sum && p.A32 != nullptr) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const anc_f32x4 w = *(const anc_f32x4 *)(p.A32 + o + 4 * i);
+            v[4 * i] = w.x + v[4 * i]; v[4 * i + 1] = w.y + v[4 * i + 1];
+            v[4 * i + 2] = w.z + v[4 * i + 2]; v[4 * i + 3] = w.w + v[4 * i + 3];
+          }
+        } else if (p.plain_sum) {
+#pragma unroll
+          for (int k = 0; k < 16; ++k) v[k] = 0.0f + v[k];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *(anc_f32x4 *)(p.X32 + o + 4 * i) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+        if (p.plain_sum && p.Yh != nullptr) {
+          uint32_t h[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) h[i] = (anc_bf16_rne_bits(v[2 * i]) & 0xFFFFu) | (anc_bf16_rne_bits(v[2 * i + 1]) << 16);
+          *(anc_u32x4 *)(p.Yh + o) = anc_u32x4{h[0], h[1], h[2], h[3]};
+          *(anc_u32x4 *)(p.Yh + o + 8) = anc_u32x4{h[4], h[5], h[6], h[7]};
+        }
+      } else {
+        // y = (a + dB) x + B X. Only the first iteration carries the input's scale.
+        const int64_t xo = mn + (p.x_panel ? pan : (int64_t)gi * N + gj);
+        const float cf = p.ca + p.dB[mv + gi];
+        const anc_u32x4 h0 = *(const anc_u32x4 *)(p.Xh + xo), h1 = *(const anc_u32x4 *)(p.Xh + xo + 8);
+        float x[16];
+        unpack(h0, x);
+        unpack(h1, x + 8);
+        if (in8) {
+          const anc_u32x4 q = *(const anc_u32x4 *)((const char *)p.Xl + mn * 2 + pan);
+          const uint32_t qq[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+          for (int k = 0; k < 16; ++k)
+            x[k] = anc_low8_decode(__float_as_uint(x[k]), (int)(qq[k >> 2] << (24 - 8 * (k & 3))) >> 24);
+        } else {
+          float xl[16];
+          unpack(*(const anc_u32x4 *)(p.Xl + xo), xl);
+          unpack(*(const anc_u32x4 *)(p.Xl + xo + 8), xl + 8);
+#pragma unroll
+          for (int k = 0; k < 16; ++k) x[k] = x[k] + xl[k];
+        }
+        if (p.scale != nullptr) {
+#pragma unroll
+          for (int k = 0; k < 16; ++k) v[k] = cf * (x[k] * sc) + v[k] * acc_scale;
+        } else {
+#pragma unroll
+          for (int k = 0; k < 16; ++k) v[k] = cf * x[k] + v[k];
+        }
+        if constexpr (VAR == VAR_UPDATE) {
+          // W -= lr O on the block's 32x32 elements of the weight (transposed where the chain ran on W^T)
+          const anc_muon_desc_t &d = p.upd[e];
+          float *W32 = (float *)d.p32;
+          uint16_t *W16 = (uint16_t *)d.p16, *W16t = (uint16_t *)d.p16t;
+          const bool wtr = d.transpose != 0;
+          const float wlr = pm.lr[d.scale_idx & (ANC_MUON_MAX_SCALES - 1)];
+          const uint32_t wseed = pm.seed_base + d.seed + ((pm.sr & ANC_SR_STEP_SEED) ? ANC_SR_SEED_STRIDE * pm.ctl->t : 0u);
+          const int wr0 = wtr ? gj0 : gi0, wc0 = wtr ? gi0 : gj0;
+          const int64_t we = (int64_t)(wr0 + row) * d.N + wc0 + c0;
+          anc_f32x4 pv[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) pv[i] = *(const anc_f32x4 *)(W32 + we + 4 * i);
+          if (wtr) {
+            put_rows();
+            get_cols();
+            lds_wave_sync();
+          }
+          uint32_t hb[16];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float pp[4] = {pv[i].x, pv[i].y, pv[i].z, pv[i].w};
+#pragma unroll
+            for (int k4 = 0; k4 < 4; ++k4) {
+              pp[k4] = pp[k4] - wlr * v[4 * i + k4];
+              const uint64_t el = (uint64_t)(we + 4 * i + k4);
+              hb[4 * i + k4] = ((pm.sr & ANC_SR_ON) ? anc_bf16_sr_bits(pp[k4], (uint32_t)(el >> 6), (uint32_t)(el & 63u), wseed)
+                                                    : anc_bf16_rne_bits(pp[k4])) & 0xFFFFu;
+            }
+            *(anc_f32x4 *)(W32 + we + 4 * i) = anc_f32x4{pp[0], pp[1], pp[2], pp[3]};
+          }
+          uint32_t hw[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) hw[i] = hb[2 * i] | (hb[2 * i + 1] << 16);
+          if (W16 != nullptr) {
+            *(anc_u32x4 *)(W16 + we) = anc_u32x4{hw[0], hw[1], hw[2], hw[3]};
+            *(anc_u32x4 *)(W16 + we + 8) = anc_u32x4{hw[4], hw[5], hw[6], hw[7]};
+          }
+          if (W16t != nullptr) {             // the (N, K) bf16 copy: the block's columns as rows
+            uint16_t *sh = (uint16_t *)sg;   // [32][40]
+            *(anc_u32x4 *)(sh + row * 40 + c0) = anc_u32x4{hw[0], hw[1], hw[2], hw[3]};
+            *(anc_u32x4 *)(sh + row * 40 + c0 + 8) = anc_u32x4{hw[4], hw[5], hw[6], hw[7]};
+            lds_wave_sync();
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              hw[i] = (uint32_t)sh[(c0 + 2 * i) * 40 + row] | ((uint32_t)sh[(c0 + 2 * i + 1) * 40 + row] << 16);
+            lds_wave_sync();
+            uint16_t *o = W16t + (int64_t)(wc0 + row) * d.K + wr0 + c0;
+            *(anc_u32x4 *)o = anc_u32x4{hw[0], hw[1], hw[2], hw[3]};
+            *(anc_u32x4 *)(o + 8) = anc_u32x4{hw[4], hw[5], hw[6], hw[7]};
+          }
+        } else if (p.X32 != nullptr) {
+          const int64_t o = mn + (int64_t)gi * N + gj;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            *(anc_f32x4 *)(p.X32 + o + 4 * i) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+        } else if (out8) {
+          uint32_t h[8], q[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            h[i] = anc_pk_bf16(v[2 * i], v[2 * i + 1]);
+            q[i >> 1] |= (anc_low8_encode(v[2 * i], h[i] << 16) | (anc_low8_encode(v[2 * i + 1], h[i] & 0xFFFF0000u) << 8)) << (16 * (i & 1));
+          }
+          *(anc_u32x4 *)(p.Yh + mn + pan) = anc_u32x4{h[0], h[1], h[2], h[3]};
+          *(anc_u32x4 *)(p.Yh + mn + pan + 8) = anc_u32x4{h[4], h[5], h[6], h[7]};
+          *(anc_u32x4 *)((char *)p.Yl + mn * 2 + pan) = anc_u32x4{q[0], q[1], q[2], q[3]};
+        } else {
+          put_bf16(p.Yh + mn + pan, p.Yl + mn + pan);
+        }
+      }
+    }
+  }
+}
+
+template <int EPI, bool AT, int VAR>
+void launch_tile(bool small, unsigned grid, hipStream_t s, const NsGemmMulti &pm) {
+  if (small) hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR>), dim3(grid), dim3(256), 0, s, pm);
+  else       hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, AT, VAR>), dim3(grid), dim3(256), 0, s, pm);
+}
+
+}  // namespace
+
+// n <= kMaxGroups problems of the same product in one launch on tiles of 64 (small) or 128. EPI_BX: `by_rows` as for the
+// 256-wide tiles; `plain`: the bare product, A transposed (by_rows) or not.
+int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool small, bool by_rows,
+                           const NsUpdate *upd, bool plain) {
+  const int T = small ? 64 : 128;
+  NsGemmMulti pm{};
+  pm.n = n;
+  int64_t grid = 0;
+  for (int k = 0; k < n; ++k) {
+    NsGemm &g = pm.g[k];
+    g = ps[k];
+    ANC_REQUIRE(g.M % 128 == 0 && g.N % 128 == 0 && g.K % (plain ? 32 : 128) == 0 && g.K > 0,
+                "anc_ns_gemm_tile: dims must be multiples of 128");
+    g.tiles_m = g.M / T;
+    g.tiles_n = (epi == EPI_BX ? g.N : g.M) / T;
+    g.lower = epi == EPI_BX ? 0 : 1;
+    int64_t per = (int64_t)g.tiles_m * g.tiles_n;
+    if (g.lower) {
+      ANC_REQUIRE((g.diag == 128 || g.diag == 256) && g.M % g.diag == 0, "anc_ns_gemm_tile: bad diagonal blocks");
+      g.blk_r = g.blk_c = g.diag / T;
+      const int64_t q = g.tiles_m / g.blk_r;
+      per = q * (q + 1) / 2 * g.blk_r * g.blk_c;
+    } else {
+      // walked in blocks of 256 x 256 (see launch_bx of the 256-wide kernel: what an XCD fetches)
+      g.blk_r = g.M % 256 == 0 ? 256 / T : 128 / T;
+      g.blk_c = g.N % 256 == 0 ? 256 / T : 128 / T;
+    }
+    ANC_REQUIRE(per > 0 && Es[k] * per < (1ll << 30), "anc_ns_gemm_tile: grid out of range");
+    pm.tiles[k] = (int)(Es[k] * per);
+    grid += pm.tiles[k];
+  }
+  ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_tile: grid out of range");
+  anc_fill_segments(pm);
+  const unsigned gr = (unsigned)grid;
+  if (plain) {
+    if (by_rows) launch_tile<EPI_BX, true, VAR_PLAIN>(small, gr, s, pm);
+    else         launch_tile<EPI_BX, false, VAR_PLAIN>(small, gr, s, pm);
+  } else if (epi == EPI_GRAM) {
+    launch_tile<EPI_GRAM, false, VAR_NONE>(small, gr, s, pm);
+  } else if (epi == EPI_BMAT) {
+    launch_tile<EPI_BMAT, false, VAR_NONE>(small, gr, s, pm);
+  } else if (upd != nullptr) {
+    for (int k = 0; k < ANC_MUON_MAX_SCALES; ++k) pm.lr[k] = upd->lr[k];
+    pm.sr = upd->sr;
+    pm.seed_base = upd->seed_base;
+    pm.ctl = upd->ctl;
+    if (by_rows) launch_tile<EPI_BX, true, VAR_UPDATE>(small, gr, s, pm);
+    else         launch_tile<EPI_BX, false, VAR_UPDATE>(small, gr, s, pm);
+  } else {
+    if (by_rows) launch_tile<EPI_BX, true, VAR_NONE>(small, gr, s, pm);
+    else         launch_tile<EPI_BX, false, VAR_NONE>(small, gr, s, pm);
+  }
+  ANC_LAUNCH_CHECK();
+  return ANC_OK;
+}

@@ -35,9 +35,12 @@ MODES = {"bf16": NS_BF16, "bf16_fast": NS_BF16_FAST, "bf16_x3": NS_BF16_X3, "fp3
          # the gated plan whatever the schedule ("bf16" turns into "bf16_late3" under Keller's
          # coefficients, see effective_mode)
          "bf16_gated": NS_BF16,
-         # same arithmetic forced onto the 128x128-tile kernel (ANC_NS_TILE128), for tests
+         # the formats of shapes that are no multiples of 256, on 128x128 tiles (ANC_NS_TILE128), for tests
          "bf16_tile128": NS_BF16 | 0x100, "bf16_fast_tile128": NS_BF16_FAST | 0x100,
-         "bf16_late3_tile128": NS_BF16_LATE3 | 0x100}
+         "bf16_late3_tile128": NS_BF16_LATE3 | 0x100,
+         # one tile size instead of the rule by launch size (ANC_NS_FORCE_T*): same bits, for tests
+         **{f"{name}_t{t}": m | flag for name, m in (("bf16", NS_BF16), ("bf16_late3", NS_BF16_LATE3), ("bf16_x3", NS_BF16_X3))
+            for t, flag in ((64, 0x200), (128, 0x400), (256, 0x800))}}
 
 
 def _coef_at(schedule, k):

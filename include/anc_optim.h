@@ -148,6 +148,7 @@ typedef struct {
  * from the step count of the control block (ctl must not be 0). */
 #define ANC_SR_ON           1
 #define ANC_SR_STEP_SEED    2
+#define ANC_MUON_P16T 4      /* anc_muon_ns_update_multi: some weights have a transposed bf16 copy to refresh */
 #define ANC_SR_SEED_STRIDE  1000003u
 
 /* ------------------------------------------------------------ grad-norm ----
@@ -497,6 +498,12 @@ int anc_quant_mxfp8_w(uint64_t w_bf16, uint64_t fp8_out, uint64_t scale_out, int
  * realisation of its rounding error (the results are then 1.2e-3 apart, each inside the accuracy
  * bar). The flag exists so that tests can show both. */
 #define ANC_NS_TILE128 0x100
+/* Flags OR-ed into a bf16 mode: run every product on tiles of 64x64, 128x128 or (dims that are multiples
+ * of 256) 256x256 / 128x256 outputs instead of choosing by the size of the launch. The bits are
+ * the same whichever runs; the flags exist so that tests can show it. */
+#define ANC_NS_FORCE_T64 0x200
+#define ANC_NS_FORCE_T128 0x400
+#define ANC_NS_FORCE_T256 0x800
 int64_t anc_ns_workspace_bytes(int64_t E, int64_t M, int64_t N, int mode);
 int anc_ns_batched(uint64_t X, int64_t E, int64_t M, int64_t N,
                    int steps, const float *coef /* host, 3*steps */, float eps,
@@ -526,7 +533,7 @@ int anc_ns_batched_pair(uint64_t Uh, uint64_t Ul, uint64_t fro_partials, int64_t
  * CUs stay busy where per-batch launches would each end in a partly filled last wave of
  * workgroups. No reference counterpart (the reference runs its shape groups one after the
  * other, ancora/optim/muon.py:257-277). Results equal anc_ns_batched_pair on each batch bit
- * for bit. n_probs <= 8; every M and N a multiple of 256; steps >= 2; bf16 modes. */
+ * for bit. n_probs <= 8; steps >= 2; bf16 modes. */
 typedef struct {
   uint64_t Uh, Ul;            /* input bf16 pair, (E,M,N) each                        */
   uint64_t fro_partials;      /* n_partials sums of u*u per matrix                     */
@@ -543,7 +550,8 @@ int anc_ns_batched_pair_multi(const anc_ns_problem_t *probs, int32_t n_probs, in
  * ancora/kernels/muon_ns.py:189-242, launched after the chain at ancora/optim/muon.py:272-277).
  * desc_tables[q] is a device array of problems[q].E anc_muon_desc_t, entry e describing the weight
  * whose orthogonalised update is matrix e of the batch (fields read: p32, p16 (may be 0), K, N,
- * transpose, scale_idx, seed; p16t must be 0). X32_out of the problems is not used. Results in
+ * transpose, scale_idx, seed, and p16t if `sr` carries ANC_MUON_P16T: a non-zero p16t then receives
+ * the transposed bf16 copy (N, K), without the flag no weight of the call may have one). X32_out of the problems is not used. Results in
  * p32 and p16 are bit-identical to the unfused sequence; the fp32 hand-off (8 bytes per parameter
  * of HBM traffic) disappears. ctl: the step's control block or 0 (skip flag honoured). sr as
  * for anc_muon_update_multi. */
@@ -563,7 +571,7 @@ int anc_ns_flops(int64_t E, int64_t M, int64_t N, int steps, int mode,
                  double *executed, double *dense);
 /* Of the E matrices of the last chain call that used `workspace`: how many took extra terms
  * through a conditioning gate, and the matrix-core work they add, all together, to
- * anc_ns_flops' `executed`. Synchronises `stream` and reads 64 bytes per matrix back. */
+ * anc_ns_flops' `executed`. Synchronises `stream` and reads 12 bytes per matrix back. */
 int anc_ns_hard_info(uint64_t workspace, int64_t E, int64_t M, int64_t N, int mode, int steps,
                      int32_t *n_gated, double *extra_flops, uint64_t stream);
 /* Executed matrix-core work of one product of one iteration of that chain: iteration k in

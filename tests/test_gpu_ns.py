@@ -175,6 +175,23 @@ def test_larger_and_odd_tile_counts_within_2e3(gpu, M, N):
         assert bits_equal(run_ns(X, mode="bf16_fast"), run_ns(X, mode="bf16_fast_tile128"))
 
 
+@pytest.mark.parametrize("M,N", [(128, 128), (128, 640), (256, 256), (384, 896), (256, 1024), (640, 640), (1024, 1024),
+                                 (1024, 1152), (1024, 2048), (1280, 2560)])
+@pytest.mark.parametrize("mode", ["bf16", "bf16_late3", "bf16_x3"])
+def test_tile_choice_keeps_the_bits(gpu, M, N, mode):
+    """A launch may run on 64x64, 128x128 or 256-wide tiles, whichever suits its size: one tile and odd tile
+    counts per side, dims that are multiples of 128 only (no 256-wide tiles there), gated and ungated matrices,
+    8-bit and 16-bit low halves. The bits are those of the choice the library makes by itself."""
+    rng = np.random.default_rng(M + 5 * N)
+    X = rng.standard_normal((3, M, N)).astype(np.float32)
+    X[1][:, : max(1, N // 100)] *= 100.0                        # outlier columns: the gates
+    X[2] = (rng.standard_normal((M, 8)) @ rng.standard_normal((8, N)) + 0.01 * X[2]).astype(np.float32)
+    want = run_ns(X, mode=mode)
+    for t in (64, 128, 256):
+        assert bits_equal(run_ns(X, mode=f"{mode}_t{t}"), want), t
+    assert rel_fro(want[0], host_ns(X[0], PE_SCHEDULE, 5)) < TOL_BF16
+
+
 def test_zero_matrix_and_scale_invariance(gpu):
     """A zero gradient (an idle expert) stays zero, no NaN; NS(cX) == NS(X) up to rounding."""
     rng = np.random.default_rng(3)
