@@ -19,6 +19,7 @@ NS_BF16, NS_FP32, NS_BF16_FAST, NS_BF16_X3, NS_BF16_LATE3 = 0, 1, 2, 3, 4   # AN
 GN_CHUNK = 8192                   # ANC_GN_CHUNK
 MUON_MAX_SCALES = 8               # ANC_MUON_MAX_SCALES
 SR_ON, SR_STEP_SEED, SR_SEED_STRIDE = 1, 2, 1000003   # ANC_SR_*
+MUON_P16T = 4                     # ANC_MUON_P16T
 ABI_VERSION = 3                   # the anc_abi_version() these prototypes were written for
 
 u64, i64, i32, u32, f32 = C.c_uint64, C.c_int64, C.c_int32, C.c_uint32, C.c_float

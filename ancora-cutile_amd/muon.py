@@ -16,11 +16,12 @@ Batching is bitwise neutral: a weight's result does not depend on which other we
 share its batch, on `chunk` or on `scope` (tests/training/test_batched_proj_muon.py:74).
 """
 import ctypes
+from operator import itemgetter
 
 import numpy as np
 
 from . import _lib
-from ._lib import api, MuonDesc, F32, BF16, MUON_MAX_SCALES, SR_ON, SR_STEP_SEED
+from ._lib import api, MuonDesc, F32, BF16, MUON_MAX_SCALES, MUON_P16T, SR_ON, SR_STEP_SEED
 from .bf16 import bf16_bits, bits_f32, bf16_round as _bf        # noqa: F401
 from .devbuf import DevBuf, upload_table
 from . import muon_ns
@@ -49,6 +50,23 @@ def _f32bf_trunc(x):
     return (np.ascontiguousarray(x, dtype=np.float32).view(np.uint32) >> np.uint32(16)).astype(np.uint16)
 
 
+_bufs_of = itemgetter("G", "p32", "p16", "buf", "p16T")     # what a descriptor is made of
+
+
+def _descs(weights, M, Nn, u_ptr, scale_index, blk0):
+    """Descriptors of one batch whose packed buffer starts at `u_ptr`, block numbers from blk0."""
+    out = []
+    for i, w in enumerate(weights):
+        K, N = w["K"], w["N"]
+        out.append(MuonDesc(w["buf"].ptr, w["G"].ptr, w["p32"].ptr,
+                            w["p16"].ptr if w["p16"] is not None else 0,
+                            u_ptr + i * M * Nn * 4, K, N, int(K > N),
+                            _g_code(w["G"].dtype), scale_index[w["scale"]], w["seed"], blk0,
+                            w["p16T"].ptr if w["p16T"] is not None else 0))
+        blk0 += (K * N) // 4096
+    return out, blk0
+
+
 class _Batch:
     """One packed Newton-Schulz batch: weights of one (M, Nn) shape, its descriptor table."""
 
@@ -61,23 +79,12 @@ class _Batch:
         self.fro = None              # per-block sums of u*u left by the pair momentum kernel
 
     def build(self, U, scale_index):
-        key = tuple((w["G"].ptr, w["G"].dtype.str, w["p32"].ptr, w["p16"].ptr if w["p16"] is not None else 0,
-                     w["buf"].ptr, w["p16T"].ptr if w.get("p16T") is not None else 0)
-                    for w in self.weights) + (U.ptr,)
+        key = [_bufs_of(w) for w in self.weights] + [U]
         if key == self.key:
             return
         if self.table is not None:
             self.table.free()
-        descs, blk0 = [], 0
-        for i, w in enumerate(self.weights):
-            K, N = w["K"], w["N"]
-            descs.append(MuonDesc(w["buf"].ptr, w["G"].ptr, w["p32"].ptr,
-                                  w["p16"].ptr if w["p16"] is not None else 0,
-                                  U.ptr + i * self.M * self.Nn * 4, K, N, int(K > N),
-                                  _g_code(w["G"].dtype), scale_index[w["scale"]], w["seed"], blk0,
-                                  w["p16T"].ptr if w.get("p16T") is not None else 0))
-            blk0 += (K * N) // 4096
-        self.total_blocks = blk0
+        descs, self.total_blocks = _descs(self.weights, self.M, self.Nn, U.ptr, scale_index, 0)
         self.table = upload_table(descs)
         self.key = key
 
@@ -88,6 +95,64 @@ class _Batch:
         if self.fro is not None:
             self.fro.free()
             self.fro = None
+
+
+class _Group:
+    """Every batch of an engine behind one descriptor table, so that a step is one momentum launch and one
+    chain call per 8 batches, whatever the number of batches. The batches' packed buffers are one
+    allocation: the high halves of all pairs first, the low halves behind them (the chain's last product
+    updates the weights itself, so nothing is handed back through the buffer)."""
+
+    PER_CALL = 8         # batches per chain call (ANC_MAX_GROUPS)
+
+    def __init__(self, batches, arena, scale_index):
+        self.batches, self.arena, self.scale_index = batches, arena, scale_index
+        self.weights = [w for b in batches for w in b.weights]
+        self.p16t = any(w["p16T"] is not None for w in self.weights)
+        self.n_el = sum(b.E * b.M * b.Nn for b in batches)
+        self.blocks = sum(w["K"] * w["N"] for w in self.weights) // 4096
+        self.fro = DevBuf.empty((self.blocks,), np.float64)
+        self.table = self.key = self.mode = None
+
+    def _calls(self, mode):
+        """(problems, count, tables) of each chain call."""
+        self.calls = []
+        el = blk = first = 0
+        for i0 in range(0, len(self.batches), self.PER_CALL):
+            part = self.batches[i0:i0 + self.PER_CALL]
+            probs, tables = (_lib.NsProblem * len(part))(), (ctypes.c_uint64 * len(part))()
+            for k, b in enumerate(part):
+                ws = b.ws.ensure(muon_ns.ns_workspace_bytes(b.E, b.M, b.Nn, mode))
+                hi = self.arena.ptr + el * 2
+                per = b.M * b.Nn // 4096
+                probs[k] = _lib.NsProblem(hi, hi + self.n_el * 2, self.fro.ptr + blk * 8, 0, ws.ptr, per, b.E, b.M, b.Nn,
+                                          ws.nbytes)
+                tables[k] = self.table.ptr + first * ctypes.sizeof(MuonDesc)
+                el += b.E * b.M * b.Nn
+                blk += b.E * per
+                first += b.E
+            self.calls.append((probs, len(part), tables))
+
+    def prepare(self, mode):
+        key = list(map(_bufs_of, self.weights))
+        if key != self.key:
+            if self.table is not None:
+                self.table.free()
+            descs, el, blk = [], 0, 0
+            for b in self.batches:
+                d, blk = _descs(b.weights, b.M, b.Nn, self.arena.ptr + el * 4, self.scale_index, blk)
+                descs += d
+                el += b.E * b.M * b.Nn
+            self.table = upload_table(descs)
+            self.key, self.mode = key, None
+        if self.mode != (mode, [b.ws.buf for b in self.batches]):
+            self._calls(mode)
+            self.mode = (mode, [b.ws.buf for b in self.batches])
+
+    def free(self):
+        self.fro.free()
+        if self.table is not None:
+            self.table.free()
 
 
 class MuonEngine:
@@ -112,14 +177,15 @@ class MuonEngine:
         # norm and scaling passes over the batch do not exist. Needs a bf16 mode and >= 2 steps
         # (the fp32 result overlays the pair); otherwise the fp32 hand-off is used.
         self.fused_prologue = mode != "fp32" and self.ns >= 2
-        # Grouped launches: the chains of up to 4 shape groups advance together, each product of
+        # Grouped launches: the chains of up to 8 batches advance together, each product of
         # each Newton-Schulz step being one launch over all of them (no partly filled last wave
-        # of workgroups per group). Needs the fused prologue, private buffers per batch and
-        # dims that are multiples of 256; other batches run one by one.
+        # of workgroups per group). Needs the fused prologue and private buffers per batch; other
+        # batches run one by one.
         self.grouped = True
         # Fused update: the epilogue of the chain's last product applies W -= lr*O itself (grouped
-        # path only; a weight with a transposed bf16 copy to refresh keeps the separate kernel).
+        # path only).
         self.fused_update = True
+        self._group = None
         groups = {}
         scales = []
         for idx, w in enumerate(weights):
@@ -130,6 +196,7 @@ class MuonEngine:
             if "scale" not in w:                                  # (a zero-padded weight brings its own)
                 w["scale"] = max(1.0, K / N) ** 0.5              # ancora/optim/muon.py:232
             w.setdefault("seed", idx)
+            w.setdefault("p16T", None)
             if w["scale"] not in scales:
                 scales.append(w["scale"])
             key = (w["M"], w["Nn"]) if scope is None else (w["M"], w["Nn"], w.get("lid", 0) // scope)
@@ -155,8 +222,12 @@ class MuonEngine:
         self._n_forked = 0
         self._streams, self._fork, self._join = [], None, []
         if self.concurrent:
+            total = sum(b.E * b.M * b.Nn for b in self.batches)
+            self.U = DevBuf.empty((total,), np.float32)          # one allocation, a slice per batch
+            off = 0
             for b in self.batches:
-                b.U = DevBuf.empty((b.E * b.M * b.Nn,), np.float32)
+                b.U = DevBuf(shape=(b.E * b.M * b.Nn,), dtype=np.float32, ptr=self.U.ptr + off * 4)
+                off += b.E * b.M * b.Nn
                 b.ws = NsWorkspace()
                 b.ws.ensure(muon_ns.ns_workspace_bytes(b.E, b.M, b.Nn, mode))
                 if len(self._streams) < self.MAX_STREAMS:
@@ -164,7 +235,6 @@ class MuonEngine:
                 self._join.append(_lib.Event())
             self._fork = _lib.Event()
             self.ws = None
-            self.U = None
         else:
             self.ws = NsWorkspace() if workspace is None else workspace
             self.U = None
@@ -179,7 +249,7 @@ class MuonEngine:
 
     def nbytes(self):
         if self.concurrent:
-            return sum(b.U.nbytes + b.ws.nbytes() for b in self.batches)
+            return self.U.nbytes + sum(b.ws.nbytes() for b in self.batches)
         return (self.U.nbytes if self.U is not None else 0) + self.ws.nbytes()
 
     def step(self, si, lr=0.02, schedule=_KELLER, guard=None, defer_join=False, device_steps=False):
@@ -201,8 +271,12 @@ class MuonEngine:
             seed_base = ((self.seed + 1000003 * self.t) & 0xFFFFFFFF) if self.sr else 0
         coef = muon_ns.coef_array(schedule, self.ns)
         self._run_mode = muon_ns.effective_mode(self.mode, schedule)
-        together = [b for b in self.batches
-                    if self.grouped and self.fused_prologue and b.M % 256 == 0 and b.Nn % 256 == 0]
+        if self.grouped and self.fused_prologue and self.fused_update and \
+                (self.concurrent or (self._own_ws and len(self.batches) == 1)):
+            self._forked = False
+            self._step_group(si, ctl, coef, lr_scales, seed_base)
+            return
+        together = list(self.batches) if self.grouped and self.fused_prologue else []
         if not self.concurrent and len(self.batches) > 1:
             # shared packed buffer and workspace: one batch per call, and only if that buys the
             # fused update
@@ -210,7 +284,7 @@ class MuonEngine:
             if not self.fused_update:
                 together = []
         else:
-            per_call = 4
+            per_call = 8
             if len(together) < 2 and not self.fused_update:
                 together = []
         alone = [b for b in self.batches if b not in together]
@@ -253,6 +327,18 @@ class MuonEngine:
         api.anc_muon_momentum_multi_pair(b.table.ptr, b.E, b.total_blocks, self.mom, int(self.nesterov),
                                          b.U.ptr, b.E * b.M * b.Nn * 2, b.fro.ptr, ctl, int(st))
 
+    def _step_group(self, si, ctl, coef, lr_scales, seed_base):
+        if self._group is None:
+            self._group = _Group(self.batches, self.U, self.scale_index)
+        g = self._group
+        g.prepare(self._run_mode)
+        api.anc_muon_momentum_multi_pair(g.table.ptr, len(g.weights), g.blocks, self.mom, int(self.nesterov),
+                                         g.arena.ptr, g.n_el * 2, g.fro.ptr, ctl, int(si))
+        sr = self._sr_arg | (MUON_P16T if g.p16t else 0)
+        for probs, n, tables in g.calls:
+            api.anc_muon_ns_update_multi(probs, n, tables, self.ns, coef, 1e-7, muon_ns.MODES[self._run_mode],
+                                         lr_scales, sr, seed_base, ctl, int(si))
+
     def _step_grouped(self, group, si, ctl, coef, lr_scales, seed_base):
         probs = (_lib.NsProblem * len(group))()
         for k, b in enumerate(group):
@@ -262,10 +348,11 @@ class MuonEngine:
             n_el = b.E * b.M * b.Nn
             probs[k] = _lib.NsProblem(b.U.ptr, b.U.ptr + n_el * 2, b.fro.ptr, b.U.ptr, buf.ptr,
                                       b.total_blocks // b.E, b.E, b.M, b.Nn, buf.nbytes)
-        if self.fused_update and not any(w.get("p16T") is not None for b in group for w in b.weights):
+        if self.fused_update:
+            sr = self._sr_arg | (MUON_P16T if any(w["p16T"] is not None for b in group for w in b.weights) else 0)
             tables = (ctypes.c_uint64 * len(group))(*[b.table.ptr for b in group])
             api.anc_muon_ns_update_multi(probs, len(group), tables, self.ns, coef, 1e-7,
-                                         muon_ns.MODES[self._run_mode], lr_scales, self._sr_arg, seed_base, ctl,
+                                         muon_ns.MODES[self._run_mode], lr_scales, sr, seed_base, ctl,
                                          int(si))
             return
         api.anc_ns_batched_pair_multi(probs, len(group), self.ns, coef, 1e-7, muon_ns.MODES[self._run_mode],
@@ -287,9 +374,13 @@ class MuonEngine:
         _lib.api.anc_device_sync()
         for b in self.batches:
             b.free()
+        if self._group is not None:
+            self._group.free()
+            self._group = None
         if self.concurrent:
+            self.U.free()
+            self.U = None
             for b in self.batches:
-                b.U.free()
                 b.ws.free()
             for st in self._streams:
                 api.anc_stream_destroy(st)
