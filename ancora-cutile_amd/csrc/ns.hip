@@ -791,13 +791,10 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       };
       // A = X X^T
       ga[q] = g;
-      ga[q].A[0] = curH[q]; ga[q].B[0] = curH[q]; ga[q].nterms = 1;
+      ga[q].A[0] = ga[q].B[0] = curH[q];
+      ga[q].A[1] = ga[q].B[1] = curL[q];
+      ga[q].nterms = split ? 3 : 1;
       const bool gated = pl.sp.gated(k);           // implies !split
-      if (split || gated || wide_g) {
-        ga[q].A[1] = curH[q]; ga[q].B[1] = curL[q];
-        ga[q].A[2] = curL[q]; ga[q].B[2] = curH[q];
-        if (split) ga[q].nterms = 3;
-      }
       if (gated) {
         ga[q].cond = pl.cond;
         ga[q].cond_thresh = (double)pl.sp.gate_tau[k] / (double)N;
@@ -812,12 +809,9 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       ga[q].K = (int)N; ga[q].strideA = mn; ga[q].strideB = mn;
       // B = b A + c A A
       gb[q] = g;
-      gb[q].A[0] = pl.Fh; gb[q].B[0] = pl.Fh; gb[q].nterms = 1;
-      if (split_fb || wide_a) {
-        gb[q].A[1] = pl.Fh; gb[q].B[1] = pl.Fl;
-        gb[q].A[2] = pl.Fl; gb[q].B[2] = pl.Fh;
-        if (split_fb) gb[q].nterms = 3;
-      }
+      gb[q].A[0] = gb[q].B[0] = pl.Fh;
+      gb[q].A[1] = gb[q].B[1] = pl.Fl;
+      gb[q].nterms = split_fb ? 3 : 1;
       if (wide_a) {
         set_wide(gb[q], 3);
         gb[q].Bl = pl.Bl;
@@ -826,20 +820,16 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       gb[q].K = (int)M; gb[q].strideA = M * M; gb[q].strideB = M * M;
       // X = a X + B X
       gx[q] = g;
-      gx[q].A[0] = pl.Bh; gx[q].B[0] = curH[q]; gx[q].nterms = 1;
-      if (split) { gx[q].A[gx[q].nterms] = pl.Bh; gx[q].B[gx[q].nterms] = curL[q]; ++gx[q].nterms; }
+      gx[q].A[0] = pl.Bh; gx[q].B[0] = curH[q];
+      gx[q].A[1] = pl.Bl; gx[q].B[1] = curL[q];
+      // (a plan never splits F and Boff before X: Bl alone does not occur)
+      gx[q].nterms = split_fb ? 3 : split ? 2 : 1;
       if (gated && ((pl.sp.gate_bx >> k) & 1u) && !split_fb) {
-        gx[q].A[1] = pl.Bh; gx[q].B[1] = curL[q];
         gx[q].cond = pl.cond;
         gx[q].cond_thresh = (double)pl.sp.gate_tau[k] / (double)N;
         gx[q].nterms_hard = 2;
       }
-      if (split_fb) { gx[q].A[gx[q].nterms] = pl.Bl; gx[q].B[gx[q].nterms] = curH[q]; ++gx[q].nterms; }
-      if (wide_a) {                                // [Bh Xh, Bh Xl, Bl Xh]: the lists above are prefixes of it
-        gx[q].A[1] = pl.Bh; gx[q].B[1] = curL[q];
-        gx[q].A[2] = pl.Bl; gx[q].B[2] = curH[q];
-        set_wide(gx[q], 3);
-      }
+      if (wide_a) set_wide(gx[q], 3);
       gx[q].K = (int)M; gx[q].strideA = M * M; gx[q].strideB = mn;
       gx[q].Xh = curH[q]; gx[q].Xl = curL[q];
       gx[q].Yh = last ? nullptr : pl.Xh[nxt[q]];

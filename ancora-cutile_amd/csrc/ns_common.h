@@ -49,9 +49,12 @@ __device__ __forceinline__ int xcd_remap(int bid, int grid) {
 }
 
 struct NsGemm {
-  const uint16_t *A[3];      // term t: rows of the output  (tiles_m*128 rows, ld = K)
-  const uint16_t *B[3];      // term t: columns of the output. GRAM, BMAT: one row per column, ld = K
+  const uint16_t *A[2];      // high and low half of the operand whose rows are the output's rows
+  const uint16_t *B[2];      // the same for the output's columns. GRAM, BMAT: one row per column, ld = K
                              // ("NT" product); BX: the iterate itself, (K, N) row-major, ld = N
+  // 1: A[0] B[0]; 2: + A[0] B[1]; 3: + A[1] B[0]. With more than one term the terms advance together, 32 k at a
+  // time: hh of k 0..15, hh of k 16..31, hl and lh of 16..31, hl and lh of 0..15. The halves of both operands are
+  // then fetched once per K tile (4 fetches for 3 products instead of 6), and every kernel adds in this order.
   int nterms;
   int K;
   int ldA;                   // elements between consecutive rows of A; 0 means K (only the plain

@@ -57,48 +57,37 @@ struct Frags {
   bf16x8 a[4], b[2];
 };
 
-template <int TK>
-__device__ __forceinline__ void load_frags(const unsigned char *sa, const unsigned char *sb, int a_base,
-                                           int b_base, int swz, Frags &f) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) f.a[i] = *(const bf16x8 *)(sa + a_base + i * (32 * TK * 2) + swz);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) f.b[i] = *(const bf16x8 *)(sb + b_base + i * (32 * TK * 2) + swz);
-}
-
-// Same fragments when the B tile is stored (k, n) row-major with 512-byte rows (the X = a X + B X
-// product reads the iterate as it lies in memory): the A fragments as above, the B fragments
-// through transposing LDS reads. tb[bj] is the lane's byte offset for k-step 0 of column
-// block bj (it carries the swizzle); a k-step advances 16 rows, the second read 4 rows.
-template <int TK>
-__device__ __forceinline__ void load_frags_bt(const unsigned char *st, int a_base, int swz, const int (&tb)[2],
-                                              int kk, Frags &f) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) f.a[i] = *(const bf16x8 *)(st + a_base + i * (32 * TK * 2) + swz);
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    f.b[i] = anc_lds_tr_frag(st + tb[i] + kk * (16 * 512), st + tb[i] + kk * (16 * 512) + 4 * 512);
-}
-
 // SWAP = false: accumulator block (bi,bj) holds C[32 bi + row][32 bj + col] with col = lane%32
 // and element r = row 8*(r/4) + 4*(lane/32) + r%4. SWAP = true computes the transposed block
 // (operands exchanged, same products, same order of summation): row = lane%32 and element
 // r = col 8*(r/4) + 4*(lane/32) + r%4, i.e. a lane holds runs of 4 consecutive columns of one
 // output row, which is what a row-major epilogue wants.
 template <bool SWAP>
-__device__ __forceinline__ void mfma1(const Frags &f, f32x16 (&acc)[4][2], int idx) {
+__device__ __forceinline__ void mfma1(const bf16x8 (&a)[4], const bf16x8 (&b)[2], f32x16 (&acc)[4][2], int idx) {
   const int bi = idx >> 1, bj = idx & 1;
-  acc[bi][bj] = SWAP ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[bj], f.a[bi], acc[bi][bj], 0, 0, 0)
-                     : __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[bi], f.b[bj], acc[bi][bj], 0, 0, 0);
+  acc[bi][bj] = SWAP ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bj], a[bi], acc[bi][bj], 0, 0, 0)
+                     : __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
+}
+// 8 MFMAs with n DMA instructions (`piece(i)`) between them, one every 8/n, instead of as a burst
+// during which the matrix pipe idles.
+template <bool SWAP, int N, typename F>
+__device__ __forceinline__ void mfma8_dma(const bf16x8 (&a)[4], const bf16x8 (&b)[2], f32x16 (&acc)[4][2], F piece) {
+#pragma unroll
+  for (int idx = 0; idx < 8; ++idx) {
+    mfma1<SWAP>(a, b, acc, idx);
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (((i + 1) * 8 + N - 1) / N - 1 == idx) {
+        __builtin_amdgcn_sched_barrier(0);
+        piece(i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  }
 }
 template <bool SWAP>
-__device__ __forceinline__ void mfma8(const Frags &f, f32x16 (&acc)[4][2]) {
+__device__ __forceinline__ void mfma8(const bf16x8 (&a)[4], const bf16x8 (&b)[2], f32x16 (&acc)[4][2]) {
 #pragma unroll
-  for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj)
-      acc[bi][bj] = SWAP ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[bj], f.a[bi], acc[bi][bj], 0, 0, 0)
-                         : __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[bi], f.b[bj], acc[bi][bj], 0, 0, 0);
+  for (int idx = 0; idx < 8; ++idx) mfma1<SWAP>(a, b, acc, idx);
 }
 
 // bf16 tile staging through LDS. `v` holds, for the wavefront's 32-row slab, the bf16 values of
@@ -226,7 +215,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / NWN, wn = wave % NWN;
-  const int K = p.K, nk = K / TK, total = anc_ns_terms(p, e) * nk;
+  const int K = p.K, nk = K / TK;
 
   // ---- DMA addressing: this wavefront moves IA*RPI rows of the A tile and IB*RPI rows of the B
   //      tile, RPI rows per instruction; lane -> (row lane/CPR, physical chunk lane%CPR). The
@@ -274,48 +263,31 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   const int64_t ubaseBT = b_pan ? (int64_t)e * p.strideB * 2 + (int64_t)(tn * (TN / 32)) * panel + (int64_t)(wave * IB * 2) * 64
                                 : ((int64_t)e * p.strideB + (int64_t)tn * TN + (int64_t)(wave * IB * 2) * ldn) * 2;
 
-  // Operand pointers of the three terms are fetched from the argument block once, here: a
-  // scalar load inside the K loop would have to be waited for with lgkmcnt(0), which also
-  // waits for the LDS fragment reads in flight. K tiles are issued strictly in order, so the
-  // running pointers just advance.
-  const char *Abase[3], *Bbase[3];
-#pragma unroll
-  for (int t3 = 0; t3 < 3; ++t3) {
-    Abase[t3] = (const char *)p.A[t3] + ubaseA;
-    Bbase[t3] = (const char *)p.B[t3] + (BT ? ubaseBT : ubaseB);
-  }
+  // K tiles are issued strictly in order, so the running pointers just advance (a scalar load inside
+  // the K loop would have to be waited for with lgkmcnt(0), which also waits for the LDS
+  // fragment reads in flight).
   // bytes from one K tile to the next, and from one DMA instruction of a tile to the next
   const int64_t advB = BT ? (b_pan ? (int64_t)TK * 64 : (int64_t)TK * ldn * 2) : (b_pan ? panel : (int64_t)ROWB);
   const int64_t advA = AT ? (a_pan ? (int64_t)TK * 64 : (int64_t)TK * ldA * 2) : (a_pan ? panel : (int64_t)ROWB);
   const int64_t roA = AT ? (a_pan ? (int64_t)4 * 64 : (int64_t)4 * ldA * 2) : (int64_t)RPI * rpA;
   const int64_t roB = BT ? (b_pan ? (int64_t)2 * 64 : (int64_t)2 * ldn * 2) : (int64_t)RPI * rpB;
-  const char *curA = Abase[0], *curB = Bbase[0];
-  int is_kt = 0, is_term = 0;
+  const char *curA = (const char *)p.A[0] + ubaseA, *curB = (const char *)p.B[0] + (BT ? ubaseBT : ubaseB);
   // DMA instruction i of a stage (0 .. IPS-1: the A tile's IA, then the B tile's IB)
-  auto issue_piece = [&](int i, unsigned char *stage) {
+  auto issue_piece = [&](int i, unsigned char *stage, const char *pa, const char *pb) {
     if (i < IA) {
       const uint32_t vo = AT ? voffAT : ((i & 1) ? voff1 : voff0);
-      dma16(curA + i * roA + vo, lds_addr(stage + (wave * IA + i) * 1024));
+      dma16(pa + i * roA + vo, lds_addr(stage + (wave * IA + i) * 1024));
     } else {
       const int j = i - IA;
       const uint32_t vo = BT ? ((j & 1) ? voffB1 : voffB0) : ((j & 1) ? voffN1 : voffN0);
-      dma16(curB + j * roB + vo, lds_addr(stage + TM * ROWB + (wave * IB + j) * 1024));
-    }
-  };
-  auto issue_advance = [&]() {
-    curA += advA;
-    curB += advB;
-    if (++is_kt == nk) {
-      is_kt = 0;
-      ++is_term;
-      curA = is_term == 1 ? Abase[1] : Abase[2];
-      curB = is_term == 1 ? Bbase[1] : Bbase[2];
+      dma16(pb + j * roB + vo, lds_addr(stage + TM * ROWB + (wave * IB + j) * 1024));
     }
   };
   auto issue = [&](unsigned char *stage) {
 #pragma unroll
-    for (int i = 0; i < IPS; ++i) issue_piece(i, stage);
-    issue_advance();
+    for (int i = 0; i < IPS; ++i) issue_piece(i, stage, curA, curB);
+    curA += advA;
+    curB += advB;
   };
 
   // ---- fragment addressing
@@ -344,16 +316,21 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       ta[bi] = (8 * (g16 >> 1) + (s16 >> 2)) * 256 + ((chunk ^ ((s16 >> 2) << 2)) * 16) + (s16 & 1) * 8;
     }
   }
+  auto frag_a = [&](const unsigned char *stg, int kk, bf16x8 (&f)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      f[i] = AT ? anc_lds_tr_frag(stg + ta[i] + kk * (16 * 256), stg + ta[i] + kk * (16 * 256) + 4 * 256)
+                : *(const bf16x8 *)(stg + a_base + i * (32 * TK * 2) + swz[kk]);
+  };
+  auto frag_b = [&](const unsigned char *stg, int kk, bf16x8 (&f)[2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      f[i] = BT ? anc_lds_tr_frag(stg + tb[i] + kk * (16 * 512), stg + tb[i] + kk * (16 * 512) + 4 * 512)
+                : *(const bf16x8 *)(stg + b_base + i * (32 * TK * 2) + swz[kk]);
+  };
   auto frags = [&](const unsigned char *stg, int kk, Frags &f) {
-    if (AT) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        f.a[i] = anc_lds_tr_frag(stg + ta[i] + kk * (16 * 256), stg + ta[i] + kk * (16 * 256) + 4 * 256);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        f.b[i] = anc_lds_tr_frag(stg + tb[i] + kk * (16 * 512), stg + tb[i] + kk * (16 * 512) + 4 * 512);
-    } else if (BT) load_frags_bt<TK>(stg, a_base, swz[kk], tb, kk, f);
-    else load_frags<TK>(stg, stg, a_base, b_base, swz[kk], f);
+    frag_a(stg, kk, f.a);
+    frag_b(stg, kk, f.b);
   };
 
   f32x16 acc[4][2];
@@ -364,66 +341,166 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[bi][bj][r] = 0.0f;
 
-  // Stage ring. Tile k lives in stage k % NS. The DMA of tile k+NS-1 is started at the top of
-  // tile k, into the stage that tile k-1 was read from (every wavefront left it before the
-  // barrier inside tile k-1). Before the last k-step of tile k each wavefront waits until its
-  // own DMA of tile k+1 has landed (NS-2 younger tiles may still be in flight), all
-  // wavefronts synchronise, and the first fragments of tile k+1 load under the last MFMAs.
-  Frags f[2];
+  const int nterms = PLAINV ? 1 : anc_ns_terms(p, e);
+  if (nterms == 1) {
+    // Stage ring. Tile k lives in stage k % NS. The DMA of tile k+NS-1 is started at the top of
+    // tile k, into the stage that tile k-1 was read from (every wavefront left it before the
+    // barrier inside tile k-1). Before the last k-step of tile k each wavefront waits until its
+    // own DMA of tile k+1 has landed (NS-2 younger tiles may still be in flight), all
+    // wavefronts synchronise, and the first fragments of tile k+1 load under the last MFMAs.
+    Frags f[2];
 #pragma unroll
-  for (int s0 = 0; s0 < NS - 1; ++s0)
-    if (s0 < total) issue(st(s0));
-  if (total >= NS - 1) wait_vm<(NS - 2) * IPS>(); else wait_vm<0>();
-  lds_barrier();
-  frags(stage0, 0, f[0]);
-
-  // f[kk&1] holds k-step kk (KSTEPS is even, so every tile starts on f[0] and ends on f[1]).
-  // `steady` (a std::true_type): the caller knows that this tile refills the ring and has a
-  // successor, so the body carries no branch.
-  auto body = [&](auto steady, int step, unsigned char *cur, unsigned char *nxt, unsigned char *fill) {
-    constexpr bool kSteady = decltype(steady)::value;
-    const bool more = kSteady || step + 1 < total;
-    const bool refill = kSteady || step + NS - 1 < total;
-    if (KSTEPS == 2) {
-      // The stage's DMA instructions go out between the MFMAs of the first k-step, one every
-      // 8/IPS matrix instructions, instead of as a burst during which the matrix pipe idles.
-      frags(cur, 1, f[1]);
-#pragma unroll
-      for (int idx = 0; idx < 8; ++idx) {
-        mfma1<BT>(f[0], acc, idx);
-#pragma unroll
-        for (int i = 0; i < IPS; ++i)
-          if (((i + 1) * 8 + IPS - 1) / IPS - 1 == idx) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (refill) issue_piece(i, fill);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-      }
-      if (refill) issue_advance();
-    } else {
-      if (refill) issue(fill);
-#pragma unroll
-      for (int kk = 0; kk < KSTEPS - 1; ++kk) {
-        frags(cur, kk + 1, f[(kk + 1) & 1]);
-        mfma8<BT>(f[kk & 1], acc);
-      }
-    }
-    if (refill) wait_vm<(NS - 2) * IPS>(); else wait_vm<0>();
+    for (int s0 = 0; s0 < NS - 1; ++s0)
+      if (s0 < nk) issue(st(s0));
+    if (nk >= NS - 1) wait_vm<(NS - 2) * IPS>(); else wait_vm<0>();
     lds_barrier();
-    if (more) frags(nxt, 0, f[0]);
-    mfma8<BT>(f[(KSTEPS - 1) & 1], acc);
-  };
-  int step = 0;
-  // rounds of NS tiles in which even the last tile (step + NS - 1) still refills the ring
-  for (; step + 2 * NS - 2 < total; step += NS) {
+    frags(stage0, 0, f[0]);
+
+    // f[kk] holds k-step kk. `steady` (a std::true_type): the caller knows that this tile refills
+    // the ring and has a successor, so the body carries no branch.
+    auto body = [&](auto steady, int step, unsigned char *cur, unsigned char *nxt, unsigned char *fill) {
+      constexpr bool kSteady = decltype(steady)::value;
+      const bool more = kSteady || step + 1 < nk;
+      const bool refill = kSteady || step + NS - 1 < nk;
+      frags(cur, 1, f[1]);
+      mfma8_dma<BT, IPS>(f[0].a, f[0].b, acc, [&](int i) { if (refill) issue_piece(i, fill, curA, curB); });
+      if (refill) {
+        curA += advA;
+        curB += advB;
+        wait_vm<(NS - 2) * IPS>();
+      } else {
+        wait_vm<0>();
+      }
+      lds_barrier();
+      if (more) frags(nxt, 0, f[0]);
+      mfma8<BT>(f[1].a, f[1].b, acc);
+    };
+    int step = 0;
+    // rounds of NS tiles in which even the last tile (step + NS - 1) still refills the ring
+    for (; step + 2 * NS - 2 < nk; step += NS) {
 #pragma unroll
-    for (int s0 = 0; s0 < NS; ++s0)
-      body(std::true_type{}, step + s0, st(s0), st((s0 + 1) % NS), st((s0 + NS - 1) % NS));
-  }
-  for (; step < total; step += NS) {
+      for (int s0 = 0; s0 < NS; ++s0)
+        body(std::true_type{}, step + s0, st(s0), st((s0 + 1) % NS), st((s0 + NS - 1) % NS));
+    }
+    for (; step < nk; step += NS) {
 #pragma unroll
-    for (int s0 = 0; s0 < NS; ++s0)
-      if (step + s0 < total) body(std::false_type{}, step + s0, st(s0), st((s0 + 1) % NS), st((s0 + NS - 1) % NS));
+      for (int s0 = 0; s0 < NS; ++s0)
+        if (step + s0 < nk) body(std::false_type{}, step + s0, st(s0), st((s0 + 1) % NS), st((s0 + NS - 1) % NS));
+    }
+  } else if constexpr (!PLAINV) {
+    // Several terms: K tile t is two stages, the high halves h_t in stage 2t % NS and the low halves l_t in
+    // the next one (of two terms only B's low half is there). Six phases of 8 MFMAs per tile,
+    //   P0 hh k 0..15, P1 hh 16..31, P2 hl 16..31, P3 lh 16..31, P4 hl 0..15, P5 lh 0..15,
+    // each under the fragment reads of the next. Everybody has read h_t and l_t when the barrier before P5 opens:
+    // both stages refill from there on, in P5 and P0 of the next tile. l_t is waited for inside P1, h_{t+1} before P5.
+    //   NS = 4: P5 fetches h_{t+2}, P0 l_{t+1};  NS = 3: P5 fetches l_{t+1}, P0 h_{t+1}.
+    // Against one term after the other the operands are fetched 4 instead of 6 times and read from LDS 30 instead of 36
+    // times per tile.
+    const char *loA = (const char *)p.A[1] + ubaseA, *loB = (const char *)p.B[1] + (BT ? ubaseBT : ubaseB);
+    auto pairs = [&](auto nt) {
+      constexpr int NT = decltype(nt)::value, PL = NT == 3 ? IPS : IB;      // DMA instructions of a low stage
+      auto piece_h = [&](int i, unsigned char *stage) { issue_piece(i, stage, curA, curB); };
+      auto piece_l = [&](int i, unsigned char *stage) { issue_piece(NT == 3 ? i : IA + i, stage, loA, loB); };
+      auto adv_h = [&]() { curA += advA; curB += advB; };
+      auto adv_l = [&]() { loA += advA; loB += advB; };
+      auto all_h = [&](unsigned char *stage) {
+#pragma unroll
+        for (int i = 0; i < IPS; ++i) piece_h(i, stage);
+        adv_h();
+      };
+      auto all_l = [&](unsigned char *stage) {
+#pragma unroll
+        for (int i = 0; i < PL; ++i) piece_l(i, stage);
+        adv_l();
+      };
+      bf16x8 a[2][4], b[2][2];
+      all_h(st(0));
+      all_l(st(1));
+      if (NS == 4) {
+        if (nk > 1) { all_h(st(2)); wait_vm<PL + IPS>(); } else wait_vm<PL>();
+      } else {
+        wait_vm<PL>();
+      }
+      lds_barrier();
+      frag_a(st(0), 0, a[0]);
+      frag_b(st(0), 0, b[0]);
+      // the fragments of hh 0..15 are in a[x], b[0]; the next tile's end up in a[1 - x], b[0]
+      auto body = [&](auto steady, auto parity, int t, unsigned char *H, unsigned char *L, unsigned char *H1, unsigned char *L1) {
+        constexpr bool kSteady = decltype(steady)::value;
+        constexpr int x = decltype(parity)::value, y = 1 - x;
+        const bool more = kSteady || t + 1 < nk, more2 = kSteady || t + 2 < nk;
+        // P0
+        frag_a(H, 1, a[y]);
+        frag_b(H, 1, b[1]);
+        if (NS == 4) {
+          mfma8_dma<BT, PL>(a[x], b[0], acc, [&](int i) { if (more) piece_l(i, L1); });
+          if (more) adv_l();
+        } else {
+          mfma8_dma<BT, IPS>(a[x], b[0], acc, [&](int i) { if (more) piece_h(i, H1); });
+          if (more) adv_h();
+        }
+        // P1
+#pragma unroll
+        for (int idx = 0; idx < 4; ++idx) mfma1<BT>(a[y], b[1], acc, idx);
+        if (more) wait_vm<NS == 4 ? IPS + PL : IPS>(); else wait_vm<0>();
+        lds_barrier();
+        frag_b(L, 1, b[0]);
+        if (NT == 3) frag_a(L, 1, a[x]);
+        else { frag_a(H, 0, a[x]); }
+#pragma unroll
+        for (int idx = 4; idx < 8; ++idx) mfma1<BT>(a[y], b[1], acc, idx);
+        if (NT == 3) {
+          // P2, P3, P4
+          mfma8<BT>(a[y], b[0], acc);
+          frag_a(H, 0, a[y]);
+          frag_b(L, 0, b[0]);
+          mfma8<BT>(a[x], b[1], acc);
+          frag_a(L, 0, a[x]);
+          frag_b(H, 0, b[1]);
+          mfma8<BT>(a[y], b[0], acc);
+        } else {
+          frag_b(L, 0, b[1]);
+          mfma8<BT>(a[y], b[0], acc);
+        }
+        if (more) wait_vm<NS == 4 ? PL : 0>(); else wait_vm<0>();
+        lds_barrier();
+        // P5 (P4 of two terms)
+        if (more) {
+          frag_a(H1, 0, a[y]);
+          frag_b(H1, 0, b[0]);
+        }
+        if (NS == 4) {
+          mfma8_dma<BT, IPS>(a[x], b[1], acc, [&](int i) { if (more2) piece_h(i, H); });
+          if (more2) adv_h();
+        } else {
+          mfma8_dma<BT, PL>(a[x], b[1], acc, [&](int i) { if (more) piece_l(i, H); });
+          if (more) adv_l();
+        }
+      };
+      constexpr int U = NS == 4 ? 2 : 6;            // tiles per round: stages and fragment roles come round
+      static_assert(NS == 3 || NS == 4, "stage ring");
+      int t = 0;
+      auto round = [&](auto steady) {
+        auto one = [&](auto s) {
+          constexpr int s0 = decltype(s)::value;
+          if (decltype(steady)::value || t + s0 < nk)
+            body(steady, std::integral_constant<int, s0 & 1>{}, t + s0, st(2 * s0 % NS), st((2 * s0 + 1) % NS),
+                 st((2 * s0 + 2) % NS), st((2 * s0 + 3) % NS));
+        };
+        one(std::integral_constant<int, 0>{});
+        one(std::integral_constant<int, 1>{});
+        if constexpr (U == 6) {
+          one(std::integral_constant<int, 2>{});
+          one(std::integral_constant<int, 3>{});
+          one(std::integral_constant<int, 4>{});
+          one(std::integral_constant<int, 5>{});
+        }
+      };
+      for (; t + U + 1 < nk; t += U) round(std::true_type{});
+      for (; t < nk; t += U) round(std::false_type{});
+    };
+    if (EPI == EPI_BX && nterms == 2) pairs(std::integral_constant<int, 2>{});
+    else pairs(std::integral_constant<int, 3>{});
   }
   __syncthreads();
 

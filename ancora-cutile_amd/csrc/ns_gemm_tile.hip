@@ -68,7 +68,8 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  const int K = p.K, nk = (K + TK - 1) / TK, total = anc_ns_terms(p, e) * nk;
+  const int K = p.K, nk = (K + TK - 1) / TK;
+  const int nterms = anc_ns_terms(p, e);
   // plain product only: K % 32 == 0, so with two panels per step the last step may hold one
   const bool half_tail = PLAINV && KP == 2 && (K & 63) != 0;
 
@@ -96,14 +97,8 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
   const int64_t baseA = (int64_t)e * p.strideA * 2 + (AT ? (int64_t)(tm * (TM / 32)) * psA : (int64_t)tm * TM * rpA);
   const int64_t baseB = (int64_t)e * p.strideB * 2 + (BT ? (int64_t)(tn * (TM / 32)) * psB : (int64_t)tn * TM * rpB);
   const int64_t advA = AT ? TK * rpA : KP * psA, advB = BT ? TK * rpB : KP * psB;
-  const char *Ab[3], *Bb[3];
-#pragma unroll
-  for (int t3 = 0; t3 < 3; ++t3) {
-    Ab[t3] = (const char *)p.A[t3] + baseA;
-    Bb[t3] = (const char *)p.B[t3] + baseB;
-  }
-  const char *curA = Ab[0], *curB = Bb[0];
-  int is_kt = 0, is_term = 0;
+  const char *curA = (const char *)p.A[0] + baseA, *curB = (const char *)p.B[0] + baseB;
+  int is_kt = 0;
   auto issue = [&](unsigned char *st) {
     const bool cut = half_tail && is_kt + 1 == nk;      // (the missing panel's pieces fetch the one that is there)
 #pragma unroll
@@ -112,20 +107,16 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
     for (int j = 0; j < 2; ++j) dma16(curB + offB[j] - (cut ? cutB[j] : 0) + voB, lds_addr(st + kHalf + (wave * 2 + j) * 1024));
     curA += advA;
     curB += advB;
-    if (++is_kt == nk) {
-      is_kt = 0;
-      ++is_term;
-      curA = is_term == 1 ? Ab[1] : Ab[2];
-      curB = is_term == 1 ? Bb[1] : Bb[2];
-    }
+    ++is_kt;
   };
 
   // ---- fragment addressing: tr = [block][k][64 B] by transposing reads, else [panel][row][64 B]
   const int l31 = lane & 31, hh = lane >> 5, g16 = lane >> 4, s16 = lane & 15;
   const int tr_lane = (8 * (g16 >> 1) + (s16 >> 2)) * 64 + 32 * (g16 & 1) + 8 * (s16 & 3);
-  auto frag = [&](auto tr, const unsigned char *half, int blk, int kk) -> bf16x8 {
+  // (rows_k: k rows of a block in the stage)
+  auto frag = [&](auto tr, const unsigned char *half, int blk, int kk, int rows_k) -> bf16x8 {
     if constexpr (decltype(tr)::value) {
-      const unsigned char *q = half + blk * (TK * 64) + kk * 16 * 64 + tr_lane;
+      const unsigned char *q = half + blk * (rows_k * 64) + kk * 16 * 64 + tr_lane;
       return anc_lds_tr_frag(q, q + 4 * 64);
     } else {
       return *(const bf16x8 *)(half + (kk >> 1) * (TM * 64) + (blk * 32 + l31) * 64 + ((((kk & 1) * 2 + hh) ^ ((l31 >> 2) & 3)) * 16));
@@ -142,37 +133,105 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[bi][bj][r] = 0.0f;
 
-  // ---- K loop. Step k lives in stage k % 4. At its top a wavefront waits for its own DMA of the step (two younger
-  // ones stay in flight), the workgroup meets, and the DMA of step k + 3 goes out into the stage everybody
-  // has just left.
+  auto mma = [&](const bf16x8 (&a)[WB], const bf16x8 (&b)[WB]) {
 #pragma unroll
-  for (int s0 = 0; s0 < kRing - 1; ++s0)
-    if (s0 < total) issue(lds + s0 * kStageBytes);
-  auto body = [&](int step, int s0) {
-    if (step + kRing - 1 <= total) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
-    lds_barrier();
-    if (step + kRing - 1 < total) issue(lds + ((s0 + kRing - 1) % kRing) * kStageBytes);
-    const unsigned char *st = lds + s0 * kStageBytes;
-    const bool cut = half_tail && step + 1 == total;
+    for (int bi = 0; bi < WB; ++bi)
 #pragma unroll
-    for (int kk = 0; kk < TK / 16; ++kk) {
-      if (PLAINV && kk >= 2 && cut) break;
-      bf16x8 a[WB], b[WB];
-#pragma unroll
-      for (int i = 0; i < WB; ++i) a[i] = frag(TrA{}, st, wm * WB + i, kk);
-#pragma unroll
-      for (int i = 0; i < WB; ++i) b[i] = frag(TrB{}, st + kHalf, wn * WB + i, kk);
-#pragma unroll
-      for (int bi = 0; bi < WB; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < WB; ++bj)      // operands exchanged: a lane ends with runs of 4 columns of one row
-          acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bj], a[bi], acc[bi][bj], 0, 0, 0);
-    }
+      for (int bj = 0; bj < WB; ++bj)      // operands exchanged: a lane ends with runs of 4 columns of one row
+        acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bj], a[bi], acc[bi][bj], 0, 0, 0);
   };
-  for (int step = 0; step < total; step += kRing) {
+
+  // ---- K loop, one term. Step k lives in stage k % 4. At its top a wavefront waits for its own DMA of the step (two
+  // younger ones stay in flight), the workgroup meets, and the DMA of step k + 3 goes out into the stage
+  // everybody has just left.
+  if (PLAINV || nterms == 1) {
 #pragma unroll
-    for (int s0 = 0; s0 < kRing; ++s0)
-      if (step + s0 < total) body(step + s0, s0);
+    for (int s0 = 0; s0 < kRing - 1; ++s0)
+      if (s0 < nk) issue(lds + s0 * kStageBytes);
+    auto body = [&](int step, int s0) {
+      if (step + kRing - 1 <= nk) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
+      lds_barrier();
+      if (step + kRing - 1 < nk) issue(lds + ((s0 + kRing - 1) % kRing) * kStageBytes);
+      const unsigned char *st = lds + s0 * kStageBytes;
+      const bool cut = half_tail && step + 1 == nk;
+#pragma unroll
+      for (int kk = 0; kk < TK / 16; ++kk) {
+        if (PLAINV && kk >= 2 && cut) break;
+        bf16x8 a[WB], b[WB];
+#pragma unroll
+        for (int i = 0; i < WB; ++i) a[i] = frag(TrA{}, st, wm * WB + i, kk, TK);
+#pragma unroll
+        for (int i = 0; i < WB; ++i) b[i] = frag(TrB{}, st + kHalf, wn * WB + i, kk, TK);
+        mma(a, b);
+      }
+    };
+    for (int step = 0; step < nk; step += kRing) {
+#pragma unroll
+      for (int s0 = 0; s0 < kRing; ++s0)
+        if (step + s0 < nk) body(step + s0, s0);
+    }
+  } else {
+    // ---- several terms: a step is one panel of 32 k of both halves of both operands, high stage then low stage.
+    constexpr int kPan = TM * 64, kPair = 4 * kPan, kPairs = kRing * kStageBytes / kPair;   // 4 (64) or 2 (128) steps in the ring
+    int64_t oA[WB], oB[WB];
+#pragma unroll
+    for (int j = 0; j < WB; ++j) {
+      const int q = wave * WB + j;
+      oA[j] = (AT ? (q >> 1) * psA + (q & 1) * 16 * rpA : q * 16 * rpA) + voA;
+      oB[j] = (BT ? (q >> 1) * psB + (q & 1) * 16 * rpB : q * 16 * rpB) + voB;
+    }
+    const char *pAl = (const char *)p.A[1] + baseA, *pBl = (const char *)p.B[1] + baseB;
+    const int64_t adA = AT ? 32 * rpA : psA, adB = BT ? 32 * rpB : psB;
+    auto terms = [&](auto nt) {
+      constexpr int NT = decltype(nt)::value, kIpp = NT == 3 ? 4 * WB : 3 * WB;   // DMA instructions per wavefront and step
+      auto issue_pair = [&](unsigned char *st) {
+#pragma unroll
+        for (int j = 0; j < WB; ++j) {
+          const int at = (wave * WB + j) * 1024;
+          dma16(curA + oA[j], lds_addr(st + at));
+          dma16(curB + oB[j], lds_addr(st + kPan + at));
+          if (NT == 3) dma16(pAl + oA[j], lds_addr(st + 2 * kPan + at));
+          dma16(pBl + oB[j], lds_addr(st + 3 * kPan + at));
+        }
+        curA += adA; curB += adB; pAl += adA; pBl += adB;
+      };
+      const int np = K / 32;
+#pragma unroll
+      for (int s0 = 0; s0 < kPairs - 1; ++s0)
+        if (s0 < np) issue_pair(lds + s0 * kPair);
+      for (int step = 0; step < np; step += kPairs) {
+#pragma unroll
+        for (int s0 = 0; s0 < kPairs; ++s0) {
+          if (step + s0 >= np) break;
+          if (step + s0 + kPairs - 1 <= np) wait_vm<(kPairs - 2) * kIpp>(); else wait_vm<0>();
+          lds_barrier();
+          if (step + s0 + kPairs - 1 < np) issue_pair(lds + ((s0 + kPairs - 1) % kPairs) * kPair);
+          const unsigned char *st = lds + s0 * kPair;
+          bf16x8 ah[2][WB], bh[2][WB], al[WB], bl[WB];
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+            for (int i = 0; i < WB; ++i) ah[kk][i] = frag(TrA{}, st, wm * WB + i, kk, 32);
+#pragma unroll
+            for (int i = 0; i < WB; ++i) bh[kk][i] = frag(TrB{}, st + kPan, wn * WB + i, kk, 32);
+            mma(ah[kk], bh[kk]);
+          }
+#pragma unroll
+          for (int kk = 1; kk >= 0; --kk) {
+#pragma unroll
+            for (int i = 0; i < WB; ++i) bl[i] = frag(TrB{}, st + 3 * kPan, wn * WB + i, kk, 32);
+            mma(ah[kk], bl);
+            if (NT == 3) {
+#pragma unroll
+              for (int i = 0; i < WB; ++i) al[i] = frag(TrA{}, st + 2 * kPan, wm * WB + i, kk, 32);
+              mma(al, bh[kk]);
+            }
+          }
+        }
+      }
+    };
+    if (EPI == EPI_BX && nterms == 2) terms(std::integral_constant<int, 2>{});
+    else terms(std::integral_constant<int, 3>{});
   }
   __syncthreads();
 
