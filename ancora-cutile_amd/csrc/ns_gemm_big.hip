@@ -834,9 +834,10 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
             if (VAR == VAR_UPDATE_T) { pv[pz].x = __uint_as_float(ho.x); pv[pz].y = __uint_as_float(ho.y); }
           }
           if (VAR == VAR_UPDATE_T && W16t != nullptr) {
-            // The transposed copy: the slab's bf16 values cross the buffer, which O has left, once more. A lane then
-            // holds 32 consecutive rows of one column of W, 64 contiguous bytes of the copy. (These stores
-            // are not in the counts of the waits above, which makes the waits longer, never shorter.)
+            // The transposed copy: the slab's bf16 values cross the buffer, which O has left, once more and leave as
+            // rows of 64 (128 for a tall weight) bytes, by ordinary stores so that L2 joins a row's pieces
+            // of neighbouring slabs. (They are not in the counts of the waits above, which makes the waits
+            // longer, never shorter.)
             lds_wave_sync();
             const int pitch = wtr ? 40 : 72;
             uint16_t *sh = (uint16_t *)b;
@@ -847,15 +848,15 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
               *(anc_u32x2 *)q = anc_u32x2{__float_as_uint(pv[pz].x), __float_as_uint(pv[pz].y)};
             }
             lds_wave_sync();
-            const int wc = wtr ? lane & 31 : lane, wr = wtr ? (lane >> 5) * 32 : 0;
-            uint16_t *o = W16t + (int64_t)((wtr ? gi0 : gj0w) + wc) * wK + (wtr ? gj0w : gi0) + wr;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
+              const int wc = wtr ? 8 * i + (lane >> 3) : 16 * i + (lane >> 2), wr = wtr ? (lane & 7) * 8 : (lane & 3) * 8;
               uint32_t w[4];
 #pragma unroll
               for (int k4 = 0; k4 < 4; ++k4)
-                w[k4] = (uint32_t)sh[(wr + 8 * i + 2 * k4) * pitch + wc] | ((uint32_t)sh[(wr + 8 * i + 2 * k4 + 1) * pitch + wc] << 16);
-              epi_st((anc_u32x4 *)(o + 8 * i), anc_u32x4{w[0], w[1], w[2], w[3]});
+                w[k4] = (uint32_t)sh[(wr + 2 * k4) * pitch + wc] | ((uint32_t)sh[(wr + 2 * k4 + 1) * pitch + wc] << 16);
+              uint16_t *o = W16t + (int64_t)((wtr ? gi0 : gj0w) + wc) * wK + (wtr ? gj0w : gi0) + wr;
+              *(anc_u32x4 *)o = anc_u32x4{w[0], w[1], w[2], w[3]};
             }
           }
         }
