@@ -68,6 +68,11 @@ class MuonDesc(C.Structure):
                 ("seed", u32), ("tile0", i64), ("p16t", u64)]
 
 
+class QuantDesc(C.Structure):
+    """anc_quant_desc_t: one weight of the multi-weight re-quantisation."""
+    _fields_ = [("w", u64), ("fp8", u64), ("scale", u64), ("tile0", i64), ("K", i32), ("N", i32)]
+
+
 class NsProblem(C.Structure):
     """anc_ns_problem_t: one batch of the multi-batch chain entry."""
     _fields_ = [("Uh", u64), ("Ul", u64), ("fro_partials", u64), ("X32_out", u64), ("workspace", u64),
@@ -134,6 +139,8 @@ _PROTOS = {
                                      u64]),
     "anc_transpose_bf16": (None, [u64, u64, i64, i64, i64, u64]),
     "anc_quant_mxfp8_w": (None, [u64, u64, u64, i64, i64, i64, C.c_int, u64]),
+    "anc_quant_mxfp8_num_tiles": (i64, [i64, i64, i64]),
+    "anc_quant_mxfp8_w_multi": (None, [u64, i32, i64, C.c_int, u64]),
     "anc_gemm_dw_workspace_bytes": (i64, [i64, i64, i64]),
     "anc_gemm_dw_multi": (None, [C.POINTER(DwProblem), i32, u64]),
     "anc_gemm_dw_info": (None, [i64, i64, i64, C.POINTER(C.c_double), C.POINTER(i32)]),

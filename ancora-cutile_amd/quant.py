@@ -5,14 +5,14 @@ Mirror of the device side of ancora/kernels/quant.py: `_quant_mxfp8_w` (:60-73) 
 QWN = 128 (column granularity), and of the dirty-flag protocol around them: the step marks the
 fp8 copies of the bf16 weights stale (ancora/model/resident_train.py:354-357) and the next
 forward re-quantises every weight once (:190-199). `Mxfp8WeightCache` holds the fp8 bytes and
-E8M0 scale bytes per weight and does exactly that; the arithmetic runs in one HIP kernel per
-weight (`anc_quant_mxfp8_w`), all-integer on the bf16 bit patterns.
+E8M0 scale bytes per weight and does exactly that; the arithmetic runs in one HIP kernel over
+all weights (`anc_quant_mxfp8_w_multi`), all-integer on the bf16 bit patterns.
 """
 import numpy as np
 
 from . import _lib
-from ._lib import api
-from .devbuf import DevBuf
+from ._lib import api, QuantDesc
+from .devbuf import DevBuf, upload_table
 
 B = 32          # MXFP8 scale block (ancora/kernels/quant.py:19)
 QWN = 128       # column granularity of the weight kernels (quant.py:22)
@@ -33,7 +33,7 @@ class Mxfp8WeightCache:
 
     weights: {name: dict(p16=DevBuf of bf16 bits, K=int, N=int, E=int (optional, stacked
     experts))}. `mark_dirty()` is what an optimizer step does; `refresh(si)` is what the forward
-    does before it reads the fp8 weights: one kernel per weight if anything is stale."""
+    does before it reads the fp8 weights: one kernel over all of them if anything is stale."""
 
     def __init__(self, weights, col_major=False):
         _lib.init()
@@ -48,6 +48,7 @@ class Mxfp8WeightCache:
             self.w[name] = dict(p16=s["p16"], E=E, K=K, N=N, fp8=DevBuf.zeros(shp8, np.uint8),
                                 scale=DevBuf.zeros(shps, np.uint8))
         self.dirty = True
+        self._table = self._key = None
 
     def mark_dirty(self):
         self.dirty = True
@@ -56,9 +57,21 @@ class Mxfp8WeightCache:
         """Re-quantise every weight if a step has run since the last call. Returns True if it did."""
         if not self.dirty:
             return False
-        for s in self.w.values():
-            quant_mxfp8_w(s["p16"], s["fp8"], s["scale"], s["K"], s["N"], si, E=s["E"],
-                          col_major=self.col_major)
+        if not self.w:
+            self.dirty = False
+            return True
+        key = [s["p16"] for s in self.w.values()]
+        if key != self._key:                       # the descriptor table: once, unless a weight is exchanged
+            if self._table is not None:
+                self._table.free()
+            descs, tiles = [], 0
+            for s in self.w.values():
+                if s["p16"].ptr % 16:
+                    raise ValueError("Mxfp8WeightCache: weights must be 16-byte aligned")
+                descs.append(QuantDesc(s["p16"].ptr, s["fp8"].ptr, s["scale"].ptr, tiles, s["K"], s["N"]))
+                tiles += api.anc_quant_mxfp8_num_tiles(s["E"], s["K"], s["N"])
+            self._table, self._tiles, self._key = upload_table(descs), tiles, key
+        api.anc_quant_mxfp8_w_multi(self._table.ptr, len(self.w), self._tiles, int(self.col_major), int(si))
         self.dirty = False
         return True
 
@@ -75,4 +88,7 @@ class Mxfp8WeightCache:
         for s in self.w.values():
             s["fp8"].free()
             s["scale"].free()
+        if self._table is not None:
+            self._table.free()
+            self._table = self._key = None
         self.w = {}

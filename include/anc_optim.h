@@ -416,6 +416,18 @@ int anc_gemm_dw_info(int64_t T, int64_t K, int64_t N, double *flops, int32_t *se
 int anc_quant_mxfp8_w(uint64_t w_bf16, uint64_t fp8_out, uint64_t scale_out, int64_t E, int64_t K,
                       int64_t N, int col_major, uint64_t stream);
 
+/* The same for every weight of a device table in one launch: what a refresh after a step is. tile0 counts
+ * the wavefront tiles of the weights before (anc_quant_mxfp8_num_tiles(E, K, N) each), total_tiles all of
+ * them. Alignment and dims as above, checked by whoever builds the table. */
+typedef struct {
+  uint64_t w, fp8, scale;     /* as w_bf16, fp8_out, scale_out above */
+  int64_t  tile0;
+  int32_t  K, N;
+} anc_quant_desc_t;
+int64_t anc_quant_mxfp8_num_tiles(int64_t E, int64_t K, int64_t N);
+int anc_quant_mxfp8_w_multi(uint64_t desc_table, int32_t n_weights, int64_t total_tiles, int col_major,
+                            uint64_t stream);
+
 /* --------------------------------------------------------- Newton-Schulz ---
  * Replaces the chains `newton_schulz_resident` / `newton_schulz_resident_e`
  * (ancora/kernels/muon_ns.py:245-283, 430-468) and the kernels they launch

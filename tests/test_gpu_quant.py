@@ -91,6 +91,26 @@ def test_cache_refreshes_once_per_step(gpu):
     cache.free(); p16.free()
 
 
+@pytest.mark.parametrize("cm", [False, True])
+def test_cache_of_many_weights_is_one_launch(gpu, cm):
+    """Weights of different sizes and a stacked one behind one descriptor table: the bytes each gets alone."""
+    from ancora_cutile_amd import DevBuf, Mxfp8WeightCache
+    rng = np.random.default_rng(4)
+    shapes = {"a": (1, 128, 128), "b": (1, 384, 256), "c": (3, 128, 384), "d": (1, 640, 128), "e": (2, 256, 128)}
+    wb = {n: bf16_rne_bits((0.1 * rng.standard_normal(sh)).astype(np.float32)).reshape(sh) for n, sh in shapes.items()}
+    bufs = {n: DevBuf(w.reshape(-1, w.shape[2])) for n, w in wb.items()}
+    cache = Mxfp8WeightCache({n: dict(p16=bufs[n], E=sh[0], K=sh[1], N=sh[2]) for n, sh in shapes.items()}, col_major=cm)
+    assert cache.refresh(0)
+    for n, (E, K, N) in shapes.items():
+        f, s = cache.fp8(n).to_numpy().reshape(E, -1), cache.scale(n).to_numpy().reshape(E, -1)
+        for e in range(E):
+            wf, ws = ref_quant(wb[n][e], col_major=cm)
+            assert np.array_equal(f[e], wf.reshape(-1)) and np.array_equal(s[e], ws.reshape(-1)), (n, e)
+    cache.free()
+    for b in bufs.values():
+        b.free()
+
+
 def test_shape_checks(gpu):
     from ancora_cutile_amd import DevBuf, _lib
     from ancora_cutile_amd._lib import api
