@@ -147,6 +147,9 @@ _PROTOS = {
     "anc_ns_workspace_bytes": (i64, [i64, i64, i64, C.c_int]),
     "anc_ns_batched": (None, [u64, i64, i64, i64, C.c_int, C.POINTER(f32), f32, C.c_int, u64, i64,
                               u64]),
+    "anc_ns_batched_bf16": (None, [u64, i64, i64, i64, C.c_int, C.POINTER(f32), f32, C.c_int, u64, i64, u64]),
+    "anc_muon_resident_step": (None, [u64, u64, C.c_int, u64, u64, u64, i64, i64, f32, C.c_int, f32, C.c_int,
+                                      C.POINTER(f32), f32, C.c_int, u64, i64, u64, u64]),
     "anc_ns_batched_pair": (None, [u64, u64, u64, i64, u64, i64, i64, i64, C.c_int, C.POINTER(f32), f32,
                                    C.c_int, u64, i64, u64]),
     "anc_ns_batched_pair_multi": (None, [C.POINTER(NsProblem), i32, C.c_int, C.POINTER(f32), f32, C.c_int,

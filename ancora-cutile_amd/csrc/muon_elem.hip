@@ -9,7 +9,7 @@
 // orientation is walked flat, 16 bytes per lane per fp32 access, exactly like AdamW.
 // A tall weight (K > N) crosses a 64x64 tile through LDS so that both the (K,N) side
 // and the transposed (N,K) side are accessed in 256-byte (fp32) row segments.
-#include "common.h"
+#include "ns_common.h"
 
 namespace {
 
@@ -345,6 +345,24 @@ k_mom_multi_pair(const anc_muon_desc_t *__restrict__ table, int n_weights, float
   }
 }
 
+// The same for one weight whose descriptor comes by value: no table to build and upload for a layer that steps
+// itself. Leaves the descriptor in device memory for the chain's last product.
+__global__ void __launch_bounds__(kThreads)
+k_mom_pair_one(anc_muon_desc_t d, float mom, int nesterov, uint64_t lo, double *__restrict__ fro,
+               anc_muon_desc_t *__restrict__ desc_out, const anc_step_ctl_t *__restrict__ ctl) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *desc_out = d;
+  float clip;
+  if (!load_ctl(ctl, clip)) return;
+  MomArgs a{(float *)d.buf, (const void *)d.g, (void *)d.u, d.K, d.N, (void *)lo, fro + blockIdx.x};
+  if (d.transpose) {
+    if (d.g_dtype == ANC_BF16) mom_tile_t<ANC_BF16, kPair>(a, (int64_t)blockIdx.x, mom, nesterov, clip);
+    else                       mom_tile_t<ANC_F32, kPair>(a, (int64_t)blockIdx.x, mom, nesterov, clip);
+  } else {
+    if (d.g_dtype == ANC_BF16) mom_flat<ANC_BF16, kPair>(a, (int64_t)blockIdx.x, mom, nesterov, clip);
+    else                       mom_flat<ANC_F32, kPair>(a, (int64_t)blockIdx.x, mom, nesterov, clip);
+  }
+}
+
 struct LrScales { float v[ANC_MUON_MAX_SCALES]; };
 
 template <int OD, int SR>
@@ -419,6 +437,16 @@ int check_kn(int64_t K, int64_t N, const char *who) {
 }
 
 }  // namespace
+
+int anc_launch_momentum_pair_one(const anc_muon_desc_t &d, float mom, int nesterov, uint64_t lo, double *fro,
+                                 anc_muon_desc_t *desc_out, const anc_step_ctl_t *ctl, hipStream_t s) {
+  if (int rc = check_kn(d.K, d.N, "anc_muon_resident_step")) return rc;
+  AncProfScope prof(ANC_PROF_MUON_MOM, s);
+  hipLaunchKernelGGL(k_mom_pair_one, dim3((unsigned)((int64_t)d.K * d.N / kBlockElems)), dim3(kThreads), 0, s, d, mom, nesterov, lo,
+                     fro, desc_out, ctl);
+  ANC_LAUNCH_CHECK();
+  return ANC_OK;
+}
 
 extern "C" int anc_muon_momentum(uint64_t buf, uint64_t g, uint64_t u, int64_t K, int64_t N,
                                  float mom, int nesterov, int transpose_out, int g_dtype,

@@ -148,10 +148,11 @@ __global__ void __launch_bounds__(kGemmThreads, 2) k_ns_gemm_f32(NsGemmF32 p) {
 }
 
 // ------------------------------------------------------------------ Frobenius prologue
+template <int GD, typename T>
 __global__ void __launch_bounds__(kThreads)
-k_fro_partials(const float *__restrict__ X, int64_t mn, int nchunks, double *__restrict__ partials) {
+k_fro_partials(const T *__restrict__ X, int64_t mn, int nchunks, double *__restrict__ partials) {
   const int64_t e = (int64_t)blockIdx.x / nchunks, c = (int64_t)blockIdx.x % nchunks;
-  chunk_partial<ANC_F32>((const void *)(X + e * mn), mn, c, partials + blockIdx.x);
+  chunk_partial<GD>((const void *)(X + e * mn), mn, c, partials + blockIdx.x);
 }
 
 // One block per matrix: lane t adds partials t, t+256, ... in order; butterfly; 4 wavefronts in order.
@@ -185,7 +186,8 @@ struct NsPrologue {
   int nchunks[kMaxGroups];
   const double *partials[kMaxGroups];
   float *recip[kMaxGroups];
-  uint16_t *Uh[kMaxGroups], *Ul[kMaxGroups];
+  uint16_t *Uh[kMaxGroups], *Ul[kMaxGroups];       // Ul null: a bf16 input without a low half,
+  uint32_t *zero16[kMaxGroups];                    // whose substitute this kernel clears
   int64_t mn[kMaxGroups];
 };
 __global__ void __launch_bounds__(kThreads) k_pair_prologue(NsPrologue a, float eps) {
@@ -199,11 +201,13 @@ __global__ void __launch_bounds__(kThreads) k_pair_prologue(NsPrologue a, float 
     r = ldexpf(r, -k);
   }
   if (threadIdx.x == 0) a.recip[q][e] = r;
+  if (a.Ul[q] == nullptr && e == 0 && threadIdx.x < 4) a.zero16[q][threadIdx.x] = 0u;
   if (sc == 1.0f) return;            // (uniform over the block)
   const int64_t mn = a.mn[q];
   for (int64_t o = (int64_t)threadIdx.x * 8; o < mn; o += (int64_t)kThreads * 8) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      if (h && a.Ul[q] == nullptr) break;
       uint16_t *p = (h ? a.Ul[q] : a.Uh[q]) + (int64_t)e * mn + o;
       anc_u32x4 w = *(const anc_u32x4 *)p;
       uint32_t u[4] = {w.x, w.y, w.z, w.w};
@@ -615,6 +619,8 @@ struct Plan {
   uint16_t *Fl, *Bl;
   double *partials;
   float *recip;
+  uint32_t *zero16;      // 16 zero bytes: the low half of a bf16 input
+  anc_muon_desc_t *desc; // one weight's descriptor (anc_muon_resident_step)
   double *condpart;      // (E, kCondParts) partial sums of the conditioning proxy, bf16 modes
   double *cond;          // (E) the proxy
   double *colpart;       // (E, col_parts, 2) column statistic, plans with a wide gate
@@ -635,7 +641,9 @@ Plan make_plan(uint64_t base, int64_t E, int64_t M, int64_t N, int mode, int ste
   pl.nchunks = (int)((M * N + ANC_GN_CHUNK - 1) / ANC_GN_CHUNK);
   pl.sp = split_plan(M, N, mode, steps);
   pl.split = pl.sp.x_from < steps;
-  pl.partials = c.take<double>(E * pl.nchunks);
+  pl.partials = c.take<double>(E * ((M * N + 4095) / 4096));   // (the momentum kernel's blocks; chunks are twice as long)
+  pl.zero16 = c.take<uint32_t>(4);
+  pl.desc = c.take<anc_muon_desc_t>(1);
   pl.recip = c.take<float>(E);
   if (mode == ANC_NS_FP32) {
     pl.Af = c.take<float>(E * M * M);
@@ -692,6 +700,7 @@ void add_prologue(NsPrologue &a, const Plan &pl, uint64_t Uh, uint64_t Ul, uint6
   a.recip[q] = pl.recip;
   a.Uh[q] = (uint16_t *)Uh;
   a.Ul[q] = (uint16_t *)Ul;
+  a.zero16[q] = pl.zero16;
   a.mn[q] = mn;
 }
 int launch_prologue(const NsPrologue &a, float eps, hipStream_t s) {
@@ -711,6 +720,7 @@ struct ChainProb {
   int nxt;                     // which pair of the plan receives the first step's output
   const float *scale0;         // per-matrix factor the first step applies to its input, or null
   float *X32;                  // fp32 result (may overlay the input pair when steps >= 2)
+  uint16_t *X16;               // or bf16 result (may overlay inH when steps >= 2)
   int64_t E, M, N;
   const anc_muon_desc_t *upd;  // or: the weights (E entries) the last step updates in its epilogue
 };
@@ -834,7 +844,10 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       gx[q].Xh = curH[q]; gx[q].Xl = curL[q];
       gx[q].Yh = last ? nullptr : pl.Xh[nxt[q]];
       gx[q].Yl = last ? nullptr : pl.Xl[nxt[q]];
+      gx[q].lo_zero = (k == 0 && cp[q].inL == nullptr) ? 1 : 0;
+      if (gx[q].lo_zero) gx[q].Xl = (const uint16_t *)pl.zero16;
       gx[q].X32 = (last && cp[q].upd == nullptr) ? cp[q].X32 : nullptr;
+      gx[q].X16 = (last && cp[q].upd == nullptr) ? cp[q].X16 : nullptr;
       gx[q].upd = last ? cp[q].upd : nullptr;
       // The next iterate's low half is one byte for the matrices whose low half no product of the
       // next iteration multiplies: every matrix outside the wide gate if that iteration has no gate,
@@ -908,6 +921,10 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
 }
 
 }  // namespace
+
+static int pair_multi_impl(const char *who, const anc_ns_problem_t *probs, int32_t n_probs,
+                           const uint64_t *desc_tables, const NsUpdate *upd, int steps, const float *coef,
+                           float eps, int mode, uint64_t stream);
 
 int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int force, hipStream_t s,
                       const NsUpdate *upd) {
@@ -1089,7 +1106,7 @@ extern "C" int anc_ns_batched(uint64_t X, int64_t E, int64_t M, int64_t N, int s
   const int64_t mn = M * N;
 
   // ---- X /= ||X||_F + eps
-  { AncProfScope prof(ANC_PROF_NS_FRO, s); hipLaunchKernelGGL(k_fro_partials, dim3((unsigned)(E * pl.nchunks)), dim3(kThreads), 0, s, X32, mn,
+  { AncProfScope prof(ANC_PROF_NS_FRO, s); hipLaunchKernelGGL((k_fro_partials<ANC_F32, float>), dim3((unsigned)(E * pl.nchunks)), dim3(kThreads), 0, s, X32, mn,
                      pl.nchunks, pl.partials); }
   ANC_LAUNCH_CHECK();
   { AncProfScope prof(ANC_PROF_NS_FRO, s); hipLaunchKernelGGL(k_fro_finalize, dim3((unsigned)E), dim3(kThreads), 0, s, pl.partials, pl.nchunks,
@@ -1138,8 +1155,73 @@ extern "C" int anc_ns_batched(uint64_t X, int64_t E, int64_t M, int64_t N, int s
   { AncProfScope prof(ANC_PROF_NS_PREP, s); hipLaunchKernelGGL(k_ns_prep, dim3(prep_grid), dim3(kThreads), 0, s, X32, pl.recip, mn, total8,
                      pl.Xh[0], pl.Xl[0]); }
   ANC_LAUNCH_CHECK();
-  ChainProb cp{pl, pl.Xh[0], pl.Xl[0], 1, nullptr, X32, E, M, N, nullptr};
+  ChainProb cp{pl, pl.Xh[0], pl.Xl[0], 1, nullptr, X32, nullptr, E, M, N, nullptr};
   return run_bf16_chain(&cp, 1, steps, coef, flags, s);
+}
+
+// The chain on bf16 matrices in place. The input is its own high half, exactly; there is no low half, no
+// widened copy, no scaling pass (the first step's epilogues carry the scale) and the last epilogue rounds. Against
+// widen + anc_ns_batched + round, 24 x (1024, 2048) drop 200 us of conversion passes. A plan that splits
+// the first iteration (M < 256, ANC_NS_BF16_X3) multiplies residuals there, so it gets a cleared low half.
+extern "C" int anc_ns_batched_bf16(uint64_t X, int64_t E, int64_t M, int64_t N, int steps, const float *coef,
+                                   float eps, int mode, uint64_t workspace, int64_t workspace_bytes,
+                                   uint64_t stream) {
+  const int flags = mode & kTileFlags;
+  mode &= ~kTileFlags;
+  if (int rc = check_shape(E, M, N, mode, "anc_ns_batched_bf16")) return rc;
+  ANC_REQUIRE(mode != ANC_NS_FP32, "anc_ns_batched_bf16: bf16 modes only");
+  ANC_REQUIRE(X != 0 && (X & 15) == 0, "anc_ns_batched_bf16: X must be a 16-byte aligned device pointer");
+  ANC_REQUIRE(steps >= 2 && steps <= 64 && coef != nullptr, "anc_ns_batched_bf16: steps=%d: 2..64 (the result overlays the input)",
+              steps);
+  ANC_REQUIRE(workspace != 0 && (workspace & 255) == 0, "anc_ns_batched_bf16: workspace must be 256-byte aligned");
+  const Plan pl = make_plan(workspace, E, M, N, mode, steps);
+  ANC_REQUIRE(workspace_bytes >= pl.bytes, "anc_ns_batched_bf16: workspace holds %lld bytes, %lld needed",
+              (long long)workspace_bytes, (long long)pl.bytes);
+  hipStream_t s = anc_stream(stream);
+  const uint16_t *lo = nullptr;
+  if (pl.sp.x_from == 0) {
+    // pair 1 is written by the second step at the earliest: its low half serves as the zeros
+    lo = pl.Xl[1];
+    if (int rc = anc_fill_u32((uint64_t)lo, 0u, E * M * N / 2, stream)) return rc;
+  }
+  { AncProfScope prof(ANC_PROF_NS_FRO, s); hipLaunchKernelGGL((k_fro_partials<ANC_BF16, uint16_t>), dim3((unsigned)(E * pl.nchunks)),
+                     dim3(kThreads), 0, s, (const uint16_t *)X, M * N, pl.nchunks, pl.partials); }
+  ANC_LAUNCH_CHECK();
+  NsPrologue pro{};
+  add_prologue(pro, pl, X, (uint64_t)lo, (uint64_t)pl.partials, pl.nchunks, E, M * N);
+  if (int rc = launch_prologue(pro, eps, s)) return rc;
+  ChainProb cp{pl, (const uint16_t *)X, lo, 0, pl.recip, nullptr, (uint16_t *)X, E, M, N, nullptr};
+  return run_bf16_chain(&cp, 1, steps, coef, flags, s);
+}
+
+// One weight's whole Muon step: momentum, chain, update.
+extern "C" int anc_muon_resident_step(uint64_t buf, uint64_t g, int g_dtype, uint64_t p32, uint64_t p16, uint64_t u,
+                                      int64_t K, int64_t N, float mom, int nesterov, float lr_scale, int steps,
+                                      const float *coef, float eps, int mode, uint64_t workspace,
+                                      int64_t workspace_bytes, uint64_t ctl, uint64_t stream) {
+  const int64_t M = K < N ? K : N, Nn = K < N ? N : K;
+  if (int rc = check_shape(1, M, Nn, mode & ~kTileFlags, "anc_muon_resident_step")) return rc;
+  ANC_REQUIRE(buf && g && p32 && u && ((buf | g | p32 | u) & 15) == 0 && (p16 & 7) == 0,
+              "anc_muon_resident_step: null or misaligned pointer");
+  ANC_REQUIRE(g_dtype == ANC_F32 || g_dtype == ANC_BF16, "anc_muon_resident_step: bad dtype");
+  ANC_REQUIRE(workspace != 0 && (workspace & 255) == 0, "anc_muon_resident_step: workspace must be 256-byte aligned");
+  const Plan pl = make_plan(workspace, 1, M, Nn, mode & ~kTileFlags, steps);
+  ANC_REQUIRE(workspace_bytes >= pl.bytes, "anc_muon_resident_step: workspace holds %lld bytes, %lld needed",
+              (long long)workspace_bytes, (long long)pl.bytes);
+  anc_muon_desc_t d{};
+  d.buf = buf; d.g = g; d.p32 = p32; d.p16 = p16; d.u = u;
+  d.K = (int32_t)K; d.N = (int32_t)N; d.transpose = K > N ? 1 : 0; d.g_dtype = g_dtype;
+  if (int rc = anc_launch_momentum_pair_one(d, mom, nesterov, u + (uint64_t)(M * Nn * 2), pl.partials, pl.desc,
+                                            (const anc_step_ctl_t *)ctl, anc_stream(stream))) return rc;
+  anc_ns_problem_t prob{};
+  prob.Uh = u; prob.Ul = u + (uint64_t)(M * Nn * 2); prob.fro_partials = (uint64_t)pl.partials;
+  prob.workspace = workspace; prob.n_partials = M * Nn / 4096; prob.E = 1; prob.M = M; prob.N = Nn;
+  prob.workspace_bytes = workspace_bytes;
+  const uint64_t table = (uint64_t)pl.desc;
+  NsUpdate up{};
+  up.lr[0] = lr_scale;
+  up.ctl = (const anc_step_ctl_t *)ctl;
+  return pair_multi_impl("anc_muon_resident_step", &prob, 1, &table, &up, steps, coef, eps, mode, stream);
 }
 
 // The chain on an unnormalised bf16 pair (what anc_muon_momentum_multi_pair leaves) with the
@@ -1167,7 +1249,7 @@ extern "C" int anc_ns_batched_pair(uint64_t Uh, uint64_t Ul, uint64_t fro_partia
   NsPrologue pro{};
   add_prologue(pro, pl, Uh, Ul, fro_partials, n_partials, E, M * N);
   if (int rc = launch_prologue(pro, eps, s)) return rc;
-  ChainProb cp{pl, (const uint16_t *)Uh, (const uint16_t *)Ul, 0, pl.recip, (float *)X32_out, E, M, N, nullptr};
+  ChainProb cp{pl, (const uint16_t *)Uh, (const uint16_t *)Ul, 0, pl.recip, (float *)X32_out, nullptr, E, M, N, nullptr};
   return run_bf16_chain(&cp, 1, steps, coef, flags, s);
 }
 
@@ -1211,7 +1293,7 @@ static int pair_multi_impl(const char *who, const anc_ns_problem_t *probs, int32
     ANC_REQUIRE(b.workspace_bytes >= pl.bytes, "%s: workspace holds %lld bytes, %lld needed", who,
                 (long long)b.workspace_bytes, (long long)pl.bytes);
     add_prologue(pro, pl, b.Uh, b.Ul, b.fro_partials, b.n_partials, b.E, b.M * b.N);
-    cp[q] = ChainProb{pl, (const uint16_t *)b.Uh, (const uint16_t *)b.Ul, 0, pl.recip, (float *)b.X32_out, b.E, b.M, b.N,
+    cp[q] = ChainProb{pl, (const uint16_t *)b.Uh, (const uint16_t *)b.Ul, 0, pl.recip, (float *)b.X32_out, nullptr, b.E, b.M, b.N,
                       desc_tables ? (const anc_muon_desc_t *)desc_tables[order[q]] : nullptr};
   }
   if (int rc = launch_prologue(pro, eps, s)) return rc;

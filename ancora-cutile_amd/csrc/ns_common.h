@@ -83,8 +83,11 @@ struct NsGemm {
   uint16_t *Bh;              // (E,M,M) bf16 off-diag B   BMAT out
   float *dB;                 // (E,M)   diag B            BMAT out, BX in
   const uint16_t *Xh, *Xl;   // (E,M,N) current iterate as a bf16 pair, X = Xh + Xl   BX in
+  int lo_zero;               // the input has no low half (a bf16 matrix): Xl is one zeroed 16-byte piece that every
+                             // read of a low half goes to
   uint16_t *Yh, *Yl;         // (E,M,N) next iterate as a bf16 pair   BX out, null on the last step
   float *X32;                // (E,M,N) fp32 result                   BX out on the last step, else null
+  uint16_t *X16;             // (E,M,N) the result rounded to bf16, instead of X32
   const anc_muon_desc_t *upd;  // BX, last step only: if set, matrix e is the Newton-Schulz result of the
                              // weight upd[e] and the epilogue applies W -= lr*O to it (p32, p16) instead
                              // of writing X32
@@ -260,6 +263,10 @@ int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, h
 // 64x64 (small) or 128x128 tiles (ns_gemm_tile.hip; M and N multiples of 128); `plain`: the bare product.
 int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool small, bool by_rows,
                            const NsUpdate *upd, bool plain);
-// Bare fp32 products C[e] = A[e] B[e] on the same K loop (ns_gemm_big.hip); a_transposed: A is
+// Bare fp32 products C[e] = A[e] B[e] on the same K loops; a_transposed: A is
 // given as (K, M) row-major with row pitch ldA (and strideA between matrices), C = A^T B.
 int anc_ns_gemm_big_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool a_transposed = false);
+// Momentum of one weight as a bf16 pair (muon_elem.hip): high halves to d.u, low halves to `lo`, a sum of u*u per 4096
+// elements to `fro`; leaves `d` in device memory at `desc_out` for the chain's last product.
+int anc_launch_momentum_pair_one(const anc_muon_desc_t &d, float mom, int nesterov, uint64_t lo, double *fro,
+                                 anc_muon_desc_t *desc_out, const anc_step_ctl_t *ctl, hipStream_t s);

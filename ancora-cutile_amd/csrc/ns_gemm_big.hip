@@ -550,6 +550,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   // LDS chunk l holds row l/2, half (l%2) ^ ((l/16)%2), which halves the bank conflicts of the
   // 4-byte accesses below (rows 8 apart would otherwise meet in one bank four at a time).
   const int l8_src = (lane >> 1) * 32 + (((lane & 1) ^ ((lane >> 4) & 1)) * 16);
+  const int64_t lo_at = p.lo_zero ? 0 : -1;                 // (no low half: every read goes to one zeroed piece)
   auto fetch_in = [&](int bi) {
     const int64_t ub = x_pan ? mn * 2 + (int64_t)(gj0w / 32) * panel + (int64_t)(gi0w + bi * 32) * 64
                              : (mn + (int64_t)(gi0w + bi * 32) * N + gj0w) * 2;
@@ -559,7 +560,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       const int64_t ro = (int64_t)(8 * j) * in_row;
       const uint32_t vo = (j & 1) ? vo_in1 : vo_in0;
       dma16_epi((const char *)p.Xh + ub + ro + vo, lds_addr(b + j * 1024));
-      if (!in8) dma16_epi((const char *)p.Xl + ub + ro + vo, lds_addr(b + 4096 + j * 1024));
+      if (!in8) dma16_epi((const char *)p.Xl + ((ub + ro) & lo_at) + (vo & (uint32_t)lo_at), lds_addr(b + 4096 + j * 1024));
     }
     if (in8) {
 #pragma unroll
@@ -624,7 +625,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     // (row&7) ^ ((row>>3)&1): the 32 rows a read touches spread over all banks.
     const int rr = lane & 31, hh = lane >> 5;
     const int key = (rr & 7) ^ ((rr >> 3) & 1);
-    const bool fp32_out = p.X32 != nullptr;
+    const bool fp32_out = p.X32 != nullptr || p.X16 != nullptr;
     // Fused weight update (last step): the slab is the Newton-Schulz result O of a 32x64 (or,
     // for a tall weight whose chain ran on its transpose, 64x32) block of the weight W; the
     // epilogue reads that block of the fp32 master, subtracts lr*O, writes it back together with
@@ -797,7 +798,9 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
           for (int pz = 0; pz < 8; ++pz) {
             const int idx = pz * 64 + lane, row = idx >> 4, c = idx & 15;
             const anc_f32x4 v4 = *(const anc_f32x4 *)(b + row * 256 + ((c ^ (row & 15)) * 16));
-            epi_st((anc_f32x4 *)(p.X32 + mn + (int64_t)(gi0 + row) * N + gj0w + c * 4), v4);
+            const int64_t off = mn + (int64_t)(gi0 + row) * N + gj0w + c * 4;
+            if (p.X32 != nullptr) epi_st((anc_f32x4 *)(p.X32 + off), v4);
+            else epi_st((anc_u32x2 *)(p.X16 + off), anc_u32x2{anc_pk_bf16(v4.x, v4.y), anc_pk_bf16(v4.z, v4.w)});
           }
         } else {
 #pragma unroll

@@ -395,11 +395,13 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
           for (int k = 0; k < 16; ++k)
             x[k] = anc_low8_decode(__float_as_uint(x[k]), (int)(qq[k >> 2] << (24 - 8 * (k & 3))) >> 24);
         } else {
-          float xl[16];
-          unpack(*(const anc_u32x4 *)(p.Xl + xo), xl);
-          unpack(*(const anc_u32x4 *)(p.Xl + xo + 8), xl + 8);
+          if (!p.lo_zero) {
+            float xl[16];
+            unpack(*(const anc_u32x4 *)(p.Xl + xo), xl);
+            unpack(*(const anc_u32x4 *)(p.Xl + xo + 8), xl + 8);
 #pragma unroll
-          for (int k = 0; k < 16; ++k) x[k] = x[k] + xl[k];
+            for (int k = 0; k < 16; ++k) x[k] = x[k] + xl[k];
+          }
         }
         if (p.scale != nullptr) {
 #pragma unroll
@@ -464,6 +466,8 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             *(anc_f32x4 *)(p.X32 + o + 4 * i) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+        } else if (p.X16 != nullptr) {
+          put_bf16(p.X16 + mn + (int64_t)gi * N + gj, nullptr);
         } else if (out8) {
           uint32_t h[8], q[4] = {0u, 0u, 0u, 0u};
 #pragma unroll

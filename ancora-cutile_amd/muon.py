@@ -452,6 +452,15 @@ class ResidentMuon:
         """g_dev: (K,N) device weight-gradient (float32, or uint16 bf16 bits)."""
         K, N, sc = self.K, self.N, self.sc
         ctl = 0 if guard is None else guard.ptr
+        schedule = muon_ns._resolve(schedule)
+        mode = muon_ns.effective_mode(self.mode, schedule)
+        if mode != "fp32" and self.ns >= 2:
+            ws = sc.ws.ensure(muon_ns.ns_workspace_bytes(1, self.M, self.Nn, mode))
+            api.anc_muon_resident_step(self.buf.ptr, g_dev.ptr, _g_code(g_dev.dtype), self.p32.ptr, self.p16.ptr, sc.u.ptr,
+                                       K, N, float(self.mom), 1, float(lr * self.shape_scale), self.ns,
+                                       muon_ns.coef_array(schedule, self.ns), 1e-7, muon_ns.MODES[mode], ws.ptr, ws.nbytes,
+                                       ctl, int(si))
+            return
         api.anc_muon_momentum(self.buf.ptr, g_dev.ptr, sc.u.ptr, K, N, float(self.mom), 1,
                               int(self.tr), _g_code(g_dev.dtype), F32, ctl, int(si))
         muon_ns.ns_batched(sc.u, 1, self.M, self.Nn, si, steps=self.ns, schedule=schedule,

@@ -8,8 +8,8 @@ and the 28-launch chain behind those drivers are replaced by one C entry point,
 
 The library carries the iterate in fp32 (operands are rounded to bf16 only at the
 matrix-core input), so its native driver `ns_batched` takes and returns fp32. The two
-reference-shaped drivers keep the reference's bf16 in / bf16 out contract on `gX`: they
-widen into a workspace, run the chain and round the result back (RNE). Their scratch
+reference-shaped drivers keep the reference's bf16 in / bf16 out contract on `gX`: the
+chain reads the bf16 matrices as they are and rounds its result back (RNE). Their scratch
 arguments (gA, gA2, gB, gBX, grecip) are accepted for call compatibility and not touched.
 """
 import ctypes
@@ -121,14 +121,20 @@ class NsWorkspace:
 
 
 _SHARED_WS = NsWorkspace()
+_WS_BYTES = {}
 
 
 def ns_workspace_bytes(E, M, N, mode="bf16"):
-    _lib.load()
-    n = api.anc_ns_workspace_bytes(E, M, N, MODES[mode])
-    if n < 0:
-        raise _lib.AncoraError(_lib._lib.anc_last_error().decode())
-    return int(n)
+    key = (E, M, N, mode)
+    n = _WS_BYTES.get(key)
+    if n is None:
+        _lib.load()
+        n = int(api.anc_ns_workspace_bytes(E, M, N, MODES[mode]))
+        if n < 0:
+            raise _lib.AncoraError(_lib._lib.anc_last_error().decode())
+        if len(_WS_BYTES) < 4096:
+            _WS_BYTES[key] = n
+    return n
 
 
 def _acct_mode(mode, schedule):
@@ -216,11 +222,16 @@ def _run_bf16(gX, E, M, N, si, steps, eps, schedule, mode, workspace):
     ws = _SHARED_WS if workspace is None else workspace
     n = E * M * N
     need = ns_workspace_bytes(E, M, N, mode)
+    coef = coef_array(schedule, steps)
+    if mode != "fp32" and steps >= 2:
+        buf = ws.ensure(need)
+        api.anc_ns_batched_bf16(gX.ptr, E, M, N, int(steps), coef, float(eps), MODES[mode], buf.ptr, buf.nbytes, int(si))
+        return
+    # fp32 arithmetic, or a chain too short to overlay its input: through a widened copy
     xbytes = (n * 4 + 255) // 256 * 256
     buf = ws.ensure(need + xbytes)
     x32 = DevBuf(shape=(E * M, N), dtype=np.float32, ptr=buf.ptr)
     api.anc_bf16_to_f32(gX.ptr, x32.ptr, n, int(si))
-    coef = coef_array(schedule, steps)
     api.anc_ns_batched(x32.ptr, E, M, N, int(steps), coef, float(eps), MODES[mode],
                        buf.ptr + xbytes, buf.nbytes - xbytes, int(si))
     api.anc_f32_to_bf16(x32.ptr, gX.ptr, n, int(si))

@@ -522,6 +522,21 @@ int anc_ns_batched(uint64_t X, int64_t E, int64_t M, int64_t N,
                    int mode, uint64_t workspace, int64_t workspace_bytes,
                    uint64_t stream);
 
+/* The same chain on (E,M,N) bf16 matrices in place (the reference-typed drivers): no widened copy; steps >= 2,
+ * bf16 modes. The input enters unscaled and exact, its norm applied by the first step's epilogues as in
+ * anc_ns_batched_pair; a matrix of norm below 9e-16 is first brought into [1, 2) by a power of two, in place. */
+int anc_ns_batched_bf16(uint64_t X, int64_t E, int64_t M, int64_t N, int steps, const float *coef, float eps,
+                        int mode, uint64_t workspace, int64_t workspace_bytes, uint64_t stream);
+
+/* One weight's Muon step in one call: anc_muon_momentum_multi_pair + anc_muon_ns_update_multi for a
+ * weight W (K,N) with momentum buffer `buf`, gradient g, master p32, bf16 copy p16 (may be 0). u: scratch of
+ * K*N fp32 elements. lr_scale = lr * sqrt(max(1, K/N)). workspace: anc_ns_workspace_bytes(1, min, max, mode). Replaces
+ * the launches of `ResidentMuon.step` (ancora/optim/muon.py:180-204). steps >= 2, bf16 modes. */
+int anc_muon_resident_step(uint64_t buf, uint64_t g, int g_dtype, uint64_t p32, uint64_t p16, uint64_t u,
+                           int64_t K, int64_t N, float mom, int nesterov, float lr_scale, int steps,
+                           const float *coef, float eps, int mode, uint64_t workspace,
+                           int64_t workspace_bytes, uint64_t ctl, uint64_t stream);
+
 /* The same chain fed by anc_muon_momentum_multi_pair: the momentum kernel leaves the
  * unnormalised input U as a bf16 pair (Uh = bf16(u), Ul = bf16(u - Uh), both (E,M,N)) and
  * n_partials sums of u*u per matrix; the reference's separate norm and scale passes

@@ -192,6 +192,25 @@ def test_tile_choice_keeps_the_bits(gpu, M, N, mode):
     assert rel_fro(want[0], host_ns(X[0], PE_SCHEDULE, 5)) < TOL_BF16
 
 
+@pytest.mark.parametrize("E,M,N", [(1, 128, 128), (3, 128, 384), (2, 256, 512), (1, 640, 768), (2, 1024, 1024), (2, 1024, 2048)])
+@pytest.mark.parametrize("sched", ["pe", "keller"])
+def test_bf16_entry_takes_the_matrix_as_it_is(gpu, E, M, N, sched):
+    """`newton_schulz_resident_e` enters the chain without a low half (a plan that splits its first iteration, M < 256,
+    gets a cleared one) and rounds in the last epilogue; a matrix of tiny norm is rescaled by a power of two."""
+    from ancora_cutile_amd import DevBuf, newton_schulz_resident_e
+    schedule = PE_SCHEDULE if sched == "pe" else None
+    rng = np.random.default_rng(E + M + N)
+    bits = bf16_rne_bits(rng.standard_normal((E * M, N)).astype(np.float32)).reshape(E, M, N)
+    x = bits_to_f32(bits).reshape(E, M, N)
+    bits[E - 1] = bf16_rne_bits(x[E - 1] * np.float32(2.0 ** -62)).reshape(M, N)      # exact: same matrix, tiny
+    g = DevBuf(bits.reshape(E * M, N))
+    newton_schulz_resident_e(g, None, None, None, None, None, E, M, N, 0, schedule=schedule, eps=1e-30)
+    got = bits_to_f32(g.to_numpy()).reshape(E, M, N)
+    for e in range(E):
+        assert rel_fro(got[e], host_ns(x[e], schedule, 5)) < 2.8e-3, e        # 2e-3 and the bf16 result's 1.7e-3
+    g.free()
+
+
 def test_zero_matrix_and_scale_invariance(gpu):
     """A zero gradient (an idle expert) stays zero, no NaN; NS(cX) == NS(X) up to rounding."""
     rng = np.random.default_rng(3)
