@@ -174,7 +174,7 @@ extern "C" int anc_gemm_dw_multi(const anc_dw_problem_t *probs, int32_t n_probs,
   ANC_REQUIRE(blocks < (1ll << 31), "anc_gemm_dw_multi: too large");
   {
     AncProfScope prof(ANC_PROF_DW_GEMM, s);
-    if (int rc = anc_ns_gemm_big_plain(g, Es, n_probs, s, tn)) return rc;
+    if (int rc = anc_ns_gemm_plain(g, Es, n_probs, s, tn)) return rc;
   }
   if (blocks > 0) {
     AncProfScope prof(ANC_PROF_DW_REDUCE, s);

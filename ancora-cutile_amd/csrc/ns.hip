@@ -974,6 +974,13 @@ int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int f
   return ANC_OK;
 }
 
+int anc_ns_gemm_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool a_transposed) {
+  ANC_REQUIRE(n >= 1 && n <= kMaxGroups, "anc_ns_gemm_plain: 1..%d problems per launch", kMaxGroups);
+  const int tile = pick_tile(EPI_BX, ps, Es, n);
+  if (tile == 256) return anc_ns_gemm_big_plain(ps, Es, n, s, a_transposed);
+  return anc_ns_gemm_tile_multi(EPI_BX, ps, Es, n, s, tile == 64, a_transposed, nullptr, true);
+}
+
 extern "C" int64_t anc_ns_workspace_bytes(int64_t E, int64_t M, int64_t N, int mode) {
   mode &= ~kTileFlags;
   if (check_shape(E, M, N, mode, "anc_ns_workspace_bytes")) return -1;
