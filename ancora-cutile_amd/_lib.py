@@ -100,6 +100,11 @@ _PROTOS = {
     "anc_mem_info": (None, [C.POINTER(i64), C.POINTER(i64)]),
     "anc_fill_u32": (None, [u64, u32, i64, u64]),
     "anc_memcpy_h2d": (None, [u64, C.c_void_p, i64, u64]),
+    "anc_upload_async": (None, [u64, C.c_void_p, i64, u64]),
+    "anc_upload_now": (None, [u64, C.c_void_p, i64]),
+    "anc_staging_release": (None, []),
+    "anc_id_groups": (None, [C.c_void_p, i64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.POINTER(i64)]),
+    "anc_unique_ids": (None, [C.c_void_p, i64, C.c_void_p, C.POINTER(i64)]),
     "anc_memcpy_d2h": (None, [C.c_void_p, u64, i64, u64]),
     "anc_memcpy_d2d": (None, [u64, u64, i64, u64]),
     "anc_stream_create": (None, [C.POINTER(u64)]),

@@ -48,6 +48,9 @@ struct Tensor {
   uint32_t seed;
 };
 
+// The divide form once both bias corrections have become 1.0f (160 steps at beta 0.9, 325 at 0.95): x / 1.0f is x.
+constexpr int kFormDiv1 = 2;
+
 template <int FORM>
 __device__ __forceinline__ void adamw_elem(float g, float &m, float &v, float &p,
                                            const anc_adamw_hyper_t &h, float wd, float clip) {
@@ -58,6 +61,10 @@ __device__ __forceinline__ void adamw_elem(float g, float &m, float &v, float &p
     const float mh = m / h.bc1;
     const float vh = v / h.bc2;
     p = p - h.lr * (mh / (sqrtf(vh) + h.eps) + wd * p);
+  } else if (FORM == kFormDiv1) {
+    m = h.beta1 * m + h.omb1 * gs;
+    v = h.beta2 * v + (h.omb2 * gs) * gs;
+    p = p - h.lr * (m / (sqrtf(v) + h.eps) + wd * p);
   } else {
     const float o1 = 1.0f - h.beta1, o2 = 1.0f - h.beta2;
     m = h.beta1 * m + o1 * gs;
@@ -235,7 +242,7 @@ k_adamw_rows(const int32_t *__restrict__ rows, const float *__restrict__ grads, 
   const bool with_step = grads != nullptr;
   const int t_replay = with_step ? t_now - 1 : t_now;    // replay (g = 0) through this step
   if (k0 >= t_now || (!with_step && k0 >= t_replay)) return;
-  for (int c = (int)threadIdx.x * kVec; c < H; c += kSlab) {
+  for (int c = (int)threadIdx.x * kVec; c < H; c += (int)blockDim.x * kVec) {
     const int64_t e = row * H + c;
     const anc_f32x4 m4 = *(const anc_f32x4 *)(m + e), v4 = *(const anc_f32x4 *)(v + e), p4 = *(const anc_f32x4 *)(p32 + e);
     float mm[4] = {m4.x, m4.y, m4.z, m4.w}, vv[4] = {v4.x, v4.y, v4.z, v4.w}, pp[4] = {p4.x, p4.y, p4.z, p4.w};
@@ -245,8 +252,13 @@ k_adamw_rows(const int32_t *__restrict__ rows, const float *__restrict__ grads, 
       const RowStep rs = table[s];
       hs.bc1 = rs.bc1; hs.bc2 = rs.bc2; hs.lr = rs.lr;
       seed_step = rs.seed_base;
+      if (FORM == ANC_ADAMW_FORM_DIV && rs.bc1 == 1.0f && rs.bc2 == 1.0f) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) adamw_elem<FORM>(0.0f, mm[k], vv[k], pp[k], hs, wd, 1.0f);
+        for (int k = 0; k < 4; ++k) adamw_elem<kFormDiv1>(0.0f, mm[k], vv[k], pp[k], hs, wd, 1.0f);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) adamw_elem<FORM>(0.0f, mm[k], vv[k], pp[k], hs, wd, 1.0f);
+      }
     }
     if (with_step) {
       const RowStep rs = table[t_now];
@@ -373,7 +385,9 @@ extern "C" int anc_adamw_rows(uint64_t rows, int64_t n_rows, uint64_t grads, uin
   AncProfScope prof(ANC_PROF_ADAMW, anc_stream(stream));
   dispatch_form_sr(hh.form, hh.sr, [&](auto F, auto S) {
     constexpr int f = decltype(F)::value, s = decltype(S)::value;
-    hipLaunchKernelGGL((k_adamw_rows<f, s>), dim3((unsigned)n_rows), dim3(kThreads), 0, anc_stream(stream),
+    // a narrow row takes the wavefronts it fills
+    const unsigned threads = H >= kSlab ? (unsigned)kThreads : (unsigned)((H / kVec + 63) / 64 * 64);
+    hipLaunchKernelGGL((k_adamw_rows<f, s>), dim3((unsigned)n_rows), dim3(threads), 0, anc_stream(stream),
                        (const int32_t *)rows, (const float *)grads, (float *)m, (float *)v, (float *)p32,
                        (uint16_t *)p16, (int32_t *)last_step, (int)H, V, (const RowStep *)step_table, (int)t_now, hh,
                        wd, seed, (const anc_step_ctl_t *)ctl);

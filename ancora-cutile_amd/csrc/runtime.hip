@@ -167,6 +167,78 @@ extern "C" int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint
   ANC_HIP(hipStreamSynchronize(anc_stream(stream)));
   return ANC_OK;
 }
+// ---- small uploads through a ring of pinned slots ----------------------------------------------
+// A pageable upload blocks until the copy is done, which on a busy stream means until everything before it is
+// done. Up to kSlotBytes the source is copied into a pinned slot instead and the call returns; a slot is
+// taken again once the event behind its last copy has passed. The ring is shared by all threads and streams
+// (2 MiB at most, pinned slot by slot on first use, given back by anc_staging_release).
+namespace {
+constexpr int kSlots = 8;
+constexpr int64_t kSlotBytes = 256 << 10;
+struct StageSlot {
+  void *mem = nullptr;
+  hipEvent_t done = nullptr;
+  bool busy = false;
+};
+std::mutex g_stage_mu;
+StageSlot g_stage[kSlots];
+int g_stage_next = 0;
+hipStream_t g_stage_stream = nullptr;     // for uploads that are complete on return without waiting for anybody's work
+
+int stage_copy(uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool wait) {
+  std::lock_guard<std::mutex> lk(g_stage_mu);
+  StageSlot &slot = g_stage[g_stage_next];
+  g_stage_next = (g_stage_next + 1) % kSlots;
+  if (slot.mem == nullptr) {
+    ANC_HIP(hipHostMalloc(&slot.mem, (size_t)kSlotBytes, hipHostMallocDefault));
+    if (hipError_t e = hipEventCreateWithFlags(&slot.done, hipEventDisableTiming)) {
+      (void)hipHostFree(slot.mem);
+      slot.mem = nullptr;
+      return anc_hip_fail(e, "hipEventCreateWithFlags", __FILE__, __LINE__);
+    }
+  }
+  if (slot.busy) ANC_HIP(hipEventSynchronize(slot.done));
+  slot.busy = false;
+  if (wait) {
+    if (g_stage_stream == nullptr) ANC_HIP(hipStreamCreateWithFlags(&g_stage_stream, hipStreamNonBlocking));
+    s = g_stage_stream;
+  }
+  memcpy(slot.mem, src, (size_t)bytes);
+  ANC_HIP(hipMemcpyAsync((void *)dst, slot.mem, (size_t)bytes, hipMemcpyHostToDevice, s));
+  if (wait) {
+    ANC_HIP(hipStreamSynchronize(s));
+    return ANC_OK;
+  }
+  ANC_HIP(hipEventRecord(slot.done, s));
+  slot.busy = true;
+  return ANC_OK;
+}
+}  // namespace
+extern "C" int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream) {
+  ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_upload_async: bad arguments");
+  if (bytes == 0) return ANC_OK;
+  if (bytes > kSlotBytes) return anc_memcpy_h2d(dst, src, bytes, stream);
+  return stage_copy(dst, src, bytes, anc_stream(stream), false);
+}
+extern "C" int anc_upload_now(uint64_t dst, const void *src, int64_t bytes) {
+  ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_upload_now: bad arguments");
+  for (int64_t at = 0; at < bytes; at += kSlotBytes)
+    if (int rc = stage_copy(dst + (uint64_t)at, (const char *)src + at, bytes - at < kSlotBytes ? bytes - at : kSlotBytes, nullptr, true)) return rc;
+  return ANC_OK;
+}
+extern "C" int anc_staging_release(void) {
+  std::lock_guard<std::mutex> lk(g_stage_mu);
+  for (StageSlot &slot : g_stage) {
+    if (slot.mem == nullptr) continue;
+    if (slot.busy) ANC_HIP(hipEventSynchronize(slot.done));
+    ANC_HIP(hipEventDestroy(slot.done));
+    ANC_HIP(hipHostFree(slot.mem));
+    slot = StageSlot{};
+  }
+  if (g_stage_stream != nullptr) ANC_HIP(hipStreamDestroy(g_stage_stream));
+  g_stage_stream = nullptr;
+  return ANC_OK;
+}
 extern "C" int anc_memcpy_d2h(void *dst, uint64_t src, int64_t bytes, uint64_t stream) {
   ANC_REQUIRE(dst != nullptr && src != 0 && bytes >= 0, "anc_memcpy_d2h: bad arguments");
   if (bytes == 0) return ANC_OK;

@@ -7,6 +7,7 @@ it updates only the rows a step's tokens touch and replays the steps a row misse
 next needed, so that every row it hands out is bit-identical to the dense optimizer's.
 """
 import ctypes
+import threading
 
 import numpy as np
 
@@ -16,37 +17,105 @@ from .adamw import sr_seed_base
 from .devbuf import DevBuf
 
 
+def _ids32(ids):
+    """Integer ids as a contiguous int32 vector."""
+    ids = np.asarray(ids).reshape(-1)
+    if ids.dtype != np.int32:
+        if ids.dtype.kind not in "iub" or (ids.size and ids.dtype.itemsize >= 4 and
+                                           (int(ids.max()) > 0x7FFFFFFF or int(ids.min()) < -0x80000000)):
+            raise ValueError(f"token ids must be integers of 32 bits, got {ids.dtype}")
+        ids = ids.astype(np.int32)
+    return np.ascontiguousarray(ids)
+
+
+def _id_groups(ids_flat):
+    """((4, M) int32: srt, start, cnt, gid; number of groups)."""
+    _lib.load()
+    ids = _ids32(ids_flat)
+    out = np.empty((4, ids.size), np.int32)
+    n = ctypes.c_int64(0)
+    p, step = out.ctypes.data, 4 * ids.size
+    api.anc_id_groups(ids.ctypes.data, ids.size, p, p + step, p + 2 * step, p + 3 * step, ctypes.byref(n))
+    return out, n.value
+
+
 def build_id_groups(ids_flat):
     """Stable-sort token ids into groups (ancora/kernels/fused.py:411-424). Returns
     (srt, start, cnt, gid), each (M, 1) int32: srt the stable argsort; for group g (one per
     distinct id, ascending) start[g] its first position in srt, cnt[g] its size, gid[g] its id;
     groups beyond the last are padding with cnt = 0."""
-    ids = np.asarray(ids_flat).reshape(-1)
-    M = ids.size
-    order = np.argsort(ids, kind="stable").astype(np.int32)
-    uniq, first, counts = np.unique(ids[order], return_index=True, return_counts=True)
-    U = uniq.size
-    out = [order.reshape(M, 1)]
-    for col in (first, counts, uniq):
-        a = np.zeros((M, 1), np.int32)
-        a[:U, 0] = col
-        out.append(a)
-    return tuple(out)
+    out, _ = _id_groups(ids_flat)
+    return tuple(a.reshape(-1, 1) for a in out)
+
+
+class _Blocks:
+    """Device blocks of the group arrays, kept between steps: an allocation and a release per step cost more than
+    the arrays' upload, and a release waits for the whole device. A block given back may still be read by work in
+    flight on any stream, so it is handed out again only after a device synchronisation, one for every
+    KEEP blocks. At most KEEP are kept; `trim` gives them back to the device."""
+
+    KEEP = 8
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._ready, self._waiting = [], []
+
+    def get(self, nbytes):
+        with self._lock:
+            if len(self._waiting) >= self.KEEP:
+                api.anc_device_sync()
+                self._ready += self._waiting
+                self._waiting = []
+                self._ready.sort(key=lambda b: b.nbytes)
+                for b in self._ready[:-self.KEEP]:
+                    b.free()
+                self._ready = self._ready[-self.KEEP:]
+            for i, b in enumerate(self._ready):
+                if nbytes <= b.nbytes <= 4 * nbytes + 65536:
+                    return self._ready.pop(i)
+        return DevBuf.empty((max(nbytes, 4096),), np.uint8)
+
+    def put(self, b):
+        with self._lock:
+            if len(self._waiting) < self.KEEP:
+                self._waiting.append(b)
+                return
+        b.free()
+
+    def trim(self):
+        with self._lock:
+            for b in self._ready + self._waiting:
+                b.free()
+            self._ready, self._waiting = [], []
+
+
+_blocks = _Blocks()
+trim_pool = _blocks.trim
 
 
 class IdGroups:
     """The four group arrays on the device, plus the number of distinct ids."""
 
     def __init__(self, ids_flat):
-        srt, start, cnt, gid = build_id_groups(ids_flat)
-        self.M = srt.shape[0]
-        self.n_groups = int(np.count_nonzero(cnt))
-        self.host = (srt, start, cnt, gid)
-        self.srt, self.start, self.cnt, self.gid = (DevBuf(a) for a in (srt, start, cnt, gid))
+        _lib.init()
+        self._arrays, self.n_groups = _id_groups(ids_flat)
+        self.M = M = self._arrays.shape[1]
+        self._block = _blocks.get(self._arrays.nbytes)
+        api.anc_upload_now(self._block.ptr, self._arrays.ctypes.data, self._arrays.nbytes)
+        self.srt, self.start, self.cnt, self.gid = (
+            DevBuf(shape=(M, 1), dtype=np.int32, ptr=self._block.ptr + i * 4 * M) for i in range(4))
+
+    @property
+    def host(self):
+        """The arrays as `build_id_groups` returns them."""
+        return tuple(a.reshape(-1, 1) for a in self._arrays)
 
     def free(self):
+        if self._block is not None:
+            _blocks.put(self._block)
+            self._block = None
         for b in (self.srt, self.start, self.cnt, self.gid):
-            b.free()
+            b.ptr = 0
 
 
 def embed_dw_scatter(groups, dy, si, out=None, compact=None, V=None):
@@ -88,7 +157,7 @@ class RowSparseAdamW:
         self.last = DevBuf.zeros((self.V,), np.int32)
         self._cap = int(max_steps)
         self.table = DevBuf.zeros((self._cap + 1, 4), np.uint32)
-        self._rows_buf = None
+        self._rows_buf, self._rows_si = None, 0
         self.last_skipped = False
         self._filled_to = 0          # table entries 1 .. _filled_to hold the scalars of their steps
         self._filled_lr = None       # ... computed with this learning rate
@@ -122,13 +191,15 @@ class RowSparseAdamW:
         self._filled_to, self._filled_lr = hi, self.lr
 
     def _rows(self, rows, si):
-        rows = np.ascontiguousarray(rows, dtype=np.int32).reshape(-1)
         if self._rows_buf is None or self._rows_buf.size < rows.size:
             if self._rows_buf is not None:
-                _lib.stream_sync(si)
+                _lib.stream_sync(self._rows_si)
                 self._rows_buf.free()
             self._rows_buf = DevBuf.empty((max(rows.size, 1024),), np.int32)
-        self._rows_buf.upload(rows, si)
+        elif self._rows_si != si:
+            _lib.stream_sync(self._rows_si)        # the buffer's last reader ran on another stream
+        self._rows_si = si
+        api.anc_upload_async(self._rows_buf.ptr, rows.ctypes.data, rows.nbytes, int(si))
         return self._rows_buf, rows.size
 
     def _launch(self, rows_ptr, n_rows, grads_ptr, t_now, ctl, si):
@@ -141,7 +212,12 @@ class RowSparseAdamW:
         """Replay, on the distinct rows in `row_ids` (host integers), the steps they missed."""
         if self.t == 0:
             return
-        buf, n = self._rows(np.unique(np.asarray(row_ids).reshape(-1)), si)
+        ids = _ids32(row_ids)
+        if ids.size == 0:
+            return
+        rows, n = np.empty(ids.size, np.int32), ctypes.c_int64(0)
+        api.anc_unique_ids(ids.ctypes.data, ids.size, rows.ctypes.data, ctypes.byref(n))
+        buf, n = self._rows(rows[:n.value], si)
         self._launch(buf.ptr, n, 0, self.t, 0, si)
 
     def step(self, gid, n_groups, grads, si, guard=None):

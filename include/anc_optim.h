@@ -72,6 +72,12 @@ int anc_mem_info(int64_t *free_bytes, int64_t *total_bytes);
 /* Fill with a 32-bit pattern using a kernel (safe inside graph capture). */
 int anc_fill_u32(uint64_t dptr, uint32_t value, int64_t n_words, uint64_t stream);
 int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
+/* Small uploads (up to 256 KiB each) through pinned staging: src may be reused on return. _async: ordered
+ * on `stream`, no wait (larger ones: anc_memcpy_h2d). _now: complete on return, on a stream of its own, without
+ * waiting for work queued elsewhere; nobody may be using dst. _release gives the staging memory back. */
+int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
+int anc_upload_now(uint64_t dst, const void *src, int64_t bytes);
+int anc_staging_release(void);
 int anc_memcpy_d2h(void *dst, uint64_t src, int64_t bytes, uint64_t stream);
 int anc_memcpy_d2d(uint64_t dst, uint64_t src, int64_t bytes, uint64_t stream);
 int anc_stream_create(uint64_t *stream);
@@ -293,6 +299,12 @@ int anc_adamw_rows(uint64_t rows, int64_t n_rows, uint64_t grads, uint64_t m, ui
 int anc_embed_dw_scatter(uint64_t cnt, uint64_t start, uint64_t gid, uint64_t srt, uint64_t dy,
                          uint64_t out, uint64_t compact, int64_t M, int64_t V, int64_t H,
                          uint64_t stream);
+
+/* Host side of it: the group arrays of n token ids (`build_id_groups`, fused.py:411-424), all int32[n], padded
+ * with zeros behind the last group; and the distinct ids in ascending order (out: room for n). */
+int anc_id_groups(const int32_t *ids, int64_t n, int32_t *srt, int32_t *start, int32_t *cnt, int32_t *gid,
+                  int64_t *n_groups);
+int anc_unique_ids(const int32_t *ids, int64_t n, int32_t *out, int64_t *n_out);
 
 /* p16 = bf16(p32): replaces `_cast_bf16` (ancora/kernels/fused.py:285-290). */
 int anc_cast_bf16(uint64_t p32, uint64_t p16, int64_t n, int sr, uint32_t seed,

@@ -1,5 +1,6 @@
 """Pins of oracle/embed_ref.py and of the host-side group builder (CPU only)."""
 import numpy as np
+import pytest
 
 from oracle.bf16_ref import bf16_rne_bits, bits_to_f32
 from oracle.embed_ref import id_groups, embed_dw_rows, embed_dw_scatter
@@ -32,6 +33,22 @@ def test_host_builder_matches_the_oracle_and_pads():
     assert np.array_equal(srt[:, 0], o_srt)
     assert np.array_equal(start[:U, 0], o_start) and np.array_equal(cnt[:U, 0], o_cnt)
     assert np.array_equal(gid[:U, 0], o_gid) and not cnt[U:].any() and not start[U:].any()
+
+
+@pytest.mark.parametrize("ids", [np.zeros(1), np.array([5, 5, 5]), np.array([-3, 7, -3, 0, 7]), np.array([2**31 - 1, -2**31, 0, 2**31 - 1]),
+                                 np.arange(300)[::-1], np.array([63, 64, 65, 127, 128, 64, 0])], ids=str)
+def test_host_builder_at_the_edges(ids):
+    """One id, one group, negative ids, the whole 32-bit range (sorted instead of ranked by bitmap), word borders."""
+    from ancora_cutile_amd.embed import build_id_groups, _lib, api
+    ids = ids.astype(np.int32)
+    srt, start, cnt, gid = (a[:, 0] for a in build_id_groups(ids))
+    o_srt, o_start, o_cnt, o_gid = id_groups(ids)
+    U = o_gid.size
+    assert np.array_equal(srt, o_srt) and np.array_equal(start[:U], o_start)
+    assert np.array_equal(cnt[:U], o_cnt) and np.array_equal(gid[:U], o_gid) and not cnt[U:].any()
+    out, n = np.empty(ids.size, np.int32), _lib.i64(0)
+    api.anc_unique_ids(ids.ctypes.data, ids.size, out.ctypes.data, n)
+    assert np.array_equal(out[:n.value], np.unique(ids))
 
 
 def test_scatter_sum_exact_case_and_reference_gate():
