@@ -108,6 +108,7 @@ _PROTOS = {
     "anc_memcpy_d2h": (None, [C.c_void_p, u64, i64, u64]),
     "anc_memcpy_d2d": (None, [u64, u64, i64, u64]),
     "anc_stream_create": (None, [C.POINTER(u64)]),
+    "anc_stream_create_nonblocking": (None, [C.POINTER(u64)]),
     "anc_stream_destroy": (None, [u64]),
     "anc_stream_sync": (None, [u64]),
     "anc_device_sync": (None, []),
@@ -240,6 +241,13 @@ def stream_create():
     init()
     s = u64(0)
     api.anc_stream_create(C.byref(s))
+    return int(s.value)
+
+
+def stream_create_nonblocking():
+    init()
+    s = u64(0)
+    api.anc_stream_create_nonblocking(C.byref(s))
     return int(s.value)
 
 

@@ -172,9 +172,9 @@ class AdamW:
         ibc2 = 1.0 / (1.0 - self.b2 ** self.t)
         return hyper_ibc(self.lr, self.b1, self.b2, self.eps, ibc1, ibc2, self.sr, sb)
 
-    def launch(self, grads, stream_int, guard=None, device_steps=False, t_upper=None):
+    def launch(self, grads, stream_int, guard=None, device_steps=False, t_upper=None, uploader=None):
         """Asynchronous part of the step: upload host gradients (DevBuf gradients are used in
-        place) and launch the fused kernel once over all tensors. `t` is advanced first, as in
+        place; `uploader`, if given, puts the uploads on a stream beside `stream_int`) and launch the fused kernel once over all tensors. `t` is advanced first, as in
         ancora/optim/adamw.py:89-91; a caller that later finds the step skipped calls `unstep()`.
         With `device_steps` the step count lives in the guard's control block (advanced by
         `guard.compute(..., count_step=True)` unless the step is skipped): the kernel takes the
@@ -198,8 +198,10 @@ class AdamW:
                     if g.dtype != s["g"].dtype:
                         raise TypeError(f"AdamW: gradient of '{name}' is {g.dtype}, the optimizer "
                                         f"was built for {s['g'].dtype}")
-                s["g"].upload(g.reshape(s["R"], C), stream_int)
+                s["g"].upload_async(g.reshape(s["R"], C), stream_int if uploader is None else uploader.begin())
                 gbufs.append(s["g"])
+        if uploader is not None:
+            uploader.end(stream_int)
         self._build_table(gbufs)
         if device_steps:
             if self.form == "div":

@@ -88,6 +88,13 @@ class DevBuf:
             raise ValueError(f"DevBuf.upload: {arr.nbytes} B into a buffer of {self.nbytes} B")
         api.anc_memcpy_h2d(self.ptr, arr.ctypes.data_as(C.c_void_p), arr.nbytes, int(stream))
 
+    def upload_async(self, arr, stream):
+        """`upload` that returns once `arr` may be reused: later work on `stream` sees the data."""
+        arr = np.ascontiguousarray(arr)
+        if arr.nbytes > self.nbytes:
+            raise ValueError(f"DevBuf.upload: {arr.nbytes} B into a buffer of {self.nbytes} B")
+        api.anc_upload_async(self.ptr, arr.ctypes.data_as(C.c_void_p), arr.nbytes, int(stream))
+
     def to_numpy(self, stream=0):
         out = np.empty(self.shape, self.dtype)
         api.anc_memcpy_d2h(out.ctypes.data_as(C.c_void_p), self.ptr, self.nbytes, int(stream))

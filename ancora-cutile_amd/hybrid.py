@@ -46,6 +46,36 @@ def resident_is_muon(name, p):
     return p.shape[-2] % NTM == 0 and p.shape[-1] % NTM == 0
 
 
+class _Uploader:
+    """Uploads on a stream of their own beside the optimizer's: they start once the work queued on the
+    optimizer's stream at `mark` is done and that stream waits for them at `end`."""
+
+    def __init__(self):
+        self.stream = _lib.stream_create_nonblocking()
+        self.before, self.after = _lib.Event(), _lib.Event()
+        self.used = False
+
+    def mark(self, si):
+        self.before.record(si)
+        self.used = False
+
+    def begin(self):
+        if not self.used:
+            self.before.wait_on(self.stream)
+            self.used = True
+        return self.stream
+
+    def end(self, si):
+        if self.used:
+            self.after.record(self.stream)
+            self.after.wait_on(si)
+
+    def free(self):
+        self.before.free()
+        self.after.free()
+        _lib.api.anc_stream_destroy(self.stream)
+
+
 class HybridOptimizer:
     def __init__(self, params, is_muon=default_is_muon, no_decay=None, muon_kw=None,
                  adamw_kw=None, si=None, muon_device=False, max_grad_norm=None, guard=False,
@@ -74,6 +104,7 @@ class HybridOptimizer:
                            no_decay=tuple(n for n in self.adamw_names if no_decay(n, params[n])),
                            grad_dtype=grad_dtype, **adamw_kw)
         self.guard = StepGuard(max_grad_norm) if (max_grad_norm is not None or guard) else None
+        self._uploader = None
         self._last_skipped = False
         self._last_ctl = None
         self._pending = None         # stream of an unsynchronised guarded step whose block was not read yet
@@ -134,8 +165,14 @@ class HybridOptimizer:
         `stream_int`, as the reference's resident step does (ancora/model/resident_train.py:338-339);
         `last_ctl` / `last_skipped` then read the device block when first asked."""
         if self.guard is None:
-            self.muon.step({n: grads[n] for n in self.muon_names}, stream_int)
-            self.adamw.step({n: grads[n] for n in self.adamw_names}, stream_int)
+            # AdamW's host gradients travel while Muon's chain runs, and the host waits once
+            if self._uploader is None:
+                self._uploader = _Uploader()
+            self._uploader.mark(stream_int)
+            self.muon.launch({n: grads[n] for n in self.muon_names}, stream_int)
+            self.adamw.launch({n: grads[n] for n in self.adamw_names}, stream_int, uploader=self._uploader)
+            _lib.stream_sync(stream_int)
+            self.muon.last_skipped = self.adamw.last_skipped = False
             return
         # guarded step: every gradient must be resident before the norm, so upload first
         for opt, names in ((self.muon, self.muon_names), (self.adamw, self.adamw_names)):
@@ -149,7 +186,7 @@ class HybridOptimizer:
                         g = np.asarray(g)
                         if g.dtype != s["g"].dtype and s["g"].dtype == np.float32:
                             g = g.astype(np.float32)
-                    s["g"].upload(g.reshape(s["g"].shape), stream_int)
+                    s["g"].upload_async(g.reshape(s["g"].shape), stream_int)
         resident = {}
         for opt, names in ((self.muon, self.muon_names), (self.adamw, self.adamw_names)):
             for n in names:
@@ -213,3 +250,6 @@ class HybridOptimizer:
         self.adamw.free()
         if self.guard is not None:
             self.guard.free()
+        if self._uploader is not None:
+            self._uploader.free()
+            self._uploader = None

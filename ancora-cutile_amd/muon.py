@@ -624,7 +624,7 @@ class Muon:
                     for r in self._recs_of[n]:
                         r["G"] = s["g"].at_pos(r["e"] * s["K"])
                     del self._gptr[n]
-                s["g"].upload(self.host_grad(n, g), si)
+                s["g"].upload_async(self.host_grad(n, g), si)
         if self.engine is not None:
             self.engine.step(si, self.lr, self.schedule, guard, defer_join, device_steps)
         return si

@@ -72,8 +72,8 @@ int anc_mem_info(int64_t *free_bytes, int64_t *total_bytes);
 /* Fill with a 32-bit pattern using a kernel (safe inside graph capture). */
 int anc_fill_u32(uint64_t dptr, uint32_t value, int64_t n_words, uint64_t stream);
 int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
-/* Small uploads (up to 256 KiB each) through pinned staging: src may be reused on return. _async: ordered
- * on `stream`, no wait (larger ones: anc_memcpy_h2d). _now: complete on return, on a stream of its own, without
+/* Uploads through pinned staging memory; src may be reused on return. anc_memcpy_h2d: complete on return.
+ * _async: ordered on `stream`, no wait. _now: complete on return, on a stream of its own, without
  * waiting for work queued elsewhere; nobody may be using dst. _release gives the staging memory back. */
 int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
 int anc_upload_now(uint64_t dst, const void *src, int64_t bytes);
@@ -81,6 +81,7 @@ int anc_staging_release(void);
 int anc_memcpy_d2h(void *dst, uint64_t src, int64_t bytes, uint64_t stream);
 int anc_memcpy_d2d(uint64_t dst, uint64_t src, int64_t bytes, uint64_t stream);
 int anc_stream_create(uint64_t *stream);
+int anc_stream_create_nonblocking(uint64_t *stream);   /* not ordered against the null stream */
 int anc_stream_destroy(uint64_t stream);
 int anc_stream_sync(uint64_t stream);
 int anc_device_sync(void);

@@ -56,6 +56,31 @@ def test_pinned_buffers_async_copies_and_fill(gpu):
     api.anc_stream_destroy(s)
 
 
+@pytest.mark.parametrize("n", [1, 4095, (512 << 10) - 1, 512 << 10, (512 << 10) + 1, (4 << 20) + 3, (8 << 20) - 1, 8 << 20, (37 << 20) + 5])
+@pytest.mark.parametrize("how", ["h2d", "async", "now"])
+def test_staged_uploads_arrive_whole(gpu, n, how):
+    """Uploads pass through pinned slots of 512 KiB, from 8 MiB on filled by four threads: sizes around a slot, a
+    full ring and the threaded copy, twice in a row (slots taken again), the source overwritten at once."""
+    from ancora_cutile_amd import DevBuf
+    rng = np.random.default_rng(n)
+    d = DevBuf.zeros(((n + 3) // 4 * 4,), np.uint8)
+    s = gpu.stream_create()
+    for _ in range(2):
+        a = rng.integers(0, 256, n, dtype=np.uint8)
+        want = a.copy()
+        if how == "h2d":
+            gpu.api.anc_memcpy_h2d(d.ptr, a.ctypes.data, n, s)
+        elif how == "async":
+            gpu.api.anc_upload_async(d.ptr, a.ctypes.data, n, s)
+        else:
+            gpu.api.anc_upload_now(d.ptr, a.ctypes.data, n)
+        a[:] = 0
+        assert np.array_equal(d.to_numpy(s)[:n], want)
+    gpu.api.anc_stream_destroy(s)
+    gpu.api.anc_staging_release()
+    d.free()
+
+
 def test_events_order_two_streams(gpu):
     """Stream B waits for an event recorded on stream A behind a long fill: B's copy sees the
     filled values; the elapsed time between two events around the fill is positive."""
