@@ -125,6 +125,54 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
   using TrA = std::bool_constant<AT>;
   using TrB = std::bool_constant<BT>;
 
+  // ---- what the epilogue of X = a X + B X reads at the output position is requested here, so that it has arrived
+  // when the K loop ends (16 x (1024,3072) on 128-wide tiles: 828 -> 783 us per 5 launches against fetching it
+  // block by block behind the loop; B = b A + c A A, which reads half as much, lost 2 % that way). The loads are older than
+  // every DMA below, so the waits of the ring hold.
+  const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
+  float *sg = (float *)lds + wave * 32 * kSgPitch;
+  float sc = 1.0f;
+  if (EPI != EPI_BMAT && !PLAINV && p.scale != nullptr) sc = anc_ld_const(p.scale + e);
+  const float acc_scale = (EPI == EPI_GRAM) ? sc * sc : sc;
+  const bool write_lo = (EPI == EPI_GRAM ? p.Fl != nullptr : EPI == EPI_BMAT ? p.Bl != nullptr : false) &&
+                        (p.lo_gated == 0 || anc_ns_wide(p, e));
+  const bool has_a32 = EPI != EPI_BX && anc_ns_has_a32(p, e);
+  const bool in8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_in);
+  const bool out8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_out);
+  const int row = lane >> 1, c0 = (lane & 1) * 16;      // this lane's 16 elements of a block: row `row`, columns c0 ..
+                                                        // (or, reading the block transposed, column `row`, rows c0 ..)
+  const int gi_w = tm * TM + wm * (32 * WB), gj_w = tn * TM + wn * (32 * WB);
+  // this lane's 16 elements of block b in a matrix of M rows in panel layout
+  auto pan_of = [&](int b) { return ((int64_t)((gj_w + (b % WB) * 32) / 32) * M + gi_w + (b / WB) * 32 + row) * 32 + c0; };
+  constexpr int NB = WB * WB;
+  anc_u32x4 pre[NB][4];
+  float drow[WB];
+  if constexpr (EPI == EPI_BX && !PLAINV) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int64_t xo = mn + (p.x_panel ? pan_of(b) : (int64_t)(gi_w + (b / WB) * 32 + row) * N + gj_w + (b % WB) * 32 + c0);
+      pre[b][0] = *(const anc_u32x4 *)(p.Xh + xo);
+      pre[b][1] = *(const anc_u32x4 *)(p.Xh + xo + 8);
+      if (in8) {
+        pre[b][2] = *(const anc_u32x4 *)((const char *)p.Xl + mn * 2 + pan_of(b));
+      } else if (!p.lo_zero) {
+        pre[b][2] = *(const anc_u32x4 *)(p.Xl + xo);
+        pre[b][3] = *(const anc_u32x4 *)(p.Xl + xo + 8);
+      }
+    }
+#pragma unroll
+    for (int bi = 0; bi < WB; ++bi) drow[bi] = p.dB[mv + gi_w + bi * 32 + row];
+  }
+  // (the master's block too where registers allow: one block per wavefront)
+  anc_f32x4 wpre[4];
+  if constexpr (VAR == VAR_UPDATE && WB == 1) {
+    const anc_muon_desc_t &d = p.upd[e];
+    const bool wtr = d.transpose != 0;
+    const int64_t we = (int64_t)((wtr ? gj_w : gi_w) + row) * d.N + (wtr ? gi_w : gj_w) + c0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wpre[i] = *(const anc_f32x4 *)((const float *)d.p32 + we + 4 * i);
+  }
+
   f32x16 acc[WB][WB];
 #pragma unroll
   for (int bi = 0; bi < WB; ++bi)
@@ -237,18 +285,6 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
 
   // ---- epilogue
   if (VAR == VAR_UPDATE && pm.ctl != nullptr && pm.ctl->skip != 0u) return;   // skipped step
-  const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
-  float *sg = (float *)lds + wave * 32 * kSgPitch;
-  float sc = 1.0f;
-  if (EPI != EPI_BMAT && !PLAINV && p.scale != nullptr) sc = anc_ld_const(p.scale + e);
-  const float acc_scale = (EPI == EPI_GRAM) ? sc * sc : sc;
-  const bool write_lo = (EPI == EPI_GRAM ? p.Fl != nullptr : EPI == EPI_BMAT ? p.Bl != nullptr : false) &&
-                        (p.lo_gated == 0 || anc_ns_wide(p, e));
-  const bool has_a32 = EPI != EPI_BX && anc_ns_has_a32(p, e);
-  const bool in8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_in);
-  const bool out8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_out);
-  const int row = lane >> 1, c0 = (lane & 1) * 16;      // this lane's 16 elements of a block: row `row`, columns c0 ..
-                                                        // (or, reading the block transposed, column `row`, rows c0 ..)
   float v[16];
   auto put_rows = [&]() {
 #pragma unroll
@@ -286,10 +322,9 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
   for (int bi = 0; bi < WB; ++bi) {
 #pragma unroll
     for (int bj = 0; bj < WB; ++bj) {
-      const int gi0 = tm * TM + (wm * WB + bi) * 32, gj0 = tn * TM + (wn * WB + bj) * 32;
+      const int gi0 = gi_w + bi * 32, gj0 = gj_w + bj * 32;
       const int gi = gi0 + row, gj = gj0 + c0;
-      // position of this lane's elements in a matrix of M rows in panel layout
-      const int64_t pan = ((int64_t)(gj0 / 32) * M + gi) * 32 + c0;
+      const int64_t pan = pan_of(bi * WB + bj);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const anc_f32x4 w = {acc[bi][bj][4 * q], acc[bi][bj][4 * q + 1], acc[bi][bj][4 * q + 2], acc[bi][bj][4 * q + 3]};
@@ -382,23 +417,21 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
         }
       } else {
         // y = (a + dB) x + B X. Only the first iteration carries the input's scale.
-        const int64_t xo = mn + (p.x_panel ? pan : (int64_t)gi * N + gj);
-        const float cf = p.ca + p.dB[mv + gi];
-        const anc_u32x4 h0 = *(const anc_u32x4 *)(p.Xh + xo), h1 = *(const anc_u32x4 *)(p.Xh + xo + 8);
+        const anc_u32x4 (&in)[4] = pre[bi * WB + bj];
+        const float cf = p.ca + drow[bi];
         float x[16];
-        unpack(h0, x);
-        unpack(h1, x + 8);
+        unpack(in[0], x);
+        unpack(in[1], x + 8);
         if (in8) {
-          const anc_u32x4 q = *(const anc_u32x4 *)((const char *)p.Xl + mn * 2 + pan);
-          const uint32_t qq[4] = {q.x, q.y, q.z, q.w};
+          const uint32_t qq[4] = {in[2].x, in[2].y, in[2].z, in[2].w};
 #pragma unroll
           for (int k = 0; k < 16; ++k)
             x[k] = anc_low8_decode(__float_as_uint(x[k]), (int)(qq[k >> 2] << (24 - 8 * (k & 3))) >> 24);
         } else {
           if (!p.lo_zero) {
             float xl[16];
-            unpack(*(const anc_u32x4 *)(p.Xl + xo), xl);
-            unpack(*(const anc_u32x4 *)(p.Xl + xo + 8), xl + 8);
+            unpack(in[2], xl);
+            unpack(in[3], xl + 8);
 #pragma unroll
             for (int k = 0; k < 16; ++k) x[k] = x[k] + xl[k];
           }
@@ -422,7 +455,7 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
           const int64_t we = (int64_t)(wr0 + row) * d.N + wc0 + c0;
           anc_f32x4 pv[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) pv[i] = *(const anc_f32x4 *)(W32 + we + 4 * i);
+          for (int i = 0; i < 4; ++i) pv[i] = WB == 1 ? wpre[i] : *(const anc_f32x4 *)(W32 + we + 4 * i);
           if (wtr) {
             put_rows();
             get_cols();
