@@ -221,9 +221,10 @@ class AdamW:
 
     def step(self, grads, stream_int, guard=None):
         self.launch(grads, stream_int, guard)
-        _lib.stream_sync(stream_int)                       # ancora/optim/adamw.py:98
         self.last_skipped = False
-        if guard is not None and guard.read(stream_int)["skip"]:
+        if guard is None:
+            _lib.stream_sync(stream_int)                   # ancora/optim/adamw.py:98
+        elif guard.read(stream_int)["skip"]:               # (synchronises)
             self.unstep()
             self.last_skipped = True
 

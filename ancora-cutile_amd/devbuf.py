@@ -9,6 +9,7 @@ Views share the pointer and are never freed (ancora/model/resident.py:80).
 bf16 data is held as uint16 bit patterns, as in the reference.
 """
 import ctypes as C
+import math
 
 import numpy as np
 
@@ -24,9 +25,9 @@ class DevBuf:
         if arr is not None:
             arr = np.ascontiguousarray(arr)
             shape, dtype = arr.shape, arr.dtype
-        self.shape = tuple(int(s) for s in shape)
-        self.dtype = np.dtype(dtype)
-        self.nbytes = int(np.prod(self.shape, dtype=np.int64)) * self.dtype.itemsize
+        self.shape = tuple(map(int, shape))
+        self.dtype = dtype = np.dtype(dtype)
+        self.nbytes = math.prod(self.shape) * dtype.itemsize
         if self.nbytes <= 0:
             raise ValueError(f"DevBuf: empty shape {self.shape}")
         self._owner = ptr is None
@@ -68,7 +69,7 @@ class DevBuf:
     def view(self, shape, dtype=None):
         """Same memory under another declared shape (and dtype); must fit inside this buffer."""
         dtype = self.dtype if dtype is None else np.dtype(dtype)
-        need = int(np.prod(shape, dtype=np.int64)) * dtype.itemsize
+        need = math.prod(map(int, shape)) * dtype.itemsize
         if need > self.nbytes:
             raise ValueError(f"DevBuf.view: {shape} {dtype} needs {need} B, buffer has {self.nbytes} B")
         return DevBuf(shape=shape, dtype=dtype, ptr=self.ptr)

@@ -93,29 +93,65 @@ _blocks = _Blocks()
 trim_pool = _blocks.trim
 
 
+class _GroupArray(DevBuf):
+    """One of the group arrays. Its address is the caller's to use on any stream, so asking for it waits until the
+    arrays are in place; the library's own launches on the stream they were sent on need not wait."""
+
+    def __init__(self, owner, row):
+        self.owner, self.row = owner, row
+        self.shape, self.dtype, self.nbytes, self._owner = (owner.M, 1), np.dtype(np.int32), 4 * owner.M, False
+
+    @property
+    def ptr(self):
+        return self.owner.settled() + self.row * self.nbytes
+
+    def ptr_on(self, si):
+        return self.owner.base_on(si) + self.row * self.nbytes
+
+    def free(self):
+        pass
+
+
 class IdGroups:
-    """The four group arrays on the device, plus the number of distinct ids."""
+    """The four group arrays, plus the number of distinct ids. They travel to the device with the first
+    launch that uses them, in its stream's order."""
 
     def __init__(self, ids_flat):
         _lib.init()
         self._arrays, self.n_groups = _id_groups(ids_flat)
-        self.M = M = self._arrays.shape[1]
-        self._block = _blocks.get(self._arrays.nbytes)
-        api.anc_upload_now(self._block.ptr, self._arrays.ctypes.data, self._arrays.nbytes)
-        self.srt, self.start, self.cnt, self.gid = (
-            DevBuf(shape=(M, 1), dtype=np.int32, ptr=self._block.ptr + i * 4 * M) for i in range(4))
+        self.M = self._arrays.shape[1]
+        self._block, self._si, self._settled = None, None, False
+        self.srt, self.start, self.cnt, self.gid = (_GroupArray(self, i) for i in range(4))
 
     @property
     def host(self):
         """The arrays as `build_id_groups` returns them."""
         return tuple(a.reshape(-1, 1) for a in self._arrays)
 
+    def base_on(self, si):
+        """Device address of the arrays for work queued on stream `si`."""
+        if self._block is None:
+            self._block, self._si = _blocks.get(self._arrays.nbytes), si
+            api.anc_upload_async(self._block.ptr, self._arrays.ctypes.data, self._arrays.nbytes, int(si))
+        elif self._si != si:
+            return self.settled()
+        return self._block.ptr
+
+    def settled(self):
+        """Device address of the arrays, in place for any stream."""
+        if not self._settled:
+            if self._block is None:
+                self._block = _blocks.get(self._arrays.nbytes)
+                api.anc_upload_now(self._block.ptr, self._arrays.ctypes.data, self._arrays.nbytes)
+            else:
+                _lib.stream_sync(self._si)
+            self._settled = True
+        return self._block.ptr
+
     def free(self):
         if self._block is not None:
             _blocks.put(self._block)
-            self._block = None
-        for b in (self.srt, self.start, self.cnt, self.gid):
-            b.ptr = 0
+            self._block, self._settled = None, False
 
 
 def embed_dw_scatter(groups, dy, si, out=None, compact=None, V=None):
@@ -124,7 +160,8 @@ def embed_dw_scatter(groups, dy, si, out=None, compact=None, V=None):
     M, H = dy.shape
     if out is not None:
         V = out.shape[0] if V is None else V
-    api.anc_embed_dw_scatter(groups.cnt.ptr, groups.start.ptr, groups.gid.ptr, groups.srt.ptr, dy.ptr,
+    base, step = groups.base_on(si), 4 * groups.M          # srt, start, cnt, gid
+    api.anc_embed_dw_scatter(base + 2 * step, base + step, base + 3 * step, base, dy.ptr,
                              0 if out is None else out.ptr, 0 if compact is None else compact.ptr,
                              M, 0 if V is None else V, H, int(si))
 
@@ -228,11 +265,11 @@ class RowSparseAdamW:
         self._ensure_step(self.t + 1, si)
         self.t += 1
         if n_groups > 0:
-            self._launch(gid.ptr, int(n_groups), grads.ptr, self.t, 0 if guard is None else guard.ptr, si)
+            rows = gid.ptr_on(si) if isinstance(gid, _GroupArray) else gid.ptr
+            self._launch(rows, int(n_groups), grads.ptr, self.t, 0 if guard is None else guard.ptr, si)
         self.last_skipped = False
         if guard is not None:
-            _lib.stream_sync(si)
-            if guard.read(si)["skip"]:
+            if guard.read(si)["skip"]:             # (synchronises)
                 self.t -= 1
                 self.last_skipped = True
 

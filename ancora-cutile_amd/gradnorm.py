@@ -37,6 +37,7 @@ class StepGuard:
         self._tables = {}
         self._part0 = []
         self._key = None
+        self._host = None
 
     @property
     def ptr(self):
@@ -75,7 +76,7 @@ class StepGuard:
         count `t` unless the step is skipped (for update kernels that take their per-step scalars
         from it). Asynchronous."""
         self.plan(grads)
-        produced = tuple(sorted(set(int(i) for i in produced)))
+        produced = tuple(sorted(set(int(i) for i in produced))) if produced else ()
         if produced not in self._tables:
             descs, chunk0 = [], 0
             for i, g in enumerate(grads):
@@ -92,8 +93,11 @@ class StepGuard:
 
     def read(self, stream=0):
         """Synchronise and return the control block as a dict."""
-        raw = self.ctl.to_numpy(stream)
-        c = StepCtl.from_buffer_copy(raw.tobytes())
+        if self._host is None:                   # pinned: a pageable read-back of 32 bytes takes twice as long
+            self._host = C.c_void_p()
+            api.anc_host_alloc(C.byref(self._host), C.sizeof(StepCtl))
+        api.anc_memcpy_d2h(self._host, self.ctl.ptr, C.sizeof(StepCtl), int(stream))
+        c = StepCtl.from_address(self._host.value)
         return {"sumsq": c.sumsq, "norm": c.norm, "clip_scale": c.clip_scale, "skip": bool(c.skip),
                 "t": int(c.t)}
 
@@ -107,3 +111,6 @@ class StepGuard:
     def free(self):
         self._free_tables()
         self.ctl.free()
+        if self._host is not None:
+            api.anc_host_free(self._host)
+            self._host = None

@@ -15,6 +15,7 @@ caller that must launch weight by weight can opt into `segments` (an int, "shape
 deterministic split of the token axis whose number of pieces then enters the bits.
 """
 import ctypes
+import struct
 
 import numpy as np
 
@@ -23,6 +24,8 @@ from ._lib import api, DwProblem
 from .devbuf import DevBuf
 
 MAX_PER_CALL = 8
+_DW = struct.Struct("=5Q4q2iQ2i")          # anc_dw_problem_t
+assert _DW.size == ctypes.sizeof(DwProblem)
 
 
 def dw_workspace_bytes(T, K, N):
@@ -91,13 +94,13 @@ def gemm_dW(problems, si=0, segments=None):
                     and tmin // (fill * 2) >= 256:
                 fill *= 2
         arr = (DwProblem * len(group))()
+        default = fill or (None if segments == "fill" else segments) or 1
         for k, p in enumerate(group):
-            T, K, N = int(p["T"]), int(p["K"]), int(p["N"])
-            S = p.get("segments") or fill or (None if segments == "fill" else segments) or 1
+            T, K, N = p["T"], p["K"], p["N"]
+            S = p.get("segments") or default
             if S == "shape":
                 S = dw_info(T, K, N)[1]
-            S = int(S)
-            gn = int(p.get("gn_partials") or 0)
+            gn = p.get("gn_partials") or 0
             if S == 1 and gn == 0:                 # finished by the GEMM's epilogue: no partial tiles
                 ws_ptr = ws_bytes = 0
             else:
@@ -105,7 +108,8 @@ def gemm_dW(problems, si=0, segments=None):
                 ws_ptr, ws_bytes = ws.ptr, ws.nbytes
             g16 = p.get("g16")
             x = p.get("x")
-            arr[k] = DwProblem((p["xT"] if x is None else x).ptr, p["dy"].ptr, p["dW"].ptr,
-                               0 if g16 is None else g16.ptr, ws_ptr, T, K, N, ws_bytes,
-                               int(bool(p.get("accumulate", False))), S, gn, 0 if x is None else 1, 0)
+            # (packed straight into the array: field by field it was most of a small call's time)
+            _DW.pack_into(arr, k * _DW.size, (p["xT"] if x is None else x).ptr, p["dy"].ptr, p["dW"].ptr,
+                          0 if g16 is None else g16.ptr, ws_ptr, T, K, N, ws_bytes,
+                          1 if p.get("accumulate", False) else 0, S, gn, 0 if x is None else 1, 0)
         api.anc_gemm_dw_multi(arr, len(group), int(si))

@@ -639,9 +639,10 @@ class Muon:
 
     def step(self, grads, stream_int=None, guard=None):
         si = self.launch(grads, stream_int, guard)
-        _lib.stream_sync(si)
         self.last_skipped = False
-        if guard is not None and guard.read(si)["skip"]:
+        if guard is None:
+            _lib.stream_sync(si)
+        elif guard.read(si)["skip"]:                           # (synchronises)
             self.unstep()
             self.last_skipped = True
 
