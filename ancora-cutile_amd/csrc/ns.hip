@@ -729,11 +729,12 @@ struct ChainProb {
 // (a launch ends with its longest tiles; short ones fill gaps). A CU takes operand bytes into LDS at one
 // rate whatever the tile, so small tiles finish first while they find idle CUs and lose, by the bytes they
 // fetch more often, once every CU has several. Measured, us per 5 launches on 64 / 128 / 256-wide tiles:
-//   A = X X^T   8 x (512,512) 87 / 120 / 196 (384 tiles of 64), 4 x (1024,1024) 134 / 131 / 195 (640),
-//               8 x (1024,1024) 196 / 182 / 202 (320 of 128), 16 x (1024,1024) 335 / 306 / 237 (640)
-//   X = a X + B X   1 x (1024,3072) 107 / 110 / 142 (768 of 64), 4 x (512,1536) 118 / 120 / 157 (768),
-//               8 x (512,1536) 192 / 164 / 162 (384 of 128), 8 x (1024,2048) 385 / 280 / 247 (1024)
-// hence 64 below 600 (symmetric) or 768 tiles of 64, 128 below 400 tiles of 128.
+//   A = X X^T   16 x (512,512) 114 / 121 / 199 (768 tiles of 64), 5 x (1024,1024) 138 / 130 / 197 (800),
+//               4 x (1280,2560) 205 / 177 / 283 (960), 12 x (1024,1024) 240 / 211 / 210 (1920),
+//               16 x (1024,1024) 295 / 286 / 228 (2560)
+//   X = a X + B X   6 x (512,1536) 131 / 147 / 172 (1152), 2 x (1024,3072) 158 / 145 / 152 (1536),
+//               8 x (1024,1024) 210 / 179 / 179 (2048), 3 x (1024,3072) 218 / 212 / 197 (2304)
+// hence 64 below 800 (symmetric) or 1400 tiles of 64, 128 below 2000.
 int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
@@ -742,8 +743,8 @@ int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
     const double per = epi == EPI_BX ? m * (double)(ps[k].N / 64) : m * (m + d) / 2.0;
     t64 += (double)Es[k] * per * ((double)ps[k].K / longest);
   }
-  if (t64 < (epi == EPI_BX ? 768.0 : 600.0)) return 64;
-  return t64 < 1600.0 ? 128 : 256;
+  if (t64 < (epi == EPI_BX ? 1400.0 : 800.0)) return 64;
+  return t64 < 2000.0 ? 128 : 256;
 }
 
 // What a mode's tile flags ask for (0: nothing).

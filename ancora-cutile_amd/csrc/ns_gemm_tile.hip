@@ -11,11 +11,14 @@
 //
 // Layout. 4 wavefronts as 2x2, each WB x WB blocks of v_mfma_f32_32x32x16_bf16 (tile 64 WB). A stage is 16 KiB,
 // one half per operand: KP = 2 (64x64) or 1 (128x128) panels of 32 k. Operands arrive in pieces of 16 rows x
-// 64 bytes, one LDS-DMA instruction each, four per wavefront and stage; stages form a ring of four,
-// two workgroups per CU. An operand whose rows are tile rows ("NT") lies in LDS as [panel][row][64 bytes] with the
-// 16-byte chunk index XORed with bits 2..3 of the row; an operand whose rows are k (the iterate in X = a X +
-// B X, its symmetric B from M = 1024 on, activations and output gradients) lies as [32-column block][k][64
-// bytes] without a swizzle: a transposing read touches 4 rows x 64 contiguous bytes, all banks once.
+// 64 bytes, one LDS-DMA instruction each, four per wavefront and stage. Stages form a ring of four, two
+// workgroups per CU; 64x64 tiles that outnumber the CUs run on a ring of three, three workgroups per CU, whose
+// K loops and epilogues overlap (chains of five steps: 16 x (512,512) 358 -> 331 us, 4 x (1024,3072) 625 ->
+// 570 us; a single (512,1536), one workgroup per CU, loses 3 % to the shorter ring).
+// An operand whose rows are tile rows ("NT") lies in LDS as [panel][row][64 bytes] with the 16-byte chunk index
+// XORed with bits 2..3 of the row; an operand whose rows are k (the iterate in X = a X + B X, its symmetric B
+// from M = 1024 on, activations and output gradients) lies as [32-column block][k][64 bytes] without a swizzle:
+// a transposing read touches 4 rows x 64 contiguous bytes, all banks once.
 // In panel layout both are contiguous in memory as well.
 //
 // Epilogue: block by block through a 32x36 fp32 buffer of the wavefront, so that a lane holds 16
@@ -32,11 +35,11 @@
 
 namespace {
 
-constexpr int kRing = 4, kStageBytes = 16384, kIps = 4;   // stages, their size, DMA instructions per wavefront and stage
+constexpr int kStageBytes = 16384, kIps = 4;              // a stage, DMA instructions per wavefront and stage
 constexpr int kSgPitch = 36;                              // floats per row of the epilogue buffer
 
-template <int EPI, int WB, bool AT, int VAR>
-__global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
+template <int EPI, int WB, bool AT, int VAR, int kRing>
+__global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemmMulti pm) {
   constexpr int TM = 64 * WB, KP = WB == 1 ? 2 : 1, TK = 32 * KP;
   constexpr bool BT = EPI == EPI_BX, PLAINV = VAR == VAR_PLAIN;
   constexpr int kHalf = TM * TK * 2;
@@ -189,8 +192,8 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
         acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bj], a[bi], acc[bi][bj], 0, 0, 0);
   };
 
-  // ---- K loop, one term. Step k lives in stage k % 4. At its top a wavefront waits for its own DMA of the step (two
-  // younger ones stay in flight), the workgroup meets, and the DMA of step k + 3 goes out into the stage
+  // ---- K loop, one term. Step k lives in stage k % kRing. At its top a wavefront waits for its own DMA of the step (the
+  // younger ones stay in flight), the workgroup meets, and the DMA of step k + kRing - 1 goes out into the stage
   // everybody has just left.
   if (PLAINV || nterms == 1) {
 #pragma unroll
@@ -220,7 +223,7 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
     }
   } else {
     // ---- several terms: a step is one panel of 32 k of both halves of both operands, high stage then low stage.
-    constexpr int kPan = TM * 64, kPair = 4 * kPan, kPairs = kRing * kStageBytes / kPair;   // 4 (64) or 2 (128) steps in the ring
+    constexpr int kPan = TM * 64, kPair = 4 * kPan, kPairs = kRing * kStageBytes / kPair;   // 4, 3 (64) or 2 (128) steps in the ring
     int64_t oA[WB], oB[WB];
 #pragma unroll
     for (int j = 0; j < WB; ++j) {
@@ -521,8 +524,9 @@ __global__ void __launch_bounds__(256, 2) k_ns_gemm_tile(NsGemmMulti pm) {
 
 template <int EPI, bool AT, int VAR>
 void launch_tile(bool small, unsigned grid, hipStream_t s, const NsGemmMulti &pm) {
-  if (small) hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR>), dim3(grid), dim3(256), 0, s, pm);
-  else       hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, AT, VAR>), dim3(grid), dim3(256), 0, s, pm);
+  if (!small)           hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, AT, VAR, 4>), dim3(grid), dim3(256), 0, s, pm);
+  else if (grid <= 256) hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 4>), dim3(grid), dim3(256), 0, s, pm);
+  else                  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 3>), dim3(grid), dim3(256), 0, s, pm);
 }
 
 }  // namespace

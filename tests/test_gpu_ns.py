@@ -192,6 +192,19 @@ def test_tile_choice_keeps_the_bits(gpu, M, N, mode):
     assert rel_fro(want[0], host_ns(X[0], PE_SCHEDULE, 5)) < TOL_BF16
 
 
+@pytest.mark.parametrize("E,M,N", [(86, 128, 128), (64, 128, 256), (65, 128, 256), (26, 256, 384)])
+@pytest.mark.parametrize("mode", ["bf16", "bf16_x3"])
+def test_many_small_tiles_keep_the_bits(gpu, E, M, N, mode):
+    """64x64 tiles that outnumber the CUs run on a shorter ring of stages: counts on both sides of that line,
+    with K of two to six stages. Every matrix has the bits it has alone."""
+    rng = np.random.default_rng(E + M + N)
+    X = rng.standard_normal((E, M, N)).astype(np.float32)
+    X[E - 1][:, :2] *= 100.0
+    got = run_ns(X, mode=mode)
+    for e in (0, E // 2, E - 1):
+        assert bits_equal(got[e], run_ns(X[e: e + 1], mode=mode)[0]), e
+
+
 @pytest.mark.parametrize("E,M,N", [(1, 128, 128), (3, 128, 384), (2, 256, 512), (1, 640, 768), (2, 1024, 1024), (2, 1024, 2048)])
 @pytest.mark.parametrize("sched", ["pe", "keller"])
 def test_bf16_entry_takes_the_matrix_as_it_is(gpu, E, M, N, sched):
