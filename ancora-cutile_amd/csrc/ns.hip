@@ -734,8 +734,15 @@ struct ChainProb {
 //               16 x (1024,1024) 295 / 286 / 228 (2560)
 //   X = a X + B X   6 x (512,1536) 131 / 147 / 172 (1152), 2 x (1024,3072) 158 / 145 / 152 (1536),
 //               8 x (1024,1024) 210 / 179 / 179 (2048), 3 x (1024,3072) 218 / 212 / 197 (2304)
-// hence 64 below 800 (symmetric) or 1400 tiles of 64, 128 below 2000.
-int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
+// hence 64 below 800 (symmetric) or 1400 tiles of 64, 128 up to 2000. The bare product's K is a batch of tokens,
+// up to 8192, and its operands leave the L2: weight gradients at 512 / 2048 / 8192 tokens on the three tiles,
+//   432 tiles of 64    11.3 21.1 65 / 13.9 28.2 80 / 16.5 33.9 97
+//   768                15.2 31.5 117 / 16.3 31.5 88 / 18.3 35.8 101
+//   1024               18.3 38.5 146 / 17.8 34.2 93 / 19.0 38.2 105
+//   1248               22.3 47.9 194 / 23.4 49.1 127 / 21.5 40.3 105
+// hence 64 below 768 and 128 up to one tile of 128 per CU: 1056 tiles of 64, 8 CUs with two of 128 each, take
+// 55 against 43 us at 3360 tokens.
+int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n, bool plain = false) {
   double longest = 0.0, t64 = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
   for (int k = 0; k < n; ++k) {
@@ -743,8 +750,8 @@ int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
     const double per = epi == EPI_BX ? m * (double)(ps[k].N / 64) : m * (m + d) / 2.0;
     t64 += (double)Es[k] * per * ((double)ps[k].K / longest);
   }
-  if (t64 < (epi == EPI_BX ? 1400.0 : 800.0)) return 64;
-  return t64 < 2000.0 ? 128 : 256;
+  if (t64 < (plain ? 768.0 : epi == EPI_BX ? 1400.0 : 800.0)) return 64;
+  return t64 <= (plain ? 1024.0 : 2000.0) ? 128 : 256;
 }
 
 // What a mode's tile flags ask for (0: nothing).
@@ -977,7 +984,7 @@ int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int f
 
 int anc_ns_gemm_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool a_transposed) {
   ANC_REQUIRE(n >= 1 && n <= kMaxGroups, "anc_ns_gemm_plain: 1..%d problems per launch", kMaxGroups);
-  const int tile = pick_tile(EPI_BX, ps, Es, n);
+  const int tile = pick_tile(EPI_BX, ps, Es, n, true);
   if (tile == 256) return anc_ns_gemm_big_plain(ps, Es, n, s, a_transposed);
   return anc_ns_gemm_tile_multi(EPI_BX, ps, Es, n, s, tile == 64, a_transposed, nullptr, true);
 }

@@ -38,6 +38,20 @@ namespace {
 constexpr int kStageBytes = 16384, kIps = 4;              // a stage, DMA instructions per wavefront and stage
 constexpr int kSgPitch = 36;                              // floats per row of the epilogue buffer
 
+// BYTES (4, 8 or 16) between memory and registers, one instruction.
+template <int BYTES>
+__device__ __forceinline__ void ld_run(const void *p, uint32_t *w) {
+  if constexpr (BYTES == 16) { const anc_u32x4 t = *(const anc_u32x4 *)p; w[0] = t.x; w[1] = t.y; w[2] = t.z; w[3] = t.w; }
+  else if constexpr (BYTES == 8) { const anc_u32x2 t = *(const anc_u32x2 *)p; w[0] = t.x; w[1] = t.y; }
+  else w[0] = *(const uint32_t *)p;
+}
+template <int BYTES>
+__device__ __forceinline__ void st_run(void *p, const uint32_t *w) {
+  if constexpr (BYTES == 16) *(anc_u32x4 *)p = anc_u32x4{w[0], w[1], w[2], w[3]};
+  else if constexpr (BYTES == 8) *(anc_u32x2 *)p = anc_u32x2{w[0], w[1]};
+  else *(uint32_t *)p = w[0];
+}
+
 template <int EPI, int WB, bool AT, int VAR, int kRing>
 __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemmMulti pm) {
   constexpr int TM = 64 * WB, KP = WB == 1 ? 2 : 1, TK = 32 * KP;
@@ -142,38 +156,54 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   const bool has_a32 = EPI != EPI_BX && anc_ns_has_a32(p, e);
   const bool in8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_in);
   const bool out8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_out);
-  const int row = lane >> 1, c0 = (lane & 1) * 16;      // this lane's 16 elements of a block: row `row`, columns c0 ..
-                                                        // (or, reading the block transposed, column `row`, rows c0 ..)
+  // This lane's 16 elements of a 32x32 block: NR runs of RUN consecutive columns (reading the block transposed, rows),
+  // run r in row lrow + RS r from column c0. 32/RUN neighbouring lanes share a row, so that one instruction covers
+  // whole lines.
+  constexpr int RUN = (PLAINV || VAR == VAR_UPDATE) ? 4 : 8, NR = 16 / RUN, LPR = 32 / RUN, RS = 64 / LPR;
+  const int lrow = lane / LPR, c0 = (lane % LPR) * RUN;
   const int gi_w = tm * TM + wm * (32 * WB), gj_w = tn * TM + wn * (32 * WB);
-  // this lane's 16 elements of block b in a matrix of M rows in panel layout
-  auto pan_of = [&](int b) { return ((int64_t)((gj_w + (b % WB) * 32) / 32) * M + gi_w + (b / WB) * 32 + row) * 32 + c0; };
+  // run 0 of block b in a matrix of M rows in panel layout (run r: RS * 32 r further)
+  auto pan_of = [&](int b) { return ((int64_t)((gj_w + (b % WB) * 32) / 32) * M + gi_w + (b / WB) * 32 + lrow) * 32 + c0; };
   constexpr int NB = WB * WB;
-  anc_u32x4 pre[NB][4];
-  float drow[WB];
+  uint32_t pre_h[NB][8], pre_l[NB][8];                  // 16 bf16, or (pre_l, 8-bit low halves) 16 bytes in the first 4
+  float drow[WB][NR];
   if constexpr (EPI == EPI_BX && !PLAINV) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int64_t xo = mn + (p.x_panel ? pan_of(b) : (int64_t)(gi_w + (b / WB) * 32 + row) * N + gj_w + (b % WB) * 32 + c0);
-      pre[b][0] = *(const anc_u32x4 *)(p.Xh + xo);
-      pre[b][1] = *(const anc_u32x4 *)(p.Xh + xo + 8);
+      const int64_t xo = mn + (p.x_panel ? pan_of(b) : (int64_t)(gi_w + (b / WB) * 32 + lrow) * N + gj_w + (b % WB) * 32 + c0);
+      const int64_t xr = p.x_panel ? RS * 32 : (int64_t)RS * N;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) ld_run<RUN * 2>(p.Xh + xo + r * xr, &pre_h[b][r * (RUN / 2)]);
       if (in8) {
-        pre[b][2] = *(const anc_u32x4 *)((const char *)p.Xl + mn * 2 + pan_of(b));
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          ld_run<RUN>((const char *)p.Xl + mn * 2 + pan_of(b) + r * RS * 32, &pre_l[b][r * (RUN / 4)]);
       } else if (!p.lo_zero) {
-        pre[b][2] = *(const anc_u32x4 *)(p.Xl + xo);
-        pre[b][3] = *(const anc_u32x4 *)(p.Xl + xo + 8);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) ld_run<RUN * 2>(p.Xl + xo + r * xr, &pre_l[b][r * (RUN / 2)]);
       }
     }
 #pragma unroll
-    for (int bi = 0; bi < WB; ++bi) drow[bi] = p.dB[mv + gi_w + bi * 32 + row];
+    for (int bi = 0; bi < WB; ++bi)
+#pragma unroll
+      for (int r = 0; r < NR; ++r) drow[bi][r] = p.dB[mv + gi_w + bi * 32 + lrow + RS * r];
   }
-  // (the master's block too where registers allow: one block per wavefront)
+  // (the master's block, or what the plain product adds to, too where registers allow: one block per wavefront)
+  const bool plain_add = PLAINV && p.plain_sum && p.A32 != nullptr;
   anc_f32x4 wpre[4];
   if constexpr (VAR == VAR_UPDATE && WB == 1) {
     const anc_muon_desc_t &d = p.upd[e];
     const bool wtr = d.transpose != 0;
-    const int64_t we = (int64_t)((wtr ? gj_w : gi_w) + row) * d.N + (wtr ? gi_w : gj_w) + c0;
+    const int64_t we = (int64_t)((wtr ? gj_w : gi_w) + lrow) * d.N + (wtr ? gi_w : gj_w) + c0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wpre[i] = *(const anc_f32x4 *)((const float *)d.p32 + we + 4 * i);
+    for (int r = 0; r < 4; ++r) wpre[r] = *(const anc_f32x4 *)((const float *)d.p32 + we + (int64_t)r * RS * d.N);
+  }
+  if constexpr (PLAINV && WB == 1) {
+    if (plain_add) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        wpre[r] = *(const anc_f32x4 *)(p.A32 + mn + (int64_t)(gi_w + lrow + RS * r) * N + gj_w + c0);
+    }
   }
 
   f32x16 acc[WB][WB];
@@ -293,32 +323,31 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const anc_f32x4 w = {v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
-      *(anc_f32x4 *)(sg + row * kSgPitch + c0 + 4 * i) = w;
+      *(anc_f32x4 *)(sg + (lrow + RS * (4 * i / RUN)) * kSgPitch + c0 + 4 * i % RUN) = w;
     }
     lds_wave_sync();
   };
   auto get_cols = [&]() {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = sg[(c0 + i) * kSgPitch + row];
+    for (int i = 0; i < 16; ++i) v[i] = sg[(c0 + i % RUN) * kSgPitch + lrow + RS * (i / RUN)];
   };
-  auto unpack = [&](const anc_u32x4 &w, float *x) {
-    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+  auto unpack = [&](const uint32_t (&u)[8], float (&x)[16]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) { x[2 * i] = __uint_as_float(u[i] << 16); x[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u); }
+    for (int i = 0; i < 8; ++i) { x[2 * i] = __uint_as_float(u[i] << 16); x[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u); }
   };
-  // 16 floats -> 16 bf16 at out (32 bytes), and the residuals at lo if not null
-  auto put_bf16 = [&](uint16_t *out, uint16_t *lo) {
+  // 16 floats -> bf16 runs at out + r * step, and the residuals at lo likewise if not null
+  auto put_bf16 = [&](uint16_t *out, uint16_t *lo, int64_t step) {
     uint32_t h[8], l[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       if (lo != nullptr) anc_pk_pair(v[2 * i], v[2 * i + 1], h[i], l[i]);
       else h[i] = anc_pk_bf16(v[2 * i], v[2 * i + 1]);
     }
-    *(anc_u32x4 *)out = anc_u32x4{h[0], h[1], h[2], h[3]};
-    *(anc_u32x4 *)(out + 8) = anc_u32x4{h[4], h[5], h[6], h[7]};
+#pragma unroll
+    for (int r = 0; r < NR; ++r) st_run<RUN * 2>(out + r * step, h + r * (RUN / 2));
     if (lo != nullptr) {
-      *(anc_u32x4 *)lo = anc_u32x4{l[0], l[1], l[2], l[3]};
-      *(anc_u32x4 *)(lo + 8) = anc_u32x4{l[4], l[5], l[6], l[7]};
+#pragma unroll
+      for (int r = 0; r < NR; ++r) st_run<RUN * 2>(lo + r * step, l + r * (RUN / 2));
     }
   };
 #pragma unroll
@@ -326,8 +355,16 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 #pragma unroll
     for (int bj = 0; bj < WB; ++bj) {
       const int gi0 = gi_w + bi * 32, gj0 = gj_w + bj * 32;
-      const int gi = gi0 + row, gj = gj0 + c0;
-      const int64_t pan = pan_of(bi * WB + bj);
+      const int gi = gi0 + lrow, gj = gj0 + c0;
+      const int64_t pan = pan_of(bi * WB + bj), pst = RS * 32;
+      // four consecutive columns from column gj + 4 i % RUN of row gi + RS (4 i / RUN), in a matrix with `pitch` columns
+      auto quad = [&](int i, int64_t pitch) { return (int64_t)(gi + RS * (4 * i / RUN)) * pitch + gj + 4 * i % RUN; };
+      if constexpr (PLAINV && WB > 1) {
+        if (plain_add) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) wpre[i] = *(const anc_f32x4 *)(p.A32 + mn + quad(i, N));
+        }
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const anc_f32x4 w = {acc[bi][bj][4 * q], acc[bi][bj][4 * q + 1], acc[bi][bj][4 * q + 2], acc[bi][bj][4 * q + 3]};
@@ -336,115 +373,113 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
       lds_wave_sync();
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const anc_f32x4 w = *(const anc_f32x4 *)(sg + row * kSgPitch + c0 + 4 * i);
+        const anc_f32x4 w = *(const anc_f32x4 *)(sg + (lrow + RS * (4 * i / RUN)) * kSgPitch + c0 + 4 * i % RUN);
         v[4 * i] = w.x; v[4 * i + 1] = w.y; v[4 * i + 2] = w.z; v[4 * i + 3] = w.w;
       }
       lds_wave_sync();                       // the buffer is free again
       if constexpr (EPI != EPI_BX) {
-        const bool diag = gi0 == gj0;        // the block on the diagonal: element k = row - c0 of this lane
+        const bool diag = gi0 == gj0;        // a block on the diagonal: element k's row and column may be the same
         if (EPI == EPI_GRAM) {
 #pragma unroll
           for (int k = 0; k < 16; ++k) v[k] = v[k] * acc_scale;
           if (has_a32) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-              *(anc_f32x4 *)(p.A32 + mm + (int64_t)gi * M + gj + 4 * i) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+              *(anc_f32x4 *)(p.A32 + mm + quad(i, M)) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
           }
           if (diag) {
 #pragma unroll
             for (int k = 0; k < 16; ++k)
-              if (row == c0 + k) { p.dA[mv + gi] = v[k]; v[k] = 0.0f; }
+              if (lrow + RS * (k / RUN) == c0 + k % RUN) { p.dA[mv + gj + k % RUN] = v[k]; v[k] = 0.0f; }
           }
         } else {
           float a[16];
           if (has_a32) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const anc_f32x4 w = *(const anc_f32x4 *)(p.A32 + mm + (int64_t)gi * M + gj + 4 * i);
+              const anc_f32x4 w = *(const anc_f32x4 *)(p.A32 + mm + quad(i, M));
               a[4 * i] = w.x; a[4 * i + 1] = w.y; a[4 * i + 2] = w.z; a[4 * i + 3] = w.w;
             }
           } else {
-            unpack(*(const anc_u32x4 *)(p.Fh + mm + pan), a);
-            unpack(*(const anc_u32x4 *)(p.Fh + mm + pan + 8), a + 8);
+            uint32_t u[8];
+#pragma unroll
+            for (int r = 0; r < NR; ++r) ld_run<RUN * 2>(p.Fh + mm + pan + r * pst, u + r * (RUN / 2));
+            unpack(u, a);
           }
-          const float di = p.dA[mv + gi];
+          float dj[RUN];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const anc_f32x4 dj = *(const anc_f32x4 *)(p.dA + mv + gj + 4 * i);
-            const float d[4] = {dj.x, dj.y, dj.z, dj.w};
+          for (int i = 0; i < RUN; i += 4) {
+            const anc_f32x4 w = *(const anc_f32x4 *)(p.dA + mv + gj + i);
+            dj[i] = w.x; dj[i + 1] = w.y; dj[i + 2] = w.z; dj[i + 3] = w.w;
+          }
 #pragma unroll
-            for (int k4 = 0; k4 < 4; ++k4) {
-              const int k = 4 * i + k4;
-              if (diag && row == c0 + k) {
+          for (int r = 0; r < NR; ++r) {
+            const float di = p.dA[mv + gi + RS * r];
+#pragma unroll
+            for (int c = 0; c < RUN; ++c) {
+              const int k = r * RUN + c;
+              if (diag && lrow + RS * r == c0 + c) {
                 const float a2 = v[k] + di * di;
-                p.dB[mv + gi] = p.cb * di + p.cc * a2;
+                p.dB[mv + gj + c] = p.cb * di + p.cc * a2;
                 v[k] = 0.0f;
               } else {
-                const float a2 = v[k] + (di * a[k] + a[k] * d[k4]);   // symmetric in (i,j)
+                const float a2 = v[k] + (di * a[k] + a[k] * dj[c]);   // symmetric in (i,j)
                 v[k] = p.cb * a[k] + p.cc * a2;
               }
             }
           }
         }
         uint16_t *oh = EPI == EPI_GRAM ? p.Fh : p.Bh, *ol = EPI == EPI_GRAM ? p.Fl : p.Bl;
-        put_bf16(oh + mm + pan, write_lo ? ol + mm + pan : nullptr);
+        put_bf16(oh + mm + pan, write_lo ? ol + mm + pan : nullptr, pst);
         if (tm / p.blk_r != tn / p.blk_r) {  // mirror image: rows gj0 .., 32-column panel gi0/32
           put_rows();
           get_cols();
-          const int64_t pt = ((int64_t)(gi0 / 32) * M + gj0 + row) * 32 + c0;
-          put_bf16(oh + mm + pt, write_lo ? ol + mm + pt : nullptr);
+          const int64_t pt = ((int64_t)(gi0 / 32) * M + gj0 + lrow) * 32 + c0;
+          put_bf16(oh + mm + pt, write_lo ? ol + mm + pt : nullptr, pst);
           lds_wave_sync();
         }
       } else if constexpr (PLAINV) {
-        const int64_t o = mn + (int64_t)gi * N + gj;
-        if (p.plain_sum && p.A32 != nullptr) {
+        if (p.plain_sum) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const anc_f32x4 w = *(const anc_f32x4 *)(p.A32 + o + 4 * i);
+            const anc_f32x4 w = plain_add ? wpre[i] : anc_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             v[4 * i] = w.x + v[4 * i]; v[4 * i + 1] = w.y + v[4 * i + 1];
             v[4 * i + 2] = w.z + v[4 * i + 2]; v[4 * i + 3] = w.w + v[4 * i + 3];
           }
-        } else if (p.plain_sum) {
-#pragma unroll
-          for (int k = 0; k < 16; ++k) v[k] = 0.0f + v[k];
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          *(anc_f32x4 *)(p.X32 + o + 4 * i) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+        for (int i = 0; i < 4; ++i) {
+          const anc_f32x4 w = {v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+          __builtin_nontemporal_store(w, (anc_f32x4 *)(p.X32 + mn + quad(i, N)));
+        }
         if (p.plain_sum && p.Yh != nullptr) {
-          uint32_t h[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) h[i] = (anc_bf16_rne_bits(v[2 * i]) & 0xFFFFu) | (anc_bf16_rne_bits(v[2 * i + 1]) << 16);
-          *(anc_u32x4 *)(p.Yh + o) = anc_u32x4{h[0], h[1], h[2], h[3]};
-          *(anc_u32x4 *)(p.Yh + o + 8) = anc_u32x4{h[4], h[5], h[6], h[7]};
+          for (int i = 0; i < 4; ++i) {
+            const anc_u32x2 h = {(anc_bf16_rne_bits(v[4 * i]) & 0xFFFFu) | (anc_bf16_rne_bits(v[4 * i + 1]) << 16),
+                                 (anc_bf16_rne_bits(v[4 * i + 2]) & 0xFFFFu) | (anc_bf16_rne_bits(v[4 * i + 3]) << 16)};
+            __builtin_nontemporal_store(h, (anc_u32x2 *)(p.Yh + mn + quad(i, N)));
+          }
         }
       } else {
         // y = (a + dB) x + B X. Only the first iteration carries the input's scale.
-        const anc_u32x4 (&in)[4] = pre[bi * WB + bj];
-        const float cf = p.ca + drow[bi];
         float x[16];
-        unpack(in[0], x);
-        unpack(in[1], x + 8);
+        unpack(pre_h[bi * WB + bj], x);
         if (in8) {
-          const uint32_t qq[4] = {in[2].x, in[2].y, in[2].z, in[2].w};
 #pragma unroll
           for (int k = 0; k < 16; ++k)
-            x[k] = anc_low8_decode(__float_as_uint(x[k]), (int)(qq[k >> 2] << (24 - 8 * (k & 3))) >> 24);
-        } else {
-          if (!p.lo_zero) {
-            float xl[16];
-            unpack(in[2], xl);
-            unpack(in[3], xl + 8);
+            x[k] = anc_low8_decode(__float_as_uint(x[k]), (int)(pre_l[bi * WB + bj][k >> 2] << (24 - 8 * (k & 3))) >> 24);
+        } else if (!p.lo_zero) {
+          float xl[16];
+          unpack(pre_l[bi * WB + bj], xl);
 #pragma unroll
-            for (int k = 0; k < 16; ++k) x[k] = x[k] + xl[k];
-          }
+          for (int k = 0; k < 16; ++k) x[k] = x[k] + xl[k];
         }
         if (p.scale != nullptr) {
 #pragma unroll
-          for (int k = 0; k < 16; ++k) v[k] = cf * (x[k] * sc) + v[k] * acc_scale;
+          for (int k = 0; k < 16; ++k) v[k] = (p.ca + drow[bi][k / RUN]) * (x[k] * sc) + v[k] * acc_scale;
         } else {
 #pragma unroll
-          for (int k = 0; k < 16; ++k) v[k] = cf * x[k] + v[k];
+          for (int k = 0; k < 16; ++k) v[k] = (p.ca + drow[bi][k / RUN]) * x[k] + v[k];
         }
         if constexpr (VAR == VAR_UPDATE) {
           // W -= lr O on the block's 32x32 elements of the weight (transposed where the chain ran on W^T)
@@ -455,55 +490,55 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
           const float wlr = pm.lr[d.scale_idx & (ANC_MUON_MAX_SCALES - 1)];
           const uint32_t wseed = pm.seed_base + d.seed + ((pm.sr & ANC_SR_STEP_SEED) ? ANC_SR_SEED_STRIDE * pm.ctl->t : 0u);
           const int wr0 = wtr ? gj0 : gi0, wc0 = wtr ? gi0 : gj0;
-          const int64_t we = (int64_t)(wr0 + row) * d.N + wc0 + c0;
+          const int64_t we = (int64_t)(wr0 + lrow) * d.N + wc0 + c0, wst = (int64_t)RS * d.N;
           anc_f32x4 pv[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) pv[i] = WB == 1 ? wpre[i] : *(const anc_f32x4 *)(W32 + we + 4 * i);
+          for (int r = 0; r < 4; ++r) pv[r] = WB == 1 ? wpre[r] : *(const anc_f32x4 *)(W32 + we + r * wst);
           if (wtr) {
             put_rows();
             get_cols();
             lds_wave_sync();
           }
-          uint32_t hb[16];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float pp[4] = {pv[i].x, pv[i].y, pv[i].z, pv[i].w};
-#pragma unroll
-            for (int k4 = 0; k4 < 4; ++k4) {
-              pp[k4] = pp[k4] - wlr * v[4 * i + k4];
-              const uint64_t el = (uint64_t)(we + 4 * i + k4);
-              hb[4 * i + k4] = ((pm.sr & ANC_SR_ON) ? anc_bf16_sr_bits(pp[k4], (uint32_t)(el >> 6), (uint32_t)(el & 63u), wseed)
-                                                    : anc_bf16_rne_bits(pp[k4])) & 0xFFFFu;
-            }
-            *(anc_f32x4 *)(W32 + we + 4 * i) = anc_f32x4{pp[0], pp[1], pp[2], pp[3]};
-          }
           uint32_t hw[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) hw[i] = hb[2 * i] | (hb[2 * i + 1] << 16);
+          for (int r = 0; r < 4; ++r) {
+            float pp[4] = {pv[r].x, pv[r].y, pv[r].z, pv[r].w};
+            uint32_t hb[4];
+#pragma unroll
+            for (int k4 = 0; k4 < 4; ++k4) {
+              pp[k4] = pp[k4] - wlr * v[4 * r + k4];
+              const uint64_t el = (uint64_t)(we + r * wst + k4);
+              hb[k4] = ((pm.sr & ANC_SR_ON) ? anc_bf16_sr_bits(pp[k4], (uint32_t)(el >> 6), (uint32_t)(el & 63u), wseed)
+                                            : anc_bf16_rne_bits(pp[k4])) & 0xFFFFu;
+            }
+            *(anc_f32x4 *)(W32 + we + r * wst) = anc_f32x4{pp[0], pp[1], pp[2], pp[3]};
+            hw[2 * r] = hb[0] | (hb[1] << 16);
+            hw[2 * r + 1] = hb[2] | (hb[3] << 16);
+          }
           if (W16 != nullptr) {
-            *(anc_u32x4 *)(W16 + we) = anc_u32x4{hw[0], hw[1], hw[2], hw[3]};
-            *(anc_u32x4 *)(W16 + we + 8) = anc_u32x4{hw[4], hw[5], hw[6], hw[7]};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) st_run<8>(W16 + we + r * wst, hw + 2 * r);
           }
           if (W16t != nullptr) {             // the (N, K) bf16 copy: the block's columns as rows
             uint16_t *sh = (uint16_t *)sg;   // [32][40]
-            *(anc_u32x4 *)(sh + row * 40 + c0) = anc_u32x4{hw[0], hw[1], hw[2], hw[3]};
-            *(anc_u32x4 *)(sh + row * 40 + c0 + 8) = anc_u32x4{hw[4], hw[5], hw[6], hw[7]};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) st_run<8>(sh + (lrow + RS * r) * 40 + c0, hw + 2 * r);
             lds_wave_sync();
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-              hw[i] = (uint32_t)sh[(c0 + 2 * i) * 40 + row] | ((uint32_t)sh[(c0 + 2 * i + 1) * 40 + row] << 16);
+            for (int i = 0; i < 8; ++i) {
+              const uint16_t *q = sh + (c0 + (2 * i) % RUN) * 40 + lrow + RS * (2 * i / RUN);
+              hw[i] = (uint32_t)q[0] | ((uint32_t)q[40] << 16);
+            }
             lds_wave_sync();
-            uint16_t *o = W16t + (int64_t)(wc0 + row) * d.K + wr0 + c0;
-            *(anc_u32x4 *)o = anc_u32x4{hw[0], hw[1], hw[2], hw[3]};
-            *(anc_u32x4 *)(o + 8) = anc_u32x4{hw[4], hw[5], hw[6], hw[7]};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) st_run<8>(W16t + (int64_t)(wc0 + lrow + RS * r) * d.K + wr0 + c0, hw + 2 * r);
           }
         } else if (p.X32 != nullptr) {
-          const int64_t o = mn + (int64_t)gi * N + gj;
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            *(anc_f32x4 *)(p.X32 + o + 4 * i) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+            *(anc_f32x4 *)(p.X32 + mn + quad(i, N)) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
         } else if (p.X16 != nullptr) {
-          put_bf16(p.X16 + mn + (int64_t)gi * N + gj, nullptr);
+          put_bf16(p.X16 + mn + (int64_t)gi * N + gj, nullptr, (int64_t)RS * N);
         } else if (out8) {
           uint32_t h[8], q[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -511,11 +546,13 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
             h[i] = anc_pk_bf16(v[2 * i], v[2 * i + 1]);
             q[i >> 1] |= (anc_low8_encode(v[2 * i], h[i] << 16) | (anc_low8_encode(v[2 * i + 1], h[i] & 0xFFFF0000u) << 8)) << (16 * (i & 1));
           }
-          *(anc_u32x4 *)(p.Yh + mn + pan) = anc_u32x4{h[0], h[1], h[2], h[3]};
-          *(anc_u32x4 *)(p.Yh + mn + pan + 8) = anc_u32x4{h[4], h[5], h[6], h[7]};
-          *(anc_u32x4 *)((char *)p.Yl + mn * 2 + pan) = anc_u32x4{q[0], q[1], q[2], q[3]};
+#pragma unroll
+          for (int r = 0; r < NR; ++r) {
+            st_run<RUN * 2>(p.Yh + mn + pan + r * pst, h + r * (RUN / 2));
+            st_run<RUN>((char *)p.Yl + mn * 2 + pan + r * pst, q + r * (RUN / 4));
+          }
         } else {
-          put_bf16(p.Yh + mn + pan, p.Yl + mn + pan);
+          put_bf16(p.Yh + mn + pan, p.Yl + mn + pan, pst);
         }
       }
     }
