@@ -333,6 +333,19 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     frag_b(stg, kk, f.b);
   };
 
+  // Plain product with an addend (C = A32 + A B, in place when A32 == X32): the addend of the first of the
+  // wavefront's four 32x64 slabs is requested here, the next slab's before a slab's stores go out (a wait for a
+  // load is a wait for every older store).
+  const int64_t mn = (int64_t)e * p.M * p.N;
+  const bool plain_add = PLAINV && p.plain_sum && p.A32 != nullptr;
+  anc_f32x4 addend[8];
+  auto fetch_addend = [&](int bi) {
+    if (!plain_add) return;
+    const float *q = p.A32 + mn + (int64_t)(tm * TM + wm * 128 + bi * 32 + (lane >> 4)) * p.N + tn * TN + wn * 64 + (lane & 15) * 4;
+#pragma unroll
+    for (int pz = 0; pz < 8; ++pz) addend[pz] = anc_ld_stream((const anc_f32x4 *)(q + (int64_t)(4 * pz) * p.N));
+  };
+
   f32x16 acc[4][2];
 #pragma unroll
   for (int bi = 0; bi < 4; ++bi)
@@ -507,7 +520,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   // ---- epilogue
   if ((VAR == VAR_UPDATE || VAR == VAR_UPDATE_T) && pm.ctl != nullptr && pm.ctl->skip != 0u) return;   // skipped step
   const int M = p.M, N = p.N;
-  const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
+  const int64_t mm = (int64_t)e * M * M, mv = (int64_t)e * M;
   unsigned char *region = st(wave / WPS) + (wave % WPS) * kStageRegion;
   const int gi0w = tm * TM + wm * 128, gj0w = tn * TN + wn * 64;
   const bool mirror = (EPI != EPI_BX) && (TN * (tn + 1) <= TM * tm);
@@ -616,6 +629,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     fetch_in(0);
     fetch_in(1);
   }
+  if constexpr (PLAINV) fetch_addend(0);
   if (EPI == EPI_BX) {
     // Transposed accumulator layout (see mfma8): lane l holds row l%32 of the slab and, per
     // column block bj and q = 0..3, the 4 consecutive columns bj*32 + 8q + 4*(l/32) .. +3.
@@ -664,14 +678,10 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
 #pragma unroll
         for (int pz = 0; pz < 8; ++pz) pv[pz] = anc_ld_stream((const anc_f32x4 *)(W32 + w_off(gi0, pz)));
       }
-      // Plain product with an addend (C = A32 + A B, in place when A32 == X32): same early request
-      const bool plain_add = plain && p.plain_sum && p.A32 != nullptr;
-      if (plain_add) {
+      if constexpr (plain) {
 #pragma unroll
-        for (int pz = 0; pz < 8; ++pz) {
-          const int idx = pz * 64 + lane;
-          pv[pz] = anc_ld_stream((const anc_f32x4 *)(p.A32 + mn + (int64_t)(gi0 + (idx >> 4)) * N + gj0w + (idx & 15) * 4));
-        }
+        for (int pz = 0; pz < 8; ++pz) pv[pz] = addend[pz];
+        if (bi < 3) fetch_addend(bi + 1);
       }
       // Wait for this slab's DMA only. Vector memory operations complete in issue order; after
       // the fetch of slab bi this wavefront issued the 8 row stores of slab bi-1 and the fetch
