@@ -734,15 +734,8 @@ struct ChainProb {
 //               16 x (1024,1024) 295 / 286 / 228 (2560)
 //   X = a X + B X   6 x (512,1536) 131 / 147 / 172 (1152), 2 x (1024,3072) 158 / 145 / 152 (1536),
 //               8 x (1024,1024) 210 / 179 / 179 (2048), 3 x (1024,3072) 218 / 212 / 197 (2304)
-// hence 64 below 800 (symmetric) or 1400 tiles of 64, 128 up to 2000. The bare product's K is a batch of tokens,
-// up to 8192, and its operands leave the L2: weight gradients at 512 / 2048 / 8192 tokens on the three tiles,
-//   432 tiles of 64    11.3 21.1 65 / 13.9 28.2 80 / 16.5 33.9 97
-//   768                15.2 31.5 117 / 16.3 31.5 88 / 18.3 35.8 101
-//   1024               18.3 38.5 146 / 17.8 34.2 93 / 19.0 38.2 105
-//   1248               22.3 47.9 194 / 23.4 49.1 127 / 21.5 40.3 105
-// hence 64 below 768 and 128 up to one tile of 128 per CU: 1056 tiles of 64, 8 CUs with two of 128 each, take
-// 55 against 43 us at 3360 tokens.
-int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n, bool plain = false) {
+// hence 64 below 800 (symmetric) or 1400 tiles of 64, 128 up to 2000.
+int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
   for (int k = 0; k < n; ++k) {
@@ -750,8 +743,36 @@ int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n, bool plain = 
     const double per = epi == EPI_BX ? m * (double)(ps[k].N / 64) : m * (m + d) / 2.0;
     t64 += (double)Es[k] * per * ((double)ps[k].K / longest);
   }
-  if (t64 < (plain ? 768.0 : epi == EPI_BX ? 1400.0 : 800.0)) return 64;
-  return t64 <= (plain ? 1024.0 : 2000.0) ? 128 : 256;
+  if (t64 < (epi == EPI_BX ? 1400.0 : 800.0)) return 64;
+  return t64 <= 2000.0 ? 128 : 256;
+}
+
+// The same for the bare product of weight gradients. Its K is a batch of tokens: short ones are bound by the
+// output, which small tiles spread best, long ones by operands that leave the L2, and there a second 128-wide tile
+// on a few CUs costs as much as on all. Measured, us on 64 / 128 / 256-wide tiles, gradients added up (in
+// brackets: written):
+//   tiles of 64      256 tokens             1024 tokens            3072 tokens       8192 tokens
+//   640              8.5/10.2/13.5          18.2/17.6/24.2         41.9/37.8/46.5    112/83/100
+//   1024             10.7/11.0/16.1         22.9/20.1/29.5         53.0/42.2/51.6    149/91/110
+//   1056             12.4/13.5/16.9         26.5/24.7/27.9         59.6/56.0/50.3    162/121/103
+//                    (11.5/12.4/11.7)       (23.4/23.7/21.0)
+//   1344             15.4/15.0/18.5         31.7/27.6/29.9         75.9/61.6/52.5    223/127/107
+//                    (13.0/12.8/12.4)       (28.1/25.0/24.1)
+//   2816             26.6/27.3/34.2         58.2/53.0/50.9         154/99/91         466/230/198
+//                    (21.4/21.3/21.6)       (49.6/48.0/38.1)
+// hence up to 400 tokens 64 below 1300 tiles of 64 and 128 up to 2000 (3000 where something is added to), beyond 64 below 600 and 128 up to 1024, one
+// per CU. (560 and fewer tiles of 64 are fastest at every length: 432 at 8192 tokens 65 / 80 / 97.)
+int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
+  double longest = 0.0, t64 = 0.0;
+  bool adds = false;
+  for (int k = 0; k < n; ++k) {
+    longest = ps[k].K > longest ? (double)ps[k].K : longest;
+    adds = adds || (ps[k].plain_sum && ps[k].A32 != nullptr);
+  }
+  for (int k = 0; k < n; ++k) t64 += (double)Es[k] * (ps[k].M / 64) * (ps[k].N / 64) * ((double)ps[k].K / longest);
+  const bool brief = longest <= 400.0;
+  if (t64 < (brief ? 1300.0 : 600.0)) return 64;
+  return t64 <= (!brief ? 1024.0 : adds ? 3000.0 : 2000.0) ? 128 : 256;
 }
 
 // What a mode's tile flags ask for (0: nothing).
@@ -984,7 +1005,7 @@ int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int f
 
 int anc_ns_gemm_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool a_transposed) {
   ANC_REQUIRE(n >= 1 && n <= kMaxGroups, "anc_ns_gemm_plain: 1..%d problems per launch", kMaxGroups);
-  const int tile = pick_tile(EPI_BX, ps, Es, n, true);
+  const int tile = pick_tile_plain(ps, Es, n);
   if (tile == 256) return anc_ns_gemm_big_plain(ps, Es, n, s, a_transposed);
   return anc_ns_gemm_tile_multi(EPI_BX, ps, Es, n, s, tile == 64, a_transposed, nullptr, true);
 }

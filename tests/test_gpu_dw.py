@@ -378,3 +378,32 @@ def test_accumulated_micro_batches_against_one_batch(gpu):
         opt.free(); g.free()
     same = float((new[0].view(np.uint32) == new[1].view(np.uint32)).mean())
     assert same >= 0.98, same                                          # (D): the reference's bar
+
+
+@pytest.mark.parametrize("T", [96, 384, 416])
+@pytest.mark.parametrize("K,N,n", [(640, 768, 1), (1024, 1024, 3), (1024, 1024, 5), (1024, 1280, 7), (2048, 1536, 5)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_many_weights_per_call_have_the_bits_each_has_alone(gpu, T, K, N, n, accumulate):
+    """The size and length of a call choose its tiles: calls on both sides of those lines (120 to 3840 tiles of 64,
+    token counts that end in half a step, written or added to) against a call of the weight alone."""
+    from ancora_cutile_amd import DevBuf
+    from ancora_cutile_amd.grads import gemm_dW, DwWorkspace
+    x, dy = _inputs(T, K, N, T + n)
+    dW0 = (0.5 * np.random.default_rng(n).standard_normal((K, N))).astype(np.float32)
+    xd, dyd = DevBuf(x), DevBuf(dy)
+    mk = lambda: dict(x=xd, dy=dyd, dW=DevBuf(dW0), T=T, K=K, N=N, workspace=DwWorkspace(),
+                      g16=DevBuf.zeros((K, N), np.uint16), accumulate=accumulate)
+    one, many = mk(), [mk() for _ in range(n)]
+    gemm_dW([one])
+    gemm_dW(many)
+    want = one["dW"].to_numpy()
+    assert rel_fro(want, gemm_dw(x, dy) + (dW0 if accumulate else 0.0)) < 2e-5
+    for p in (many[0], many[-1]):
+        assert bits_equal(p["dW"].to_numpy(), want)
+        assert bits_equal(p["g16"].to_numpy(), one["g16"].to_numpy())
+    for p in [one] + many:
+        p["dW"].free()
+        p["g16"].free()
+        p["workspace"].free()
+    xd.free()
+    dyd.free()
