@@ -53,10 +53,6 @@ template <typename T> __device__ __forceinline__ void epi_st(T *p, T v) { anc_st
 
 namespace {
 
-struct Frags {
-  bf16x8 a[4], b[2];
-};
-
 // SWAP = false: accumulator block (bi,bj) holds C[32 bi + row][32 bj + col] with col = lane%32
 // and element r = row 8*(r/4) + 4*(lane/32) + r%4. SWAP = true computes the transposed block
 // (operands exchanged, same products, same order of summation): row = lane%32 and element
@@ -68,26 +64,20 @@ __device__ __forceinline__ void mfma1(const bf16x8 (&a)[4], const bf16x8 (&b)[2]
   acc[bi][bj] = SWAP ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bj], a[bi], acc[bi][bj], 0, 0, 0)
                      : __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
 }
-// 8 MFMAs with n DMA instructions (`piece(i)`) between them, one every 8/n, instead of as a burst
-// during which the matrix pipe idles.
-template <bool SWAP, int N, typename F>
-__device__ __forceinline__ void mfma8_dma(const bf16x8 (&a)[4], const bf16x8 (&b)[2], f32x16 (&acc)[4][2], F piece) {
+// 8 MFMAs with the fragment reads of the next 8 (`load(idx)`) and N DMA instructions (`piece(i)`) between them, instead
+// of as bursts during which the matrix pipe idles and the LDS serves all wavefronts at once.
+template <bool SWAP, int N, typename L, typename F>
+__device__ __forceinline__ void mfma8_with(const bf16x8 (&a)[4], const bf16x8 (&b)[2], f32x16 (&acc)[4][2], L load, F piece) {
 #pragma unroll
   for (int idx = 0; idx < 8; ++idx) {
     mfma1<SWAP>(a, b, acc, idx);
+    __builtin_amdgcn_sched_barrier(0);
+    load(idx);
 #pragma unroll
     for (int i = 0; i < N; ++i)
-      if (((i + 1) * 8 + N - 1) / N - 1 == idx) {
-        __builtin_amdgcn_sched_barrier(0);
-        piece(i);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      if ((idx + 1) * N >= (i + 1) * 8 && idx * N < (i + 1) * 8) piece(i);
+    __builtin_amdgcn_sched_barrier(0);
   }
-}
-template <bool SWAP>
-__device__ __forceinline__ void mfma8(const bf16x8 (&a)[4], const bf16x8 (&b)[2], f32x16 (&acc)[4][2]) {
-#pragma unroll
-  for (int idx = 0; idx < 8; ++idx) mfma1<SWAP>(a, b, acc, idx);
 }
 
 // bf16 tile staging through LDS. `v` holds, for the wavefront's 32-row slab, the bf16 values of
@@ -316,21 +306,23 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       ta[bi] = (8 * (g16 >> 1) + (s16 >> 2)) * 256 + ((chunk ^ ((s16 >> 2) << 2)) * 16) + (s16 & 1) * 8;
     }
   }
-  auto frag_a = [&](const unsigned char *stg, int kk, bf16x8 (&f)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      f[i] = AT ? anc_lds_tr_frag(stg + ta[i] + kk * (16 * 256), stg + ta[i] + kk * (16 * 256) + 4 * 256)
-                : *(const bf16x8 *)(stg + a_base + i * (32 * TK * 2) + swz[kk]);
+  auto frag_a = [&](const unsigned char *stg, int kk, int i) -> bf16x8 {
+    return AT ? anc_lds_tr_frag(stg + ta[i] + kk * (16 * 256), stg + ta[i] + kk * (16 * 256) + 4 * 256)
+              : *(const bf16x8 *)(stg + a_base + i * (32 * TK * 2) + swz[kk]);
   };
-  auto frag_b = [&](const unsigned char *stg, int kk, bf16x8 (&f)[2]) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      f[i] = BT ? anc_lds_tr_frag(stg + tb[i] + kk * (16 * 512), stg + tb[i] + kk * (16 * 512) + 4 * 512)
-                : *(const bf16x8 *)(stg + b_base + i * (32 * TK * 2) + swz[kk]);
+  auto frag_b = [&](const unsigned char *stg, int kk, int i) -> bf16x8 {
+    return BT ? anc_lds_tr_frag(stg + tb[i] + kk * (16 * 512), stg + tb[i] + kk * (16 * 512) + 4 * 512)
+              : *(const bf16x8 *)(stg + b_base + i * (32 * TK * 2) + swz[kk]);
   };
-  auto frags = [&](const unsigned char *stg, int kk, Frags &f) {
-    frag_a(stg, kk, f.a);
-    frag_b(stg, kk, f.b);
+  // fragment j (0..5, others: none) of a k-step, in the order its matrix instructions need them: a0, b0, b1, a1, a2, a3
+  auto frag = [&](const unsigned char *sa, const unsigned char *sb, int kk, int j, bf16x8 (&a)[4], bf16x8 (&b)[2]) {
+    if (j == 1 || j == 2) b[j - 1] = frag_b(sb, kk, j - 1);
+    else if (j == 0) a[0] = frag_a(sa, kk, 0);
+    else if (j > 2 && j < 6) a[j - 2] = frag_a(sa, kk, j - 2);
+  };
+  auto frags = [&](const unsigned char *stg, int kk, bf16x8 (&a)[4], bf16x8 (&b)[2]) {
+#pragma unroll
+    for (int j = 0; j < 6; ++j) frag(stg, stg, kk, j, a, b);
   };
 
   // Plain product with an addend (C = A32 + A B, in place when A32 == X32): the addend of the first of the
@@ -361,22 +353,22 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     // barrier inside tile k-1). Before the last k-step of tile k each wavefront waits until its
     // own DMA of tile k+1 has landed (NS-2 younger tiles may still be in flight), all
     // wavefronts synchronise, and the first fragments of tile k+1 load under the last MFMAs.
-    Frags f[2];
+    bf16x8 a[2][4], b[2][2];
 #pragma unroll
     for (int s0 = 0; s0 < NS - 1; ++s0)
       if (s0 < nk) issue(st(s0));
     if (nk >= NS - 1) wait_vm<(NS - 2) * IPS>(); else wait_vm<0>();
     lds_barrier();
-    frags(stage0, 0, f[0]);
+    frags(stage0, 0, a[0], b[0]);
 
-    // f[kk] holds k-step kk. `steady` (a std::true_type): the caller knows that this tile refills
+    // a[kk], b[kk] hold k-step kk. `steady` (a std::true_type): the caller knows that this tile refills
     // the ring and has a successor, so the body carries no branch.
     auto body = [&](auto steady, int step, unsigned char *cur, unsigned char *nxt, unsigned char *fill) {
       constexpr bool kSteady = decltype(steady)::value;
       const bool more = kSteady || step + 1 < nk;
       const bool refill = kSteady || step + NS - 1 < nk;
-      frags(cur, 1, f[1]);
-      mfma8_dma<BT, IPS>(f[0].a, f[0].b, acc, [&](int i) { if (refill) issue_piece(i, fill, curA, curB); });
+      mfma8_with<BT, IPS>(a[0], b[0], acc, [&](int idx) { frag(cur, cur, 1, idx, a[1], b[1]); },
+                          [&](int i) { if (refill) issue_piece(i, fill, curA, curB); });
       if (refill) {
         curA += advA;
         curB += advB;
@@ -385,8 +377,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         wait_vm<0>();
       }
       lds_barrier();
-      if (more) frags(nxt, 0, f[0]);
-      mfma8<BT>(f[1].a, f[1].b, acc);
+      mfma8_with<BT, 0>(a[1], b[1], acc, [&](int idx) { if (more) frag(nxt, nxt, 0, idx - 1, a[0], b[0]); }, [](int) {});
     };
     int step = 0;
     // rounds of NS tiles in which even the last tile (step + NS - 1) still refills the ring
@@ -435,21 +426,20 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         wait_vm<PL>();
       }
       lds_barrier();
-      frag_a(st(0), 0, a[0]);
-      frag_b(st(0), 0, b[0]);
+      frags(st(0), 0, a[0], b[0]);
       // the fragments of hh 0..15 are in a[x], b[0]; the next tile's end up in a[1 - x], b[0]
       auto body = [&](auto steady, auto parity, int t, unsigned char *H, unsigned char *L, unsigned char *H1, unsigned char *L1) {
         constexpr bool kSteady = decltype(steady)::value;
         constexpr int x = decltype(parity)::value, y = 1 - x;
         const bool more = kSteady || t + 1 < nk, more2 = kSteady || t + 2 < nk;
+        auto none = [](int) {};
         // P0
-        frag_a(H, 1, a[y]);
-        frag_b(H, 1, b[1]);
+        auto load0 = [&](int idx) { frag(H, H, 1, idx, a[y], b[1]); };
         if (NS == 4) {
-          mfma8_dma<BT, PL>(a[x], b[0], acc, [&](int i) { if (more) piece_l(i, L1); });
+          mfma8_with<BT, PL>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_l(i, L1); });
           if (more) adv_l();
         } else {
-          mfma8_dma<BT, IPS>(a[x], b[0], acc, [&](int i) { if (more) piece_h(i, H1); });
+          mfma8_with<BT, IPS>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_h(i, H1); });
           if (more) adv_h();
         }
         // P1
@@ -457,36 +447,33 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         for (int idx = 0; idx < 4; ++idx) mfma1<BT>(a[y], b[1], acc, idx);
         if (more) wait_vm<NS == 4 ? IPS + PL : IPS>(); else wait_vm<0>();
         lds_barrier();
-        frag_b(L, 1, b[0]);
-        if (NT == 3) frag_a(L, 1, a[x]);
-        else { frag_a(H, 0, a[x]); }
 #pragma unroll
-        for (int idx = 4; idx < 8; ++idx) mfma1<BT>(a[y], b[1], acc, idx);
+        for (int idx = 4; idx < 8; ++idx) {
+          mfma1<BT>(a[y], b[1], acc, idx);
+          __builtin_amdgcn_sched_barrier(0);
+          if (idx < 6) b[0][idx - 4] = frag_b(L, 1, idx - 4);
+          else a[x][idx - 6] = NT == 3 ? frag_a(L, 1, idx - 6) : frag_a(H, 0, idx - 6);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // P2 (of two terms: its last half, P4 has two fragments of A yet to come)
+        mfma8_with<BT, 0>(a[y], b[0], acc, [&](int idx) {
+          if (idx < 2) a[x][2 + idx] = NT == 3 ? frag_a(L, 1, 2 + idx) : frag_a(H, 0, 2 + idx);
+          else if (NT == 2 && idx < 4) b[1][idx - 2] = frag_b(L, 0, idx - 2);
+        }, none);
         if (NT == 3) {
-          // P2, P3, P4
-          mfma8<BT>(a[y], b[0], acc);
-          frag_a(H, 0, a[y]);
-          frag_b(L, 0, b[0]);
-          mfma8<BT>(a[x], b[1], acc);
-          frag_a(L, 0, a[x]);
-          frag_b(H, 0, b[1]);
-          mfma8<BT>(a[y], b[0], acc);
-        } else {
-          frag_b(L, 0, b[1]);
-          mfma8<BT>(a[y], b[0], acc);
+          // P3, P4
+          mfma8_with<BT, 0>(a[x], b[1], acc, [&](int idx) { frag(H, L, 0, idx, a[y], b[0]); }, none);
+          mfma8_with<BT, 0>(a[y], b[0], acc, [&](int idx) { frag(L, H, 0, idx, a[x], b[1]); }, none);
         }
         if (more) wait_vm<NS == 4 ? PL : 0>(); else wait_vm<0>();
         lds_barrier();
         // P5 (P4 of two terms)
-        if (more) {
-          frag_a(H1, 0, a[y]);
-          frag_b(H1, 0, b[0]);
-        }
+        auto load5 = [&](int idx) { if (more) frag(H1, H1, 0, idx - 1, a[y], b[0]); };
         if (NS == 4) {
-          mfma8_dma<BT, IPS>(a[x], b[1], acc, [&](int i) { if (more2) piece_h(i, H); });
+          mfma8_with<BT, IPS>(a[x], b[1], acc, load5, [&](int i) { if (more2) piece_h(i, H); });
           if (more2) adv_h();
         } else {
-          mfma8_dma<BT, PL>(a[x], b[1], acc, [&](int i) { if (more) piece_l(i, H); });
+          mfma8_with<BT, PL>(a[x], b[1], acc, load5, [&](int i) { if (more) piece_l(i, H); });
           if (more) adv_l();
         }
       };
