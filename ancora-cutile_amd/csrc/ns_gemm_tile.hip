@@ -52,7 +52,8 @@ __device__ __forceinline__ void st_run(void *p, const uint32_t *w) {
   else *(uint32_t *)p = w[0];
 }
 
-template <int EPI, int WB, bool AT, int VAR, int kRing>
+// SOLO: the launch has one problem, its arguments lie at fixed places.
+template <int EPI, int WB, bool AT, int VAR, int kRing, bool SOLO>
 __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemmMulti pm) {
   constexpr int TM = 64 * WB, KP = WB == 1 ? 2 : 1, TK = 32 * KP;
   constexpr bool BT = EPI == EPI_BX, PLAINV = VAR == VAR_PLAIN;
@@ -61,26 +62,31 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   static_assert(!AT || BT, "A by rows k: X = a X + B X and the plain product only");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing * kStageBytes];
 
-  int gsel, L;
-  if (PLAINV && pm.seq) anc_seq_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
+  int gsel = 0, L;
+  if (SOLO) L = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  else if (PLAINV && pm.seq) anc_seq_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
   else anc_group_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
   const NsGemm &p = pm.g[gsel];
-  int e, tm, tn;
-  if (p.lower) {
+  int e = 0, tm, tn;
+  // (the blocks' edges are powers of two; a division of two variables is 40 instructions, and a launch that this
+  // kernel is made for has little else to do)
+  const int sr = __builtin_ctz(p.blk_r), sc_ = __builtin_ctz(p.blk_c);
+  if (EPI != EPI_BX) {
     // lower triangle of blocks of G x G tiles (G = blk_r), every tile of a block computed
-    const int G = p.blk_r, q = p.tiles_m / G, per = G * G * (q * (q + 1) / 2);
-    e = L / per;
-    const int t = L % per, i = t % (G * G);
-    int b = t / (G * G), bm = 0;
+    const int q = p.tiles_m >> sr, per = (q * (q + 1) / 2) << (2 * sr);
+    if (L >= per) { e = L / per; L -= e * per; }
+    const int i = L & (p.blk_r * p.blk_r - 1);
+    int b = L >> (2 * sr), bm = 0;
     while (b > bm) { b -= bm + 1; ++bm; }
-    tm = bm * G + i / G;
-    tn = b * G + i % G;
+    tm = (bm << sr) + (i >> sr);
+    tn = (b << sr) + (i & (p.blk_r - 1));
   } else {
-    const int per = p.tiles_m * p.tiles_n, bper = p.blk_r * p.blk_c, across = p.tiles_n / p.blk_c;
-    e = L / per;
-    const int t = L % per, b = t / bper, i = t % bper;
-    tm = (b / across) * p.blk_r + i / p.blk_c;
-    tn = (b % across) * p.blk_c + i % p.blk_c;
+    const int per = p.tiles_m * p.tiles_n, across = p.tiles_n >> sc_;
+    if (L >= per) { e = L / per; L -= e * per; }
+    const int b = L >> (sr + sc_), i = L & (p.blk_r * p.blk_c - 1);
+    const int br = b / across, bc = b - br * across;
+    tm = (br << sr) + (i >> sc_);
+    tn = (bc << sc_) + (i & (p.blk_c - 1));
   }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -144,7 +150,7 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 
   // ---- what the epilogue of X = a X + B X reads at the output position is requested here, so that it has arrived
   // when the K loop ends (16 x (1024,3072) on 128-wide tiles: 828 -> 783 us per 5 launches against fetching it
-  // block by block behind the loop; B = b A + c A A, which reads half as much, lost 2 % that way). The loads are older than
+  // block by block behind the loop; B = b A + c A A, which reads half as much, lost 2 % that way on such launches). The loads are older than
   // every DMA below, so the waits of the ring hold.
   const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
   float *sg = (float *)lds + wave * 32 * kSgPitch;
@@ -203,6 +209,28 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         wpre[r] = *(const anc_f32x4 *)(p.A32 + mn + (int64_t)(gi_w + lrow + RS * r) * N + gj_w + c0);
+    }
+  }
+
+  // A at the output position, with at most one workgroup per CU
+  constexpr bool kEarlyA = EPI == EPI_BMAT && WB == 1 && kRing == 4;
+  anc_f32x4 a32[4];
+  float pre_di[NR], pre_dj[RUN];
+  if constexpr (kEarlyA) {
+    if (has_a32) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        a32[i] = *(const anc_f32x4 *)(p.A32 + mm + (int64_t)(gi_w + lrow + RS * (4 * i / RUN)) * M + gj_w + c0 + 4 * i % RUN);
+    } else {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) ld_run<RUN * 2>(p.Fh + mm + pan_of(0) + r * RS * 32, &pre_h[0][r * (RUN / 2)]);
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) pre_di[r] = p.dA[mv + gi_w + lrow + RS * r];
+#pragma unroll
+    for (int c = 0; c < RUN; c += 4) {
+      const anc_f32x4 w = *(const anc_f32x4 *)(p.dA + mv + gj_w + c0 + c);
+      pre_dj[c] = w.x; pre_dj[c + 1] = w.y; pre_dj[c + 2] = w.z; pre_dj[c + 3] = w.w;
     }
   }
 
@@ -397,24 +425,28 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
           if (has_a32) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const anc_f32x4 w = *(const anc_f32x4 *)(p.A32 + mm + quad(i, M));
+              const anc_f32x4 w = kEarlyA ? a32[i] : *(const anc_f32x4 *)(p.A32 + mm + quad(i, M));
               a[4 * i] = w.x; a[4 * i + 1] = w.y; a[4 * i + 2] = w.z; a[4 * i + 3] = w.w;
             }
           } else {
-            uint32_t u[8];
+            if constexpr (!kEarlyA) {
 #pragma unroll
-            for (int r = 0; r < NR; ++r) ld_run<RUN * 2>(p.Fh + mm + pan + r * pst, u + r * (RUN / 2));
-            unpack(u, a);
+              for (int r = 0; r < NR; ++r) ld_run<RUN * 2>(p.Fh + mm + pan + r * pst, &pre_h[0][r * (RUN / 2)]);
+            }
+            unpack(pre_h[0], a);
           }
-          float dj[RUN];
+          if constexpr (!kEarlyA) {
 #pragma unroll
-          for (int i = 0; i < RUN; i += 4) {
-            const anc_f32x4 w = *(const anc_f32x4 *)(p.dA + mv + gj + i);
-            dj[i] = w.x; dj[i + 1] = w.y; dj[i + 2] = w.z; dj[i + 3] = w.w;
+            for (int i = 0; i < RUN; i += 4) {
+              const anc_f32x4 w = *(const anc_f32x4 *)(p.dA + mv + gj + i);
+              pre_dj[i] = w.x; pre_dj[i + 1] = w.y; pre_dj[i + 2] = w.z; pre_dj[i + 3] = w.w;
+            }
+#pragma unroll
+            for (int r = 0; r < NR; ++r) pre_di[r] = p.dA[mv + gi + RS * r];
           }
 #pragma unroll
           for (int r = 0; r < NR; ++r) {
-            const float di = p.dA[mv + gi + RS * r];
+            const float di = pre_di[r];
 #pragma unroll
             for (int c = 0; c < RUN; ++c) {
               const int k = r * RUN + c;
@@ -423,7 +455,7 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
                 p.dB[mv + gj + c] = p.cb * di + p.cc * a2;
                 v[k] = 0.0f;
               } else {
-                const float a2 = v[k] + (di * a[k] + a[k] * dj[c]);   // symmetric in (i,j)
+                const float a2 = v[k] + (di * a[k] + a[k] * pre_dj[c]);   // symmetric in (i,j)
                 v[k] = p.cb * a[k] + p.cc * a2;
               }
             }
@@ -561,9 +593,10 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 
 template <int EPI, bool AT, int VAR>
 void launch_tile(bool small, unsigned grid, hipStream_t s, const NsGemmMulti &pm) {
-  if (!small)           hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, AT, VAR, 4>), dim3(grid), dim3(256), 0, s, pm);
-  else if (grid <= 256) hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 4>), dim3(grid), dim3(256), 0, s, pm);
-  else                  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 3>), dim3(grid), dim3(256), 0, s, pm);
+  if (!small)           hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+  else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 3, false>), dim3(grid), dim3(256), 0, s, pm);
+  else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+  else                  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 4, true>), dim3(grid), dim3(256), 0, s, pm);
 }
 
 }  // namespace
