@@ -729,12 +729,14 @@ struct ChainProb {
 // (a launch ends with its longest tiles; short ones fill gaps). A CU takes operand bytes into LDS at one
 // rate whatever the tile, so small tiles finish first while they find idle CUs and lose, by the bytes they
 // fetch more often, once every CU has several. Measured, us per 5 launches on 64 / 128 / 256-wide tiles:
-//   A = X X^T   16 x (512,512) 114 / 121 / 199 (768 tiles of 64), 5 x (1024,1024) 138 / 130 / 197 (800),
-//               4 x (1280,2560) 205 / 177 / 283 (960), 12 x (1024,1024) 240 / 211 / 210 (1920),
-//               16 x (1024,1024) 295 / 286 / 228 (2560)
-//   X = a X + B X   6 x (512,1536) 131 / 147 / 172 (1152), 2 x (1024,3072) 158 / 145 / 152 (1536),
-//               8 x (1024,1024) 210 / 179 / 179 (2048), 3 x (1024,3072) 218 / 212 / 197 (2304)
-// hence 64 below 800 (symmetric) or 1400 tiles of 64, 128 up to 2000.
+//   A = X X^T   16 x (512,512) 101 / 108 / 193 (768 tiles of 64), 4 x (1024,1024) 105 / 110 / 189 (640),
+//               5 x (1024,1024) 127 / 116 / 190 (800), 12 x (1024,1024) 221 / 178 / 204 (1920),
+//               16 x (1024,1024) 280 / 245 / 225 (2560)
+//   X = a X + B X   8 x (512,512) 72 / 99 / 157 (512), 4 x (1024,1024) 123 / 114 / 157 (1024),
+//               6 x (512,1536) 124 / 142 / 166 (1152), 2 x (1024,3072) 151 / 136 / 148 (1536),
+//               3 x (1024,3072) 202 / 193 / 199 (2304), 4 x (1024,3072) 258 / 222 / 211 (3072)
+// hence 64 below 800 (symmetric), or below 1400 tiles of 64 except from 800 to 1024, where one tile of 128 per
+// CU does; 128 up to 2200 (symmetric) or 2700.
 int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
@@ -743,8 +745,9 @@ int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
     const double per = epi == EPI_BX ? m * (double)(ps[k].N / 64) : m * (m + d) / 2.0;
     t64 += (double)Es[k] * per * ((double)ps[k].K / longest);
   }
-  if (t64 < (epi == EPI_BX ? 1400.0 : 800.0)) return 64;
-  return t64 <= 2000.0 ? 128 : 256;
+  if (epi != EPI_BX) return t64 < 800.0 ? 64 : t64 <= 2200.0 ? 128 : 256;
+  if (t64 < 1400.0 && !(t64 > 800.0 && t64 <= 1024.0)) return 64;
+  return t64 <= 2700.0 ? 128 : 256;
 }
 
 // The same for the bare product of weight gradients. Its K is a batch of tokens: short ones are bound by the
