@@ -460,7 +460,12 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
       }
       lds_wave_sync();                       // the buffer is free again
       if constexpr (EPI != EPI_BX) {
-        const bool diag = gi0 == gj0;        // a block on the diagonal: element k's row and column may be the same
+        // A block on the diagonal: one of the lane's elements, at most, has its row for a column. Picked by selects,
+        // not branches: these blocks are in the launch's longest workgroups.
+        const bool diag = gi0 == gj0;
+        auto on_diag = [&](int k) { return diag && lrow + RS * (k / RUN) == c0 + k % RUN; };
+        float dv = 0.0f;
+        int dc = -1;                         // its value and column
         if (EPI == EPI_GRAM) {
 #pragma unroll
           for (int k = 0; k < 16; ++k) v[k] = v[k] * acc_scale;
@@ -471,8 +476,13 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
           }
           if (diag) {
 #pragma unroll
-            for (int k = 0; k < 16; ++k)
-              if (lrow + RS * (k / RUN) == c0 + k % RUN) { p.dA[mv + gj + k % RUN] = v[k]; v[k] = 0.0f; }
+            for (int k = 0; k < 16; ++k) {
+              const bool on = on_diag(k);
+              dv = on ? v[k] : dv;
+              dc = on ? k % RUN : dc;
+              v[k] = on ? 0.0f : v[k];
+            }
+            if (dc >= 0) p.dA[mv + gj + dc] = dv;
           }
         } else {
           float a[16];
@@ -504,16 +514,16 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 #pragma unroll
             for (int c = 0; c < RUN; ++c) {
               const int k = r * RUN + c;
-              if (diag && lrow + RS * r == c0 + c) {
-                const float a2 = v[k] + di * di;
-                p.dB[mv + gj + c] = p.cb * di + p.cc * a2;
-                v[k] = 0.0f;
-              } else {
-                const float a2 = v[k] + (di * a[k] + a[k] * pre_dj[c]);   // symmetric in (i,j)
-                v[k] = p.cb * a[k] + p.cc * a2;
-              }
+              const bool on = on_diag(k);
+              const float dd = di * di, da = di * a[k] + a[k] * pre_dj[c];         // symmetric in (i,j)
+              const float a2 = v[k] + (on ? dd : da);
+              v[k] = p.cb * (on ? di : a[k]) + p.cc * a2;
+              dv = on ? v[k] : dv;
+              dc = on ? c : dc;
+              v[k] = on ? 0.0f : v[k];
             }
           }
+          if (dc >= 0) p.dB[mv + gj + dc] = dv;
         }
         uint16_t *oh = EPI == EPI_GRAM ? p.Fh : p.Bh, *ol = EPI == EPI_GRAM ? p.Fl : p.Bl;
         put_bf16(oh + mm + pan, write_lo ? ol + mm + pan : nullptr, pst);
