@@ -175,12 +175,14 @@ __device__ __forceinline__ int anc_ns_terms(const NsGemm &p, int e) {
 #define ANC_MAX_GROUPS 8
 #endif
 constexpr int kMaxGroups = ANC_MAX_GROUPS;
-struct NsGemmMulti {
+// G: problems there is room for. A launch's arguments travel to the device with it, 3.5 KB for eight problems (a chain of
+// one (128,128) matrix, which the host's launches bound: 76.7 -> 73.4 us with room for one).
+template <int G> struct NsGemmArgs {
   int n;
   int seq;                   // plain product: 1 = anc_seq_tile dealing, 0 = anc_group_tile
-  int tiles[kMaxGroups];     // 0 past n
+  int tiles[G];     // 0 past n
   int seg_start[kXcds + 1];  // anc_group_tile: first logical tile of each XCD's segment (anc_fill_segments)
-  NsGemm g[kMaxGroups];
+  NsGemm g[G];
   // fused weight update (problems with `upd` set): lr*shape_scale by descriptor scale index,
   // stochastic-rounding switch and seed, the step's control block (skip flag) or null
   float lr[ANC_MUON_MAX_SCALES];
@@ -188,6 +190,7 @@ struct NsGemmMulti {
   uint32_t seed_base;
   const anc_step_ctl_t *ctl;
 };
+using NsGemmMulti = NsGemmArgs<kMaxGroups>;
 // Segment x holds the x-th eighth of every problem's tiles, problems in the order given.
 inline void anc_fill_segments(NsGemmMulti &pm) {
   int at = 0;

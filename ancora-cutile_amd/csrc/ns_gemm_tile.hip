@@ -54,7 +54,7 @@ __device__ __forceinline__ void st_run(void *p, const uint32_t *w) {
 
 // SOLO: the launch has one problem, its arguments lie at fixed places.
 template <int EPI, int WB, bool AT, int VAR, int kRing, bool SOLO>
-__global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemmMulti pm) {
+__global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemmArgs<SOLO ? 1 : kMaxGroups> pm) {
   constexpr int TM = 64 * WB, KP = WB == 1 ? 2 : 1, TK = 32 * KP;
   constexpr bool BT = EPI == EPI_BX, PLAINV = VAR == VAR_PLAIN;
   constexpr int kHalf = TM * TK * 2;
@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing * kStageBytes];
 
   int gsel = 0, L;
-  if (SOLO) L = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  if constexpr (SOLO) L = xcd_remap((int)blockIdx.x, (int)gridDim.x);
   else if (PLAINV && pm.seq) anc_seq_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
   else anc_group_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
   const NsGemm &p = pm.g[gsel];
@@ -660,7 +660,17 @@ void launch_tile(bool small, unsigned grid, hipStream_t s, const NsGemmMulti &pm
   if (!small)           hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
   else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 3, false>), dim3(grid), dim3(256), 0, s, pm);
   else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
-  else                  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 4, true>), dim3(grid), dim3(256), 0, s, pm);
+  else {
+    NsGemmArgs<1> one;
+    one.n = 1;
+    one.seq = pm.seq;
+    one.g[0] = pm.g[0];
+    for (int k = 0; k < ANC_MUON_MAX_SCALES; ++k) one.lr[k] = pm.lr[k];
+    one.sr = pm.sr;
+    one.seed_base = pm.seed_base;
+    one.ctl = pm.ctl;
+    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 4, true>), dim3(grid), dim3(256), 0, s, one);
+  }
 }
 
 }  // namespace
