@@ -18,6 +18,14 @@ __device__ __forceinline__ void dma16(const void *g, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(g)
                : "memory", "m0");
 }
+// The same from a wavefront-uniform address and 32-bit offsets per lane: no 64-bit addition in vector registers. The
+// address is copied by a scalar instruction, which is the wait state that the write of M0 needs and makes it safe to
+// use at once even where a vector instruction (v_readfirstlane) has just produced it.
+__device__ __forceinline__ void dma16(const void *g, uint32_t off, uint32_t lds_base) {
+  uint64_t base;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+               : "=&s"(base) : "s"(lds_base), "v"(off), "s"(g) : "memory", "m0");
+}
 __device__ __forceinline__ uint32_t lds_addr(const void *p) {
   return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const void *)p);
 }

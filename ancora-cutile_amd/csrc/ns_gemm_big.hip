@@ -266,11 +266,15 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   auto issue_piece = [&](int i, unsigned char *stage, const char *pa, const char *pb) {
     if (i < IA) {
       const uint32_t vo = AT ? voffAT : ((i & 1) ? voff1 : voff0);
-      dma16(pa + i * roA + vo, lds_addr(stage + (wave * IA + i) * 1024));
+      // (scalar addition of addresses: chain of 24 x (1024,2048) 1214 -> 1192 us; the weight-gradient product, which is at
+      // its power limit, is 0.5 % faster with vector ones)
+      if (PLAINV) dma16(pa + i * roA + vo, lds_addr(stage + (wave * IA + i) * 1024));
+      else        dma16(pa + i * roA, vo, lds_addr(stage + (wave * IA + i) * 1024));
     } else {
       const int j = i - IA;
       const uint32_t vo = BT ? ((j & 1) ? voffB1 : voffB0) : ((j & 1) ? voffN1 : voffN0);
-      dma16(pb + j * roB + vo, lds_addr(stage + TM * ROWB + (wave * IB + j) * 1024));
+      if (PLAINV) dma16(pb + j * roB + vo, lds_addr(stage + TM * ROWB + (wave * IB + j) * 1024));
+      else        dma16(pb + j * roB, vo, lds_addr(stage + TM * ROWB + (wave * IB + j) * 1024));
     }
   };
   auto issue = [&](unsigned char *stage) {

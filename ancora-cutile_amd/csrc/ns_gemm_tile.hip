@@ -104,8 +104,8 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   const int64_t rpA = a_pan ? 64 : (int64_t)(p.ldA > 0 ? p.ldA : K) * 2, rpB = b_pan ? 64 : (int64_t)(BT ? N : K) * 2;
   const int64_t psA = a_pan ? panel : 64, psB = b_pan ? panel : 64;
   const int dr = lane >> 2, dc = lane & 3;
-  const int64_t voA = (int64_t)dr * rpA + (AT ? dc : dc ^ (dr >> 2)) * 16;
-  const int64_t voB = (int64_t)dr * rpB + (BT ? dc : dc ^ (dr >> 2)) * 16;
+  const uint32_t voA = (uint32_t)(dr * rpA) + (AT ? dc : dc ^ (dr >> 2)) * 16;
+  const uint32_t voB = (uint32_t)(dr * rpB) + (BT ? dc : dc ^ (dr >> 2)) * 16;
   int64_t offA[2], offB[2], cutA[2], cutB[2];     // this wavefront's two pieces of each operand; cut: see half_tail
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -122,11 +122,19 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   const int64_t advA = AT ? TK * rpA : KP * psA, advB = BT ? TK * rpB : KP * psB;
   const char *curA = (const char *)p.A[0] + baseA, *curB = (const char *)p.B[0] + baseB;
   int is_kt = 0;
+  // Adding up addresses in scalar registers leaves the vector pipe to the matrix instructions; a wavefront that has its
+  // SIMD to itself is quicker without the longer chain of scalar instructions (the step of one (1024,3072) weight: 1.4 % slower with it).
+  // (`lane_at`: at + off)
+  auto dma = [&](const char *g, int64_t at, int64_t lane_at, uint32_t off, uint32_t lds_base) {
+    if (WB == 1 && kRing == 4) dma16(g + lane_at, lds_base);
+    else                       dma16(g + at, off, lds_base);
+  };
+  const int64_t lA[2] = {offA[0] + voA, offA[1] + voA}, lB[2] = {offB[0] + voB, offB[1] + voB};
   auto piece = [&](int i, unsigned char *st) {          // DMA instruction i of a stage: two of A, two of B
     const bool cut = half_tail && is_kt + 1 == nk;      // (the missing panel's pieces fetch the one that is there)
     const int j = i & 1;
-    if (i < 2) dma16(curA + offA[j] - (cut ? cutA[j] : 0) + voA, lds_addr(st + (wave * 2 + j) * 1024));
-    else       dma16(curB + offB[j] - (cut ? cutB[j] : 0) + voB, lds_addr(st + kHalf + (wave * 2 + j) * 1024));
+    if (i < 2) dma(curA - (cut ? cutA[j] : 0), offA[j], lA[j], voA, lds_addr(st + (wave * 2 + j) * 1024));
+    else       dma(curB - (cut ? cutB[j] : 0), offB[j], lB[j], voB, lds_addr(st + kHalf + (wave * 2 + j) * 1024));
   };
   auto advance = [&]() { curA += advA; curB += advB; ++is_kt; };
   auto issue = [&](unsigned char *st) {
@@ -336,12 +344,14 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   } else {
     // ---- several terms: a step is one panel of 32 k of both halves of both operands, high stage then low stage.
     constexpr int kPan = TM * 64, kPair = 4 * kPan, kPairs = kRing * kStageBytes / kPair;   // 4, 3 (64) or 2 (128) steps in the ring
-    int64_t oA[WB], oB[WB];
+    int64_t oA[WB], oB[WB], vA[WB], vB[WB];
 #pragma unroll
     for (int j = 0; j < WB; ++j) {
       const int q = wave * WB + j;
-      oA[j] = (AT ? (q >> 1) * psA + (q & 1) * 16 * rpA : q * 16 * rpA) + voA;
-      oB[j] = (BT ? (q >> 1) * psB + (q & 1) * 16 * rpB : q * 16 * rpB) + voB;
+      oA[j] = (AT ? (q >> 1) * psA + (q & 1) * 16 * rpA : q * 16 * rpA);
+      oB[j] = (BT ? (q >> 1) * psB + (q & 1) * 16 * rpB : q * 16 * rpB);
+      vA[j] = oA[j] + voA;
+      vB[j] = oB[j] + voB;
     }
     const char *pAl = (const char *)p.A[1] + baseA, *pBl = (const char *)p.B[1] + baseB;
     const int64_t adA = AT ? 32 * rpA : psA, adB = BT ? 32 * rpB : psB;
@@ -351,10 +361,10 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 #pragma unroll
         for (int j = 0; j < WB; ++j) {
           const int at = (wave * WB + j) * 1024;
-          dma16(curA + oA[j], lds_addr(st + at));
-          dma16(curB + oB[j], lds_addr(st + kPan + at));
-          if (NT == 3) dma16(pAl + oA[j], lds_addr(st + 2 * kPan + at));
-          dma16(pBl + oB[j], lds_addr(st + 3 * kPan + at));
+          dma(curA, oA[j], vA[j], voA, lds_addr(st + at));
+          dma(curB, oB[j], vB[j], voB, lds_addr(st + kPan + at));
+          if (NT == 3) dma(pAl, oA[j], vA[j], voA, lds_addr(st + 2 * kPan + at));
+          dma(pBl, oB[j], vB[j], voB, lds_addr(st + 3 * kPan + at));
         }
         curA += adA; curB += adB; pAl += adA; pBl += adB;
       };
