@@ -181,7 +181,6 @@ template <int G> struct NsGemmArgs {
   int n;
   int seq;                   // plain product: 1 = anc_seq_tile dealing, 0 = anc_group_tile
   int tiles[G];     // 0 past n
-  int seg_start[kXcds + 1];  // anc_group_tile: first logical tile of each XCD's segment (anc_fill_segments)
   NsGemm g[G];
   // fused weight update (problems with `upd` set): lr*shape_scale by descriptor scale index,
   // stochastic-rounding switch and seed, the step's control block (skip flag) or null
@@ -191,15 +190,6 @@ template <int G> struct NsGemmArgs {
   const anc_step_ctl_t *ctl;
 };
 using NsGemmMulti = NsGemmArgs<kMaxGroups>;
-// Segment x holds the x-th eighth of every problem's tiles, problems in the order given.
-inline void anc_fill_segments(NsGemmMulti &pm) {
-  int at = 0;
-  for (int x = 0; x < kXcds; ++x) {
-    pm.seg_start[x] = at;
-    for (int k = 0; k < pm.n; ++k) at += pm.tiles[k] / kXcds + (x < pm.tiles[k] % kXcds ? 1 : 0);
-  }
-  pm.seg_start[kXcds] = at;
-}
 struct NsUpdate {
   float lr[ANC_MUON_MAX_SCALES];
   int sr;
@@ -207,39 +197,26 @@ struct NsUpdate {
   const anc_step_ctl_t *ctl;
 };
 
-// Workgroup id -> (problem, tile index inside the problem). The logical tile sequence is cut
-// into 8 segments, one per XCD (xcd_remap hands XCD x a contiguous range that coincides with
-// segment x up to a few tiles); segment x holds the x-th eighth of every problem's tiles,
-// problems in the order given (longest tiles first), so that every XCD gets the same mix and a
-// problem's consecutive tiles -- the tiles of one matrix -- stay on one XCD.
-__device__ __forceinline__ void anc_group_tile(const NsGemmMulti &pm, int bid, int grid, int &g, int &L) {
-  int pos = xcd_remap(bid, grid);
-  g = 0;
-  L = pos;
-  if (pm.n == 1) return;
-  // the segment, from the starts the host summed up (anc_fill_segments); then the problem inside
-  // it: all in scalar registers, no memory access inside the loops
-  int T[kMaxGroups];
+// Workgroup id -> (problem, tile index inside the problem). Every XCD gets an eighth of every problem's tiles, a run
+// of consecutive ones, problems in the order given (longest tiles first), so that all have the same mix and a
+// problem's consecutive tiles -- the tiles of one matrix -- stay on one XCD. What a problem's count leaves over 8
+// goes to the XCDs after those that the problems before it gave one more tile to, which is how the hardware deals the
+// launch's workgroup ids: an XCD's counts add up to the workgroups it runs. (About ten scalar instructions per problem;
+// a tile of the 256-wide symmetric kernel has a CU to itself and waits for them.)
+template <int G>
+__device__ __forceinline__ void anc_group_tile(const NsGemmArgs<G> &pm, int bid, int &g, int &L) {
+  const int x = bid % kXcds;
+  int q = bid / kXcds, off = 0;
 #pragma unroll
-  for (int k = 0; k < kMaxGroups; ++k) T[k] = pm.tiles[k];          // (entries past pm.n are 0)
-  int x = 0, start = 0;
-#pragma unroll
-  for (int xx = 1; xx < kXcds; ++xx) {
-    const int st = pm.seg_start[xx];
-    if (pos >= st) { x = xx; start = st; }
-  }
-  pos -= start;
-  bool found = false;
-#pragma unroll
-  for (int k = 0; k < kMaxGroups; ++k) {
-    const int base = T[k] / kXcds, rem = T[k] % kXcds;
-    const int c = base + (x < rem ? 1 : 0);
-    if (!found && pos < c) {
-      found = true;
-      g = k;
-      L = x * base + (x < rem ? x : rem) + pos;
+  for (g = 0; g < G; ++g) {
+    const int base = pm.tiles[g] / kXcds, rem = pm.tiles[g] % kXcds, xr = (x - off) & (kXcds - 1);
+    const int c = base + (xr < rem ? 1 : 0);
+    if (q < c || g + 1 >= pm.n) {
+      L = xr * base + (xr < rem ? xr : rem) + q;
+      return;
     }
-    if (!found) pos -= c;
+    q -= c;
+    off += rem;
   }
 }
 

@@ -173,7 +173,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   int gsel, L;
   constexpr bool PLAINV = (VAR == VAR_PLAIN);
   if (PLAINV && pm.seq) anc_seq_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
-  else anc_group_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
+  else anc_group_tile(pm, (int)blockIdx.x, gsel, L);
   const NsGemm &p = pm.g[gsel];
   // Symmetric outputs: only tiles that reach the diagonal or lie below it. Row tm of TM-row
   // tiles has tm/R + 1 of them (R = TN/TM); a tile entirely below the diagonal is mirrored.
@@ -186,14 +186,19 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   } else {
     tiles_per = p.tiles_m * p.tiles_n;
   }
-  const int e = L / tiles_per;
-  const int t = L % tiles_per;
-  int tm, tn;
+  int e = 0, t = L, tm, tn;
+  if (t >= tiles_per) { e = t / tiles_per; t -= e * tiles_per; }
   if (p.lower) {
     tm = 0;
     int left = t;
     while (left >= tm / R + 1) { left -= tm / R + 1; ++tm; }
     tn = left;
+  } else if (!PLAINV) {
+    // (blocks of 1, 2 or 4 tiles a side)
+    const int sr = __builtin_ctz(p.blk_r), sc_ = __builtin_ctz(p.blk_c), across = p.tiles_n >> sc_;
+    const int b = t >> (sr + sc_), i = t & (p.blk_r * p.blk_c - 1), br = b / across;
+    tm = (br << sr) + (i >> sc_);
+    tn = ((b - br * across) << sc_) + (i & (p.blk_c - 1));
   } else if (p.blk_r > 0) {
     const int per = p.blk_r * p.blk_c, b = t / per, i = t % per, across = p.tiles_n / p.blk_c;
     tm = (b / across) * p.blk_r + i / p.blk_c;
@@ -1084,7 +1089,6 @@ int launch_sym(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s) {
     grid += t;
   }
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_big: grid out of range");
-  anc_fill_segments(pm);
   hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 32, 4, 1>), dim3((unsigned)grid), dim3(512), 0, s, pm);
   ANC_LAUNCH_CHECK();
   return ANC_OK;
@@ -1126,7 +1130,6 @@ int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const N
     grid += t;
   }
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_big: grid out of range");
-  anc_fill_segments(pm);
   const bool fused = ps[0].upd != nullptr;
   if (fused) {
     for (int k = 0; k < ANC_MUON_MAX_SCALES; ++k) pm.lr[k] = upd->lr[k];
@@ -1193,7 +1196,6 @@ int anc_ns_gemm_big_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_
     grid += t;
   }
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_big_plain: grid out of range");
-  anc_fill_segments(pm);
   // Every XCD has an L2 of its own, so which tiles it runs decides how often an operand byte is
   // fetched from HBM. A launch that fits the GPU's 512 workgroup slots runs in one round: its
   // problems' tile sequences are dealt one after the other (anc_seq_tile), an XCD works on one or

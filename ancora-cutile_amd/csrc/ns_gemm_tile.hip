@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   int gsel = 0, L;
   if constexpr (SOLO) L = xcd_remap((int)blockIdx.x, (int)gridDim.x);
   else if (PLAINV && pm.seq) anc_seq_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
-  else anc_group_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
+  else anc_group_tile(pm, (int)blockIdx.x, gsel, L);
   const NsGemm &p = pm.g[gsel];
   int e = 0, tm, tn;
   // (the blocks' edges are powers of two; a division of two variables is 40 instructions, and a launch that this
@@ -717,7 +717,6 @@ int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, 
     grid += pm.tiles[k];
   }
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_tile: grid out of range");
-  anc_fill_segments(pm);
   const unsigned gr = (unsigned)grid;
   if (plain) {
     if (by_rows) launch_tile<EPI_BX, true, VAR_PLAIN>(small, gr, s, pm);
