@@ -26,6 +26,7 @@ from ._lib import (api, AdamWHyper, AdamWDesc, AdamWStepEntry, F32, BF16, FORM_D
                    SR_STEP_SEED)
 from .bf16 import bf16_bits as _bf16_bits, bits_f32 as _bits_f32  # noqa: F401  (re-exported)
 from .devbuf import DevBuf, upload_table
+from .gradnorm import ctl_ptr
 
 C = 64   # every tensor is a flat (numel // 64, 64) view (ancora/optim/adamw.py:20)
 
@@ -213,7 +214,7 @@ class AdamW:
         else:
             h = self._hyper()
         api.anc_adamw_multi(self._table.ptr, len(self.st), self._total_blocks, ctypes.byref(h),
-                            0 if guard is None else guard.ptr, int(stream_int))
+                            ctl_ptr(guard), int(stream_int))
 
     def unstep(self):
         """Undo the counter advance of a step the guard skipped (state was left untouched)."""

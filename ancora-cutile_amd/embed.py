@@ -15,6 +15,7 @@ from . import _lib
 from ._lib import api, AdamWHyper, FORM_DIV, FORM_IBC
 from .adamw import sr_seed_base
 from .devbuf import DevBuf
+from .gradnorm import ctl_ptr
 
 
 def _ids32(ids):
@@ -266,7 +267,7 @@ class RowSparseAdamW:
         self.t += 1
         if n_groups > 0:
             rows = gid.ptr_on(si) if isinstance(gid, _GroupArray) else gid.ptr
-            self._launch(rows, int(n_groups), grads.ptr, self.t, 0 if guard is None else guard.ptr, si)
+            self._launch(rows, int(n_groups), grads.ptr, self.t, ctl_ptr(guard), si)
         self.last_skipped = False
         if guard is not None:
             if guard.read(si)["skip"]:             # (synchronises)

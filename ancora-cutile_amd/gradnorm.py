@@ -8,6 +8,7 @@ deterministic reduction over every gradient of the step and leaves
 kernels read directly: no host round trip between the norm and the update.
 """
 import ctypes as C
+import threading
 
 import numpy as np
 
@@ -25,6 +26,45 @@ def _dtype_code(dtype):
     raise TypeError(f"gradient dtype {dtype}: expected float32 or uint16 (bf16 bits)")
 
 
+class _HostBlocks:
+    """Pinned host memory for control blocks, 64 to a 4 KiB page: pinning is 0.1 ms, which every new guard would pay.
+    One empty page is kept, others are given back as they empty."""
+    PER = 64
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._free = {}                          # page -> its free slots
+
+    def take(self):
+        with self._lock:
+            page = next((p for p, f in self._free.items() if f), None)
+            if page is None:
+                h = C.c_void_p()
+                api.anc_host_alloc(C.byref(h), 4096)
+                page = h.value
+                self._free[page] = [page + 64 * i for i in range(self.PER)]
+            return self._free[page].pop()
+
+    def give(self, block):
+        page = block & ~4095
+        with self._lock:
+            self._free[page].append(block)
+            empty = [p for p, f in self._free.items() if len(f) == self.PER]
+            for p in empty[1:]:
+                del self._free[p]
+                api.anc_host_free(C.c_void_p(p))
+
+
+_blocks = _HostBlocks()
+
+
+def ctl_ptr(guard):
+    """The control block's device address for a kernel of this package, which only reads it; 0 without a guard."""
+    if guard is None:
+        return 0
+    return guard._ctl.ptr if isinstance(guard, StepGuard) else guard.ptr
+
+
 class StepGuard:
     """max_norm: clip threshold (None or <= 0 disables clipping; the non-finite guard stays on)."""
 
@@ -32,12 +72,22 @@ class StepGuard:
         _lib.init()
         self.max_norm = 0.0 if max_norm is None else float(max_norm)
         self.eps = float(eps)
-        self.ctl = DevBuf.zeros((8,), np.uint32)
+        self._ctl = DevBuf.zeros((8,), np.uint32)
         self._partials = None
         self._tables = {}
         self._part0 = []
         self._key = None
-        self._host = None
+        # `compute` leaves a copy of the block in pinned host memory, which `read` takes instead of copying 32
+        # bytes from the device. `_copied`: the stream that copy comes from, None where the block has been written
+        # some other way since. A block whose address has been handed out may be: then never.
+        self._host = _blocks.take()
+        self._copied = None
+        self._private = True
+
+    @property
+    def ctl(self):
+        self._private = False
+        return self._ctl
 
     @property
     def ptr(self):
@@ -67,7 +117,8 @@ class StepGuard:
         count). The rest of the block is rewritten by the next `compute`."""
         raw = np.zeros(8, np.uint32)
         raw[5] = np.uint32(int(t))
-        self.ctl.upload(raw, stream)
+        self._copied = None
+        self._ctl.upload(raw, stream)
 
     def compute(self, grads, stream=0, produced=(), count_step=False):
         """grads: list of DevBuf (float32 or uint16/bf16), in a fixed order. `produced`: indices
@@ -86,18 +137,19 @@ class StepGuard:
                 chunk0 += api.anc_gradnorm_num_partials(g.size)
             self._tables[produced] = (upload_table(descs) if descs else None, len(descs), chunk0)
         table, n_tensors, n_chunks = self._tables[produced]
-        if table is not None:
-            api.anc_gradnorm_partials_multi(table.ptr, n_tensors, n_chunks, self._partials.ptr, int(stream))
-        api.anc_gradnorm_finalize(self._partials.ptr, self._n_partials, self.max_norm, self.eps,
-                                  int(bool(count_step)), self.ctl.ptr, int(stream))
+        api.anc_gradnorm_compute(0 if table is None else table.ptr, n_tensors, n_chunks, self._partials.ptr,
+                                 self._n_partials, self.max_norm, self.eps, int(bool(count_step)), self._ctl.ptr,
+                                 self._host, int(stream))
+        self._copied = int(stream)
 
     def read(self, stream=0):
         """Synchronise and return the control block as a dict."""
-        if self._host is None:                   # pinned: a pageable read-back of 32 bytes takes twice as long
-            self._host = C.c_void_p()
-            api.anc_host_alloc(C.byref(self._host), C.sizeof(StepCtl))
-        api.anc_memcpy_d2h(self._host, self.ctl.ptr, C.sizeof(StepCtl), int(stream))
-        c = StepCtl.from_address(self._host.value)
+        if self._private and self._copied == int(stream):
+            api.anc_stream_sync(int(stream))
+        else:
+            api.anc_memcpy_d2h(C.c_void_p(self._host), self._ctl.ptr, C.sizeof(StepCtl), int(stream))
+            self._copied = None
+        c = StepCtl.from_address(self._host)
         return {"sumsq": c.sumsq, "norm": c.norm, "clip_scale": c.clip_scale, "skip": bool(c.skip),
                 "t": int(c.t)}
 
@@ -110,7 +162,7 @@ class StepGuard:
 
     def free(self):
         self._free_tables()
-        self.ctl.free()
+        self._ctl.free()                         # (waits for the device: nothing writes the host's copy any more)
         if self._host is not None:
-            api.anc_host_free(self._host)
+            _blocks.give(self._host)
             self._host = None

@@ -15,6 +15,7 @@ from . import _lib
 from ._lib import api
 from .adamw import _adamw, _pick_otm, C as AC
 from .devbuf import DevBuf
+from .gradnorm import ctl_ptr
 from .muon import MuonEngine
 from .muon_ns import NsWorkspace, ns_workspace_bytes, _KELLER
 
@@ -97,7 +98,7 @@ class ExpertOptimizer:
         b1, b2 = self._betas
         ibc1 = 1.0 / (1.0 - b1 ** self._t)
         ibc2 = 1.0 / (1.0 - b2 ** self._t)
-        ctl = 0 if guard is None else guard.ptr
+        ctl = ctl_ptr(guard)
         if self.optimizer == "muon":
             self._muon_engine(grads).step(si, muon_lr, schedule, guard)
         else:

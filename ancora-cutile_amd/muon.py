@@ -24,6 +24,7 @@ from . import _lib
 from ._lib import api, MuonDesc, F32, BF16, MUON_MAX_SCALES, MUON_P16T, SR_ON, SR_STEP_SEED
 from .bf16 import bf16_bits, bits_f32, bf16_round as _bf        # noqa: F401
 from .devbuf import DevBuf, upload_table
+from .gradnorm import ctl_ptr
 from . import muon_ns
 from .muon_ns import NTM, _KELLER, NsWorkspace
 
@@ -258,7 +259,7 @@ class MuonEngine:
         `device_steps`: the step count lives in the guard's control block (see `AdamW.launch`); the
         kernels form the rounding seed from it and `t` here is left alone."""
         schedule = muon_ns._resolve(schedule)
-        ctl = 0 if guard is None else guard.ptr
+        ctl = ctl_ptr(guard)
         lr_scales = (ctypes.c_float * MUON_MAX_SCALES)(*[lr * s for s in self.scales])
         if device_steps:
             if guard is None:
@@ -451,7 +452,7 @@ class ResidentMuon:
     def step(self, g_dev, si, lr=0.02, schedule=_KELLER, guard=None):
         """g_dev: (K,N) device weight-gradient (float32, or uint16 bf16 bits)."""
         K, N, sc = self.K, self.N, self.sc
-        ctl = 0 if guard is None else guard.ptr
+        ctl = ctl_ptr(guard)
         schedule = muon_ns._resolve(schedule)
         mode = muon_ns.effective_mode(self.mode, schedule)
         if mode != "fp32" and self.ns >= 2:

@@ -186,6 +186,12 @@ int anc_gradnorm_partials_multi(uint64_t desc_table, int32_t n_tensors,
 int anc_gradnorm_finalize(uint64_t partials, int64_t n_partials,
                           float max_norm, float eps, int32_t count_step,
                           uint64_t ctl /* anc_step_ctl_t* */, uint64_t stream);
+/* anc_gradnorm_partials_multi (unless n_tensors is 0: all partials are in place) and anc_gradnorm_finalize in one call.
+ * host_ctl: 0, or an anc_step_ctl_t in pinned host memory (anc_host_alloc) that receives a copy of the block; it may be
+ * read once the stream has been waited for. */
+int anc_gradnorm_compute(uint64_t desc_table, int32_t n_tensors, int64_t total_chunks, uint64_t partials,
+                         int64_t n_partials, float max_norm, float eps, int32_t count_step,
+                         uint64_t ctl /* anc_step_ctl_t* */, uint64_t host_ctl, uint64_t stream);
 
 /* The same norm for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc): no counterpart in the reference. One

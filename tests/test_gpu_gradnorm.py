@@ -130,3 +130,37 @@ def test_clip_scale_feeds_adamw(gpu):
     ref.step({"x": g}, clip=c["clip_scale"])
     assert max_ulp(opt.master()["x"], ref.st["x"]["p"]) == 0
     gdev.free(); guard.free(); opt.free()
+
+
+@pytest.mark.parametrize("touch", ["nothing", "set_t", "address"])
+def test_host_copy_of_the_block_follows_the_block(gpu, touch):
+    """`read` takes the copy that `compute` left in host memory unless the block may have been written since: by
+    `set_t`, or by someone who was given its address."""
+    from ancora_cutile_amd import StepGuard, DevBuf
+    rng = np.random.default_rng(5)
+    guards = [StepGuard(1.0) for _ in range(70)]                     # more than one page of copies
+    g = DevBuf(rng.standard_normal(4096).astype(np.float32))
+    bad = DevBuf(np.full(4096, np.inf, np.float32))
+    guard = guards[-1]
+    guard.compute([g], 0, count_step=True)
+    guard.compute([bad], 0, count_step=True)
+    c = guard.read(0)
+    assert c["skip"] and c["t"] == 1
+    guards[0].compute([g], 0)
+    assert not guards[0].read(0)["skip"] and guard.read(0)["skip"]
+    if touch == "set_t":
+        guard.set_t(41)
+        assert guard.read(0)["t"] == 41
+    elif touch == "address":
+        raw = guard.ctl.to_numpy()
+        raw[5] = 17
+        guard.ctl.upload(raw)
+        assert guard.read(0)["t"] == 17
+    guard.compute([g], 0, count_step=True)
+    c = guard.read(0)
+    assert not c["skip"] and c["t"] == {"nothing": 2, "set_t": 42, "address": 18}[touch]
+    assert bits_equal(guard.ctl.to_numpy()[:2].view(np.float64), np.float64(c["sumsq"]).reshape(1))
+    for x in guards:
+        x.free()
+    g.free()
+    bad.free()
