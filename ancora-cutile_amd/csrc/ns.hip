@@ -736,7 +736,10 @@ struct ChainProb {
 //               6 x (512,1536) 124 / 142 / 166 (1152), 2 x (1024,3072) 151 / 136 / 148 (1536),
 //               3 x (1024,3072) 202 / 193 / 199 (2304), 4 x (1024,3072) 258 / 222 / 211 (3072)
 // hence 64 below 800 (symmetric), or below 1400 tiles of 64 except from 800 to 1024, where one tile of 128 per
-// CU does; 128 up to 2200 (symmetric) or 2700.
+// CU does; 128 up to 2200 (symmetric) or 2700. The large tiles fill the chip once at 4096; just beyond, 128 again:
+//   A = X X^T   26 x (1024,1024) 374 / 430 on 128 / 256 (4160), 48 x (768,768) 535 / 569 (4608),
+//               22 x (1280,1280) 558 / 535 (5280);   X = a X + B X   33 x (768,768) 474 / 499 (4752),
+//               20 x (1024,1024) 370 / 392 (5120), 26 x (1024,1024) 515 / 487 (6656)
 int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
@@ -745,6 +748,7 @@ int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
     const double per = epi == EPI_BX ? m * (double)(ps[k].N / 64) : m * (m + d) / 2.0;
     t64 += (double)Es[k] * per * ((double)ps[k].K / longest);
   }
+  if (t64 > 4096.0 && t64 <= 4900.0) return 128;      // a second round of large tiles that is nearly empty
   if (epi != EPI_BX) return t64 < 800.0 ? 64 : t64 <= 2200.0 ? 128 : 256;
   if (t64 < 1400.0 && !(t64 > 800.0 && t64 <= 1024.0)) return 64;
   return t64 <= 2700.0 ? 128 : 256;
