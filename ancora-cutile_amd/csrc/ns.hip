@@ -20,12 +20,11 @@
 // split_plan below) late iterations add the residual products: A gets Xh Xl^T + Xl Xh^T and
 // B X gets Boff Xl as extra accumulation terms of the same tile. The symmetric products are
 // "NT" (both operands K-contiguous rows of X or F); B X reads the iterate as (k, n) tiles
-// and transposes inside LDS reads, so no transposed copy of X exists. The 256-tile kernels
-// keep every matrix the chain writes for itself in panel layout (32-column panels, see NsGemm);
-// the input pair and everything the 128-tile kernels touch is row-major. The
+// and transposes inside LDS reads, so no transposed copy of X exists. Every matrix the chain
+// writes for itself is in panel layout (32-column panels, see NsGemm); the input pair is row-major. The
 // fp32 input is read once (normalisation) and the fp32 result written once (last step).
 //
-// Determinism: one workgroup owns one 128x128 output tile and its whole K loop, terms in
+// Determinism: one workgroup owns one output tile (64 to 256 wide) and its whole K loop, terms in
 // a fixed order, K tiles in ascending order; no split-K, no atomics. A matrix's result
 // does not depend on the batch size E or on its position in the batch. Symmetric outputs
 // (A, B) compute the tiles on or below the diagonal and mirror them; without residual terms
@@ -34,12 +33,8 @@
 // Xl Xh^T enter one accumulator in a fixed order, so elements computed directly inside a
 // diagonal tile differ from their mirror images in the last bits; nothing depends on it.
 //
-// GEMM tile: 128x128x64, 256 lanes = 4 wavefronts in 2x2, each 64x64 as 2x2
-// v_mfma_f32_32x32x16_bf16 blocks (fp32 accumulate). Operand tiles are staged through LDS
-// with a 144-byte row pitch (16-byte fragment reads of 16 consecutive rows hit 64 distinct
-// banks); the next K tile is fetched into registers while the current one is multiplied.
-// Workgroup ids are remapped so that consecutive tiles -- the tiles of one matrix -- run on
-// the same XCD and share its L2.
+// The products run on the tiles of ns_gemm_big.hip (256 wide) and ns_gemm_tile.hip (128 and 64 wide), chosen per
+// launch by the number of tiles (pick_tile); the bits are the same on all of them.
 #include <vector>
 
 #include "reduce.h"

@@ -519,13 +519,13 @@ int anc_quant_mxfp8_w_multi(uint64_t desc_table, int32_t n_weights, int64_t tota
 #define ANC_NS_BF16_FAST 2
 #define ANC_NS_BF16_X3 3
 #define ANC_NS_BF16_LATE3 4
-/* Flag OR-ed into a bf16 mode: use the 128x128-tile GEMM kernel even where the 256x256-tile
- * kernel applies. The two produce the same bits in ANC_NS_BF16_FAST (no residual terms). Residual
- * terms are added in an order that depends on which elements of a symmetric product are computed
- * and which are mirrored, hence on the tile size: the results then differ in the last fp32 bits
- * of A and B (1e-6 .. 4e-4 of the result, largest on gated outlier-column inputs). ANC_NS_BF16 on
- * N >= 2M keeps 8-bit low halves of the iterate with the 256-tile kernels only: the 24-bit iterate
- * differs from the 32-bit pair by 2^-16 per element, which the chain turns into another
+/* Flag OR-ed into a bf16 mode: treat a matrix whose dims are multiples of 256 like one whose dims are not. Its
+ * products then run on 128-wide tiles with diagonal blocks of 128 computed in full (256 otherwise; everything
+ * below is mirrored), and N >= 2M keeps 16-bit low halves of the iterate instead of 8-bit ones. Without residual
+ * terms (ANC_NS_BF16_FAST) the bits are the same. Residual terms are added in an order that
+ * depends on which elements of a symmetric product are computed and which are mirrored: the results then differ in
+ * the last fp32 bits of A and B (1e-6 .. 4e-4 of the result, largest on gated outlier-column inputs). The other
+ * low halves differ by 2^-16 per element, which the chain turns into another
  * realisation of its rounding error (the results are then 1.2e-3 apart, each inside the accuracy
  * bar). The flag exists so that tests can show both. */
 #define ANC_NS_TILE128 0x100
