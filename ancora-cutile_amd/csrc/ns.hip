@@ -35,6 +35,7 @@
 //
 // The products run on the tiles of ns_gemm_big.hip (256 wide) and ns_gemm_tile.hip (128 and 64 wide), chosen per
 // launch by the number of tiles (pick_tile); the bits are the same on all of them.
+#include <cfloat>
 #include <vector>
 
 #include "reduce.h"
@@ -170,11 +171,13 @@ k_fro_finalize(const double *__restrict__ partials, int nchunks, float eps, floa
   if (threadIdx.x == 0) recip[blockIdx.x] = 1.0f / ((float)sqrt(t) + eps);
 }
 
-// The same for the bf16 pairs of up to kMaxGroups batches in one launch. A matrix whose sum of squares is below
-// 2^-100 (products of its elements would underflow fp32 in the first A = U U^T) is multiplied in place by
-// the power of two 2^k that brings ||U|| into [1, 2), exactly, and its reciprocal carries 2^-k, so the
-// first step sees the same scale*U as without. One launch instead of two per batch: 7 batches of a small model
-// took 52 us of launches here.
+// The same for the bf16 pairs of up to kMaxGroups batches in one launch. The first step multiplies the input as it
+// is, A = scale^2 * (U U^T), so U has to lie where neither those products nor scale^2 leave the fp32 range: a matrix
+// whose sum of squares is outside 2^-100 .. 2^100 is multiplied in place by the power of two 2^k that brings ||U||
+// into [1, 2), and its reciprocal carries 2^-k, so the first step sees the same scale*U as without. (Exact but for
+// elements 2^-126 of the norm and less, which become subnormal.) Partial sums that are not finite, from runs of
+// squares added up in fp32, are replaced by a sum over the matrix itself. One launch instead of two per batch: 7
+// batches of a small model took 52 us of launches here.
 struct NsPrologue {
   int n;
   int blocks[kMaxGroups];            // matrices per batch
@@ -185,20 +188,36 @@ struct NsPrologue {
   uint32_t *zero16[kMaxGroups];                    // whose substitute this kernel clears
   int64_t mn[kMaxGroups];
 };
+// Sum of squares of one matrix, every square and sum in fp64: lane t adds the 8-element vectors t, t+256, ... in
+// order; butterfly; 4 wavefronts in order. `lo` null: no low half.
+__device__ __forceinline__ double pair_sum(const uint16_t *hi, const uint16_t *lo, int64_t mn) {
+  __shared__ double wave_sum[kThreads / 64];
+  double acc = 0.0;
+  for (int64_t o = (int64_t)threadIdx.x * 8; o < mn; o += (int64_t)kThreads * 8)
+    for (int i = 0; i < 8; ++i) {
+      const double x = (double)anc_bf16_bits_to_f32(hi[o + i]) + (lo == nullptr ? 0.0 : (double)anc_bf16_bits_to_f32(lo[o + i]));
+      acc = acc + x * x;
+    }
+  acc = anc_wave_sum_f64(acc);
+  if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  double t = wave_sum[0];
+#pragma unroll
+  for (int w = 1; w < kThreads / 64; ++w) t = t + wave_sum[w];
+  return t;
+}
 __global__ void __launch_bounds__(kThreads) k_pair_prologue(NsPrologue a, float eps) {
   int e = (int)blockIdx.x, q = 0;
   while (q + 1 < a.n && e >= a.blocks[q]) { e -= a.blocks[q]; ++q; }
-  const double t = fro_sum(a.partials[q] + (int64_t)e * a.nchunks[q], a.nchunks[q]);
-  float r = 1.0f / ((float)sqrt(t) + eps), sc = 1.0f;
-  if (t > 0.0 && t < 0x1p-100) {
-    const int k = -ilogb(sqrt(t));
-    sc = ldexpf(1.0f, k);
-    r = ldexpf(r, -k);
-  }
+  double t = fro_sum(a.partials[q] + (int64_t)e * a.nchunks[q], a.nchunks[q]);
+  const int64_t mn = a.mn[q];
+  if (!(t <= DBL_MAX)) t = pair_sum(a.Uh[q] + (int64_t)e * mn, a.Ul[q] == nullptr ? nullptr : a.Ul[q] + (int64_t)e * mn, mn);
+  int k = 0;
+  if (t > 0.0 && t <= DBL_MAX && !(t >= 0x1p-100 && t <= 0x1p100)) k = -ilogb(sqrt(t));
+  const float r = 1.0f / ((float)ldexp(sqrt(t), k) + ldexpf(eps, k));       // (of the matrix times 2^k)
   if (threadIdx.x == 0) a.recip[q][e] = r;
   if (a.Ul[q] == nullptr && e == 0 && threadIdx.x < 4) a.zero16[q][threadIdx.x] = 0u;
-  if (sc == 1.0f) return;            // (uniform over the block)
-  const int64_t mn = a.mn[q];
+  if (k == 0) return;                // (uniform over the block)
   for (int64_t o = (int64_t)threadIdx.x * 8; o < mn; o += (int64_t)kThreads * 8) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -208,7 +227,7 @@ __global__ void __launch_bounds__(kThreads) k_pair_prologue(NsPrologue a, float 
       uint32_t u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float lo = __uint_as_float(u[i] << 16) * sc, hi = __uint_as_float(u[i] & 0xFFFF0000u) * sc;
+        const float lo = ldexpf(__uint_as_float(u[i] << 16), k), hi = ldexpf(__uint_as_float(u[i] & 0xFFFF0000u), k);
         u[i] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
       }
       *(anc_u32x4 *)p = anc_u32x4{u[0], u[1], u[2], u[3]};

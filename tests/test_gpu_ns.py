@@ -224,6 +224,50 @@ def test_bf16_entry_takes_the_matrix_as_it_is(gpu, E, M, N, sched):
     g.free()
 
 
+@pytest.mark.parametrize("M,N", [(128, 384), (1024, 2048)])
+@pytest.mark.parametrize("sched", ["pe", "keller"])
+def test_bf16_entry_takes_large_magnitudes(gpu, M, N, sched):
+    """Products of elements beyond 1e17 overflow fp32 and beyond 6e18 so do the runs of squares in the norm: up to the
+    largest bf16 numbers the matrix has the result of its multiple of ordinary size, and its neighbour in the
+    batch keeps its bits."""
+    from ancora_cutile_amd import DevBuf, newton_schulz_resident_e
+    schedule = PE_SCHEDULE if sched == "pe" else None
+    rng = np.random.default_rng(M + N)
+    bits = bf16_rne_bits(rng.standard_normal((2 * M, N)).astype(np.float32)).reshape(2, M, N)
+    x = bits_to_f32(bits).reshape(2, M, N)
+    want = [host_ns(x[e], schedule, 5) for e in range(2)]
+    first = None
+    for k in (0, 58, 62, 100, 124):
+        b = bits.copy()
+        b[1] = bf16_rne_bits(np.ldexp(x[1], k).astype(np.float32)).reshape(M, N)
+        g = DevBuf(b.reshape(2 * M, N))
+        newton_schulz_resident_e(g, None, None, None, None, None, 2, M, N, 0, schedule=schedule)
+        out = g.to_numpy().reshape(2, M, N)
+        g.free()
+        first = out[0] if first is None else first
+        got = bits_to_f32(out).reshape(2, M, N)
+        assert bits_equal(out[0], first), k
+        assert rel_fro(got[1], want[1]) < 2.8e-3, k          # 2e-3 and the bf16 result's 1.7e-3
+
+
+@pytest.mark.parametrize("M,N", [(256, 512), (1024, 1024)])
+def test_pair_entry_takes_the_largest_and_smallest_magnitudes(gpu, M, N):
+    """X * 2^k on the unnormalised bf16 pair, eps = 0: the bits of X, up to where the largest element still fits and,
+    for four single elements, down to the smallest bf16 numbers, where 2^-k itself leaves the fp32 range."""
+    rng = np.random.default_rng(M + N)
+    X = bits_to_f32(bf16_rne_bits(rng.standard_normal((2, M, N)).astype(np.float32))).reshape(2, M, N)
+    few = X.copy()
+    few[1] = 0.0
+    few[1, [0, 3, 100, 255], [7, 0, 511 % N, 64]] = 1.0
+    for x, ks in ((X, (58, 100, 124)), (few, (125, -130, -133))):
+        want = _pair_run(x, 0.0)
+        assert np.all(np.isfinite(want))
+        for k in ks:
+            y = x.copy()
+            y[1] = np.ldexp(x[1], k)
+            assert bits_equal(_pair_run(y, 0.0), want), k
+
+
 def test_zero_matrix_and_scale_invariance(gpu):
     """A zero gradient (an idle expert) stays zero, no NaN; NS(cX) == NS(X) up to rounding."""
     rng = np.random.default_rng(3)

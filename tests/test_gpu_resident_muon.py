@@ -117,6 +117,28 @@ def test_resident_muon_shares_one_scratch_across_shapes(gpu, gdtype):
     sc.free()
 
 
+@pytest.mark.parametrize("K,N", [(256, 512), (2048, 1024)])
+@pytest.mark.parametrize("size", [1e18, 1e30])
+def test_resident_muon_takes_gradients_of_any_magnitude(gpu, K, N, size):
+    """Gradients whose products leave the fp32 range: the update is that of the same gradient at ordinary size (the
+    orthogonalised step has no scale), and nothing of it is NaN."""
+    from ancora_cutile_amd import ResidentMuon, MuonScratch, DevBuf
+    rng = np.random.default_rng(K)
+    W0 = (0.05 * rng.standard_normal((K, N))).astype(np.float32)
+    g = rng.standard_normal((K, N)).astype(np.float32)
+    host = MuonRef({"w": W0}, lr=0.02, momentum=0.95, ns_steps=5, sched=PE_SCHEDULE)
+    host.step({"w": g})
+    sc = MuonScratch([(K, N)])
+    p32, p16, gd = DevBuf(W0.copy()), DevBuf.zeros((K, N), np.uint16), DevBuf(g * np.float32(size))
+    rm = ResidentMuon(p32, p16, K, N, sc, momentum=0.95, ns_steps=5)
+    rm.step(gd, 0, 0.02, schedule=PE_SCHEDULE)
+    got = p32.to_numpy()
+    assert rel_fro(W0 - got, W0 - host.w["w"]) < 2e-3
+    assert bits_equal(p16.to_numpy(), bf16_rne_bits(got))
+    for b in (p32, p16, gd, rm, sc):
+        b.free()
+
+
 def test_device_newton_schulz5_matches_the_host_function(gpu):
     """`newton_schulz5(G)`: host matrix in, host matrix out, Keller by default, tall inputs
     transposed in and out (ancora/optim/muon.py:67-80)."""
