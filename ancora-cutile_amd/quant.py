@@ -60,15 +60,18 @@ class Mxfp8WeightCache:
         if not self.w:
             self.dirty = False
             return True
-        key = [s["p16"] for s in self.w.values()]
-        if key != self._key:                       # the descriptor table: once, unless a weight is exchanged
+        key = [(s["p16"].ptr, s["fp8"].ptr, s["scale"].ptr) for s in self.w.values()]
+        if key != self._key:                       # the descriptor table: once, unless an address changes
+            for name, (w, fp8, scale) in zip(self.w, key):
+                if not (w and fp8 and scale) or (w | fp8) % 16 or scale % 8:
+                    raise _lib.AncoraError(f"Mxfp8WeightCache: {name} at {w:#x} with fp8 copy at {fp8:#x} and scales at "
+                                           f"{scale:#x}: freed, or not 16-byte aligned")
             if self._table is not None:
                 self._table.free()
+                self._table = self._key = None
             descs, tiles = [], 0
-            for s in self.w.values():
-                if s["p16"].ptr % 16:
-                    raise ValueError("Mxfp8WeightCache: weights must be 16-byte aligned")
-                descs.append(QuantDesc(s["p16"].ptr, s["fp8"].ptr, s["scale"].ptr, tiles, s["K"], s["N"]))
+            for s, (w, fp8, scale) in zip(self.w.values(), key):
+                descs.append(QuantDesc(w, fp8, scale, tiles, s["K"], s["N"]))
                 tiles += api.anc_quant_mxfp8_num_tiles(s["E"], s["K"], s["N"])
             self._table, self._tiles, self._key = upload_table(descs), tiles, key
         api.anc_quant_mxfp8_w_multi(self._table.ptr, len(self.w), self._tiles, int(self.col_major), int(si))
