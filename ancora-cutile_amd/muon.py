@@ -51,7 +51,13 @@ def _f32bf_trunc(x):
     return (np.ascontiguousarray(x, dtype=np.float32).view(np.uint32) >> np.uint32(16)).astype(np.uint16)
 
 
-_bufs_of = itemgetter("G", "p32", "p16", "buf", "p16T")     # what a descriptor is made of
+_bufs_of = itemgetter("G", "p32", "p16", "buf", "p16T")
+
+
+def _made_of(weights):
+    """What the descriptors of `weights` are made of: addresses, which a buffer object does not keep for life (`free`)
+    and another object may share, and the gradients' types."""
+    return [b and b.ptr for w in weights for b in _bufs_of(w)], [w["G"].dtype for w in weights]
 
 
 def _descs(weights, M, Nn, u_ptr, scale_index, blk0):
@@ -59,6 +65,8 @@ def _descs(weights, M, Nn, u_ptr, scale_index, blk0):
     out = []
     for i, w in enumerate(weights):
         K, N = w["K"], w["N"]
+        if not (w["buf"].ptr and w["G"].ptr and w["p32"].ptr):
+            raise _lib.AncoraError(f"Muon: momentum, gradient or master of weight {w.get('name', i)} ({K},{N}) was freed")
         out.append(MuonDesc(w["buf"].ptr, w["G"].ptr, w["p32"].ptr,
                             w["p16"].ptr if w["p16"] is not None else 0,
                             u_ptr + i * M * Nn * 4, K, N, int(K > N),
@@ -80,12 +88,12 @@ class _Batch:
         self.fro = None              # per-block sums of u*u left by the pair momentum kernel
 
     def build(self, U, scale_index):
-        key = [_bufs_of(w) for w in self.weights] + [U]
+        key = _made_of(self.weights), U.ptr
         if key == self.key:
             return
+        descs, self.total_blocks = _descs(self.weights, self.M, self.Nn, U.ptr, scale_index, 0)
         if self.table is not None:
             self.table.free()
-        descs, self.total_blocks = _descs(self.weights, self.M, self.Nn, U.ptr, scale_index, 0)
         self.table = upload_table(descs)
         self.key = key
 
@@ -135,15 +143,15 @@ class _Group:
             self.calls.append((probs, len(part), tables))
 
     def prepare(self, mode):
-        key = list(map(_bufs_of, self.weights))
+        key = _made_of(self.weights)
         if key != self.key:
-            if self.table is not None:
-                self.table.free()
             descs, el, blk = [], 0, 0
             for b in self.batches:
                 d, blk = _descs(b.weights, b.M, b.Nn, self.arena.ptr + el * 4, self.scale_index, blk)
                 descs += d
                 el += b.E * b.M * b.Nn
+            if self.table is not None:
+                self.table.free()
             self.table = upload_table(descs)
             self.key, self.mode = key, None
         if self.mode != (mode, [b.ws.buf for b in self.batches]):

@@ -41,3 +41,60 @@ def test_fp8_cache_follows_its_weights_addresses(fake_device):
         cache.refresh(0)
     assert cache.dirty and len(fake_device.calls("anc_quant_mxfp8_w_multi")) == n
     cache.free()
+
+
+def _muon_weights(dev, shapes):
+    from ancora_cutile_amd import DevBuf
+    return [dict(buf=DevBuf.zeros((K, N), np.float32), p32=DevBuf.zeros((K, N), np.float32),
+                 p16=DevBuf.zeros((K, N), np.uint16), G=DevBuf.zeros((K, N), np.float32), K=K, N=N) for K, N in shapes]
+
+
+@pytest.mark.parametrize("fused_update", [True, False])
+def test_muon_tables_follow_the_weights_addresses(fake_device, fused_update):
+    """One table for many steps, also with fresh views of the same memory; another one when a gradient's address or
+    type changes, in the same object or another; a freed buffer is refused and nothing launched. With the
+    group's table and with a table per batch."""
+    from ancora_cutile_amd import DevBuf, _lib
+    from ancora_cutile_amd.muon import MuonEngine
+    ws = _muon_weights(fake_device, [(128, 256), (256, 128), (128, 128)])
+    eng = MuonEngine(ws, chunk=None)
+    eng.fused_update = fused_update
+    G = ws[1]["G"]
+
+    def step():
+        """(table, weights) of each momentum launch"""
+        n = len(fake_device.calls("anc_muon_momentum_multi_pair"))
+        eng.step(0)
+        return [a[:2] for a in fake_device.calls("anc_muon_momentum_multi_pair")[n:]]
+
+    def entry(launches):
+        """(gradient's address, its type) of weight 1"""
+        for ptr, n in launches:
+            raw = bytes(fake_device.at(ptr, ctypes.sizeof(_lib.MuonDesc) * n))
+            for i in range(n):
+                d = _lib.MuonDesc.from_buffer_copy(raw, i * ctypes.sizeof(_lib.MuonDesc))
+                if d.buf == ws[1]["buf"].ptr:
+                    return d.g, d.g_dtype
+
+    first = step()
+    assert len(first) == (1 if fused_update else 2) and entry(first) == (G.ptr, _lib.F32)
+    ws[1]["G"] = G.view((256, 128))
+    assert step() == first
+    ws[1]["G"] = G.view((256, 128), np.uint16)
+    assert entry(step()) == (G.ptr, _lib.BF16)
+    other = DevBuf.zeros((256, 128), np.uint16)
+    ws[1]["G"].ptr = other.ptr
+    assert entry(step()) == (other.ptr, _lib.BF16)
+    ws[1]["G"] = G
+    before = step()
+    assert entry(before) == (G.ptr, _lib.F32)
+    for key in ("buf", "G", "p32"):
+        keep, n = ws[2][key], len(fake_device.calls("anc_muon_ns_update_multi"))
+        ws[2][key] = keep.view(keep.shape)
+        ws[2][key].free()
+        with pytest.raises(_lib.AncoraError):
+            eng.step(0)
+        assert len(fake_device.calls("anc_muon_ns_update_multi")) == n
+        ws[2][key] = keep
+    assert step() == before
+    eng.free()
