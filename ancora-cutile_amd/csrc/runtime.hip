@@ -166,21 +166,41 @@ extern "C" int anc_fill_u32(uint64_t dptr, uint32_t value, int64_t n_words, uint
 // 57, and blocks until everything before it on the stream is done. So a source is copied slot by slot into pinned
 // memory, the DMA of one slot under the copy into the next, and the call can return as soon as the last slot
 // is filled. 4 MiB: 132 -> 95 us. A source beyond the caches is read at 32 GB/s by one thread, so from 8 MiB on
-// four threads copy, two slots each. A slot is taken again once the event behind its last DMA has passed. The
-// ring is shared by all threads and streams (4 MiB, pinned slot by slot on first use, given back by
-// anc_staging_release).
+// four threads copy, two slots each. A slot is taken again once the event behind its last DMA has passed. Events
+// and streams belong to a device, so every device has a ring of its own, shared by all threads and streams (4 MiB,
+// pinned slot by slot on first use, given back by anc_staging_release).
 namespace {
-constexpr int kSlots = 8, kCopyThreads = 4;
+constexpr int kSlots = 8, kCopyThreads = 4, kMaxDevices = 32;
 constexpr int64_t kSlotBytes = 512 << 10, kThreadedBytes = 8 << 20;
 struct StageSlot {
   void *mem = nullptr;
   hipEvent_t done = nullptr;
   bool busy = false;
 };
-std::mutex g_stage_mu;
-StageSlot g_stage[kSlots];
-int g_stage_next = 0;
-hipStream_t g_stage_stream = nullptr;     // for uploads that are complete on return without waiting for anybody's work
+struct StageRing {
+  std::mutex mu;
+  StageSlot slot[kSlots];
+  int next = 0;
+  hipStream_t own = nullptr;     // for uploads that are complete on return without waiting for anybody's work
+};
+StageRing g_ring[kMaxDevices];
+
+// The device a stream belongs to is current while this lives (the null stream's is the current one already).
+struct OnDeviceOf {
+  int dev = 0, before = -1;
+  int enter(hipStream_t s) {
+    int cur = 0;
+    ANC_HIP(hipGetDevice(&cur));
+    dev = cur;
+    if (s != nullptr && s != hipStreamLegacy && s != hipStreamPerThread) ANC_HIP(hipStreamGetDevice(s, &dev));
+    ANC_REQUIRE(dev >= 0 && dev < kMaxDevices, "upload: device %d beyond %d", dev, kMaxDevices - 1);
+    if (dev == cur) return ANC_OK;
+    ANC_HIP(hipSetDevice(dev));
+    before = cur;
+    return ANC_OK;
+  }
+  ~OnDeviceOf() { if (before >= 0) (void)hipSetDevice(before); }
+};
 
 int slot_copy(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
   if (slot.mem == nullptr) {
@@ -199,8 +219,8 @@ int slot_copy(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hip
   slot.busy = true;
   return ANC_OK;
 }
-// Every slot's copy into place is queued on `s` on return.
-int stage_upload(uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
+// Every slot's copy into place is queued on `s` on return. The ring's device is current.
+int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
   const int64_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes;
   auto piece = [&](StageSlot &slot, int64_t c) {
     const int64_t at = c * kSlotBytes, left = bytes - at;
@@ -208,18 +228,16 @@ int stage_upload(uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
   };
   if (bytes < kThreadedBytes) {
     for (int64_t c = 0; c < pieces; ++c) {
-      if (int rc = piece(g_stage[g_stage_next], c)) return rc;
-      g_stage_next = (g_stage_next + 1) % kSlots;
+      if (int rc = piece(r.slot[r.next], c)) return rc;
+      r.next = (r.next + 1) % kSlots;
     }
     return ANC_OK;
   }
-  int dev = 0;
-  ANC_HIP(hipGetDevice(&dev));
   int rcs[kCopyThreads] = {};
   char errs[kCopyThreads][sizeof(g_err)] = {};
   auto work = [&](int k) {
     for (int64_t c = k; c < pieces && rcs[k] == 0; c += kCopyThreads)
-      rcs[k] = piece(g_stage[2 * k + (int)((c / kCopyThreads) & 1)], c);
+      rcs[k] = piece(r.slot[2 * k + (int)((c / kCopyThreads) & 1)], c);
     if (rcs[k] != 0) memcpy(errs[k], g_err, sizeof(g_err));       // (the message is the thread's own)
   };
   std::thread th[kCopyThreads - 1];
@@ -242,37 +260,48 @@ static_assert(kSlots == 2 * kCopyThreads, "two slots per copying thread");
 extern "C" int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream) {
   ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_upload_async: bad arguments");
   if (bytes == 0) return ANC_OK;
-  std::lock_guard<std::mutex> lk(g_stage_mu);
-  return stage_upload(dst, src, bytes, anc_stream(stream));
+  OnDeviceOf on;
+  if (int rc = on.enter(anc_stream(stream))) return rc;
+  StageRing &r = g_ring[on.dev];
+  std::lock_guard<std::mutex> lk(r.mu);
+  return stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream));
 }
 extern "C" int anc_upload_now(uint64_t dst, const void *src, int64_t bytes) {
   ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_upload_now: bad arguments");
   if (bytes == 0) return ANC_OK;
-  std::lock_guard<std::mutex> lk(g_stage_mu);
-  if (g_stage_stream == nullptr) ANC_HIP(hipStreamCreateWithFlags(&g_stage_stream, hipStreamNonBlocking));
-  if (int rc = stage_upload(dst, src, bytes, g_stage_stream)) return rc;
-  ANC_HIP(hipStreamSynchronize(g_stage_stream));
+  OnDeviceOf on;
+  if (int rc = on.enter(nullptr)) return rc;
+  StageRing &r = g_ring[on.dev];
+  std::lock_guard<std::mutex> lk(r.mu);
+  if (r.own == nullptr) ANC_HIP(hipStreamCreateWithFlags(&r.own, hipStreamNonBlocking));
+  if (int rc = stage_upload(r, on.dev, dst, src, bytes, r.own)) return rc;
+  ANC_HIP(hipStreamSynchronize(r.own));
   return ANC_OK;
 }
 extern "C" int anc_staging_release(void) {
-  std::lock_guard<std::mutex> lk(g_stage_mu);
-  for (StageSlot &slot : g_stage) {
-    if (slot.mem == nullptr) continue;
-    if (slot.busy) ANC_HIP(hipEventSynchronize(slot.done));
-    ANC_HIP(hipEventDestroy(slot.done));
-    ANC_HIP(hipHostFree(slot.mem));
-    slot = StageSlot{};
+  for (StageRing &r : g_ring) {
+    std::lock_guard<std::mutex> lk(r.mu);
+    for (StageSlot &slot : r.slot) {
+      if (slot.mem == nullptr) continue;
+      if (slot.busy) ANC_HIP(hipEventSynchronize(slot.done));
+      ANC_HIP(hipEventDestroy(slot.done));
+      ANC_HIP(hipHostFree(slot.mem));
+      slot = StageSlot{};
+    }
+    if (r.own != nullptr) ANC_HIP(hipStreamDestroy(r.own));
+    r.own = nullptr;
   }
-  if (g_stage_stream != nullptr) ANC_HIP(hipStreamDestroy(g_stage_stream));
-  g_stage_stream = nullptr;
   return ANC_OK;
 }
 extern "C" int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint64_t stream) {
   ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_memcpy_h2d: bad arguments");
   if (bytes == 0) return ANC_OK;
   if (bytes <= 2 * kSlotBytes) {
-    std::lock_guard<std::mutex> lk(g_stage_mu);
-    if (int rc = stage_upload(dst, src, bytes, anc_stream(stream))) return rc;
+    OnDeviceOf on;
+    if (int rc = on.enter(anc_stream(stream))) return rc;
+    StageRing &r = g_ring[on.dev];
+    std::lock_guard<std::mutex> lk(r.mu);
+    if (int rc = stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream))) return rc;
   } else {
     // a state as it is set up, often memory that no one has touched yet: the runtime's own path takes its page
     // faults in larger pieces (622 MB of fresh zeros: 18 ms against 80 through the slots, 5 MB 0.1 ms less)

@@ -74,7 +74,8 @@ int anc_fill_u32(uint64_t dptr, uint32_t value, int64_t n_words, uint64_t stream
 int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
 /* Uploads through pinned staging memory; src may be reused on return. anc_memcpy_h2d: complete on return.
  * _async: ordered on `stream`, no wait. _now: complete on return, on a stream of its own, without
- * waiting for work queued elsewhere; nobody may be using dst. _release gives the staging memory back. */
+ * waiting for work queued elsewhere; nobody may be using dst. Each device has its ring of staging memory, the
+ * stream's device decides (the null stream and _now: the current one); _release gives it all back. */
 int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
 int anc_upload_now(uint64_t dst, const void *src, int64_t bytes);
 int anc_staging_release(void);

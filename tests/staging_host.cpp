@@ -1,0 +1,168 @@
+// The upload entry points of the library (runtime.hip, compiled for the host alone) on a stand-in for the HIP runtime:
+// devices, streams that can be held, events, pageable and pinned memory. Each case checks one property and
+// prints "ok"; a failed check or a call the stand-in refuses ends the program with a message.
+#include <hip/hip_runtime_api.h>
+
+#include <condition_variable>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <deque>
+#include <functional>
+#include <future>
+#include <map>
+#include <mutex>
+#include <set>
+#include <string>
+#include <vector>
+
+extern "C" {
+int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
+int anc_upload_now(uint64_t dst, const void *src, int64_t bytes);
+int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
+int anc_staging_release(void);
+const char *anc_last_error(void);
+}
+
+#define CHECK(c) do { if (!(c)) { printf("line %d: %s (%s)\n", __LINE__, #c, anc_last_error()); exit(1); } } while (0)
+
+// ---- the stand-in
+struct Stream {
+  int dev;
+  bool held = false, capturing = false;
+  std::deque<std::function<void()>> queue;
+};
+struct Event { int dev; bool done = true, captured = false; };
+static std::mutex mu;
+static std::condition_variable cv;
+static Stream null_stream[4] = {{0}, {1}, {2}, {3}};
+static std::set<Event *> events;
+static std::map<char *, size_t> pinned;
+static int live_streams = 0;
+static thread_local int cur = 0;
+static thread_local hipError_t last = hipSuccess;
+
+static hipError_t ret(hipError_t e) { if (e != hipSuccess) last = e; return e; }
+static Stream *str(hipStream_t s) { return s == nullptr ? &null_stream[cur] : (Stream *)s; }
+static void push(Stream *s, std::function<void()> f) {       // mu held
+  if (s->held) s->queue.push_back(f); else f();
+}
+static void release(Stream *s) {
+  std::lock_guard<std::mutex> lk(mu);
+  s->held = false;
+  while (!s->queue.empty()) { s->queue.front()(); s->queue.pop_front(); }
+  cv.notify_all();
+}
+static bool is_pinned(const void *p) {
+  auto it = pinned.upper_bound((char *)p);
+  return it != pinned.begin() && (--it, (char *)p < it->first + it->second);
+}
+static uint64_t handle(Stream *s) { return (uint64_t)s; }
+
+extern "C" {
+hipError_t hipGetDevice(int *d) { *d = cur; return hipSuccess; }
+hipError_t hipSetDevice(int d) { cur = d; return hipSuccess; }
+hipError_t hipGetLastError(void) { hipError_t e = last; last = hipSuccess; return e; }
+const char *hipGetErrorString(hipError_t) { return "refused by the stand-in"; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  std::lock_guard<std::mutex> lk(mu);
+  *p = malloc(n);
+  pinned[(char *)*p] = n;
+  return hipSuccess;
+}
+hipError_t hipHostFree(void *p) { std::lock_guard<std::mutex> lk(mu); pinned.erase((char *)p); free(p); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+  std::lock_guard<std::mutex> lk(mu);
+  Event *n = new Event{cur};
+  events.insert(n);
+  *e = (hipEvent_t)n;
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) { std::lock_guard<std::mutex> lk(mu); events.erase((Event *)e); delete (Event *)e; return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  std::lock_guard<std::mutex> lk(mu);
+  Event *ev = (Event *)e;
+  Stream *st = str(s);
+  if (ev->dev != st->dev) return ret(hipErrorInvalidHandle);       // as the runtime does
+  ev->captured = st->capturing;
+  ev->done = false;
+  push(st, [ev] { ev->done = true; });
+  return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) {
+  std::lock_guard<std::mutex> lk(mu);
+  if (((Event *)e)->captured) return ret(hipErrorCapturedEvent);
+  return ((Event *)e)->done ? hipSuccess : ret(hipErrorNotReady);
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  std::unique_lock<std::mutex> lk(mu);
+  if (((Event *)e)->captured) return ret(hipErrorCapturedEvent);
+  cv.wait(lk, [e] { return ((Event *)e)->done; });
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t s) {
+  std::unique_lock<std::mutex> lk(mu);
+  Stream *st = str(s);
+  if (st->capturing) return hipSuccess;                            // (recorded)
+  if (is_pinned(src)) { push(st, [=] { memcpy(dst, src, n); }); return hipSuccess; }
+  cv.wait(lk, [st] { return !st->held; });                         // pageable: in the stream's turn, and blocking
+  memcpy(dst, src, n);
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) {
+  std::unique_lock<std::mutex> lk(mu);
+  Stream *st = str(s);
+  if (st->capturing) return ret(hipErrorStreamCaptureUnsupported);
+  cv.wait(lk, [st] { return !st->held; });
+  return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = (hipStream_t)new Stream{cur}; ++live_streams; return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { delete (Stream *)s; --live_streams; return hipSuccess; }
+hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t *d) { *d = str(s)->dev; return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c) {
+  *c = str(s)->capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }
+void **__hipRegisterFatBinary(const void *) { return nullptr; }
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, void *, void *, int *) {}
+}
+
+// ---- the cases
+static std::vector<char> bytes(size_t n, int seed) {
+  std::vector<char> v(n);
+  for (size_t i = 0; i < n; ++i) v[i] = (char)(i * 7 + i / 251 + (size_t)seed);
+  return v;
+}
+
+// Uploads of every kind with each device current in turn, and on a stream of another device than the current one:
+// all arrive, and the caller's device stays current.
+static void two_devices() {
+  Stream s[2] = {{0}, {1}};
+  for (int round = 0; round < 2; ++round)
+    for (int dev = 0; dev < 2; ++dev) {
+      cur = dev;
+      for (size_t n : {100u, 600u << 10, 9u << 20}) {
+        const std::vector<char> want = bytes(n, dev + round);
+        for (Stream *on : {&s[0], &s[1], (Stream *)nullptr}) {
+          std::vector<char> src = want, a(n), b(n), c(n);
+          CHECK(anc_upload_async((uint64_t)a.data(), src.data(), (int64_t)n, handle(on)) == 0);
+          CHECK(anc_memcpy_h2d((uint64_t)b.data(), src.data(), (int64_t)n, handle(on)) == 0);
+          CHECK(anc_upload_now((uint64_t)c.data(), src.data(), (int64_t)n) == 0);
+          CHECK(a == want && b == want && c == want && cur == dev);
+        }
+      }
+    }
+  CHECK(pinned.size() == 16 && events.size() == 16 && live_streams == 2);       // 8 slots per device and no more
+  CHECK(anc_staging_release() == 0);
+  CHECK(pinned.empty() && events.empty() && live_streams == 0);
+}
+
+int main(int argc, char **argv) {
+  const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}};
+  if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
+  cases.at(argv[1])();
+  printf("ok\n");
+  return 0;
+}
