@@ -166,22 +166,28 @@ extern "C" int anc_fill_u32(uint64_t dptr, uint32_t value, int64_t n_words, uint
 // 57, and blocks until everything before it on the stream is done. So a source is copied slot by slot into pinned
 // memory, the DMA of one slot under the copy into the next, and the call can return as soon as the last slot
 // is filled. 4 MiB: 132 -> 95 us. A source beyond the caches is read at 32 GB/s by one thread, so from 8 MiB on
-// four threads copy, two slots each. A slot is taken again once the event behind its last DMA has passed. Events
-// and streams belong to a device, so every device has a ring of its own, shared by all threads and streams (4 MiB,
-// pinned slot by slot on first use, given back by anc_staging_release).
+// four threads copy. A slot is taken again once the event behind its last DMA has passed. An upload waits for
+// slots in use on its own stream, where its data queue up behind the same work anyway, and never for those of
+// another: if those hold all of them it goes the pageable way. No lock is held while anyone waits or copies.
+// Events and streams belong to a device, so every device has a ring of its own, shared by all threads and streams
+// (4 MiB, pinned slot by slot on first use, given back by anc_staging_release).
 namespace {
 constexpr int kSlots = 8, kCopyThreads = 4, kMaxDevices = 32;
 constexpr int64_t kSlotBytes = 512 << 10, kThreadedBytes = 8 << 20;
 struct StageSlot {
   void *mem = nullptr;
   hipEvent_t done = nullptr;
-  bool busy = false;
+  hipStream_t user = nullptr;    // the stream of its last DMA,
+  uint64_t turn = 0;             // the older the smaller
+  bool busy = false;             // that DMA was not seen to end yet
+  bool taken = false;            // a call is filling it, or waiting to
 };
 struct StageRing {
-  std::mutex mu;
+  std::mutex mu;                 // guards the flags, not the copies
   StageSlot slot[kSlots];
-  int next = 0;
+  uint64_t turn = 0;
   hipStream_t own = nullptr;     // for uploads that are complete on return without waiting for anybody's work
+  int own_users = 0;
 };
 StageRing g_ring[kMaxDevices];
 
@@ -202,42 +208,91 @@ struct OnDeviceOf {
   ~OnDeviceOf() { if (before >= 0) (void)hipSetDevice(before); }
 };
 
-int slot_copy(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
-  if (slot.mem == nullptr) {
-    ANC_HIP(hipHostMalloc(&slot.mem, (size_t)kSlotBytes, hipHostMallocDefault));
-    if (hipError_t e = hipEventCreateWithFlags(&slot.done, hipEventDisableTiming)) {
-      (void)hipHostFree(slot.mem);
-      slot.mem = nullptr;
-      return anc_hip_fail(e, "hipEventCreateWithFlags", __FILE__, __LINE__);
+// A slot for an upload on `s`: *out stays null if work of other streams holds them all.
+int slot_take(StageRing &r, hipStream_t s, StageSlot **out) {
+  *out = nullptr;
+  StageSlot *mine = nullptr;
+  {
+    std::lock_guard<std::mutex> lk(r.mu);
+    for (StageSlot &slot : r.slot) {
+      if (slot.taken) continue;
+      if (slot.busy) {
+        const hipError_t e = hipEventQuery(slot.done);
+        if (e == hipErrorNotReady) {
+          (void)hipGetLastError();          // (not an error: a launch check must not find it)
+          if (slot.user == s && (mine == nullptr || slot.turn < mine->turn)) mine = &slot;
+          continue;
+        }
+        ANC_HIP(e);
+      }
+      slot.busy = false;
+      slot.taken = true;
+      *out = &slot;
+      return ANC_OK;
     }
+    if (mine == nullptr) return ANC_OK;
+    mine->taken = true;
   }
-  if (slot.busy) ANC_HIP(hipEventSynchronize(slot.done));
-  slot.busy = false;
-  memcpy(slot.mem, src, (size_t)bytes);
-  ANC_HIP(hipMemcpyAsync((void *)dst, slot.mem, (size_t)bytes, hipMemcpyHostToDevice, s));
-  ANC_HIP(hipEventRecord(slot.done, s));
-  slot.busy = true;
+  const hipError_t e = hipEventSynchronize(mine->done);
+  if (e != hipSuccess) {
+    std::lock_guard<std::mutex> lk(r.mu);
+    mine->taken = false;
+  }
+  ANC_HIP(e);
+  *out = mine;
   return ANC_OK;
 }
-// Every slot's copy into place is queued on `s` on return. The ring's device is current.
+int slot_fill(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
+  if (slot.mem == nullptr) {
+    void *mem = nullptr;
+    ANC_HIP(hipHostMalloc(&mem, (size_t)kSlotBytes, hipHostMallocDefault));
+    if (hipError_t e = hipEventCreateWithFlags(&slot.done, hipEventDisableTiming)) {
+      (void)hipHostFree(mem);
+      return anc_hip_fail(e, "hipEventCreateWithFlags", __FILE__, __LINE__);
+    }
+    slot.mem = mem;
+  }
+  memcpy(slot.mem, src, (size_t)bytes);
+  ANC_HIP(hipMemcpyAsync((void *)dst, slot.mem, (size_t)bytes, hipMemcpyHostToDevice, s));
+  if (hipError_t e = hipEventRecord(slot.done, s)) {
+    (void)hipStreamSynchronize(s);          // nothing marks the end of that copy
+    return anc_hip_fail(e, "hipEventRecord", __FILE__, __LINE__);
+  }
+  return ANC_OK;
+}
+// Up to a slot's worth: on return `src` may be reused and the copy into place is queued on `s`, or done.
+int stage_piece(StageRing &r, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
+  StageSlot *slot;
+  if (int rc = slot_take(r, s, &slot)) return rc;
+  if (slot == nullptr) {
+    ANC_HIP(hipMemcpyAsync((void *)dst, src, (size_t)bytes, hipMemcpyHostToDevice, s));
+    ANC_HIP(hipStreamSynchronize(s));
+    return ANC_OK;
+  }
+  const int rc = slot_fill(*slot, dst, src, bytes, s);
+  std::lock_guard<std::mutex> lk(r.mu);
+  slot->busy = rc == ANC_OK;
+  slot->user = s;
+  slot->turn = ++r.turn;
+  slot->taken = false;
+  return rc;
+}
+// The ring's device is current.
 int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
   const int64_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes;
-  auto piece = [&](StageSlot &slot, int64_t c) {
+  auto piece = [&](int64_t c) {
     const int64_t at = c * kSlotBytes, left = bytes - at;
-    return slot_copy(slot, dst + (uint64_t)at, (const char *)src + at, left < kSlotBytes ? left : kSlotBytes, s);
+    return stage_piece(r, dst + (uint64_t)at, (const char *)src + at, left < kSlotBytes ? left : kSlotBytes, s);
   };
   if (bytes < kThreadedBytes) {
-    for (int64_t c = 0; c < pieces; ++c) {
-      if (int rc = piece(r.slot[r.next], c)) return rc;
-      r.next = (r.next + 1) % kSlots;
-    }
+    for (int64_t c = 0; c < pieces; ++c)
+      if (int rc = piece(c)) return rc;
     return ANC_OK;
   }
   int rcs[kCopyThreads] = {};
   char errs[kCopyThreads][sizeof(g_err)] = {};
   auto work = [&](int k) {
-    for (int64_t c = k; c < pieces && rcs[k] == 0; c += kCopyThreads)
-      rcs[k] = piece(r.slot[2 * k + (int)((c / kCopyThreads) & 1)], c);
+    for (int64_t c = k; c < pieces && rcs[k] == 0; c += kCopyThreads) rcs[k] = piece(c);
     if (rcs[k] != 0) memcpy(errs[k], g_err, sizeof(g_err));       // (the message is the thread's own)
   };
   std::thread th[kCopyThreads - 1];
@@ -255,7 +310,6 @@ int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t b
     if (rcs[k] != 0) { memcpy(g_err, errs[k], sizeof(g_err)); return rcs[k]; }
   return ANC_OK;
 }
-static_assert(kSlots == 2 * kCopyThreads, "two slots per copying thread");
 }  // namespace
 extern "C" int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream) {
   ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_upload_async: bad arguments");
@@ -263,7 +317,6 @@ extern "C" int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, ui
   OnDeviceOf on;
   if (int rc = on.enter(anc_stream(stream))) return rc;
   StageRing &r = g_ring[on.dev];
-  std::lock_guard<std::mutex> lk(r.mu);
   return stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream));
 }
 extern "C" int anc_upload_now(uint64_t dst, const void *src, int64_t bytes) {
@@ -272,23 +325,36 @@ extern "C" int anc_upload_now(uint64_t dst, const void *src, int64_t bytes) {
   OnDeviceOf on;
   if (int rc = on.enter(nullptr)) return rc;
   StageRing &r = g_ring[on.dev];
+  {
+    std::lock_guard<std::mutex> lk(r.mu);
+    if (r.own == nullptr) ANC_HIP(hipStreamCreateWithFlags(&r.own, hipStreamNonBlocking));
+    ++r.own_users;
+  }
+  int rc = stage_upload(r, on.dev, dst, src, bytes, r.own);
+  if (rc == ANC_OK)
+    if (hipError_t e = hipStreamSynchronize(r.own)) rc = anc_hip_fail(e, "hipStreamSynchronize", __FILE__, __LINE__);
   std::lock_guard<std::mutex> lk(r.mu);
-  if (r.own == nullptr) ANC_HIP(hipStreamCreateWithFlags(&r.own, hipStreamNonBlocking));
-  if (int rc = stage_upload(r, on.dev, dst, src, bytes, r.own)) return rc;
-  ANC_HIP(hipStreamSynchronize(r.own));
-  return ANC_OK;
+  --r.own_users;
+  return rc;
 }
 extern "C" int anc_staging_release(void) {
   for (StageRing &r : g_ring) {
-    std::lock_guard<std::mutex> lk(r.mu);
     for (StageSlot &slot : r.slot) {
-      if (slot.mem == nullptr) continue;
-      if (slot.busy) ANC_HIP(hipEventSynchronize(slot.done));
-      ANC_HIP(hipEventDestroy(slot.done));
-      ANC_HIP(hipHostFree(slot.mem));
-      slot = StageSlot{};
+      {
+        std::lock_guard<std::mutex> lk(r.mu);
+        if (slot.taken || slot.mem == nullptr) continue;       // (in use by a call: it stays)
+        slot.taken = true;
+      }
+      hipError_t e = slot.busy ? hipEventSynchronize(slot.done) : hipSuccess;
+      if (e == hipSuccess) e = hipEventDestroy(slot.done);
+      if (e == hipSuccess) e = hipHostFree(slot.mem);
+      std::lock_guard<std::mutex> lk(r.mu);
+      if (e == hipSuccess) slot = StageSlot{}; else slot.taken = false;
+      ANC_HIP(e);
     }
-    if (r.own != nullptr) ANC_HIP(hipStreamDestroy(r.own));
+    std::lock_guard<std::mutex> lk(r.mu);
+    if (r.own == nullptr || r.own_users != 0) continue;
+    ANC_HIP(hipStreamDestroy(r.own));
     r.own = nullptr;
   }
   return ANC_OK;
@@ -300,7 +366,6 @@ extern "C" int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint
     OnDeviceOf on;
     if (int rc = on.enter(anc_stream(stream))) return rc;
     StageRing &r = g_ring[on.dev];
-    std::lock_guard<std::mutex> lk(r.mu);
     if (int rc = stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream))) return rc;
   } else {
     // a state as it is set up, often memory that no one has touched yet: the runtime's own path takes its page

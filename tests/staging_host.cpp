@@ -3,6 +3,7 @@
 // prints "ok"; a failed check or a call the stand-in refuses ends the program with a message.
 #include <hip/hip_runtime_api.h>
 
+#include <chrono>
 #include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
@@ -16,6 +17,8 @@
 #include <string>
 #include <vector>
 
+#include <unistd.h>
+
 extern "C" {
 int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
 int anc_upload_now(uint64_t dst, const void *src, int64_t bytes);
@@ -24,7 +27,7 @@ int anc_staging_release(void);
 const char *anc_last_error(void);
 }
 
-#define CHECK(c) do { if (!(c)) { printf("line %d: %s (%s)\n", __LINE__, #c, anc_last_error()); exit(1); } } while (0)
+#define CHECK(c) do { if (!(c)) { printf("line %d: %s (%s)\n", __LINE__, #c, anc_last_error()); fflush(stdout); _exit(1); } } while (0)
 
 // ---- the stand-in
 struct Stream {
@@ -154,13 +157,71 @@ static void two_devices() {
         }
       }
     }
-  CHECK(pinned.size() == 16 && events.size() == 16 && live_streams == 2);       // 8 slots per device and no more
+  CHECK(pinned.size() <= 16 && events.size() == pinned.size() && live_streams == 2);       // 8 slots per device and no more
   CHECK(anc_staging_release() == 0);
   CHECK(pinned.empty() && events.empty() && live_streams == 0);
 }
 
+static bool soon(std::future<int> &f) { return f.wait_for(std::chrono::seconds(5)) == std::future_status::ready; }
+
+// Work that holds stream A, and with it every slot, holds no upload on stream B, nor one that is complete on return,
+// from the same thread or while another thread waits for A.
+static void other_streams_do_not_wait() {
+  Stream A{0}, B{0};
+  const size_t n = 100;
+  const std::vector<char> want = bytes(n, 1);
+  std::vector<std::vector<char>> onA(9, std::vector<char>(n));
+  std::future<int> ninth;
+  A.held = true;
+  for (int i = 0; i < 8; ++i) CHECK(anc_upload_async((uint64_t)onA[(size_t)i].data(), want.data(), (int64_t)n, handle(&A)) == 0);
+  for (int blocked = 0; blocked < 2; ++blocked) {
+    std::future<int> onB = std::async(std::launch::async, [&]() -> int {
+      std::vector<char> src = want, a(n), b(n), c(n);
+      const int rc = anc_upload_async((uint64_t)a.data(), src.data(), (int64_t)n, handle(&B)) |
+                     anc_upload_now((uint64_t)b.data(), src.data(), (int64_t)n) |
+                     anc_memcpy_h2d((uint64_t)c.data(), src.data(), (int64_t)n, handle(&B));
+      return rc != 0 || a != want || b != want || c != want || hipGetLastError() != hipSuccess;
+    });
+    CHECK(soon(onB) && onB.get() == 0);
+    if (blocked == 0) {
+      ninth = std::async(std::launch::async, [&]() -> int {
+        return anc_upload_async((uint64_t)onA[8].data(), want.data(), (int64_t)n, handle(&A));
+      });
+      CHECK(ninth.wait_for(std::chrono::milliseconds(200)) == std::future_status::timeout);       // A's own turn
+    }
+  }
+  release(&A);
+  CHECK(ninth.get() == 0);
+  for (const auto &a : onA) CHECK(a == want);
+  CHECK(anc_staging_release() == 0);
+  CHECK(pinned.empty() && events.empty() && live_streams == 0);
+}
+
+// Several threads on streams of their own, sizes on both sides of a slot and of the threaded copy.
+static void many_threads() {
+  std::vector<std::future<int>> all;
+  for (int t = 0; t < 6; ++t)
+    all.push_back(std::async(std::launch::async, [t] {
+      Stream s{t & 1};
+      for (int i = 0; i < 20; ++i)
+        for (size_t n : {64u, (512u << 10) + 1, 9u << 20}) {
+          if (n > (8u << 20) && i % 8 != 0) continue;
+          const std::vector<char> want = bytes(n, t * 31 + i);
+          std::vector<char> src = want, a(n);
+          if (anc_upload_async((uint64_t)a.data(), src.data(), (int64_t)n, handle(&s)) != 0) return 1;
+          memset(src.data(), 0, n);
+          if (a != want) return 2;
+        }
+      return 0;
+    }));
+  for (auto &f : all) CHECK(f.get() == 0);
+  CHECK(anc_staging_release() == 0);
+  CHECK(pinned.empty() && events.empty());
+}
+
 int main(int argc, char **argv) {
-  const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}};
+  const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}, {"other_streams_do_not_wait", other_streams_do_not_wait},
+                                                   {"many_threads", many_threads}};
   if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
   cases.at(argv[1])();
   printf("ok\n");
