@@ -110,6 +110,7 @@ _PROTOS = {
     "anc_stream_create": (None, [C.POINTER(u64)]),
     "anc_stream_create_nonblocking": (None, [C.POINTER(u64)]),
     "anc_stream_destroy": (None, [u64]),
+    "anc_stream_is_capturing": (None, [u64, C.POINTER(i32)]),
     "anc_stream_sync": (None, [u64]),
     "anc_device_sync": (None, []),
     "anc_event_create": (None, [C.POINTER(u64)]),
@@ -250,6 +251,12 @@ def stream_create_nonblocking():
     s = u64(0)
     api.anc_stream_create_nonblocking(C.byref(s))
     return int(s.value)
+
+
+def stream_is_capturing(stream=0):
+    c = i32(0)
+    api.anc_stream_is_capturing(int(stream), C.byref(c))
+    return bool(c.value)
 
 
 def stream_sync(stream=0):

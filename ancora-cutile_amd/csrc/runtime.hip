@@ -191,21 +191,36 @@ struct StageRing {
 };
 StageRing g_ring[kMaxDevices];
 
-// The device a stream belongs to is current while this lives (the null stream's is the current one already).
-struct OnDeviceOf {
+// A graph would read host memory, or a slot, whose contents have changed.
+int refuse_capture(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  ANC_HIP(hipStreamIsCapturing(s, &st));
+  ANC_REQUIRE(st == hipStreamCaptureStatusNone, "upload: the stream is being captured, and host memory is read once, at the call");
+  return ANC_OK;
+}
+// While this lives the device `s` belongs to is current (the null stream's is the current one already), and a capture
+// of another stream by this or another thread leaves events and pinned memory usable.
+struct StageScope {
   int dev = 0, before = -1;
+  bool relaxed = false;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   int enter(hipStream_t s) {
     int cur = 0;
     ANC_HIP(hipGetDevice(&cur));
     dev = cur;
     if (s != nullptr && s != hipStreamLegacy && s != hipStreamPerThread) ANC_HIP(hipStreamGetDevice(s, &dev));
     ANC_REQUIRE(dev >= 0 && dev < kMaxDevices, "upload: device %d beyond %d", dev, kMaxDevices - 1);
+    ANC_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    relaxed = true;
     if (dev == cur) return ANC_OK;
     ANC_HIP(hipSetDevice(dev));
     before = cur;
     return ANC_OK;
   }
-  ~OnDeviceOf() { if (before >= 0) (void)hipSetDevice(before); }
+  ~StageScope() {
+    if (before >= 0) (void)hipSetDevice(before);
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
 };
 
 // A slot for an upload on `s`: *out stays null if work of other streams holds them all.
@@ -299,7 +314,12 @@ int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t b
   int started = 0;
   try {
     for (; started < kCopyThreads - 1; ++started)
-      th[started] = std::thread([&, k = started + 1]() { (void)hipSetDevice(dev); work(k); });
+      th[started] = std::thread([&, k = started + 1]() {
+        hipStreamCaptureMode relaxed = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&relaxed);
+        (void)hipSetDevice(dev);
+        work(k);
+      });
   } catch (const std::system_error &) {
     // no thread to be had: this one copies the remaining shares too
   }
@@ -314,7 +334,8 @@ int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t b
 extern "C" int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream) {
   ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_upload_async: bad arguments");
   if (bytes == 0) return ANC_OK;
-  OnDeviceOf on;
+  if (int rc = refuse_capture(anc_stream(stream))) return rc;
+  StageScope on;
   if (int rc = on.enter(anc_stream(stream))) return rc;
   StageRing &r = g_ring[on.dev];
   return stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream));
@@ -322,7 +343,7 @@ extern "C" int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, ui
 extern "C" int anc_upload_now(uint64_t dst, const void *src, int64_t bytes) {
   ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_upload_now: bad arguments");
   if (bytes == 0) return ANC_OK;
-  OnDeviceOf on;
+  StageScope on;
   if (int rc = on.enter(nullptr)) return rc;
   StageRing &r = g_ring[on.dev];
   {
@@ -362,8 +383,9 @@ extern "C" int anc_staging_release(void) {
 extern "C" int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint64_t stream) {
   ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_memcpy_h2d: bad arguments");
   if (bytes == 0) return ANC_OK;
+  if (int rc = refuse_capture(anc_stream(stream))) return rc;
   if (bytes <= 2 * kSlotBytes) {
-    OnDeviceOf on;
+    StageScope on;
     if (int rc = on.enter(anc_stream(stream))) return rc;
     StageRing &r = g_ring[on.dev];
     if (int rc = stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream))) return rc;
@@ -408,6 +430,13 @@ extern "C" int anc_stream_create_nonblocking(uint64_t *stream) {
 extern "C" int anc_stream_destroy(uint64_t stream) {
   ANC_REQUIRE(stream != 0, "anc_stream_destroy: the null stream is not destroyable");
   ANC_HIP(hipStreamDestroy(anc_stream(stream)));
+  return ANC_OK;
+}
+extern "C" int anc_stream_is_capturing(uint64_t stream, int32_t *capturing) {
+  ANC_REQUIRE(capturing != nullptr, "anc_stream_is_capturing: null output");
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  ANC_HIP(hipStreamIsCapturing(anc_stream(stream), &st));
+  *capturing = st != hipStreamCaptureStatusNone;
   return ANC_OK;
 }
 extern "C" int anc_stream_sync(uint64_t stream) {

@@ -115,13 +115,17 @@ class _GroupArray(DevBuf):
 
 class IdGroups:
     """The four group arrays, plus the number of distinct ids. They travel to the device with the first
-    launch that uses them, in its stream's order."""
+    launch that uses them, in its stream's order; if that stream is being captured into a graph they are in place
+    before it, once, and the graph's replays read them there."""
 
     def __init__(self, ids_flat):
         _lib.init()
         self._arrays, self.n_groups = _id_groups(ids_flat)
         self.M = self._arrays.shape[1]
-        self._block, self._si, self._settled = None, None, False
+        if self.M == 0:
+            raise ValueError("IdGroups: no ids")
+        self._block = _blocks.get(self._arrays.nbytes)         # (here: a capture may not allocate)
+        self._si, self._settled = None, False
         self.srt, self.start, self.cnt, self.gid = (_GroupArray(self, i) for i in range(4))
 
     @property
@@ -132,17 +136,20 @@ class IdGroups:
     def base_on(self, si):
         """Device address of the arrays for work queued on stream `si`."""
         if self._block is None:
-            self._block, self._si = _blocks.get(self._arrays.nbytes), si
+            raise _lib.AncoraError("IdGroups: freed")
+        if self._si is None and not self._settled and not _lib.stream_is_capturing(si):
             api.anc_upload_async(self._block.ptr, self._arrays.ctypes.data, self._arrays.nbytes, int(si))
+            self._si = si
         elif self._si != si:
             return self.settled()
         return self._block.ptr
 
     def settled(self):
         """Device address of the arrays, in place for any stream."""
+        if self._block is None:
+            raise _lib.AncoraError("IdGroups: freed")
         if not self._settled:
-            if self._block is None:
-                self._block = _blocks.get(self._arrays.nbytes)
+            if self._si is None:
                 api.anc_upload_now(self._block.ptr, self._arrays.ctypes.data, self._arrays.nbytes)
             else:
                 _lib.stream_sync(self._si)
@@ -152,7 +159,7 @@ class IdGroups:
     def free(self):
         if self._block is not None:
             _blocks.put(self._block)
-            self._block, self._settled = None, False
+            self._block = None
 
 
 def embed_dw_scatter(groups, dy, si, out=None, compact=None, V=None):

@@ -75,7 +75,8 @@ int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint64_t stream
 /* Uploads through pinned staging memory; src may be reused on return. anc_memcpy_h2d: complete on return.
  * _async: ordered on `stream`, no wait. _now: complete on return, on a stream of its own, without
  * waiting for work queued elsewhere; nobody may be using dst. Each device has its ring of staging memory, the
- * stream's device decides (the null stream and _now: the current one); _release gives it all back. */
+ * stream's device decides (the null stream and _now: the current one); _release gives it all back. A stream under
+ * graph capture is refused (the graph would read host memory later than the call); _now may be called meanwhile. */
 int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
 int anc_upload_now(uint64_t dst, const void *src, int64_t bytes);
 int anc_staging_release(void);
@@ -84,6 +85,7 @@ int anc_memcpy_d2d(uint64_t dst, uint64_t src, int64_t bytes, uint64_t stream);
 int anc_stream_create(uint64_t *stream);
 int anc_stream_create_nonblocking(uint64_t *stream);   /* not ordered against the null stream */
 int anc_stream_destroy(uint64_t stream);
+int anc_stream_is_capturing(uint64_t stream, int32_t *capturing);
 int anc_stream_sync(uint64_t stream);
 int anc_device_sync(void);
 int anc_event_create(uint64_t *event);

@@ -27,7 +27,8 @@ class FakeDevice:
     def __init__(self):
         self.blocks = {}             # address -> bytearray
         self.next = 1 << 20
-        self.log = []                # (entry point, arguments) of everything else
+        self.log = []                # (entry point, arguments) of every call
+        self.capturing = set()       # streams
 
     def at(self, ptr, n):
         base = max(b for b in self.blocks if b <= ptr)
@@ -47,6 +48,9 @@ class FakeDevice:
 
     def anc_fill_u32(self, ptr, value, n, stream):
         self.at(ptr, 4 * n)[:] = int(value).to_bytes(4, "little") * n
+
+    def anc_stream_is_capturing(self, stream, out):
+        out._obj.value = stream in self.capturing
 
     def _upload(self, ptr, src, n, *stream):
         import ctypes

@@ -219,9 +219,32 @@ static void many_threads() {
   CHECK(pinned.empty() && events.empty());
 }
 
+// Uploads on a stream under capture are refused and leave no slot behind whose event belongs to the graph; those that
+// are complete on return go through meanwhile, and so does everything afterwards.
+static void capture() {
+  Stream s{0}, other{0};
+  const size_t n = 100;
+  const std::vector<char> want = bytes(n, 1);
+  s.capturing = true;
+  for (size_t big : {n, (size_t)2 << 20}) {
+    std::vector<char> src(big), a(big);
+    CHECK(anc_upload_async((uint64_t)a.data(), src.data(), (int64_t)big, handle(&s)) != 0);
+    CHECK(anc_memcpy_h2d((uint64_t)a.data(), src.data(), (int64_t)big, handle(&s)) != 0);
+  }
+  for (int captured = 1; captured >= 0; --captured) {
+    s.capturing = captured != 0;
+    for (int i = 0; i < 10; ++i) {
+      std::vector<char> a(n), b(n);
+      CHECK(anc_upload_now((uint64_t)a.data(), want.data(), (int64_t)n) == 0);
+      CHECK(anc_upload_async((uint64_t)b.data(), want.data(), (int64_t)n, handle(captured ? &other : &s)) == 0);
+      CHECK(a == want && b == want && hipGetLastError() == hipSuccess);
+    }
+  }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}, {"other_streams_do_not_wait", other_streams_do_not_wait},
-                                                   {"many_threads", many_threads}};
+                                                   {"many_threads", many_threads}, {"capture", capture}};
   if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
   cases.at(argv[1])();
   printf("ok\n");

@@ -42,6 +42,41 @@ def test_embed_dw_scatter_is_the_sequential_sum(gpu, M, V, H, seed):
     grp.free()
 
 
+def test_first_scatter_of_a_batch_inside_a_graph(gpu):
+    """Group arrays made before a capture and first used in it: every replay, with other groups in use between them,
+    adds the batch's sums."""
+    import ctypes
+    from ancora_cutile_amd import DevBuf
+    from ancora_cutile_amd.embed import IdGroups, embed_dw_scatter
+    hip = ctypes.CDLL("libamdhip64.so")
+    M, V, H = 96, 40, 128
+    rng = np.random.default_rng(6)
+    dyb = bf16_rne_bits(rng.standard_normal((M, H)).astype(np.float32)).reshape(M, H)
+    gdy, compact, other = DevBuf(dyb), DevBuf.zeros((M, H), np.float32), DevBuf.zeros((M, H), np.float32)
+    ids = rng.integers(0, V, M).astype(np.int32)
+    grp, s = IdGroups(ids), gpu.stream_create()
+    gid, rows = embed_dw_rows(ids, dyb)
+    graph, graph_exec = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(ctypes.c_void_p(s), 0) == 0
+    embed_dw_scatter(grp, gdy, s, compact=compact)
+    assert hip.hipStreamEndCapture(ctypes.c_void_p(s), ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(graph_exec), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(4):
+        compact.fill_zero(s)
+        for _ in range(12):                            # every slot and block a later upload could take
+            g2 = IdGroups(rng.integers(0, V, M).astype(np.int32))
+            embed_dw_scatter(g2, gdy, 0, compact=other)
+            g2.free()
+        gpu.stream_sync(0)
+        assert hip.hipGraphLaunch(graph_exec, ctypes.c_void_p(s)) == 0
+        assert bits_equal(compact.to_numpy(s)[:gid.size], rows)
+    hip.hipGraphExecDestroy(graph_exec)
+    hip.hipGraphDestroy(graph)
+    for b in (grp, gdy, compact, other):
+        b.free()
+    gpu.api.anc_stream_destroy(s)
+
+
 @pytest.mark.parametrize("sr", [False, True])
 def test_row_sparse_adamw_equals_the_dense_optimizer(gpu, sr):
     """Eight steps on a (4096, 256) table; each step's tokens come from a skewed distribution, so

@@ -98,3 +98,31 @@ def test_muon_tables_follow_the_weights_addresses(fake_device, fused_update):
         ws[2][key] = keep
     assert step() == before
     eng.free()
+
+
+def test_id_groups_are_in_place_before_a_captured_launch(fake_device):
+    """A launch on a stream under capture finds the arrays uploaded outside the graph, whether they were on their way
+    on another stream or not at all, and allocates nothing; outside a capture they go in the stream's order."""
+    from ancora_cutile_amd import DevBuf, _lib
+    from ancora_cutile_amd.embed import IdGroups, embed_dw_scatter
+    dy, out = DevBuf.zeros((6, 64), np.uint16), DevBuf.zeros((8, 64), np.float32)
+    for first, uploads in ((None, ["anc_upload_now"]), (3, ["anc_upload_async", "anc_stream_sync"]), (7, ["anc_upload_async"])):
+        fake_device.capturing = set()
+        grp = IdGroups([5, 2, 5, 5, 0, 2])
+        if first is not None:
+            embed_dw_scatter(grp, dy, first, out=out)
+        fake_device.capturing = {7}
+        mallocs = len(fake_device.calls("anc_malloc"))
+        embed_dw_scatter(grp, dy, 7, out=out)
+        assert len(fake_device.calls("anc_malloc")) == mallocs
+        names = [n for n, _ in fake_device.log]
+        last = len(names) - 1 - names[::-1].index("anc_malloc") if first is None else 0
+        assert [n for n in names[last:] if n in ("anc_upload_now", "anc_upload_async", "anc_stream_sync")] == uploads
+        cnt = fake_device.calls("anc_embed_dw_scatter")[-1][0]
+        assert list(np.frombuffer(fake_device.at(cnt, 24), np.int32)) == [1, 2, 3, 0, 0, 0]
+        grp.free()
+        with pytest.raises(_lib.AncoraError):
+            embed_dw_scatter(grp, dy, 7, out=out)
+        fake_device.log.clear()
+    with pytest.raises(ValueError):
+        IdGroups(np.zeros(0, np.int32))
