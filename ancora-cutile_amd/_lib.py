@@ -92,6 +92,7 @@ _PROTOS = {
     "anc_last_error": (C.c_char_p, []),
     "anc_abi_version": (C.c_int, []),
     "anc_init": (None, [C.c_int]),
+    "anc_current_device": (None, [C.POINTER(i32)]),
     "anc_device_info": (None, [C.POINTER(DeviceInfo)]),
     "anc_malloc": (None, [C.POINTER(u64), i64]),
     "anc_free": (None, [u64]),
@@ -226,6 +227,12 @@ def init(device=0):
     if not _initialised:
         api.anc_init(int(device))
         _initialised = True
+
+
+def current_device():
+    d = i32(0)
+    api.anc_current_device(C.byref(d))
+    return int(d.value)
 
 
 def device_info():

@@ -94,6 +94,12 @@ extern "C" int anc_init(int device) {
   return anc_gradnorm_static_init();
 }
 
+extern "C" int anc_current_device(int32_t *device) {
+  ANC_REQUIRE(device != nullptr, "anc_current_device: null output");
+  ANC_HIP(hipGetDevice(device));
+  return ANC_OK;
+}
+
 extern "C" int anc_device_info(anc_device_info_t *out) {
   ANC_REQUIRE(out != nullptr, "anc_device_info: null output");
   int dev = 0;

@@ -53,41 +53,47 @@ class _Blocks:
     """Device blocks of the group arrays, kept between steps: an allocation and a release per step cost more than
     the arrays' upload, and a release waits for the whole device. A block given back may still be read by work in
     flight on any stream, so it is handed out again only after a device synchronisation, one for every
-    KEEP blocks. At most KEEP are kept; `trim` gives them back to the device."""
+    KEEP blocks. A device's blocks stay on that device; at most 2 * KEEP of each are kept, `trim` gives them back."""
 
     KEEP = 8
 
     def __init__(self):
         self._lock = threading.Lock()
-        self._ready, self._waiting = [], []
+        self._ready, self._waiting = {}, {}          # device -> blocks
 
     def get(self, nbytes):
+        dev = _lib.current_device()
         with self._lock:
-            if len(self._waiting) >= self.KEEP:
-                api.anc_device_sync()
-                self._ready += self._waiting
-                self._waiting = []
-                self._ready.sort(key=lambda b: b.nbytes)
-                for b in self._ready[:-self.KEEP]:
-                    b.free()
-                self._ready = self._ready[-self.KEEP:]
-            for i, b in enumerate(self._ready):
-                if nbytes <= b.nbytes <= 4 * nbytes + 65536:
-                    return self._ready.pop(i)
-        return DevBuf.empty((max(nbytes, 4096),), np.uint8)
+            idle = self._waiting.pop(dev) if len(self._waiting.get(dev, ())) >= self.KEEP else []
+        if idle:
+            api.anc_device_sync()                    # (outside the lock: other threads need not wait for this device)
+        with self._lock:
+            ready = self._ready.setdefault(dev, [])
+            ready += idle
+            ready.sort(key=lambda b: b.nbytes)
+            spare, ready[:] = ready[:-self.KEEP], ready[-self.KEEP:]
+            block = next((ready.pop(i) for i, b in enumerate(ready) if nbytes <= b.nbytes <= 4 * nbytes + 65536), None)
+        for b in spare:
+            b.free()
+        if block is None:
+            block = DevBuf.empty((max(nbytes, 4096),), np.uint8)
+            block.device = dev
+        return block
 
     def put(self, b):
         with self._lock:
-            if len(self._waiting) < self.KEEP:
-                self._waiting.append(b)
+            waiting = self._waiting.setdefault(b.device, [])
+            if len(waiting) < self.KEEP:
+                waiting.append(b)
                 return
         b.free()
 
     def trim(self):
         with self._lock:
-            for b in self._ready + self._waiting:
-                b.free()
-            self._ready, self._waiting = [], []
+            blocks = [b for kept in (self._ready, self._waiting) for bs in kept.values() for b in bs]
+            self._ready, self._waiting = {}, {}
+        for b in blocks:
+            b.free()
 
 
 _blocks = _Blocks()

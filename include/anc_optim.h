@@ -63,6 +63,7 @@ typedef struct {
 } anc_device_info_t;
 
 int anc_init(int device);                        /* hipSetDevice + arch check (gfx950 only) */
+int anc_current_device(int32_t *device);
 int anc_device_info(anc_device_info_t *out);
 int anc_malloc(uint64_t *dptr, int64_t bytes);
 int anc_free(uint64_t dptr);

@@ -29,6 +29,8 @@ class FakeDevice:
         self.next = 1 << 20
         self.log = []                # (entry point, arguments) of every call
         self.capturing = set()       # streams
+        self.current = 0
+        self.home = {}               # address -> device
 
     def at(self, ptr, n):
         base = max(b for b in self.blocks if b <= ptr)
@@ -41,6 +43,7 @@ class FakeDevice:
     def anc_malloc(self, out, n):
         self.blocks[self.next] = bytearray(n)
         out._obj.value = self.next
+        self.home[self.next] = self.current
         self.next += (n + 511) // 256 * 256
 
     def anc_free(self, ptr):
@@ -48,6 +51,9 @@ class FakeDevice:
 
     def anc_fill_u32(self, ptr, value, n, stream):
         self.at(ptr, 4 * n)[:] = int(value).to_bytes(4, "little") * n
+
+    def anc_current_device(self, out):
+        out._obj.value = self.current
 
     def anc_stream_is_capturing(self, stream, out):
         out._obj.value = stream in self.capturing

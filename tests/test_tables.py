@@ -126,3 +126,32 @@ def test_id_groups_are_in_place_before_a_captured_launch(fake_device):
         fake_device.log.clear()
     with pytest.raises(ValueError):
         IdGroups(np.zeros(0, np.int32))
+
+
+def test_group_blocks_are_reused_after_a_synchronisation_and_stay_on_their_device(fake_device, monkeypatch):
+    """Blocks of 3 * KEEP batches on two devices in turn: one that was given back is handed out again only after a
+    synchronisation of its device, on its device alone, within a factor of its size; a bounded number is kept and all
+    are given back."""
+    from ancora_cutile_amd import embed
+    pool = embed._Blocks()
+    monkeypatch.setattr(embed, "_blocks", pool)
+    rng = np.random.default_rng(0)
+    dirty, live = set(), []                    # given back and not synchronised since; in use
+
+    def sync():
+        fake_device.log.append(("anc_device_sync", ()))
+        dirty.difference_update([p for p in dirty if fake_device.home[p] == fake_device.current])
+    monkeypatch.setattr(embed.api, "anc_device_sync", sync)
+    for i in range(6 * pool.KEEP):
+        fake_device.current = i & 1
+        grp = embed.IdGroups(rng.integers(0, 50, int(rng.integers(1, 20000))))
+        base = grp.base_on(4)
+        assert fake_device.home[base] == fake_device.current and base not in dirty and base not in live
+        live.append(base)
+        grp.free()
+        live.remove(base)
+        dirty.add(base)
+    assert len(fake_device.calls("anc_device_sync")) <= 6
+    assert len(fake_device.blocks) <= 2 * 2 * pool.KEEP
+    pool.trim()
+    assert not fake_device.blocks
