@@ -19,14 +19,11 @@ from .gradnorm import ctl_ptr
 
 
 def _ids32(ids):
-    """Integer ids as a contiguous int32 vector."""
+    """Ids of any type as a contiguous int32 vector: fractions are cut off, what 32 bits do not hold wraps (an
+    unsigned -1 as padding), and a row outside the table is left out by the kernels."""
     ids = np.asarray(ids).reshape(-1)
-    if ids.dtype != np.int32:
-        if ids.dtype.kind not in "iub" or (ids.size and ids.dtype.itemsize >= 4 and
-                                           (int(ids.max()) > 0x7FFFFFFF or int(ids.min()) < -0x80000000)):
-            raise ValueError(f"token ids must be integers of 32 bits, got {ids.dtype}")
-        ids = ids.astype(np.int32)
-    return np.ascontiguousarray(ids)
+    with np.errstate(invalid="ignore"):
+        return np.ascontiguousarray(ids, dtype=np.int32)
 
 
 def _id_groups(ids_flat):
@@ -264,8 +261,6 @@ class RowSparseAdamW:
         if self.t == 0:
             return
         ids = _ids32(row_ids)
-        if ids.size == 0:
-            return
         rows, n = np.empty(ids.size, np.int32), ctypes.c_int64(0)
         api.anc_unique_ids(ids.ctypes.data, ids.size, rows.ctypes.data, ctypes.byref(n))
         buf, n = self._rows(rows[:n.value], si)

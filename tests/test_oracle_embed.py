@@ -51,6 +51,22 @@ def test_host_builder_at_the_edges(ids):
     assert np.array_equal(out[:n.value], np.unique(ids))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.float16, np.int64, np.uint16, np.uint32, np.int8, bool])
+def test_host_builder_takes_ids_of_any_type(dtype):
+    """Token ids as a data loader may hold them, floating point among them, group as their int32 values."""
+    from ancora_cutile_amd.embed import build_id_groups
+    ids = np.random.default_rng(3).integers(0, 97, 400).astype(dtype)
+    for got, want in zip(build_id_groups(ids.reshape(20, 20)), build_id_groups(ids.astype(np.int32))):
+        assert np.array_equal(got, want)
+    if dtype is np.uint32:
+        ids[::9] = 0xFFFFFFFF                                        # padding
+        srt, start, cnt, gid = (a[:, 0] for a in build_id_groups(ids))
+        o_srt, o_start, o_cnt, o_gid = id_groups(ids.view(np.int32))
+        U = o_gid.size
+        assert np.array_equal(gid[:U], o_gid) and -1 in o_gid and np.array_equal(srt, o_srt) and np.array_equal(cnt[:U], o_cnt)
+    assert [a.shape for a in build_id_groups([])] == [(0, 1)] * 4
+
+
 def test_scatter_sum_exact_case_and_reference_gate():
     rng = np.random.default_rng(2)
     M, V, H = 512, 64, 128
