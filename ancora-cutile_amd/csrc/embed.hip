@@ -12,6 +12,7 @@
 // of 150 rows among 8192 took 33 us. Most groups are one row and want a short path: guarding each of 32
 // loads instead took 77 us.)
 #include <algorithm>
+#include <new>
 #include <type_traits>
 #include <vector>
 
@@ -170,10 +171,14 @@ IdRank make_rank(const int32_t *ids, int64_t n) {
   if (hw_popcnt()) rank_fill_hw(r, ids, n); else rank_fill(r, ids, n);
   return r;
 }
+int no_memory(const char *who, int64_t n) {
+  anc_set_error("%s: no memory to group %lld ids", who, (long long)n);
+  return ANC_ERR_ARG;
+}
 
 }  // namespace
 
-extern "C" int anc_unique_ids(const int32_t *ids, int64_t n, int32_t *out, int64_t *n_out) {
+extern "C" int anc_unique_ids(const int32_t *ids, int64_t n, int32_t *out, int64_t *n_out) try {
   ANC_REQUIRE(ids != nullptr && out != nullptr && n_out != nullptr && n >= 0 && n < (1ll << 31), "anc_unique_ids: bad arguments");
   *n_out = 0;
   if (n == 0) return ANC_OK;
@@ -187,10 +192,12 @@ extern "C" int anc_unique_ids(const int32_t *ids, int64_t n, int32_t *out, int64
   std::sort(v.begin(), v.end());
   *n_out = (int64_t)(std::unique_copy(v.begin(), v.end(), out) - out);
   return ANC_OK;
+} catch (const std::bad_alloc &) {
+  return no_memory("anc_unique_ids", n);
 }
 
 extern "C" int anc_id_groups(const int32_t *ids, int64_t n, int32_t *srt, int32_t *start, int32_t *cnt, int32_t *gid,
-                             int64_t *n_groups) {
+                             int64_t *n_groups) try {
   ANC_REQUIRE(ids != nullptr && srt != nullptr && start != nullptr && cnt != nullptr && gid != nullptr && n_groups != nullptr &&
                   n >= 0 && n < (1ll << 31),
               "anc_id_groups: bad arguments");
@@ -215,4 +222,6 @@ extern "C" int anc_id_groups(const int32_t *ids, int64_t n, int32_t *srt, int32_
   }
   *n_groups = g + 1;
   return ANC_OK;
+} catch (const std::bad_alloc &) {
+  return no_memory("anc_id_groups", n);
 }

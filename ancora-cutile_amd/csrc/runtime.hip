@@ -23,7 +23,7 @@ extern "C" const char *anc_last_error(void) { return g_err; }
 
 // ---- per-launch profiler -------------------------------------------------------------
 #include <mutex>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <vector>
 namespace {
@@ -326,7 +326,7 @@ int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t b
         (void)hipSetDevice(dev);
         work(k);
       });
-  } catch (const std::system_error &) {
+  } catch (const std::exception &) {
     // no thread to be had: this one copies the remaining shares too
   }
   work(0);

@@ -179,3 +179,35 @@ def test_bench_reads_gemm_traffic_from_a_counter_database(tmp_path):
     assert unit == 2.0 and n == 2 and per_launch == (1000.0 + 3000.0) * 2.0 * 1024.0 / 2
     with pytest.raises(RuntimeError):
         bench.gemm_bytes_from_counter_db(db, "WRITE_SIZE")          # no copy kernel row for this counter
+
+
+@pytest.mark.parametrize("entry", ["anc_id_groups", "anc_unique_ids"])
+def test_grouping_ids_without_memory_is_an_error(entry):
+    """Scratch memory that cannot be had is a status and a message at the C boundary, not the process's end."""
+    import subprocess
+    import sys
+    code = f"""
+import resource, sys
+import numpy as np
+sys.path.insert(0, {ROOT!r})
+from ancora_cutile_amd import _lib
+_lib.load()
+n = 20_000_000
+ids, out = np.arange(n, dtype=np.int32)[::-1].copy(), np.empty((4, n), np.int32)
+ids[0] = 2**31 - 1                     # (a range too wide for the bitmap where the ids are only listed)
+p = [out[i].ctypes.data for i in range(4)]
+if {entry!r} == "anc_id_groups":
+    ids[0] = n
+size = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (size + (16 << 20),) * 2)
+try:
+    m = _lib.i64(0)
+    if {entry!r} == "anc_id_groups":
+        _lib.api.anc_id_groups(ids.ctypes.data, n, *p, m)
+    else:
+        _lib.api.anc_unique_ids(ids.ctypes.data, n, p[0], m)
+except _lib.AncoraError as e:
+    print("refused:", e)
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "no memory" in r.stdout, (r.returncode, r.stdout, r.stderr[-500:])
