@@ -96,11 +96,11 @@ def gemm_dW(problems, si=0, segments=None):
         arr = (DwProblem * len(group))()
         default = fill or (None if segments == "fill" else segments) or 1
         for k, p in enumerate(group):
-            T, K, N = p["T"], p["K"], p["N"]
+            T, K, N = int(p["T"]), int(p["K"]), int(p["N"])
             S = p.get("segments") or default
             if S == "shape":
                 S = dw_info(T, K, N)[1]
-            gn = p.get("gn_partials") or 0
+            S, gn = int(S), int(p.get("gn_partials") or 0)
             if S == 1 and gn == 0:                 # finished by the GEMM's epilogue: no partial tiles
                 ws_ptr = ws_bytes = 0
             else:

@@ -155,3 +155,17 @@ def test_group_blocks_are_reused_after_a_synchronisation_and_stay_on_their_devic
     assert len(fake_device.blocks) <= 2 * 2 * pool.KEEP
     pool.trim()
     assert not fake_device.blocks
+
+
+def test_weight_gradient_sizes_of_any_number_type(fake_device):
+    """Sizes, segments and addresses as numpy numbers or whole floats reach the native call as integers."""
+    from ancora_cutile_amd import DevBuf, _lib
+    from ancora_cutile_amd.grads import DwWorkspace, gemm_dW
+    b = DevBuf.zeros((256, 256), np.float32)
+    problem = dict(x=b, dy=b, dW=b, T=256.0, K=np.int64(128), N=np.float32(256), workspace=DwWorkspace(),
+                   gn_partials=np.uint64(b.ptr), accumulate=np.True_)
+    gemm_dW([problem], segments=np.int32(2))
+    arr, n = fake_device.calls("anc_gemm_dw_multi")[-1][:2]
+    d = arr[0]
+    assert n == 1 and (d.T, d.K, d.N, d.segments, d.gn_partials, d.accumulate) == (256, 128, 256, 2, b.ptr, 1)
+    assert d.workspace_bytes == 2 * 128 * 256 * 4 and d.x_row_major == 1 and (d.xT, d.dy, d.dW, d.g16) == (b.ptr, b.ptr, b.ptr, 0)
