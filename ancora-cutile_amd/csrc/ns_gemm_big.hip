@@ -13,10 +13,9 @@
 //
 // Data path. Operand tiles go from HBM/L2 straight into LDS with global_load_lds_dwordx4 (no
 // register staging): one instruction moves 1 KiB, a lane writes 16 bytes at lds_base + 16*lane.
-// "NT" operand tiles ([row][k], TK*2-byte rows, no padding) avoid bank conflicts by an XOR
-// swizzle of the 16-byte chunk index with row bits (bits 1..3 for 128-byte rows, bits 2..3 for
-// 64-byte rows), applied when choosing which global chunk a lane fetches and undone when a
-// fragment is read: 16 consecutive rows then cover all 64 banks once. The B operand of
+// "NT" operand tiles ([row][k], 64-byte rows, no padding) avoid bank conflicts by an XOR
+// swizzle of the 16-byte chunk index with row bits 2..3, applied when choosing which global chunk
+// a lane fetches and undone when a fragment is read: 16 consecutive rows then cover all 64 banks once. The B operand of
 // X = a X + B X is the iterate itself, (k, n) row-major: its tile is [k][256 columns], fetched
 // as whole 512-byte rows, and its fragments come from transposing LDS reads
 // (ds_read_b64_tr_b16), so no transposed copy of the iterate exists anywhere.
@@ -41,8 +40,8 @@
 //
 // One launch covers up to 8 problems (the shape groups of an optimizer step), see NsGemmMulti.
 //
-// Accumulation order per output element is the same in every tile configuration and in the
-// 128x128 kernel of ns.hip (terms in order, k ascending, one accumulator).
+// Accumulation order per output element is the same in every tile configuration and in ns_gemm_tile.hip (one
+// accumulator, k ascending, the terms of a step together; see NsGemm::nterms).
 #include <type_traits>
 
 #include "lds_dma.h"
@@ -144,9 +143,10 @@ __device__ __forceinline__ void dma16_epi(const void *g, uint32_t lds_base) { dm
 // for the activations of a weight-gradient GEMM as they lie (C = x^T dy) and for the chain's
 // own B X, whose B is symmetric (stored in full): B read by rows k is B^T read by rows m, the
 // same values in the same order of summation.
-template <int EPI, int TM, int TN, int TK, int NS, int MINBLOCKS, int VAR = VAR_NONE, bool AT = false>
+template <int EPI, int TM, int TN, int NS, int MINBLOCKS, int VAR = VAR_NONE, bool AT = false>
 __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_gemm_big(NsGemmMulti pm) {
   constexpr int NWN = TN / 64, NWAVES = (TM / 128) * NWN;
+  constexpr int TK = 32;                            // a K tile is one 32-column panel
   constexpr int ROWB = TK * 2;                      // bytes per LDS row
   constexpr int CPR = TK / 8;                       // 16-byte chunks per row
   constexpr int RPI = 64 / CPR;                     // rows per DMA instruction
@@ -215,24 +215,18 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   // ---- DMA addressing: this wavefront moves IA*RPI rows of the A tile and IB*RPI rows of the B
   //      tile, RPI rows per instruction; lane -> (row lane/CPR, physical chunk lane%CPR). The
   //      global address is a wavefront-uniform base plus a per-lane byte offset that carries
-  //      the swizzle: 128-byte rows use chunk ^ ((row>>1)&7), which alternates with the parity
-  //      of the instruction index (RPI = 8); 64-byte rows use chunk ^ ((row>>2)&3), the same
-  //      for every instruction (RPI = 16).
+  //      the swizzle, chunk ^ ((row>>2)&3), the same for every instruction (RPI = 16).
   // Panel layout (see NsGemm): rows of a tile lie 64 bytes apart, consecutive K tiles one panel
   // (rows_of_the_matrix * 64 bytes) apart; a (k, n) tile is one 2 KiB block per 32 columns.
   const int ldA = p.ldA > 0 ? p.ldA : K;
-  static_assert(TK == 32, "a K tile is one 32-column panel");
   const bool a_pan = !PLAINV && (EPI != EPI_GRAM || p.x_panel != 0);
   const bool b_pan = !PLAINV && (EPI == EPI_BMAT || p.x_panel != 0);
   const int64_t panel = (int64_t)p.M * 64;          // bytes per panel (every matrix of the chain has M rows)
   const int rpA = a_pan ? 64 : ldA * 2;             // bytes between consecutive rows of the A operand
   const int rpB = b_pan ? 64 : K * 2;               // the same for an "NT" B operand
   const int lrow = lane / CPR, pchunk = lane % CPR;
-  const int key0 = (TK == 64) ? (lrow >> 1) : ((lrow >> 2) & 3);
-  const uint32_t voff0 = (uint32_t)(lrow * rpA + ((pchunk ^ key0) * 16));
-  const uint32_t voff1 = (uint32_t)(lrow * rpA + ((pchunk ^ key0 ^ (TK == 64 ? 4 : 0)) * 16));
-  const uint32_t voffN0 = (uint32_t)(lrow * rpB + ((pchunk ^ key0) * 16));
-  const uint32_t voffN1 = (uint32_t)(lrow * rpB + ((pchunk ^ key0 ^ (TK == 64 ? 4 : 0)) * 16));
+  const uint32_t swiz = (uint32_t)((pchunk ^ ((lrow >> 2) & 3)) * 16);
+  const uint32_t voffA = (uint32_t)(lrow * rpA) + swiz, voffN = (uint32_t)(lrow * rpB) + swiz;
   // (k, m) A tile (AT): TK rows of TM*2 = 256 bytes, four rows per DMA instruction; lane -> (row
   // lane/16, physical chunk lane%16), chunk index XORed with 4*(row&3) as for the B tile.
   static_assert(!AT || (TM == 128 && IA * NWAVES * 4 == TK), "(k,m) tile layout");
@@ -270,14 +264,14 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   // DMA instruction i of a stage (0 .. IPS-1: the A tile's IA, then the B tile's IB)
   auto issue_piece = [&](int i, unsigned char *stage, const char *pa, const char *pb) {
     if (i < IA) {
-      const uint32_t vo = AT ? voffAT : ((i & 1) ? voff1 : voff0);
+      const uint32_t vo = AT ? voffAT : voffA;
       // (scalar addition of addresses: chain of 24 x (1024,2048) 1214 -> 1192 us; the weight-gradient product, which is at
       // its power limit, is 0.5 % faster with vector ones)
       if (PLAINV) dma16(pa + i * roA + vo, lds_addr(stage + (wave * IA + i) * 1024));
       else        dma16(pa + i * roA, vo, lds_addr(stage + (wave * IA + i) * 1024));
     } else {
       const int j = i - IA;
-      const uint32_t vo = BT ? ((j & 1) ? voffB1 : voffB0) : ((j & 1) ? voffN1 : voffN0);
+      const uint32_t vo = BT ? ((j & 1) ? voffB1 : voffB0) : voffN;
       if (PLAINV) dma16(pb + j * roB + vo, lds_addr(stage + TM * ROWB + (wave * IB + j) * 1024));
       else        dma16(pb + j * roB, vo, lds_addr(stage + TM * ROWB + (wave * IB + j) * 1024));
     }
@@ -295,7 +289,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   int swz[KSTEPS];
 #pragma unroll
   for (int kk = 0; kk < KSTEPS; ++kk)
-    swz[kk] = ((kk * 2 + (lane >> 5)) ^ (TK == 64 ? ((lane >> 1) & 7) : ((lane >> 2) & 3))) * 16;
+    swz[kk] = ((kk * 2 + (lane >> 5)) ^ ((lane >> 2) & 3)) * 16;
 
   int tb[2] = {0, 0};
   if (BT) {
@@ -1089,7 +1083,7 @@ int launch_sym(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s) {
     grid += t;
   }
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_big: grid out of range");
-  hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 32, 4, 1>), dim3((unsigned)grid), dim3(512), 0, s, pm);
+  hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 4, 1>), dim3((unsigned)grid), dim3(512), 0, s, pm);
   ANC_LAUNCH_CHECK();
   return ANC_OK;
 }
@@ -1139,19 +1133,19 @@ int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const N
   }
   if (fused && (upd->sr & ANC_MUON_P16T)) {
     if (by_rows)
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_UPDATE_T, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE_T, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
     else
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_UPDATE_T, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE_T, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   } else if (fused) {
     if (by_rows)
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_UPDATE, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
     else
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_UPDATE, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   } else {
     if (by_rows)
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_NONE, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_NONE, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
     else
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_NONE, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_NONE, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   }
   ANC_LAUNCH_CHECK();
   return ANC_OK;
@@ -1224,9 +1218,9 @@ int anc_ns_gemm_big_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_
     }
   }
   if (a_transposed)
-    hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_PLAIN, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+    hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_PLAIN, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   else
-    hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 32, 3, 2, VAR_PLAIN>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+    hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_PLAIN>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   ANC_LAUNCH_CHECK();
   return ANC_OK;
 }

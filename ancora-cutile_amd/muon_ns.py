@@ -37,10 +37,7 @@ MODES = {"bf16": NS_BF16, "bf16_fast": NS_BF16_FAST, "bf16_x3": NS_BF16_X3, "fp3
          "bf16_gated": NS_BF16,
          # the formats of shapes that are no multiples of 256, on 128x128 tiles (ANC_NS_TILE128), for tests
          "bf16_tile128": NS_BF16 | 0x100, "bf16_fast_tile128": NS_BF16_FAST | 0x100,
-         "bf16_late3_tile128": NS_BF16_LATE3 | 0x100,
-         # one tile size instead of the rule by launch size (ANC_NS_FORCE_T*): same bits, for tests
-         **{f"{name}_t{t}": m | flag for name, m in (("bf16", NS_BF16), ("bf16_late3", NS_BF16_LATE3), ("bf16_x3", NS_BF16_X3))
-            for t, flag in ((64, 0x200), (128, 0x400), (256, 0x800))}}
+         "bf16_late3_tile128": NS_BF16_LATE3 | 0x100}
 
 
 def _coef_at(schedule, k):

@@ -15,8 +15,11 @@ def pytest_configure(config):
 @pytest.fixture(scope="session")
 def gpu():
     """Initialise the library on device 0; a missing library or GPU is an error, not a skip."""
-    from ancora_cutile_amd import _lib
+    from ancora_cutile_amd import _lib, muon_ns
     _lib.init(0)
+    # modes that force one tile size instead of the rule by launch size (ANC_NS_FORCE_T*)
+    muon_ns.MODES.update({f"{m}_t{t}": muon_ns.MODES[m] | flag for m in ("bf16", "bf16_late3", "bf16_x3")
+                          for t, flag in ((64, 0x200), (128, 0x400), (256, 0x800))})
     return _lib
 
 
