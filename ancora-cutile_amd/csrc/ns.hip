@@ -754,6 +754,8 @@ struct ChainProb {
 //   A = X X^T   26 x (1024,1024) 374 / 430 on 128 / 256 (4160), 48 x (768,768) 535 / 569 (4608),
 //               22 x (1280,1280) 558 / 535 (5280);   X = a X + B X   33 x (768,768) 474 / 499 (4752),
 //               20 x (1024,1024) 370 / 392 (5120), 26 x (1024,1024) 515 / 487 (6656)
+// One line, 4900, ends that band for both kinds. It is the symmetric products'; X = a X + B X would gain from a later
+// one (5120 tiles run on 256-wide tiles and lose those 6 %).
 int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
@@ -781,8 +783,10 @@ int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
 //                    (13.0/12.8/12.4)       (28.1/25.0/24.1)
 //   2816             26.6/27.3/34.2         58.2/53.0/50.9         154/99/91         466/230/198
 //                    (21.4/21.3/21.6)       (49.6/48.0/38.1)
-// hence up to 400 tokens 64 below 1300 tiles of 64 and 128 up to 2000 (3000 where something is added to), beyond 64 below 600 and 128 up to 1024, one
-// per CU. (560 and fewer tiles of 64 are fastest at every length: 432 at 8192 tokens 65 / 80 / 97.)
+// hence up to 400 tokens 64 below 1300 tiles of 64 and 128 up to 2000 (3000 where something is added to), beyond 64
+// below 600 and 128 up to 1024, one per CU. (560 and fewer tiles of 64 are fastest at every length: 432 at 8192 tokens
+// 65 / 80 / 97.) Beyond 400 tokens the lines are those of a long batch: around 1024 tokens with gradients added up
+// 128-wide tiles would still be 13 % ahead at 1056 tiles and 8 % at 1344.
 int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0;
   bool adds = false;
@@ -1313,7 +1317,7 @@ extern "C" int anc_ns_batched_pair(uint64_t Uh, uint64_t Ul, uint64_t fro_partia
 // n_probs <= 8 independent batches (the shape groups of one optimizer step) through the chain
 // side by side: each product of each step is one launch over all of them, which keeps the
 // CUs busy where per-batch launches would each end in a partly filled last wave. Same
-// results, bit for bit, as anc_ns_batched_pair on each batch. All dims multiples of 256.
+// results, bit for bit, as anc_ns_batched_pair on each batch. All dims multiples of 128.
 static int pair_multi_impl(const char *who, const anc_ns_problem_t *probs, int32_t n_probs,
                            const uint64_t *desc_tables, const NsUpdate *upd, int steps, const float *coef,
                            float eps, int mode, uint64_t stream) {
