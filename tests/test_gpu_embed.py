@@ -42,6 +42,36 @@ def test_embed_dw_scatter_is_the_sequential_sum(gpu, M, V, H, seed):
     grp.free()
 
 
+def test_groups_used_on_two_streams_and_blocks_taken_again(gpu):
+    """Batches in flight on two streams, each also read on the other stream, more of them than blocks are kept, given
+    back while their work is queued: every sum is the batch's own."""
+    from ancora_cutile_amd import DevBuf
+    from ancora_cutile_amd.embed import IdGroups, _Blocks, embed_dw_scatter
+    M, V, H, n = 2048, 300, 512, 3 * _Blocks.KEEP
+    rng = np.random.default_rng(7)
+    streams = [gpu.stream_create(), gpu.stream_create()]
+    dyb = bf16_rne_bits(rng.standard_normal((M, H)).astype(np.float32)).reshape(M, H)
+    gdy = DevBuf(dyb)
+    outs, ids = [], [rng.integers(0, V, M).astype(np.int32) for _ in range(n)]
+    for i in range(n):
+        outs.append([DevBuf.zeros((M, H), np.float32, s) for s in streams])
+    gpu.api.anc_device_sync()
+    for i in range(n):
+        grp = IdGroups(ids[i])
+        for k in (i & 1, 1 - (i & 1)):
+            embed_dw_scatter(grp, gdy, streams[k], compact=outs[i][k])
+        grp.free()
+    gpu.api.anc_device_sync()
+    for i in range(n):
+        gid, rows = embed_dw_rows(ids[i], dyb)
+        for o in outs[i]:
+            assert bits_equal(o.to_numpy()[:gid.size], rows), i
+            o.free()
+    gdy.free()
+    for s in streams:
+        gpu.api.anc_stream_destroy(s)
+
+
 def test_first_scatter_of_a_batch_inside_a_graph(gpu):
     """Group arrays made before a capture and first used in it: every replay, with other groups in use between them,
     adds the batch's sums."""

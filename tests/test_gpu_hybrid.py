@@ -511,3 +511,61 @@ def test_wide_spectrum_gradients_through_the_grouped_step(gpu):
     alone.step({"l0.q_proj": grads["l0.q_proj"]}, 0)
     assert bits_equal(alone.master()["l0.q_proj"], got["l0.q_proj"])
     alone.free()
+
+
+def _engine_run(W0, G, shapes, steps=2, transposed=(), **kw):
+    """Masters, bf16 copies, momenta and transposed copies after `steps` of one MuonEngine over all the weights."""
+    from ancora_cutile_amd import DevBuf, PE_SCHEDULE as PE
+    from ancora_cutile_amd.muon import MuonEngine
+    fused = kw.pop("fused_update", True)
+    ws = [dict(buf=DevBuf.zeros(s, np.float32), p32=DevBuf(w), p16=DevBuf.zeros(s, np.uint16), G=DevBuf(g), K=s[0], N=s[1],
+               seed=10 + i, p16T=DevBuf.zeros(s[::-1], np.uint16) if i in transposed else None)
+          for i, (s, w, g) in enumerate(zip(shapes, W0, G))]
+    eng = MuonEngine(ws, **kw)
+    eng.fused_update = fused
+    for _ in range(steps):
+        eng.step(0, lr=0.02, schedule=PE)
+    out = [[None if w[k] is None else w[k].to_numpy() for k in ("p32", "p16", "buf", "p16T")] for w in ws]
+    n_batches = len(eng.batches)
+    eng.free()
+    for w in ws:
+        for k in ("buf", "p32", "p16", "G", "p16T"):
+            if w[k] is not None:
+                w[k].free()
+    return out, n_batches
+
+
+def _same(a, b):
+    return all((u is None and v is None) or bits_equal(u, v) for x, y in zip(a, b) for u, v in zip(x, y))
+
+
+@pytest.mark.parametrize("sr", [False, True])
+@pytest.mark.parametrize("shapes", [[(128, 128)], [(128, 384), (384, 128)], [(256, 512), (512, 256), (256, 256)],
+                                    [(640, 896), (896, 640)], [(1024, 1024), (2048, 1024)]], ids=str)
+def test_fused_update_on_every_tile_width(gpu, sr, shapes):
+    """Update, stochastic rounding and the transposed copy in the last epilogue of 64-, 128- and 256-wide tiles, square,
+    wide and tall weights: the bits of the chain followed by the update kernel."""
+    rng = np.random.default_rng(shapes[0][0] + shapes[0][1])
+    W0 = [(0.02 * rng.standard_normal(s)).astype(np.float32) for s in shapes]
+    G = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+    for transposed in ((), tuple(range(len(shapes))), (0,)):
+        want, _ = _engine_run(W0, G, shapes, transposed=transposed, sr=sr, seed=3, fused_update=False)
+        for mode in ("bf16", "bf16_t64", "bf16_t128", "bf16_t256"):
+            got, _ = _engine_run(W0, G, shapes, transposed=transposed, sr=sr, seed=3, mode=mode)
+            assert _same(got, want), (transposed, mode)
+        for i in transposed:
+            assert bits_equal(want[i][3], np.ascontiguousarray(want[i][1].T)), i
+
+
+def test_engine_of_more_batches_than_a_chain_call_takes(gpu):
+    """Eleven batches: one momentum launch, two chain calls, every weight with the bits it has alone."""
+    shapes = [(128, 128), (128, 256), (256, 128), (256, 256), (128, 384), (384, 128), (256, 512), (384, 384), (128, 640),
+              (512, 512), (640, 256)]
+    rng = np.random.default_rng(12)
+    W0 = [(0.02 * rng.standard_normal(s)).astype(np.float32) for s in shapes]
+    G = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+    got, n = _engine_run(W0, G, shapes, chunk=1, transposed=(2, 9))
+    assert n == 11
+    for i, s in enumerate(shapes):
+        alone, _ = _engine_run(W0[i:i + 1], G[i:i + 1], [s], transposed=(0,) if i in (2, 9) else ())
+        assert _same(alone, got[i:i + 1]), s

@@ -224,6 +224,23 @@ def test_bf16_entry_takes_the_matrix_as_it_is(gpu, E, M, N, sched):
     g.free()
 
 
+@pytest.mark.parametrize("M,N", [(128, 128), (128, 640), (256, 512), (640, 640), (1024, 1024), (1024, 1152), (1024, 2048)])
+def test_bf16_entry_on_every_tile_width(gpu, M, N):
+    """A matrix without a low half on tiles of 64, 128 and 256: the bits of the choice by launch size."""
+    from ancora_cutile_amd import DevBuf, newton_schulz_resident_e
+    rng = np.random.default_rng(M + 3 * N)
+    x = rng.standard_normal((2 * M, N)).astype(np.float32)
+    x[M:, : max(1, N // 100)] *= 100.0                          # outlier columns: the gates
+    want = None
+    for mode in ("bf16", "bf16_t64", "bf16_t128", "bf16_t256"):
+        g = DevBuf(bf16_rne_bits(x).reshape(2 * M, N))
+        newton_schulz_resident_e(g, None, None, None, None, None, 2, M, N, 0, schedule=PE_SCHEDULE, mode=mode)
+        got = g.to_numpy()
+        g.free()
+        want = got if want is None else want
+        assert bits_equal(got, want), mode
+
+
 @pytest.mark.parametrize("M,N", [(128, 384), (1024, 2048)])
 @pytest.mark.parametrize("sched", ["pe", "keller"])
 def test_bf16_entry_takes_large_magnitudes(gpu, M, N, sched):
