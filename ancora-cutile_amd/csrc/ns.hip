@@ -1044,10 +1044,10 @@ extern "C" int64_t anc_ns_workspace_bytes(int64_t E, int64_t M, int64_t N, int m
   return a > b ? a : b;
 }
 
-// FLOPs of the output tiles a symmetric M x M product really multiplies, per unit of K: the tiles
-// on or below the diagonal, 256x256 where the 256-tile kernel runs (dims multiples of 256 and the
-// 128-tile kernel not forced), else 128x128. A diagonal tile is multiplied in full, so the count is
-// 10/16 of the dense product at M = 1024 with 256-tiles and 36/64 with 128-tiles; the matrix-
+// FLOPs of the output blocks a symmetric M x M product really multiplies, per unit of K: those on or below
+// the diagonal, 256x256 where both dims are multiples of 256 and ANC_NS_TILE128 is not set, else 128x128
+// (NsGemm::diag), whatever the launch's tiles. A block on the diagonal is multiplied in full, so the count is
+// 10/16 of the dense product at M = 1024 with 256-wide blocks and 36/64 with 128-wide ones; the matrix-
 // instruction counter of the profiler reads exactly this.
 static double sym_tile_flops(int64_t M, int64_t N, bool force_small) {
   const double ts = (!force_small && M % 256 == 0 && N % 256 == 0) ? 256.0 : 128.0;

@@ -244,8 +244,8 @@ int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, h
 int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool small, bool by_rows,
                            const NsUpdate *upd, bool plain);
 // Bare fp32 products C[e] = A[e] B[e] on the same K loops; a_transposed: A is
-// given as (K, M) row-major with row pitch ldA (and strideA between matrices), C = A^T B. The tiles are chosen as
-// for X = a X + B X, by the same rule and with the same bits.
+// given as (K, M) row-major with row pitch ldA (and strideA between matrices), C = A^T B. The tiles are chosen
+// by a rule of their own (pick_tile_plain); the bits are the same on all.
 int anc_ns_gemm_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool a_transposed);
 int anc_ns_gemm_big_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool a_transposed = false);
 // Momentum of one weight as a bf16 pair (muon_elem.hip): high halves to d.u, low halves to `lo`, a sum of u*u per 4096

@@ -7,7 +7,7 @@
 // product lasts as long as the CU with the most tiles needs for its operands: a single 1024x1024
 // output is 10 tiles of 256x256 (10 CUs at work, 512 K-bytes each step) or 160 of 64x64 (160 CUs,
 // 128), a quarter of the time although the operands are fetched four times as often. Which tile a
-// launch takes is anc_ns_gemm_multi's rule (below).
+// launch takes is a rule of ns.hip (pick_tile, pick_tile_plain).
 //
 // Layout. 4 wavefronts as 2x2, each WB x WB blocks of v_mfma_f32_32x32x16_bf16 (tile 64 WB). A stage is 16 KiB,
 // one half per operand: KP = 2 (64x64) or 1 (128x128) panels of 32 k. Operands arrive in pieces of 16 rows x
@@ -25,7 +25,7 @@
 // consecutive columns of a row (or, for mirrored halves, transposed weights and their transposed copies, 16
 // consecutive rows of a column): a 32x32 block in panel layout is 2 KiB contiguous.
 //
-// Same bits as the 256-wide tiles: terms in order, k ascending, one accumulator, and a symmetric product is
+// Same bits as the 256-wide tiles: one accumulator, k ascending, the terms of a step together, and a symmetric product is
 // computed directly inside the 256x256 blocks on the diagonal (128x128 where M is no multiple of 256) and mirrored outside,
 // where residual terms make element (i, j) and element (j, i) differ in the last bit.
 #include <type_traits>

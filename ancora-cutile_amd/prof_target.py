@@ -97,11 +97,11 @@ def main(argv):
         xT = DevBuf(bits(0.1 * rng.standard_normal((K, T))))
         probs = [dict(xT=xT, dy=DevBuf(bits(0.1 * rng.standard_normal((T, N)))), dW=DevBuf.zeros((K, N), np.float32),
                       g16=DevBuf.zeros((K, N), np.uint16), T=T, K=K, N=N, workspace=DwWorkspace()) for N in Ns]
-        gemm_dW(probs)
+        gemm_dW(probs, 0, segments="shape")
         _lib.stream_sync(0)
         _lib.profile_enable(True)
         for _ in range(calls):
-            gemm_dW(probs)
+            gemm_dW(probs, 0, segments="shape")
         pr = _lib.profile_read()
         _lib.profile_enable(False)
         fl = sum(dw_info(T, K, N)[0] for N in Ns)
