@@ -175,8 +175,8 @@ def main(argv):
             grp.free()
         print(f"(V, H) = ({V}, {H}), {T} tokens per step, {uniq / steps:.0f} distinct rows on average, {steps} steps")
         print(f"  catch-up of the rows the forward gathers  {t_cu / steps * 1e3:8.1f} us (includes the upload of the row list)")
-        print(f"  sorted-scatter gradient rows              {t_sc / steps * 1e3:8.1f} us")
-        print(f"  row-sparse AdamW step                     {t_sp / steps * 1e3:8.1f} us (includes the 16-byte step-table upload)")
+        print(f"  sorted-scatter gradient rows              {t_sc / steps * 1e3:8.1f} us (includes the upload of the group arrays)")
+        print(f"  row-sparse AdamW step                     {t_sp / steps * 1e3:8.1f} us (every 256th with an upload of the step table)")
         print(f"  dense AdamW sweep of the same table       {t_de / steps * 1e3:8.1f} us ({28.0 * V * H / (t_de / steps) / 1e9:.2f} TB/s)")
     else:
         raise SystemExit(__doc__)
