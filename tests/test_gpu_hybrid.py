@@ -569,3 +569,47 @@ def test_engine_of_more_batches_than_a_chain_call_takes(gpu):
     for i, s in enumerate(shapes):
         alone, _ = _engine_run(W0[i:i + 1], G[i:i + 1], [s], transposed=(0,) if i in (2, 9) else ())
         assert _same(alone, got[i:i + 1]), s
+
+
+def test_guarded_step_in_a_graph(gpu):
+    """A guarded step on resident gradients, captured after a first one, replayed four times with other steps and
+    synchronisations between: the state of as many ordinary steps. A host gradient cannot be captured and leaves
+    the capture and later uploads alone."""
+    import ctypes
+    from ancora_cutile_amd import DevBuf, HybridOptimizer, PE_SCHEDULE as PE, _lib
+    hip = ctypes.CDLL("libamdhip64.so")
+    rng = np.random.default_rng(31)
+    shapes = {"embed": (640, 64), "norm": (256,), "q_proj": (256, 384), "o_proj": (512, 256), "k_proj": (256, 256)}
+    params = {n: (0.02 * rng.standard_normal(s)).astype(np.float32) for n, s in shapes.items()}
+    host = {n: (1e-3 * rng.standard_normal(s)).astype(np.float32) for n, s in shapes.items()}
+    grads = {n: DevBuf(g) for n, g in host.items()}
+
+    def make():
+        return HybridOptimizer(params, muon_kw=dict(schedule=PE, sr=True), max_grad_norm=0.5,
+                               adamw_kw=dict(lr=3e-4, betas=(0.9, 0.95), eps=1e-8, wd=0.1, sr=True))
+
+    eager, captured, s = make(), make(), gpu.stream_create()
+    eager.step(grads, s)
+    captured.step(grads, s)
+    graph, graph_exec = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(ctypes.c_void_p(s), 0) == 0
+    with pytest.raises(_lib.AncoraError):
+        captured.muon.st["q_proj"]["g"].upload_async(host["q_proj"], s)
+    captured.step(grads, s, sync=False)
+    assert hip.hipStreamEndCapture(ctypes.c_void_p(s), ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(graph_exec), graph, None, None, ctypes.c_size_t(0)) == 0
+    for i in range(4):
+        eager.step(grads if i & 1 else host, s)            # (uploads through every slot between the replays)
+        assert hip.hipGraphLaunch(graph_exec, ctypes.c_void_p(s)) == 0
+        gpu.stream_sync(s)
+        a, b = eager.muon.state_dict(), captured.muon.state_dict()
+        assert all(bits_equal(a[k], b[k]) for k in a if k != "t"), i
+        a, b = eager.adamw.state_dict(), captured.adamw.state_dict()
+        assert all(bits_equal(a[k], b[k]) for k in a if k != "t"), i
+    assert captured.guard.read(s)["t"] == eager.guard.read(s)["t"] == 5
+    hip.hipGraphExecDestroy(graph_exec)
+    hip.hipGraphDestroy(graph)
+    eager.free(); captured.free()
+    for g in grads.values():
+        g.free()
+    gpu.api.anc_stream_destroy(s)
