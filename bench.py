@@ -555,7 +555,7 @@ def side_workload(args):
                           "activations": "x (T,K) as they lie" if args.dw_acts == "x" else "x^T (K,T), transposed by the caller"},
                "roofline": {"bound": "mfma", "achieved": round(gtf, 1), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                             "frac": round(gtf / PEAK_BF16_TFLOPS, 4), "traffic": None,
-                            "kernel": "k_ns_gemm_big<EPI_BX, ..., VAR_PLAIN> (partial tiles of x^T dy)",
+                            "kernel": "the bare product of k_ns_gemm_big or k_ns_gemm_tile, by the size of the call (x^T dy)",
                             "launches_per_step": pr["dw_gemm"][1], "avg_launch_ms": round(g_ms / pr["dw_gemm"][1], 4),
                             "tflop_per_step": round(layers * flops / 1e12, 3)},
                "whole_tflops_per_s": round(tf, 1),

@@ -547,7 +547,8 @@ int anc_ns_batched(uint64_t X, int64_t E, int64_t M, int64_t N,
 
 /* The same chain on (E,M,N) bf16 matrices in place (the reference-typed drivers): no widened copy; steps >= 2,
  * bf16 modes. The input enters unscaled and exact, its norm applied by the first step's epilogues as in
- * anc_ns_batched_pair; a matrix of norm below 9e-16 is first brought into [1, 2) by a power of two, in place. */
+ * anc_ns_batched_pair; a matrix of norm outside 9e-16 .. 1.1e15 is first brought into [1, 2) by a power of two, in
+ * place. */
 int anc_ns_batched_bf16(uint64_t X, int64_t E, int64_t M, int64_t N, int steps, const float *coef, float eps,
                         int mode, uint64_t workspace, int64_t workspace_bytes, uint64_t stream);
 
@@ -569,10 +570,11 @@ int anc_muon_resident_step(uint64_t buf, uint64_t g, int g_dtype, uint64_t p32, 
  * (Uh at X32_out, Ul right behind it: the same 4 bytes per element); steps >= 2. bf16
  * modes only. Results differ from anc_ns_batched on the same data only by where the bf16
  * rounding of the first operand falls (before instead of after the scaling). The first products
- * run on the unnormalised values: a matrix whose sum of squares is below 2^-100 (||U||_F < 9e-16,
- * where products of two elements would underflow fp32) is first multiplied in place, Uh and Ul,
- * by the power of two that brings its norm into [1, 2), exactly, and its scale carries the
- * inverse; every other matrix is left as it is. */
+ * run on the unnormalised values: a matrix whose sum of squares is outside 2^-100 .. 2^100 (||U||_F
+ * below 9e-16 or above 1.1e15, where products of two elements, or the scale's square, would leave the range of
+ * fp32) is first multiplied in place, Uh and Ul, by the power of two that brings its norm into [1, 2),
+ * exactly, and its scale carries the inverse; every other matrix is left as it is. Partial sums that
+ * are not finite are replaced by a sum over the matrix itself. */
 int anc_ns_batched_pair(uint64_t Uh, uint64_t Ul, uint64_t fro_partials, int64_t n_partials,
                         uint64_t X32_out, int64_t E, int64_t M, int64_t N,
                         int steps, const float *coef, float eps, int mode,
