@@ -27,11 +27,11 @@
 // Determinism: one workgroup owns one output tile (64 to 256 wide) and its whole K loop, terms in
 // a fixed order, K tiles in ascending order; no split-K, no atomics. A matrix's result
 // does not depend on the batch size E or on its position in the batch. Symmetric outputs
-// (A, B) compute the tiles on or below the diagonal and mirror them; without residual terms
-// that is bit-identical to computing both halves (same products, same order, and an epilogue
+// (A, B) are multiplied in the 64x64 blocks on and below the diagonal, whatever the launch's tiles, and mirrored;
+// without residual terms that is bit-identical to computing both halves (same products, same order, and an epilogue
 // that is symmetric in (i,j)). With residual terms the two cross products Xh Xl^T and
 // Xl Xh^T enter one accumulator in a fixed order, so elements computed directly inside a
-// diagonal tile differ from their mirror images in the last bits; nothing depends on it.
+// diagonal block differ from their mirror images in the last bits; nothing depends on it.
 //
 // The products run on the tiles of ns_gemm_big.hip (256 wide) and ns_gemm_tile.hip (128 and 64 wide), chosen per
 // launch by the number of tiles (pick_tile); the bits are the same on all of them.
@@ -739,35 +739,42 @@ struct ChainProb {
   const anc_muon_desc_t *upd;  // or: the weights (E entries) the last step updates in its epilogue
 };
 
-// Tiles of a launch, from the tiles each size would give it, weighted by their K against the longest
-// (a launch ends with its longest tiles; short ones fill gaps). A CU takes operand bytes into LDS at one
-// rate whatever the tile, so small tiles finish first while they find idle CUs and lose, by the bytes they
-// fetch more often, once every CU has several. Measured, us per 5 launches on 64 / 128 / 256-wide tiles:
-//   A = X X^T   16 x (512,512) 101 / 108 / 193 (768 tiles of 64), 4 x (1024,1024) 105 / 110 / 189 (640),
-//               5 x (1024,1024) 127 / 116 / 190 (800), 12 x (1024,1024) 221 / 178 / 204 (1920),
-//               16 x (1024,1024) 280 / 245 / 225 (2560)
-//   X = a X + B X   8 x (512,512) 72 / 99 / 157 (512), 4 x (1024,1024) 123 / 114 / 157 (1024),
-//               6 x (512,1536) 124 / 142 / 166 (1152), 2 x (1024,3072) 151 / 136 / 148 (1536),
-//               3 x (1024,3072) 202 / 193 / 199 (2304), 4 x (1024,3072) 258 / 222 / 211 (3072)
-// hence 64 below 800 (symmetric), or below 1400 tiles of 64 except from 800 to 1024, where one tile of 128 per
-// CU does; 128 up to 2200 (symmetric) or 2700. The large tiles fill the chip once at 4096; just beyond, 128 again:
-//   A = X X^T   26 x (1024,1024) 374 / 430 on 128 / 256 (4160), 48 x (768,768) 535 / 569 (4608),
-//               22 x (1280,1280) 558 / 535 (5280);   X = a X + B X   33 x (768,768) 474 / 499 (4752),
-//               20 x (1024,1024) 370 / 392 (5120), 26 x (1024,1024) 515 / 487 (6656)
-// One line, 4900, ends that band for both kinds. It is the symmetric products'; X = a X + B X would gain from a later
-// one (5120 tiles run on 256-wide tiles and lose those 6 %).
+// Tiles of a launch, from the number of 64x64 tiles it has (symmetric products: those on and below the diagonal),
+// problems weighted by their K against the longest (a launch ends with its longest tiles; short ones fill gaps). A CU
+// takes operand bytes into LDS at one rate whatever the tile, so small tiles finish first while they find idle CUs and
+// lose, by the bytes they fetch more often, once every CU has several; large ones lose where the last of them have
+// the chip to themselves. With residual terms a K tile brings three products, so small tiles hold out longer.
+// Measured, us per 5 launches on 64 / 128 / 256-wide tiles (tiles of 64):
+//   A = X X^T, mostly one term     4 x (1024,1024) 102 / 104 / 179 (544), 6 x 126 / 111 / 185 (816), 12 x 193 / 171 / 203
+//               (1632), 20 x 310 / 266 / 238 (2720);  3 x (1024,3072) 121 / 155 / 293 (408), 6 x 213 / 172 / 307 (816)
+//   residual terms                 20 x (512,1536) 178 / 191 / 392 (720), 18 x (640,1792) 257 / 315 (990), 16 x (768,768)
+//               172 / 183 / 251 (1248), 24 x 248 / 226 / 268 (1872), 30 x 329 / 320 / 286 (2340)
+//   just over one round of 256-wide tiles    26 x (1024,1024) 393 / 334 / 387 (260 of them), 48 x (768,768) 555 / 465 / 522
+//               (288), 33 x (1024,1024) 520 / 449 / 437 (330)
+//   X = a X + B X, mostly one term 2 x (1024,2048) 107 / 95 / 144 (1024), 5 x (1024,1024) 137 / 140 / 156 (1280), 6 x 156 / 147 /
+//               155 (1536), 5 x (1024,2048) 207 / 188 / 198 (2560), 4 x (1024,3072) 235 / 206 / 204 (3072),
+//               8 x (1024,2048) 303 / 258 / 233 (4096)
+//   residual terms                 8 x (512,1536) 136 / 139 / 159 (1536), 12 x 192 / 203 / 212 (2304), 16 x 241 / 221 / 229
+//               (3072), 20 x 291 / 273 / 267 (3840)
+//   just over one round of large tiles (4096)    6 x (1024,3072) 327 / 295 / 305 (4608), 20 x (1024,1024) 429 / 361 / 389
+//               (5120), 28 x (512,1536) 394 / 387 / 382 (5376), 8 x (1024,3072) 432 / 357 / 335 (6144)
 int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
-  double longest = 0.0, t64 = 0.0;
+  double longest = 0.0, t64 = 0.0, t256 = 0.0, several = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
   for (int k = 0; k < n; ++k) {
-    const double m = (double)(ps[k].M / 64), d = (double)(ps[k].diag / 64);
-    const double per = epi == EPI_BX ? m * (double)(ps[k].N / 64) : m * (m + d) / 2.0;
-    t64 += (double)Es[k] * per * ((double)ps[k].K / longest);
+    const double m = (double)(ps[k].M / 64), q = (double)ps[k].M / 256.0, w = (double)Es[k] * ((double)ps[k].K / longest);
+    const double t = w * (epi == EPI_BX ? m * (double)(ps[k].N / 64) : m * (m + 1.0) / 2.0);
+    t64 += t;
+    t256 += w * (q * (q + 1.0) / 2.0);
+    if (ps[k].nterms > 1) several += t;
   }
-  if (t64 > 4096.0 && t64 <= 4900.0) return 128;      // a second round of large tiles that is nearly empty
-  if (epi != EPI_BX) return t64 < 800.0 ? 64 : t64 <= 2200.0 ? 128 : 256;
-  if (t64 < 1400.0 && !(t64 > 800.0 && t64 <= 1024.0)) return 64;
-  return t64 <= 2700.0 ? 128 : 256;
+  const bool terms = several > 0.5 * t64;
+  if (epi != EPI_BX) {
+    if (t64 <= (terms ? 1300.0 : 520.0)) return 64;
+    return t64 <= 2050.0 || (t256 > 256.0 && t256 <= 306.0) ? 128 : 256;
+  }
+  if (t64 <= (terms ? 2350.0 : 1400.0) && (terms || !(t64 > 800.0 && t64 <= 1024.0))) return 64;
+  return t64 <= 3500.0 || (t64 > 4096.0 && t64 <= 5200.0) ? 128 : 256;
 }
 
 // The same for the bare product of weight gradients. Its K is a batch of tokens: short ones are bound by the
@@ -829,12 +836,11 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       const int64_t M = cp[q].M, N = cp[q].N, mn = M * N;
       const bool split = k >= pl.sp.x_from;        // X residual terms
       const bool split_fb = k >= pl.sp.fb_from;    // F and Boff residual terms
-      // a property of the shape, whatever the tiles: blocks on the diagonal of a symmetric product that are
-      // computed in full, and whether low halves of the iterate may be 8 bits
+      // a property of the shape: whether 256-wide tiles fit, and with them 8-bit low halves of the iterate
       const bool wide256 = !(flags & ANC_NS_TILE128) && M % 256 == 0 && N % 256 == 0;
       NsGemm g{};
       g.M = (int)M; g.N = (int)N;
-      g.diag = wide256 ? 256 : 128;
+      g.fits256 = wide256 ? 1 : 0;
       g.A32 = pl.A32; g.Fh = pl.Fh; g.dA = pl.dA; g.Bh = pl.Bh; g.dB = pl.dB;
       if (pl.sp.drop_a32) {
         // the first iteration runs before the classification: nobody is flagged yet
@@ -1005,24 +1011,25 @@ int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int f
       int m = 0;
       for (int k = 0; k < n; ++k) {
         if (epi == EPI_BX ? (ps[k].M >= 1024) != by_rows : (pass & 1) != 0) continue;
-        if (!all && (ps[k].diag == 256) != wide) continue;
+        if (!all && (ps[k].fits256 != 0) != wide) continue;
         part[m] = ps[k];
         pe[m++] = Es[k];
       }
       return m;
     };
     const auto pick = [&](int m) { return force ? force : pick_tile(epi, part, pe, m); };
+    const auto narrow = [](int tile) { return tile == 256 ? 128 : tile; };
     const NsUpdate *u = any_upd ? upd : nullptr;
     const int m_wide = collect(false);
     if (wide) {
       if (m_wide > 0 && pick(m_wide) == 256) {
         if (int rc = anc_ns_gemm_big_multi(epi, part, pe, m_wide, s, by_rows, u)) return rc;
       } else if (const int m = collect(true)) {
-        if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m, s, pick(m) == 64, by_rows, u, false)) return rc;
+        if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m, s, narrow(pick(m)), by_rows, u, false)) return rc;
         done[pass & 1] = true;
       }
     } else if (m_wide > 0 && !done[pass & 1]) {
-      if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m_wide, s, pick(m_wide) == 64, by_rows, u, false)) return rc;
+      if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m_wide, s, narrow(pick(m_wide)), by_rows, u, false)) return rc;
     }
   }
   return ANC_OK;
@@ -1032,7 +1039,7 @@ int anc_ns_gemm_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s,
   ANC_REQUIRE(n >= 1 && n <= kMaxGroups, "anc_ns_gemm_plain: 1..%d problems per launch", kMaxGroups);
   const int tile = pick_tile_plain(ps, Es, n);
   if (tile == 256) return anc_ns_gemm_big_plain(ps, Es, n, s, a_transposed);
-  return anc_ns_gemm_tile_multi(EPI_BX, ps, Es, n, s, tile == 64, a_transposed, nullptr, true);
+  return anc_ns_gemm_tile_multi(EPI_BX, ps, Es, n, s, tile, a_transposed, nullptr, true);
 }
 
 extern "C" int64_t anc_ns_workspace_bytes(int64_t E, int64_t M, int64_t N, int mode) {
@@ -1044,11 +1051,9 @@ extern "C" int64_t anc_ns_workspace_bytes(int64_t E, int64_t M, int64_t N, int m
   return a > b ? a : b;
 }
 
-// FLOPs of the output blocks a symmetric M x M product really multiplies, per unit of K: those on or below
-// the diagonal, 256x256 where both dims are multiples of 256 and ANC_NS_TILE128 is not set, else 128x128
-// (NsGemm::diag), whatever the launch's tiles. A block on the diagonal is multiplied in full, so the count is
-// 10/16 of the dense product at M = 1024 with 256-wide blocks and 36/64 with 128-wide ones; the matrix-
-// instruction counter of the profiler reads exactly this.
+// FLOPs of a symmetric M x M product, per unit of K, counted in blocks on or below the diagonal: 256x256 where both
+// dims are multiples of 256 and ANC_NS_TILE128 is not set, else 128x128: M^2 + 256 M or M^2 + 128 M. The kernels multiply
+// 64x64 blocks, M^2 + 64 M.
 static double sym_tile_flops(int64_t M, int64_t N, bool force_small) {
   const double ts = (!force_small && M % 256 == 0 && N % 256 == 0) ? 256.0 : 128.0;
   const double t = (double)M / ts;

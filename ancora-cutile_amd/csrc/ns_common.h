@@ -61,11 +61,10 @@ struct NsGemm {
                              // product sets it: its A is a K-range of a longer row)
   int64_t strideA, strideB;  // elements between consecutive matrices
   int tiles_m, tiles_n;
-  int lower;                 // symmetric output: tiles with tn <= tm only, mirrored
+  int lower;                 // symmetric output: 64x64 blocks on and below the diagonal only, mirrored
   int plain_sum;             // plain product: 1 = write X32 = (A32, if not null, else 0) + A B and, if Yh is
                              // not null, its bf16 copy (RNE) to Yh; 0 = write X32 = A B
-  int diag;                  // symmetric output: width of the blocks on the diagonal that are computed in full
-                             // (256 or 128); everything below them is mirrored
+  int fits256;               // the chain's dims are multiples of 256 (and no flag says otherwise): 256-wide tiles may run
   int blk_r, blk_c;          // plain product and X = a X + B X: the tile sequence of a matrix runs block by block, blocks of
                              // blk_r x blk_c tiles (rows x columns): (tiles_m, 1) = column panel by column
                              // panel, (1, tiles_n) or 0 = row by row
@@ -240,8 +239,10 @@ int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int f
 // (ns_gemm_big.hip; M and N multiples of 256); `by_rows`: X = a X + B X reads its B by rows k.
 int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool by_rows,
                           const NsUpdate *upd);
-// 64x64 (small) or 128x128 tiles (ns_gemm_tile.hip; M and N multiples of 128); `plain`: the bare product.
-int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool small, bool by_rows,
+// Tiles of 64x64 (`tile` 64), 128x64 (kTile128x64) or 128x128 (128) outputs (ns_gemm_tile.hip; M and N multiples of 128);
+// `plain`: the bare product.
+constexpr int kTile128x64 = 12864;
+int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int tile, bool by_rows,
                            const NsUpdate *upd, bool plain);
 // Bare fp32 products C[e] = A[e] B[e] on the same K loops; a_transposed: A is
 // given as (K, M) row-major with row pitch ldA (and strideA between matrices), C = A^T B. The tiles are chosen

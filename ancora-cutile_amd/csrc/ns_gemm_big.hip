@@ -6,7 +6,9 @@
 // of the per-XCD L2 than it delivers. Every wavefront here owns 128x64 outputs: 8 accumulator
 // blocks of 32x32 (128 accumulator registers per lane), 6 operand fragments per 8 MFMAs.
 //   symmetric products (A, B): 256x256x32 tile, 8 wavefronts (2 x 4), four 32 KiB LDS stages,
-//     128 FLOP per byte staged, one workgroup per CU;
+//     128 FLOP per byte staged, one workgroup per CU; of a tile on the diagonal the 64x64 blocks on and below it,
+//     5/8 of the products (chains of 48 x (1024,1024) 1794 -> 1725 us, 24 x (1024,2048) 1160 -> 1133 us: fewer
+//     products at the board's power limit as much as shorter tiles);
 //   X = a X + B X: 128x256x32 tile, 4 wavefronts (1 x 4), three 24 KiB stages, two workgroups
 //     per CU. Its epilogue moves 8 bytes of HBM traffic per element (the bf16 pair of the
 //     iterate read and written) and runs at the HBM rate.
@@ -52,6 +54,11 @@ template <typename T> __device__ __forceinline__ void epi_st(T *p, T v) { anc_st
 
 namespace {
 
+// A tile on the diagonal of a symmetric product is multiplied in 64x64 blocks on and below the diagonal: a wavefront's
+// 128x64 outputs are all of that (kFull), their lower half (kLower) or nothing (kNone: it moves its share of the
+// operands only). The blocks above are mirrored from below.
+constexpr int kFull = 0, kLower = 1, kNone = 2;
+
 // SWAP = false: accumulator block (bi,bj) holds C[32 bi + row][32 bj + col] with col = lane%32
 // and element r = row 8*(r/4) + 4*(lane/32) + r%4. SWAP = true computes the transposed block
 // (operands exchanged, same products, same order of summation): row = lane%32 and element
@@ -65,11 +72,12 @@ __device__ __forceinline__ void mfma1(const bf16x8 (&a)[4], const bf16x8 (&b)[2]
 }
 // 8 MFMAs with the fragment reads of the next 8 (`load(idx)`) and N DMA instructions (`piece(i)`) between them, instead
 // of as bursts during which the matrix pipe idles and the LDS serves all wavefronts at once.
-template <bool SWAP, int N, typename L, typename F>
+// (PART: the wavefront's part of a tile, see kFull)
+template <bool SWAP, int N, int PART, typename L, typename F>
 __device__ __forceinline__ void mfma8_with(const bf16x8 (&a)[4], const bf16x8 (&b)[2], f32x16 (&acc)[4][2], L load, F piece) {
 #pragma unroll
   for (int idx = 0; idx < 8; ++idx) {
-    mfma1<SWAP>(a, b, acc, idx);
+    if (PART == kFull || (PART == kLower && idx >= 4)) mfma1<SWAP>(a, b, acc, idx);
     __builtin_amdgcn_sched_barrier(0);
     load(idx);
 #pragma unroll
@@ -209,7 +217,17 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / NWN, wn = wave % NWN;
+  int wm = wave / NWN, wn = wave % NWN, part = kFull;
+  if constexpr (EPI != EPI_BX) {
+    static_assert(TM == 256 && TN == 256, "the dealing below");
+    if (tm == tn) {
+      // Wavefronts w and w + 4 share a SIMD, so a full and a half part meet: (0,0) with (0,1), (1,2) with (1,3), and
+      // (1,0), (1,1) each with one of the two that have nothing to do. The tile takes three quarters of the time.
+      wm = (0x2E >> wave) & 1;
+      wn = (0xED48 >> (2 * wave)) & 3;
+      part = 2 * wm + 1 < wn ? kNone : 2 * wm < wn ? kLower : kFull;
+    }
+  }
   const int K = p.K, nk = K / TK;
 
   // ---- DMA addressing: this wavefront moves IA*RPI rows of the A tile and IB*RPI rows of the B
@@ -350,7 +368,8 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       for (int r = 0; r < 16; ++r) acc[bi][bj][r] = 0.0f;
 
   const int nterms = PLAINV ? 1 : anc_ns_terms(p, e);
-  if (nterms == 1) {
+  auto single = [&](auto prt) {
+    constexpr int P = decltype(prt)::value;
     // Stage ring. Tile k lives in stage k % NS. The DMA of tile k+NS-1 is started at the top of
     // tile k, into the stage that tile k-1 was read from (every wavefront left it before the
     // barrier inside tile k-1). Before the last k-step of tile k each wavefront waits until its
@@ -362,7 +381,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       if (s0 < nk) issue(st(s0));
     if (nk >= NS - 1) wait_vm<(NS - 2) * IPS>(); else wait_vm<0>();
     lds_barrier();
-    frags(stage0, 0, a[0], b[0]);
+    if (P != kNone) frags(stage0, 0, a[0], b[0]);
 
     // a[kk], b[kk] hold k-step kk. `steady` (a std::true_type): the caller knows that this tile refills
     // the ring and has a successor, so the body carries no branch.
@@ -370,7 +389,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       constexpr bool kSteady = decltype(steady)::value;
       const bool more = kSteady || step + 1 < nk;
       const bool refill = kSteady || step + NS - 1 < nk;
-      mfma8_with<BT, IPS>(a[0], b[0], acc, [&](int idx) { frag(cur, cur, 1, idx, a[1], b[1]); },
+      mfma8_with<BT, IPS, P>(a[0], b[0], acc, [&](int idx) { if (P != kNone) frag(cur, cur, 1, idx, a[1], b[1]); },
                           [&](int i) { if (refill) issue_piece(i, fill, curA, curB); });
       if (refill) {
         curA += advA;
@@ -380,11 +399,11 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         wait_vm<0>();
       }
       lds_barrier();
-      mfma8_with<BT, 0>(a[1], b[1], acc, [&](int idx) { if (more) frag(nxt, nxt, 0, idx - 1, a[0], b[0]); }, [](int) {});
+      mfma8_with<BT, 0, P>(a[1], b[1], acc, [&](int idx) { if (P != kNone && more) frag(nxt, nxt, 0, idx - 1, a[0], b[0]); }, [](int) {});
     };
     int step = 0;
     // rounds of NS tiles in which even the last tile (step + NS - 1) still refills the ring
-    for (; step + 2 * NS - 2 < nk; step += NS) {
+    for (; P == kFull && step + 2 * NS - 2 < nk; step += NS) {
 #pragma unroll
       for (int s0 = 0; s0 < NS; ++s0)
         body(std::true_type{}, step + s0, st(s0), st((s0 + 1) % NS), st((s0 + NS - 1) % NS));
@@ -394,7 +413,9 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       for (int s0 = 0; s0 < NS; ++s0)
         if (step + s0 < nk) body(std::false_type{}, step + s0, st(s0), st((s0 + 1) % NS), st((s0 + NS - 1) % NS));
     }
-  } else if constexpr (!PLAINV) {
+  };
+  auto several = [&](auto prt) {
+    constexpr int P = decltype(prt)::value;
     // Several terms: K tile t is two stages, the high halves h_t in stage 2t % NS and the low halves l_t in
     // the next one (of two terms only B's low half is there). Six phases of 8 MFMAs per tile,
     //   P0 hh k 0..15, P1 hh 16..31, P2 hl 16..31, P3 lh 16..31, P4 hl 0..15, P5 lh 0..15,
@@ -429,7 +450,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         wait_vm<PL>();
       }
       lds_barrier();
-      frags(st(0), 0, a[0], b[0]);
+      if (P != kNone) frags(st(0), 0, a[0], b[0]);
       // the fragments of hh 0..15 are in a[x], b[0]; the next tile's end up in a[1 - x], b[0]
       auto body = [&](auto steady, auto parity, int t, unsigned char *H, unsigned char *L, unsigned char *H1, unsigned char *L1) {
         constexpr bool kSteady = decltype(steady)::value;
@@ -437,21 +458,24 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         const bool more = kSteady || t + 1 < nk, more2 = kSteady || t + 2 < nk;
         auto none = [](int) {};
         // P0
-        auto load0 = [&](int idx) { frag(H, H, 1, idx, a[y], b[1]); };
+        auto load0 = [&](int idx) { if (P != kNone) frag(H, H, 1, idx, a[y], b[1]); };
         if (NS == 4) {
-          mfma8_with<BT, PL>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_l(i, L1); });
+          mfma8_with<BT, PL, P>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_l(i, L1); });
           if (more) adv_l();
         } else {
-          mfma8_with<BT, IPS>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_h(i, H1); });
+          mfma8_with<BT, IPS, P>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_h(i, H1); });
           if (more) adv_h();
         }
         // P1
+        if (P == kFull) {
 #pragma unroll
-        for (int idx = 0; idx < 4; ++idx) mfma1<BT>(a[y], b[1], acc, idx);
+          for (int idx = 0; idx < 4; ++idx) mfma1<BT>(a[y], b[1], acc, idx);
+        }
         if (more) wait_vm<NS == 4 ? IPS + PL : IPS>(); else wait_vm<0>();
         lds_barrier();
 #pragma unroll
         for (int idx = 4; idx < 8; ++idx) {
+          if (P == kNone) break;
           mfma1<BT>(a[y], b[1], acc, idx);
           __builtin_amdgcn_sched_barrier(0);
           if (idx < 6) b[0][idx - 4] = frag_b(L, 1, idx - 4);
@@ -459,24 +483,25 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
           __builtin_amdgcn_sched_barrier(0);
         }
         // P2 (of two terms: its last half, P4 has two fragments of A yet to come)
-        mfma8_with<BT, 0>(a[y], b[0], acc, [&](int idx) {
+        mfma8_with<BT, 0, P>(a[y], b[0], acc, [&](int idx) {
+          if (P == kNone) return;
           if (idx < 2) a[x][2 + idx] = NT == 3 ? frag_a(L, 1, 2 + idx) : frag_a(H, 0, 2 + idx);
           else if (NT == 2 && idx < 4) b[1][idx - 2] = frag_b(L, 0, idx - 2);
         }, none);
         if (NT == 3) {
           // P3, P4
-          mfma8_with<BT, 0>(a[x], b[1], acc, [&](int idx) { frag(H, L, 0, idx, a[y], b[0]); }, none);
-          mfma8_with<BT, 0>(a[y], b[0], acc, [&](int idx) { frag(L, H, 0, idx, a[x], b[1]); }, none);
+          mfma8_with<BT, 0, P>(a[x], b[1], acc, [&](int idx) { if (P != kNone) frag(H, L, 0, idx, a[y], b[0]); }, none);
+          mfma8_with<BT, 0, P>(a[y], b[0], acc, [&](int idx) { if (P != kNone) frag(L, H, 0, idx, a[x], b[1]); }, none);
         }
         if (more) wait_vm<NS == 4 ? PL : 0>(); else wait_vm<0>();
         lds_barrier();
         // P5 (P4 of two terms)
-        auto load5 = [&](int idx) { if (more) frag(H1, H1, 0, idx - 1, a[y], b[0]); };
+        auto load5 = [&](int idx) { if (P != kNone && more) frag(H1, H1, 0, idx - 1, a[y], b[0]); };
         if (NS == 4) {
-          mfma8_with<BT, IPS>(a[x], b[1], acc, load5, [&](int i) { if (more2) piece_h(i, H); });
+          mfma8_with<BT, IPS, P>(a[x], b[1], acc, load5, [&](int i) { if (more2) piece_h(i, H); });
           if (more2) adv_h();
         } else {
-          mfma8_with<BT, PL>(a[x], b[1], acc, load5, [&](int i) { if (more) piece_l(i, H); });
+          mfma8_with<BT, PL, P>(a[x], b[1], acc, load5, [&](int i) { if (more) piece_l(i, H); });
           if (more) adv_l();
         }
       };
@@ -499,13 +524,26 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
           one(std::integral_constant<int, 5>{});
         }
       };
-      for (; t + U + 1 < nk; t += U) round(std::true_type{});
+      for (; P == kFull && t + U + 1 < nk; t += U) round(std::true_type{});
       for (; t < nk; t += U) round(std::false_type{});
     };
     if (EPI == EPI_BX && nterms == 2) pairs(std::integral_constant<int, 2>{});
     else pairs(std::integral_constant<int, 3>{});
+  };
+  auto multiply = [&](auto prt) {
+    if constexpr (PLAINV) single(prt);
+    else if (nterms == 1) single(prt);
+    else several(prt);
+  };
+  if constexpr (EPI == EPI_BX) {
+    multiply(std::integral_constant<int, kFull>{});
+  } else {
+    if (part == kFull) multiply(std::integral_constant<int, kFull>{});
+    else if (part == kLower) multiply(std::integral_constant<int, kLower>{});
+    else multiply(std::integral_constant<int, kNone>{});
   }
   __syncthreads();
+  if (EPI != EPI_BX && part == kNone) return;
 
   // ---- epilogue
   if ((VAR == VAR_UPDATE || VAR == VAR_UPDATE_T) && pm.ctl != nullptr && pm.ctl->skip != 0u) return;   // skipped step
@@ -513,7 +551,9 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   const int64_t mm = (int64_t)e * M * M, mv = (int64_t)e * M;
   unsigned char *region = st(wave / WPS) + (wave % WPS) * kStageRegion;
   const int gi0w = tm * TM + wm * 128, gj0w = tn * TN + wn * 64;
-  const bool mirror = (EPI != EPI_BX) && (TN * (tn + 1) <= TM * tm);
+  const int bi0 = part == kLower ? 2 : 0;           // the first slab of 32 rows that was multiplied
+  // a slab below the diagonal's 64x64 blocks is written twice
+  auto mirrored = [&](int bi) { return EPI != EPI_BX && ((gi0w + bi * 32) >> 6) > (gj0w >> 6); };
   float sc = 1.0f;
   if (EPI != EPI_BMAT && p.scale != nullptr) sc = anc_ld_const(p.scale + e);
   const float acc_scale = (EPI == EPI_GRAM) ? sc * sc : sc;
@@ -606,8 +646,8 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     // dA of the wavefront's rows (lanes 0..31) and columns (lanes 32..47, repeated by 48..63)
     const float *dsrc = (lane < 32) ? p.dA + mv + gi0w + lane * 4 : p.dA + mv + gj0w + (lane & 15) * 4;
     dma16(dsrc, lds_addr(aux_w));
-    fetch_a(0);
-    fetch_a(1);
+    fetch_a(bi0);
+    fetch_a(bi0 + 1);
   }
   unsigned char *dvec_lds = aux_w;
   if (EPI == EPI_BX && !PLAINV) {
@@ -934,7 +974,9 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   }
 #pragma unroll
   for (int bi = 0; bi < 4; ++bi) {
+    if (bi < bi0) continue;
     const int gi0 = gi0w + bi * 32;
+    const bool mirror = mirrored(bi);
     // operands of the epilogue first (all loads in flight together), arithmetic after
     float in[2][16], drow[16], dcol[2];
     if (EPI == EPI_BMAT) {
@@ -942,8 +984,8 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       // staged bf16 block (Bh, its mirror, and the same for Bl); the conditional dB stores of
       // diagonal tiles only add to what may stay outstanding, so leaving them out is safe.
       // A slab's fetch is 8 DMA instructions (A32) or 4 (Fh).
-      const int nst = 4 * ((mirror ? 2 : 1) * (write_lo ? 2 : 1));
-      const int young = bi == 0 ? (has_a32 ? 8 : 4) : bi == 3 ? nst : nst + (has_a32 ? 8 : 4);
+      const int nst = bi == bi0 ? 0 : 4 * ((mirrored(bi - 1) ? 2 : 1) * (write_lo ? 2 : 1));
+      const int young = nst + (bi == 3 ? 0 : has_a32 ? 8 : 4);
       if (young >= 24) wait_vm<24>();
       else if (young >= 20) wait_vm<20>();
       else if (young >= 16) wait_vm<16>();
@@ -1073,7 +1115,6 @@ int launch_sym(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s) {
   pm.n = n;
   int64_t grid = 0;
   for (int k = 0; k < n; ++k) {
-    ANC_REQUIRE(ps[k].diag == 256, "anc_ns_gemm_big: 256-wide blocks on the diagonal");
     pm.g[k] = ps[k];
     pm.g[k].tiles_m = pm.g[k].tiles_n = ps[k].M / 256;
     pm.g[k].lower = 1;

@@ -9,10 +9,10 @@
 // 128), a quarter of the time although the operands are fetched four times as often. Which tile a
 // launch takes is a rule of ns.hip (pick_tile, pick_tile_plain).
 //
-// Layout. 4 wavefronts as 2x2, each WB x WB blocks of v_mfma_f32_32x32x16_bf16 (tile 64 WB). A stage is 16 KiB,
-// one half per operand: KP = 2 (64x64) or 1 (128x128) panels of 32 k. Operands arrive in pieces of 16 rows x
-// 64 bytes, one LDS-DMA instruction each, four per wavefront and stage. Stages form a ring of four, two
-// workgroups per CU; 64x64 tiles that outnumber the CUs run on a ring of three, three workgroups per CU, whose
+// Layout. 4 wavefronts as 2x2, each WM x WN blocks of v_mfma_f32_32x32x16_bf16 (tile 64 WM x 64 WN). A stage is
+// KP = 2 (64x64) or 1 panels of 32 k of both operands, 16 KiB (12 KiB of a 128x64 tile). Operands arrive in pieces of 16
+// rows x 64 bytes, one LDS-DMA instruction each. Stages form a ring of four, two workgroups per CU (three of 128x64
+// tiles); 64x64 tiles that outnumber the CUs run on a ring of three, three workgroups per CU, whose
 // K loops and epilogues overlap (chains of five steps: 16 x (512,512) 358 -> 331 us, 4 x (1024,3072) 625 ->
 // 570 us; a single (512,1536), one workgroup per CU, loses 3 % to the shorter ring).
 // An operand whose rows are tile rows ("NT") lies in LDS as [panel][row][64 bytes] with the 16-byte chunk index
@@ -26,8 +26,9 @@
 // consecutive rows of a column): a 32x32 block in panel layout is 2 KiB contiguous.
 //
 // Same bits as the 256-wide tiles: one accumulator, k ascending, the terms of a step together, and a symmetric product is
-// computed directly inside the 256x256 blocks on the diagonal (128x128 where M is no multiple of 256) and mirrored outside,
-// where residual terms make element (i, j) and element (j, i) differ in the last bit.
+// computed directly inside the 64x64 blocks on the diagonal and mirrored from below, where residual terms make element
+// (i, j) and element (j, i) differ in the last bit. (Blocks of 256 before: 24 x (256,512) 150 -> 131 us per chain, 12 x
+// (512,1536) 424 -> 354 us with the order of the several terms' reads below.)
 #include <type_traits>
 
 #include "lds_dma.h"
@@ -35,7 +36,6 @@
 
 namespace {
 
-constexpr int kStageBytes = 16384, kIps = 4;              // a stage, DMA instructions per wavefront and stage
 constexpr int kSgPitch = 36;                              // floats per row of the epilogue buffer
 
 // BYTES (4, 8 or 16) between memory and registers, one instruction.
@@ -52,13 +52,21 @@ __device__ __forceinline__ void st_run(void *p, const uint32_t *w) {
   else *(uint32_t *)p = w[0];
 }
 
+// Workgroups a CU takes: what its 160 KiB of LDS hold, but not more than two rings of four 16 KiB stages.
+constexpr int tile_per_cu(int wm, int wn, int ring) { return (wm == 1 ? ring == 3 : wn == 1) ? 3 : 2; }
+
+// Tiles of the first `rows` rows of TM x TN tiles that hold something on or below the 64x64
+// blocks of the diagonal.
+template <int TM, int TN>
+__host__ __device__ constexpr int anc_sym_tiles(int rows) { return (TM / TN) * (rows * (rows + 1) / 2); }
+
 // SOLO: the launch has one problem, its arguments lie at fixed places.
-template <int EPI, int WB, bool AT, int VAR, int kRing, bool SOLO>
-__global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemmArgs<SOLO ? 1 : kMaxGroups> pm) {
-  constexpr int TM = 64 * WB, KP = WB == 1 ? 2 : 1, TK = 32 * KP;
+template <int EPI, int WM, int WN, bool AT, int VAR, int kRing, bool SOLO>
+__global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_tile(NsGemmArgs<SOLO ? 1 : kMaxGroups> pm) {
+  constexpr int TM = 64 * WM, TN = 64 * WN, KP = WM == 1 ? 2 : 1, TK = 32 * KP;
   constexpr bool BT = EPI == EPI_BX, PLAINV = VAR == VAR_PLAIN;
-  constexpr int kHalf = TM * TK * 2;
-  static_assert(2 * kHalf == kStageBytes && kHalf / 1024 == 8, "stage");
+  constexpr int kHalf = TM * TK * 2, kStageBytes = kHalf + TN * TK * 2;      // A's part of a stage, a stage
+  constexpr int PA = TM * KP / 64, PB = TN * KP / 64, kIps = PA + PB;        // DMA instructions per wavefront and stage
   static_assert(!AT || BT, "A by rows k: X = a X + B X and the plain product only");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing * kStageBytes];
 
@@ -72,14 +80,24 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   // kernel is made for has little else to do)
   const int sr = __builtin_ctz(p.blk_r), sc_ = __builtin_ctz(p.blk_c);
   if (EPI != EPI_BX) {
-    // lower triangle of blocks of G x G tiles (G = blk_r), every tile of a block computed
-    const int q = p.tiles_m >> sr, per = (q * (q + 1) / 2) << (2 * sr);
+    // Tiles that reach the diagonal's 64x64 blocks or lie below them, in rows of blocks of blk_r x blk_c tiles: the
+    // whole blocks of a row, then the tiles of its block on the diagonal.
+    const int per = anc_sym_tiles<TM, TN>(p.tiles_m);
     if (L >= per) { e = L / per; L -= e * per; }
-    const int i = L & (p.blk_r * p.blk_r - 1);
-    int b = L >> (2 * sr), bm = 0;
-    while (b > bm) { b -= bm + 1; ++bm; }
-    tm = (bm << sr) + (i >> sr);
-    tn = (b << sr) + (i & (p.blk_r - 1));
+    const int on_diag = anc_sym_tiles<TM, TN>(p.blk_r);
+    int bm = 0, row = on_diag;
+    while (L >= row) { L -= row; row += p.blk_r * p.blk_c; ++bm; }
+    const int whole = row - on_diag;
+    if (L < whole) {
+      const int i = L & (p.blk_r * p.blk_c - 1);
+      tm = (bm << sr) + (i >> sc_);
+      tn = ((L >> (sr + sc_)) << sc_) + (i & (p.blk_c - 1));
+    } else {
+      int i = L - whole, r = 0;
+      while (i >= (r + 1) * (TM / TN)) { i -= (r + 1) * (TM / TN); ++r; }
+      tm = (bm << sr) + r;
+      tn = (bm << sc_) + i;
+    }
   } else {
     const int per = p.tiles_m * p.tiles_n, across = p.tiles_n >> sc_;
     if (L >= per) { e = L / per; L -= e * per; }
@@ -106,19 +124,23 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   const int dr = lane >> 2, dc = lane & 3;
   const uint32_t voA = (uint32_t)(dr * rpA) + (AT ? dc : dc ^ (dr >> 2)) * 16;
   const uint32_t voB = (uint32_t)(dr * rpB) + (BT ? dc : dc ^ (dr >> 2)) * 16;
-  int64_t offA[2], offB[2], cutA[2], cutB[2];     // this wavefront's two pieces of each operand; cut: see half_tail
+  int64_t offA[PA], offB[PB], lA[PA], lB[PB], cutA[PA], cutB[PB];     // this wavefront's pieces; cut: see half_tail
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int q = wave * 2 + j;
-    const int pa = AT ? q / (TK / 16) : q / (TM / 16), ra = AT ? q % (TK / 16) : q % (TM / 16);
-    const int pb = BT ? q / (TK / 16) : q / (TM / 16), rb = BT ? q % (TK / 16) : q % (TM / 16);
+  for (int j = 0; j < PA; ++j) {
+    const int q = wave * PA + j, pa = AT ? q / (TK / 16) : q / (TM / 16), ra = AT ? q % (TK / 16) : q % (TM / 16);
     offA[j] = pa * psA + ra * 16 * rpA;
-    offB[j] = pb * psB + rb * 16 * rpB;
+    lA[j] = offA[j] + voA;
     cutA[j] = AT ? (ra >= 2 ? 32 * rpA : 0) : (pa >= 1 ? psA : 0);
+  }
+#pragma unroll
+  for (int j = 0; j < PB; ++j) {
+    const int q = wave * PB + j, pb = BT ? q / (TK / 16) : q / (TN / 16), rb = BT ? q % (TK / 16) : q % (TN / 16);
+    offB[j] = pb * psB + rb * 16 * rpB;
+    lB[j] = offB[j] + voB;
     cutB[j] = BT ? (rb >= 2 ? 32 * rpB : 0) : (pb >= 1 ? psB : 0);
   }
   const int64_t baseA = (int64_t)e * p.strideA * 2 + (AT ? (int64_t)(tm * (TM / 32)) * psA : (int64_t)tm * TM * rpA);
-  const int64_t baseB = (int64_t)e * p.strideB * 2 + (BT ? (int64_t)(tn * (TM / 32)) * psB : (int64_t)tn * TM * rpB);
+  const int64_t baseB = (int64_t)e * p.strideB * 2 + (BT ? (int64_t)(tn * (TN / 32)) * psB : (int64_t)tn * TN * rpB);
   const int64_t advA = AT ? TK * rpA : KP * psA, advB = BT ? TK * rpB : KP * psB;
   const char *curA = (const char *)p.A[0] + baseA, *curB = (const char *)p.B[0] + baseB;
   int is_kt = 0;
@@ -126,15 +148,17 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   // SIMD to itself is quicker without the longer chain of scalar instructions (the step of one (1024,3072) weight: 1.4 % slower with it).
   // (`lane_at`: at + off)
   auto dma = [&](const char *g, int64_t at, int64_t lane_at, uint32_t off, uint32_t lds_base) {
-    if (WB == 1 && kRing == 4) dma16(g + lane_at, lds_base);
+    if (WM == 1 && kRing == 4) dma16(g + lane_at, lds_base);
     else                       dma16(g + at, off, lds_base);
   };
-  const int64_t lA[2] = {offA[0] + voA, offA[1] + voA}, lB[2] = {offB[0] + voB, offB[1] + voB};
-  auto piece = [&](int i, unsigned char *st) {          // DMA instruction i of a stage: two of A, two of B
+  auto piece = [&](int i, unsigned char *st) {          // DMA instruction i of a stage: PA of A, PB of B
     const bool cut = half_tail && is_kt + 1 == nk;      // (the missing panel's pieces fetch the one that is there)
-    const int j = i & 1;
-    if (i < 2) dma(curA - (cut ? cutA[j] : 0), offA[j], lA[j], voA, lds_addr(st + (wave * 2 + j) * 1024));
-    else       dma(curB - (cut ? cutB[j] : 0), offB[j], lB[j], voB, lds_addr(st + kHalf + (wave * 2 + j) * 1024));
+    if (i < PA) {
+      dma(curA - (cut ? cutA[i] : 0), offA[i], lA[i], voA, lds_addr(st + (wave * PA + i) * 1024));
+    } else {
+      const int j = i - PA;
+      dma(curB - (cut ? cutB[j] : 0), offB[j], lB[j], voB, lds_addr(st + kHalf + (wave * PB + j) * 1024));
+    }
   };
   auto advance = [&]() { curA += advA; curB += advB; ++is_kt; };
   auto issue = [&](unsigned char *st) {
@@ -147,12 +171,13 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   const int l31 = lane & 31, hh = lane >> 5, g16 = lane >> 4, s16 = lane & 15;
   const int tr_lane = (8 * (g16 >> 1) + (s16 >> 2)) * 64 + 32 * (g16 & 1) + 8 * (s16 & 3);
   // (rows_k: k rows of a block in the stage)
-  auto frag = [&](auto tr, const unsigned char *half, int blk, int kk, int rows_k) -> bf16x8 {
+  // (rows: the operand's rows per panel)
+  auto frag = [&](auto tr, const unsigned char *half, int blk, int kk, int rows_k, int rows) -> bf16x8 {
     if constexpr (decltype(tr)::value) {
       const unsigned char *q = half + blk * (rows_k * 64) + kk * 16 * 64 + tr_lane;
       return anc_lds_tr_frag(q, q + 4 * 64);
     } else {
-      return *(const bf16x8 *)(half + (kk >> 1) * (TM * 64) + (blk * 32 + l31) * 64 + ((((kk & 1) * 2 + hh) ^ ((l31 >> 2) & 3)) * 16));
+      return *(const bf16x8 *)(half + (kk >> 1) * (rows * 64) + (blk * 32 + l31) * 64 + ((((kk & 1) * 2 + hh) ^ ((l31 >> 2) & 3)) * 16));
     }
   };
   using TrA = std::bool_constant<AT>;
@@ -177,16 +202,18 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   // whole lines.
   constexpr int RUN = (PLAINV || VAR == VAR_UPDATE) ? 4 : 8, NR = 16 / RUN, LPR = 32 / RUN, RS = 64 / LPR;
   const int lrow = lane / LPR, c0 = (lane % LPR) * RUN;
-  const int gi_w = tm * TM + wm * (32 * WB), gj_w = tn * TM + wn * (32 * WB);
+  const int gi_w = tm * TM + wm * (32 * WM), gj_w = tn * TN + wn * (32 * WN);
+  // symmetric output: this wavefront's block lies above the 64x64 blocks of the diagonal (nobody needs it), or below
+  const bool idle = EPI != EPI_BX && WM > 1 && (gi_w >> 6) < (gj_w >> 6), mirror = EPI != EPI_BX && (gi_w >> 6) > (gj_w >> 6);
   // run 0 of block b in a matrix of M rows in panel layout (run r: RS * 32 r further)
-  auto pan_of = [&](int b) { return ((int64_t)((gj_w + (b % WB) * 32) / 32) * M + gi_w + (b / WB) * 32 + lrow) * 32 + c0; };
-  constexpr int NB = WB * WB;
+  auto pan_of = [&](int b) { return ((int64_t)((gj_w + (b % WN) * 32) / 32) * M + gi_w + (b / WN) * 32 + lrow) * 32 + c0; };
+  constexpr int NB = WM * WN;
   uint32_t pre_h[NB][8], pre_l[NB][8];                  // 16 bf16, or (pre_l, 8-bit low halves) 16 bytes in the first 4
-  float drow[WB][NR];
+  float drow[WM][NR];
   if constexpr (EPI == EPI_BX && !PLAINV) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int64_t xo = mn + (p.x_panel ? pan_of(b) : (int64_t)(gi_w + (b / WB) * 32 + lrow) * N + gj_w + (b % WB) * 32 + c0);
+      const int64_t xo = mn + (p.x_panel ? pan_of(b) : (int64_t)(gi_w + (b / WN) * 32 + lrow) * N + gj_w + (b % WN) * 32 + c0);
       const int64_t xr = p.x_panel ? RS * 32 : (int64_t)RS * N;
 #pragma unroll
       for (int r = 0; r < NR; ++r) ld_run<RUN * 2>(p.Xh + xo + r * xr, &pre_h[b][r * (RUN / 2)]);
@@ -200,21 +227,21 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
       }
     }
 #pragma unroll
-    for (int bi = 0; bi < WB; ++bi)
+    for (int bi = 0; bi < WM; ++bi)
 #pragma unroll
       for (int r = 0; r < NR; ++r) drow[bi][r] = p.dB[mv + gi_w + bi * 32 + lrow + RS * r];
   }
   // (the master's block, or what the plain product adds to, too where registers allow: one block per wavefront)
   const bool plain_add = PLAINV && p.plain_sum && p.A32 != nullptr;
   anc_f32x4 wpre[4];
-  if constexpr (VAR == VAR_UPDATE && WB == 1) {
+  if constexpr (VAR == VAR_UPDATE && NB == 1) {
     const anc_muon_desc_t &d = p.upd[e];
     const bool wtr = d.transpose != 0;
     const int64_t we = (int64_t)((wtr ? gj_w : gi_w) + lrow) * d.N + (wtr ? gi_w : gj_w) + c0;
 #pragma unroll
     for (int r = 0; r < 4; ++r) wpre[r] = *(const anc_f32x4 *)((const float *)d.p32 + we + (int64_t)r * RS * d.N);
   }
-  if constexpr (PLAINV && WB == 1) {
+  if constexpr (PLAINV && NB == 1) {
     if (plain_add) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -223,7 +250,7 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
   }
 
   // A at the output position, with at most one workgroup per CU
-  constexpr bool kEarlyA = EPI == EPI_BMAT && WB == 1 && kRing == 4;
+  constexpr bool kEarlyA = EPI == EPI_BMAT && NB == 1 && kRing == 4;
   anc_f32x4 a32[4];
   float pre_di[NR], pre_dj[RUN];
   if constexpr (kEarlyA) {
@@ -244,31 +271,31 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
     }
   }
 
-  f32x16 acc[WB][WB];
+  f32x16 acc[WM][WN];
 #pragma unroll
-  for (int bi = 0; bi < WB; ++bi)
+  for (int bi = 0; bi < WM; ++bi)
 #pragma unroll
-    for (int bj = 0; bj < WB; ++bj)
+    for (int bj = 0; bj < WN; ++bj)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[bi][bj][r] = 0.0f;
 
-  auto mma = [&](const bf16x8 (&a)[WB], const bf16x8 (&b)[WB]) {
+  auto mma = [&](const bf16x8 (&a)[WM], const bf16x8 (&b)[WN]) {
 #pragma unroll
-    for (int bi = 0; bi < WB; ++bi)
+    for (int bi = 0; bi < WM; ++bi)
 #pragma unroll
-      for (int bj = 0; bj < WB; ++bj)      // operands exchanged: a lane ends with runs of 4 columns of one row
+      for (int bj = 0; bj < WN; ++bj)      // operands exchanged: a lane ends with runs of 4 columns of one row
         acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bj], a[bi], acc[bi][bj], 0, 0, 0);
   };
 
-  auto frags = [&](const unsigned char *st, int kk, bf16x8 (&fa)[WB], bf16x8 (&fb)[WB]) {
+  auto frags = [&](const unsigned char *st, int kk, bf16x8 (&fa)[WM], bf16x8 (&fb)[WN]) {
 #pragma unroll
-    for (int i = 0; i < WB; ++i) fa[i] = frag(TrA{}, st, wm * WB + i, kk, TK);
+    for (int i = 0; i < WM; ++i) fa[i] = frag(TrA{}, st, wm * WM + i, kk, TK, TM);
 #pragma unroll
-    for (int i = 0; i < WB; ++i) fb[i] = frag(TrB{}, st + kHalf, wn * WB + i, kk, TK);
+    for (int i = 0; i < WN; ++i) fb[i] = frag(TrB{}, st + kHalf, wn * WN + i, kk, TK, TN);
   };
   // ---- K loop, one term. Step k lives in stage k % kRing.
   if (PLAINV || nterms == 1) {
-    if constexpr (WB == 1) {
+    if constexpr (WM == 1) {
       // At the top of step k a wavefront waits for its own DMA of the step (the younger ones stay in flight), the
       // workgroup meets, and the DMA of step k + kRing - 1 goes out into the stage everybody has just left.
 #pragma unroll
@@ -283,7 +310,7 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 #pragma unroll
         for (int kk = 0; kk < TK / 16; ++kk) {
           if (PLAINV && kk >= 2 && cut) break;
-          bf16x8 a[WB], b[WB];
+          bf16x8 a[WM], b[WN];
           frags(st, kk, a, b);
           mma(a, b);
         }
@@ -301,107 +328,173 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
       // longer way to the first product costs 0.7 us and gives nothing.)
       constexpr int KK = TK / 16, U = kRing;
       static_assert(kRing == 4, "rounds of four");
-      bf16x8 a[2][KK][WB], b[2][KK][WB];
+      bf16x8 a[2][KK][WM], b[2][KK][WN];
 #pragma unroll
       for (int s0 = 0; s0 < kRing; ++s0)
         if (s0 < nk) issue(lds + s0 * kStageBytes);
       if (kRing <= nk) wait_vm<(kRing - 1) * kIps>(); else wait_vm<0>();
       lds_barrier();
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk) frags(lds, kk, a[0][kk], b[0][kk]);
-      auto body = [&](auto steady, int step, auto s0v) {
-        constexpr bool kSteady = decltype(steady)::value;
-        constexpr int s0 = decltype(s0v)::value % kRing, x = decltype(s0v)::value % 2;
-        const bool more = kSteady || step + 1 < nk, refill = kSteady || step + kRing < nk;
-        if (kSteady || step + kRing <= nk) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
-        lds_barrier();
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
-          mma(a[x][kk], b[x][kk]);
-          __builtin_amdgcn_sched_barrier(0);
-          if (refill) {
-#pragma unroll
-            for (int i = kk * kIps / KK; i < (kk + 1) * kIps / KK; ++i) piece(i, lds + s0 * kStageBytes);
-          }
-          if (more) frags(lds + (s0 + 1) % kRing * kStageBytes, kk, a[1 - x][kk], b[1 - x][kk]);
-          __builtin_amdgcn_sched_barrier(0);
+      if (idle) {                        // (its share of the DMA, and the meetings)
+        for (int step = 0, at = 0; step < nk; ++step) {
+          if (step + kRing <= nk) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
+          lds_barrier();
+          if (step + kRing < nk) issue(lds + at);
+          at = at + kStageBytes == kRing * kStageBytes ? 0 : at + kStageBytes;
         }
-        if (refill) advance();
-      };
-      auto round = [&](auto steady, int step) {
-        auto one = [&](auto s0) {
-          if (decltype(steady)::value || step + decltype(s0)::value < nk) body(steady, step + decltype(s0)::value, s0);
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) frags(lds, kk, a[0][kk], b[0][kk]);
+        auto body = [&](auto steady, int step, auto s0v) {
+          constexpr bool kSteady = decltype(steady)::value;
+          constexpr int s0 = decltype(s0v)::value % kRing, x = decltype(s0v)::value % 2;
+          const bool more = kSteady || step + 1 < nk, refill = kSteady || step + kRing < nk;
+          if (kSteady || step + kRing <= nk) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
+          lds_barrier();
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) {
+            mma(a[x][kk], b[x][kk]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (refill) {
+#pragma unroll
+              for (int i = kk * kIps / KK; i < (kk + 1) * kIps / KK; ++i) piece(i, lds + s0 * kStageBytes);
+            }
+            if (more) frags(lds + (s0 + 1) % kRing * kStageBytes, kk, a[1 - x][kk], b[1 - x][kk]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (refill) advance();
         };
-        one(std::integral_constant<int, 0>{});
-        one(std::integral_constant<int, 1>{});
-        one(std::integral_constant<int, 2>{});
-        one(std::integral_constant<int, 3>{});
-      };
-      int step = 0;
-      for (; step + U - 1 + kRing < nk; step += U) round(std::true_type{}, step);
-      for (; step < nk; step += U) round(std::false_type{}, step);
+        auto round = [&](auto steady, int step) {
+          auto one = [&](auto s0) {
+            if (decltype(steady)::value || step + decltype(s0)::value < nk) body(steady, step + decltype(s0)::value, s0);
+          };
+          one(std::integral_constant<int, 0>{});
+          one(std::integral_constant<int, 1>{});
+          one(std::integral_constant<int, 2>{});
+          one(std::integral_constant<int, 3>{});
+        };
+        int step = 0;
+        for (; step + U - 1 + kRing < nk; step += U) round(std::true_type{}, step);
+        for (; step < nk; step += U) round(std::false_type{}, step);
+      }
     }
   } else {
     // ---- several terms: a step is one panel of 32 k of both halves of both operands, high stage then low stage.
-    constexpr int kPan = TM * 64, kPair = 4 * kPan, kPairs = kRing * kStageBytes / kPair;   // 4, 3 (64) or 2 (128) steps in the ring
-    int64_t oA[WB], oB[WB], vA[WB], vB[WB];
+    constexpr int kPanA = TM * 64, kPanB = TN * 64, kLow = kPanA + kPanB, kPair = 2 * kLow, kPairs = kRing * kStageBytes / kPair;
+    int64_t oA[WM], oB[WN], vA[WM], vB[WN];
 #pragma unroll
-    for (int j = 0; j < WB; ++j) {
-      const int q = wave * WB + j;
+    for (int j = 0; j < WM; ++j) {
+      const int q = wave * WM + j;
       oA[j] = (AT ? (q >> 1) * psA + (q & 1) * 16 * rpA : q * 16 * rpA);
-      oB[j] = (BT ? (q >> 1) * psB + (q & 1) * 16 * rpB : q * 16 * rpB);
       vA[j] = oA[j] + voA;
+    }
+#pragma unroll
+    for (int j = 0; j < WN; ++j) {
+      const int q = wave * WN + j;
+      oB[j] = (BT ? (q >> 1) * psB + (q & 1) * 16 * rpB : q * 16 * rpB);
       vB[j] = oB[j] + voB;
     }
     const char *pAl = (const char *)p.A[1] + baseA, *pBl = (const char *)p.B[1] + baseB;
     const int64_t adA = AT ? 32 * rpA : psA, adB = BT ? 32 * rpB : psB;
     auto terms = [&](auto nt) {
-      constexpr int NT = decltype(nt)::value, kIpp = NT == 3 ? 4 * WB : 3 * WB;   // DMA instructions per wavefront and step
+      constexpr int NT = decltype(nt)::value, kIpp = NT == 3 ? 2 * (WM + WN) : WM + 2 * WN;   // DMA instructions per wavefront and step
       auto issue_pair = [&](unsigned char *st) {
 #pragma unroll
-        for (int j = 0; j < WB; ++j) {
-          const int at = (wave * WB + j) * 1024;
-          dma(curA, oA[j], vA[j], voA, lds_addr(st + at));
-          dma(curB, oB[j], vB[j], voB, lds_addr(st + kPan + at));
-          if (NT == 3) dma(pAl, oA[j], vA[j], voA, lds_addr(st + 2 * kPan + at));
-          dma(pBl, oB[j], vB[j], voB, lds_addr(st + 3 * kPan + at));
+        for (int j = 0; j < WM; ++j) {
+          dma(curA, oA[j], vA[j], voA, lds_addr(st + (wave * WM + j) * 1024));
+          if (NT == 3) dma(pAl, oA[j], vA[j], voA, lds_addr(st + kLow + (wave * WM + j) * 1024));
+        }
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+          dma(curB, oB[j], vB[j], voB, lds_addr(st + kPanA + (wave * WN + j) * 1024));
+          dma(pBl, oB[j], vB[j], voB, lds_addr(st + kLow + kPanA + (wave * WN + j) * 1024));
         }
         curA += adA; curB += adB; pAl += adA; pBl += adB;
       };
       const int np = K / 32;
+      // The first fragments of step k are in registers when it begins, the others are read under its matrix
+      // instructions. Before its last product a wavefront waits for its own DMA of step k + 1 and the workgroup meets:
+      // everybody has read stage k, which takes the DMA of step k + kPairs, and the next step's first fragments are read
+      // under that product. B's fragments of k 0..15 and 16..31 change places from step to step.
 #pragma unroll
-      for (int s0 = 0; s0 < kPairs - 1; ++s0)
+      for (int s0 = 0; s0 < kPairs; ++s0)
         if (s0 < np) issue_pair(lds + s0 * kPair);
-      for (int step = 0; step < np; step += kPairs) {
-#pragma unroll
-        for (int s0 = 0; s0 < kPairs; ++s0) {
-          if (step + s0 >= np) break;
-          if (step + s0 + kPairs - 1 <= np) wait_vm<(kPairs - 2) * kIpp>(); else wait_vm<0>();
+      if (kPairs <= np) wait_vm<(kPairs - 1) * kIpp>(); else wait_vm<0>();
+      lds_barrier();
+      if (idle) {
+        for (int step = 0, at = 0; step < np; ++step) {
+          if (step + kPairs <= np) wait_vm<(kPairs - 2) * kIpp>(); else wait_vm<0>();
           lds_barrier();
-          if (step + s0 + kPairs - 1 < np) issue_pair(lds + ((s0 + kPairs - 1) % kPairs) * kPair);
-          const unsigned char *st = lds + s0 * kPair;
-          bf16x8 ah[2][WB], bh[2][WB], al[WB], bl[WB];
-#pragma unroll
-          for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-            for (int i = 0; i < WB; ++i) ah[kk][i] = frag(TrA{}, st, wm * WB + i, kk, 32);
-#pragma unroll
-            for (int i = 0; i < WB; ++i) bh[kk][i] = frag(TrB{}, st + kPan, wn * WB + i, kk, 32);
-            mma(ah[kk], bh[kk]);
-          }
-#pragma unroll
-          for (int kk = 1; kk >= 0; --kk) {
-#pragma unroll
-            for (int i = 0; i < WB; ++i) bl[i] = frag(TrB{}, st + 3 * kPan, wn * WB + i, kk, 32);
-            mma(ah[kk], bl);
-            if (NT == 3) {
-#pragma unroll
-              for (int i = 0; i < WB; ++i) al[i] = frag(TrA{}, st + 2 * kPan, wm * WB + i, kk, 32);
-              mma(al, bh[kk]);
-            }
-          }
+          if (step + kPairs < np) issue_pair(lds + at);
+          at = at + kPair == kPairs * kPair ? 0 : at + kPair;
         }
+        return;
       }
+      bf16x8 ah[2][WM], bh[2][WN], al[2][WM], bl[2][WN];
+      auto rd_a = [&](const unsigned char *half, int kk, bf16x8 (&f)[WM]) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i) f[i] = frag(TrA{}, half, wm * WM + i, kk, 32, TM);
+      };
+      auto rd_b = [&](const unsigned char *half, int kk, bf16x8 (&f)[WN]) {
+#pragma unroll
+        for (int i = 0; i < WN; ++i) f[i] = frag(TrB{}, half, wn * WN + i, kk, 32, TN);
+      };
+      auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
+      rd_a(lds, 0, ah[0]);
+      rd_b(lds + kPanA, 0, bh[0]);
+      auto body = [&](auto steady, int step, auto s0v) {
+        constexpr int s0 = decltype(s0v)::value % kPairs, x = decltype(s0v)::value % 2, y = 1 - x;
+        const unsigned char *st = lds + s0 * kPair, *nx = lds + (s0 + 1) % kPairs * kPair;
+        const bool more = decltype(steady)::value || step + 1 < np, refill = decltype(steady)::value || step + kPairs < np;
+        rd_a(st, 1, ah[1]);
+        rd_b(st + kPanA, 1, bh[y]);
+        fence();
+        mma(ah[0], bh[x]);                                    // hh 0..15
+        fence();
+        rd_b(st + kLow + kPanA, 1, bl[1]);
+        if (NT == 3) rd_a(st + kLow, 1, al[1]);
+        fence();
+        mma(ah[1], bh[y]);                                    // hh 16..31
+        fence();
+        rd_b(st + kLow + kPanA, 0, bl[0]);
+        if (NT == 3) rd_a(st + kLow, 0, al[0]);
+        fence();
+        mma(ah[1], bl[1]);                                    // hl 16..31
+        if (NT == 3) {
+          mma(al[1], bh[y]);                                  // lh 16..31
+          mma(ah[0], bl[0]);                                  // hl 0..15
+        }
+        fence();
+        if (decltype(steady)::value || step + kPairs <= np) wait_vm<(kPairs - 2) * kIpp>(); else wait_vm<0>();
+        lds_barrier();
+        if (refill) issue_pair(lds + s0 * kPair);
+        if (NT == 3 && more) rd_a(nx, 0, ah[0]);
+        if (more) rd_b(nx + kPanA, 0, bh[y]);
+        fence();
+        if (NT == 3) mma(al[0], bh[x]);                       // lh 0..15
+        else         mma(ah[0], bl[0]);                       // (of two terms: hl 0..15)
+        fence();
+        if (NT != 3 && more) rd_a(nx, 0, ah[0]);
+      };
+      constexpr int U = kPairs % 2 == 0 ? kPairs : 2 * kPairs;
+      static_assert(U == 2 || U == 4 || U == 6, "rounds");
+      auto round = [&](auto steady, int step) {
+        auto one = [&](auto s0) {
+          if (decltype(steady)::value || step + decltype(s0)::value < np) body(steady, step + decltype(s0)::value, s0);
+        };
+        one(std::integral_constant<int, 0>{});
+        one(std::integral_constant<int, 1>{});
+        if constexpr (U > 2) {
+          one(std::integral_constant<int, 2>{});
+          one(std::integral_constant<int, 3>{});
+        }
+        if constexpr (U > 4) {
+          one(std::integral_constant<int, 4>{});
+          one(std::integral_constant<int, 5>{});
+        }
+      };
+      int step = 0;
+      for (; step + U - 1 + kPairs < np; step += U) round(std::true_type{}, step);
+      for (; step < np; step += U) round(std::false_type{}, step);
     };
     if (EPI == EPI_BX && nterms == 2) terms(std::integral_constant<int, 2>{});
     else terms(std::integral_constant<int, 3>{});
@@ -410,6 +503,7 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 
   // ---- epilogue
   if (VAR == VAR_UPDATE && pm.ctl != nullptr && pm.ctl->skip != 0u) return;   // skipped step
+  if (idle) return;
   float v[16];
   auto put_rows = [&]() {
 #pragma unroll
@@ -443,15 +537,15 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
     }
   };
 #pragma unroll
-  for (int bi = 0; bi < WB; ++bi) {
+  for (int bi = 0; bi < WM; ++bi) {
 #pragma unroll
-    for (int bj = 0; bj < WB; ++bj) {
+    for (int bj = 0; bj < WN; ++bj) {
       const int gi0 = gi_w + bi * 32, gj0 = gj_w + bj * 32;
       const int gi = gi0 + lrow, gj = gj0 + c0;
-      const int64_t pan = pan_of(bi * WB + bj), pst = RS * 32;
+      const int64_t pan = pan_of(bi * WN + bj), pst = RS * 32;
       // four consecutive columns from column gj + 4 i % RUN of row gi + RS (4 i / RUN), in a matrix with `pitch` columns
       auto quad = [&](int i, int64_t pitch) { return (int64_t)(gi + RS * (4 * i / RUN)) * pitch + gj + 4 * i % RUN; };
-      if constexpr (PLAINV && WB > 1) {
+      if constexpr (PLAINV && NB > 1) {
         if (plain_add) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) wpre[i] = *(const anc_f32x4 *)(p.A32 + mn + quad(i, N));
@@ -537,7 +631,7 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
         }
         uint16_t *oh = EPI == EPI_GRAM ? p.Fh : p.Bh, *ol = EPI == EPI_GRAM ? p.Fl : p.Bl;
         put_bf16(oh + mm + pan, write_lo ? ol + mm + pan : nullptr, pst);
-        if (tm / p.blk_r != tn / p.blk_r) {  // mirror image: rows gj0 .., 32-column panel gi0/32
+        if (mirror) {                        // mirror image: rows gj0 .., 32-column panel gi0/32
           put_rows();
           get_cols();
           const int64_t pt = ((int64_t)(gi0 / 32) * M + gj0 + lrow) * 32 + c0;
@@ -569,14 +663,14 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
       } else {
         // y = (a + dB) x + B X. Only the first iteration carries the input's scale.
         float x[16];
-        unpack(pre_h[bi * WB + bj], x);
+        unpack(pre_h[bi * WN + bj], x);
         if (in8) {
 #pragma unroll
           for (int k = 0; k < 16; ++k)
-            x[k] = anc_low8_decode(__float_as_uint(x[k]), (int)(pre_l[bi * WB + bj][k >> 2] << (24 - 8 * (k & 3))) >> 24);
+            x[k] = anc_low8_decode(__float_as_uint(x[k]), (int)(pre_l[bi * WN + bj][k >> 2] << (24 - 8 * (k & 3))) >> 24);
         } else if (!p.lo_zero) {
           float xl[16];
-          unpack(pre_l[bi * WB + bj], xl);
+          unpack(pre_l[bi * WN + bj], xl);
 #pragma unroll
           for (int k = 0; k < 16; ++k) x[k] = x[k] + xl[k];
         }
@@ -599,7 +693,7 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
           const int64_t we = (int64_t)(wr0 + lrow) * d.N + wc0 + c0, wst = (int64_t)RS * d.N;
           anc_f32x4 pv[4];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) pv[r] = WB == 1 ? wpre[r] : *(const anc_f32x4 *)(W32 + we + r * wst);
+          for (int r = 0; r < 4; ++r) pv[r] = NB == 1 ? wpre[r] : *(const anc_f32x4 *)(W32 + we + r * wst);
           if (wtr) {
             put_rows();
             get_cols();
@@ -666,10 +760,10 @@ __global__ void __launch_bounds__(256, kRing == 3 ? 3 : 2) k_ns_gemm_tile(NsGemm
 }
 
 template <int EPI, bool AT, int VAR>
-void launch_tile(bool small, unsigned grid, hipStream_t s, const NsGemmMulti &pm) {
-  if (!small)           hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
-  else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 3, false>), dim3(grid), dim3(256), 0, s, pm);
-  else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) {
+  if (tile == 128)      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 2, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+  else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, AT, VAR, 3, false>), dim3(grid), dim3(256), 0, s, pm);
+  else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
   else {
     NsGemmArgs<1> one;
     one.n = 1;
@@ -679,17 +773,17 @@ void launch_tile(bool small, unsigned grid, hipStream_t s, const NsGemmMulti &pm
     one.sr = pm.sr;
     one.seed_base = pm.seed_base;
     one.ctl = pm.ctl;
-    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, AT, VAR, 4, true>), dim3(grid), dim3(256), 0, s, one);
+    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, AT, VAR, 4, true>), dim3(grid), dim3(256), 0, s, one);
   }
 }
 
 }  // namespace
 
-// n <= kMaxGroups problems of the same product in one launch on tiles of 64 (small) or 128. EPI_BX: `by_rows` as for the
-// 256-wide tiles; `plain`: the bare product, A transposed (by_rows) or not.
-int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool small, bool by_rows,
+// n <= kMaxGroups problems of the same product in one launch on tiles of 64, 128 or 128x64 (kTile128x64). EPI_BX:
+// `by_rows` as for the 256-wide tiles; `plain`: the bare product, A transposed (by_rows) or not.
+int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int tile, bool by_rows,
                            const NsUpdate *upd, bool plain) {
-  const int T = small ? 64 : 128;
+  const int TM = tile == 64 ? 64 : 128, TN = tile == 128 ? 128 : 64;
   NsGemmMulti pm{};
   pm.n = n;
   int64_t grid = 0;
@@ -698,20 +792,15 @@ int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, 
     g = ps[k];
     ANC_REQUIRE(g.M % 128 == 0 && g.N % 128 == 0 && g.K % (plain ? 32 : 128) == 0 && g.K > 0,
                 "anc_ns_gemm_tile: dims must be multiples of 128");
-    g.tiles_m = g.M / T;
-    g.tiles_n = (epi == EPI_BX ? g.N : g.M) / T;
+    g.tiles_m = g.M / TM;
+    g.tiles_n = (epi == EPI_BX ? g.N : g.M) / TN;
     g.lower = epi == EPI_BX ? 0 : 1;
-    int64_t per = (int64_t)g.tiles_m * g.tiles_n;
-    if (g.lower) {
-      ANC_REQUIRE((g.diag == 128 || g.diag == 256) && g.M % g.diag == 0, "anc_ns_gemm_tile: bad diagonal blocks");
-      g.blk_r = g.blk_c = g.diag / T;
-      const int64_t q = g.tiles_m / g.blk_r;
-      per = q * (q + 1) / 2 * g.blk_r * g.blk_c;
-    } else {
-      // walked in blocks of 256 x 256 (see launch_bx of the 256-wide kernel: what an XCD fetches)
-      g.blk_r = g.M % 256 == 0 ? 256 / T : 128 / T;
-      g.blk_c = g.N % 256 == 0 ? 256 / T : 128 / T;
-    }
+    // walked in blocks of 256 x 256 (see launch_bx of the 256-wide kernel: what an XCD fetches)
+    const int cols = epi == EPI_BX ? g.N : g.M;
+    g.blk_r = (g.M % 256 == 0 ? 256 : 128) / TM;
+    g.blk_c = (cols % 256 == 0 ? 256 : 128) / TN;
+    const int64_t per = !g.lower ? (int64_t)g.tiles_m * g.tiles_n
+                      : TM == TN ? anc_sym_tiles<64, 64>(g.tiles_m) : anc_sym_tiles<128, 64>(g.tiles_m);
     ANC_REQUIRE(per > 0 && Es[k] * per < (1ll << 30), "anc_ns_gemm_tile: grid out of range");
     pm.tiles[k] = (int)(Es[k] * per);
     grid += pm.tiles[k];
@@ -719,22 +808,22 @@ int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, 
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_tile: grid out of range");
   const unsigned gr = (unsigned)grid;
   if (plain) {
-    if (by_rows) launch_tile<EPI_BX, true, VAR_PLAIN>(small, gr, s, pm);
-    else         launch_tile<EPI_BX, false, VAR_PLAIN>(small, gr, s, pm);
+    if (by_rows) launch_tile<EPI_BX, true, VAR_PLAIN>(tile, gr, s, pm);
+    else         launch_tile<EPI_BX, false, VAR_PLAIN>(tile, gr, s, pm);
   } else if (epi == EPI_GRAM) {
-    launch_tile<EPI_GRAM, false, VAR_NONE>(small, gr, s, pm);
+    launch_tile<EPI_GRAM, false, VAR_NONE>(tile, gr, s, pm);
   } else if (epi == EPI_BMAT) {
-    launch_tile<EPI_BMAT, false, VAR_NONE>(small, gr, s, pm);
+    launch_tile<EPI_BMAT, false, VAR_NONE>(tile, gr, s, pm);
   } else if (upd != nullptr) {
     for (int k = 0; k < ANC_MUON_MAX_SCALES; ++k) pm.lr[k] = upd->lr[k];
     pm.sr = upd->sr;
     pm.seed_base = upd->seed_base;
     pm.ctl = upd->ctl;
-    if (by_rows) launch_tile<EPI_BX, true, VAR_UPDATE>(small, gr, s, pm);
-    else         launch_tile<EPI_BX, false, VAR_UPDATE>(small, gr, s, pm);
+    if (by_rows) launch_tile<EPI_BX, true, VAR_UPDATE>(tile, gr, s, pm);
+    else         launch_tile<EPI_BX, false, VAR_UPDATE>(tile, gr, s, pm);
   } else {
-    if (by_rows) launch_tile<EPI_BX, true, VAR_NONE>(small, gr, s, pm);
-    else         launch_tile<EPI_BX, false, VAR_NONE>(small, gr, s, pm);
+    if (by_rows) launch_tile<EPI_BX, true, VAR_NONE>(tile, gr, s, pm);
+    else         launch_tile<EPI_BX, false, VAR_NONE>(tile, gr, s, pm);
   }
   ANC_LAUNCH_CHECK();
   return ANC_OK;

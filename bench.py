@@ -250,7 +250,7 @@ def ns_config(steps):
             e1.sync()
             total_ms += e0.elapsed_ms(e1) / k
             ex, de = ns_flops(E, M, N, 5, mode)
-            ex_t += ex
+            ex_t += ex if mode == "fp32" else multiplied(ex, ns_flops(E, M, N, 5, "bf16_tile128")[0])
             de_t += de
             X.free()
         res[mode] = {"ms": round(total_ms, 3), "executed_tflop": round(ex_t / 1e12, 3),
@@ -310,16 +310,25 @@ def adamw_flat_config(steps, warmup):
 GEMM_KINDS = ("ns_gemm_gram", "ns_gemm_bmat", "ns_gemm_bx", "ns_gemm_bx_update")
 
 
+def multiplied(in256, in128):
+    """FLOPs really multiplied, from the counts in blocks of 256 and of 128 (dims multiples of 256): the kernels take the
+    64x64 blocks on and below the diagonal, and M^2 + 64 M lies half as far beyond M^2 + 128 M as that beyond
+    M^2 + 256 M."""
+    return in128 - (in256 - in128) / 2
+
+
 def chain_work(opt, schedule):
     """(executed FLOPs, dense FLOPs, matrices that took a conditioning gate) of the optimizer's last
     step, from the plan of the mode it ran in and the gate decisions left in the workspaces."""
-    from ancora_cutile_amd.muon_ns import ns_flops, ns_hard_info
+    from ancora_cutile_amd.muon_ns import effective_mode, ns_flops, ns_hard_info
     executed = dense = 0.0
     hard = 0
     for b in opt.muon.engine.batches:
         ex, de = ns_flops(b.E, b.M, b.Nn, 5, "bf16", schedule=schedule)
         nh, extra = ns_hard_info(b.ws.buf.ptr, b.E, b.M, b.Nn, 5, "bf16", schedule=schedule)
-        executed += ex + extra
+        small = "bf16_late3_tile128" if effective_mode("bf16", schedule) == "bf16_late3" else "bf16_tile128"
+        ex128, _ = ns_flops(b.E, b.M, b.Nn, 5, small)
+        executed += multiplied(ex + extra, ex128 + ns_hard_info(b.ws.buf.ptr, b.E, b.M, b.Nn, 5, small)[1])
         dense += de
         hard += nh
     return executed, dense, hard
@@ -711,12 +720,12 @@ def main():
     for b in opt.muon.engine.batches:
         ex, de = ns_flops(b.E, b.M, b.Nn, 5, "bf16")
         nh, extra = ns_hard_info(b.ws.buf.ptr, b.E, b.M, b.Nn, 5, "bf16")
-        executed += ex + extra
         dense += de
         hard += nh
-        ex128, _ = ns_flops(b.E, b.M, b.Nn, 5, "bf16_tile128")    # the same chain counted in 128x128 tiles
+        ex128, _ = ns_flops(b.E, b.M, b.Nn, 5, "bf16_tile128")    # the same chain counted in 128x128 blocks
         nh128, extra128 = ns_hard_info(b.ws.buf.ptr, b.E, b.M, b.Nn, 5, "bf16_tile128")
         lower128 += ex128 + extra128
+        executed += multiplied(ex + extra, ex128 + extra128)
         last_bx += ns_product_flops(b.E, b.M, b.Nn, 4, 2, 5, "bf16")
     # What the board sustains: the shader clock while the step runs (the nominal 2.4 GHz is not
     # held under the power limit) and the matrix pipe's register-only rate on zero / random operands
@@ -806,7 +815,7 @@ def main():
                                                          if sclk and info["clock_khz"] else None),
                      "executed_tflop_per_step": round(executed / 1e12, 3),
                      "executed_counts": "what the kernels multiply: residual and gated terms, and of the symmetric "
-                                        "products the 256x256 tiles on or below the diagonal, each in full "
+                                        "products the 64x64 blocks on or below the diagonal, each in full "
                                         "(= the profiler's matrix-instruction count)",
                      "lower_triangle_128_tflop_per_step": round(lower128 / 1e12, 3),
                      "frac_on_lower_triangle_128": round(lower128 / (gemm_ms * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 4) if gemm_ms else 0.0,

@@ -524,14 +524,10 @@ int anc_quant_mxfp8_w_multi(uint64_t desc_table, int32_t n_weights, int64_t tota
 #define ANC_NS_BF16_X3 3
 #define ANC_NS_BF16_LATE3 4
 /* Flag OR-ed into a bf16 mode: treat a matrix whose dims are multiples of 256 like one whose dims are not. Its
- * products then run on 128-wide tiles with diagonal blocks of 128 computed in full (256 otherwise; everything
- * below is mirrored), and N >= 2M keeps 16-bit low halves of the iterate instead of 8-bit ones. Without residual
- * terms (ANC_NS_BF16_FAST) the bits are the same. Residual terms are added in an order that
- * depends on which elements of a symmetric product are computed and which are mirrored: the results then differ in
- * the last fp32 bits of A and B (1e-6 .. 4e-4 of the result, largest on gated outlier-column inputs). The other
- * low halves differ by 2^-16 per element, which the chain turns into another
- * realisation of its rounding error (the results are then 1.2e-3 apart, each inside the accuracy
- * bar). The flag exists so that tests can show both. */
+ * products then run on 128-wide tiles, and N >= 2M, M >= 1024 keeps 16-bit low halves of the iterate instead of
+ * 8-bit ones (ANC_NS_BF16). Elsewhere the bits are the same. The other low halves differ by 2^-16 per element, which
+ * the chain turns into another realisation of its rounding error (the results are then 1.2e-3 apart, each inside
+ * the accuracy bar). The flag exists so that tests can show both. */
 #define ANC_NS_TILE128 0x100
 /* Flags OR-ed into a bf16 mode: run every product on tiles of 64x64, 128x128 or (dims that are multiples
  * of 256) 256x256 / 128x256 outputs instead of choosing by the size of the launch. The bits are
@@ -612,13 +608,13 @@ int anc_muon_ns_update_multi(const anc_ns_problem_t *problems, int32_t n_problem
                              int mode, const float *lr_scales /* [ANC_MUON_MAX_SCALES] */, int sr,
                              uint32_t seed_base, uint64_t ctl, uint64_t stream);
 
-/* Matrix-core FLOPs of one anc_ns_batched call: `executed` counts the tiles and terms the
- * kernels really multiply (residual terms; of the symmetric products the tiles on or below the
- * diagonal, each in full: 256x256 tiles where dims are multiples of 256, i.e. 10/16 of the dense
- * product at M = 1024, else, or with ANC_NS_TILE128 in `mode`, 128x128 tiles, 36/64; the
- * profiler's matrix-instruction counter reads this number), `dense` is steps*(4 M^2 N + 2 M^3)
- * per matrix. Roofline figures use `executed`; matrices that take the conditioning gate add
- * anc_ns_hard_info's extra work. */
+/* Matrix-core FLOPs of one anc_ns_batched call: `executed` counts the terms the kernels multiply (residual
+ * terms too) and of the symmetric products the blocks on or below the diagonal, each in full: 256x256
+ * blocks where dims are multiples of 256, i.e. 10/16 of the dense product at M = 1024, else, or with
+ * ANC_NS_TILE128 in `mode`, 128x128 blocks, 36/64. `dense` is steps*(4 M^2 N + 2 M^3) per matrix. The kernels
+ * multiply 64x64 blocks, 136/256: with S = executed without and T = with ANC_NS_TILE128, dims multiples of 256,
+ * that is T - (S - T) / 2, the number that the profiler's matrix-instruction counter reads. Matrices that take the
+ * conditioning gate add anc_ns_hard_info's extra work, counted the same way. */
 int anc_ns_flops(int64_t E, int64_t M, int64_t N, int steps, int mode,
                  double *executed, double *dense);
 /* Of the E matrices of the last chain call that used `workspace`: how many took extra terms
