@@ -778,22 +778,19 @@ int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
 }
 
 // The same for the bare product of weight gradients. Its K is a batch of tokens: short ones are bound by the
-// output, which small tiles spread best, long ones by operands that leave the L2, and there a second 128-wide tile
-// on a few CUs costs as much as on all. Measured, us on 64 / 128 / 256-wide tiles, gradients added up (in
-// brackets: written):
-//   tiles of 64      256 tokens             1024 tokens            3072 tokens       8192 tokens
-//   640              8.5/10.2/13.5          18.2/17.6/24.2         41.9/37.8/46.5    112/83/100
-//   1024             10.7/11.0/16.1         22.9/20.1/29.5         53.0/42.2/51.6    149/91/110
-//   1056             12.4/13.5/16.9         26.5/24.7/27.9         59.6/56.0/50.3    162/121/103
-//                    (11.5/12.4/11.7)       (23.4/23.7/21.0)
-//   1344             15.4/15.0/18.5         31.7/27.6/29.9         75.9/61.6/52.5    223/127/107
-//                    (13.0/12.8/12.4)       (28.1/25.0/24.1)
-//   2816             26.6/27.3/34.2         58.2/53.0/50.9         154/99/91         466/230/198
-//                    (21.4/21.3/21.6)       (49.6/48.0/38.1)
-// hence up to 400 tokens 64 below 1300 tiles of 64 and 128 up to 2000 (3000 where something is added to), beyond 64
-// below 600 and 128 up to 1024, one per CU. (560 and fewer tiles of 64 are fastest at every length: 432 at 8192 tokens
-// 65 / 80 / 97.) Beyond 400 tokens the lines are those of a long batch: around 1024 tokens with gradients added up
-// 128-wide tiles would still be 13 % ahead at 1056 tiles and 8 % at 1344.
+// output, which small tiles spread best, long ones by operands that leave the L2, and there a second tile
+// on a few CUs costs as much as on all: the widest tile of which every CU has at most one. Measured, us on tiles of
+// 64 / 128x64 / 128 / 256, written (in brackets: added up):
+//   tiles of 64      256 tokens                768 tokens                2048 tokens            8192 tokens
+//   288              5.7/6.0/7.6/10.7          8.2/7.6/10.5/14.9         16.0/13.5/18.0/26.8    61/43/54/84
+//   432              5.5/6.0/7.6/10.7          8.1/7.9/10.6/15.0         16.7/14.6/18.2/27.5    64/46/54/85
+//                    (5.7/6.6/8.3/12.7)        (9.1/8.9/11.6/17.3)       (19/16/20/31)          (67/46/56/87)
+//   640              6.7/7.1/8.3/11.2          10.7/9.8/10.9/15.0        26.8/28.3/18.7/27.8    113/105/58/85
+//   896              11.0/7.8/8.9/11.3         14.3/12.4/12.3/15.2       28.9/27.8/22.8/27.8    125/101/71/85
+//   1056             10.2/10.1/10.6/11.3       16.5/17.6/17.3/15.2       36.4/38.6/36.3/27.8    142/145/122/87
+//   1344             18.0/10.9/12.0/11.6       20.5/17.8/17.6/16.5       42.5/40.6/36.0/29.9    183/149/121/93
+//                    (18.7/12.4/13.5/17.1)     (23.6/21.2/20.3/22.5)     (47/42/38/36)          (185/152/124/98)
+// (up to 256 tiles of 64 those are fastest at every length: 128 of them at 1504 tokens 8.3 / 10.2 / 14.7 / 20.3.)
 int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0;
   bool adds = false;
@@ -802,9 +799,8 @@ int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
     adds = adds || (ps[k].plain_sum && ps[k].A32 != nullptr);
   }
   for (int k = 0; k < n; ++k) t64 += (double)Es[k] * (ps[k].M / 64) * (ps[k].N / 64) * ((double)ps[k].K / longest);
-  const bool brief = longest <= 400.0;
-  if (t64 < (brief ? 1300.0 : 600.0)) return 64;
-  return t64 <= (!brief ? 1024.0 : adds ? 3000.0 : 2000.0) ? 128 : 256;
+  if (longest <= 640.0) return t64 <= 640.0 ? 64 : t64 <= 1536.0 ? kTile128x64 : t64 <= (adds ? 3000.0 : 2000.0) ? 128 : 256;
+  return t64 <= 256.0 ? 64 : t64 <= 512.0 ? kTile128x64 : t64 <= 1024.0 ? 128 : 256;
 }
 
 // What a mode's tile flags ask for (0: nothing).

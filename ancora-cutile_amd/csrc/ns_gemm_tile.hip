@@ -1,6 +1,6 @@
 // The products of the Newton-Schulz chain (A = X X^T, B = b A + c A A, X = a X + B X with their
 // epilogues; see ns.hip for the arithmetic) on 64x64 and 128x128 tiles, and the bare product of the
-// weight-gradient GEMM on the same tiles: for launches that the 256-wide tiles of ns_gemm_big.hip
+// weight-gradient GEMM on the same tiles and on 128x64 ones: for launches that the 256-wide tiles of ns_gemm_big.hip
 // would leave most of the chip idle, and for dims that are multiples of 128 only.
 //
 // What bounds it. Operand bytes come into LDS at about 24 B per clock and CU whatever the tile, so a
@@ -761,6 +761,12 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
 
 template <int EPI, bool AT, int VAR>
 void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) {
+  if constexpr (VAR == VAR_PLAIN) {
+    if (tile == kTile128x64) {
+      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+      return;
+    }
+  }
   if (tile == 128)      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 2, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
   else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, AT, VAR, 3, false>), dim3(grid), dim3(256), 0, s, pm);
   else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);

@@ -380,6 +380,39 @@ def test_accumulated_micro_batches_against_one_batch(gpu):
     assert same >= 0.98, same                                          # (D): the reference's bar
 
 
+@pytest.mark.parametrize("T,K,N,n", [(672, 640, 1792, 1), (736, 384, 3072, 1), (1504, 1024, 2048, 1), (32, 512, 1280, 5), (608, 1024, 1536, 4),
+                                     (96, 640, 2304, 3)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_tiles_of_128x64(gpu, T, K, N, n, accumulate):
+    """Calls on both ends of the range that runs on 128x64 tiles (257 .. 512 tiles of 64 beyond 640 tokens, 641 .. 1536
+    up to there), with one K tile, fewer than the ring has stages, and remainders of a round: the fp64 product, and
+    for n weights the bits each has alone."""
+    from ancora_cutile_amd import DevBuf
+    from ancora_cutile_amd.grads import gemm_dW, DwWorkspace
+    rng = np.random.default_rng(T + K + N)
+    x = _inputs(T, K, N, T + K + N)[0]
+    xd = DevBuf(x)
+    probs, want = [], []
+    for i in range(n):
+        dy = _inputs(T, K, N, T + i)[1]
+        old = (0.1 * rng.standard_normal((K, N))).astype(np.float32)
+        want.append(gemm_dw(x, dy) + (old if accumulate else 0.0))
+        probs.append(dict(x=xd, dy=DevBuf(dy), dW=DevBuf(old), g16=DevBuf.zeros((K, N), np.uint16), T=T, K=K, N=N,
+                          workspace=DwWorkspace(), accumulate=accumulate, old=old))
+    gemm_dW(probs)
+    for i, p in enumerate(probs):
+        got = p["dW"].to_numpy()
+        assert rel_fro(got, want[i]) < 2e-5
+        assert bits_equal(p["g16"].to_numpy(), bf16_rne_bits(got).reshape(K, N))
+        if n > 1:
+            p["dW"].upload(p["old"])
+            gemm_dW([p])
+            assert bits_equal(p["dW"].to_numpy(), got), i
+    for p in probs:
+        _free(p)
+    xd.free()
+
+
 @pytest.mark.parametrize("T", [96, 384, 416])
 @pytest.mark.parametrize("K,N,n", [(640, 768, 1), (1024, 1024, 3), (1024, 1024, 5), (1024, 1280, 7), (2048, 1536, 5)])
 @pytest.mark.parametrize("accumulate", [False, True])
