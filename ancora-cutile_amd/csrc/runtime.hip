@@ -239,12 +239,11 @@ int slot_take(StageRing &r, hipStream_t s, StageSlot **out) {
       if (slot.taken) continue;
       if (slot.busy) {
         const hipError_t e = hipEventQuery(slot.done);
-        if (e == hipErrorNotReady) {
-          (void)hipGetLastError();          // (not an error: a launch check must not find it)
-          if (slot.user == s && (mine == nullptr || slot.turn < mine->turn)) mine = &slot;
+        if (e != hipSuccess) {
+          (void)hipGetLastError();          // (not this upload's error: a launch check must not find it)
+          if (e == hipErrorNotReady && slot.user == s && (mine == nullptr || slot.turn < mine->turn)) mine = &slot;
           continue;
         }
-        ANC_HIP(e);
       }
       slot.busy = false;
       slot.taken = true;
@@ -264,15 +263,8 @@ int slot_take(StageRing &r, hipStream_t s, StageSlot **out) {
   return ANC_OK;
 }
 int slot_fill(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
-  if (slot.mem == nullptr) {
-    void *mem = nullptr;
-    ANC_HIP(hipHostMalloc(&mem, (size_t)kSlotBytes, hipHostMallocDefault));
-    if (hipError_t e = hipEventCreateWithFlags(&slot.done, hipEventDisableTiming)) {
-      (void)hipHostFree(mem);
-      return anc_hip_fail(e, "hipEventCreateWithFlags", __FILE__, __LINE__);
-    }
-    slot.mem = mem;
-  }
+  if (slot.mem == nullptr) ANC_HIP(hipHostMalloc(&slot.mem, (size_t)kSlotBytes, hipHostMallocDefault));
+  if (slot.done == nullptr) ANC_HIP(hipEventCreateWithFlags(&slot.done, hipEventDisableTiming));
   memcpy(slot.mem, src, (size_t)bytes);
   ANC_HIP(hipMemcpyAsync((void *)dst, slot.mem, (size_t)bytes, hipMemcpyHostToDevice, s));
   if (hipError_t e = hipEventRecord(slot.done, s)) {
@@ -297,6 +289,28 @@ int stage_piece(StageRing &r, uint64_t dst, const void *src, int64_t bytes, hipS
   slot->turn = ++r.turn;
   slot->taken = false;
   return rc;
+}
+// `s` is about to be destroyed. An event keeps the address of the stream it was last recorded on, and a query looks
+// there (uploads failed now and then with "an event last recorded in a capturing stream" after the second stream of
+// an optimizer was gone): slots last used on `s` wait for their copy and get a new event.
+int stage_forget(hipStream_t s) {
+  for (StageRing &r : g_ring)
+    for (StageSlot &slot : r.slot) {
+      {
+        std::lock_guard<std::mutex> lk(r.mu);
+        if (slot.taken || slot.done == nullptr || slot.user != s) continue;
+        slot.taken = true;
+      }
+      hipError_t e = slot.busy ? hipEventSynchronize(slot.done) : hipSuccess;
+      if (e == hipSuccess) e = hipEventDestroy(slot.done);
+      std::lock_guard<std::mutex> lk(r.mu);
+      slot.taken = false;
+      ANC_HIP(e);
+      slot.done = nullptr;
+      slot.user = nullptr;
+      slot.busy = false;
+    }
+  return ANC_OK;
 }
 // The ring's device is current.
 int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
@@ -373,7 +387,7 @@ extern "C" int anc_staging_release(void) {
         slot.taken = true;
       }
       hipError_t e = slot.busy ? hipEventSynchronize(slot.done) : hipSuccess;
-      if (e == hipSuccess) e = hipEventDestroy(slot.done);
+      if (e == hipSuccess && slot.done != nullptr) e = hipEventDestroy(slot.done);
       if (e == hipSuccess) e = hipHostFree(slot.mem);
       std::lock_guard<std::mutex> lk(r.mu);
       if (e == hipSuccess) slot = StageSlot{}; else slot.taken = false;
@@ -435,6 +449,7 @@ extern "C" int anc_stream_create_nonblocking(uint64_t *stream) {
 }
 extern "C" int anc_stream_destroy(uint64_t stream) {
   ANC_REQUIRE(stream != 0, "anc_stream_destroy: the null stream is not destroyable");
+  if (int rc = stage_forget(anc_stream(stream))) return rc;
   ANC_HIP(hipStreamDestroy(anc_stream(stream)));
   return ANC_OK;
 }

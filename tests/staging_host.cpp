@@ -24,6 +24,8 @@ int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stre
 int anc_upload_now(uint64_t dst, const void *src, int64_t bytes);
 int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
 int anc_staging_release(void);
+int anc_stream_create(uint64_t *stream);
+int anc_stream_destroy(uint64_t stream);
 const char *anc_last_error(void);
 }
 
@@ -35,13 +37,14 @@ struct Stream {
   bool held = false, capturing = false;
   std::deque<std::function<void()>> queue;
 };
-struct Event { int dev; bool done = true, captured = false; };
+struct Event { int dev; bool done = true, captured = false; Stream *on = nullptr; };
 static std::mutex mu;
 static std::condition_variable cv;
 static Stream null_stream[4] = {{0}, {1}, {2}, {3}};
 static std::set<Event *> events;
 static std::map<char *, size_t> pinned;
 static int live_streams = 0;
+static std::set<Stream *> gone;        // destroyed streams (their memory is kept, so that no new one has their address)
 static thread_local int cur = 0;
 static thread_local hipError_t last = hipSuccess;
 
@@ -88,13 +91,14 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   Stream *st = str(s);
   if (ev->dev != st->dev) return ret(hipErrorInvalidHandle);       // as the runtime does
   ev->captured = st->capturing;
+  ev->on = st;
   ev->done = false;
   push(st, [ev] { ev->done = true; });
   return hipSuccess;
 }
 hipError_t hipEventQuery(hipEvent_t e) {
   std::lock_guard<std::mutex> lk(mu);
-  if (((Event *)e)->captured) return ret(hipErrorCapturedEvent);
+  if (((Event *)e)->captured || gone.count(((Event *)e)->on)) return ret(hipErrorCapturedEvent);     // (or anything else)
   return ((Event *)e)->done ? hipSuccess : ret(hipErrorNotReady);
 }
 hipError_t hipEventSynchronize(hipEvent_t e) {
@@ -120,7 +124,8 @@ hipError_t hipStreamSynchronize(hipStream_t s) {
   return hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = (hipStream_t)new Stream{cur}; ++live_streams; return hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t s) { delete (Stream *)s; --live_streams; return hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t *s) { return hipStreamCreateWithFlags(s, 0); }
+hipError_t hipStreamDestroy(hipStream_t s) { std::lock_guard<std::mutex> lk(mu); gone.insert((Stream *)s); --live_streams; return hipSuccess; }
 hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t *d) { *d = str(s)->dev; return hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c) {
   *c = str(s)->capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
@@ -242,9 +247,45 @@ static void capture() {
   }
 }
 
+// Streams come and go with the objects that made them: uploads afterwards go through the same slots, whatever the
+// events of those streams would say by then.
+static void streams_that_end() {
+  const size_t n = 100;
+  const std::vector<char> want = bytes(n, 1);
+  Stream stays{0};
+  for (int round = 0; round < 4; ++round) {
+    uint64_t s = 0;
+    CHECK(anc_stream_create(&s) == 0);
+    std::vector<std::vector<char>> a(12, std::vector<char>(n));
+    for (auto &x : a) CHECK(anc_upload_async((uint64_t)x.data(), want.data(), (int64_t)n, s) == 0);
+    CHECK(anc_stream_destroy(s) == 0);
+    for (const auto &x : a) CHECK(x == want);
+    for (int i = 0; i < 12; ++i) {
+      std::vector<char> b(n);
+      CHECK(anc_upload_async((uint64_t)b.data(), want.data(), (int64_t)n, handle(&stays)) == 0);
+      CHECK(b == want && hipGetLastError() == hipSuccess);
+    }
+  }
+  // a stream that ends without the library's knowledge costs its slots, not the uploads after it
+  Stream other{0};
+  for (int i = 0; i < 3; ++i) {
+    std::vector<char> b(n);
+    CHECK(anc_upload_async((uint64_t)b.data(), want.data(), (int64_t)n, handle(&other)) == 0);
+  }
+  gone.insert(&other);
+  for (int i = 0; i < 12; ++i) {
+    std::vector<char> b(n);
+    CHECK(anc_upload_async((uint64_t)b.data(), want.data(), (int64_t)n, handle(&stays)) == 0);
+    CHECK(b == want && hipGetLastError() == hipSuccess);
+  }
+  CHECK(pinned.size() <= 8 && events.size() <= 8);
+  CHECK(anc_staging_release() == 0);
+  CHECK(pinned.empty() && events.empty() && live_streams == 0);
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}, {"other_streams_do_not_wait", other_streams_do_not_wait},
-                                                   {"many_threads", many_threads}, {"capture", capture}};
+                                                   {"many_threads", many_threads}, {"capture", capture}, {"streams_that_end", streams_that_end}};
   if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
   cases.at(argv[1])();
   printf("ok\n");
