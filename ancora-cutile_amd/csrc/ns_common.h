@@ -95,6 +95,7 @@ struct NsGemm {
                              // nterms_hard terms instead of nterms (its list is a prefix of the hard one)
   double cond_thresh;
   int nterms_hard;
+  const int32_t *order;      // (E) or null (as they come): the matrix in each place of the launch's sequence of matrices
   // Second gate: a matrix that k_ns_classify flagged (a spectrum spread over decades, many
   // moderately large columns, a low-rank signal over weak noise) multiplies nterms_wide terms;
   // wide_flag null or nterms_wide 0 = no such gate. It takes precedence over the gate above. With
@@ -160,6 +161,8 @@ __device__ __forceinline__ uint32_t anc_low8_encode(float y, uint32_t htop) {
 __device__ __forceinline__ float anc_low8_decode(uint32_t htop, int q) {
   return __uint_as_float(htop + ((uint32_t)q << 8));
 }
+// The matrix in place e of a launch's sequence
+__device__ __forceinline__ int anc_ns_matrix(const NsGemm &p, int e) { return p.order == nullptr ? e : anc_ld_const(p.order + e); }
 // Number of accumulation terms of matrix e: p.nterms, or more for a matrix that a gate marks.
 __device__ __forceinline__ int anc_ns_terms(const NsGemm &p, int e) {
   if (p.nterms_wide > 0 && anc_ns_wide(p, e)) return p.nterms_wide;

@@ -196,6 +196,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   }
   int e = 0, t = L, tm, tn;
   if (t >= tiles_per) { e = t / tiles_per; t -= e * tiles_per; }
+  if constexpr (!PLAINV) e = anc_ns_matrix(p, e);
   if (p.lower) {
     tm = 0;
     int left = t;

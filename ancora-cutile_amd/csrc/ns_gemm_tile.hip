@@ -106,6 +106,7 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
     tm = (br << sr) + (i >> sc_);
     tn = (bc << sc_) + (i & (p.blk_c - 1));
   }
+  if constexpr (!PLAINV) e = anc_ns_matrix(p, e);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;

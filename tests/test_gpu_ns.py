@@ -192,6 +192,24 @@ def test_tile_choice_keeps_the_bits(gpu, M, N, mode):
     assert rel_fro(want[0], host_ns(X[0], PE_SCHEDULE, 5)) < TOL_BF16
 
 
+@pytest.mark.parametrize("E,M,N", [(1, 1024, 1024), (3, 1024, 2048), (8, 1024, 1024), (19, 1024, 1024), (9, 1024, 2048)])
+@pytest.mark.parametrize("tiles", ["", "_t256"])
+def test_gated_matrices_are_dealt_in_turn(gpu, E, M, N, tiles):
+    """Launches of a gated iteration take the matrices in another order, gated ones first: batches of fewer matrices than
+    there are runs, as many, and more with a remainder; none, some side by side, and all gated. Every matrix
+    has the bits it has alone."""
+    rng = np.random.default_rng(E + M + N)
+    X = rng.standard_normal((E, M, N)).astype(np.float32)
+    cols = rng.choice(N, N // 100, replace=False)
+    for hard in ((), range(E // 3, E // 3 + (E + 2) // 3), range(E)):
+        Y = X.copy()
+        for e in hard:
+            Y[e][:, cols] *= np.float32(100.0)
+        got = run_ns(Y, mode="bf16" + tiles)
+        for e in sorted({0, E // 3, E // 2, E - 1}):
+            assert bits_equal(got[e], run_ns(Y[e: e + 1], mode="bf16")[0]), (list(hard), e)
+
+
 @pytest.mark.parametrize("E,M,N", [(86, 128, 128), (64, 128, 256), (65, 128, 256), (26, 256, 384)])
 @pytest.mark.parametrize("mode", ["bf16", "bf16_x3"])
 def test_many_small_tiles_keep_the_bits(gpu, E, M, N, mode):
