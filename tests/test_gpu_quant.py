@@ -60,6 +60,27 @@ def test_every_bf16_bit_pattern(gpu, cm):
     assert np.array_equal(f[nan_w] & 0x80, wf[nan_w] & 0x80)
 
 
+@pytest.mark.parametrize("cm", [False, True])
+def test_every_element_of_ordinary_blocks(gpu, cm):
+    """Blocks of finite numbers only: every mantissa at every distance from the block's amax down to results of zero,
+    both signs, ties included, at the scales around the one from which on the hardware converts, in the middle and
+    at the top; then whole columns of zeros beside them."""
+    K, N = 1792, 128
+    at = np.array([28, 30, 31, 32, 60, 127, 200, 254], np.uint32)[np.arange(N) % 8 if cm else np.arange(N) // 16]
+    d, m = np.divmod(np.arange(K // 32 * 31, dtype=np.uint32) % (13 * 128), 128)
+    rest = (np.maximum(at[None, :].astype(np.int64) - d[:, None], 1).astype(np.uint32) << 7) | m[:, None]
+    rest |= ((np.arange(rest.shape[0])[:, None] + np.arange(N)[None, :]) & 1).astype(np.uint32) << 15
+    blk = np.concatenate([np.broadcast_to((at << 7) | 0x7F, (K // 32, 1, N)), rest.reshape(K // 32, 31, N)], axis=1)
+    wb = blk.reshape(K, N).astype(np.uint16)
+    for zeros in (False, True):
+        if zeros:
+            wb[:, 3::5] = 0
+            wb[1::2, 3::5] = 0x8000
+        f, s = _run(wb, 1, K, N, cm)
+        wf, ws = ref_quant(wb, col_major=cm)
+        assert np.array_equal(s, ws) and np.array_equal(f, wf)
+
+
 def test_dequantised_weights_are_close(gpu):
     """The reference-held acceptance (tests/kernels/test_gpu_quant.py:45-47,68): max |deq - w| /
     max |w| below 8 %."""
