@@ -131,6 +131,19 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c) {
   *c = str(s)->capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
+// (the one kernel of these entry points copies: source, destination, bytes)
+struct Launch { dim3 grid, block; size_t shared; hipStream_t s; };
+static thread_local Launch launch;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t m, hipStream_t s) { launch = {g, b, m, s}; return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *m, hipStream_t *s) {
+  *g = launch.grid; *b = launch.block; *m = launch.shared; *s = launch.s;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **args, size_t, hipStream_t s) {
+  const void *src = *(const void **)args[0];
+  if (!is_pinned(src)) return ret(hipErrorInvalidValue);
+  return hipMemcpyAsync(*(void **)args[1], src, (size_t)*(int64_t *)args[2], hipMemcpyHostToDevice, s);
+}
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }
 void **__hipRegisterFatBinary(const void *) { return nullptr; }
 void __hipUnregisterFatBinary(void **) {}
