@@ -152,8 +152,8 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
     if (WM == 1 && kRing == 4) dma16(g + lane_at, lds_base);
     else                       dma16(g + at, off, lds_base);
   };
-  auto piece = [&](int i, unsigned char *st) {          // DMA instruction i of a stage: PA of A, PB of B
-    const bool cut = half_tail && is_kt + 1 == nk;      // (the missing panel's pieces fetch the one that is there)
+  auto piece = [&](int i, unsigned char *st, bool whole = false) {      // DMA instruction i of a stage: PA of A, PB of B
+    const bool cut = !whole && half_tail && is_kt + 1 == nk;            // (the missing panel's pieces fetch the one that is there)
     if (i < PA) {
       dma(curA - (cut ? cutA[i] : 0), offA[i], lA[i], voA, lds_addr(st + (wave * PA + i) * 1024));
     } else {
@@ -162,9 +162,9 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
     }
   };
   auto advance = [&]() { curA += advA; curB += advB; ++is_kt; };
-  auto issue = [&](unsigned char *st) {
+  auto issue = [&](unsigned char *st, bool whole = false) {
 #pragma unroll
-    for (int i = 0; i < kIps; ++i) piece(i, st);
+    for (int i = 0; i < kIps; ++i) piece(i, st, whole);
     advance();
   };
 
@@ -302,12 +302,13 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
 #pragma unroll
       for (int s0 = 0; s0 < kRing - 1; ++s0)
         if (s0 < nk) issue(lds + s0 * kStageBytes);
-      auto body = [&](int step, int s0) {
-        if (step + kRing - 1 <= nk) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
+      auto body = [&](auto steady, int step, int s0) {
+        constexpr bool kSteady = decltype(steady)::value;
+        if (kSteady || step + kRing - 1 <= nk) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
         lds_barrier();
-        if (step + kRing - 1 < nk) issue(lds + ((s0 + kRing - 1) % kRing) * kStageBytes);
+        if (kSteady || step + kRing - 1 < nk) issue(lds + ((s0 + kRing - 1) % kRing) * kStageBytes, kSteady);
         const unsigned char *st = lds + s0 * kStageBytes;
-        const bool cut = half_tail && step + 1 == nk;
+        const bool cut = !kSteady && half_tail && step + 1 == nk;
 #pragma unroll
         for (int kk = 0; kk < TK / 16; ++kk) {
           if (PLAINV && kk >= 2 && cut) break;
@@ -316,10 +317,18 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
           mma(a, b);
         }
       };
-      for (int step = 0; step < nk; step += kRing) {
+      int step = 0;
+      // Rounds in which even the last step's refill is a whole stage that is there, without a branch (one (1024,3072) matrix
+      // 203 -> 194 us per chain, (1024,1024) 147 -> 142. Three workgroups per CU hide the branches, and lose 1 % by the
+      // code: 4 x (1024,1024) 293 -> 297. Fragments a step ahead give nothing here either.)
+      for (; kRing == 4 && step + 2 * kRing - 1 < nk; step += kRing) {
+#pragma unroll
+        for (int s0 = 0; s0 < kRing; ++s0) body(std::true_type{}, step + s0, s0);
+      }
+      for (; step < nk; step += kRing) {
 #pragma unroll
         for (int s0 = 0; s0 < kRing; ++s0)
-          if (step + s0 < nk) body(step + s0, s0);
+          if (step + s0 < nk) body(std::false_type{}, step + s0, s0);
       }
     } else {
       // Fragments are read into registers one step ahead. At the top of step k a wavefront waits for its own DMA of step
