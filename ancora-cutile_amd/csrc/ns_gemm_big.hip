@@ -219,9 +219,10 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int wm = wave / NWN, wn = wave % NWN, part = kFull;
+  const bool on_diag = EPI != EPI_BX && tm == tn;
   if constexpr (EPI != EPI_BX) {
     static_assert(TM == 256 && TN == 256, "the dealing below");
-    if (tm == tn) {
+    if (on_diag) {
       // Wavefronts w and w + 4 share a SIMD, so a full and a half part meet: (0,0) with (0,1), (1,2) with (1,3), and
       // (1,0), (1,1) each with one of the two that have nothing to do. The tile takes three quarters of the time.
       wm = (0x2E >> wave) & 1;
@@ -295,16 +296,10 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       else        dma16(pb + j * roB, vo, lds_addr(stage + TM * ROWB + (wave * IB + j) * 1024));
     }
   };
-  auto issue = [&](unsigned char *stage) {
-#pragma unroll
-    for (int i = 0; i < IPS; ++i) issue_piece(i, stage, curA, curB);
-    curA += advA;
-    curB += advB;
-  };
 
   // ---- fragment addressing
   const int a_base = (wm * 128 + (lane & 31)) * ROWB;
-  const int b_base = TM * ROWB + (wn * 64 + (lane & 31)) * ROWB;
+  const int b_base = (on_diag ? 0 : TM * ROWB) + (wn * 64 + (lane & 31)) * ROWB;
   int swz[KSTEPS];
 #pragma unroll
   for (int kk = 0; kk < KSTEPS; ++kk)
@@ -369,8 +364,18 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       for (int r = 0; r < 16; ++r) acc[bi][bj][r] = 0.0f;
 
   const int nterms = PLAINV ? 1 : anc_ns_terms(p, e);
-  auto single = [&](auto prt) {
+  // (one_operand: a tile on the diagonal of a symmetric product. Its two operands are the same rows, so A's alone are
+  // fetched, half of the bytes, and b_base points at them: chains of 48 x (1024,1024) 1806 -> 1795 us, 24 x (1024,2048) 1199 -> 1194,
+  // the 196 matrices of a 0.6 B parameter model 0.1 ms of 10.3.)
+  auto single = [&](auto prt, auto one_operand) {
     constexpr int P = decltype(prt)::value;
+    constexpr int IPT = decltype(one_operand)::value ? IA : IPS;          // DMA instructions per wavefront per stage
+    auto issue = [&](unsigned char *stage) {
+#pragma unroll
+      for (int i = 0; i < IPT; ++i) issue_piece(i, stage, curA, curB);
+      curA += advA;
+      curB += advB;
+    };
     // Stage ring. Tile k lives in stage k % NS. The DMA of tile k+NS-1 is started at the top of
     // tile k, into the stage that tile k-1 was read from (every wavefront left it before the
     // barrier inside tile k-1). Before the last k-step of tile k each wavefront waits until its
@@ -380,7 +385,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
 #pragma unroll
     for (int s0 = 0; s0 < NS - 1; ++s0)
       if (s0 < nk) issue(st(s0));
-    if (nk >= NS - 1) wait_vm<(NS - 2) * IPS>(); else wait_vm<0>();
+    if (nk >= NS - 1) wait_vm<(NS - 2) * IPT>(); else wait_vm<0>();
     lds_barrier();
     if (P != kNone) frags(stage0, 0, a[0], b[0]);
 
@@ -390,12 +395,12 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       constexpr bool kSteady = decltype(steady)::value;
       const bool more = kSteady || step + 1 < nk;
       const bool refill = kSteady || step + NS - 1 < nk;
-      mfma8_with<BT, IPS, P>(a[0], b[0], acc, [&](int idx) { if (P != kNone) frag(cur, cur, 1, idx, a[1], b[1]); },
+      mfma8_with<BT, IPT, P>(a[0], b[0], acc, [&](int idx) { if (P != kNone) frag(cur, cur, 1, idx, a[1], b[1]); },
                           [&](int i) { if (refill) issue_piece(i, fill, curA, curB); });
       if (refill) {
         curA += advA;
         curB += advB;
-        wait_vm<(NS - 2) * IPS>();
+        wait_vm<(NS - 2) * IPT>();
       } else {
         wait_vm<0>();
       }
@@ -415,8 +420,9 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         if (step + s0 < nk) body(std::false_type{}, step + s0, st(s0), st((s0 + 1) % NS), st((s0 + NS - 1) % NS));
     }
   };
-  auto several = [&](auto prt) {
+  auto several = [&](auto prt, auto one_operand) {
     constexpr int P = decltype(prt)::value;
+    constexpr bool ONE = decltype(one_operand)::value;
     // Several terms: K tile t is two stages, the high halves h_t in stage 2t % NS and the low halves l_t in
     // the next one (of two terms only B's low half is there). Six phases of 8 MFMAs per tile,
     //   P0 hh k 0..15, P1 hh 16..31, P2 hl 16..31, P3 lh 16..31, P4 hl 0..15, P5 lh 0..15,
@@ -427,14 +433,14 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     // times per tile.
     const char *loA = (const char *)p.A[1] + ubaseA, *loB = (const char *)p.B[1] + (BT ? ubaseBT : ubaseB);
     auto pairs = [&](auto nt) {
-      constexpr int NT = decltype(nt)::value, PL = NT == 3 ? IPS : IB;      // DMA instructions of a low stage
+      constexpr int NT = decltype(nt)::value, PH = ONE ? IA : IPS, PL = NT == 3 ? PH : IB;      // DMA instructions of a high and a low stage
       auto piece_h = [&](int i, unsigned char *stage) { issue_piece(i, stage, curA, curB); };
       auto piece_l = [&](int i, unsigned char *stage) { issue_piece(NT == 3 ? i : IA + i, stage, loA, loB); };
       auto adv_h = [&]() { curA += advA; curB += advB; };
       auto adv_l = [&]() { loA += advA; loB += advB; };
       auto all_h = [&](unsigned char *stage) {
 #pragma unroll
-        for (int i = 0; i < IPS; ++i) piece_h(i, stage);
+        for (int i = 0; i < PH; ++i) piece_h(i, stage);
         adv_h();
       };
       auto all_l = [&](unsigned char *stage) {
@@ -446,7 +452,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       all_h(st(0));
       all_l(st(1));
       if (NS == 4) {
-        if (nk > 1) { all_h(st(2)); wait_vm<PL + IPS>(); } else wait_vm<PL>();
+        if (nk > 1) { all_h(st(2)); wait_vm<PL + PH>(); } else wait_vm<PL>();
       } else {
         wait_vm<PL>();
       }
@@ -464,7 +470,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
           mfma8_with<BT, PL, P>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_l(i, L1); });
           if (more) adv_l();
         } else {
-          mfma8_with<BT, IPS, P>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_h(i, H1); });
+          mfma8_with<BT, PH, P>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_h(i, H1); });
           if (more) adv_h();
         }
         // P1
@@ -472,7 +478,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
 #pragma unroll
           for (int idx = 0; idx < 4; ++idx) mfma1<BT>(a[y], b[1], acc, idx);
         }
-        if (more) wait_vm<NS == 4 ? IPS + PL : IPS>(); else wait_vm<0>();
+        if (more) wait_vm<NS == 4 ? PH + PL : PH>(); else wait_vm<0>();
         lds_barrier();
 #pragma unroll
         for (int idx = 4; idx < 8; ++idx) {
@@ -499,7 +505,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         // P5 (P4 of two terms)
         auto load5 = [&](int idx) { if (P != kNone && more) frag(H1, H1, 0, idx - 1, a[y], b[0]); };
         if (NS == 4) {
-          mfma8_with<BT, IPS, P>(a[x], b[1], acc, load5, [&](int i) { if (more2) piece_h(i, H); });
+          mfma8_with<BT, PH, P>(a[x], b[1], acc, load5, [&](int i) { if (more2) piece_h(i, H); });
           if (more2) adv_h();
         } else {
           mfma8_with<BT, PL, P>(a[x], b[1], acc, load5, [&](int i) { if (more) piece_l(i, H); });
@@ -531,17 +537,18 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     if (EPI == EPI_BX && nterms == 2) pairs(std::integral_constant<int, 2>{});
     else pairs(std::integral_constant<int, 3>{});
   };
-  auto multiply = [&](auto prt) {
-    if constexpr (PLAINV) single(prt);
-    else if (nterms == 1) single(prt);
-    else several(prt);
+  auto multiply = [&](auto prt, auto one_operand) {
+    if constexpr (PLAINV) single(prt, one_operand);
+    else if (nterms == 1) single(prt, one_operand);
+    else several(prt, one_operand);
   };
   if constexpr (EPI == EPI_BX) {
-    multiply(std::integral_constant<int, kFull>{});
+    multiply(std::integral_constant<int, kFull>{}, std::false_type{});
   } else {
-    if (part == kFull) multiply(std::integral_constant<int, kFull>{});
-    else if (part == kLower) multiply(std::integral_constant<int, kLower>{});
-    else multiply(std::integral_constant<int, kNone>{});
+    if (!on_diag) multiply(std::integral_constant<int, kFull>{}, std::false_type{});
+    else if (part == kFull) multiply(std::integral_constant<int, kFull>{}, std::true_type{});
+    else if (part == kLower) multiply(std::integral_constant<int, kLower>{}, std::true_type{});
+    else multiply(std::integral_constant<int, kNone>{}, std::true_type{});
   }
   __syncthreads();
   if (EPI != EPI_BX && part == kNone) return;

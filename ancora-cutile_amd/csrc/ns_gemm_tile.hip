@@ -162,11 +162,11 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
     }
   };
   auto advance = [&]() { curA += advA; curB += advB; ++is_kt; };
-  auto issue = [&](unsigned char *st, bool whole = false) {
-#pragma unroll
-    for (int i = 0; i < kIps; ++i) piece(i, st, whole);
-    advance();
-  };
+  // A 128-wide tile on the diagonal of a symmetric product: its two operands are the same rows, so A's alone are fetched
+  // and B's fragments come from A's part of a stage (42 x (640,640) 978 -> 968 us per chain). 64-wide tiles lose by
+  // the second K loop: 16 x (768,768) 593 -> 611.
+  constexpr bool kDiag = EPI != EPI_BX && WM > 1;
+  const bool on_diag = kDiag && tm == tn;
 
   // ---- fragment addressing: tr = [block][k][64 B] by transposing reads, else [panel][row][64 B]
   const int l31 = lane & 31, hh = lane >> 5, g16 = lane >> 4, s16 = lane & 15;
@@ -292,10 +292,16 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
 #pragma unroll
     for (int i = 0; i < WM; ++i) fa[i] = frag(TrA{}, st, wm * WM + i, kk, TK, TM);
 #pragma unroll
-    for (int i = 0; i < WN; ++i) fb[i] = frag(TrB{}, st + kHalf, wn * WN + i, kk, TK, TN);
+    for (int i = 0; i < WN; ++i) fb[i] = frag(TrB{}, st + (on_diag ? 0 : kHalf), wn * WN + i, kk, TK, TN);
   };
-  // ---- K loop, one term. Step k lives in stage k % kRing.
-  if (PLAINV || nterms == 1) {
+  // ---- one term. Step k lives in stage k % kRing.
+  auto single = [&](auto one_operand) {
+    constexpr int kI = decltype(one_operand)::value ? PA : kIps;      // DMA instructions per wavefront and stage
+    auto issue = [&](unsigned char *st, bool whole = false) {
+#pragma unroll
+      for (int i = 0; i < kI; ++i) piece(i, st, whole);
+      advance();
+    };
     if constexpr (WM == 1) {
       // At the top of step k a wavefront waits for its own DMA of the step (the younger ones stay in flight), the
       // workgroup meets, and the DMA of step k + kRing - 1 goes out into the stage everybody has just left.
@@ -304,7 +310,7 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
         if (s0 < nk) issue(lds + s0 * kStageBytes);
       auto body = [&](auto steady, int step, int s0) {
         constexpr bool kSteady = decltype(steady)::value;
-        if (kSteady || step + kRing - 1 <= nk) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
+        if (kSteady || step + kRing - 1 <= nk) wait_vm<(kRing - 2) * kI>(); else wait_vm<0>();
         lds_barrier();
         if (kSteady || step + kRing - 1 < nk) issue(lds + ((s0 + kRing - 1) % kRing) * kStageBytes, kSteady);
         const unsigned char *st = lds + s0 * kStageBytes;
@@ -342,11 +348,11 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
 #pragma unroll
       for (int s0 = 0; s0 < kRing; ++s0)
         if (s0 < nk) issue(lds + s0 * kStageBytes);
-      if (kRing <= nk) wait_vm<(kRing - 1) * kIps>(); else wait_vm<0>();
+      if (kRing <= nk) wait_vm<(kRing - 1) * kI>(); else wait_vm<0>();
       lds_barrier();
       if (idle) {                        // (its share of the DMA, and the meetings)
         for (int step = 0, at = 0; step < nk; ++step) {
-          if (step + kRing <= nk) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
+          if (step + kRing <= nk) wait_vm<(kRing - 2) * kI>(); else wait_vm<0>();
           lds_barrier();
           if (step + kRing < nk) issue(lds + at);
           at = at + kStageBytes == kRing * kStageBytes ? 0 : at + kStageBytes;
@@ -358,7 +364,7 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
           constexpr bool kSteady = decltype(steady)::value;
           constexpr int s0 = decltype(s0v)::value % kRing, x = decltype(s0v)::value % 2;
           const bool more = kSteady || step + 1 < nk, refill = kSteady || step + kRing < nk;
-          if (kSteady || step + kRing <= nk) wait_vm<(kRing - 2) * kIps>(); else wait_vm<0>();
+          if (kSteady || step + kRing <= nk) wait_vm<(kRing - 2) * kI>(); else wait_vm<0>();
           lds_barrier();
 #pragma unroll
           for (int kk = 0; kk < KK; ++kk) {
@@ -366,7 +372,7 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
             __builtin_amdgcn_sched_barrier(0);
             if (refill) {
 #pragma unroll
-              for (int i = kk * kIps / KK; i < (kk + 1) * kIps / KK; ++i) piece(i, lds + s0 * kStageBytes);
+              for (int i = kk * kI / KK; i < (kk + 1) * kI / KK; ++i) piece(i, lds + s0 * kStageBytes);
             }
             if (more) frags(lds + (s0 + 1) % kRing * kStageBytes, kk, a[1 - x][kk], b[1 - x][kk]);
             __builtin_amdgcn_sched_barrier(0);
@@ -387,6 +393,15 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
         for (; step < nk; step += U) round(std::false_type{}, step);
       }
     }
+  };
+  // ---- K loop
+  if (PLAINV || nterms == 1) {
+    if constexpr (kDiag) {
+      if (on_diag) single(std::true_type{});
+      else single(std::false_type{});
+    } else {
+      single(std::false_type{});
+    }
   } else {
     // ---- several terms: a step is one panel of 32 k of both halves of both operands, high stage then low stage.
     constexpr int kPanA = TM * 64, kPanB = TN * 64, kLow = kPanA + kPanB, kPair = 2 * kLow, kPairs = kRing * kStageBytes / kPair;
@@ -405,8 +420,10 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
     }
     const char *pAl = (const char *)p.A[1] + baseA, *pBl = (const char *)p.B[1] + baseB;
     const int64_t adA = AT ? 32 * rpA : psA, adB = BT ? 32 * rpB : psB;
-    auto terms = [&](auto nt) {
-      constexpr int NT = decltype(nt)::value, kIpp = NT == 3 ? 2 * (WM + WN) : WM + 2 * WN;   // DMA instructions per wavefront and step
+    const int at_b = on_diag ? 0 : kPanA;
+    auto terms = [&](auto nt, auto one_operand) {
+      constexpr bool ONE = decltype(one_operand)::value;
+      constexpr int NT = decltype(nt)::value, kIpp = ONE ? 2 * WM : NT == 3 ? 2 * (WM + WN) : WM + 2 * WN;   // DMA instructions per wavefront and step
       auto issue_pair = [&](unsigned char *st) {
 #pragma unroll
         for (int j = 0; j < WM; ++j) {
@@ -414,7 +431,7 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
           if (NT == 3) dma(pAl, oA[j], vA[j], voA, lds_addr(st + kLow + (wave * WM + j) * 1024));
         }
 #pragma unroll
-        for (int j = 0; j < WN; ++j) {
+        for (int j = 0; j < (ONE ? 0 : WN); ++j) {
           dma(curB, oB[j], vB[j], voB, lds_addr(st + kPanA + (wave * WN + j) * 1024));
           dma(pBl, oB[j], vB[j], voB, lds_addr(st + kLow + kPanA + (wave * WN + j) * 1024));
         }
@@ -450,22 +467,22 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
       };
       auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
       rd_a(lds, 0, ah[0]);
-      rd_b(lds + kPanA, 0, bh[0]);
+      rd_b(lds + at_b, 0, bh[0]);
       auto body = [&](auto steady, int step, auto s0v) {
         constexpr int s0 = decltype(s0v)::value % kPairs, x = decltype(s0v)::value % 2, y = 1 - x;
         const unsigned char *st = lds + s0 * kPair, *nx = lds + (s0 + 1) % kPairs * kPair;
         const bool more = decltype(steady)::value || step + 1 < np, refill = decltype(steady)::value || step + kPairs < np;
         rd_a(st, 1, ah[1]);
-        rd_b(st + kPanA, 1, bh[y]);
+        rd_b(st + at_b, 1, bh[y]);
         fence();
         mma(ah[0], bh[x]);                                    // hh 0..15
         fence();
-        rd_b(st + kLow + kPanA, 1, bl[1]);
+        rd_b(st + kLow + at_b, 1, bl[1]);
         if (NT == 3) rd_a(st + kLow, 1, al[1]);
         fence();
         mma(ah[1], bh[y]);                                    // hh 16..31
         fence();
-        rd_b(st + kLow + kPanA, 0, bl[0]);
+        rd_b(st + kLow + at_b, 0, bl[0]);
         if (NT == 3) rd_a(st + kLow, 0, al[0]);
         fence();
         mma(ah[1], bl[1]);                                    // hl 16..31
@@ -478,7 +495,7 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
         lds_barrier();
         if (refill) issue_pair(lds + s0 * kPair);
         if (NT == 3 && more) rd_a(nx, 0, ah[0]);
-        if (more) rd_b(nx + kPanA, 0, bh[y]);
+        if (more) rd_b(nx + at_b, 0, bh[y]);
         fence();
         if (NT == 3) mma(al[0], bh[x]);                       // lh 0..15
         else         mma(ah[0], bl[0]);                       // (of two terms: hl 0..15)
@@ -506,8 +523,14 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
       for (; step + U - 1 + kPairs < np; step += U) round(std::true_type{}, step);
       for (; step < np; step += U) round(std::false_type{}, step);
     };
-    if (EPI == EPI_BX && nterms == 2) terms(std::integral_constant<int, 2>{});
-    else terms(std::integral_constant<int, 3>{});
+    if (EPI == EPI_BX && nterms == 2) {
+      terms(std::integral_constant<int, 2>{}, std::false_type{});
+    } else if constexpr (kDiag) {
+      if (on_diag) terms(std::integral_constant<int, 3>{}, std::true_type{});
+      else terms(std::integral_constant<int, 3>{}, std::false_type{});
+    } else {
+      terms(std::integral_constant<int, 3>{}, std::false_type{});
+    }
   }
   __syncthreads();
 
