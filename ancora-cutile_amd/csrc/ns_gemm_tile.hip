@@ -45,11 +45,16 @@ __device__ __forceinline__ void ld_run(const void *p, uint32_t *w) {
   else if constexpr (BYTES == 8) { const anc_u32x2 t = *(const anc_u32x2 *)p; w[0] = t.x; w[1] = t.y; }
   else w[0] = *(const uint32_t *)p;
 }
-template <int BYTES>
+// (STREAM: past the caches)
+template <int BYTES, bool STREAM = false>
 __device__ __forceinline__ void st_run(void *p, const uint32_t *w) {
-  if constexpr (BYTES == 16) *(anc_u32x4 *)p = anc_u32x4{w[0], w[1], w[2], w[3]};
-  else if constexpr (BYTES == 8) *(anc_u32x2 *)p = anc_u32x2{w[0], w[1]};
-  else *(uint32_t *)p = w[0];
+  auto st = [](auto *q, auto v) {
+    if constexpr (STREAM) anc_st_stream(q, v);
+    else *q = v;
+  };
+  if constexpr (BYTES == 16) st((anc_u32x4 *)p, anc_u32x4{w[0], w[1], w[2], w[3]});
+  else if constexpr (BYTES == 8) st((anc_u32x2 *)p, anc_u32x2{w[0], w[1]});
+  else st((uint32_t *)p, w[0]);
 }
 
 // What the weight update reads and writes once: past the caches where a launch has many tiles (WIDE: the 128-wide ones), so
@@ -574,10 +579,10 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
       else h[i] = anc_pk_bf16(v[2 * i], v[2 * i + 1]);
     }
 #pragma unroll
-    for (int r = 0; r < NR; ++r) st_run<RUN * 2>(out + r * step, h + r * (RUN / 2));
+    for (int r = 0; r < NR; ++r) st_run<RUN * 2, VAR == VAR_STREAM>(out + r * step, h + r * (RUN / 2));
     if (lo != nullptr) {
 #pragma unroll
-      for (int r = 0; r < NR; ++r) st_run<RUN * 2>(lo + r * step, l + r * (RUN / 2));
+      for (int r = 0; r < NR; ++r) st_run<RUN * 2, VAR == VAR_STREAM>(lo + r * step, l + r * (RUN / 2));
     }
   };
 #pragma unroll
@@ -793,8 +798,8 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
           }
 #pragma unroll
           for (int r = 0; r < NR; ++r) {
-            st_run<RUN * 2>(p.Yh + mn + pan + r * pst, h + r * (RUN / 2));
-            st_run<RUN>((char *)p.Yl + mn * 2 + pan + r * pst, q + r * (RUN / 4));
+            st_run<RUN * 2, VAR == VAR_STREAM>(p.Yh + mn + pan + r * pst, h + r * (RUN / 2));
+            st_run<RUN, VAR == VAR_STREAM>((char *)p.Yl + mn * 2 + pan + r * pst, q + r * (RUN / 4));
           }
         } else {
           put_bf16(p.Yh + mn + pan, p.Yl + mn + pan, pst);
@@ -809,6 +814,12 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) 
   if constexpr (VAR == VAR_PLAIN) {
     if (tile == kTile128x64) {
       hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+      return;
+    }
+  }
+  if constexpr (VAR == VAR_NONE && EPI == EPI_BX) {
+    if (tile == 128 && pm.g[0].stream_out) {
+      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 2, AT, VAR_STREAM, 4, false>), dim3(grid), dim3(256), 0, s, pm);
       return;
     }
   }

@@ -223,6 +223,20 @@ def test_many_small_tiles_keep_the_bits(gpu, E, M, N, mode):
         assert bits_equal(got[e], run_ns(X[e: e + 1], mode=mode)[0]), e
 
 
+@pytest.mark.parametrize("E,M,N,mode", [(159, 384, 384, "bf16"), (160, 384, 384, "bf16"), (160, 384, 384, "bf16_x3"),
+                                        (46, 512, 1024, "bf16_t128"), (12, 1024, 2048, "bf16_t128")])
+def test_iterates_past_the_caches_keep_the_bits(gpu, E, M, N, mode):
+    """128-wide tiles store iterates of 90 MiB and more past the caches: batches on both sides of that line, and with an
+    8-bit low half. Every matrix has the bits it has alone, and meets the bar."""
+    rng = np.random.default_rng(E + M + N)
+    X = rng.standard_normal((E, M, N), dtype=np.float32)
+    X[E - 1][:, :2] *= 100.0
+    got = run_ns(X, mode=mode)
+    for e in (0, E // 2, E - 1):
+        assert bits_equal(got[e], run_ns(X[e: e + 1], mode=mode)[0]), e
+    assert rel_fro(got[0], host_ns(X[0], PE_SCHEDULE, 5)) < TOL_BF16
+
+
 @pytest.mark.parametrize("E,M,N", [(1, 128, 128), (3, 128, 384), (2, 256, 512), (1, 640, 768), (2, 1024, 1024), (2, 1024, 2048)])
 @pytest.mark.parametrize("sched", ["pe", "keller"])
 def test_bf16_entry_takes_the_matrix_as_it_is(gpu, E, M, N, sched):
