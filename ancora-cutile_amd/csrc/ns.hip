@@ -880,11 +880,12 @@ int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
   return t64 <= 256.0 ? 64 : t64 <= 512.0 ? kTile128x64 : t64 <= 1024.0 ? 128 : 256;
 }
 
-// Does the next iterate leave its launch past the caches (NsGemm::stream_out; the 256-wide tiles always store it so)? A
-// bf16 pair of about three times what the L2s hold (32 MiB) pushes the operands of the tiles still to come out of them;
-// of a smaller one A = X X^T finds enough there, and 64-wide tiles of that product read every row so often that they
-// want it there at any size. Up to M = 256 a column panel of the iterate has two readers at most and nothing is gained.
-// Measured, us per chain, kept / past the caches:
+// What leaves a launch past the caches (NsGemm::stream_out): the caches are left to the operands of the tiles still to
+// come, but the next launch finds nothing there.
+// The next iterate, on 128-wide tiles. A bf16 pair of about three times what the L2s hold (32 MiB) pushes operands out of
+// them; of a smaller one A = X X^T finds enough there, and 64-wide tiles of that product read every row so often that
+// they want it there at any size. Up to M = 256 a column panel of the iterate has two readers at most and nothing is
+// gained. Measured, us per chain, kept / past the caches:
 //   38 MB       12 x (512,1536) on 128-wide tiles 447 / 478, 24 x (384,1024) 375 / 393
 //   79 .. 85    48 x (640,640) 1060 / 1035, 24 x (640,1280) 821 / 842, 16 x (1152,1152) 979 / 988
 //   96 .. 118   30 x (896,896) 1480 / 1460, 60 x (640,640) 1252 / 1233, 100 x (384,768) 998 / 978
@@ -892,7 +893,13 @@ int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
 //               24 x (1152,1152) 1451 / 1450, 12 x (1152,2304) 1063 / 1071
 //   M <= 256    300 x (256,256) 786 / 763, 200 x (256,768) 1073 / 1082, 600 x (128,256) 580 / 587
 //   A on 64-wide tiles   12 x (512,1536) 356 / 360, 60 x (384,768) 560 / 581, 18 x (640,1792) 755 / 803
-constexpr int64_t kStreamPair = 90 << 20;
+// The next iterate, on 256-wide tiles: kept where A = X X^T does not run on 256-wide ones, which is where few matrices
+// are wide, and reads the high halves only: 12 x (1024,2048) 678 / 705, 12 x (1024,3072) 923 / 949, 6 x (1536,4096) 1174 / 1205;
+// on 256-wide ones 12 x (1536,1536) 1282 / 1252, 24 x (1024,3072) 1589 / 1565, 40 x (1024,1024) 1542 / 1522; both halves
+// 40 x (512,1536) 1018 / 1011, 20 x (768,2304) 1436 / 1429.
+// A and B on 256-wide tiles: kept up to 24 Mi elements. 16 x (1024,1024) 667 / 684, 20 x (1024,1024) 793 / 815, 24 x (1024,1024)
+// 899 / 900, 24 x (1024,2048) 1134 / 1153; 32 x (1024,1024) 1338 / 1335, 40 x (1024,1024) 1539 / 1522, 12 x (1536,1536) 1264 / 1252.
+constexpr int64_t kStreamPair = 90 << 20, kKeepSquare = 24 << 20;
 
 // What a mode's tile flags ask for (0: nothing).
 int forced_tile(int flags) {
@@ -1010,16 +1017,21 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       gx[q].l8_out = l8_next;
       l8_cur[q] = l8_next;
     }
-    if (!last) {
-      NsGemm next[kMaxGroups];               // the product that reads the next iterate
-      int64_t pair = 0;
-      for (int q = 0; q < n; ++q) {
-        next[q] = ga[q];
-        next[q].nterms = k + 1 >= cp[q].pl.sp.x_from ? 3 : 1;
-        if (cp[q].M > 256) pair += Es[q] * cp[q].M * cp[q].N * 4;
-      }
-      const bool stream = pair >= kStreamPair && (force != 0 ? force : pick_tile(EPI_GRAM, next, Es, n)) != 64;
-      for (int q = 0; q < n; ++q) gx[q].stream_out = stream ? 1 : 0;
+    // (on the last step too, where nobody reads on: one kernel for all steps)
+    NsGemm next[kMaxGroups];                 // the product that reads the next iterate
+    int64_t pair = 0, square = 0;
+    bool terms = false;
+    for (int q = 0; q < n; ++q) {
+      next[q] = ga[q];
+      next[q].nterms = k + 1 >= cp[q].pl.sp.x_from ? 3 : 1;
+      terms = terms || next[q].nterms > 1;
+      if (cp[q].M > 256) pair += Es[q] * cp[q].M * cp[q].N * 4;
+      square += Es[q] * cp[q].M * cp[q].M;
+    }
+    const int reader = force != 0 ? force : pick_tile(EPI_GRAM, next, Es, n);
+    for (int q = 0; q < n; ++q) {
+      gx[q].stream_out = (reader != 64 && pair >= kStreamPair ? kStream128 : 0) | (reader == 256 || terms ? kStream256 : 0);
+      ga[q].stream_out = gb[q].stream_out = square > kKeepSquare ? kStream256 : 0;
     }
     {
       AncProfScope prof(ANC_PROF_NS_GRAM, s);

@@ -38,7 +38,8 @@ constexpr int kCondParts = 64;           // partial sums per matrix of the condi
 constexpr int kXcds = 8;
 
 enum { EPI_GRAM = 0, EPI_BMAT = 1, EPI_BX = 2 };
-enum { VAR_NONE = 0, VAR_UPDATE = 1, VAR_PLAIN = 2, VAR_UPDATE_T = 3, VAR_STREAM = 4 };   // variants of the EPI_BX epilogue
+enum { VAR_NONE = 0, VAR_UPDATE = 1, VAR_PLAIN = 2, VAR_UPDATE_T = 3, VAR_STREAM = 4 };   // variants of the epilogue (1 .. 3: of EPI_BX)
+enum { kStream128 = 1, kStream256 = 2 };                                                  // NsGemm::stream_out
 
 // Workgroup id -> logical tile id such that logical ids [start(x), start(x+1)) run on XCD x
 // (hardware deals consecutive workgroup ids round-robin over the 8 XCDs).
@@ -84,7 +85,8 @@ struct NsGemm {
   const uint16_t *Xh, *Xl;   // (E,M,N) current iterate as a bf16 pair, X = Xh + Xl   BX in
   int lo_zero;               // the input has no low half (a bf16 matrix): Xl is one zeroed 16-byte piece that every
                              // read of a low half goes to
-  int stream_out;            // BX on 128-wide tiles: the pair is stored past the caches (VAR_STREAM; a rule of ns.hip, one answer per launch)
+  int stream_out;            // what the launch writes is stored past the caches on tiles of 128 (kStream128; BX) or 256 (kStream256)
+                             // (VAR_STREAM; rules of ns.hip, one answer per launch)
   uint16_t *Yh, *Yl;         // (E,M,N) next iterate as a bf16 pair   BX out, null on the last step
   float *X32;                // (E,M,N) fp32 result                   BX out on the last step, else null
   uint16_t *X16;             // (E,M,N) the result rounded to bf16, instead of X32

@@ -49,8 +49,12 @@
 #include "lds_dma.h"
 #include "ns_common.h"
 
-// Epilogue store: streaming, the written tile is not read again by this launch.
-template <typename T> __device__ __forceinline__ void epi_st(T *p, T v) { anc_st_stream(p, v); }
+// Epilogue store: the written tile is not read again by this launch, and past the caches it leaves them to the operands; kept
+// (STREAM false) where the next launch finds it there (NsGemm::stream_out).
+template <bool STREAM = true, typename T> __device__ __forceinline__ void epi_st(T *p, T v) {
+  if constexpr (STREAM) anc_st_stream(p, v);
+  else *p = v;
+}
 
 namespace {
 
@@ -92,6 +96,7 @@ __device__ __forceinline__ void mfma8_with(const bf16x8 (&a)[4], const bf16x8 (&
 // bj*32 + lane%32), packed two per dword: v[bj][i] = elements r = 2i (low half), 2i+1 (high).
 // `out` addresses the slab's first row in its first 32-column panel; the second panel lies pstride
 // elements further. The transposed slab is 64 rows of one panel.
+template <bool STREAM>
 __device__ __forceinline__ void stage_rows(unsigned char *region, const uint32_t (&v)[2][8], int lane,
                                            uint16_t *out, int64_t pstride) {
   uint16_t *t = (uint16_t *)region;                 // [32][72]
@@ -107,13 +112,14 @@ __device__ __forceinline__ void stage_rows(unsigned char *region, const uint32_t
   for (int p = 0; p < 4; ++p) {
     const int idx = p * 64 + lane, row = idx >> 3, c8 = (idx & 7) * 8;
     const anc_u32x4 q = *(const anc_u32x4 *)(t + row * 72 + c8);
-    epi_st((anc_u32x4 *)(out + (int64_t)(c8 >> 5) * pstride + row * 32 + (c8 & 31)), q);
+    epi_st<STREAM>((anc_u32x4 *)(out + (int64_t)(c8 >> 5) * pstride + row * 32 + (c8 & 31)), q);
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);
   __builtin_amdgcn_wave_barrier();
 }
 // Transposed: a lane's 4 consecutive rows are 4 consecutive elements of an output row, so they
 // go to LDS as one 8-byte write.
+template <bool STREAM>
 __device__ __forceinline__ void stage_cols(unsigned char *region, const uint32_t (&v)[2][8], int lane,
                                            uint16_t *outT) {
   uint16_t *t = (uint16_t *)region;                 // [64][40]
@@ -130,7 +136,7 @@ __device__ __forceinline__ void stage_cols(unsigned char *region, const uint32_t
   for (int p = 0; p < 4; ++p) {
     const int idx = p * 64 + lane, col = idx >> 2, r8 = (idx & 3) * 8;
     const anc_u32x4 q = *(const anc_u32x4 *)(t + col * 40 + r8);
-    epi_st((anc_u32x4 *)(outT + col * 32 + r8), q);
+    epi_st<STREAM>((anc_u32x4 *)(outT + col * 32 + r8), q);
   }
   __builtin_amdgcn_s_waitcnt(0xC07F);
   __builtin_amdgcn_wave_barrier();
@@ -953,7 +959,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
           const int idx = pz * 64 + lane, row = idx >> 3, c = idx & 7;
           const int off = row * 128 + ((c ^ ((row & 7) ^ ((row >> 3) & 1))) * 16);
           const anc_u32x4 qh = *(const anc_u32x4 *)(b + off);
-          epi_st((anc_u32x4 *)(p.Yh + y_off(row, c)), qh);
+          epi_st<VAR == VAR_STREAM>((anc_u32x4 *)(p.Yh + y_off(row, c)), qh);
         }
         if (!out8) {
 #pragma unroll
@@ -961,14 +967,14 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
             const int idx = pz * 64 + lane, row = idx >> 3, c = idx & 7;
             const int off = row * 128 + ((c ^ ((row & 7) ^ ((row >> 3) & 1))) * 16);
             const anc_u32x4 ql = *(const anc_u32x4 *)(b + 4096 + off);
-            epi_st((anc_u32x4 *)(p.Yl + y_off(row, c)), ql);
+            epi_st<VAR == VAR_STREAM>((anc_u32x4 *)(p.Yl + y_off(row, c)), ql);
           }
         } else {
           // one byte per element: the slab's 32 rows of a panel are 1 KiB contiguous
 #pragma unroll
           for (int pz = 0; pz < 2; ++pz) {
             const anc_u32x4 ql = *(const anc_u32x4 *)(b + 4096 + pz * 1024 + lane * 16);
-            epi_st((anc_u32x4 *)((char *)p.Yl + mn * 2 + ((int64_t)(gj0w / 32 + pz) * M + gi0) * 32 + l8_src), ql);
+            epi_st<VAR == VAR_STREAM>((anc_u32x4 *)((char *)p.Yl + mn * 2 + ((int64_t)(gj0w / 32 + pz) * M + gi0) * 32 + l8_src), ql);
           }
         }
       }
@@ -1097,18 +1103,18 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     const int64_t o_cols = mm + ((int64_t)(gi0 / 32) * M + gj0w) * 32;
     const int64_t ps = (int64_t)M * 32;
     if (EPI == EPI_GRAM) {
-      stage_rows(region, hv, lane, p.Fh + o_rows, ps);
-      if (mirror) stage_cols(region, hv, lane, p.Fh + o_cols);
+      stage_rows<VAR == VAR_STREAM>(region, hv, lane, p.Fh + o_rows, ps);
+      if (mirror) stage_cols<VAR == VAR_STREAM>(region, hv, lane, p.Fh + o_cols);
       if (write_lo) {
-        stage_rows(region, lv, lane, p.Fl + o_rows, ps);
-        if (mirror) stage_cols(region, lv, lane, p.Fl + o_cols);
+        stage_rows<VAR == VAR_STREAM>(region, lv, lane, p.Fl + o_rows, ps);
+        if (mirror) stage_cols<VAR == VAR_STREAM>(region, lv, lane, p.Fl + o_cols);
       }
     } else if (EPI == EPI_BMAT) {
-      stage_rows(region, hv, lane, p.Bh + o_rows, ps);
-      if (mirror) stage_cols(region, hv, lane, p.Bh + o_cols);
+      stage_rows<VAR == VAR_STREAM>(region, hv, lane, p.Bh + o_rows, ps);
+      if (mirror) stage_cols<VAR == VAR_STREAM>(region, hv, lane, p.Bh + o_cols);
       if (write_lo) {
-        stage_rows(region, lv, lane, p.Bl + o_rows, ps);
-        if (mirror) stage_cols(region, lv, lane, p.Bl + o_cols);
+        stage_rows<VAR == VAR_STREAM>(region, lv, lane, p.Bl + o_rows, ps);
+        if (mirror) stage_cols<VAR == VAR_STREAM>(region, lv, lane, p.Bl + o_cols);
       }
       __builtin_amdgcn_s_waitcnt(0xC07F);
       asm volatile("" ::: "memory");
@@ -1132,7 +1138,10 @@ int launch_sym(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s) {
     grid += t;
   }
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_big: grid out of range");
-  hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 4, 1>), dim3((unsigned)grid), dim3(512), 0, s, pm);
+  if (ps[0].stream_out & kStream256)
+    hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 4, 1, VAR_STREAM>), dim3((unsigned)grid), dim3(512), 0, s, pm);
+  else
+    hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 4, 1, VAR_NONE>), dim3((unsigned)grid), dim3(512), 0, s, pm);
   ANC_LAUNCH_CHECK();
   return ANC_OK;
 }
@@ -1190,6 +1199,11 @@ int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const N
       hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
     else
       hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+  } else if (ps[0].stream_out & kStream256) {
+    if (by_rows)
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_STREAM, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+    else
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_STREAM, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   } else {
     if (by_rows)
       hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_NONE, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);

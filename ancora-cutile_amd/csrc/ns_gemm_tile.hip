@@ -818,7 +818,7 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) 
     }
   }
   if constexpr (VAR == VAR_NONE && EPI == EPI_BX) {
-    if (tile == 128 && pm.g[0].stream_out) {
+    if (tile == 128 && (pm.g[0].stream_out & kStream128)) {
       hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 2, AT, VAR_STREAM, 4, false>), dim3(grid), dim3(256), 0, s, pm);
       return;
     }
