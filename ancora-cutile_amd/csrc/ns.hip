@@ -816,42 +816,49 @@ struct ChainProb {
   const anc_muon_desc_t *upd;  // or: the weights (E entries) the last step updates in its epilogue
 };
 
-// Tiles of a launch, from the number of 64x64 tiles it has (symmetric products: those on and below the diagonal),
-// problems weighted by their K against the longest (a launch ends with its longest tiles; short ones fill gaps). A CU
-// takes operand bytes into LDS at one rate whatever the tile, so small tiles finish first while they find idle CUs and
-// lose, by the bytes they fetch more often, once every CU has several; large ones lose where the last of them have
-// the chip to themselves. With residual terms a K tile brings three products, so small tiles hold out longer.
-// Measured, us per 5 launches on 64 / 128 / 256-wide tiles (tiles of 64):
-//   A = X X^T, mostly one term     4 x (1024,1024) 102 / 104 / 179 (544), 6 x 126 / 111 / 185 (816), 12 x 193 / 171 / 203
-//               (1632), 20 x 310 / 266 / 238 (2720);  3 x (1024,3072) 121 / 155 / 293 (408), 6 x 213 / 172 / 307 (816)
-//   residual terms                 20 x (512,1536) 178 / 191 / 392 (720), 18 x (640,1792) 257 / 315 (990), 16 x (768,768)
-//               172 / 183 / 251 (1248), 24 x 248 / 226 / 268 (1872), 30 x 329 / 320 / 286 (2340)
-//   just over one round of 256-wide tiles    26 x (1024,1024) 393 / 334 / 387 (260 of them), 48 x (768,768) 555 / 465 / 522
-//               (288), 33 x (1024,1024) 520 / 449 / 437 (330)
-//   X = a X + B X, mostly one term 2 x (1024,2048) 107 / 95 / 144 (1024), 5 x (1024,1024) 137 / 140 / 156 (1280), 6 x 156 / 147 /
-//               155 (1536), 5 x (1024,2048) 207 / 188 / 198 (2560), 4 x (1024,3072) 235 / 206 / 204 (3072),
-//               8 x (1024,2048) 303 / 258 / 233 (4096)
-//   residual terms                 8 x (512,1536) 136 / 139 / 159 (1536), 12 x 192 / 203 / 212 (2304), 16 x 241 / 221 / 229
-//               (3072), 20 x 291 / 273 / 267 (3840)
-//   just over one round of large tiles (4096)    6 x (1024,3072) 327 / 295 / 305 (4608), 20 x (1024,1024) 429 / 361 / 389
-//               (5120), 28 x (512,1536) 394 / 387 / 382 (5376), 8 x (1024,3072) 432 / 357 / 335 (6144)
+// Tiles of a launch, from the number of tiles it has (symmetric products: those on and below the diagonal), problems
+// weighted by their K against the longest (a launch ends with its longest tiles; short ones fill gaps). A CU takes
+// operand bytes into LDS at one rate whatever the tile, so small tiles finish first while they find idle CUs and lose,
+// by the bytes they fetch more often, once every CU has several; large ones lose where the last of them have the chip
+// to themselves. With residual terms a K tile brings three products, so small tiles hold out longer, and what counts
+// is how many rounds the 128-wide ones make: one per CU (symmetric products) or two (X = a X + B X), or just over that.
+// Measured, us per chain with the product on 64 / 128 / 256-wide tiles (tiles of 64, of 128):
+//   A and B, mostly one term       3 x (1024,1024) 238 / 261 / 424 (408, 108), 4 x 291 / 280 / 440 (544, 144), 10 x 527 / 503 / 572
+//               (1360, 360), 14 x (1024,2048) 901 / 791 / 853 (1904, 504), 16 x (1024,1024) 755 / 704 / 686 (2176, 576)
+//   residual terms                 16 x (512,1536) 444 / 458 (576, 160), 20 x 544 / 542 (720, 200), 14 x (640,1792) 655 / 615
+//               (770, 210), 16 x (640,640) 407 / 386 (880, 240), 9 x (896,896) 514 / 492 (945, 252), 18 x (640,1792) 773 / 849
+//               (990, 270), 16 x (768,768) 559 / 588 (1248, 336), 24 x (640,640) 540 / 531 (1320, 360), 20 x (768,768) 672 / 639
+//               (1560, 420)
+//   just over one round of 256-wide tiles    26 x (1024,1024) 393 / 334 / 387 (5 launches alone; 260 of them), 48 x (768,768)
+//               555 / 465 / 522 (288), 33 x (1024,1024) 520 / 449 / 437 (330)
+//   X = a X + B X, mostly one term 1 x (1024,2048) 163 / 171 (512, 128), 1 x (1536,1536) 281 / 275 (576, 144), 1 x (1024,3072) 199 /
+//               193 (768, 192; with the update of the weight 270 / 274), 3 x (1152,1152) 307 / 290 (972, 243), 5 x (1024,1024) 313 / 309 /
+//               326 (1280, 320), 6 x (1024,2048) 437 / 395 / 401 (3072, 768), 14 x (1024,1024) 653 / 595 / 584
+//               (3584, 896), 8 x (1024,2048) 596 / 528 / 506 (4096, 1024)
+//   residual terms                 12 x (640,640) 329 / 334 (1200, 300), 6 x (896,896) 389 / 401 (1176, 294), 24 x (512,512) 345 / 338 /
+//               381 (1536, 384), 12 x (768,768) 459 / 435 / 492 (1728, 432), 30 x (384,768) 346 / 353 (2160, 540), 24 x (640,640)
+//               549 / 530 (2400, 600), 16 x (512,1536) 476 / 441 / 483 (3072, 768), 24 x 647 / 605 / 682 (4608, 1152), 30 x 809 /
+//               777 / 799 (5760, 1440), 24 x (768,1536) 1324 / 1145 / 1147 (6912, 1728)
+//   just over one round of large tiles       18 x (1024,1024) 811 / 774 / 786 (4608), 20 x 890 / 825 / 809 (5120)
 int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
-  double longest = 0.0, t64 = 0.0, t256 = 0.0, several = 0.0;
+  double longest = 0.0, t64 = 0.0, t128 = 0.0, t256 = 0.0, several = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
   for (int k = 0; k < n; ++k) {
-    const double m = (double)(ps[k].M / 64), q = (double)ps[k].M / 256.0, w = (double)Es[k] * ((double)ps[k].K / longest);
+    const double m = (double)(ps[k].M / 64), h = (double)(ps[k].M / 128), q = (double)ps[k].M / 256.0;
+    const double w = (double)Es[k] * ((double)ps[k].K / longest);
     const double t = w * (epi == EPI_BX ? m * (double)(ps[k].N / 64) : m * (m + 1.0) / 2.0);
     t64 += t;
+    t128 += epi == EPI_BX ? t / 4.0 : w * (h * (h + 1.0) / 2.0);
     t256 += w * (q * (q + 1.0) / 2.0);
     if (ps[k].nterms > 1) several += t;
   }
   const bool terms = several > 0.5 * t64;
   if (epi != EPI_BX) {
-    if (t64 <= (terms ? 1300.0 : 520.0)) return 64;
+    if (terms ? t128 <= 205.0 || (t128 > 256.0 && t128 <= 345.0) : t64 <= 520.0) return 64;
     return t64 <= 2050.0 || (t256 > 256.0 && t256 <= 306.0) ? 128 : 256;
   }
-  if (t64 <= (terms ? 2350.0 : 1400.0) && (terms || !(t64 > 800.0 && t64 <= 1024.0))) return 64;
-  return t64 <= 3500.0 || (t64 > 4096.0 && t64 <= 5200.0) ? 128 : 256;
+  if (terms ? t128 <= 345.0 || (t128 > 512.0 && t128 <= 580.0) : t64 <= (ps[0].upd != nullptr ? 780.0 : 540.0)) return 64;
+  return t64 <= (terms && longest < 1024.0 ? 7000.0 : 3500.0) || (t64 > 4096.0 && t64 <= 4900.0) ? 128 : 256;
 }
 
 // The same for the bare product of weight gradients. Its K is a batch of tokens: short ones are bound by the

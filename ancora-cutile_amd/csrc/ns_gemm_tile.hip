@@ -9,8 +9,11 @@
 // 128), a quarter of the time although the operands are fetched four times as often. Which tile a
 // launch takes is a rule of ns.hip (pick_tile, pick_tile_plain).
 //
-// Layout. 4 wavefronts as 2x2, each WM x WN blocks of v_mfma_f32_32x32x16_bf16 (tile 64 WM x 64 WN). A stage is
-// KP = 2 (64x64) or 1 panels of 32 k of both operands, 16 KiB (12 KiB of a 128x64 tile). Operands arrive in pieces of 16
+// Layout. NW = 4 or 8 wavefronts as 2 x NW/2, each WM x WN blocks of v_mfma_f32_32x32x16_bf16 (tile 64 WM x 16 NW WN). 128x128 tiles run on
+// eight, four per SIMD with two workgroups on a CU: with half as many the matrix pipe was busy for 40 % of X = a X + B X of
+// the projections of six 640-wide layers, and a wavefront waiting for its fragments or storing its outputs for the rest (that step
+// 1230 -> 1201 us; chains of 24 x (512,512) on such tiles 354 -> 332, 42 x (640,640) 961 -> 913, 24 x (1152,1152) 1442 -> 1411).
+// A stage is KP = 2 (64x64) or 1 panels of 32 k of both operands, 16 KiB (12 KiB of a 128x64 tile). Operands arrive in pieces of 16
 // rows x 64 bytes, one LDS-DMA instruction each. Stages form a ring of four, two workgroups per CU (three of 128x64
 // tiles); 64x64 tiles that outnumber the CUs run on a ring of three, three workgroups per CU, whose
 // K loops and epilogues overlap (chains of five steps: 16 x (512,512) 358 -> 331 us, 4 x (1024,3072) 625 ->
@@ -77,12 +80,12 @@ template <int TM, int TN>
 __host__ __device__ constexpr int anc_sym_tiles(int rows) { return (TM / TN) * (rows * (rows + 1) / 2); }
 
 // SOLO: the launch has one problem, its arguments lie at fixed places.
-template <int EPI, int WM, int WN, bool AT, int VAR, int kRing, bool SOLO>
-__global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_tile(NsGemmArgs<SOLO ? 1 : kMaxGroups> pm) {
-  constexpr int TM = 64 * WM, TN = 64 * WN, KP = WM == 1 ? 2 : 1, TK = 32 * KP;
+template <int EPI, int WM, int WN, int NW, bool AT, int VAR, int kRing, bool SOLO>
+__global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) * NW / 4) k_ns_gemm_tile(NsGemmArgs<SOLO ? 1 : kMaxGroups> pm) {
+  constexpr int WC = NW / 2, TM = 64 * WM, TN = 32 * WN * WC, KP = WM == 1 ? 2 : 1, TK = 32 * KP;
   constexpr bool BT = EPI == EPI_BX, PLAINV = VAR == VAR_PLAIN;
   constexpr int kHalf = TM * TK * 2, kStageBytes = kHalf + TN * TK * 2;      // A's part of a stage, a stage
-  constexpr int PA = TM * KP / 64, PB = TN * KP / 64, kIps = PA + PB;        // DMA instructions per wavefront and stage
+  constexpr int PA = TM * KP / (16 * NW), PB = TN * KP / (16 * NW), kIps = PA + PB;        // DMA instructions per wavefront and stage
   static_assert(!AT || BT, "A by rows k: X = a X + B X and the plain product only");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing * kStageBytes];
 
@@ -125,7 +128,7 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
   if constexpr (!PLAINV) e = anc_ns_matrix(p, e);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / WC, wn = wave % WC;
   const int K = p.K, nk = (K + TK - 1) / TK;
   const int nterms = anc_ns_terms(p, e);
   // plain product only: K % 32 == 0, so with two panels per step the last step may hold one
@@ -200,10 +203,11 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
   using TrA = std::bool_constant<AT>;
   using TrB = std::bool_constant<BT>;
 
-  // ---- what the epilogue of X = a X + B X reads at the output position is requested here, so that it has arrived
-  // when the K loop ends (16 x (1024,3072) on 128-wide tiles: 828 -> 783 us per 5 launches against fetching it
-  // block by block behind the loop; B = b A + c A A, which reads half as much, lost 2 % that way on such launches). The loads are older than
-  // every DMA below, so the waits of the ring hold.
+  // ---- what the epilogue of X = a X + B X reads at the output position is requested before the K loop, so that it has
+  // arrived when the loop ends (16 x (1024,3072) on 128-wide tiles of four wavefronts: 828 -> 783 us per 5 launches against
+  // fetching it block by block behind the loop; B = b A + c A A, which reads half as much, lost 2 % that way on such
+  // launches). The loads are older than every DMA below, so the waits of the ring hold. Eight wavefronts have no
+  // registers for it (16 .. 32 would spill, 42 x (640,640) 913 -> 970) and request it behind the loop, all blocks at once.
   const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
   float *sg = (float *)lds + wave * 32 * kSgPitch;
   float sc = 1.0f;
@@ -227,7 +231,7 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
   constexpr int NB = WM * WN;
   uint32_t pre_h[NB][8], pre_l[NB][8];                  // 16 bf16, or (pre_l, 8-bit low halves) 16 bytes in the first 4
   float drow[WM][NR];
-  if constexpr (EPI == EPI_BX && !PLAINV) {
+  if constexpr (EPI == EPI_BX && !PLAINV && NW == 4) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const int64_t xo = mn + (p.x_panel ? pan_of(b) : (int64_t)(gi_w + (b / WN) * 32 + lrow) * N + gj_w + (b % WN) * 32 + c0);
@@ -421,16 +425,17 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
   } else {
     // ---- several terms: a step is one panel of 32 k of both halves of both operands, high stage then low stage.
     constexpr int kPanA = TM * 64, kPanB = TN * 64, kLow = kPanA + kPanB, kPair = 2 * kLow, kPairs = kRing * kStageBytes / kPair;
-    int64_t oA[WM], oB[WN], vA[WM], vB[WN];
+    constexpr int QA = TM / (16 * NW), QB = TN / (16 * NW);         // pieces per wavefront of a panel of A and of B
+    int64_t oA[QA], oB[QB], vA[QA], vB[QB];
 #pragma unroll
-    for (int j = 0; j < WM; ++j) {
-      const int q = wave * WM + j;
+    for (int j = 0; j < QA; ++j) {
+      const int q = wave * QA + j;
       oA[j] = (AT ? (q >> 1) * psA + (q & 1) * 16 * rpA : q * 16 * rpA);
       vA[j] = oA[j] + voA;
     }
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-      const int q = wave * WN + j;
+    for (int j = 0; j < QB; ++j) {
+      const int q = wave * QB + j;
       oB[j] = (BT ? (q >> 1) * psB + (q & 1) * 16 * rpB : q * 16 * rpB);
       vB[j] = oB[j] + voB;
     }
@@ -439,17 +444,17 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
     const int at_b = on_diag ? 0 : kPanA;
     auto terms = [&](auto nt, auto one_operand) {
       constexpr bool ONE = decltype(one_operand)::value;
-      constexpr int NT = decltype(nt)::value, kIpp = ONE ? 2 * WM : NT == 3 ? 2 * (WM + WN) : WM + 2 * WN;   // DMA instructions per wavefront and step
+      constexpr int NT = decltype(nt)::value, kIpp = ONE ? 2 * QA : NT == 3 ? 2 * (QA + QB) : QA + 2 * QB;   // DMA instructions per wavefront and step
       auto issue_pair = [&](unsigned char *st) {
 #pragma unroll
-        for (int j = 0; j < WM; ++j) {
-          dma(curA, oA[j], vA[j], voA, lds_addr(st + (wave * WM + j) * 1024));
-          if (NT == 3) dma(pAl, oA[j], vA[j], voA, lds_addr(st + kLow + (wave * WM + j) * 1024));
+        for (int j = 0; j < QA; ++j) {
+          dma(curA, oA[j], vA[j], voA, lds_addr(st + (wave * QA + j) * 1024));
+          if (NT == 3) dma(pAl, oA[j], vA[j], voA, lds_addr(st + kLow + (wave * QA + j) * 1024));
         }
 #pragma unroll
-        for (int j = 0; j < (ONE ? 0 : WN); ++j) {
-          dma(curB, oB[j], vB[j], voB, lds_addr(st + kPanA + (wave * WN + j) * 1024));
-          dma(pBl, oB[j], vB[j], voB, lds_addr(st + kLow + kPanA + (wave * WN + j) * 1024));
+        for (int j = 0; j < (ONE ? 0 : QB); ++j) {
+          dma(curB, oB[j], vB[j], voB, lds_addr(st + kPanA + (wave * QB + j) * 1024));
+          dma(pBl, oB[j], vB[j], voB, lds_addr(st + kLow + kPanA + (wave * QB + j) * 1024));
         }
         curA += adA; curB += adB; pAl += adA; pBl += adB;
       };
@@ -547,6 +552,29 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
     } else {
       terms(std::integral_constant<int, 3>{}, std::false_type{});
     }
+  }
+  // (the requests from above once more: as one lambda they cost the 64-wide kernels 40 instructions, 1 % of the chain of
+  // one (512,512) matrix)
+  if constexpr (EPI == EPI_BX && !PLAINV && NW > 4) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int64_t xo = mn + (p.x_panel ? pan_of(b) : (int64_t)(gi_w + (b / WN) * 32 + lrow) * N + gj_w + (b % WN) * 32 + c0);
+      const int64_t xr = p.x_panel ? RS * 32 : (int64_t)RS * N;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) ld_run<RUN * 2>(p.Xh + xo + r * xr, &pre_h[b][r * (RUN / 2)]);
+      if (in8) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          ld_run<RUN>((const char *)p.Xl + mn * 2 + pan_of(b) + r * RS * 32, &pre_l[b][r * (RUN / 4)]);
+      } else if (!p.lo_zero) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) ld_run<RUN * 2>(p.Xl + xo + r * xr, &pre_l[b][r * (RUN / 2)]);
+      }
+    }
+#pragma unroll
+    for (int bi = 0; bi < WM; ++bi)
+#pragma unroll
+      for (int r = 0; r < NR; ++r) drow[bi][r] = p.dB[mv + gi_w + bi * 32 + lrow + RS * r];
   }
   __syncthreads();
 
@@ -809,23 +837,33 @@ __global__ void __launch_bounds__(256, tile_per_cu(WM, WN, kRing)) k_ns_gemm_til
   }
 }
 
+// Weight gradients on 128x128 tiles, us at 288 / 432 / 768 / 1344 tiles of 64 (written), four / eight wavefronts: 768 tokens
+// 10.4 / 9.5, 10.7 / 9.4, 11.4 / 10.6, 17.4 / 17.5; 2048 tokens 17.8 / 16.4, 18.7 / 16.6, 19.2 / 18.5, 34.9 / 35.8; 8192 tokens
+// 54 / 52, 55 / 51, 61 / 57, 119 / 122, and 1024 tiles at 4096 tokens 36.8 / 39.7.
+constexpr int kLongPlain = 2048;
+
 template <int EPI, bool AT, int VAR>
 void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) {
   if constexpr (VAR == VAR_PLAIN) {
     if (tile == kTile128x64) {
-      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, 4, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+      return;
+    }
+    // (see kLongPlain)
+    if (tile == 128 && pm.g[0].K > kLongPlain) {
+      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 2, 4, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
       return;
     }
   }
   if constexpr (VAR == VAR_NONE && EPI == EPI_BX) {
     if (tile == 128 && (pm.g[0].stream_out & kStream128)) {
-      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 2, AT, VAR_STREAM, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, 8, AT, VAR_STREAM, 4, false>), dim3(grid), dim3(512), 0, s, pm);
       return;
     }
   }
-  if (tile == 128)      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 2, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
-  else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, AT, VAR, 3, false>), dim3(grid), dim3(256), 0, s, pm);
-  else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
+  if (tile == 128)      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, 8, AT, VAR, 4, false>), dim3(grid), dim3(512), 0, s, pm);
+  else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 3, false>), dim3(grid), dim3(256), 0, s, pm);
+  else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
   else {
     NsGemmArgs<1> one;
     one.n = 1;
@@ -835,7 +873,7 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) 
     one.sr = pm.sr;
     one.seed_base = pm.seed_base;
     one.ctl = pm.ctl;
-    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, AT, VAR, 4, true>), dim3(grid), dim3(256), 0, s, one);
+    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 4, true>), dim3(grid), dim3(256), 0, s, one);
   }
 }
 

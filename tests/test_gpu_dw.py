@@ -413,6 +413,14 @@ def test_tiles_of_128x64(gpu, T, K, N, n, accumulate):
     xd.free()
 
 
+@pytest.mark.parametrize("T,K,N,n", [(672, 1152, 2048, 1), (800, 640, 1792, 2), (2048, 1152, 2048, 1), (2080, 1152, 2048, 1)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_tiles_of_128(gpu, T, K, N, n, accumulate):
+    """513 .. 1024 tiles of 64 beyond 640 tokens run on 128x128 tiles, of eight wavefronts up to 2048 tokens and of four
+    beyond."""
+    test_tiles_of_128x64(gpu, T, K, N, n, accumulate)
+
+
 @pytest.mark.parametrize("T", [96, 384, 416])
 @pytest.mark.parametrize("K,N,n", [(640, 768, 1), (1024, 1024, 3), (1024, 1024, 5), (1024, 1280, 7), (2048, 1536, 5)])
 @pytest.mark.parametrize("accumulate", [False, True])
