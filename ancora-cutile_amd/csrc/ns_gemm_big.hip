@@ -36,7 +36,7 @@
 // iterate for X = a X + B X, the diagonal vectors) arrives by LDS-DMA in buffers private to the
 // wavefront, two 32-row slabs ahead; a slab waits with an exact vmcnt for its own fetch only.
 // bf16 outputs are converted with v_cvt_pk_bf16_f32 and pass through LDS so that rows and
-// mirrored rows leave as 16-byte nontemporal stores. X = a X + B X issues its MFMAs with the
+// mirrored rows leave as 16-byte stores, past the caches where they are many (NsGemm::stream_out). X = a X + B X issues its MFMAs with the
 // operands exchanged (transposed accumulator layout: a lane holds runs of 4 consecutive columns
 // of one output row) and reads and writes LDS 8 or 16 bytes at a time.
 //

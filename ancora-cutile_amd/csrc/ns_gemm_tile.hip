@@ -3,11 +3,11 @@
 // weight-gradient GEMM on the same tiles and on 128x64 ones: for launches that the 256-wide tiles of ns_gemm_big.hip
 // would leave most of the chip idle, and for dims that are multiples of 128 only.
 //
-// What bounds it. Operand bytes come into LDS at about 24 B per clock and CU whatever the tile, so a
-// product lasts as long as the CU with the most tiles needs for its operands: a single 1024x1024
-// output is 10 tiles of 256x256 (10 CUs at work, 512 K-bytes each step) or 160 of 64x64 (160 CUs,
-// 128), a quarter of the time although the operands are fetched four times as often. Which tile a
-// launch takes is a rule of ns.hip (pick_tile, pick_tile_plain).
+// What bounds it. Operand bytes come into LDS at some 20 .. 25 B per clock and CU with the L2 hits these launches have (50 .. 58
+// where all hit, 12 where none does), and a wavefront has its instructions to issue, so a product lasts as long as the
+// CU with the most tiles needs: a single 1024x1024 output is 10 tiles of 256x256 (10 CUs at work, 512 K-bytes each
+// step) or 136 of 64x64 (136 CUs, 128), a quarter of the time although the operands are fetched four times as
+// often. Which tile a launch takes is a rule of ns.hip (pick_tile, pick_tile_plain).
 //
 // Layout. NW = 4 or 8 wavefronts as 2 x NW/2, each WM x WN blocks of v_mfma_f32_32x32x16_bf16 (tile 64 WM x 16 NW WN). 128x128 tiles run on
 // eight, four per SIMD with two workgroups on a CU: with half as many the matrix pipe was busy for 40 % of X = a X + B X of
@@ -61,7 +61,7 @@ __device__ __forceinline__ void st_run(void *p, const uint32_t *w) {
 }
 
 // What the weight update reads and writes once: past the caches where a launch has many tiles (WIDE: the 128-wide ones), so
-// that the operands stay in them. The full step of a model of 4 layers, hidden size 512: 602 -> 576 us, its last product 82 -> 59.
+// that the operands stay in them. The full step of a model of 4 layers, hidden size 512: 602 -> 576 us.
 template <bool WIDE, typename T> __device__ __forceinline__ T ld_once(const T *p) {
   if constexpr (WIDE) return anc_ld_stream(p);
   else return *p;
