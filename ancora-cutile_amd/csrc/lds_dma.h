@@ -18,7 +18,12 @@ __device__ __forceinline__ void dma16(const void *g, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(g)
                : "memory", "m0");
 }
-// The same from a wavefront-uniform address and 32-bit offsets per lane: no 64-bit addition in vector registers. The
+// The same for bytes that nobody reads again: the first to leave the caches.
+__device__ __forceinline__ void dma16_once(const void *g, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds_base), "v"(g)
+               : "memory", "m0");
+}
+// The same as the first from a wavefront-uniform address and 32-bit offsets per lane: no 64-bit addition in vector registers. The
 // address is copied by a scalar instruction, which is the wait state that the write of M0 needs and makes it safe to
 // use at once even where a vector instruction (v_readfirstlane) has just produced it.
 __device__ __forceinline__ void dma16(const void *g, uint32_t off, uint32_t lds_base) {

@@ -144,7 +144,11 @@ __device__ __forceinline__ void stage_cols(unsigned char *region, const uint32_t
 
 constexpr int kStageRegion = 6144;      // bytes of epilogue staging per wavefront (>= 64*40*2)
 
-__device__ __forceinline__ void dma16_epi(const void *g, uint32_t lds_base) { dma16(g, lds_base); }
+template <bool ONCE = false>
+__device__ __forceinline__ void dma16_epi(const void *g, uint32_t lds_base) {
+  if constexpr (ONCE) dma16_once(g, lds_base);
+  else dma16(g, lds_base);
+}
 
 // VAR (X = a X + B X only) selects a variant of the epilogue as its own instantiation, so that
 // the extra registers and branches do not weigh on the other launches: VAR_UPDATE applies the
@@ -608,6 +612,9 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   // 4-byte accesses below (rows 8 apart would otherwise meet in one bank four at a time).
   const int l8_src = (lane >> 1) * 32 + (((lane & 1) ^ ((lane >> 4) & 1)) * 16);
   const int64_t lo_at = p.lo_zero ? 0 : -1;                 // (no low half: every read goes to one zeroed piece)
+  // Low halves that are no operand are read once, here (chains of 24 x (1024,3072) 1600 -> 1563 us, the full step of the Qwen3-0.6B set
+  // 12611 -> 12591; where they are one 20 x (768,2304) 1412 -> 1440).
+  const bool low_once = nterms == 1;
   auto fetch_in = [&](int bi) {
     const int64_t ub = x_pan ? mn * 2 + (int64_t)(gj0w / 32) * panel + (int64_t)(gi0w + bi * 32) * 64
                              : (mn + (int64_t)(gi0w + bi * 32) * N + gj0w) * 2;
@@ -617,15 +624,21 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       const int64_t ro = (int64_t)(8 * j) * in_row;
       const uint32_t vo = (j & 1) ? vo_in1 : vo_in0;
       dma16_epi((const char *)p.Xh + ub + ro + vo, lds_addr(b + j * 1024));
-      if (!in8) dma16_epi((const char *)p.Xl + ((ub + ro) & lo_at) + (vo & (uint32_t)lo_at), lds_addr(b + 4096 + j * 1024));
+      if (!in8) {
+        const char *q = (const char *)p.Xl + ((ub + ro) & lo_at) + (vo & (uint32_t)lo_at);
+        if (low_once) dma16_epi<true>(q, lds_addr(b + 4096 + j * 1024));
+        else          dma16_epi(q, lds_addr(b + 4096 + j * 1024));
+      }
     }
     if (in8) {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        dma16_epi((const char *)p.Xl + mn * 2 + ((int64_t)(gj0w / 32 + j) * M + gi0w + bi * 32) * 32 + l8_src,
+        dma16_epi<true>((const char *)p.Xl + mn * 2 + ((int64_t)(gj0w / 32 + j) * M + gi0w + bi * 32) * 32 + l8_src,
                   lds_addr(b + 4096 + j * 1024));
     }
   };
+  // (A32 is read once: of a large batch the first to leave the caches, 48 x (1024,1024) 1799 -> 1772 us per chain; of 16 that is 704 ->
+  // 706.)
   // B = b A + c A A reads A32 at the output position the same way: a 32x64 fp32 slab is 32 rows
   // of 256 bytes, 8 DMA instructions (4 rows each, lane -> row lane/16, chunk lane%16), chunk
   // index XORed with 8*((row>>2)&1).
@@ -636,7 +649,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
     unsigned char *b = inbuf(bi);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      dma16_epi((const char *)p.A32 + ub + (int64_t)(4 * j) * M * 4 + ((j & 1) ? vo_a1 : vo_a0), lds_addr(b + j * 1024));
+      dma16_epi<VAR == VAR_STREAM>((const char *)p.A32 + ub + (int64_t)(4 * j) * M * 4 + ((j & 1) ? vo_a1 : vo_a0), lds_addr(b + j * 1024));
   };
   // Without an fp32 copy of A (see NsGemm::a32_gated) B takes the off-diagonal entries of A from
   // Fh: in panel layout a 32x64 slab is 32 rows of two panels, 2 KiB contiguous each, 4 DMA
