@@ -906,7 +906,9 @@ int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
 // 40 x (512,1536) 1018 / 1011, 20 x (768,2304) 1436 / 1429.
 // A and B on 256-wide tiles: kept up to 24 Mi elements. 16 x (1024,1024) 667 / 684, 20 x (1024,1024) 793 / 815, 24 x (1024,1024)
 // 899 / 900, 24 x (1024,2048) 1134 / 1153; 32 x (1024,1024) 1338 / 1335, 40 x (1024,1024) 1539 / 1522, 12 x (1536,1536) 1264 / 1252.
-constexpr int64_t kStreamPair = 90 << 20, kKeepSquare = 24 << 20;
+// The fp32 copy of A that B reads on 128-wide tiles, from 22 Mi elements on: 42 x (640,640) (16 Mi) 888 / 891, 30 x (896,896) (23 Mi)
+// 1434 / 1421, 60 x (640,640) (23 Mi) 1208 / 1198, 24 x (1152,1152) (30 Mi) 1353 / 1308; 12 x (768,768) 419 / 430.
+constexpr int64_t kStreamPair = 90 << 20, kKeepSquare = 24 << 20, kKeepA32 = 22 << 20;
 
 // What a mode's tile flags ask for (0: nothing).
 int forced_tile(int flags) {
@@ -1039,6 +1041,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
     for (int q = 0; q < n; ++q) {
       gx[q].stream_out = (reader != 64 && pair >= kStreamPair ? kStream128 : 0) | (reader == 256 || terms ? kStream256 : 0);
       ga[q].stream_out = gb[q].stream_out = square > kKeepSquare ? kStream256 : 0;
+      if (square > kKeepA32) gb[q].stream_out |= kStream128;
     }
     {
       AncProfScope prof(ANC_PROF_NS_GRAM, s);

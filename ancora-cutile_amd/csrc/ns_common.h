@@ -85,7 +85,8 @@ struct NsGemm {
   const uint16_t *Xh, *Xl;   // (E,M,N) current iterate as a bf16 pair, X = Xh + Xl   BX in
   int lo_zero;               // the input has no low half (a bf16 matrix): Xl is one zeroed 16-byte piece that every
                              // read of a low half goes to
-  int stream_out;            // what the launch writes is stored past the caches on tiles of 128 (kStream128; BX) or 256 (kStream256)
+  int stream_out;            // past the caches: on tiles of 256 (kStream256) what the launch writes, on tiles of 128 (kStream128) the
+                             // iterate that BX writes and the A32 that BMAT reads
                              // (VAR_STREAM; rules of ns.hip, one answer per launch)
   uint16_t *Yh, *Yl;         // (E,M,N) next iterate as a bf16 pair   BX out, null on the last step
   float *X32;                // (E,M,N) fp32 result                   BX out on the last step, else null

@@ -598,6 +598,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
 #pragma unroll
     for (int i = 0; i < 8; ++i) { x[2 * i] = __uint_as_float(u[i] << 16); x[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u); }
   };
+  constexpr bool kStreamX = EPI == EPI_BX && VAR == VAR_STREAM;
   // 16 floats -> bf16 runs at out + r * step, and the residuals at lo likewise if not null
   auto put_bf16 = [&](uint16_t *out, uint16_t *lo, int64_t step) {
     uint32_t h[8], l[8];
@@ -607,10 +608,10 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
       else h[i] = anc_pk_bf16(v[2 * i], v[2 * i + 1]);
     }
 #pragma unroll
-    for (int r = 0; r < NR; ++r) st_run<RUN * 2, VAR == VAR_STREAM>(out + r * step, h + r * (RUN / 2));
+    for (int r = 0; r < NR; ++r) st_run<RUN * 2, kStreamX>(out + r * step, h + r * (RUN / 2));
     if (lo != nullptr) {
 #pragma unroll
-      for (int r = 0; r < NR; ++r) st_run<RUN * 2, VAR == VAR_STREAM>(lo + r * step, l + r * (RUN / 2));
+      for (int r = 0; r < NR; ++r) st_run<RUN * 2, kStreamX>(lo + r * step, l + r * (RUN / 2));
     }
   };
 #pragma unroll
@@ -670,7 +671,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
           if (has_a32) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const anc_f32x4 w = kEarlyA ? a32[i] : *(const anc_f32x4 *)(p.A32 + mm + quad(i, M));
+              const anc_f32x4 w = kEarlyA ? a32[i] : ld_once<VAR == VAR_STREAM>((const anc_f32x4 *)(p.A32 + mm + quad(i, M)));
               a[4 * i] = w.x; a[4 * i + 1] = w.y; a[4 * i + 2] = w.z; a[4 * i + 3] = w.w;
             }
           } else {
@@ -826,8 +827,8 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
           }
 #pragma unroll
           for (int r = 0; r < NR; ++r) {
-            st_run<RUN * 2, VAR == VAR_STREAM>(p.Yh + mn + pan + r * pst, h + r * (RUN / 2));
-            st_run<RUN, VAR == VAR_STREAM>((char *)p.Yl + mn * 2 + pan + r * pst, q + r * (RUN / 4));
+            st_run<RUN * 2, kStreamX>(p.Yh + mn + pan + r * pst, h + r * (RUN / 2));
+            st_run<RUN, kStreamX>((char *)p.Yl + mn * 2 + pan + r * pst, q + r * (RUN / 4));
           }
         } else {
           put_bf16(p.Yh + mn + pan, p.Yl + mn + pan, pst);
@@ -855,7 +856,7 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) 
       return;
     }
   }
-  if constexpr (VAR == VAR_NONE && EPI == EPI_BX) {
+  if constexpr (VAR == VAR_NONE && EPI != EPI_GRAM) {
     if (tile == 128 && (pm.g[0].stream_out & kStream128)) {
       hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, 8, AT, VAR_STREAM, 4, false>), dim3(grid), dim3(512), 0, s, pm);
       return;

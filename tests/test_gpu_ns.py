@@ -225,10 +225,11 @@ def test_many_small_tiles_keep_the_bits(gpu, E, M, N, mode):
 
 @pytest.mark.parametrize("E,M,N,mode", [(159, 384, 384, "bf16"), (160, 384, 384, "bf16"), (160, 384, 384, "bf16_x3"),
                                         (46, 512, 1024, "bf16_t128"), (12, 1024, 2048, "bf16_t128"),
-                                        (12, 1024, 2048, "bf16"), (24, 1024, 1024, "bf16_t256"), (25, 1024, 1024, "bf16_t256")])
+                                        (12, 1024, 2048, "bf16"), (24, 1024, 1024, "bf16_t256"), (25, 1024, 1024, "bf16_t256"),
+                                        (18, 1152, 1152, "bf16")])
 def test_iterates_past_the_caches_keep_the_bits(gpu, E, M, N, mode):
     """Iterates of 90 MiB and more on 128-wide tiles, most on 256-wide ones, and A and B of more than 24 Mi elements are stored
-    past the caches: batches on both sides of these lines, and with an 8-bit low half. Every matrix has the bits
+    past the caches, and A's fp32 copy of more than 22 Mi elements is read past them on 128-wide ones: batches on both sides of these lines, and with an 8-bit low half. Every matrix has the bits
     it has alone, and meets the bar."""
     rng = np.random.default_rng(E + M + N)
     X = rng.standard_normal((E, M, N), dtype=np.float32)
