@@ -168,7 +168,8 @@ extern "C" int anc_fill_u32(uint64_t dptr, uint32_t value, int64_t n_words, uint
 }
 
 // From pinned memory into place, 16 bytes per lane and access; what is left over 16 bytes by bytes. The link bounds it
-// (50 GB/s of a large copy), or the launch. Against the runtime's copy, which hands over to another engine and back:
+// (50 GB/s of a large copy), or the launch. For uploads that are ordered on a caller's stream: it shares a hardware queue and
+// the compute units with other streams' kernels. Against the runtime's copy, which hands over to another engine and back:
 // between two kernels 28 KB 22.5 -> 9.4 us, 128 KB 24.9 -> 11.3, 512 KB 31.5 -> 18.2; in a row 512 KB 23.8 -> 14.5.
 template <int U>
 __global__ void __launch_bounds__(256) k_stage_in(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int64_t bytes) {
@@ -279,11 +280,12 @@ int slot_take(StageRing &r, hipStream_t s, StageSlot **out) {
   *out = mine;
   return ANC_OK;
 }
-int slot_fill(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
+// `kernel`: k_stage_in may do the transfer, else the runtime's copy does.
+int slot_fill(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool kernel) {
   if (slot.mem == nullptr) ANC_HIP(hipHostMalloc(&slot.mem, (size_t)kSlotBytes, hipHostMallocDefault));
   if (slot.done == nullptr) ANC_HIP(hipEventCreateWithFlags(&slot.done, hipEventDisableTiming));
   memcpy(slot.mem, src, (size_t)bytes);
-  if ((dst & 15) != 0) {
+  if (!kernel || (dst & 15) != 0) {
     ANC_HIP(hipMemcpyAsync((void *)dst, slot.mem, (size_t)bytes, hipMemcpyHostToDevice, s));
   } else if (bytes <= 128 << 10) {          // (few bytes: as many loads at once as there are)
     hipLaunchKernelGGL(k_stage_in<1>, dim3((unsigned)(bytes / 4096 + 1)), dim3(256), 0, s, (const uint8_t *)slot.mem, (uint8_t *)dst, bytes);
@@ -299,7 +301,7 @@ int slot_fill(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hip
   return ANC_OK;
 }
 // Up to a slot's worth: on return `src` may be reused and the copy into place is queued on `s`, or done.
-int stage_piece(StageRing &r, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
+int stage_piece(StageRing &r, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool kernel) {
   StageSlot *slot;
   if (int rc = slot_take(r, s, &slot)) return rc;
   if (slot == nullptr) {
@@ -307,7 +309,7 @@ int stage_piece(StageRing &r, uint64_t dst, const void *src, int64_t bytes, hipS
     ANC_HIP(hipStreamSynchronize(s));
     return ANC_OK;
   }
-  const int rc = slot_fill(*slot, dst, src, bytes, s);
+  const int rc = slot_fill(*slot, dst, src, bytes, s, kernel);
   std::lock_guard<std::mutex> lk(r.mu);
   slot->busy = rc == ANC_OK;
   slot->user = s;
@@ -337,12 +339,13 @@ int stage_forget(hipStream_t s) {
     }
   return ANC_OK;
 }
-// The ring's device is current.
-int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t bytes, hipStream_t s) {
+// The ring's device is current. On the ring's own stream (anc_upload_now) nothing may wait for other streams' kernels, as
+// k_stage_in would in a hardware queue it shares with them, or on a chip that they fill.
+int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool kernel) {
   const int64_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes;
   auto piece = [&](int64_t c) {
     const int64_t at = c * kSlotBytes, left = bytes - at;
-    return stage_piece(r, dst + (uint64_t)at, (const char *)src + at, left < kSlotBytes ? left : kSlotBytes, s);
+    return stage_piece(r, dst + (uint64_t)at, (const char *)src + at, left < kSlotBytes ? left : kSlotBytes, s, kernel);
   };
   if (bytes < kThreadedBytes) {
     for (int64_t c = 0; c < pieces; ++c)
@@ -383,7 +386,7 @@ extern "C" int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, ui
   StageScope on;
   if (int rc = on.enter(anc_stream(stream))) return rc;
   StageRing &r = g_ring[on.dev];
-  return stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream));
+  return stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream), true);
 }
 extern "C" int anc_upload_now(uint64_t dst, const void *src, int64_t bytes) {
   ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_upload_now: bad arguments");
@@ -396,7 +399,7 @@ extern "C" int anc_upload_now(uint64_t dst, const void *src, int64_t bytes) {
     if (r.own == nullptr) ANC_HIP(hipStreamCreateWithFlags(&r.own, hipStreamNonBlocking));
     ++r.own_users;
   }
-  int rc = stage_upload(r, on.dev, dst, src, bytes, r.own);
+  int rc = stage_upload(r, on.dev, dst, src, bytes, r.own, false);
   if (rc == ANC_OK)
     if (hipError_t e = hipStreamSynchronize(r.own)) rc = anc_hip_fail(e, "hipStreamSynchronize", __FILE__, __LINE__);
   std::lock_guard<std::mutex> lk(r.mu);
@@ -433,7 +436,7 @@ extern "C" int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint
     StageScope on;
     if (int rc = on.enter(anc_stream(stream))) return rc;
     StageRing &r = g_ring[on.dev];
-    if (int rc = stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream))) return rc;
+    if (int rc = stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream), true)) return rc;
   } else {
     // a state as it is set up, often memory that no one has touched yet: the runtime's own path takes its page
     // faults in larger pieces (622 MB of fresh zeros: 18 ms against 80 through the slots, 5 MB 0.1 ms less)

@@ -44,6 +44,7 @@ static Stream null_stream[4] = {{0}, {1}, {2}, {3}};
 static std::set<Event *> events;
 static std::map<char *, size_t> pinned;
 static int live_streams = 0;
+static bool chip_full = false;         // kernels do not start: their streams are held
 static std::set<Stream *> gone;        // destroyed streams (their memory is kept, so that no new one has their address)
 static thread_local int cur = 0;
 static thread_local hipError_t last = hipSuccess;
@@ -142,6 +143,7 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *m, hipStream_t *s
 hipError_t hipLaunchKernel(const void *, dim3, dim3, void **args, size_t, hipStream_t s) {
   const void *src = *(const void **)args[0];
   if (!is_pinned(src)) return ret(hipErrorInvalidValue);
+  if (chip_full) str(s)->held = true;
   return hipMemcpyAsync(*(void **)args[1], src, (size_t)*(int64_t *)args[2], hipMemcpyHostToDevice, s);
 }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }
@@ -296,9 +298,23 @@ static void streams_that_end() {
   CHECK(pinned.empty() && events.empty() && live_streams == 0);
 }
 
+// Kernels of other streams that hold every compute unit, or the hardware queue, do not hold uploads that are complete on return.
+static void now_waits_for_no_kernel() {
+  chip_full = true;
+  for (size_t n : {100u, 600u << 10, 9u << 20}) {
+    const std::vector<char> want = bytes(n, 1);
+    std::vector<char> a(n);
+    std::future<int> f = std::async(std::launch::async, [&] { return anc_upload_now((uint64_t)a.data(), want.data(), (int64_t)n); });
+    CHECK(soon(f) && f.get() == 0 && a == want);
+  }
+  CHECK(anc_staging_release() == 0);
+  CHECK(pinned.empty() && events.empty() && live_streams == 0);
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}, {"other_streams_do_not_wait", other_streams_do_not_wait},
-                                                   {"many_threads", many_threads}, {"capture", capture}, {"streams_that_end", streams_that_end}};
+                                                   {"many_threads", many_threads}, {"capture", capture}, {"streams_that_end", streams_that_end},
+                                                   {"now_waits_for_no_kernel", now_waits_for_no_kernel}};
   if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
   cases.at(argv[1])();
   printf("ok\n");
