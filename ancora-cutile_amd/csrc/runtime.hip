@@ -247,6 +247,17 @@ struct StageScope {
   }
 };
 
+// Does k_stage_in on device `dev` reach `dst`? The runtime's copy finds the owner of an address; a kernel writes it from the
+// stream's device, and memory of another device, or of none, is a fault there.
+bool kernel_reaches(uint64_t dst, int dev) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, (const void *)dst) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return at.type == hipMemoryTypeDevice && at.device == dev;
+}
+
 // A slot for an upload on `s`: *out stays null if work of other streams holds them all.
 int slot_take(StageRing &r, hipStream_t s, StageSlot **out) {
   *out = nullptr;
@@ -343,6 +354,7 @@ int stage_forget(hipStream_t s) {
 // k_stage_in would in a hardware queue it shares with them, or on a chip that they fill.
 int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool kernel) {
   const int64_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes;
+  kernel = kernel && kernel_reaches(dst, dev);
   auto piece = [&](int64_t c) {
     const int64_t at = c * kSlotBytes, left = bytes - at;
     return stage_piece(r, dst + (uint64_t)at, (const char *)src + at, left < kSlotBytes ? left : kSlotBytes, s, kernel);

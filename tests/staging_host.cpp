@@ -44,6 +44,8 @@ static Stream null_stream[4] = {{0}, {1}, {2}, {3}};
 static std::set<Event *> events;
 static std::map<char *, size_t> pinned;
 static int live_streams = 0;
+struct Region { size_t size; int dev; };
+static std::map<char *, Region> device_memory;       // allocations; any other address is memory of the current device, without an end
 static bool chip_full = false;         // kernels do not start: their streams are held
 static std::set<Stream *> gone;        // destroyed streams (their memory is kept, so that no new one has their address)
 static thread_local int cur = 0;
@@ -63,6 +65,12 @@ static void release(Stream *s) {
 static bool is_pinned(const void *p) {
   auto it = pinned.upper_bound((char *)p);
   return it != pinned.begin() && (--it, (char *)p < it->first + it->second);
+}
+static const Region *region_of(const void *p, char **base) {
+  auto it = device_memory.upper_bound((char *)p);
+  if (it == device_memory.begin() || (--it, (char *)p >= it->first + it->second.size)) return nullptr;
+  *base = it->first;
+  return &it->second;
 }
 static uint64_t handle(Stream *s) { return (uint64_t)s; }
 
@@ -108,6 +116,15 @@ hipError_t hipEventSynchronize(hipEvent_t e) {
   cv.wait(lk, [e] { return ((Event *)e)->done; });
   return hipSuccess;
 }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
+  std::lock_guard<std::mutex> lk(mu);
+  char *base;
+  const Region *r = region_of(p, &base);
+  *a = hipPointerAttribute_t{};
+  a->type = hipMemoryTypeDevice;
+  a->device = r != nullptr ? r->dev : cur;
+  return hipSuccess;
+}
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t s) {
   std::unique_lock<std::mutex> lk(mu);
   Stream *st = str(s);
@@ -143,6 +160,9 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *m, hipStream_t *s
 hipError_t hipLaunchKernel(const void *, dim3, dim3, void **args, size_t, hipStream_t s) {
   const void *src = *(const void **)args[0];
   if (!is_pinned(src)) return ret(hipErrorInvalidValue);
+  char *base;
+  const Region *r = region_of(*(void **)args[1], &base);
+  if (r != nullptr && r->dev != str(s)->dev) { printf("a kernel writes another device's memory\n"); fflush(stdout); _exit(1); }
   if (chip_full) str(s)->held = true;
   return hipMemcpyAsync(*(void **)args[1], src, (size_t)*(int64_t *)args[2], hipMemcpyHostToDevice, s);
 }
@@ -311,10 +331,27 @@ static void now_waits_for_no_kernel() {
   CHECK(pinned.empty() && events.empty() && live_streams == 0);
 }
 
+// Memory of another device than the stream's (or, without a stream, the current one): no kernel writes there.
+static void memory_of_another_device() {
+  Stream s{0};
+  for (size_t n : {112u, 600u << 10, 9u << 20}) {
+    const std::vector<char> want = bytes(n, 1);
+    std::vector<char> a(n), b(n), c(n), d(n);
+    for (std::vector<char> *v : {&a, &b, &c, &d}) device_memory[v->data()] = Region{n, 1};
+    CHECK(anc_upload_async((uint64_t)a.data(), want.data(), (int64_t)n, handle(&s)) == 0);
+    CHECK(anc_memcpy_h2d((uint64_t)b.data(), want.data(), (int64_t)n, handle(&s)) == 0);
+    CHECK(anc_upload_now((uint64_t)c.data(), want.data(), (int64_t)n) == 0);
+    CHECK(anc_upload_async((uint64_t)d.data(), want.data(), (int64_t)n, 0) == 0);
+    CHECK(a == want && b == want && c == want && d == want && cur == 0);
+    device_memory.clear();
+  }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}, {"other_streams_do_not_wait", other_streams_do_not_wait},
                                                    {"many_threads", many_threads}, {"capture", capture}, {"streams_that_end", streams_that_end},
-                                                   {"now_waits_for_no_kernel", now_waits_for_no_kernel}};
+                                                   {"now_waits_for_no_kernel", now_waits_for_no_kernel},
+                                                   {"memory_of_another_device", memory_of_another_device}};
   if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
   cases.at(argv[1])();
   printf("ok\n");
