@@ -296,18 +296,20 @@ int slot_fill(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hip
   if (slot.mem == nullptr) ANC_HIP(hipHostMalloc(&slot.mem, (size_t)kSlotBytes, hipHostMallocDefault));
   if (slot.done == nullptr) ANC_HIP(hipEventCreateWithFlags(&slot.done, hipEventDisableTiming));
   memcpy(slot.mem, src, (size_t)bytes);
+  hipError_t e;
   if (!kernel || (dst & 15) != 0) {
-    ANC_HIP(hipMemcpyAsync((void *)dst, slot.mem, (size_t)bytes, hipMemcpyHostToDevice, s));
-  } else if (bytes <= 128 << 10) {          // (few bytes: as many loads at once as there are)
-    hipLaunchKernelGGL(k_stage_in<1>, dim3((unsigned)(bytes / 4096 + 1)), dim3(256), 0, s, (const uint8_t *)slot.mem, (uint8_t *)dst, bytes);
-    ANC_LAUNCH_CHECK();
+    e = hipMemcpyAsync((void *)dst, slot.mem, (size_t)bytes, hipMemcpyHostToDevice, s);
   } else {
-    hipLaunchKernelGGL(k_stage_in<4>, dim3((unsigned)(bytes / 16384 + 1)), dim3(256), 0, s, (const uint8_t *)slot.mem, (uint8_t *)dst, bytes);
-    ANC_LAUNCH_CHECK();
+    // (a launch's own status: an error that someone else left on this thread says nothing about it)
+    void *args[] = {&slot.mem, &dst, &bytes};
+    const bool few = bytes <= 128 << 10;    // (as many loads at once as there are)
+    e = few ? hipLaunchKernel((const void *)k_stage_in<1>, dim3((unsigned)(bytes / 4096 + 1)), dim3(256), args, 0, s)
+            : hipLaunchKernel((const void *)k_stage_in<4>, dim3((unsigned)(bytes / 16384 + 1)), dim3(256), args, 0, s);
   }
-  if (hipError_t e = hipEventRecord(slot.done, s)) {
-    (void)hipStreamSynchronize(s);          // nothing marks the end of that copy
-    return anc_hip_fail(e, "hipEventRecord", __FILE__, __LINE__);
+  if (e == hipSuccess) e = hipEventRecord(slot.done, s);
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(s);          // nothing marks the end of a transfer that may be under way
+    return anc_hip_fail(e, "a transfer out of a slot", __FILE__, __LINE__);
   }
   return ANC_OK;
 }

@@ -347,11 +347,27 @@ static void memory_of_another_device() {
   }
 }
 
+// An error that someone else left on the thread is not an upload's: it succeeds, and its slot is not taken again before its
+// transfer has ended.
+static void errors_of_others() {
+  for (size_t n : {112u, 300u << 10}) {
+    Stream A{0};
+    const std::vector<char> first = bytes(n, 1), second = bytes(n, 2);
+    std::vector<char> a(n), b(n);
+    A.held = true;
+    last = hipErrorInvalidValue;
+    CHECK(anc_upload_async((uint64_t)a.data(), first.data(), (int64_t)n, handle(&A)) == 0);
+    CHECK(anc_upload_async((uint64_t)b.data(), second.data(), (int64_t)n, handle(&A)) == 0);
+    release(&A);
+    CHECK(a == first && b == second);
+  }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}, {"other_streams_do_not_wait", other_streams_do_not_wait},
                                                    {"many_threads", many_threads}, {"capture", capture}, {"streams_that_end", streams_that_end},
                                                    {"now_waits_for_no_kernel", now_waits_for_no_kernel},
-                                                   {"memory_of_another_device", memory_of_another_device}};
+                                                   {"memory_of_another_device", memory_of_another_device}, {"errors_of_others", errors_of_others}};
   if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
   cases.at(argv[1])();
   printf("ok\n");
