@@ -247,15 +247,22 @@ struct StageScope {
   }
 };
 
-// Does k_stage_in on device `dev` reach `dst`? The runtime's copy finds the owner of an address; a kernel writes it from the
-// stream's device, and memory of another device, or of none, is a fault there.
-bool kernel_reaches(uint64_t dst, int dev) {
+// Does k_stage_in on device `dev` reach `bytes` bytes from `dst`? The runtime's copy finds the owner of an address and refuses
+// what does not fit into the allocation; a kernel writes from the stream's device whatever it is given, and memory of
+// another device, or past an end, is a fault there.
+bool kernel_reaches(uint64_t dst, int64_t bytes, int dev) {
   hipPointerAttribute_t at{};
-  if (hipPointerGetAttributes(&at, (const void *)dst) != hipSuccess) {
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  hipError_t e = hipPointerGetAttributes(&at, (const void *)dst);
+  if (e == hipSuccess && (at.type != hipMemoryTypeDevice || at.device != dev)) return false;
+  if (e == hipSuccess) e = hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)dst);
+  if (e != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  return at.type == hipMemoryTypeDevice && at.device == dev;
+  const uint64_t before = dst - (uint64_t)base;
+  return before <= size && (uint64_t)bytes <= size - before;
 }
 
 // A slot for an upload on `s`: *out stays null if work of other streams holds them all.
@@ -356,7 +363,7 @@ int stage_forget(hipStream_t s) {
 // k_stage_in would in a hardware queue it shares with them, or on a chip that they fill.
 int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool kernel) {
   const int64_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes;
-  kernel = kernel && kernel_reaches(dst, dev);
+  kernel = kernel && kernel_reaches(dst, bytes, dev);
   auto piece = [&](int64_t c) {
     const int64_t at = c * kSlotBytes, left = bytes - at;
     return stage_piece(r, dst + (uint64_t)at, (const char *)src + at, left < kSlotBytes ? left : kSlotBytes, s, kernel);

@@ -5,6 +5,7 @@
 
 #include <chrono>
 #include <condition_variable>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -125,10 +126,21 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
   a->device = r != nullptr ? r->dev : cur;
   return hipSuccess;
 }
+hipError_t hipMemGetAddressRange(hipDeviceptr_t *b, size_t *size, hipDeviceptr_t p) {
+  std::lock_guard<std::mutex> lk(mu);
+  char *base = nullptr;
+  const Region *r = region_of(p, &base);
+  *b = r != nullptr ? base : nullptr;
+  *size = r != nullptr ? r->size : SIZE_MAX;
+  return hipSuccess;
+}
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t s) {
   std::unique_lock<std::mutex> lk(mu);
   Stream *st = str(s);
   if (st->capturing) return hipSuccess;                            // (recorded)
+  char *base;
+  const Region *r = region_of(dst, &base);
+  if (r != nullptr && (char *)dst + n > base + r->size) return ret(hipErrorInvalidValue);
   if (is_pinned(src)) { push(st, [=] { memcpy(dst, src, n); }); return hipSuccess; }
   cv.wait(lk, [st] { return !st->held; });                         // pageable: in the stream's turn, and blocking
   memcpy(dst, src, n);
@@ -163,6 +175,11 @@ hipError_t hipLaunchKernel(const void *, dim3, dim3, void **args, size_t, hipStr
   char *base;
   const Region *r = region_of(*(void **)args[1], &base);
   if (r != nullptr && r->dev != str(s)->dev) { printf("a kernel writes another device's memory\n"); fflush(stdout); _exit(1); }
+  if (r != nullptr && *(char **)args[1] + *(int64_t *)args[2] > base + r->size) {
+    printf("a kernel writes past an allocation\n");
+    fflush(stdout);
+    _exit(1);
+  }
   if (chip_full) str(s)->held = true;
   return hipMemcpyAsync(*(void **)args[1], src, (size_t)*(int64_t *)args[2], hipMemcpyHostToDevice, s);
 }
@@ -363,11 +380,31 @@ static void errors_of_others() {
   }
 }
 
+// What does not fit into its allocation is refused, and nothing behind it is touched; anywhere inside it fits.
+static void past_the_end() {
+  Stream s{0};
+  for (size_t n : {112u, 600u << 10, (9u << 20) - 4080})
+    for (size_t at : {0u, 16u, 32u}) {
+      const std::vector<char> want = bytes(n, 1), rest = bytes(64, 2);
+      std::vector<char> a(n + 64);
+      memcpy(a.data() + n, rest.data(), 64);
+      device_memory[a.data()] = Region{n, 0};
+      const uint64_t dst = (uint64_t)a.data() + at;
+      CHECK(anc_upload_async(dst, want.data(), (int64_t)(n - at), handle(&s)) == 0);
+      CHECK(memcmp(a.data() + at, want.data(), n - at) == 0);
+      CHECK(anc_upload_async(dst, want.data(), (int64_t)(n - at + 1), handle(&s)) != 0);
+      CHECK(anc_memcpy_h2d(dst, want.data(), (int64_t)(n - at + 64), handle(&s)) != 0);
+      CHECK(anc_upload_now(dst, want.data(), (int64_t)(n - at + 1)) != 0);
+      CHECK(memcmp(a.data() + n, rest.data(), 64) == 0);
+      device_memory.clear();
+    }
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}, {"other_streams_do_not_wait", other_streams_do_not_wait},
                                                    {"many_threads", many_threads}, {"capture", capture}, {"streams_that_end", streams_that_end},
                                                    {"now_waits_for_no_kernel", now_waits_for_no_kernel},
-                                                   {"memory_of_another_device", memory_of_another_device}, {"errors_of_others", errors_of_others}};
+                                                   {"memory_of_another_device", memory_of_another_device}, {"errors_of_others", errors_of_others}, {"past_the_end", past_the_end}};
   if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
   cases.at(argv[1])();
   printf("ok\n");
