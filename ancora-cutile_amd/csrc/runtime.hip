@@ -22,6 +22,7 @@ int anc_hip_fail(hipError_t e, const char *what, const char *file, int line) {
 extern "C" const char *anc_last_error(void) { return g_err; }
 
 // ---- per-launch profiler -------------------------------------------------------------
+#include <chrono>
 #include <mutex>
 #include <exception>
 #include <thread>
@@ -167,12 +168,17 @@ extern "C" int anc_fill_u32(uint64_t dptr, uint32_t value, int64_t n_words, uint
   return ANC_OK;
 }
 
+// A word in pinned memory that the host reads while the kernel may still run. It says that a block has read its part of
+// a slot, no more: nothing that it wrote has to be visible, so the store is not ordered behind it.
+__device__ __forceinline__ void stage_mark(uint32_t *mark) {
+  __hip_atomic_store(mark, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // From pinned memory into place, 16 bytes per lane and access; what is left over 16 bytes by bytes. The link bounds it
 // (50 GB/s of a large copy), or the launch. For uploads that are ordered on a caller's stream: it shares a hardware queue and
 // the compute units with other streams' kernels. Against the runtime's copy, which hands over to another engine and back:
 // between two kernels 28 KB 22.5 -> 9.4 us, 128 KB 24.9 -> 11.3, 512 KB 31.5 -> 18.2; in a row 512 KB 23.8 -> 14.5.
 template <int U>
-__global__ void __launch_bounds__(256) k_stage_in(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int64_t bytes) {
+__global__ void __launch_bounds__(256) k_stage_in(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int64_t bytes, uint32_t *mark) {
   const int64_t n = bytes / 16, i = (int64_t)blockIdx.x * (256 * U) + threadIdx.x;
   anc_u32x4 v[U];
 #pragma unroll
@@ -183,6 +189,12 @@ __global__ void __launch_bounds__(256) k_stage_in(const uint8_t *__restrict__ sr
     if (i + u * 256 < n) *((anc_u32x4 *)dst + i + u * 256) = v[u];
   const int64_t j = n * 16 + threadIdx.x;
   if (blockIdx.x == 0 && j < bytes) dst[j] = src[j];
+  __syncthreads();                          // (what went into a store has been read)
+  if (threadIdx.x == 0) stage_mark(mark + blockIdx.x);
+}
+// The same mark behind a copy of the runtime's.
+__global__ void __launch_bounds__(64) k_stage_mark(uint32_t *mark) {
+  if (threadIdx.x == 0) stage_mark(mark);
 }
 
 // ---- uploads through a ring of pinned slots ------------------------------------------------------
@@ -190,17 +202,23 @@ __global__ void __launch_bounds__(256) k_stage_in(const uint8_t *__restrict__ sr
 // 57, and blocks until everything before it on the stream is done. So a source is copied slot by slot into pinned
 // memory, the transfer of one slot (k_stage_in) under the copy into the next, and the call can return as soon as the last
 // slot is filled. 4 MiB: 132 -> 95 us (with the runtime's copies, k_stage_in is quicker still). A source beyond the caches is read at 32 GB/s by one thread, so from 8 MiB on
-// four threads copy. A slot is taken again once the event behind its last transfer has passed. An upload waits for
+// four threads copy. A slot is taken again once its last transfer has read it, which the transfer itself marks in the slot's
+// memory: an event keeps the address of the stream it was recorded on, and a query looks there, but a caller's stream
+// may be gone by then. (On the ring's own stream, where no kernel runs, an event it is.) An upload waits for
 // slots in use on its own stream, where its data queue up behind the same work anyway, and never for those of
 // another: if those hold all of them it goes the pageable way. No lock is held while anyone waits or copies.
 // Events and streams belong to a device, so every device has a ring of its own, shared by all threads and streams
 // (4 MiB, pinned slot by slot on first use, given back by anc_staging_release).
 namespace {
 constexpr int kSlots = 8, kCopyThreads = 4, kMaxDevices = 32;
-constexpr int64_t kSlotBytes = 512 << 10, kThreadedBytes = 8 << 20;
+constexpr int64_t kSlotBytes = 512 << 10, kThreadedBytes = 8 << 20, kFewBytes = 128 << 10;
+constexpr int kMarks = 64;         // words behind a slot's bytes
+constexpr int64_t stage_blocks(int64_t bytes) { return bytes <= kFewBytes ? bytes / 4096 + 1 : bytes / 16384 + 1; }
+static_assert(stage_blocks(kFewBytes) <= kMarks && stage_blocks(kSlotBytes) <= kMarks, "a mark per block");
 struct StageSlot {
   void *mem = nullptr;
   hipEvent_t done = nullptr;
+  int marks = 0;                 // the marks that the transfer under way sets; 0: it has the event
   hipStream_t user = nullptr;    // the stream of its last transfer,
   uint64_t turn = 0;             // the older the smaller
   bool busy = false;             // that transfer was not seen to end yet
@@ -265,6 +283,26 @@ bool kernel_reaches(uint64_t dst, int64_t bytes, int dev) {
   return before <= size && (uint64_t)bytes <= size - before;
 }
 
+uint32_t *slot_marks(const StageSlot &slot) { return (uint32_t *)((char *)slot.mem + kSlotBytes); }
+// hipErrorNotReady: the slot's transfer is under way.
+hipError_t slot_ended(const StageSlot &slot) {
+  if (slot.marks == 0) {
+    const hipError_t e = hipEventQuery(slot.done);
+    if (e == hipErrorNotReady) (void)hipGetLastError();        // (not an error: a launch check must not find it)
+    return e;
+  }
+  for (int i = 0; i < slot.marks; ++i)
+    if (__atomic_load_n(slot_marks(slot) + i, __ATOMIC_ACQUIRE) == 0u) return hipErrorNotReady;
+  return hipSuccess;
+}
+hipError_t slot_wait(const StageSlot &slot) {
+  if (slot.marks == 0) return hipEventSynchronize(slot.done);
+  for (int turn = 0; slot_ended(slot) != hipSuccess; ++turn)
+    if (turn < 2000) std::this_thread::yield();
+    else             std::this_thread::sleep_for(std::chrono::microseconds(20));
+  return hipSuccess;
+}
+
 // A slot for an upload on `s`: *out stays null if work of other streams holds them all.
 int slot_take(StageRing &r, hipStream_t s, StageSlot **out) {
   *out = nullptr;
@@ -274,12 +312,12 @@ int slot_take(StageRing &r, hipStream_t s, StageSlot **out) {
     for (StageSlot &slot : r.slot) {
       if (slot.taken) continue;
       if (slot.busy) {
-        const hipError_t e = hipEventQuery(slot.done);
-        if (e != hipSuccess) {
-          (void)hipGetLastError();          // (not this upload's error: a launch check must not find it)
-          if (e == hipErrorNotReady && slot.user == s && (mine == nullptr || slot.turn < mine->turn)) mine = &slot;
+        const hipError_t e = slot_ended(slot);
+        if (e == hipErrorNotReady) {
+          if (slot.user == s && (mine == nullptr || slot.turn < mine->turn)) mine = &slot;
           continue;
         }
+        ANC_HIP(e);
       }
       slot.busy = false;
       slot.taken = true;
@@ -289,7 +327,7 @@ int slot_take(StageRing &r, hipStream_t s, StageSlot **out) {
     if (mine == nullptr) return ANC_OK;
     mine->taken = true;
   }
-  const hipError_t e = hipEventSynchronize(mine->done);
+  const hipError_t e = slot_wait(*mine);
   if (e != hipSuccess) {
     std::lock_guard<std::mutex> lk(r.mu);
     mine->taken = false;
@@ -298,22 +336,26 @@ int slot_take(StageRing &r, hipStream_t s, StageSlot **out) {
   *out = mine;
   return ANC_OK;
 }
-// `kernel`: k_stage_in may do the transfer, else the runtime's copy does.
-int slot_fill(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool kernel) {
-  if (slot.mem == nullptr) ANC_HIP(hipHostMalloc(&slot.mem, (size_t)kSlotBytes, hipHostMallocDefault));
+// `own`: on the ring's own stream. `kernel`: k_stage_in may do the transfer, else the runtime's copy does.
+int slot_fill(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool own, bool kernel) {
+  if (slot.mem == nullptr) ANC_HIP(hipHostMalloc(&slot.mem, (size_t)kSlotBytes + 4 * kMarks, hipHostMallocCoherent));
   if (slot.done == nullptr) ANC_HIP(hipEventCreateWithFlags(&slot.done, hipEventDisableTiming));
   memcpy(slot.mem, src, (size_t)bytes);
+  kernel = kernel && !own && (dst & 15) == 0;
+  uint32_t *mark = slot_marks(slot);
+  slot.marks = own ? 0 : kernel ? (int)stage_blocks(bytes) : 1;
+  memset(mark, 0, 4 * (size_t)slot.marks);
+  // (launches return their own status: an error that someone else left on this thread says nothing about them)
   hipError_t e;
-  if (!kernel || (dst & 15) != 0) {
-    e = hipMemcpyAsync((void *)dst, slot.mem, (size_t)bytes, hipMemcpyHostToDevice, s);
+  if (kernel) {
+    void *args[] = {&slot.mem, &dst, &bytes, &mark};       // (few bytes: as many loads at once as there are)
+    e = hipLaunchKernel(bytes <= kFewBytes ? (const void *)k_stage_in<1> : (const void *)k_stage_in<4>, dim3((unsigned)slot.marks),
+                        dim3(256), args, 0, s);
   } else {
-    // (a launch's own status: an error that someone else left on this thread says nothing about it)
-    void *args[] = {&slot.mem, &dst, &bytes};
-    const bool few = bytes <= 128 << 10;    // (as many loads at once as there are)
-    e = few ? hipLaunchKernel((const void *)k_stage_in<1>, dim3((unsigned)(bytes / 4096 + 1)), dim3(256), args, 0, s)
-            : hipLaunchKernel((const void *)k_stage_in<4>, dim3((unsigned)(bytes / 16384 + 1)), dim3(256), args, 0, s);
+    e = hipMemcpyAsync((void *)dst, slot.mem, (size_t)bytes, hipMemcpyHostToDevice, s);
+    void *args[] = {&mark};
+    if (e == hipSuccess) e = own ? hipEventRecord(slot.done, s) : hipLaunchKernel((const void *)k_stage_mark, dim3(1), dim3(64), args, 0, s);
   }
-  if (e == hipSuccess) e = hipEventRecord(slot.done, s);
   if (e != hipSuccess) {
     (void)hipStreamSynchronize(s);          // nothing marks the end of a transfer that may be under way
     return anc_hip_fail(e, "a transfer out of a slot", __FILE__, __LINE__);
@@ -321,7 +363,7 @@ int slot_fill(StageSlot &slot, uint64_t dst, const void *src, int64_t bytes, hip
   return ANC_OK;
 }
 // Up to a slot's worth: on return `src` may be reused and the copy into place is queued on `s`, or done.
-int stage_piece(StageRing &r, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool kernel) {
+int stage_piece(StageRing &r, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool own, bool kernel) {
   StageSlot *slot;
   if (int rc = slot_take(r, s, &slot)) return rc;
   if (slot == nullptr) {
@@ -329,7 +371,7 @@ int stage_piece(StageRing &r, uint64_t dst, const void *src, int64_t bytes, hipS
     ANC_HIP(hipStreamSynchronize(s));
     return ANC_OK;
   }
-  const int rc = slot_fill(*slot, dst, src, bytes, s, kernel);
+  const int rc = slot_fill(*slot, dst, src, bytes, s, own, kernel);
   std::lock_guard<std::mutex> lk(r.mu);
   slot->busy = rc == ANC_OK;
   slot->user = s;
@@ -337,36 +379,14 @@ int stage_piece(StageRing &r, uint64_t dst, const void *src, int64_t bytes, hipS
   slot->taken = false;
   return rc;
 }
-// `s` is about to be destroyed. An event keeps the address of the stream it was last recorded on, and a query looks
-// there (uploads failed now and then with "an event last recorded in a capturing stream" after the second stream of
-// an optimizer was gone): slots last used on `s` wait for their copy and get a new event.
-int stage_forget(hipStream_t s) {
-  for (StageRing &r : g_ring)
-    for (StageSlot &slot : r.slot) {
-      {
-        std::lock_guard<std::mutex> lk(r.mu);
-        if (slot.taken || slot.done == nullptr || slot.user != s) continue;
-        slot.taken = true;
-      }
-      hipError_t e = slot.busy ? hipEventSynchronize(slot.done) : hipSuccess;
-      if (e == hipSuccess) e = hipEventDestroy(slot.done);
-      std::lock_guard<std::mutex> lk(r.mu);
-      slot.taken = false;
-      ANC_HIP(e);
-      slot.done = nullptr;
-      slot.user = nullptr;
-      slot.busy = false;
-    }
-  return ANC_OK;
-}
 // The ring's device is current. On the ring's own stream (anc_upload_now) nothing may wait for other streams' kernels, as
 // k_stage_in would in a hardware queue it shares with them, or on a chip that they fill.
-int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool kernel) {
+int stage_upload(StageRing &r, int dev, uint64_t dst, const void *src, int64_t bytes, hipStream_t s, bool own) {
   const int64_t pieces = (bytes + kSlotBytes - 1) / kSlotBytes;
-  kernel = kernel && kernel_reaches(dst, bytes, dev);
+  const bool kernel = !own && kernel_reaches(dst, bytes, dev);
   auto piece = [&](int64_t c) {
     const int64_t at = c * kSlotBytes, left = bytes - at;
-    return stage_piece(r, dst + (uint64_t)at, (const char *)src + at, left < kSlotBytes ? left : kSlotBytes, s, kernel);
+    return stage_piece(r, dst + (uint64_t)at, (const char *)src + at, left < kSlotBytes ? left : kSlotBytes, s, own, kernel);
   };
   if (bytes < kThreadedBytes) {
     for (int64_t c = 0; c < pieces; ++c)
@@ -407,7 +427,7 @@ extern "C" int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, ui
   StageScope on;
   if (int rc = on.enter(anc_stream(stream))) return rc;
   StageRing &r = g_ring[on.dev];
-  return stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream), true);
+  return stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream), false);
 }
 extern "C" int anc_upload_now(uint64_t dst, const void *src, int64_t bytes) {
   ANC_REQUIRE(dst != 0 && src != nullptr && bytes >= 0, "anc_upload_now: bad arguments");
@@ -420,7 +440,7 @@ extern "C" int anc_upload_now(uint64_t dst, const void *src, int64_t bytes) {
     if (r.own == nullptr) ANC_HIP(hipStreamCreateWithFlags(&r.own, hipStreamNonBlocking));
     ++r.own_users;
   }
-  int rc = stage_upload(r, on.dev, dst, src, bytes, r.own, false);
+  int rc = stage_upload(r, on.dev, dst, src, bytes, r.own, true);
   if (rc == ANC_OK)
     if (hipError_t e = hipStreamSynchronize(r.own)) rc = anc_hip_fail(e, "hipStreamSynchronize", __FILE__, __LINE__);
   std::lock_guard<std::mutex> lk(r.mu);
@@ -435,7 +455,7 @@ extern "C" int anc_staging_release(void) {
         if (slot.taken || slot.mem == nullptr) continue;       // (in use by a call: it stays)
         slot.taken = true;
       }
-      hipError_t e = slot.busy ? hipEventSynchronize(slot.done) : hipSuccess;
+      hipError_t e = slot.busy ? slot_wait(slot) : hipSuccess;
       if (e == hipSuccess && slot.done != nullptr) e = hipEventDestroy(slot.done);
       if (e == hipSuccess) e = hipHostFree(slot.mem);
       std::lock_guard<std::mutex> lk(r.mu);
@@ -457,7 +477,7 @@ extern "C" int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint
     StageScope on;
     if (int rc = on.enter(anc_stream(stream))) return rc;
     StageRing &r = g_ring[on.dev];
-    if (int rc = stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream), true)) return rc;
+    if (int rc = stage_upload(r, on.dev, dst, src, bytes, anc_stream(stream), false)) return rc;
   } else {
     // a state as it is set up, often memory that no one has touched yet: the runtime's own path takes its page
     // faults in larger pieces (622 MB of fresh zeros: 18 ms against 80 through the slots, 5 MB 0.1 ms less)
@@ -498,7 +518,6 @@ extern "C" int anc_stream_create_nonblocking(uint64_t *stream) {
 }
 extern "C" int anc_stream_destroy(uint64_t stream) {
   ANC_REQUIRE(stream != 0, "anc_stream_destroy: the null stream is not destroyable");
-  if (int rc = stage_forget(anc_stream(stream))) return rc;
   ANC_HIP(hipStreamDestroy(anc_stream(stream)));
   return ANC_OK;
 }

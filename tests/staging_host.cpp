@@ -13,6 +13,7 @@
 #include <functional>
 #include <future>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <set>
 #include <string>
@@ -63,6 +64,12 @@ static void release(Stream *s) {
   while (!s->queue.empty()) { s->queue.front()(); s->queue.pop_front(); }
   cv.notify_all();
 }
+static void look_at(Stream *s) {              // (in the runtime: at memory that is freed, or another stream's)
+  if (gone.count(s) == 0) return;
+  printf("a stream that is gone is looked at\n");
+  fflush(stdout);
+  _exit(1);
+}
 static bool is_pinned(const void *p) {
   auto it = pinned.upper_bound((char *)p);
   return it != pinned.begin() && (--it, (char *)p < it->first + it->second);
@@ -72,6 +79,10 @@ static const Region *region_of(const void *p, char **base) {
   if (it == device_memory.begin() || (--it, (char *)p >= it->first + it->second.size)) return nullptr;
   *base = it->first;
   return &it->second;
+}
+static std::string &kernel_of(const void *f) {       // (registered before this file's globals are made)
+  static std::map<const void *, std::string> *names = new std::map<const void *, std::string>;
+  return (*names)[f];
 }
 static uint64_t handle(Stream *s) { return (uint64_t)s; }
 
@@ -108,11 +119,13 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
 }
 hipError_t hipEventQuery(hipEvent_t e) {
   std::lock_guard<std::mutex> lk(mu);
-  if (((Event *)e)->captured || gone.count(((Event *)e)->on)) return ret(hipErrorCapturedEvent);     // (or anything else)
+  look_at(((Event *)e)->on);
+  if (((Event *)e)->captured) return ret(hipErrorCapturedEvent);
   return ((Event *)e)->done ? hipSuccess : ret(hipErrorNotReady);
 }
 hipError_t hipEventSynchronize(hipEvent_t e) {
   std::unique_lock<std::mutex> lk(mu);
+  look_at(((Event *)e)->on);
   if (((Event *)e)->captured) return ret(hipErrorCapturedEvent);
   cv.wait(lk, [e] { return ((Event *)e)->done; });
   return hipSuccess;
@@ -161,32 +174,35 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c) {
   *c = str(s)->capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
-// (the one kernel of these entry points copies: source, destination, bytes)
-struct Launch { dim3 grid, block; size_t shared; hipStream_t s; };
-static thread_local Launch launch;
-hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t m, hipStream_t s) { launch = {g, b, m, s}; return hipSuccess; }
-hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *m, hipStream_t *s) {
-  *g = launch.grid; *b = launch.block; *m = launch.shared; *s = launch.s;
-  return hipSuccess;
-}
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **args, size_t, hipStream_t s) {
-  const void *src = *(const void **)args[0];
-  if (!is_pinned(src)) return ret(hipErrorInvalidValue);
+// (the kernels of these entry points: k_stage_in copies, source, destination, bytes, and then sets a mark per block; k_stage_mark
+// sets one)
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **args, size_t, hipStream_t s) {
+  const bool copies = kernel_of(f).find("k_stage_in") != std::string::npos;
+  uint32_t *mark = *(uint32_t **)args[copies ? 3 : 0];
+  const void *src = copies ? *(const void **)args[0] : nullptr;
+  char *dst = copies ? *(char **)args[1] : nullptr;
+  const int64_t n = copies ? *(int64_t *)args[2] : 0;
+  std::lock_guard<std::mutex> lk(mu);
+  Stream *st = str(s);
+  if (!is_pinned(mark + grid.x - 1) || (copies && !is_pinned(src))) return ret(hipErrorInvalidValue);
   char *base;
-  const Region *r = region_of(*(void **)args[1], &base);
-  if (r != nullptr && r->dev != str(s)->dev) { printf("a kernel writes another device's memory\n"); fflush(stdout); _exit(1); }
-  if (r != nullptr && *(char **)args[1] + *(int64_t *)args[2] > base + r->size) {
-    printf("a kernel writes past an allocation\n");
-    fflush(stdout);
-    _exit(1);
-  }
-  if (chip_full) str(s)->held = true;
-  return hipMemcpyAsync(*(void **)args[1], src, (size_t)*(int64_t *)args[2], hipMemcpyHostToDevice, s);
+  const Region *r = region_of(dst, &base);
+  const char *fault = r == nullptr ? nullptr : r->dev != st->dev ? "a kernel writes another device's memory"
+                                             : dst + n > base + r->size ? "a kernel writes past an allocation" : nullptr;
+  if (fault != nullptr) { printf("%s\n", fault); fflush(stdout); _exit(1); }
+  if (chip_full) st->held = true;
+  push(st, [=] {
+    if (copies) memcpy(dst, src, (size_t)n);
+    for (unsigned i = 0; i < grid.x; ++i) mark[i] = 1;
+  });
+  return hipSuccess;
 }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }
 void **__hipRegisterFatBinary(const void *) { return nullptr; }
 void __hipUnregisterFatBinary(void **) {}
-void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, void *, void *, int *) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, void *, void *, int *) { kernel_of(f) = name; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipErrorInvalidValue; }        // (stubs of kernels launched otherwise)
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipErrorInvalidValue; }
 }
 
 // ---- the cases
@@ -318,7 +334,7 @@ static void streams_that_end() {
       CHECK(b == want && hipGetLastError() == hipSuccess);
     }
   }
-  // a stream that ends without the library's knowledge costs its slots, not the uploads after it
+  // a stream that ends without the library's knowledge
   Stream other{0};
   for (int i = 0; i < 3; ++i) {
     std::vector<char> b(n);
@@ -400,11 +416,45 @@ static void past_the_end() {
     }
 }
 
+// Streams that others made and destroyed leave every slot usable, also where a transfer was under way: nobody looks at
+// them again, and eight uploads on a stream that is held still find a slot each.
+static void streams_of_others() {
+  const size_t n = 100;
+  const std::vector<char> want = bytes(n, 1);
+  for (int round = 0; round < 3; ++round) {
+    std::vector<std::unique_ptr<Stream>> s;
+    std::vector<std::vector<char>> a(8, std::vector<char>(n + 4));
+    for (size_t i = 0; i < 8; ++i) {
+      s.emplace_back(new Stream{0});
+      s[i]->held = i % 2 != 0;
+      CHECK(anc_upload_async((uint64_t)a[i].data() + i / 2, want.data(), (int64_t)n, handle(s[i].get())) == 0);
+      gone.insert(s[i].get());
+    }
+    for (auto &x : s) release(x.get());
+    for (size_t i = 0; i < 8; ++i) CHECK(memcmp(a[i].data() + i / 2, want.data(), n) == 0);
+    Stream A{0};
+    A.held = true;
+    std::vector<std::vector<char>> b(8, std::vector<char>(n));
+    std::future<int> f = std::async(std::launch::async, [&] {
+      int rc = 0;
+      for (auto &x : b) rc |= anc_upload_async((uint64_t)x.data(), want.data(), (int64_t)n, handle(&A));
+      return rc;
+    });
+    CHECK(soon(f) && f.get() == 0);
+    release(&A);
+    for (auto &x : b) CHECK(x == want);
+    gone.clear();
+  }
+  CHECK(anc_staging_release() == 0);
+  CHECK(pinned.empty() && events.empty() && live_streams == 0);
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}, {"other_streams_do_not_wait", other_streams_do_not_wait},
                                                    {"many_threads", many_threads}, {"capture", capture}, {"streams_that_end", streams_that_end},
                                                    {"now_waits_for_no_kernel", now_waits_for_no_kernel},
-                                                   {"memory_of_another_device", memory_of_another_device}, {"errors_of_others", errors_of_others}, {"past_the_end", past_the_end}};
+                                                   {"memory_of_another_device", memory_of_another_device}, {"errors_of_others", errors_of_others}, {"past_the_end", past_the_end},
+                                                   {"streams_of_others", streams_of_others}};
   if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
   cases.at(argv[1])();
   printf("ok\n");
