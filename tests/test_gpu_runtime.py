@@ -81,6 +81,32 @@ def test_staged_uploads_arrive_whole(gpu, n, how):
     d.free()
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 4095, 4096, 4097, (128 << 10) - 1, 128 << 10, (128 << 10) + 1, 147456, (512 << 10) - 1])
+@pytest.mark.parametrize("at", [0, 1, 4, 8, 16])
+def test_staged_uploads_write_their_bytes_only(gpu, n, at):
+    """Around the size where the transfer kernel takes more bytes per lane, and into destinations on and off its 16-byte
+    alignment: the bytes arrive, those before and behind them stay. More uploads in a row than there are slots, and
+    streams that are gone when their slots are taken again."""
+    from ancora_cutile_amd import DevBuf
+    rng = np.random.default_rng(n + at)
+    rows = 20
+    d = DevBuf.zeros((rows, (n + 64 + 15) // 16 * 16), np.uint8)
+    want = rng.integers(0, 256, d.shape, dtype=np.uint8)
+    d.upload(want)
+    for turn in range(2):
+        s = gpu.stream_create()
+        for i in range(rows):
+            a = rng.integers(0, 256, n, dtype=np.uint8)
+            want[i, at:at + n] = a
+            gpu.api.anc_upload_async(d.ptr + i * d.shape[1] + at, a.ctypes.data, n, s)
+            a[:] = 0
+        gpu.stream_sync(s)
+        gpu.api.anc_stream_destroy(s)
+        assert np.array_equal(d.to_numpy(), want)
+    gpu.api.anc_staging_release()
+    d.free()
+
+
 def test_events_order_two_streams(gpu):
     """Stream B waits for an event recorded on stream A behind a long fill: B's copy sees the
     filled values; the elapsed time between two events around the fill is positive."""
