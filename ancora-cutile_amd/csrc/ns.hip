@@ -415,18 +415,48 @@ __global__ void __launch_bounds__(kThreads) k_ns_colstat(NsColArgs a) {
   }
 }
 static_assert(kColBlock % 64 == 0 && kColBlock <= kThreads, "k_ns_colstat: whole wavefronts of one lane per column in the final sum");
+// The wide gate's decision on matrix e, from its proxy's sum and, where that asks for them, the column norms
+__device__ __forceinline__ bool is_wide(const NsColArgs &a, int q, int e, double sum) {
+  const WideRule r = a.rule[q];
+  const double p = sum * (double)a.N[q];
+  if (p > r.lo && p < r.hi) return true;
+  if (!wants_colstat(r, p)) return false;
+  const double *c = a.part[q] + (int64_t)e * a.parts[q] * 2;
+  double s2 = c[0], s4 = c[1], lightest = c[0];
+#pragma unroll 16
+  for (int i = 1; i < a.parts[q]; ++i) {
+    const double x2 = c[2 * i], x4 = c[2 * i + 1];
+    s2 = s2 + x2;
+    s4 = s4 + x4;
+    lightest = x2 < lightest ? x2 : lightest;
+  }
+  const double colc = s2 > 0.0 ? (double)a.N[q] * s4 / (s2 * s2) : 1.0;
+  // outlier columns: the share of the mass outside them, from the lightest block of columns
+  const double bulk = s2 > 0.0 ? (double)a.parts[q] * lightest / s2 : 1.0;
+  if (p < r.hi && r.near_diff > 0.0) return p - colc > r.near_diff;
+  return colc < kColcFrac * p || (p >= r.hi && bulk < kBulkShare);
+}
+// The flag alone, one wavefront per matrix: for batches that no gated launch takes in another order.
+__global__ void __launch_bounds__(kThreads) k_ns_classify(NsColArgs a) {
+  int e = (int)(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6)), q = 0;
+  while (q + 1 < a.n && e >= a.blocks[q]) { e -= a.blocks[q]; ++q; }
+  if (e >= a.blocks[q]) return;
+  const double sum = cond_sum(a.cond[q] + (int64_t)e * kCondParts);
+  if ((threadIdx.x & 63) != 0) return;
+  a.sum[q][e] = sum;
+  if (a.flag[q] != nullptr) a.flag[q][e] = is_wide(a, q, e, sum) ? 1 : 0;
+}
 // One block per batch: the wide gate's flag per matrix, and the order in which the launches of a gated
 // iteration take the matrices. A matrix that takes a gate's terms has three times the products of one that does not;
 // such matrices lie together (the tall weights of a stack) and a launch's sequence is cut into eight runs, one per XCD,
 // so they are dealt over the runs in turn, each run's first. (Qwen3-0.6B set, 59 of 196 matrices gated, A = X X^T of
-// iteration 2: 1114 -> 729 us.)
+// iteration 2: 1114 -> 729 us, for 1 to 3 us that this kernel takes longer than k_ns_classify.)
 constexpr int kClassifyThreads = 1024, kMaxOrdered = 8192;
-__global__ void __launch_bounds__(kClassifyThreads) k_ns_classify(NsColArgs a) {
+__global__ void __launch_bounds__(kClassifyThreads) k_ns_classify_order(NsColArgs a) {
   constexpr int kWaves = kClassifyThreads / 64, kAhead = 4;
   __shared__ uint8_t heavy[kMaxOrdered];
   __shared__ int count[kWaves];
-  const int q = (int)blockIdx.x, E = a.blocks[q], N = a.N[q], wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
-  const WideRule r = a.rule[q];
+  const int q = (int)blockIdx.x, E = a.blocks[q], wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
   for (int e0 = wave; e0 < E; e0 += kWaves * kAhead) {
     double parts[kAhead];
 #pragma unroll
@@ -444,28 +474,9 @@ __global__ void __launch_bounds__(kClassifyThreads) k_ns_classify(NsColArgs a) {
   }
   __syncthreads();
   for (int e = (int)threadIdx.x; e < E; e += kClassifyThreads) {      // (a matrix per lane)
-    const double sum = a.sum[q][e], p = sum * (double)N;
-    bool wide = false;
-    if (a.flag[q] != nullptr) {
-      wide = p > r.lo && p < r.hi;
-      if (!wide && wants_colstat(r, p)) {
-        const double *c = a.part[q] + (int64_t)e * a.parts[q] * 2;
-        double s2 = c[0], s4 = c[1], lightest = c[0];
-#pragma unroll 16
-        for (int i = 1; i < a.parts[q]; ++i) {
-          const double x2 = c[2 * i], x4 = c[2 * i + 1];
-          s2 = s2 + x2;
-          s4 = s4 + x4;
-          lightest = x2 < lightest ? x2 : lightest;
-        }
-        const double colc = s2 > 0.0 ? (double)N * s4 / (s2 * s2) : 1.0;
-        // outlier columns: the share of the mass outside them, from the lightest block of columns
-        const double bulk = s2 > 0.0 ? (double)a.parts[q] * lightest / s2 : 1.0;
-        if (p < r.hi && r.near_diff > 0.0) wide = p - colc > r.near_diff;
-        else wide = colc < kColcFrac * p || (p >= r.hi && bulk < kBulkShare);
-      }
-      a.flag[q][e] = wide ? 1 : 0;
-    }
+    const double sum = a.sum[q][e];
+    const bool wide = a.flag[q] != nullptr && is_wide(a, q, e, sum);
+    if (a.flag[q] != nullptr) a.flag[q][e] = wide ? 1 : 0;
     if (e < kMaxOrdered) heavy[e] = wide || sum > a.gate[q] ? 1 : 0;
   }
   __syncthreads();
@@ -929,6 +940,12 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
   for (int q = 0; q < n; ++q) { curH[q] = cp[q].inH; curL[q] = cp[q].inL; nxt[q] = cp[q].nxt; Es[q] = cp[q].E; }
   bool want_cond = false;      // some later iteration gates a product on the proxy
   for (int q = 0; q < n; ++q) want_cond = want_cond || cp[q].pl.sp.any_gate(steps);
+  // the matrices are dealt over the launches' runs (k_ns_classify_order) where a gate picks some of several
+  auto ordered = [&](int q) {
+    bool gated = false;
+    for (int j = 1; j < steps; ++j) gated = gated || cp[q].pl.sp.gated(j);
+    return gated && cp[q].E > 1;
+  };
   double l8_cur[kMaxGroups];   // the proxy bound the current iterate's 8-bit low halves were written with (0: none)
   for (int q = 0; q < n; ++q) l8_cur[q] = 0.0;
   for (int k = 0; k < steps; ++k) {
@@ -971,7 +988,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       if (gated) {
         ga[q].cond = pl.cond;
         ga[q].cond_thresh = (double)pl.sp.gate_tau[k] / (double)N;
-        ga[q].order = pl.order;
+        ga[q].order = ordered(q) ? pl.order : nullptr;
         ga[q].nterms_hard = 3;
       }
       if (wide_g) set_wide(ga[q], 3);
@@ -1001,7 +1018,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       if (gated && ((pl.sp.gate_bx >> k) & 1u) && !split_fb) {
         gx[q].cond = pl.cond;
         gx[q].cond_thresh = (double)pl.sp.gate_tau[k] / (double)N;
-        gx[q].order = pl.order;
+        gx[q].order = ordered(q) ? pl.order : nullptr;
         gx[q].nterms_hard = 2;
       }
       if (wide_a) set_wide(gx[q], 3);
@@ -1063,16 +1080,18 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       ANC_LAUNCH_CHECK();
       // the wide gate's decision per matrix, from the proxy and, where it asks, the column norms
       NsColArgs cs{}, cf{};
-      int cs_blocks = 0;
+      int cs_blocks = 0, cf_mats = 0;
+      bool any_ordered = false;
       for (int q = 0; q < n; ++q) {
         const Plan &pl = cp[q].pl;
         if (!pl.sp.any_gate(steps)) continue;
         const int i = cs.n;
         cs.Xh[i] = cp[q].inH; cs.cond[i] = pl.condpart; cs.sum[i] = pl.cond; cs.part[i] = pl.colpart; cs.flag[i] = pl.wide_flag;
-        cs.order[i] = pl.order;
         cs.gate[i] = 1e300;
         for (int j = 1; j < steps; ++j)
           if (pl.sp.gated(j)) cs.gate[i] = std::min(cs.gate[i], (double)pl.sp.gate_tau[j] / (double)cp[q].N);
+        cs.order[i] = ordered(q) ? pl.order : nullptr;
+        any_ordered = any_ordered || ordered(q);
         cs.M[i] = (int)cp[q].M; cs.N[i] = (int)cp[q].N; cs.parts[i] = pl.col_parts;
         cs.rule[i] = WideRule{(double)pl.sp.wide_near, (double)pl.sp.wide_lo, (double)pl.sp.wide_hi,
                               (double)pl.sp.wide_near_diff};
@@ -1082,12 +1101,15 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       }
       cf = cs;
       for (int i = 0, q = 0; q < n; ++q)
-        if (cp[q].pl.sp.any_gate(steps)) cf.blocks[i++] = (int)cp[q].E;
+        if (cp[q].pl.sp.any_gate(steps)) { cf.blocks[i++] = (int)cp[q].E; cf_mats += (int)cp[q].E; }
       if (cs_blocks > 0) {
         hipLaunchKernelGGL(k_ns_colstat, dim3((unsigned)cs_blocks), dim3(kThreads), 0, s, cs);
         ANC_LAUNCH_CHECK();
       }
-      hipLaunchKernelGGL(k_ns_classify, dim3((unsigned)cf.n), dim3(kClassifyThreads), 0, s, cf);
+      if (any_ordered)
+        hipLaunchKernelGGL(k_ns_classify_order, dim3((unsigned)cf.n), dim3(kClassifyThreads), 0, s, cf);
+      else
+        hipLaunchKernelGGL(k_ns_classify, dim3((unsigned)((cf_mats + kThreads / 64 - 1) / (kThreads / 64))), dim3(kThreads), 0, s, cf);
       ANC_LAUNCH_CHECK();
     }
     {

@@ -210,6 +210,22 @@ def test_gated_matrices_are_dealt_in_turn(gpu, E, M, N, tiles):
             assert bits_equal(got[e], run_ns(Y[e: e + 1], mode="bf16")[0]), (list(hard), e)
 
 
+@pytest.mark.parametrize("E,mode,scale", [(64, "bf16", 100.0), (65, "bf16", 100.0), (77, "bf16", 1000.0), (6, "bf16_late3", 1000.0)])
+def test_gates_in_mixed_batches(gpu, E, mode, scale):
+    """A gate's decision and a matrix's place in the launches belong to the same matrix: with outlier columns in some of
+    them (x100 the cheap gate, x1000 the wide one, which alone a plan without an order has), every matrix of a batch has
+    the bits it has alone."""
+    M = N = 1024
+    rng = np.random.default_rng(E)
+    one = rng.standard_normal((2, M, N), dtype=np.float32)
+    one[1][:, rng.choice(N, N // 100, replace=False)] *= np.float32(scale)
+    want = [run_ns(one[i: i + 1], mode=mode)[0] for i in range(2)]
+    hard = rng.integers(0, 2, E)
+    got = run_ns(one[hard], mode=mode)
+    for e in range(E):
+        assert bits_equal(got[e], want[hard[e]]), e
+
+
 @pytest.mark.parametrize("E,M,N", [(86, 128, 128), (64, 128, 256), (65, 128, 256), (26, 256, 384)])
 @pytest.mark.parametrize("mode", ["bf16", "bf16_x3"])
 def test_many_small_tiles_keep_the_bits(gpu, E, M, N, mode):
