@@ -62,7 +62,8 @@ struct NsGemm {
                              // product sets it: its A is a K-range of a longer row)
   int64_t strideA, strideB;  // elements between consecutive matrices
   int tiles_m, tiles_n;
-  int lower;                 // symmetric output: 64x64 blocks on and below the diagonal only, mirrored
+  int lower;                 // symmetric output: 64x64 blocks on and below the diagonal only, mirrored: 1 = by the workgroup that
+                             // multiplied them, 2 (64-wide tiles) = by another that multiplies the same block again
   int plain_sum;             // plain product: 1 = write X32 = (A32, if not null, else 0) + A B and, if Yh is
                              // not null, its bf16 copy (RNE) to Yh; 0 = write X32 = A B
   int fits256;               // the chain's dims are multiples of 256 (and no flag says otherwise): 256-wide tiles may run

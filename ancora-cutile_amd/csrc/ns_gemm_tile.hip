@@ -95,19 +95,25 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   else anc_group_tile(pm, (int)blockIdx.x, gsel, L);
   const NsGemm &p = pm.g[gsel];
   int e = 0, tm, tn;
+  constexpr bool kImages = EPI != EPI_BX && WM == 1 && kRing == 4;      // (see NsGemm::lower)
+  bool image = false;
   // (the blocks' edges are powers of two; a division of two variables is 40 instructions, and a launch that this
   // kernel is made for has little else to do)
   const int sr = __builtin_ctz(p.blk_r), sc_ = __builtin_ctz(p.blk_c);
   if (EPI != EPI_BX) {
     // Tiles that reach the diagonal's 64x64 blocks or lie below them, in rows of blocks of blk_r x blk_c tiles: the
     // whole blocks of a row, then the tiles of its block on the diagonal.
-    const int per = anc_sym_tiles<TM, TN>(p.tiles_m);
+    const int tri = anc_sym_tiles<TM, TN>(p.tiles_m), per = kImages && p.lower == 2 ? p.tiles_m * p.tiles_m : tri;
     if (L >= per) { e = L / per; L -= e * per; }
     const int on_diag = anc_sym_tiles<TM, TN>(p.blk_r);
     int bm = 0, row = on_diag;
-    while (L >= row) { L -= row; row += p.blk_r * p.blk_c; ++bm; }
+    image = kImages && L >= tri;
+    while (!image && L >= row) { L -= row; row += p.blk_r * p.blk_c; ++bm; }
     const int whole = row - on_diag;
-    if (L < whole) {
+    if (image) {
+      tn = L - tri;
+      for (tm = 1; tn >= tm; ++tm) tn -= tm;
+    } else if (L < whole) {
       const int i = L & (p.blk_r * p.blk_c - 1);
       tm = (bm << sr) + (i >> sc_);
       tn = ((L >> (sr + sc_)) << sc_) + (i & (p.blk_c - 1));
@@ -225,7 +231,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   const int lrow = lane / LPR, c0 = (lane % LPR) * RUN;
   const int gi_w = tm * TM + wm * (32 * WM), gj_w = tn * TN + wn * (32 * WN);
   // symmetric output: this wavefront's block lies above the 64x64 blocks of the diagonal (nobody needs it), or below
-  const bool idle = EPI != EPI_BX && WM > 1 && (gi_w >> 6) < (gj_w >> 6), mirror = EPI != EPI_BX && (gi_w >> 6) > (gj_w >> 6);
+  const bool idle = EPI != EPI_BX && WM > 1 && (gi_w >> 6) < (gj_w >> 6), mirror = EPI != EPI_BX && (gi_w >> 6) > (gj_w >> 6) && (!kImages || p.lower != 2 || image);
   // run 0 of block b in a matrix of M rows in panel layout (run r: RS * 32 r further)
   auto pan_of = [&](int b) { return ((int64_t)((gj_w + (b % WN) * 32) / 32) * M + gi_w + (b / WN) * 32 + lrow) * 32 + c0; };
   constexpr int NB = WM * WN;
@@ -651,7 +657,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
         if (EPI == EPI_GRAM) {
 #pragma unroll
           for (int k = 0; k < 16; ++k) v[k] = v[k] * acc_scale;
-          if (has_a32) {
+          if (has_a32 && !image) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
               *(anc_f32x4 *)(p.A32 + mm + quad(i, M)) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
@@ -708,7 +714,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
           if (dc >= 0) p.dB[mv + gj + dc] = dv;
         }
         uint16_t *oh = EPI == EPI_GRAM ? p.Fh : p.Bh, *ol = EPI == EPI_GRAM ? p.Fl : p.Bl;
-        put_bf16(oh + mm + pan, write_lo ? ol + mm + pan : nullptr, pst);
+        if (!image) put_bf16(oh + mm + pan, write_lo ? ol + mm + pan : nullptr, pst);
         if (mirror) {                        // mirror image: rows gj0 .., 32-column panel gi0/32
           put_rows();
           get_cols();
@@ -887,7 +893,20 @@ int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, 
   const int TM = tile == 64 ? 64 : 128, TN = tile == 128 ? 128 : 64;
   NsGemmMulti pm{};
   pm.n = n;
-  int64_t grid = 0;
+  int64_t grid = 0, full = 0, longest = 0;
+  for (int k = 0; k < n; ++k) {
+    full += Es[k] * (ps[k].M / 64) * (ps[k].M / 64);
+    longest = ps[k].K > longest ? ps[k].K : longest;
+  }
+  // Where CUs are left over, a symmetric product's tile above the diagonal is a workgroup of its own, instead of a second, transposed
+  // store behind the one below: the launch lasts as long as its longest workgroup, and a short K has nothing to hide the store
+  // behind. Long ones, and launches of more than half the CUs, lose by the tiles fetched twice. Measured, us per chain, one
+  // workgroup per pair of tiles / one per tile (tiles in all):
+  //   1 x (128,128) 79.5 / 75.7 (4), 1 x (256,256) 89.4 / 85.7 (16), 8 x (256,512) 99.0 / 95.9 (128), 1 x (512,1536) 134.3 / 129.2 (64),
+  //   1 x (640,640) 125.7 / 121.9 (100), 2 x (512,512) 116.7 / 116.7 (128), 2 x (512,3072) 208.2 / 206.8 (128)
+  //   8 x (256,4096) 247 / 250 (128), 7 x (384,768) 139 / 147 (252), 4 x (512,512) 126 / 134 (256), 1 x (1024,3072) 191 / 195 (256)
+  //   K <= 256: 16 x (256,256) 97.1 / 94.3 (256), 64 x (128,128) 92.6 / 90.2 (256), 16 x (256,512) 117.9 / 117.7 (256, half of it K = 512)
+  const bool images = epi != EPI_BX && tile == 64 && (full <= 128 ? longest <= 3072 : full <= 256 && longest <= 256);
   for (int k = 0; k < n; ++k) {
     NsGemm &g = pm.g[k];
     g = ps[k];
@@ -895,12 +914,12 @@ int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, 
                 "anc_ns_gemm_tile: dims must be multiples of 128");
     g.tiles_m = g.M / TM;
     g.tiles_n = (epi == EPI_BX ? g.N : g.M) / TN;
-    g.lower = epi == EPI_BX ? 0 : 1;
+    g.lower = epi == EPI_BX ? 0 : images ? 2 : 1;
     // walked in blocks of 256 x 256 (see launch_bx of the 256-wide kernel: what an XCD fetches)
     const int cols = epi == EPI_BX ? g.N : g.M;
     g.blk_r = (g.M % 256 == 0 ? 256 : 128) / TM;
     g.blk_c = (cols % 256 == 0 ? 256 : 128) / TN;
-    const int64_t per = !g.lower ? (int64_t)g.tiles_m * g.tiles_n
+    const int64_t per = !g.lower || images ? (int64_t)g.tiles_m * g.tiles_n
                       : TM == TN ? anc_sym_tiles<64, 64>(g.tiles_m) : anc_sym_tiles<128, 64>(g.tiles_m);
     ANC_REQUIRE(per > 0 && Es[k] * per < (1ll << 30), "anc_ns_gemm_tile: grid out of range");
     pm.tiles[k] = (int)(Es[k] * per);

@@ -192,6 +192,21 @@ def test_tile_choice_keeps_the_bits(gpu, M, N, mode):
     assert rel_fro(want[0], host_ns(X[0], PE_SCHEDULE, 5)) < TOL_BF16
 
 
+@pytest.mark.parametrize("E,M,N", [(1, 128, 128), (32, 128, 256), (33, 128, 256), (64, 128, 128), (65, 128, 128), (2, 128, 3072), (2, 128, 3200),
+                                   (8, 256, 512), (9, 256, 512), (16, 256, 256), (3, 384, 640), (2, 512, 768), (1, 640, 640), (1, 768, 768)])
+@pytest.mark.parametrize("mode", ["bf16", "bf16_x3"])
+def test_mirror_images_of_small_launches(gpu, E, M, N, mode):
+    """Where CUs are left over a symmetric product's tiles above the diagonal have workgroups of their own: batches on both sides of
+    the rule's lines (128 tiles of 64 and K = 3072, 256 tiles and K = 256) have the bits that 128-wide tiles give, which have none."""
+    rng = np.random.default_rng(E + M + N)
+    X = rng.standard_normal((E, M, N)).astype(np.float32)
+    X[E // 2][:, :2] *= 100.0
+    want = run_ns(X, mode=f"{mode}_t128")
+    assert bits_equal(run_ns(X, mode=f"{mode}_t64"), want)
+    assert bits_equal(run_ns(X, mode=mode), want)
+    assert rel_fro(want[0], host_ns(X[0], PE_SCHEDULE, 5)) < TOL_BF16
+
+
 @pytest.mark.parametrize("E,M,N", [(1, 1024, 1024), (3, 1024, 2048), (8, 1024, 1024), (19, 1024, 1024), (9, 1024, 2048)])
 @pytest.mark.parametrize("tiles", ["", "_t256"])
 def test_gated_matrices_are_dealt_in_turn(gpu, E, M, N, tiles):
@@ -475,7 +490,7 @@ def test_grouped_launch_equals_per_batch_bits(gpu):
         ns_batched_pair(U, fro, 2, E, M, N, 0, steps=5, schedule=PE_SCHEDULE, mode="bf16")
         alone.append(U.to_numpy())
         U.free(); fro.free()
-    for order in ([0, 1, 2], [2, 0, 1], [3, 4, 5, 0, 1, 2], [3]):
+    for order in ([0, 1, 2], [2, 0, 1], [3, 4, 5, 0, 1, 2], [3], [0, 1, 5], [5, 1]):
         bufs, probs = [], (_lib.NsProblem * len(order))()
         for k, q in enumerate(order):
             E, M, N = shapes[q]
