@@ -873,19 +873,32 @@ int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
 }
 
 // The same for the bare product of weight gradients. Its K is a batch of tokens: short ones are bound by the
-// output, which small tiles spread best, long ones by operands that leave the L2, and there a second tile
-// on a few CUs costs as much as on all: the widest tile of which every CU has at most one. Measured, us on tiles of
+// output, which small tiles spread best, long ones by operands that leave the L2; and a launch lasts as long as the CU with
+// the most tiles, of which it takes three 64-wide or 128x64 ones at once, two 128-wide, one 256-wide. Measured, us on tiles of
 // 64 / 128x64 / 128 / 256, written (in brackets: added up):
-//   tiles of 64      256 tokens                768 tokens                2048 tokens            8192 tokens
-//   288              5.7/6.0/7.6/10.7          8.2/7.6/10.5/14.9         16.0/13.5/18.0/26.8    61/43/54/84
-//   432              5.5/6.0/7.6/10.7          8.1/7.9/10.6/15.0         16.7/14.6/18.2/27.5    64/46/54/85
-//                    (5.7/6.6/8.3/12.7)        (9.1/8.9/11.6/17.3)       (19/16/20/31)          (67/46/56/87)
-//   640              6.7/7.1/8.3/11.2          10.7/9.8/10.9/15.0        26.8/28.3/18.7/27.8    113/105/58/85
-//   896              11.0/7.8/8.9/11.3         14.3/12.4/12.3/15.2       28.9/27.8/22.8/27.8    125/101/71/85
-//   1056             10.2/10.1/10.6/11.3       16.5/17.6/17.3/15.2       36.4/38.6/36.3/27.8    142/145/122/87
-//   1344             18.0/10.9/12.0/11.6       20.5/17.8/17.6/16.5       42.5/40.6/36.0/29.9    183/149/121/93
-//                    (18.7/12.4/13.5/17.1)     (23.6/21.2/20.3/22.5)     (47/42/38/36)          (185/152/124/98)
-// (up to 256 tiles of 64 those are fastest at every length: 128 of them at 1504 tokens 8.3 / 10.2 / 14.7 / 20.3.)
+//   tiles of 64      256 tokens             512 tokens             768 tokens             1024 tokens            2048 tokens
+//   288              5.5/6.2/7.1/11.0       6.7/7.1/8.3/13.1       8.0/7.8/9.5/15.0       9.2/8.6/10.6/16.8      15.6/13.5/16.1/26.9
+//                    (5.7/6.4/7.3/12.0)     (6.9/7.3/8.5/14.0)     (8.1/8.2/9.8/16.1)     (9.3/9.1/11.2/18.5)    (16.8/14.5/17.1/29.3)
+//   432              5.8/6.6/7.4/11.2       6.8/7.2/8.3/13.1       7.8/7.9/9.5/14.9       9.2/9.0/10.9/16.9      16.6/14.3/16.4/27.5
+//                    (6.0/6.9/7.6/12.3)     (7.0/7.8/8.9/14.4)     (8.4/8.8/10.3/17.0)    (10.6/10.3/11.9/19.5)  (18.5/15.6/17.7/30)
+//   512              6.1/6.9/7.6/11.5       7.0/7.4/8.4/13.1       7.9/8.2/9.5/14.9       9.1/9.1/10.9/16.9      17.9/14.5/16.5/28.0
+//                    (6.5/7.1/7.9/12.1)     (7.2/7.9/9.1/14.0)     (8.1/8.8/10.4/16.1)    (9.6/10.0/12.1/18.6)   (19.1/15.7/18.0/31)
+//   640              6.3/7.0/7.6/11.7       8.5/8.6/9.5/13.3       12.8/13.7/11.0/14.9    16.4/17.3/12.8/16.9    27.7/29.0/19.3/27.7
+//                    (7.3/8.3/8.3/12.3)     (11.5/12.2/11.1/15.9)  (15.1/15.7/12.8/17.8)  (18.2/18.8/14.4/20.1)  (29.7/30/21.0/31)
+//   768              6.9/7.3/7.9/11.6       8.8/8.5/9.3/13.1       10.8/10.6/10.5/14.8    13.9/14.6/12.1/17.3    25.1/26.3/17.9/27.8
+//                    (7.1/8.2/8.5/14.1)     (9.8/10.4/10.1/16.7)   (13.1/13.8/12.2/19.4)  (16.3/17.0/13.9/21.9)  (26.8/27.5/19.8/32)
+//   896              8.3/7.8/8.1/11.5       10.5/9.4/10.0/13.2     13.0/11.2/11.4/15.0    16.1/15.4/12.9/17.6    27.5/26.4/19.4/27.9
+//                    (8.8/8.8/8.9/14.6)     (11.9/11.1/10.9/17.9)  (15.4/14.8/13.1/20.3)  (18.3/17.5/14.9/22.9)  (30/27.9/21.2/33)
+//   1056             9.0/9.8/10.0/11.5      12.2/13.1/13.7/13.3    15.9/16.8/16.3/15.1    19.9/21.0/21.0/17.7    35/37/35/27.8
+//                    (10.3/10.6/11.8/15.3)  (14.8/15.9/16.4/18.4)  (18.7/20.4/20.2/20.6)  (22.9/24.3/23.7/23.2)  (38/40/37/33)
+//   1344             10.2/10.4/11.1/11.5    14.7/13.4/14.1/13.8    18.8/17.1/16.8/16.1    23.4/21.7/20.9/18.6    41/39/35/28.8
+//                    (12.7/12.3/12.8/16.9)  (18.0/16.4/16.7/19.6)  (22.8/20.6/20.3/22.0)  (27.7/24.6/23.7/24.9)  (46/41/37/35)
+//   1536             10.5/11.9/12.0/12.7    14.6/13.6/14.0/14.8    20.4/19.0/17.0/17.0    25.2/23.3/20.7/19.4    44/40/35/30
+//                    (14.8/14.5/14.1/17.6)  (20.0/18.3/17.3/20.2)  (24.5/22.0/20.4/22.8)  (29.7/25.7/23.7/25.8)  (50/42/37/37)
+// (up to 256 tiles of 64 those are fastest at every length: 128 of them at 1504 tokens 6.7 / 10.4 / 13.2 / 20.8. Beyond 640 tokens
+// and 1024 tiles with gradients added up, smaller tiles would be up to 16 % ahead of 256-wide ones; 512 at 1024 tokens, added up, lose
+// 4 % on 128x64.) The lines in between: 448 tokens 704 tiles 8.0 / 8.2 / 8.6 / 12.5, 832 9.5 / 8.6 / 9.3 / 12.4, 1152 11.5 / 12.2 / 13.0 / 12.7;
+// 640 tokens 640 tiles 10.3 / 10.9 / 10.3 / 14.0, added up 13.4 / 14.2 / 12.1 / 16.7, 960 tiles 12.6 / 10.9 / 11.1 / 14.2.
 int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0;
   bool adds = false;
@@ -894,8 +907,17 @@ int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
     adds = adds || (ps[k].plain_sum && ps[k].A32 != nullptr);
   }
   for (int k = 0; k < n; ++k) t64 += (double)Es[k] * (ps[k].M / 64) * (ps[k].N / 64) * ((double)ps[k].K / longest);
-  if (longest <= 640.0) return t64 <= 640.0 ? 64 : t64 <= 1536.0 ? kTile128x64 : t64 <= (adds ? 3000.0 : 2000.0) ? 128 : 256;
-  return t64 <= 256.0 ? 64 : t64 <= 512.0 ? kTile128x64 : t64 <= 1024.0 ? 128 : 256;
+  if (t64 <= 512.0) return t64 <= 256.0 || longest <= (adds ? 900.0 : 768.0) ? 64 : kTile128x64;
+  if (longest > 640.0) return t64 <= 1024.0 ? 128 : 256;
+  if (longest <= 448.0) {
+    if (t64 <= 768.0 || (t64 > 990.0 && t64 <= 1300.0)) return 64;
+    if (t64 <= (adds && longest > 192.0 ? 1450.0 : 1536.0)) return kTile128x64;
+  } else {
+    if ((t64 <= 640.0 && !(adds && longest > 576.0)) || (t64 > 1024.0 && t64 <= 1300.0)) return 64;
+    if ((t64 <= 1024.0 && !adds) || (t64 > 768.0 && t64 <= 990.0) || (t64 > 1300.0 && t64 <= (adds || longest > 544.0 ? 1450.0 : 1536.0)))
+      return kTile128x64;
+  }
+  return t64 <= (adds ? 3000.0 : 2000.0) ? 128 : 256;
 }
 
 // What leaves a launch past the caches (NsGemm::stream_out): the caches are left to the operands of the tiles still to

@@ -71,13 +71,12 @@ template <bool WIDE, typename T> __device__ __forceinline__ void st_once(T *p, T
   else *p = v;
 }
 
-// Workgroups a CU takes: what its 160 KiB of LDS hold, but not more than two rings of four 16 KiB stages.
+// Workgroups a CU takes: what its 160 KiB of LDS hold, but not more than two rings of four 16 KiB stages. (wm, wn: 64-row and
+// 64-column blocks of a tile)
 constexpr int tile_per_cu(int wm, int wn, int ring) { return (wm == 1 ? ring == 3 : wn == 1) ? 3 : 2; }
 
-// Tiles of the first `rows` rows of TM x TN tiles that hold something on or below the 64x64
-// blocks of the diagonal.
-template <int TM, int TN>
-__host__ __device__ constexpr int anc_sym_tiles(int rows) { return (TM / TN) * (rows * (rows + 1) / 2); }
+// Tiles on and below the diagonal in the first `rows` rows of square tiles
+__host__ __device__ constexpr int anc_sym_tiles(int rows) { return rows * (rows + 1) / 2; }
 
 // SOLO: the launch has one problem, its arguments lie at fixed places.
 template <int EPI, int WM, int WN, int NW, bool AT, int VAR, int kRing, bool SOLO>
@@ -101,27 +100,28 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   // kernel is made for has little else to do)
   const int sr = __builtin_ctz(p.blk_r), sc_ = __builtin_ctz(p.blk_c);
   if (EPI != EPI_BX) {
-    // Tiles that reach the diagonal's 64x64 blocks or lie below them, in rows of blocks of blk_r x blk_c tiles: the
-    // whole blocks of a row, then the tiles of its block on the diagonal.
-    const int tri = anc_sym_tiles<TM, TN>(p.tiles_m), per = kImages && p.lower == 2 ? p.tiles_m * p.tiles_m : tri;
+    // Tiles on and below the diagonal, in rows of blocks of blk_r x blk_r tiles: the whole blocks of a row, then the
+    // tiles of its block on the diagonal.
+    static_assert(EPI == EPI_BX || TM == TN, "symmetric products: square tiles");
+    const int tri = anc_sym_tiles(p.tiles_m), per = kImages && p.lower == 2 ? p.tiles_m * p.tiles_m : tri;
     if (L >= per) { e = L / per; L -= e * per; }
-    const int on_diag = anc_sym_tiles<TM, TN>(p.blk_r);
+    const int on_diag = anc_sym_tiles(p.blk_r);
     int bm = 0, row = on_diag;
     image = kImages && L >= tri;
-    while (!image && L >= row) { L -= row; row += p.blk_r * p.blk_c; ++bm; }
+    while (!image && L >= row) { L -= row; row += p.blk_r * p.blk_r; ++bm; }
     const int whole = row - on_diag;
     if (image) {
       tn = L - tri;
       for (tm = 1; tn >= tm; ++tm) tn -= tm;
     } else if (L < whole) {
-      const int i = L & (p.blk_r * p.blk_c - 1);
-      tm = (bm << sr) + (i >> sc_);
-      tn = ((L >> (sr + sc_)) << sc_) + (i & (p.blk_c - 1));
+      const int i = L & (p.blk_r * p.blk_r - 1);
+      tm = (bm << sr) + (i >> sr);
+      tn = ((L >> (2 * sr)) << sr) + (i & (p.blk_r - 1));
     } else {
       int i = L - whole, r = 0;
-      while (i >= (r + 1) * (TM / TN)) { i -= (r + 1) * (TM / TN); ++r; }
+      while (i >= r + 1) { i -= r + 1; ++r; }
       tm = (bm << sr) + r;
-      tn = (bm << sc_) + i;
+      tn = (bm << sr) + i;
     }
   } else {
     const int per = p.tiles_m * p.tiles_n, across = p.tiles_n >> sc_;
@@ -196,8 +196,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   // ---- fragment addressing: tr = [block][k][64 B] by transposing reads, else [panel][row][64 B]
   const int l31 = lane & 31, hh = lane >> 5, g16 = lane >> 4, s16 = lane & 15;
   const int tr_lane = (8 * (g16 >> 1) + (s16 >> 2)) * 64 + 32 * (g16 & 1) + 8 * (s16 & 3);
-  // (rows_k: k rows of a block in the stage)
-  // (rows: the operand's rows per panel)
+  // (rows_k: k rows of a block in the stage; rows: the operand's rows per panel)
   auto frag = [&](auto tr, const unsigned char *half, int blk, int kk, int rows_k, int rows) -> bf16x8 {
     if constexpr (decltype(tr)::value) {
       const unsigned char *q = half + blk * (rows_k * 64) + kk * 16 * 64 + tr_lane;
@@ -846,7 +845,8 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
 
 // Weight gradients on 128x128 tiles, us at 288 / 432 / 768 / 1344 tiles of 64 (written), four / eight wavefronts: 768 tokens
 // 10.4 / 9.5, 10.7 / 9.4, 11.4 / 10.6, 17.4 / 17.5; 2048 tokens 17.8 / 16.4, 18.7 / 16.6, 19.2 / 18.5, 34.9 / 35.8; 8192 tokens
-// 54 / 52, 55 / 51, 61 / 57, 119 / 122, and 1024 tiles at 4096 tokens 36.8 / 39.7.
+// 54 / 52, 55 / 51, 61 / 57, 119 / 122, and 1024 tiles at 4096 tokens 36.8 / 39.7. Added up in two workgroups per CU, level up to
+// 640 tokens (1536 tiles 15.6 / 15.7 at 384, 18.7 / 19.0 at 640), but with eight some of the cards took 16 .. 21 there.
 constexpr int kLongPlain = 2048;
 
 template <int EPI, bool AT, int VAR>
@@ -857,7 +857,8 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) 
       return;
     }
     // (see kLongPlain)
-    if (tile == 128 && pm.g[0].K > kLongPlain) {
+    const bool adds = pm.g[0].plain_sum != 0 && pm.g[0].A32 != nullptr;
+    if (tile == 128 && (pm.g[0].K > kLongPlain || (adds && grid > 256 && grid <= 512))) {
       hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 2, 4, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
       return;
     }
@@ -891,6 +892,7 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) 
 int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int tile, bool by_rows,
                            const NsUpdate *upd, bool plain) {
   const int TM = tile == 64 ? 64 : 128, TN = tile == 128 ? 128 : 64;
+  ANC_REQUIRE(plain || TM == TN, "anc_ns_gemm_tile: tiles of 128x64 are the plain product's");
   NsGemmMulti pm{};
   pm.n = n;
   int64_t grid = 0, full = 0, longest = 0;
@@ -919,8 +921,7 @@ int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, 
     const int cols = epi == EPI_BX ? g.N : g.M;
     g.blk_r = (g.M % 256 == 0 ? 256 : 128) / TM;
     g.blk_c = (cols % 256 == 0 ? 256 : 128) / TN;
-    const int64_t per = !g.lower || images ? (int64_t)g.tiles_m * g.tiles_n
-                      : TM == TN ? anc_sym_tiles<64, 64>(g.tiles_m) : anc_sym_tiles<128, 64>(g.tiles_m);
+    const int64_t per = !g.lower || images ? (int64_t)g.tiles_m * g.tiles_n : anc_sym_tiles(g.tiles_m);
     ANC_REQUIRE(per > 0 && Es[k] * per < (1ll << 30), "anc_ns_gemm_tile: grid out of range");
     pm.tiles[k] = (int)(Es[k] * per);
     grid += pm.tiles[k];

@@ -380,13 +380,13 @@ def test_accumulated_micro_batches_against_one_batch(gpu):
     assert same >= 0.98, same                                          # (D): the reference's bar
 
 
-@pytest.mark.parametrize("T,K,N,n", [(672, 640, 1792, 1), (736, 384, 3072, 1), (1504, 1024, 2048, 1), (32, 512, 1280, 5), (608, 1024, 1536, 4),
-                                     (96, 640, 2304, 3)])
+@pytest.mark.parametrize("T,K,N,n", [(928, 640, 1792, 1), (928, 384, 3072, 1), (1504, 1024, 2048, 1), (32, 512, 1280, 5), (448, 768, 2304, 2),
+                                     (96, 1408, 1024, 4), (608, 1408, 1024, 4), (512, 1024, 2816, 1)])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_tiles_of_128x64(gpu, T, K, N, n, accumulate):
-    """Calls on both ends of the range that runs on 128x64 tiles (257 .. 512 tiles of 64 beyond 640 tokens, 641 .. 1536
-    up to there), with one K tile, fewer than the ring has stages, and remainders of a round: the fp64 product, and
-    for n weights the bits each has alone."""
+    """Calls in the ranges that run on 128x64 tiles (257 .. 512 tiles of 64 beyond 900 tokens, 769 .. 990 and 1301 .. 1450 up to 448,
+    769 .. 990, 1301 .. 1450 and, written, 641 .. 1024 up to 640), with one K tile, fewer than the ring has stages, and remainders of a
+    round: the fp64 product, and for n weights the bits each has alone."""
     from ancora_cutile_amd import DevBuf
     from ancora_cutile_amd.grads import gemm_dW, DwWorkspace
     rng = np.random.default_rng(T + K + N)
@@ -413,10 +413,12 @@ def test_tiles_of_128x64(gpu, T, K, N, n, accumulate):
     xd.free()
 
 
-@pytest.mark.parametrize("T,K,N,n", [(672, 1152, 2048, 1), (800, 640, 1792, 2), (2048, 1152, 2048, 1), (2080, 1152, 2048, 1)])
+@pytest.mark.parametrize("T,K,N,n", [(672, 1152, 2048, 1), (800, 640, 1792, 2), (2048, 1152, 2048, 1), (2080, 1152, 2048, 1),
+                                     (640, 640, 4096, 1), (384, 1024, 3072, 2), (640, 2048, 4096, 1), (416, 2048, 4352, 1)])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_tiles_of_128(gpu, T, K, N, n, accumulate):
     """513 .. 1024 tiles of 64 beyond 640 tokens run on 128x128 tiles, of eight wavefronts up to 2048 tokens and of four
+    beyond; so do, added up, 513 .. 768 and 991 .. 1024 beyond 448 or 576 tokens, and more, of four wavefronts up to 2048 tiles of 64, of eight
     beyond."""
     test_tiles_of_128x64(gpu, T, K, N, n, accumulate)
 
