@@ -100,28 +100,28 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   // kernel is made for has little else to do)
   const int sr = __builtin_ctz(p.blk_r), sc_ = __builtin_ctz(p.blk_c);
   if (EPI != EPI_BX) {
-    // Tiles on and below the diagonal, in rows of blocks of blk_r x blk_r tiles: the whole blocks of a row, then the
-    // tiles of its block on the diagonal.
+    // Tiles on and below the diagonal, in rows of blocks of blk_r x blk_c tiles, blk_r = blk_c: the whole blocks of a row, then the
+    // tiles of its block on the diagonal. (Written with blk_r alone, 24 x (512,512) 323.0 -> 325.2 us per chain.)
     static_assert(EPI == EPI_BX || TM == TN, "symmetric products: square tiles");
     const int tri = anc_sym_tiles(p.tiles_m), per = kImages && p.lower == 2 ? p.tiles_m * p.tiles_m : tri;
     if (L >= per) { e = L / per; L -= e * per; }
     const int on_diag = anc_sym_tiles(p.blk_r);
     int bm = 0, row = on_diag;
     image = kImages && L >= tri;
-    while (!image && L >= row) { L -= row; row += p.blk_r * p.blk_r; ++bm; }
+    while (!image && L >= row) { L -= row; row += p.blk_r * p.blk_c; ++bm; }
     const int whole = row - on_diag;
     if (image) {
       tn = L - tri;
       for (tm = 1; tn >= tm; ++tm) tn -= tm;
     } else if (L < whole) {
-      const int i = L & (p.blk_r * p.blk_r - 1);
-      tm = (bm << sr) + (i >> sr);
-      tn = ((L >> (2 * sr)) << sr) + (i & (p.blk_r - 1));
+      const int i = L & (p.blk_r * p.blk_c - 1);
+      tm = (bm << sr) + (i >> sc_);
+      tn = ((L >> (sr + sc_)) << sc_) + (i & (p.blk_c - 1));
     } else {
       int i = L - whole, r = 0;
       while (i >= r + 1) { i -= r + 1; ++r; }
       tm = (bm << sr) + r;
-      tn = (bm << sr) + i;
+      tn = (bm << sc_) + i;
     }
   } else {
     const int per = p.tiles_m * p.tiles_n, across = p.tiles_n >> sc_;
