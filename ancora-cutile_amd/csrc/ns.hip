@@ -843,7 +843,7 @@ struct ChainProb {
 //   just over one round of 256-wide tiles    26 x (1024,1024) 393 / 334 / 387 (5 launches alone; 260 of them), 48 x (768,768)
 //               555 / 465 / 522 (288), 33 x (1024,1024) 520 / 449 / 437 (330)
 //   X = a X + B X, mostly one term 1 x (1024,2048) 163 / 171 (512, 128), 1 x (1536,1536) 281 / 275 (576, 144), 1 x (1024,3072) 199 /
-//               193 (768, 192; with the update of the weight 270 / 274), 3 x (1152,1152) 307 / 290 (972, 243), 5 x (1024,1024) 313 / 309 /
+//               193 (768, 192), 3 x (1152,1152) 307 / 290 (972, 243), 5 x (1024,1024) 313 / 309 /
 //               326 (1280, 320), 6 x (1024,2048) 437 / 395 / 401 (3072, 768), 14 x (1024,1024) 653 / 595 / 584
 //               (3584, 896), 8 x (1024,2048) 596 / 528 / 506 (4096, 1024)
 //   residual terms                 12 x (640,640) 329 / 334 (1200, 300), 6 x (896,896) 389 / 401 (1176, 294), 24 x (512,512) 345 / 338 /
@@ -851,6 +851,13 @@ struct ChainProb {
 //               549 / 530 (2400, 600), 16 x (512,1536) 476 / 441 / 483 (3072, 768), 24 x 647 / 605 / 682 (4608, 1152), 30 x 809 /
 //               777 / 799 (5760, 1440), 24 x (768,1536) 1324 / 1145 / 1147 (6912, 1728)
 //   just over one round of large tiles       18 x (1024,1024) 811 / 774 / 786 (4608), 20 x 890 / 825 / 809 (5120)
+//   with the update of the weight, the whole step of one: (1024,2048) 167.5 / 172.2 (512), (1024,2304) 185.7 / 182.2 (576), (1536,1536) 279.8 /
+//               285.1 (576), (1024,2560) 191.0 / 187.0, (1280,2048) 221.5 / 225.5 (640), (1280,2304) 230.4 / 235.3 (720), (1024,3072) 199.8 /
+//               200.1 (768), (1024,3328) 210.1 / 207.0 (832): level to 2 % from 512 to 832 tiles, and one line in between
+// What the lines and the 64x64 blocks on the diagonal, with a second store below them, cost: against earlier lines and whole 256-wide
+// blocks 20 x (1024,1024) and 60 x (512,512) 1.6 .. 2 %, batches of (128,128) 2 .. 4 % (12: 77.6 -> 80.6), launches of 257 .. 330
+// workgroups 2 .. 4 % (28 x (256,256) 131 -> 136, 14 x (384,384) 158 -> 161, 8 x (512,512) 168 -> 172); 565 batches of 1 .. 60 matrices of
+// 23 shapes are 5.7 % faster in the mean.
 int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0, t128 = 0.0, t256 = 0.0, several = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
@@ -1223,15 +1230,15 @@ extern "C" int64_t anc_ns_workspace_bytes(int64_t E, int64_t M, int64_t N, int m
 
 // FLOPs of a symmetric M x M product, per unit of K, counted in blocks on or below the diagonal: 256x256 where both
 // dims are multiples of 256 and ANC_NS_TILE128 is not set, else 128x128: M^2 + 256 M or M^2 + 128 M. The kernels multiply
-// 64x64 blocks, M^2 + 64 M.
+// 64x64 blocks, M^2 + 64 M (see anc_optim.h).
 static double sym_tile_flops(int64_t M, int64_t N, bool force_small) {
   const double ts = (!force_small && M % 256 == 0 && N % 256 == 0) ? 256.0 : 128.0;
   const double t = (double)M / ts;
   return t * (t + 1) / 2 * 2.0 * ts * ts;
 }
 
-// Matrix-core work of one chain call: `executed` counts the tiles and terms actually
-// multiplied (symmetric products compute the lower tiles only; residual terms count),
+// Matrix-core work of one chain call: `executed` counts the terms multiplied (residual terms too), of symmetric products
+// the blocks of sym_tile_flops,
 // `dense` is the textbook steps*(4 M^2 N + 2 M^3) per matrix.
 extern "C" int anc_ns_flops(int64_t E, int64_t M, int64_t N, int steps, int mode,
                             double *executed, double *dense) {

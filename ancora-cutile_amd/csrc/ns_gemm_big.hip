@@ -150,8 +150,9 @@ __device__ __forceinline__ void dma16_epi(const void *g, uint32_t lds_base) {
   else dma16(g, lds_base);
 }
 
-// VAR (X = a X + B X only) selects a variant of the epilogue as its own instantiation, so that
-// the extra registers and branches do not weigh on the other launches: VAR_UPDATE applies the
+// VAR selects a variant of the epilogue as its own instantiation, so that
+// the extra registers and branches do not weigh on the other launches: VAR_STREAM stores past the caches
+// (NsGemm::stream_out); the others are those of X = a X + B X: VAR_UPDATE applies the
 // weight update, VAR_UPDATE_T refreshes a transposed bf16 copy of the weight as well; VAR_PLAIN is the bare product C = A B written as fp32 (no iterate at the output
 // position, no row scaling), which the weight-gradient GEMM uses; with `plain_sum` set it writes
 // C = (A32 or 0) + A B and, if Yh is set, the bf16 copy of C.

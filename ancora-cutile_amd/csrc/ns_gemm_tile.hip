@@ -209,9 +209,9 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   using TrB = std::bool_constant<BT>;
 
   // ---- what the epilogue of X = a X + B X reads at the output position is requested before the K loop, so that it has
-  // arrived when the loop ends (16 x (1024,3072) on 128-wide tiles of four wavefronts: 828 -> 783 us per 5 launches against
-  // fetching it block by block behind the loop; B = b A + c A A, which reads half as much, lost 2 % that way on such
-  // launches). The loads are older than every DMA below, so the waits of the ring hold. Eight wavefronts have no
+  // arrived when the loop ends (one (256,512) matrix 124.8 -> 121.5 us per chain against fetching it behind the loop; B = b A +
+  // c A A reads half as much, and only launches of one workgroup per CU gain by it, kEarlyA). The loads are older than
+  // every DMA below, so the waits of the ring hold. Eight wavefronts have no
   // registers for it (16 .. 32 would spill, 42 x (640,640) 913 -> 970) and request it behind the loop, all blocks at once.
   const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
   float *sg = (float *)lds + wave * 32 * kSgPitch;

@@ -75,7 +75,8 @@ int anc_fill_u32(uint64_t dptr, uint32_t value, int64_t n_words, uint64_t stream
 int anc_memcpy_h2d(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
 /* Uploads through pinned staging memory; src may be reused on return. anc_memcpy_h2d: complete on return.
  * _async: ordered on `stream`, no wait. _now: complete on return, on a stream of its own, without
- * waiting for work queued elsewhere; nobody may be using dst. Each device has its ring of staging memory, the
+ * waiting for work queued elsewhere; nobody may be using dst. A kernel on the caller's stream does the transfer where
+ * dst lies in one allocation of that stream's device, 16-byte aligned; the runtime's copy does it elsewhere, and for _now. Each device has its ring of staging memory, the
  * stream's device decides (the null stream and _now: the current one); _release gives it all back. A stream under
  * graph capture is refused (the graph would read host memory later than the call); _now may be called meanwhile. */
 int anc_upload_async(uint64_t dst, const void *src, int64_t bytes, uint64_t stream);
@@ -608,12 +609,15 @@ int anc_muon_ns_update_multi(const anc_ns_problem_t *problems, int32_t n_problem
                              int mode, const float *lr_scales /* [ANC_MUON_MAX_SCALES] */, int sr,
                              uint32_t seed_base, uint64_t ctl, uint64_t stream);
 
-/* Matrix-core FLOPs of one anc_ns_batched call: `executed` counts the terms the kernels multiply (residual
- * terms too) and of the symmetric products the blocks on or below the diagonal, each in full: 256x256
- * blocks where dims are multiples of 256, i.e. 10/16 of the dense product at M = 1024, else, or with
- * ANC_NS_TILE128 in `mode`, 128x128 blocks, 36/64. `dense` is steps*(4 M^2 N + 2 M^3) per matrix. The kernels
- * multiply 64x64 blocks, 136/256: with S = executed without and T = with ANC_NS_TILE128, dims multiples of 256,
- * that is T - (S - T) / 2, the number that the profiler's matrix-instruction counter reads. Matrices that take the
+/* Matrix-core FLOPs of one anc_ns_batched call, in blocks of 256 or 128: `executed` counts the terms the kernels
+ * multiply (residual terms too) and of the symmetric products the blocks on or below the diagonal, each in full:
+ * 256x256 blocks where dims are multiples of 256, i.e. 10/16 of the dense product at M = 1024, else, or with
+ * ANC_NS_TILE128 in `mode`, 128x128 blocks, 36/64. `dense` is steps*(4 M^2 N + 2 M^3) per matrix. What the kernels
+ * multiply is less, 64x64 blocks, 136/256: a symmetric product's (anc_ns_product_flops, products 0 and 1) share
+ * (M + 64) / (M + 256) or (M + 64) / (M + 128) of its count, all together, with S = executed without and T = with
+ * ANC_NS_TILE128, T - (S - T) / 2 where dims are multiples of 256. (8.697 TFLOP of a step of Qwen3-0.6B's 196 matrices
+ * by that and by the profiler's matrix-instruction counter. Symmetric products of at most 256 tiles of 64 in a launch may
+ * be multiplied above the diagonal too, which no count has.) Matrices that take the
  * conditioning gate add anc_ns_hard_info's extra work, counted the same way. */
 int anc_ns_flops(int64_t E, int64_t M, int64_t N, int steps, int mode,
                  double *executed, double *dense);
