@@ -464,6 +464,9 @@ extern "C" int anc_staging_release(void) {
     }
     std::lock_guard<std::mutex> lk(r.mu);
     if (r.own == nullptr || r.own_users != 0) continue;
+    // (a slot that a call held above may have its event from this stream: that call has waited for its transfer)
+    for (StageSlot &slot : r.slot)
+      if (!slot.taken && slot.user == r.own) slot.busy = false;
     ANC_HIP(hipStreamDestroy(r.own));
     r.own = nullptr;
   }

@@ -48,6 +48,7 @@ static std::map<char *, size_t> pinned;
 static int live_streams = 0;
 struct Region { size_t size; int dev; };
 static std::map<char *, Region> device_memory;       // allocations; any other address is memory of the current device, without an end
+static std::function<void()> at_copy, at_host_free;       // called on entry, where set
 static bool chip_full = false;         // kernels do not start: their streams are held
 static std::set<Stream *> gone;        // destroyed streams (their memory is kept, so that no new one has their address)
 static thread_local int cur = 0;
@@ -97,7 +98,7 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   pinned[(char *)*p] = n;
   return hipSuccess;
 }
-hipError_t hipHostFree(void *p) { std::lock_guard<std::mutex> lk(mu); pinned.erase((char *)p); free(p); return hipSuccess; }
+hipError_t hipHostFree(void *p) { if (at_host_free) at_host_free(); std::lock_guard<std::mutex> lk(mu); pinned.erase((char *)p); free(p); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
   std::lock_guard<std::mutex> lk(mu);
   Event *n = new Event{cur};
@@ -148,6 +149,7 @@ hipError_t hipMemGetAddressRange(hipDeviceptr_t *b, size_t *size, hipDeviceptr_t
   return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t s) {
+  if (at_copy) at_copy();
   std::unique_lock<std::mutex> lk(mu);
   Stream *st = str(s);
   if (st->capturing) return hipSuccess;                            // (recorded)
@@ -449,12 +451,42 @@ static void streams_of_others() {
   CHECK(pinned.empty() && events.empty() && live_streams == 0);
 }
 
+// The ring is given back while an upload that is complete on return holds a slot, and that call ends before the ring's own
+// stream is destroyed: the slot stays, and nobody looks at that stream again.
+static void released_beside_an_upload() {
+  const size_t n = 100;
+  const std::vector<char> want = bytes(n, 1);
+  std::vector<char> a(n), b(n), c(n);
+  Stream A{0};
+  A.held = true;                       // two slots in use, so that there is one to be freed beside the call's
+  CHECK(anc_upload_async((uint64_t)a.data(), want.data(), (int64_t)n, handle(&A)) == 0);
+  CHECK(anc_upload_async((uint64_t)b.data(), want.data(), (int64_t)n, handle(&A)) == 0);
+  release(&A);
+  std::promise<void> copying, freeing;
+  at_copy = [&] { copying.set_value(); freeing.get_future().wait(); };
+  std::future<int> now = std::async(std::launch::async, [&] { return anc_upload_now((uint64_t)c.data(), want.data(), (int64_t)n); });
+  copying.get_future().wait();
+  int ended = -1;
+  at_host_free = [&] { freeing.set_value(); ended = now.get(); };
+  CHECK(anc_staging_release() == 0);
+  at_copy = at_host_free = nullptr;
+  CHECK(ended == 0 && c == want && pinned.size() == 1 && live_streams == 0);
+  for (int i = 0; i < 12; ++i) {
+    std::vector<char> x(n), y(n);
+    CHECK(anc_upload_async((uint64_t)x.data(), want.data(), (int64_t)n, handle(&A)) == 0);
+    CHECK(anc_upload_now((uint64_t)y.data(), want.data(), (int64_t)n) == 0);
+    CHECK(x == want && y == want);
+  }
+  CHECK(anc_staging_release() == 0);
+  CHECK(pinned.empty() && events.empty() && live_streams == 0);
+}
+
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> cases = {{"two_devices", two_devices}, {"other_streams_do_not_wait", other_streams_do_not_wait},
                                                    {"many_threads", many_threads}, {"capture", capture}, {"streams_that_end", streams_that_end},
                                                    {"now_waits_for_no_kernel", now_waits_for_no_kernel},
                                                    {"memory_of_another_device", memory_of_another_device}, {"errors_of_others", errors_of_others}, {"past_the_end", past_the_end},
-                                                   {"streams_of_others", streams_of_others}};
+                                                   {"streams_of_others", streams_of_others}, {"released_beside_an_upload", released_beside_an_upload}};
   if (argc != 2 || cases.find(argv[1]) == cases.end()) return 2;
   cases.at(argv[1])();
   printf("ok\n");

@@ -26,7 +26,8 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["two_devices", "other_streams_do_not_wait", "many_threads", "capture", "streams_that_end",
-                                  "now_waits_for_no_kernel", "memory_of_another_device", "errors_of_others", "past_the_end", "streams_of_others"])
+                                  "now_waits_for_no_kernel", "memory_of_another_device", "errors_of_others", "past_the_end", "streams_of_others",
+                                  "released_beside_an_upload"])
 def test_uploads(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
