@@ -902,13 +902,18 @@ int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, 
   }
   // Where CUs are left over, a symmetric product's tile above the diagonal is a workgroup of its own, instead of a second, transposed
   // store behind the one below: the launch lasts as long as its longest workgroup, and a short K has nothing to hide the store
-  // behind. Long ones, and launches of more than half the CUs, lose by the tiles fetched twice. Measured, us per chain, one
-  // workgroup per pair of tiles / one per tile (tiles in all):
-  //   1 x (128,128) 79.5 / 75.7 (4), 1 x (256,256) 89.4 / 85.7 (16), 8 x (256,512) 99.0 / 95.9 (128), 1 x (512,1536) 134.3 / 129.2 (64),
-  //   1 x (640,640) 125.7 / 121.9 (100), 2 x (512,512) 116.7 / 116.7 (128), 2 x (512,3072) 208.2 / 206.8 (128)
-  //   8 x (256,4096) 247 / 250 (128), 7 x (384,768) 139 / 147 (252), 4 x (512,512) 126 / 134 (256), 1 x (1024,3072) 191 / 195 (256)
-  //   K <= 256: 16 x (256,256) 97.1 / 94.3 (256), 64 x (128,128) 92.6 / 90.2 (256), 16 x (256,512) 117.9 / 117.7 (256, half of it K = 512)
-  const bool images = epi != EPI_BX && tile == 64 && (full <= 128 ? longest <= 3072 : full <= 256 && longest <= 256);
+  // behind. The tiles fetched twice cost more the more workgroups share what they fetch and the longer K is. Measured, us per
+  // chain, one workgroup per pair of tiles / one per tile in A = X X^T (K = N) and B / in B alone (tiles in all, tiles * K of A in Ki):
+  //   up to 128 tiles  1 x (128,128) 78.7 / 75.1 (4, 1), 4 x (128,4096) 208.4 / 201.8 / 206.1 (16, 64), 1 x (256,256) 90.5 / 85.8 (16, 4), 8 x (256,512)
+  //               100.7 / 98.1 / 99.2 (128, 64), 2 x (512,1536) 155.6 / 153.3 / 155.4 (128, 192), 16 x (128,3072) 216.4 / 214.1 / 214.5 (64, 192),
+  //               32 x (128,1536) 191.7 / 190.3 / 189.9 (128, 192), 1 x (640,2048) 172.4 / 171.3 / 172.1 (100, 200), 3 x (384,2048) 176.6 /
+  //               175.4 / 176.8 (108, 216); 1 x (640,2560) 190.8 / 192.0 / 191.0 (100, 250), 2 x (512,2048) 176.1 / 174.9 / 175.9 (128, 256), 8 x
+  //               (256,2048) 173.9 / 173.3 / 172.7 (128, 256), 1 x (640,3072) 211.7 / 215.4 / 211.7 (100, 300), 8 x (256,3072) 218.4 / 221.6 / 217.6
+  //               (128, 384), 2 x (512,4096) 256.1 / 261.7 / 255.7 (128, 512)
+  //   more        64 x (128,128) 95.9 / 93.4 (256), 64 x (128,256) 110.8 / 108.4 / 108.7 (256), 16 x (256,256) 99.4 / 97.2 (256); 16 x (256,512) 120.4 /
+  //               125.8 / 118.2 (256), 3 x (512,512) 121.4 / 120.8 (192), 7 x (384,384) 114.5 / 116.2 (252), 2 x (640,1024) 153.6 / 157.5 / 155.8
+  //               (200), 4 x (512,512) 126.5 / 172.3 (256)
+  const bool images = epi != EPI_BX && tile == 64 && (full <= 128 ? full * longest <= 225 << 10 : full <= 256 && longest <= 256);
   for (int k = 0; k < n; ++k) {
     NsGemm &g = pm.g[k];
     g = ps[k];

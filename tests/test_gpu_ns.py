@@ -193,11 +193,11 @@ def test_tile_choice_keeps_the_bits(gpu, M, N, mode):
 
 
 @pytest.mark.parametrize("E,M,N", [(1, 128, 128), (32, 128, 256), (33, 128, 256), (64, 128, 128), (65, 128, 128), (2, 128, 3072), (2, 128, 3200),
-                                   (8, 256, 512), (9, 256, 512), (16, 256, 256), (3, 384, 640), (2, 512, 768), (1, 640, 640), (1, 768, 768)])
+                                   (32, 128, 1792), (32, 128, 1920), (1, 640, 2304), (1, 640, 2432), (8, 256, 512), (9, 256, 512), (16, 256, 256), (3, 384, 640), (2, 512, 768), (1, 640, 640), (1, 768, 768)])
 @pytest.mark.parametrize("mode", ["bf16", "bf16_x3"])
 def test_mirror_images_of_small_launches(gpu, E, M, N, mode):
     """Where CUs are left over a symmetric product's tiles above the diagonal have workgroups of their own: batches on both sides of
-    the rule's lines (128 tiles of 64 and K = 3072, 256 tiles and K = 256) have the bits that 128-wide tiles give, which have none."""
+    the rule's lines (up to 128 tiles of 64 tiles times K = 225 Ki, beyond 256 tiles and K = 256) have the bits that 128-wide tiles give, which have none."""
     rng = np.random.default_rng(E + M + N)
     X = rng.standard_normal((E, M, N)).astype(np.float32)
     X[E // 2][:, :2] *= 100.0
