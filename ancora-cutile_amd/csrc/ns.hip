@@ -906,6 +906,10 @@ int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
 // and 1024 tiles with gradients added up, smaller tiles would be up to 16 % ahead of 256-wide ones; 512 at 1024 tokens, added up, lose
 // 4 % on 128x64.) The lines in between: 448 tokens 704 tiles 8.0 / 8.2 / 8.6 / 12.5, 832 9.5 / 8.6 / 9.3 / 12.4, 1152 11.5 / 12.2 / 13.0 / 12.7;
 // 640 tokens 640 tiles 10.3 / 10.9 / 10.3 / 14.0, added up 13.4 / 14.2 / 12.1 / 16.7, 960 tiles 12.6 / 10.9 / 11.1 / 14.2.
+// Calls of several weights have the lines of one. Seven weights in 1008 tiles 352 tokens 10.6 / 10.1 / 10.3 / 11.6, added up 12.7 / 11.9 / 11.8 /
+// 17.1; two in 1024 tiles 9.0 / 9.5 / 9.7 / 11.9 (12.6 / 11.5 / 11.9 / 17.1), four 9.7 / 9.3 / 10.0 / 12.0 (12.3 / 11.5 / 11.8 / 17.9); seven in 1152
+// tiles 11.8 / 12.0 / 13.1 / 12.0 (14.8 / 14.3 / 14.9 / 18.1), in 1248 at 256 tokens 10.2 / 10.9 / 11.8 / 11.1 (13.8 / 13.0 / 13.9 / 17.5); added up
+// at 512 tokens 1056 tiles 15.2 / 16.4 / 15.5 / 18.9, seven weights in 1248 17.7 / 16.7 / 16.8 / 20.4.
 int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0;
   bool adds = false;
@@ -914,13 +918,15 @@ int pick_tile_plain(const NsGemm *ps, const int64_t *Es, int n) {
     adds = adds || (ps[k].plain_sum && ps[k].A32 != nullptr);
   }
   for (int k = 0; k < n; ++k) t64 += (double)Es[k] * (ps[k].M / 64) * (ps[k].N / 64) * ((double)ps[k].K / longest);
-  if (t64 <= 512.0) return t64 <= 256.0 || longest <= (adds ? 900.0 : 768.0) ? 64 : kTile128x64;
+  if (t64 <= 512.0) return t64 <= 256.0 || longest <= (adds && t64 > 352.0 ? 900.0 : 768.0) ? 64 : kTile128x64;
   if (longest > 640.0) return t64 <= 1024.0 ? 128 : 256;
+  // beyond 1024 tiles of 64, 128x64 ones no longer fit in two rounds of one per CU
+  const bool third = t64 > 1024.0 && t64 <= (adds ? 1070.0 : 1300.0);
   if (longest <= 448.0) {
-    if (t64 <= 768.0 || (t64 > 990.0 && t64 <= 1300.0)) return 64;
+    if (t64 <= 768.0 || third) return 64;
     if (t64 <= (adds && longest > 192.0 ? 1450.0 : 1536.0)) return kTile128x64;
   } else {
-    if ((t64 <= 640.0 && !(adds && longest > 576.0)) || (t64 > 1024.0 && t64 <= 1300.0)) return 64;
+    if ((t64 <= 640.0 && !(adds && longest > 576.0)) || third) return 64;
     if ((t64 <= 1024.0 && !adds) || (t64 > 768.0 && t64 <= 990.0) || (t64 > 1300.0 && t64 <= (adds || longest > 544.0 ? 1450.0 : 1536.0)))
       return kTile128x64;
   }

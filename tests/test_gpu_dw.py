@@ -381,11 +381,11 @@ def test_accumulated_micro_batches_against_one_batch(gpu):
 
 
 @pytest.mark.parametrize("T,K,N,n", [(928, 640, 1792, 1), (928, 384, 3072, 1), (1504, 1024, 2048, 1), (32, 512, 1280, 5), (448, 768, 2304, 2),
-                                     (96, 1408, 1024, 4), (608, 1408, 1024, 4), (512, 1024, 2816, 1)])
+                                     (96, 1408, 1024, 4), (608, 1408, 1024, 4), (512, 1024, 2816, 1), (352, 896, 4608, 1), (256, 1280, 2048, 2)])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_tiles_of_128x64(gpu, T, K, N, n, accumulate):
-    """Calls in the ranges that run on 128x64 tiles (257 .. 512 tiles of 64 beyond 900 tokens, 769 .. 990 and 1301 .. 1450 up to 448,
-    769 .. 990, 1301 .. 1450 and, written, 641 .. 1024 up to 640), with one K tile, fewer than the ring has stages, and remainders of a
+    """Calls in the ranges that run on 128x64 tiles (257 .. 512 tiles of 64 beyond 900 tokens, 769 .. 1024 and 1301 .. 1450, added up
+    1071 .. 1450, up to 448, 769 .. 990, 1301 .. 1450 and, written, 641 .. 1024 up to 640), with one K tile, fewer than the ring has stages, and remainders of a
     round: the fp64 product, and for n weights the bits each has alone."""
     from ancora_cutile_amd import DevBuf
     from ancora_cutile_amd.grads import gemm_dW, DwWorkspace
