@@ -854,10 +854,11 @@ struct ChainProb {
 //   with the update of the weight, the whole step of one: (1024,2048) 167.5 / 172.2 (512), (1024,2304) 185.7 / 182.2 (576), (1536,1536) 279.8 /
 //               285.1 (576), (1024,2560) 191.0 / 187.0, (1280,2048) 221.5 / 225.5 (640), (1280,2304) 230.4 / 235.3 (720), (1024,3072) 199.8 /
 //               200.1 (768), (1024,3328) 210.1 / 207.0 (832): level to 2 % from 512 to 832 tiles, and one line in between
-// What the lines and the 64x64 blocks on the diagonal, with a second store below them, cost: against earlier lines and whole 256-wide
-// blocks 20 x (1024,1024) and 60 x (512,512) 1.6 .. 2 %, batches of (128,128) 2 .. 4 % (12: 77.6 -> 80.6), launches of 257 .. 330
-// workgroups 2 .. 4 % (28 x (256,256) 131 -> 136, 14 x (384,384) 158 -> 161, 8 x (512,512) 168 -> 172); 565 batches of 1 .. 60 matrices of
-// 23 shapes are 5.7 % faster in the mean.
+// What the lines and the 64x64 blocks on the diagonal, with a second store below them, cost against earlier lines and whole
+// 256-wide blocks: batches of (128,128) 1 .. 3.5 % (12: 77.8 -> 80.5, 40: 82.4 -> 84.3, 100: 121.0 -> 124.2), 4 x (256,256) 87.8 -> 89.1. Launches
+// of 257 .. 330 workgroups are level (28 x (256,256) 137.4 -> 136.9, 14 x (384,384) 163.7 -> 161.9, 8 x (512,512) 174.8 -> 175.9), the rest gains
+// (20 x (256,256) 125.7 -> 110.8, 60 x (512,512) 767 -> 757, 20 x (1024,1024) 871 -> 827; 565 batches of 1 .. 60 matrices of 23 shapes
+// 5.7 % in the mean).
 int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0, t128 = 0.0, t256 = 0.0, several = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
