@@ -856,9 +856,9 @@ struct ChainProb {
 //               200.1 (768), (1024,3328) 210.1 / 207.0 (832): level to 2 % from 512 to 832 tiles, and one line in between
 // What the lines and the 64x64 blocks on the diagonal, with a second store below them, cost against earlier lines and whole
 // 256-wide blocks: batches of (128,128) 1 .. 3.5 % (12: 77.8 -> 80.5, 40: 82.4 -> 84.3, 100: 121.0 -> 124.2), 4 x (256,256) 87.8 -> 89.1. Launches
-// of 257 .. 330 workgroups are level (28 x (256,256) 137.4 -> 136.9, 14 x (384,384) 163.7 -> 161.9, 8 x (512,512) 174.8 -> 175.9), the rest gains
-// (20 x (256,256) 125.7 -> 110.8, 60 x (512,512) 767 -> 757, 20 x (1024,1024) 871 -> 827; 565 batches of 1 .. 60 matrices of 23 shapes
-// 5.7 % in the mean).
+// of 257 .. 330 workgroups are level on one card and 1 .. 5 % slower on another (28 x (256,256) 137.4 -> 136.9, 130.6 -> 137.2; 14 x (384,384) 163.7 ->
+// 161.9, 153.8 -> 155.8; 8 x (512,512) 174.8 -> 175.9, 160.8 -> 165.0). The rest gains (20 x (256,256) 125.7 -> 110.8, 60 x (512,512) 767 -> 757,
+// 20 x (1024,1024) 871 -> 827; 565 batches of 1 .. 60 matrices of 23 shapes 5.7 % in the mean).
 int pick_tile(int epi, const NsGemm *ps, const int64_t *Es, int n) {
   double longest = 0.0, t64 = 0.0, t128 = 0.0, t256 = 0.0, several = 0.0;
   for (int k = 0; k < n; ++k) longest = ps[k].K > longest ? (double)ps[k].K : longest;
