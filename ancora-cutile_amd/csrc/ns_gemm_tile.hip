@@ -236,9 +236,16 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   constexpr int NB = WM * WN;
   uint32_t pre_h[NB][8], pre_l[NB][8];                  // 16 bf16, or (pre_l, 8-bit low halves) 16 bytes in the first 4
   float drow[WM][NR];
+  // With several terms the K loop brings both halves of all rows of the tile's columns of X through LDS, those at the output position
+  // among them: they are kept in registers as they pass, and X is not read again behind the loop (a launch over the
+  // projections of six 640-wide layers reads 295 MB instead of 368, 109 -> 106 us, the last one with the weight update 140 -> 134; chains of
+  // 24 x (640,1792) 1016 -> 1010, 24 x (512,512) 309 -> 304, 40 x (256,768) 248 -> 240; the full step of a model of 4 layers, hidden size 512,
+  // 525 -> 520). One workgroup per CU (the ring of four) has them earlier by a request before the loop.
+  constexpr bool kKeep = EPI == EPI_BX && !PLAINV && (NW == 8 || kRing == 3);
   if constexpr (EPI == EPI_BX && !PLAINV && NW == 4) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
+      if (kKeep && nterms > 1) break;
       const int64_t xo = mn + (p.x_panel ? pan_of(b) : (int64_t)(gi_w + (b / WN) * 32 + lrow) * N + gj_w + (b % WN) * 32 + c0);
       const int64_t xr = p.x_panel ? RS * 32 : (int64_t)RS * N;
 #pragma unroll
@@ -465,7 +472,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
       };
       const int np = K / 32;
       // The first fragments of step k are in registers when it begins, the others are read under its matrix
-      // instructions. Before its last product a wavefront waits for its own DMA of step k + 1 and the workgroup meets:
+      // instructions (the low ones of k 0..15 take the place of those of 16..31, which leaves eight wavefronts the registers for kKeep). Before its last product a wavefront waits for its own DMA of step k + 1 and the workgroup meets:
       // everybody has read stage k, which takes the DMA of step k + kPairs, and the next step's first fragments are read
       // under that product. B's fragments of k 0..15 and 16..31 change places from step to step.
 #pragma unroll
@@ -482,7 +489,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
         }
         return;
       }
-      bf16x8 ah[2][WM], bh[2][WN], al[2][WM], bl[2][WN];
+      bf16x8 ah[2][WM], bh[2][WN], al[WM], bl[WN];
       auto rd_a = [&](const unsigned char *half, int kk, bf16x8 (&f)[WM]) {
 #pragma unroll
         for (int i = 0; i < WM; ++i) f[i] = frag(TrA{}, half, wm * WM + i, kk, 32, TM);
@@ -494,37 +501,56 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
       auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
       rd_a(lds, 0, ah[0]);
       rd_b(lds + at_b, 0, bh[0]);
+      // (see kKeep: the step's rows of X are those of block row bi of this wavefront's outputs)
+      auto keep = [&](const unsigned char *st, int step) {
+#pragma unroll
+        for (int bi = 0; bi < WM; ++bi)
+          if (step == (gi_w >> 5) + bi) {
+#pragma unroll
+            for (int bj = 0; bj < WN; ++bj) {
+              const unsigned char *q = st + kPanA + (wn * WN + bj) * 2048 + lrow * 64 + c0 * 2;
+#pragma unroll
+              for (int r = 0; r < NR; ++r) {
+                ld_run<RUN * 2>(q + r * RS * 64, &pre_h[bi * WN + bj][r * (RUN / 2)]);
+                ld_run<RUN * 2>(q + kLow + r * RS * 64, &pre_l[bi * WN + bj][r * (RUN / 2)]);
+              }
+            }
+          }
+      };
       auto body = [&](auto steady, int step, auto s0v) {
         constexpr int s0 = decltype(s0v)::value % kPairs, x = decltype(s0v)::value % 2, y = 1 - x;
         const unsigned char *st = lds + s0 * kPair, *nx = lds + (s0 + 1) % kPairs * kPair;
         const bool more = decltype(steady)::value || step + 1 < np, refill = decltype(steady)::value || step + kPairs < np;
         rd_a(st, 1, ah[1]);
         rd_b(st + at_b, 1, bh[y]);
+        if constexpr (kKeep) keep(st, step);
         fence();
         mma(ah[0], bh[x]);                                    // hh 0..15
         fence();
-        rd_b(st + kLow + at_b, 1, bl[1]);
-        if (NT == 3) rd_a(st + kLow, 1, al[1]);
+        rd_b(st + kLow + at_b, 1, bl);
+        if (NT == 3) rd_a(st + kLow, 1, al);
         fence();
         mma(ah[1], bh[y]);                                    // hh 16..31
+        mma(ah[1], bl);                                       // hl 16..31
         fence();
-        rd_b(st + kLow + at_b, 0, bl[0]);
-        if (NT == 3) rd_a(st + kLow, 0, al[0]);
+        rd_b(st + kLow + at_b, 0, bl);
         fence();
-        mma(ah[1], bl[1]);                                    // hl 16..31
         if (NT == 3) {
-          mma(al[1], bh[y]);                                  // lh 16..31
-          mma(ah[0], bl[0]);                                  // hl 0..15
+          mma(al, bh[y]);                                     // lh 16..31
+          fence();
+          rd_a(st + kLow, 0, al);
+          fence();
+          mma(ah[0], bl);                                     // hl 0..15
+          fence();
         }
-        fence();
         if (decltype(steady)::value || step + kPairs <= np) wait_vm<(kPairs - 2) * kIpp>(); else wait_vm<0>();
         lds_barrier();
         if (refill) issue_pair(lds + s0 * kPair);
         if (NT == 3 && more) rd_a(nx, 0, ah[0]);
         if (more) rd_b(nx + at_b, 0, bh[y]);
         fence();
-        if (NT == 3) mma(al[0], bh[x]);                       // lh 0..15
-        else         mma(ah[0], bl[0]);                       // (of two terms: hl 0..15)
+        if (NT == 3) mma(al, bh[x]);                          // lh 0..15
+        else         mma(ah[0], bl);                          // (of two terms: hl 0..15)
         fence();
         if (NT != 3 && more) rd_a(nx, 0, ah[0]);
       };
@@ -563,6 +589,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   if constexpr (EPI == EPI_BX && !PLAINV && NW > 4) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
+      if (kKeep && nterms > 1) break;
       const int64_t xo = mn + (p.x_panel ? pan_of(b) : (int64_t)(gi_w + (b / WN) * 32 + lrow) * N + gj_w + (b % WN) * 32 + c0);
       const int64_t xr = p.x_panel ? RS * 32 : (int64_t)RS * N;
 #pragma unroll
