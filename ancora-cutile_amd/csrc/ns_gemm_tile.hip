@@ -241,8 +241,9 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   // among them: they are kept in registers as they pass, and X is not read again behind the loop (a launch over the
   // projections of six 640-wide layers reads 295 MB instead of 368, 109 -> 106 us, the last one with the weight update 140 -> 134; chains of
   // 24 x (640,1792) 1016 -> 1010, 24 x (512,512) 309 -> 304, 40 x (256,768) 248 -> 240; the full step of a model of 4 layers, hidden size 512,
-  // 525 -> 520). One workgroup per CU (the ring of four) has them earlier by a request before the loop.
-  constexpr bool kKeep = EPI == EPI_BX && !PLAINV && (NW == 8 || kRing == 3);
+  // 525 -> 520). One workgroup per CU (the ring of four) has them earlier by a request before the loop. Eight wavefronts make room by
+  // sharing the registers of a step's low fragments (kShare); four have it, and lose by the sharing (4 x (512,1536) 180 -> 184 us per chain).
+  constexpr bool kKeep = EPI == EPI_BX && !PLAINV && (NW == 8 || kRing == 3), kShare = EPI == EPI_BX && NW == 8;
   if constexpr (EPI == EPI_BX && !PLAINV && NW == 4) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -473,7 +474,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
       };
       const int np = K / 32;
       // The first fragments of step k are in registers when it begins, the others are read under its matrix
-      // instructions (the low ones of k 0..15 take the place of those of 16..31, which leaves eight wavefronts the registers for kKeep). Before its last product a wavefront waits for its own DMA of step k + 1 and the workgroup meets:
+      // instructions (kShare: the low ones of k 0..15 take the place of those of 16..31, which leaves eight wavefronts the registers for kKeep). Before its last product a wavefront waits for its own DMA of step k + 1 and the workgroup meets:
       // everybody has read stage k, which takes the DMA of step k + kPairs, and the next step's first fragments are read
       // under that product. B's fragments of k 0..15 and 16..31 change places from step to step.
 #pragma unroll
@@ -490,7 +491,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
         }
         return;
       }
-      bf16x8 ah[2][WM], bh[2][WN], al[WM], bl[WN];
+      bf16x8 ah[2][WM], bh[2][WN], al[kShare ? 1 : 2][WM], bl[kShare ? 1 : 2][WN];
       auto rd_a = [&](const unsigned char *half, int kk, bf16x8 (&f)[WM]) {
 #pragma unroll
         for (int i = 0; i < WM; ++i) f[i] = frag(TrA{}, half, wm * WM + i, kk, 32, TM);
@@ -528,30 +529,46 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
         fence();
         mma(ah[0], bh[x]);                                    // hh 0..15
         fence();
-        rd_b(st + kLow + at_b, 1, bl);
-        if (NT == 3) rd_a(st + kLow, 1, al);
-        fence();
-        mma(ah[1], bh[y]);                                    // hh 16..31
-        mma(ah[1], bl);                                       // hl 16..31
-        fence();
-        rd_b(st + kLow + at_b, 0, bl);
-        fence();
-        if (NT == 3) {
-          mma(al, bh[y]);                                     // lh 16..31
+        if constexpr (kShare) {
+          rd_b(st + kLow + at_b, 1, bl[0]);
+          if (NT == 3) rd_a(st + kLow, 1, al[0]);
           fence();
-          rd_a(st + kLow, 0, al);
+          mma(ah[1], bh[y]);                                  // hh 16..31
+          mma(ah[1], bl[0]);                                  // hl 16..31
           fence();
-          mma(ah[0], bl);                                     // hl 0..15
+          rd_b(st + kLow + at_b, 0, bl[0]);
           fence();
+          if (NT == 3) {
+            mma(al[0], bh[y]);                                // lh 16..31
+            fence();
+            rd_a(st + kLow, 0, al[0]);
+            fence();
+            mma(ah[0], bl[0]);                                // hl 0..15
+          }
+        } else {
+          rd_b(st + kLow + at_b, 1, bl[1]);
+          if (NT == 3) rd_a(st + kLow, 1, al[1]);
+          fence();
+          mma(ah[1], bh[y]);
+          fence();
+          rd_b(st + kLow + at_b, 0, bl[0]);
+          if (NT == 3) rd_a(st + kLow, 0, al[0]);
+          fence();
+          mma(ah[1], bl[1]);
+          if (NT == 3) {
+            mma(al[1], bh[y]);
+            mma(ah[0], bl[0]);
+          }
         }
+        fence();
         if (decltype(steady)::value || step + kPairs <= np) wait_vm<(kPairs - 2) * kIpp>(); else wait_vm<0>();
         lds_barrier();
         if (refill) issue_pair(lds + s0 * kPair);
         if (NT == 3 && more) rd_a(nx, 0, ah[0]);
         if (more) rd_b(nx + at_b, 0, bh[y]);
         fence();
-        if (NT == 3) mma(al, bh[x]);                          // lh 0..15
-        else         mma(ah[0], bl);                          // (of two terms: hl 0..15)
+        if (NT == 3) mma(al[0], bh[x]);                       // lh 0..15
+        else         mma(ah[0], bl[0]);                       // (of two terms: hl 0..15)
         fence();
         if (NT != 3 && more) rd_a(nx, 0, ah[0]);
       };
