@@ -274,8 +274,8 @@ k_ns_prep(float *__restrict__ X, const float *__restrict__ recip, int64_t mn, in
 // in r directions that are spread over the rows (outlier columns). Read from Fh (bf16, zero
 // diagonal). kCondParts blocks per matrix, each over M*M/kCondParts consecutive elements: lane t
 // takes the 8-element vectors t, t+256, ..., adds their squares left to right in fp32, widens to
-// fp64; butterfly over the wavefront; the 4 wavefront sums in order. k_ns_colstat and k_ns_classify combine the
-// kCondParts partial sums by the same butterfly (one wavefront, a part per lane); classify leaves the sum for
+// fp64; butterfly over the wavefront; the 4 wavefront sums in order. k_ns_colstat and k_ns_classify_order combine the
+// kCondParts partial sums by the same butterfly (one wavefront, a part per lane); whichever decides leaves the sum for
 // the products to read. (64 parts: a single 1024x1024 matrix in 8 parts took 36 us, latency of a
 // few wavefronts.)
 struct NsCondArgs {
@@ -283,6 +283,7 @@ struct NsCondArgs {
   int blocks[kMaxGroups];
   const uint16_t *Fh[kMaxGroups];
   double *out[kMaxGroups];
+  int32_t *arrived[kMaxGroups];      // (E) cleared for k_ns_colstat<true>, or null
   int M[kMaxGroups];
 };
 __global__ void __launch_bounds__(kThreads) k_ns_cond(NsCondArgs a) {
@@ -301,6 +302,7 @@ __global__ void __launch_bounds__(kThreads) k_ns_cond(NsCondArgs a) {
 #pragma unroll
     for (int w = 1; w < kThreads / 64; ++w) t = t + wave_sum[w];
     a.out[q][b] = t;
+    if (a.arrived[q] != nullptr && b % kCondParts == 0) a.arrived[q][b / kCondParts] = 0;
   }
 }
 
@@ -319,8 +321,10 @@ __global__ void __launch_bounds__(kThreads) k_ns_cond(NsCondArgs a) {
 // 16-byte loads, the 32 row groups walk the M rows (fp64 sums of squares: the pair entries run on
 // unnormalised input) and are added in order through LDS; the block leaves (sum c^2, sum c^4) of
 // its columns (one wavefront's butterfly). A block returns at
-// once unless the matrix's proxy asks for the statistic. k_ns_classify: one wavefront per matrix adds
-// the partial sums in order and writes the flag every later product reads.
+// once unless the matrix's proxy asks for the statistic. Then the partial sums are added in order and the flag is written that
+// every later product reads: DECIDE, by the matrix's first block where nobody asks and by the last to arrive where it does;
+// otherwise by k_ns_classify_order, for batches that a gated launch takes in another order. (A launch of its own, one wavefront per
+// matrix, was almost all start and end: the step of one (1024,3072) weight 216.7 -> 210.0 us without it.)
 struct WideRule {
   double near_lo, lo, hi;    // in units of the proxy N * ||offdiag(A0)||^2; near_lo == lo: no near range
   double near_diff;          // > 0: in the near range the gate takes a matrix whose proxy exceeds its column
@@ -353,12 +357,13 @@ __device__ __host__ __forceinline__ bool wants_colstat(const WideRule &r, double
 struct NsColArgs {
   int n;
   int blocks[kMaxGroups];          // colstat: E * parts, classify: E
-  double *sum[kMaxGroups];         // (E) the proxy's sum, classify's output
+  double *sum[kMaxGroups];         // (E) the proxy's sum, for the products to read
   const uint16_t *Xh[kMaxGroups];  // (E, M, N) row-major
   const double *cond[kMaxGroups];  // (E, kCondParts)
   double *part[kMaxGroups];        // (E, parts, 2)
   int32_t *flag[kMaxGroups];       // (E) or null (no wide gate)
   int32_t *order[kMaxGroups];      // (E) or null
+  int32_t *arrived[kMaxGroups];    // (E) blocks of k_ns_colstat<true> whose partial sums are written
   double gate[kMaxGroups];         // matrices whose sum exceeds it take a gate's terms some time
   int M[kMaxGroups], N[kMaxGroups], parts[kMaxGroups];
   WideRule rule[kMaxGroups];
@@ -369,6 +374,28 @@ constexpr int kColLanes = kColBlock / 8, kColRowGroups = kThreads / kColLanes;
 constexpr int kColRowStep = 4;      // every fourth row: the thresholds are coarse (a quarter of the proxy; 1.3
                                     // against 1.0 and 1.9+), a quarter of the rows places a matrix as well as all
                                     // of them (flat columns read 1 + 8/M more) and costs a quarter of the bytes
+// The wide gate's decision on matrix e, from its proxy's sum and, where that asks for them, the column norms
+__device__ __forceinline__ bool is_wide(const NsColArgs &a, int q, int e, double sum) {
+  const WideRule r = a.rule[q];
+  const double p = sum * (double)a.N[q];
+  if (p > r.lo && p < r.hi) return true;
+  if (!wants_colstat(r, p)) return false;
+  const double *c = a.part[q] + (int64_t)e * a.parts[q] * 2;
+  double s2 = c[0], s4 = c[1], lightest = c[0];
+#pragma unroll 16
+  for (int i = 1; i < a.parts[q]; ++i) {
+    const double x2 = c[2 * i], x4 = c[2 * i + 1];
+    s2 = s2 + x2;
+    s4 = s4 + x4;
+    lightest = x2 < lightest ? x2 : lightest;
+  }
+  const double colc = s2 > 0.0 ? (double)a.N[q] * s4 / (s2 * s2) : 1.0;
+  // outlier columns: the share of the mass outside them, from the lightest block of columns
+  const double bulk = s2 > 0.0 ? (double)a.parts[q] * lightest / s2 : 1.0;
+  if (p < r.hi && r.near_diff > 0.0) return p - colc > r.near_diff;
+  return colc < kColcFrac * p || (p >= r.hi && bulk < kBulkShare);
+}
+template <bool DECIDE>
 __global__ void __launch_bounds__(kThreads) k_ns_colstat(NsColArgs a) {
   __shared__ double colsum[kColRowGroups][kColBlock];
   __shared__ double wave_sum[2][kColBlock / 64];
@@ -376,7 +403,14 @@ __global__ void __launch_bounds__(kThreads) k_ns_colstat(NsColArgs a) {
   while (q + 1 < a.n && b >= a.blocks[q]) { b -= a.blocks[q]; ++q; }
   const int e = b / a.parts[q], part = b % a.parts[q];
   const int M = a.M[q], N = a.N[q];
-  if (!wants_colstat(a.rule[q], cond_sum(a.cond[q] + (int64_t)e * kCondParts) * (double)N)) return;
+  const double sum = cond_sum(a.cond[q] + (int64_t)e * kCondParts);
+  if (!wants_colstat(a.rule[q], sum * (double)N)) {
+    if (DECIDE && part == 0 && threadIdx.x == 0) {
+      a.sum[q][e] = sum;
+      a.flag[q][e] = is_wide(a, q, e, sum) ? 1 : 0;
+    }
+    return;
+  }
   // lane (rg, cg): columns part*64 + 8*cg .. +7 (one 16-byte load per row), rows 4 rg, 4 (rg + 32), ...
   const int cg = (int)threadIdx.x % kColLanes, rg = (int)threadIdx.x / kColLanes;
   const int j = part * kColBlock + 8 * cg;
@@ -413,45 +447,20 @@ __global__ void __launch_bounds__(kThreads) k_ns_colstat(NsColArgs a) {
     double *out = a.part[q] + ((int64_t)e * a.parts[q] + part) * 2;
     out[0] = t2;
     out[1] = t4;
+    if constexpr (DECIDE) {
+      if (__hip_atomic_fetch_add(a.arrived[q] + e, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == a.parts[q] - 1) {
+        a.sum[q][e] = sum;
+        a.flag[q][e] = is_wide(a, q, e, sum) ? 1 : 0;
+      }
+    }
   }
 }
 static_assert(kColBlock % 64 == 0 && kColBlock <= kThreads, "k_ns_colstat: whole wavefronts of one lane per column in the final sum");
-// The wide gate's decision on matrix e, from its proxy's sum and, where that asks for them, the column norms
-__device__ __forceinline__ bool is_wide(const NsColArgs &a, int q, int e, double sum) {
-  const WideRule r = a.rule[q];
-  const double p = sum * (double)a.N[q];
-  if (p > r.lo && p < r.hi) return true;
-  if (!wants_colstat(r, p)) return false;
-  const double *c = a.part[q] + (int64_t)e * a.parts[q] * 2;
-  double s2 = c[0], s4 = c[1], lightest = c[0];
-#pragma unroll 16
-  for (int i = 1; i < a.parts[q]; ++i) {
-    const double x2 = c[2 * i], x4 = c[2 * i + 1];
-    s2 = s2 + x2;
-    s4 = s4 + x4;
-    lightest = x2 < lightest ? x2 : lightest;
-  }
-  const double colc = s2 > 0.0 ? (double)a.N[q] * s4 / (s2 * s2) : 1.0;
-  // outlier columns: the share of the mass outside them, from the lightest block of columns
-  const double bulk = s2 > 0.0 ? (double)a.parts[q] * lightest / s2 : 1.0;
-  if (p < r.hi && r.near_diff > 0.0) return p - colc > r.near_diff;
-  return colc < kColcFrac * p || (p >= r.hi && bulk < kBulkShare);
-}
-// The flag alone, one wavefront per matrix: for batches that no gated launch takes in another order.
-__global__ void __launch_bounds__(kThreads) k_ns_classify(NsColArgs a) {
-  int e = (int)(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6)), q = 0;
-  while (q + 1 < a.n && e >= a.blocks[q]) { e -= a.blocks[q]; ++q; }
-  if (e >= a.blocks[q]) return;
-  const double sum = cond_sum(a.cond[q] + (int64_t)e * kCondParts);
-  if ((threadIdx.x & 63) != 0) return;
-  a.sum[q][e] = sum;
-  if (a.flag[q] != nullptr) a.flag[q][e] = is_wide(a, q, e, sum) ? 1 : 0;
-}
 // One block per batch: the wide gate's flag per matrix, and the order in which the launches of a gated
 // iteration take the matrices. A matrix that takes a gate's terms has three times the products of one that does not;
 // such matrices lie together (the tall weights of a stack) and a launch's sequence is cut into eight runs, one per XCD,
 // so they are dealt over the runs in turn, each run's first. (Qwen3-0.6B set, 59 of 196 matrices gated, A = X X^T of
-// iteration 2: 1114 -> 729 us, for 1 to 3 us that this kernel takes longer than k_ns_classify.)
+// iteration 2: 1114 -> 729 us, for 1 to 3 us.)
 constexpr int kClassifyThreads = 1024, kMaxOrdered = 8192;
 __global__ void __launch_bounds__(kClassifyThreads) k_ns_classify_order(NsColArgs a) {
   constexpr int kWaves = kClassifyThreads / 64, kAhead = 4;
@@ -548,7 +557,7 @@ struct SplitPlan {
   float gate_tau[kGateIters];
   unsigned gate_bx;
   // The wide gate: a matrix whose proxy lies in (wide_lo, wide_hi), or outside it with a column
-  // statistic that says so (k_ns_classify), adds the residual of X to A = X X^T from iteration
+  // statistic that says so (is_wide), adds the residual of X to A = X X^T from iteration
   // wide_gram_from on and the residuals of X, F and Boff to all three products from iteration
   // wide_all_from on. wide_hi == 0: no such gate.
   float wide_lo, wide_hi, wide_near;   // wide_near: start of the near range below the band (== wide_lo: none)
@@ -1156,8 +1165,12 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       // the proxy of every problem that gates a later product, from the Fh this launch wrote
       NsCondArgs ca{};
       int blocks = 0;
+      bool any_ordered = false;
+      for (int q = 0; q < n; ++q) any_ordered = any_ordered || (cp[q].pl.sp.any_gate(steps) && ordered(q));
       for (int q = 0; q < n; ++q) {
         if (!cp[q].pl.sp.any_gate(steps)) continue;
+        ANC_REQUIRE(cp[q].pl.sp.wide(), "Newton-Schulz chain: a plan with gates has the wide one");
+        ca.arrived[ca.n] = any_ordered ? nullptr : cp[q].pl.order;       // (no order: its place counts arrivals)
         ca.Fh[ca.n] = cp[q].pl.Fh; ca.out[ca.n] = cp[q].pl.condpart; ca.M[ca.n] = (int)cp[q].M;
         ca.blocks[ca.n] = (int)(cp[q].E * kCondParts);
         blocks += ca.blocks[ca.n];
@@ -1168,8 +1181,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       ANC_LAUNCH_CHECK();
       // the wide gate's decision per matrix, from the proxy and, where it asks, the column norms
       NsColArgs cs{}, cf{};
-      int cs_blocks = 0, cf_mats = 0;
-      bool any_ordered = false;
+      int cs_blocks = 0;
       for (int q = 0; q < n; ++q) {
         const Plan &pl = cp[q].pl;
         if (!pl.sp.any_gate(steps)) continue;
@@ -1179,26 +1191,24 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
         for (int j = 1; j < steps; ++j)
           if (pl.sp.gated(j)) cs.gate[i] = std::min(cs.gate[i], (double)pl.sp.gate_tau[j] / (double)cp[q].N);
         cs.order[i] = ordered(q) ? pl.order : nullptr;
-        any_ordered = any_ordered || ordered(q);
+        cs.arrived[i] = any_ordered ? nullptr : pl.order;
         cs.M[i] = (int)cp[q].M; cs.N[i] = (int)cp[q].N; cs.parts[i] = pl.col_parts;
         cs.rule[i] = WideRule{(double)pl.sp.wide_near, (double)pl.sp.wide_lo, (double)pl.sp.wide_hi,
                               (double)pl.sp.wide_near_diff};
-        cs.blocks[i] = (int)(cp[q].E * pl.col_parts);    // 0 without a wide gate
+        cs.blocks[i] = (int)(cp[q].E * pl.col_parts);
         cs_blocks += cs.blocks[i];
         ++cs.n;
       }
-      cf = cs;
-      for (int i = 0, q = 0; q < n; ++q)
-        if (cp[q].pl.sp.any_gate(steps)) { cf.blocks[i++] = (int)cp[q].E; cf_mats += (int)cp[q].E; }
-      if (cs_blocks > 0) {
-        hipLaunchKernelGGL(k_ns_colstat, dim3((unsigned)cs_blocks), dim3(kThreads), 0, s, cs);
+      if (any_ordered) hipLaunchKernelGGL((k_ns_colstat<false>), dim3((unsigned)cs_blocks), dim3(kThreads), 0, s, cs);
+      else             hipLaunchKernelGGL((k_ns_colstat<true>), dim3((unsigned)cs_blocks), dim3(kThreads), 0, s, cs);
+      ANC_LAUNCH_CHECK();
+      if (any_ordered) {
+        cf = cs;
+        for (int i = 0, q = 0; q < n; ++q)
+          if (cp[q].pl.sp.any_gate(steps)) cf.blocks[i++] = (int)cp[q].E;
+        hipLaunchKernelGGL(k_ns_classify_order, dim3((unsigned)cf.n), dim3(kClassifyThreads), 0, s, cf);
         ANC_LAUNCH_CHECK();
       }
-      if (any_ordered)
-        hipLaunchKernelGGL(k_ns_classify_order, dim3((unsigned)cf.n), dim3(kClassifyThreads), 0, s, cf);
-      else
-        hipLaunchKernelGGL(k_ns_classify, dim3((unsigned)((cf_mats + kThreads / 64 - 1) / (kThreads / 64))), dim3(kThreads), 0, s, cf);
-      ANC_LAUNCH_CHECK();
     }
     {
       AncProfScope prof(ANC_PROF_NS_BMAT, s);

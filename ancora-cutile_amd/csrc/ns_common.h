@@ -144,7 +144,7 @@ struct NsGemm {
   double cond_thresh;
   int nterms_hard;
   const int32_t *order;      // (E) or null (as they come): the matrix in each place of the launch's sequence of matrices
-  // Second gate: a matrix that k_ns_classify flagged (a spectrum spread over decades, many
+  // Second gate: a matrix flagged from its statistics (a spectrum spread over decades, many
   // moderately large columns, a low-rank signal over weak noise) multiplies nterms_wide terms;
   // wide_flag null or nterms_wide 0 = no such gate. It takes precedence over the gate above. With
   // lo_gated set, the residual outputs Fl / Bl are written for such matrices only (else for every

@@ -95,7 +95,7 @@ def statistics(Xh, Fh0):
     """(proxy, colc, bulk) as the kernels compute them: the proxy N * ||Fh||_F^2 from the first
     iteration's bf16 off-diagonal A (k_ns_cond), the column concentration and the share of the mass
     in the lightest block of 64 columns from every fourth row of the input's high half
-    (k_ns_colstat, k_ns_classify)."""
+    (k_ns_colstat, is_wide)."""
     M, N = Xh.shape
     proxy = float(N) * float(np.sum(Fh0.astype(np.float64) ** 2))
     c2 = np.sum(Xh[::COL_ROW_STEP].astype(np.float64) ** 2, axis=0)
@@ -110,7 +110,7 @@ def statistics(Xh, Fh0):
 
 
 def wide_flag(plan, proxy, colc, bulk):
-    """k_ns_classify's decision."""
+    """is_wide's decision."""
     if not plan.wide:
         return False
     if TAU_WIDE_LO < proxy < TAU_WIDE_HI:

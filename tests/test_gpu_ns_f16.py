@@ -64,3 +64,35 @@ def test_zero_tiny_and_non_finite_matrices_on_fp16(gpu, sched):
     got = run_ns(X, schedule=sched, mode="bf16_late3")
     assert np.all(got[1] == 0.0) and np.all(np.isnan(got[3]))
     assert rel_fro(got[0], host_ns(X[0], sched, 5)) < 6e-4
+
+
+@pytest.mark.parametrize("E,M,N", [(1, 1024, 1024), (1, 1024, 4096), (3, 1024, 1152), (7, 1152, 2304)])
+def test_the_last_block_decides_on_the_column_statistic(gpu, E, M, N):
+    """Batches that no launch takes in another order: matrices in the band (no statistic asked for), above it with columns that
+    explain the proxy and without, and plain ones. The flags are the model's, each call again (the count of arrivals starts over),
+    and the matrices have the bits they have alone."""
+    from ancora_cutile_amd.muon_ns import PE_SCHEDULE
+    from test_gpu_ns import _hard_count
+    rng = np.random.default_rng(E + N)
+    kinds = ("lowrank", "cols", "plain", "band", "lowrank", "cols", "band")
+
+    def make(kind):
+        X = rng.standard_normal((M, N)).astype(np.float32)
+        if kind == "lowrank":
+            X = (_input(M, 8, "plain", 7) @ _input(8, N, "plain", 8) + 0.01 * X).astype(np.float32)
+        elif kind == "band":
+            X[:, rng.choice(N, N // 10, replace=False)] *= 10
+        elif kind == "cols":
+            X[:, rng.choice(N, N // 100, replace=False)] *= 100
+        return X
+    X = np.stack([make(k) for k in kinds[:E]])
+    wide = sum(k in ("lowrank", "band") for k in kinds[:E])
+    want = run_ns(X, schedule=None)
+    for _ in range(3):
+        assert _hard_count(E, M, N, "bf16_late3")[0] == wide
+        assert bits_equal(run_ns(X, schedule=None), want)
+    for e in range(E):
+        assert bits_equal(run_ns(X[e: e + 1], schedule=None)[0], want[e]), e
+        assert _hard_count(1, M, N, "bf16_late3")[0] == int(kinds[e] in ("lowrank", "band")), e
+    run_ns(X[:1], schedule=PE_SCHEDULE)                    # one matrix under the proxy's gates has no order either
+    assert _hard_count(1, M, N)[0] == 1
