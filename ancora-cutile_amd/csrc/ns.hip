@@ -286,6 +286,9 @@ struct NsCondArgs {
   int32_t *arrived[kMaxGroups];      // (E) cleared for k_ns_colstat<true>, or null
   int M[kMaxGroups];
 };
+// 16-byte loads in flight per lane: a part of a 1024x1024 matrix. (One at a time, behind a test for the end: 5.3 -> 4.6 us for one such
+// matrix, 19.3 -> 17.3 for 48, 5.8 TB/s; with loads that the caches keep instead of streamed ones 34.9.)
+constexpr int kCondAhead = 8;
 __global__ void __launch_bounds__(kThreads) k_ns_cond(NsCondArgs a) {
   __shared__ double wave_sum[kThreads / 64];
   int b = (int)blockIdx.x, q = 0;
@@ -293,7 +296,27 @@ __global__ void __launch_bounds__(kThreads) k_ns_cond(NsCondArgs a) {
   const int64_t per = (int64_t)a.M[q] * a.M[q] / kCondParts;
   const uint16_t *src = a.Fh[q] + (int64_t)b * per;          // b = e * kCondParts + part
   double acc = 0.0;
-  for (int64_t v = threadIdx.x; v < per / kRun; v += kThreads) acc = acc + (double)run_sumsq<ANC_BF16>(src, v * kRun, per);
+  const int n = (int)(per / kRun);                           // (per: a multiple of 256)
+  int v = (int)threadIdx.x;
+  auto add = [&](anc_u32x4 r) {                              // run_sumsq of eight elements
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+    float s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float x0 = __uint_as_float(w[k] << 16), x1 = __uint_as_float(w[k] & 0xFFFF0000u);
+      s = s + x0 * x0;
+      s = s + x1 * x1;
+    }
+    acc = acc + (double)s;
+  };
+  for (; v + (kCondAhead - 1) * kThreads < n; v += kCondAhead * kThreads) {
+    anc_u32x4 r[kCondAhead];
+#pragma unroll
+    for (int k = 0; k < kCondAhead; ++k) r[k] = anc_ld_stream((const anc_u32x4 *)src + v + k * kThreads);
+#pragma unroll
+    for (int k = 0; k < kCondAhead; ++k) add(r[k]);
+  }
+  for (; v < n; v += kThreads) add(anc_ld_stream((const anc_u32x4 *)src + v));
   acc = anc_wave_sum_f64(acc);
   if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = acc;
   __syncthreads();
