@@ -40,7 +40,7 @@
 #include <cmath>
 #include <vector>
 
-#include "reduce.h"
+#include "ns_stats.h"
 #include "ns_common.h"
 
 namespace {
@@ -188,6 +188,7 @@ struct NsPrologue {
   float *recip[kMaxGroups];
   uint16_t *Uh[kMaxGroups], *Ul[kMaxGroups];       // Ul null: a bf16 input without a low half,
   uint32_t *zero16[kMaxGroups];                    // whose substitute this kernel clears
+  int32_t *arrived[kMaxGroups];                    // (E) cleared, see NsStatOne
   int64_t mn[kMaxGroups];
 };
 // Sum of squares of one matrix, every square and sum in fp64: lane t adds the 8-element vectors t, t+256, ... in
@@ -217,7 +218,7 @@ __global__ void __launch_bounds__(kThreads) k_pair_prologue(NsPrologue a, float 
   int k = 0;
   if (t > 0.0 && t <= DBL_MAX && !(t >= 0x1p-100 && t <= 0x1p100)) k = -ilogb(sqrt(t));
   const float r = 1.0f / ((float)ldexp(sqrt(t), k) + ldexpf(eps, k));       // (of the matrix times 2^k)
-  if (threadIdx.x == 0) a.recip[q][e] = r;
+  if (threadIdx.x == 0) { a.recip[q][e] = r; a.arrived[q][e] = 0; }
   if (a.Ul[q] == nullptr && e == 0 && threadIdx.x < 4) a.zero16[q][threadIdx.x] = 0u;
   if (k == 0) return;                // (uniform over the block)
   for (int64_t o = (int64_t)threadIdx.x * 8; o < mn; o += (int64_t)kThreads * 8) {
@@ -286,44 +287,12 @@ struct NsCondArgs {
   int32_t *arrived[kMaxGroups];      // (E) cleared for k_ns_colstat<true>, or null
   int M[kMaxGroups];
 };
-// 16-byte loads in flight per lane: a part of a 1024x1024 matrix. (One at a time, behind a test for the end: 5.3 -> 4.6 us for one such
-// matrix, 19.3 -> 17.3 for 48, 5.8 TB/s; with loads that the caches keep instead of streamed ones 34.9.)
-constexpr int kCondAhead = 8;
 __global__ void __launch_bounds__(kThreads) k_ns_cond(NsCondArgs a) {
   __shared__ double wave_sum[kThreads / 64];
   int b = (int)blockIdx.x, q = 0;
   while (q + 1 < a.n && b >= a.blocks[q]) { b -= a.blocks[q]; ++q; }
-  const int64_t per = (int64_t)a.M[q] * a.M[q] / kCondParts;
-  const uint16_t *src = a.Fh[q] + (int64_t)b * per;          // b = e * kCondParts + part
-  double acc = 0.0;
-  const int n = (int)(per / kRun);                           // (per: a multiple of 256)
-  int v = (int)threadIdx.x;
-  auto add = [&](anc_u32x4 r) {                              // run_sumsq of eight elements
-    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
-    float s = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float x0 = __uint_as_float(w[k] << 16), x1 = __uint_as_float(w[k] & 0xFFFF0000u);
-      s = s + x0 * x0;
-      s = s + x1 * x1;
-    }
-    acc = acc + (double)s;
-  };
-  for (; v + (kCondAhead - 1) * kThreads < n; v += kCondAhead * kThreads) {
-    anc_u32x4 r[kCondAhead];
-#pragma unroll
-    for (int k = 0; k < kCondAhead; ++k) r[k] = anc_ld_stream((const anc_u32x4 *)src + v + k * kThreads);
-#pragma unroll
-    for (int k = 0; k < kCondAhead; ++k) add(r[k]);
-  }
-  for (; v < n; v += kThreads) add(anc_ld_stream((const anc_u32x4 *)src + v));
-  acc = anc_wave_sum_f64(acc);
-  if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = acc;
-  __syncthreads();
+  const double t = cond_part(a.Fh[q], a.M[q], b, wave_sum);  // b = e * kCondParts + part
   if (threadIdx.x == 0) {
-    double t = wave_sum[0];
-#pragma unroll
-    for (int w = 1; w < kThreads / 64; ++w) t = t + wave_sum[w];
     a.out[q][b] = t;
     if (a.arrived[q] != nullptr && b % kCondParts == 0) a.arrived[q][b / kCondParts] = 0;
   }
@@ -348,25 +317,6 @@ __global__ void __launch_bounds__(kThreads) k_ns_cond(NsCondArgs a) {
 // every later product reads: DECIDE, by the matrix's first block where nobody asks and by the last to arrive where it does;
 // otherwise by k_ns_classify_order, for batches that a gated launch takes in another order. (A launch of its own, one wavefront per
 // matrix, was almost all start and end: the step of one (1024,3072) weight 216.7 -> 210.0 us without it.)
-struct WideRule {
-  double near_lo, lo, hi;    // in units of the proxy N * ||offdiag(A0)||^2; near_lo == lo: no near range
-  double near_diff;          // > 0: in the near range the gate takes a matrix whose proxy exceeds its column
-                             // concentration by more than this; 0: the kColcFrac rule there as above the band
-};
-// kBulkShare: outlier columns keep the cheap gates while the other columns still hold a few
-// thousandths of the mass (1 % of the columns x100: 1e-2 of it, 8e-4 .. 1.6e-3 with those gates);
-// beyond that the bulk's directions drown in the rounding of the outliers (x300: share 1e-3, 1.4e-3
-// .. 1.9e-3; x1000: 1e-4, 3.6e-3 .. 4.0e-3; x3000: 5.2e-3 .. 5.8e-3) and only every residual
-// term from iteration 1 on recovers them (8e-5 .. 2.9e-4).
-// kColcFrac: a matrix keeps the cheap gates only if its column norms explain its proxy (colc at least
-// 0.85 of it: pure outlier columns and scaled columns read 1.00 .. 1.01). Anything less is a
-// mixture (a low-rank signal WITH outlier columns: 3.5e-3 at a ratio of 0.28 and 6.6e-3 at 0.5 with
-// the cheap gates at 1024x3072, 1e-4 .. 2e-4 with every residual term) or has its mass in directions
-// that are not columns at all (near-duplicate rows: ratio 0.5 .. 0.75).
-constexpr double kColcFrac = 0.85, kBulkShare = 3e-3;
-// sum of a matrix's partial sums, called by whole wavefronts
-__device__ __forceinline__ double cond_sum(const double *parts) { return anc_wave_sum_f64(parts[threadIdx.x & 63]); }
-static_assert(kCondParts == 64, "a partial sum per lane");
 __device__ __forceinline__ int anc_wave_sum_i32(int v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -374,9 +324,6 @@ __device__ __forceinline__ int anc_wave_sum_i32(int v) {
 }
 // First of E matrices in run x of the eight that a launch's sequence is cut into
 __device__ __forceinline__ int anc_run_start(int x, int E) { return (int)(((int64_t)x * E + kXcds - 1) / kXcds); }
-__device__ __host__ __forceinline__ bool wants_colstat(const WideRule &r, double p) {
-  return p >= r.hi || (p > r.near_lo && p <= r.lo);
-}
 struct NsColArgs {
   int n;
   int blocks[kMaxGroups];          // colstat: E * parts, classify: E
@@ -391,37 +338,12 @@ struct NsColArgs {
   int M[kMaxGroups], N[kMaxGroups], parts[kMaxGroups];
   WideRule rule[kMaxGroups];
 };
-constexpr int kColBlock = 64;       // columns per block of k_ns_colstat (measured: 64 -> 92 us, 256 -> 104 us
-                                    // per Qwen3-0.6B step: more blocks beat longer row pieces)
-constexpr int kColLanes = kColBlock / 8, kColRowGroups = kThreads / kColLanes;
-constexpr int kColRowStep = 4;      // every fourth row: the thresholds are coarse (a quarter of the proxy; 1.3
-                                    // against 1.0 and 1.9+), a quarter of the rows places a matrix as well as all
-                                    // of them (flat columns read 1 + 8/M more) and costs a quarter of the bytes
-// The wide gate's decision on matrix e, from its proxy's sum and, where that asks for them, the column norms
-__device__ __forceinline__ bool is_wide(const NsColArgs &a, int q, int e, double sum) {
-  const WideRule r = a.rule[q];
-  const double p = sum * (double)a.N[q];
-  if (p > r.lo && p < r.hi) return true;
-  if (!wants_colstat(r, p)) return false;
-  const double *c = a.part[q] + (int64_t)e * a.parts[q] * 2;
-  double s2 = c[0], s4 = c[1], lightest = c[0];
-#pragma unroll 16
-  for (int i = 1; i < a.parts[q]; ++i) {
-    const double x2 = c[2 * i], x4 = c[2 * i + 1];
-    s2 = s2 + x2;
-    s4 = s4 + x4;
-    lightest = x2 < lightest ? x2 : lightest;
-  }
-  const double colc = s2 > 0.0 ? (double)a.N[q] * s4 / (s2 * s2) : 1.0;
-  // outlier columns: the share of the mass outside them, from the lightest block of columns
-  const double bulk = s2 > 0.0 ? (double)a.parts[q] * lightest / s2 : 1.0;
-  if (p < r.hi && r.near_diff > 0.0) return p - colc > r.near_diff;
-  return colc < kColcFrac * p || (p >= r.hi && bulk < kBulkShare);
+__device__ __forceinline__ bool wide_at(const NsColArgs &a, int q, int e, double sum) {
+  return is_wide(a.rule[q], a.N[q], a.parts[q], a.part[q] + (int64_t)e * a.parts[q] * 2, sum);
 }
 template <bool DECIDE>
 __global__ void __launch_bounds__(kThreads) k_ns_colstat(NsColArgs a) {
-  __shared__ double colsum[kColRowGroups][kColBlock];
-  __shared__ double wave_sum[2][kColBlock / 64];
+  __shared__ ColLds lds;
   int b = (int)blockIdx.x, q = 0;
   while (q + 1 < a.n && b >= a.blocks[q]) { b -= a.blocks[q]; ++q; }
   const int e = b / a.parts[q], part = b % a.parts[q];
@@ -430,55 +352,24 @@ __global__ void __launch_bounds__(kThreads) k_ns_colstat(NsColArgs a) {
   if (!wants_colstat(a.rule[q], sum * (double)N)) {
     if (DECIDE && part == 0 && threadIdx.x == 0) {
       a.sum[q][e] = sum;
-      a.flag[q][e] = is_wide(a, q, e, sum) ? 1 : 0;
+      a.flag[q][e] = wide_at(a, q, e, sum) ? 1 : 0;
     }
     return;
   }
-  // lane (rg, cg): columns part*64 + 8*cg .. +7 (one 16-byte load per row), rows 4 rg, 4 (rg + 32), ...
-  const int cg = (int)threadIdx.x % kColLanes, rg = (int)threadIdx.x / kColLanes;
-  const int j = part * kColBlock + 8 * cg;
-  double c[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  if (j < N) {
-    const uint16_t *src = a.Xh[q] + (int64_t)e * M * N + j;
-#pragma unroll 8
-    for (int i = kColRowStep * rg; i < M; i += kColRowStep * kColRowGroups) {
-      const anc_u32x4 w = *(const anc_u32x4 *)(src + (int64_t)i * N);
-      const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const double x0 = (double)__uint_as_float(u[k] << 16), x1 = (double)__uint_as_float(u[k] & 0xFFFF0000u);
-        c[2 * k] = c[2 * k] + x0 * x0;
-        c[2 * k + 1] = c[2 * k + 1] + x1 * x1;
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 8; ++k) colsum[rg][8 * cg + k] = c[k];
-  __syncthreads();
-  if (threadIdx.x < kColBlock) {               // one lane per column: the row groups in order
-    double c2 = colsum[0][threadIdx.x];
-#pragma unroll
-    for (int r = 1; r < kColRowGroups; ++r) c2 = c2 + colsum[r][threadIdx.x];
-    const double s2 = anc_wave_sum_f64(c2), s4 = anc_wave_sum_f64(c2 * c2);
-    if ((threadIdx.x & 63) == 0) { wave_sum[0][threadIdx.x >> 6] = s2; wave_sum[1][threadIdx.x >> 6] = s4; }
-  }
-  __syncthreads();
+  double t2, t4;
+  col_part(a.Xh[q] + (int64_t)e * M * N, M, N, part, lds, t2, t4);
   if (threadIdx.x == 0) {
-    double t2 = wave_sum[0][0], t4 = wave_sum[1][0];
-#pragma unroll
-    for (int w = 1; w < kColBlock / 64; ++w) { t2 = t2 + wave_sum[0][w]; t4 = t4 + wave_sum[1][w]; }
     double *out = a.part[q] + ((int64_t)e * a.parts[q] + part) * 2;
     out[0] = t2;
     out[1] = t4;
     if constexpr (DECIDE) {
       if (__hip_atomic_fetch_add(a.arrived[q] + e, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == a.parts[q] - 1) {
         a.sum[q][e] = sum;
-        a.flag[q][e] = is_wide(a, q, e, sum) ? 1 : 0;
+        a.flag[q][e] = wide_at(a, q, e, sum) ? 1 : 0;
       }
     }
   }
 }
-static_assert(kColBlock % 64 == 0 && kColBlock <= kThreads, "k_ns_colstat: whole wavefronts of one lane per column in the final sum");
 // One block per batch: the wide gate's flag per matrix, and the order in which the launches of a gated
 // iteration take the matrices. A matrix that takes a gate's terms has three times the products of one that does not;
 // such matrices lie together (the tall weights of a stack) and a launch's sequence is cut into eight runs, one per XCD,
@@ -508,7 +399,7 @@ __global__ void __launch_bounds__(kClassifyThreads) k_ns_classify_order(NsColArg
   __syncthreads();
   for (int e = (int)threadIdx.x; e < E; e += kClassifyThreads) {      // (a matrix per lane)
     const double sum = a.sum[q][e];
-    const bool wide = a.flag[q] != nullptr && is_wide(a, q, e, sum);
+    const bool wide = a.flag[q] != nullptr && wide_at(a, q, e, sum);
     if (a.flag[q] != nullptr) a.flag[q][e] = wide ? 1 : 0;
     if (e < kMaxOrdered) heavy[e] = wide || sum > a.gate[q] ? 1 : 0;
   }
@@ -854,6 +745,7 @@ void add_prologue(NsPrologue &a, const Plan &pl, uint64_t Uh, uint64_t Ul, uint6
   a.Uh[q] = (uint16_t *)Uh;
   a.Ul[q] = (uint16_t *)Ul;
   a.zero16[q] = pl.zero16;
+  a.arrived[q] = pl.order;
   a.mn[q] = mn;
 }
 int launch_prologue(const NsPrologue &a, float eps, hipStream_t s) {
@@ -1040,6 +932,10 @@ bool f16_range(const float *coef, int steps) {
   return true;
 }
 
+WideRule wide_rule(const SplitPlan &sp) {
+  return WideRule{(double)sp.wide_near, (double)sp.wide_lo, (double)sp.wide_hi, (double)sp.wide_near_diff};
+}
+
 // steps x { A = X X^T; B = b A + c A A; X = a X + B X } on n problems side by side: every
 // product of a step is ONE launch over all problems (problems in the order given; put the
 // longest K first). First step's output goes to pair `nxt` of each plan, later steps ping-pong;
@@ -1184,7 +1080,18 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       AncProfScope prof(ANC_PROF_NS_GRAM, s);
       if (int rc = anc_ns_gemm_multi(EPI_GRAM, ga, Es, n, force, k > 0 ? f16 : FMT_BF16, s)) return rc;
     }
-    if (k == 0 && want_cond) {
+    // One matrix whose B = b A + c A A runs on 64-wide tiles that leave CUs over: the statistics are workgroups of that launch, unless X = a X + B X
+    // of this iteration asks for them (8-bit low halves out). The step of one (1024,3072) weight 215.0 -> 212.0 us,
+    // the default step of a 1024x1024 model 358.6 -> 352.3: a launch's start and end twice less, B's own launch longer by part of that.
+    NsStatOne beside{};
+    const bool with_b = k == 0 && want_cond && n == 1 && Es[0] == 1 && cp[0].scale0 != nullptr && !(gx[0].l8_out > 0.0) &&
+                        !ordered(0) && (cp[0].M / 64) * (cp[0].M / 64 + 1) / 2 <= kStatTiles &&
+                        (force != 0 ? force : pick_tile(EPI_BMAT, gb, Es, n)) == 64;
+    if (with_b) {
+      const Plan &pl = cp[0].pl;
+      beside = NsStatOne{pl.Fh, cp[0].inH, pl.condpart, pl.cond, pl.colpart, pl.wide_flag, pl.order, (int)cp[0].M, (int)cp[0].N, pl.col_parts,
+                         wide_rule(pl.sp)};
+    } else if (k == 0 && want_cond) {
       // the proxy of every problem that gates a later product, from the Fh this launch wrote
       NsCondArgs ca{};
       int blocks = 0;
@@ -1216,8 +1123,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
         cs.order[i] = ordered(q) ? pl.order : nullptr;
         cs.arrived[i] = any_ordered ? nullptr : pl.order;
         cs.M[i] = (int)cp[q].M; cs.N[i] = (int)cp[q].N; cs.parts[i] = pl.col_parts;
-        cs.rule[i] = WideRule{(double)pl.sp.wide_near, (double)pl.sp.wide_lo, (double)pl.sp.wide_hi,
-                              (double)pl.sp.wide_near_diff};
+        cs.rule[i] = wide_rule(pl.sp);
         cs.blocks[i] = (int)(cp[q].E * pl.col_parts);
         cs_blocks += cs.blocks[i];
         ++cs.n;
@@ -1235,7 +1141,9 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
     }
     {
       AncProfScope prof(ANC_PROF_NS_BMAT, s);
-      if (int rc = anc_ns_gemm_multi(EPI_BMAT, gb, Es, n, force, k > 0 ? f16 : FMT_BF16, s)) return rc;
+      if (with_b) {
+        if (int rc = anc_ns_gemm_tile_multi(EPI_BMAT, gb, Es, 1, s, 64, false, FMT_BF16, nullptr, false, &beside)) return rc;
+      } else if (int rc = anc_ns_gemm_multi(EPI_BMAT, gb, Es, n, force, k > 0 ? f16 : FMT_BF16, s)) return rc;
     }
     {
       AncProfScope prof(last && upd != nullptr ? ANC_PROF_NS_BX_UPD : ANC_PROF_NS_BX, s);

@@ -81,7 +81,7 @@ constexpr int kCondParts = 64;           // partial sums per matrix of the condi
 constexpr int kXcds = 8;
 
 enum { EPI_GRAM = 0, EPI_BMAT = 1, EPI_BX = 2 };
-enum { VAR_NONE = 0, VAR_UPDATE = 1, VAR_PLAIN = 2, VAR_UPDATE_T = 3, VAR_STREAM = 4 };   // variants of the epilogue (1 .. 3: of EPI_BX)
+enum { VAR_NONE = 0, VAR_UPDATE = 1, VAR_PLAIN = 2, VAR_UPDATE_T = 3, VAR_STREAM = 4, VAR_STATS = 5 };   // variants of the epilogue (1 .. 3: of EPI_BX)
 enum { kStream128 = 1, kStream256 = 2 };                                                  // NsGemm::stream_out
 
 // Workgroup id -> logical tile id such that logical ids [start(x), start(x+1)) run on XCD x
@@ -300,7 +300,7 @@ int anc_ns_gemm_big_f16(int epi, const NsGemm *ps, const int64_t *Es, int n, hip
 void anc_ns_gemm_tile_f16(int epi, int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm, bool update);
 void anc_ns_gemm_tile_to_f16(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm);
 int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int tile, bool by_rows, int fmt,
-                           const NsUpdate *upd, bool plain);
+                           const NsUpdate *upd, bool plain, const struct NsStatOne *stat = nullptr);
 // Bare fp32 products C[e] = A[e] B[e] on the same K loops; a_transposed: A is
 // given as (K, M) row-major with row pitch ldA (and strideA between matrices), C = A^T B. The tiles are chosen
 // by a rule of their own (pick_tile_plain); the bits are the same on all.

@@ -36,6 +36,7 @@
 
 #include "lds_dma.h"
 #include "ns_common.h"
+#include "ns_stats.h"
 
 namespace {
 
@@ -80,8 +81,12 @@ __host__ __device__ constexpr int anc_sym_tiles(int rows) { return rows * (rows 
 
 // SOLO: the launch has one problem, its arguments lie at fixed places.
 // FMT: the 16-bit floats of operands and outputs (FMT_BF16 ..).
+// VAR_STATS (B = b A + c A A of one matrix): the workgroups behind the tiles make the gates' statistics.
+// (by specialisation: an expression in the kernel's signature enters its name, and an unnamed enum has other names there on the host)
+template <int VAR, bool SOLO> struct TileArgs { using type = NsGemmArgs<SOLO ? 1 : kMaxGroups>; };
+template <> struct TileArgs<VAR_STATS, true> { using type = NsStatArgs; };
 template <int EPI, int WM, int WN, int NW, bool AT, int VAR, int kRing, bool SOLO, int FMT = FMT_BF16>
-__global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) * NW / 4) k_ns_gemm_tile(NsGemmArgs<SOLO ? 1 : kMaxGroups> pm) {
+__global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) * NW / 4) k_ns_gemm_tile(typename TileArgs<VAR, SOLO>::type pm) {
   constexpr int WC = NW / 2, TM = 64 * WM, TN = 32 * WN * WC, KP = WM == 1 ? 2 : 1, TK = 32 * KP;
   constexpr bool BT = EPI == EPI_BX, PLAINV = VAR == VAR_PLAIN, F16 = FMT == FMT_F16, F16OUT = FMT != FMT_BF16;
   constexpr int kHalf = TM * TK * 2, kStageBytes = kHalf + TN * TK * 2;      // A's part of a stage, a stage
@@ -90,7 +95,14 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kRing * kStageBytes];
 
   int gsel = 0, L;
-  if constexpr (SOLO) L = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  if constexpr (VAR == VAR_STATS) {
+    static_assert(SOLO && NW == 4 && sizeof(lds) >= sizeof(ColLds), "a statistic's workgroup");
+    if ((int)blockIdx.x >= pm.tiles_only) {
+      stat_block(pm.stat, (int)blockIdx.x - pm.tiles_only, lds);
+      return;
+    }
+    L = xcd_remap((int)blockIdx.x, pm.tiles_only);
+  } else if constexpr (SOLO) L = xcd_remap((int)blockIdx.x, (int)gridDim.x);
   else if (PLAINV && pm.seq) anc_seq_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
   else anc_group_tile(pm, (int)blockIdx.x, gsel, L);
   const NsGemm &p = pm.g[gsel];
@@ -903,7 +915,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
 constexpr int kLongPlain = 2048;
 
 template <int EPI, bool AT, int VAR, int FMT>
-void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) {
+void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm, const NsStatOne *stat = nullptr) {
   if constexpr (VAR == VAR_PLAIN) {
     if (tile == kTile128x64) {
       hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, 4, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
@@ -926,7 +938,7 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) 
   else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 3, false, FMT>), dim3(grid), dim3(256), 0, s, pm);
   else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 4, false, FMT>), dim3(grid), dim3(256), 0, s, pm);
   else {
-    NsGemmArgs<1> one;
+    NsStatArgs one;
     one.n = 1;
     one.seq = pm.seq;
     one.g[0] = pm.g[0];
@@ -934,7 +946,15 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm) 
     one.sr = pm.sr;
     one.seed_base = pm.seed_base;
     one.ctl = pm.ctl;
-    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 4, true, FMT>), dim3(grid), dim3(256), 0, s, one);
+    if constexpr (EPI == EPI_BMAT && VAR == VAR_NONE && FMT == FMT_BF16) {
+      if (stat != nullptr) {
+        one.tiles_only = (int)grid;
+        one.stat = *stat;
+        hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR_STATS, 4, true, FMT>), dim3(grid + kCondParts + stat->parts), dim3(256), 0, s, one);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 4, true, FMT>), dim3(grid), dim3(256), 0, s, (const NsGemmArgs<1> &)one);
   }
 }
 
@@ -967,7 +987,7 @@ void anc_ns_gemm_tile_to_f16(int tile, unsigned gr, hipStream_t s, const NsGemmM
 // n <= kMaxGroups problems of the same product in one launch on tiles of 64, 128 or 128x64 (kTile128x64). EPI_BX:
 // `by_rows` as for the 256-wide tiles; `plain`: the bare product, A transposed (by_rows) or not.
 int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int tile, bool by_rows, int fmt,
-                           const NsUpdate *upd, bool plain) {
+                           const NsUpdate *upd, bool plain, const NsStatOne *stat) {
   const int TM = tile == 64 ? 64 : 128, TN = tile == 128 ? 128 : 64;
   ANC_REQUIRE(plain || TM == TN, "anc_ns_gemm_tile: tiles of 128x64 are the plain product's");
   NsGemmMulti pm{};
@@ -1016,8 +1036,11 @@ int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, 
     pm.seed_base = upd->seed_base;
     pm.ctl = upd->ctl;
   }
+  ANC_REQUIRE(stat == nullptr || (n == 1 && epi == EPI_BMAT && tile == 64 && grid <= kStatTiles && fmt == FMT_BF16),
+              "anc_ns_gemm_tile: statistics go with one matrix's B on tiles of 64");
   ANC_REQUIRE(fmt == FMT_BF16 || epi != EPI_BX || by_rows, "anc_ns_gemm_tile: fp16 reads B by rows k");
-  if (fmt == FMT_F16)         anc_ns_gemm_tile_f16(epi, tile, gr, s, pm, upd != nullptr);
+  if (stat != nullptr)        launch_tile<EPI_BMAT, false, VAR_NONE, FMT_BF16>(tile, gr, s, pm, stat);
+  else if (fmt == FMT_F16)    anc_ns_gemm_tile_f16(epi, tile, gr, s, pm, upd != nullptr);
   else if (fmt == FMT_TO_F16) anc_ns_gemm_tile_to_f16(tile, gr, s, pm);
   else if (!plain)            launch_tiles<FMT_BF16>(epi, tile, gr, s, pm, by_rows, upd != nullptr);
   else if (by_rows)           launch_tile<EPI_BX, true, VAR_PLAIN, FMT_BF16>(tile, gr, s, pm);

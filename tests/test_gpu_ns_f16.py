@@ -96,3 +96,34 @@ def test_the_last_block_decides_on_the_column_statistic(gpu, E, M, N):
         assert _hard_count(1, M, N, "bf16_late3")[0] == int(kinds[e] in ("lowrank", "band")), e
     run_ns(X[:1], schedule=PE_SCHEDULE)                    # one matrix under the proxy's gates has no order either
     assert _hard_count(1, M, N)[0] == 1
+
+
+@pytest.mark.parametrize("M,N", [(1024, 1024), (1024, 3072), (1152, 2432), (1408, 1408), (1536, 1536)])
+@pytest.mark.parametrize("sched", ["keller", "pe"])
+def test_statistics_beside_the_second_product(gpu, M, N, sched):
+    """One matrix whose B has up to 256 tiles of 64 has its statistics made in that launch (1408: 253; 1536 has them made by kernels of
+    their own, like two matrices and tiles of 128): flags and bits of the same matrix among two, for each answer of the statistics, call after call."""
+    from ancora_cutile_amd import DevBuf, newton_schulz_resident_e
+    from ancora_cutile_amd.muon_ns import NsWorkspace, PE_SCHEDULE, ns_hard_info
+    from oracle.bf16_ref import bf16_rne_bits
+    schedule, counted = (PE_SCHEDULE, "bf16") if sched == "pe" else (None, "bf16_late3")
+    ws = NsWorkspace()
+
+    def run(X, mode="bf16"):
+        g = DevBuf(bf16_rne_bits(X).reshape(-1, N))
+        newton_schulz_resident_e(g, None, None, None, None, None, X.shape[0], M, N, 0, schedule=schedule, mode=mode, workspace=ws)
+        out, flags = g.to_numpy().reshape(X.shape), ns_hard_info(ws.buf.ptr, X.shape[0], M, N, 5, counted)
+        g.free()
+        return out, flags
+    band = _input(M, N, "plain", 5)
+    band[:, :: 10] *= 10
+    low = (_input(M, 8, "plain", 7) @ _input(8, N, "plain", 8) + 0.01 * _input(M, N, "plain", 9)).astype(np.float32)
+    for X in (_input(M, N, "plain", 1), _input(M, N, "cols", 2), band, low, _input(M, N, "rows", 3), np.zeros((M, N), np.float32)):
+        pair, (n2, extra2) = run(np.stack([X, X]))
+        one, (n1, extra1) = run(X[None])
+        assert bits_equal(one[0], pair[0]) and bits_equal(pair[0], pair[1])
+        assert 2 * n1 == n2 and abs(2 * extra1 - extra2) <= 1e-9 * extra2
+    assert run(band[None])[1][0] == 1 and run(low[None])[1][0] == 1 and run(_input(M, N, "plain", 1)[None])[1][0] == 0
+    t128 = run(low[None], "bf16_t128" if sched == "pe" else "bf16_late3_t128")[0]
+    assert bits_equal(t128, run(low[None])[0])
+    ws.free()
