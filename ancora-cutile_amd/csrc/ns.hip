@@ -37,7 +37,6 @@
 // launch by the number of tiles (pick_tile); the bits are the same on all of them.
 #include <algorithm>
 #include <cfloat>
-#include <cmath>
 #include <vector>
 
 #include "ns_stats.h"
@@ -493,8 +492,6 @@ struct SplitPlan {
   // realisation of its own rounding error (an exact low half moves it as far). Measured: X = a X +
   // B X 4.85 -> 4.69 ms per step of Qwen3-0.6B, 2.0 GB less HBM traffic.
   bool low8;
-  // fp16 operands and iterates from iteration 1 on (f16_range). M >= 1024 only, which anc_ns_gemm_multi relies on
-  bool f16;
   bool gated(int k) const { return k >= 0 && k < kGateIters && k < x_from && gate_tau[k] > 0.0f; }
   bool wide() const { return wide_hi > 0.0f; }
   bool wide_gram(int k) const { return wide() && k >= wide_gram_from && k < x_from; }
@@ -556,10 +553,9 @@ struct SplitPlan {
 //     again: a GPU fault in the test run that carried it, cause not found.)
 constexpr float kTauWideNear2M = 1.15f, kNearDiff2M = 0.15f;
 constexpr float kTauHard = 2.5f, kTauPlain = 1.3f, kTauWideLo = 2.5f, kTauWideHi = 40.0f, kTauWideNear = 1.5f;
-SplitPlan split_plan(int64_t M, int64_t N, int mode, int steps, bool in_range = true) {
+SplitPlan split_plan(int64_t M, int64_t N, int mode, int steps) {
   SplitPlan sp{};
   sp.x_from = sp.fb_from = steps;
-  sp.f16 = mode == ANC_NS_BF16_LATE3 && M >= 1024 && steps == 5 && in_range;
   if (mode == ANC_NS_BF16_X3) {
     // every product with the residuals of both operands' bf16 roundings, in every iteration:
     // about 1e-5 on every input tried, three times the matrix-core work
@@ -583,21 +579,6 @@ SplitPlan split_plan(int64_t M, int64_t N, int mode, int steps, bool in_range = 
     // for 2.05 instead of 2.2 times the plain chain's work. (F and Boff first and X later, or the
     // last two iterations only: 2.0e-3 .. 2.3e-3.)
     if (steps >= 5) sp.fb_from = sp.x_from + 1;
-    // Operands in fp16 leave an eighth of bf16's rounding, so fewer residuals reach the same distance from the chain in 64
-    // bits, and what they save is most of the difference to a chain without any: X's in the last iteration (M = 1024), in the last two (up
-    // to M = 1280 and N = 3M), all in the last two. What counts is how late the singular values arrive: at entries of 1 / sqrt(M N) the
-    // later the larger M. Bf16 with the residuals above, then fp16 with X's from 4 / X's from 3 / all from 3, in 1e-4, independent entries:
-    //   1024x1024 8.1, 5.6 / 4.6 / 2.7     1024x4096 3.2, 2.4            1152x3456 2.9, 2.8 / 2.0 / 0.8
-    //   1280x1280 5.3, 5.2 / 4.0 / 1.9     1280x3840 2.1, 2.9 / 2.0 / 0.6     1408x4224 1.7, 3.0 / 2.0 / 0.5
-    //   2048x2048 1.7, 4.6 / 3.2 / 0.6     3072x4096 0.9, 3.9 / 2.4 / 0.3
-    // and with 1 % of the rows x100 1024x1024 1.2, 0.7, transposed 7.9, 1.6, 1024x3072 0.7, 0.4, transposed 7.6, 1.9. The
-    // step of one (1024,3072) weight 258 -> 212 us, of the Qwen3-0.6B set 18.2 -> 14.0 ms, chains of 24 x (1024,2048) 1935 -> 1430 us, 16 x
-    // (1408,2816) 3532 -> 3305. (M < 1024 needs all residuals from iteration 1 on in either format, fp16 without has 2 .. 6 times the
-    // error, and with them fp16 is no faster: 3 x (768,1536) 243 -> 249 us.)
-    if (sp.f16) {
-      sp.x_from = M < 1152 ? 4 : 3;
-      sp.fb_from = M < 1152 || (M <= 1280 && N <= 3 * M) ? 5 : 3;
-    }
     // and the matrices the wide gate flags (below) start one iteration earlier, as they do under
     // Polar Express: a rank-32 signal over 1 % noise is 2.1e-3 at 1024x1024 with the terms from
     // iteration 2 and 3e-4 from iteration 1
@@ -906,32 +887,6 @@ int forced_tile(int flags) {
          : (flags & ANC_NS_FORCE_T256) ? 256 : 0;
 }
 
-// Do the chain's values stay in fp16's range? From X's singular values in 0 .. 1: s' = |a s + b s^3 + c s^5| is largest at the ends or
-// where its derivative, a quadratic in s^2, is zero; entries of X, A and B are at most their largest singular values. (Keller's
-// and the Polar-Express coefficients: 311 of 65504 at most.)
-bool f16_range(const float *coef, int steps) {
-  double top = 1.0;
-  for (int k = 0; k < steps; ++k) {
-    const double a = coef[3 * k], b = coef[3 * k + 1], c = coef[3 * k + 2], t2 = top * top;
-    const double most = std::max(std::max(t2, top * kF16Iterate), std::fabs(b) * t2 + std::fabs(c) * t2 * t2);
-    if (!(most <= 32752.0)) return false;
-    auto p = [&](double s) { return std::fabs(s * (a + s * s * (b + s * s * c))); };
-    double m = p(top);
-    const double d = 9.0 * b * b - 20.0 * a * c;
-    if (c != 0.0 && d >= 0.0) {
-      for (int i = -1; i <= 1; i += 2) {
-        const double s2 = (-3.0 * b + i * std::sqrt(d)) / (10.0 * c);
-        if (s2 > 0.0 && s2 < t2) m = std::max(m, p(std::sqrt(s2)));
-      }
-    } else if (c == 0.0 && b != 0.0 && -a / (3.0 * b) > 0.0 && -a / (3.0 * b) < t2) {
-      m = std::max(m, p(std::sqrt(-a / (3.0 * b))));
-    }
-    if (!(m < 1e6)) return false;
-    top = 1.01 * m;                // (rounding; Keller's polynomial keeps 0 .. 1.25 in itself, and little more)
-  }
-  return true;
-}
-
 WideRule wide_rule(const SplitPlan &sp) {
   return WideRule{(double)sp.wide_near, (double)sp.wide_lo, (double)sp.wide_hi, (double)sp.wide_near_diff};
 }
@@ -943,13 +898,6 @@ WideRule wide_rule(const SplitPlan &sp) {
 int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags, hipStream_t s,
                    const NsUpdate *upd = nullptr) {
   const int force = forced_tile(flags);
-  int f16 = FMT_BF16;          // the format of iterations after the first, where M >= 1024 (the plans of a call are of one mode and length)
-  for (int q = 0; q < n; ++q)
-    if (cp[q].pl.sp.f16) f16 = FMT_F16;
-  if (f16 && !f16_range(coef, steps)) {
-    f16 = FMT_BF16;
-    for (int q = 0; q < n; ++q) cp[q].pl.sp = split_plan(cp[q].M, cp[q].N, ANC_NS_BF16_LATE3, steps, false);
-  }
   const uint16_t *curH[kMaxGroups], *curL[kMaxGroups];
   int nxt[kMaxGroups];
   int64_t Es[kMaxGroups];
@@ -1078,7 +1026,7 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
     }
     {
       AncProfScope prof(ANC_PROF_NS_GRAM, s);
-      if (int rc = anc_ns_gemm_multi(EPI_GRAM, ga, Es, n, force, k > 0 ? f16 : FMT_BF16, s)) return rc;
+      if (int rc = anc_ns_gemm_multi(EPI_GRAM, ga, Es, n, force, s)) return rc;
     }
     // One matrix whose B = b A + c A A runs on 64-wide tiles that leave CUs over: the statistics are workgroups of that launch, unless X = a X + B X
     // of this iteration asks for them (8-bit low halves out). The step of one (1024,3072) weight 215.0 -> 212.0 us,
@@ -1142,12 +1090,12 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
     {
       AncProfScope prof(ANC_PROF_NS_BMAT, s);
       if (with_b) {
-        if (int rc = anc_ns_gemm_tile_multi(EPI_BMAT, gb, Es, 1, s, 64, false, FMT_BF16, nullptr, false, &beside)) return rc;
-      } else if (int rc = anc_ns_gemm_multi(EPI_BMAT, gb, Es, n, force, k > 0 ? f16 : FMT_BF16, s)) return rc;
+        if (int rc = anc_ns_gemm_tile_multi(EPI_BMAT, gb, Es, 1, s, 64, false, nullptr, false, &beside)) return rc;
+      } else if (int rc = anc_ns_gemm_multi(EPI_BMAT, gb, Es, n, force, s)) return rc;
     }
     {
       AncProfScope prof(last && upd != nullptr ? ANC_PROF_NS_BX_UPD : ANC_PROF_NS_BX, s);
-      if (int rc = anc_ns_gemm_multi(EPI_BX, gx, Es, n, force, k > 0 ? f16 : f16 ? FMT_TO_F16 : FMT_BF16, s, last ? upd : nullptr)) return rc;
+      if (int rc = anc_ns_gemm_multi(EPI_BX, gx, Es, n, force, s, last ? upd : nullptr)) return rc;
     }
     for (int q = 0; q < n; ++q) {
       curH[q] = cp[q].pl.Xh[nxt[q]]; curL[q] = cp[q].pl.Xl[nxt[q]];
@@ -1163,7 +1111,7 @@ static int pair_multi_impl(const char *who, const anc_ns_problem_t *probs, int32
                            const uint64_t *desc_tables, const NsUpdate *upd, int steps, const float *coef,
                            float eps, int mode, uint64_t stream);
 
-int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int force, int fmt, hipStream_t s,
+int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int force, hipStream_t s,
                       const NsUpdate *upd) {
   ANC_REQUIRE(n >= 1 && n <= kMaxGroups, "Newton-Schulz chain: 1..%d problems per launch", kMaxGroups);
   bool any_upd = false, all_upd = true;
@@ -1178,19 +1126,16 @@ int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int f
   // element (i, j) and element (j, i) add the same products in a different order and may differ
   // in the last bit. So the way of reading is a property of the problem's shape, never of what
   // it shares a call with: a call with problems of both kinds becomes two launches.
-  // Fp16 products, which M >= 1024 alone has, are apart in the same way.
   // Where 256-wide tiles are the choice, problems whose dims do not allow them get a launch of their own.
   NsGemm part[kMaxGroups];
   int64_t pe[kMaxGroups];
   bool done[2] = {false, false};
   for (int pass = 0; pass < 4; ++pass) {
-    const bool apart = epi == EPI_BX || fmt != FMT_BF16, large = (pass & 1) == 0, wide = pass < 2;
-    const bool by_rows = epi == EPI_BX && large;
-    const int f = large ? fmt : (int)FMT_BF16;
+    const bool by_rows = epi == EPI_BX && (pass & 1) == 0, wide = pass < 2;
     auto collect = [&](bool all) {
       int m = 0;
       for (int k = 0; k < n; ++k) {
-        if (apart ? (ps[k].M >= 1024) != large : !large) continue;
+        if (epi == EPI_BX ? (ps[k].M >= 1024) != by_rows : (pass & 1) != 0) continue;
         if (!all && (ps[k].fits256 != 0) != wide) continue;
         part[m] = ps[k];
         pe[m++] = Es[k];
@@ -1203,13 +1148,13 @@ int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int f
     const int m_wide = collect(false);
     if (wide) {
       if (m_wide > 0 && pick(m_wide) == 256) {
-        if (int rc = anc_ns_gemm_big_multi(epi, part, pe, m_wide, s, by_rows, f, u)) return rc;
+        if (int rc = anc_ns_gemm_big_multi(epi, part, pe, m_wide, s, by_rows, u)) return rc;
       } else if (const int m = collect(true)) {
-        if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m, s, narrow(pick(m)), by_rows, f, u, false)) return rc;
+        if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m, s, narrow(pick(m)), by_rows, u, false)) return rc;
         done[pass & 1] = true;
       }
     } else if (m_wide > 0 && !done[pass & 1]) {
-      if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m_wide, s, narrow(pick(m_wide)), by_rows, f, u, false)) return rc;
+      if (int rc = anc_ns_gemm_tile_multi(epi, part, pe, m_wide, s, narrow(pick(m_wide)), by_rows, u, false)) return rc;
     }
   }
   return ANC_OK;
@@ -1219,7 +1164,7 @@ int anc_ns_gemm_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s,
   ANC_REQUIRE(n >= 1 && n <= kMaxGroups, "anc_ns_gemm_plain: 1..%d problems per launch", kMaxGroups);
   const int tile = pick_tile_plain(ps, Es, n);
   if (tile == 256) return anc_ns_gemm_big_plain(ps, Es, n, s, a_transposed);
-  return anc_ns_gemm_tile_multi(EPI_BX, ps, Es, n, s, tile, a_transposed, FMT_BF16, nullptr, true);
+  return anc_ns_gemm_tile_multi(EPI_BX, ps, Es, n, s, tile, a_transposed, nullptr, true);
 }
 
 extern "C" int64_t anc_ns_workspace_bytes(int64_t E, int64_t M, int64_t N, int mode) {

@@ -34,49 +34,6 @@ __device__ __forceinline__ void anc_pk_pair(float a, float b, uint32_t &hi, uint
   lo = anc_pk_bf16(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xFFFF0000u));
 }
 
-
-// 16-bit floats of the chain. A launch's operands and what it writes for the chain are bf16, or fp16: 11 significant bits instead
-// of 8, in a range that the caller has checked (ns.hip, f16_range). F and B, whose norms are near 1, are kept as they are (what is below
-// 6e-5 has an absolute error, 3e-8), the iterate 256 times as large, which is exact: its entries begin at 1 / sqrt(M N), those beside
-// outliers at a hundredth of that. So X X^T carries a factor of 65536, which its epilogue takes out with the scale it has anyway, and B X the
-// iterate's own.
-enum { FMT_BF16 = 0, FMT_TO_F16 = 1, FMT_F16 = 2 };     // (TO_F16: X = a X + B X on bf16 that writes an fp16 iterate)
-constexpr float kF16Iterate = 256.0f, kF16Inv = 1.0f / kF16Iterate;
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 anc_f16x2 __attribute__((ext_vector_type(2)));
-template <bool F16> __device__ __forceinline__ f32x16 anc_mfma(bf16x8 a, bf16x8 b, f32x16 c) {
-  if constexpr (F16) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else               return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-// The two values of a dword, as they are stored
-template <bool F16> __device__ __forceinline__ float anc_half_lo(uint32_t w) {
-  if constexpr (F16) return (float)__builtin_bit_cast(anc_f16x2, w).x;
-  else               return __uint_as_float(w << 16);
-}
-template <bool F16> __device__ __forceinline__ float anc_half_hi(uint32_t w) {
-  if constexpr (F16) return (float)__builtin_bit_cast(anc_f16x2, w).y;
-  else               return __uint_as_float(w & 0xFFFF0000u);
-}
-template <bool F16> __device__ __forceinline__ uint32_t anc_pk(float a, float b) {
-  if constexpr (F16) {
-    const anc_f32x2v v = {a, b};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, anc_f16x2));
-  } else {
-    return anc_pk_bf16(a, b);
-  }
-}
-template <bool F16> __device__ __forceinline__ void anc_pk_pair_as(float a, float b, uint32_t &hi, uint32_t &lo) {
-  if constexpr (F16) {
-    const anc_f32x2v v = {a, b};
-    const anc_f16x2 h = __builtin_convertvector(v, anc_f16x2);
-    const anc_f32x2v d = {a - (float)h.x, b - (float)h.y};
-    hi = __builtin_bit_cast(uint32_t, h);
-    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(d, anc_f16x2));
-  } else {
-    anc_pk_pair(a, b, hi, lo);
-  }
-}
-
 constexpr int kCondParts = 64;           // partial sums per matrix of the conditioning proxy
 constexpr int kXcds = 8;
 
@@ -283,23 +240,17 @@ __device__ __forceinline__ void anc_seq_tile(const NsGemmMulti &pm, int bid, int
 
 // One product of the chain for n <= kMaxGroups problems (ps[k] with batch size Es[k]) on the tiles that suit
 // the launch (ns.hip: the rule), or on tiles of `force` (64, 128, 256; 0: the rule). Every choice gives the
-// same bits. `fmt`: the 16-bit floats of problems with M >= 1024 (FMT_BF16 ..); others are bf16. `upd` carries the scalars of the fused weight update for problems whose
-// `upd` is set.
-int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int force, int fmt, hipStream_t s,
+// same bits. `upd` carries the scalars of the fused weight update for problems whose `upd` is set.
+int anc_ns_gemm_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, int force, hipStream_t s,
                       const NsUpdate *upd = nullptr);
 // The kernels behind it. 256x256 tiles for the symmetric products, 128x256 for X = a X + B X
 // (ns_gemm_big.hip; M and N multiples of 256); `by_rows`: X = a X + B X reads its B by rows k.
-int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool by_rows, int fmt,
+int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool by_rows,
                           const NsUpdate *upd);
 // Tiles of 64x64 (`tile` 64), 128x64 (kTile128x64) or 128x128 (128) outputs (ns_gemm_tile.hip; M and N multiples of 128);
 // `plain`: the bare product.
 constexpr int kTile128x64 = 12864;
-// The launches on fp16 operands or with an fp16 iterate out, which live in units of their own (ns_gemm_big_f16.hip, ns_gemm_tile_f16.hip)
-// (X = a X + B X reads its B by rows k there)
-int anc_ns_gemm_big_f16(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int fmt, const NsUpdate *upd);
-void anc_ns_gemm_tile_f16(int epi, int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm, bool update);
-void anc_ns_gemm_tile_to_f16(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm);
-int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int tile, bool by_rows, int fmt,
+int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int tile, bool by_rows,
                            const NsUpdate *upd, bool plain, const struct NsStatOne *stat = nullptr);
 // Bare fp32 products C[e] = A[e] B[e] on the same K loops; a_transposed: A is
 // given as (K, M) row-major with row pitch ldA (and strideA between matrices), C = A^T B. The tiles are chosen

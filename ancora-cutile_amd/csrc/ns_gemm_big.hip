@@ -68,19 +68,20 @@ constexpr int kFull = 0, kLower = 1, kNone = 2;
 // (operands exchanged, same products, same order of summation): row = lane%32 and element
 // r = col 8*(r/4) + 4*(lane/32) + r%4, i.e. a lane holds runs of 4 consecutive columns of one
 // output row, which is what a row-major epilogue wants.
-template <bool SWAP, bool F16>
+template <bool SWAP>
 __device__ __forceinline__ void mfma1(const bf16x8 (&a)[4], const bf16x8 (&b)[2], f32x16 (&acc)[4][2], int idx) {
   const int bi = idx >> 1, bj = idx & 1;
-  acc[bi][bj] = SWAP ? anc_mfma<F16>(b[bj], a[bi], acc[bi][bj]) : anc_mfma<F16>(a[bi], b[bj], acc[bi][bj]);
+  acc[bi][bj] = SWAP ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bj], a[bi], acc[bi][bj], 0, 0, 0)
+                     : __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
 }
 // 8 MFMAs with the fragment reads of the next 8 (`load(idx)`) and N DMA instructions (`piece(i)`) between them, instead
 // of as bursts during which the matrix pipe idles and the LDS serves all wavefronts at once.
 // (PART: the wavefront's part of a tile, see kFull)
-template <bool SWAP, bool F16, int N, int PART, typename L, typename F>
+template <bool SWAP, int N, int PART, typename L, typename F>
 __device__ __forceinline__ void mfma8_with(const bf16x8 (&a)[4], const bf16x8 (&b)[2], f32x16 (&acc)[4][2], L load, F piece) {
 #pragma unroll
   for (int idx = 0; idx < 8; ++idx) {
-    if (PART == kFull || (PART == kLower && idx >= 4)) mfma1<SWAP, F16>(a, b, acc, idx);
+    if (PART == kFull || (PART == kLower && idx >= 4)) mfma1<SWAP>(a, b, acc, idx);
     __builtin_amdgcn_sched_barrier(0);
     load(idx);
 #pragma unroll
@@ -161,8 +162,7 @@ __device__ __forceinline__ void dma16_epi(const void *g, uint32_t lds_base) {
 // for the activations of a weight-gradient GEMM as they lie (C = x^T dy) and for the chain's
 // own B X, whose B is symmetric (stored in full): B read by rows k is B^T read by rows m, the
 // same values in the same order of summation.
-// FMT: the 16-bit floats of operands and outputs (FMT_BF16 ..).
-template <int EPI, int TM, int TN, int NS, int MINBLOCKS, int VAR = VAR_NONE, bool AT = false, int FMT = FMT_BF16>
+template <int EPI, int TM, int TN, int NS, int MINBLOCKS, int VAR = VAR_NONE, bool AT = false>
 __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_gemm_big(NsGemmMulti pm) {
   constexpr int NWN = TN / 64, NWAVES = (TM / 128) * NWN;
   constexpr int TK = 32;                            // a K tile is one 32-column panel
@@ -190,7 +190,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   __shared__ __attribute__((aligned(1024))) unsigned char aux[EPI != EPI_GRAM ? NWAVES * 1024 : 16];
 
   int gsel, L;
-  constexpr bool PLAINV = (VAR == VAR_PLAIN), F16 = FMT == FMT_F16, F16OUT = FMT != FMT_BF16;
+  constexpr bool PLAINV = (VAR == VAR_PLAIN);
   if (PLAINV && pm.seq) anc_seq_tile(pm, (int)blockIdx.x, (int)gridDim.x, gsel, L);
   else anc_group_tile(pm, (int)blockIdx.x, gsel, L);
   const NsGemm &p = pm.g[gsel];
@@ -406,7 +406,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
       constexpr bool kSteady = decltype(steady)::value;
       const bool more = kSteady || step + 1 < nk;
       const bool refill = kSteady || step + NS - 1 < nk;
-      mfma8_with<BT, F16, IPT, P>(a[0], b[0], acc, [&](int idx) { if (P != kNone) frag(cur, cur, 1, idx, a[1], b[1]); },
+      mfma8_with<BT, IPT, P>(a[0], b[0], acc, [&](int idx) { if (P != kNone) frag(cur, cur, 1, idx, a[1], b[1]); },
                           [&](int i) { if (refill) issue_piece(i, fill, curA, curB); });
       if (refill) {
         curA += advA;
@@ -416,7 +416,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         wait_vm<0>();
       }
       lds_barrier();
-      mfma8_with<BT, F16, 0, P>(a[1], b[1], acc, [&](int idx) { if (P != kNone && more) frag(nxt, nxt, 0, idx - 1, a[0], b[0]); }, [](int) {});
+      mfma8_with<BT, 0, P>(a[1], b[1], acc, [&](int idx) { if (P != kNone && more) frag(nxt, nxt, 0, idx - 1, a[0], b[0]); }, [](int) {});
     };
     int step = 0;
     // rounds of NS tiles in which even the last tile (step + NS - 1) still refills the ring
@@ -478,48 +478,48 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         // P0
         auto load0 = [&](int idx) { if (P != kNone) frag(H, H, 1, idx, a[y], b[1]); };
         if (NS == 4) {
-          mfma8_with<BT, F16, PL, P>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_l(i, L1); });
+          mfma8_with<BT, PL, P>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_l(i, L1); });
           if (more) adv_l();
         } else {
-          mfma8_with<BT, F16, PH, P>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_h(i, H1); });
+          mfma8_with<BT, PH, P>(a[x], b[0], acc, load0, [&](int i) { if (more) piece_h(i, H1); });
           if (more) adv_h();
         }
         // P1
         if (P == kFull) {
 #pragma unroll
-          for (int idx = 0; idx < 4; ++idx) mfma1<BT, F16>(a[y], b[1], acc, idx);
+          for (int idx = 0; idx < 4; ++idx) mfma1<BT>(a[y], b[1], acc, idx);
         }
         if (more) wait_vm<NS == 4 ? PH + PL : PH>(); else wait_vm<0>();
         lds_barrier();
 #pragma unroll
         for (int idx = 4; idx < 8; ++idx) {
           if (P == kNone) break;
-          mfma1<BT, F16>(a[y], b[1], acc, idx);
+          mfma1<BT>(a[y], b[1], acc, idx);
           __builtin_amdgcn_sched_barrier(0);
           if (idx < 6) b[0][idx - 4] = frag_b(L, 1, idx - 4);
           else a[x][idx - 6] = NT == 3 ? frag_a(L, 1, idx - 6) : frag_a(H, 0, idx - 6);
           __builtin_amdgcn_sched_barrier(0);
         }
         // P2 (of two terms: its last half, P4 has two fragments of A yet to come)
-        mfma8_with<BT, F16, 0, P>(a[y], b[0], acc, [&](int idx) {
+        mfma8_with<BT, 0, P>(a[y], b[0], acc, [&](int idx) {
           if (P == kNone) return;
           if (idx < 2) a[x][2 + idx] = NT == 3 ? frag_a(L, 1, 2 + idx) : frag_a(H, 0, 2 + idx);
           else if (NT == 2 && idx < 4) b[1][idx - 2] = frag_b(L, 0, idx - 2);
         }, none);
         if (NT == 3) {
           // P3, P4
-          mfma8_with<BT, F16, 0, P>(a[x], b[1], acc, [&](int idx) { if (P != kNone) frag(H, L, 0, idx, a[y], b[0]); }, none);
-          mfma8_with<BT, F16, 0, P>(a[y], b[0], acc, [&](int idx) { if (P != kNone) frag(L, H, 0, idx, a[x], b[1]); }, none);
+          mfma8_with<BT, 0, P>(a[x], b[1], acc, [&](int idx) { if (P != kNone) frag(H, L, 0, idx, a[y], b[0]); }, none);
+          mfma8_with<BT, 0, P>(a[y], b[0], acc, [&](int idx) { if (P != kNone) frag(L, H, 0, idx, a[x], b[1]); }, none);
         }
         if (more) wait_vm<NS == 4 ? PL : 0>(); else wait_vm<0>();
         lds_barrier();
         // P5 (P4 of two terms)
         auto load5 = [&](int idx) { if (P != kNone && more) frag(H1, H1, 0, idx - 1, a[y], b[0]); };
         if (NS == 4) {
-          mfma8_with<BT, F16, PH, P>(a[x], b[1], acc, load5, [&](int i) { if (more2) piece_h(i, H); });
+          mfma8_with<BT, PH, P>(a[x], b[1], acc, load5, [&](int i) { if (more2) piece_h(i, H); });
           if (more2) adv_h();
         } else {
-          mfma8_with<BT, F16, PL, P>(a[x], b[1], acc, load5, [&](int i) { if (more) piece_l(i, H); });
+          mfma8_with<BT, PL, P>(a[x], b[1], acc, load5, [&](int i) { if (more) piece_l(i, H); });
           if (more) adv_l();
         }
       };
@@ -574,8 +574,8 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   // a slab below the diagonal's 64x64 blocks is written twice
   auto mirrored = [&](int bi) { return EPI != EPI_BX && ((gi0w + bi * 32) >> 6) > (gj0w >> 6); };
   float sc = 1.0f;
-  if (EPI != EPI_BMAT && !F16 && p.scale != nullptr) sc = anc_ld_const(p.scale + e);
-  const float acc_scale = F16 ? kF16Inv * kF16Inv : (EPI == EPI_GRAM) ? sc * sc : sc;
+  if (EPI != EPI_BMAT && p.scale != nullptr) sc = anc_ld_const(p.scale + e);
+  const float acc_scale = (EPI == EPI_GRAM) ? sc * sc : sc;
   // residual output (Fl of GRAM, Bl of BMAT): for every matrix, or only for those in the band of
   // the second conditioning gate (uniform over the workgroup: a function of the matrix)
   const bool write_lo = (EPI == EPI_GRAM ? p.Fl != nullptr : EPI == EPI_BMAT ? p.Bl != nullptr : false) &&
@@ -606,8 +606,8 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   // matrix): a 32x64 slab of bytes is 32 rows of two (M, 32)-byte panels, 1 KiB contiguous each: 2
   // DMA instructions instead of 4, in the buffer [panel][row][32 bytes].
   // (readfirstlane: the flags live in scalar registers, so the branches on them are scalar branches)
-  const bool in8 = EPI == EPI_BX && !PLAINV && FMT == FMT_BF16 && __builtin_amdgcn_readfirstlane((int)anc_ns_low8(p, e, p.l8_in)) != 0;
-  const bool out8 = EPI == EPI_BX && !PLAINV && FMT == FMT_BF16 && __builtin_amdgcn_readfirstlane((int)anc_ns_low8(p, e, p.l8_out)) != 0;
+  const bool in8 = EPI == EPI_BX && !PLAINV && __builtin_amdgcn_readfirstlane((int)anc_ns_low8(p, e, p.l8_in)) != 0;
+  const bool out8 = EPI == EPI_BX && !PLAINV && __builtin_amdgcn_readfirstlane((int)anc_ns_low8(p, e, p.l8_out)) != 0;
   // In the buffer the two 16-byte halves of a row's 32 bytes are swapped for rows with bit 3 set:
   // LDS chunk l holds row l/2, half (l%2) ^ ((l/16)%2), which halves the bank conflicts of the
   // 4-byte accesses below (rows 8 apart would otherwise meet in one bank four at a time).
@@ -794,7 +794,8 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
             for (int r = 0; r < 16; ++r) {
               const uint32_t wh = (r & 2) ? xh[bj][r >> 2].y : xh[bj][r >> 2].x;
               const uint32_t wl = (r & 2) ? xl[bj][r >> 2].y : xl[bj][r >> 2].x;
-              const float x = ((r & 1) ? anc_half_hi<F16>(wh) : anc_half_lo<F16>(wh)) + ((r & 1) ? anc_half_hi<F16>(wl) : anc_half_lo<F16>(wl));
+              const float x = ((r & 1) ? __uint_as_float(wh & 0xFFFF0000u) : __uint_as_float(wh << 16)) +
+                              ((r & 1) ? __uint_as_float(wl & 0xFFFF0000u) : __uint_as_float(wl << 16));
               y[bj][r] = x;
             }
         } else {
@@ -821,7 +822,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
         // y = (a + dB) x + B X; only the first iteration carries the input's scale (times 1.0f is the
         // identity, so leaving the factors out elsewhere changes no bit; the fused instantiation,
         // which has no register to spare for a second version, keeps them)
-        if (!F16 && (fused || p.scale != nullptr)) {
+        if (fused || p.scale != nullptr) {
 #pragma unroll
           for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
@@ -831,14 +832,6 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
           for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
             for (int r = 0; r < 16; ++r) y[bj][r] = cf * y[bj][r] + acc[bi][bj][r];
-        }
-        // (fp16: the iterate's factor, gone in a result, there in an iterate)
-        constexpr float kOut = F16 ? kF16Inv : kF16Iterate;
-        if (F16 ? fused || fp32_out : F16OUT) {
-#pragma unroll
-          for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) y[bj][r] = y[bj][r] * kOut;
         }
       }
       if (fp32_out || fused || plain) {
@@ -945,8 +938,8 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               uint32_t h0, l0, h1, l1;
-              anc_pk_pair_as<F16OUT>(y[bj][4 * q], y[bj][4 * q + 1], h0, l0);
-              anc_pk_pair_as<F16OUT>(y[bj][4 * q + 2], y[bj][4 * q + 3], h1, l1);
+              anc_pk_pair(y[bj][4 * q], y[bj][4 * q + 1], h0, l0);
+              anc_pk_pair(y[bj][4 * q + 2], y[bj][4 * q + 3], h1, l1);
               const anc_u32x2 wh = {h0, h1}, wl = {l0, l1};
               const int off = rr * 128 + (((bj * 4 + q) ^ key) * 16) + hh * 8;
               *(anc_u32x2 *)(b + off) = wh;
@@ -1040,8 +1033,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int row = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            const uint32_t h = *(const uint16_t *)(b + bj * 2048 + row * 64 + (lane & 31) * 2);
-            in[bj][r] = anc_half_lo<F16>(h);
+            in[bj][r] = anc_bf16_bits_to_f32(*(const uint16_t *)(b + bj * 2048 + row * 64 + (lane & 31) * 2));
           }
       }
 #pragma unroll
@@ -1112,12 +1104,12 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
 #pragma unroll
       for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) anc_pk_pair_as<F16>(ov[bj][2 * i], ov[bj][2 * i + 1], hv[bj][i], lv[bj][i]);
+        for (int i = 0; i < 8; ++i) anc_pk_pair(ov[bj][2 * i], ov[bj][2 * i + 1], hv[bj][i], lv[bj][i]);
     } else {
 #pragma unroll
       for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) { hv[bj][i] = anc_pk<F16>(ov[bj][2 * i], ov[bj][2 * i + 1]); lv[bj][i] = 0u; }
+        for (int i = 0; i < 8; ++i) { hv[bj][i] = anc_pk_bf16(ov[bj][2 * i], ov[bj][2 * i + 1]); lv[bj][i] = 0u; }
     }
     // Where the slab (rows gi0.., columns gj0w..) and its mirror image (rows gj0w.., columns gi0..:
     // 64 rows of one 32-column panel, a contiguous 4 KiB in panel layout) go in an (M, M) matrix.
@@ -1145,7 +1137,7 @@ __global__ void __launch_bounds__((TM / 128) * (TN / 64) * 64, MINBLOCKS) k_ns_g
   }
 }
 
-template <int EPI, int FMT>
+template <int EPI>
 int launch_sym(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s) {
   NsGemmMulti pm{};
   pm.n = n;
@@ -1161,9 +1153,9 @@ int launch_sym(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s) {
   }
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_big: grid out of range");
   if (ps[0].stream_out & kStream256)
-    hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 4, 1, VAR_STREAM, false, FMT>), dim3((unsigned)grid), dim3(512), 0, s, pm);
+    hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 4, 1, VAR_STREAM>), dim3((unsigned)grid), dim3(512), 0, s, pm);
   else
-    hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 4, 1, VAR_NONE, false, FMT>), dim3((unsigned)grid), dim3(512), 0, s, pm);
+    hipLaunchKernelGGL((k_ns_gemm_big<EPI, 256, 256, 4, 1, VAR_NONE>), dim3((unsigned)grid), dim3(512), 0, s, pm);
   ANC_LAUNCH_CHECK();
   return ANC_OK;
 }
@@ -1172,8 +1164,7 @@ int launch_sym(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s) {
 
 namespace {
 
-// One X = a X + B X launch over the given problems, B fetched by rows k or (bf16 alone) by rows m.
-template <int FMT>
+// One X = a X + B X launch over the given problems, B fetched by rows k or by rows m.
 int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const NsUpdate *upd, bool by_rows) {
   NsGemmMulti pm{};
   pm.n = n;
@@ -1206,8 +1197,6 @@ int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const N
   }
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_big: grid out of range");
   const bool fused = ps[0].upd != nullptr;
-  constexpr bool kRows = FMT != FMT_BF16;
-  constexpr int kLastFmt = FMT == FMT_TO_F16 ? FMT_F16 : FMT;           // (the last product writes no iterate)
   if (fused) {
     for (int k = 0; k < ANC_MUON_MAX_SCALES; ++k) pm.lr[k] = upd->lr[k];
     pm.sr = upd->sr;
@@ -1216,24 +1205,24 @@ int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const N
   }
   if (fused && (upd->sr & ANC_MUON_P16T)) {
     if (by_rows)
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE_T, true, kLastFmt>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE_T, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
     else
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE_T, kRows, kLastFmt>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE_T, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   } else if (fused) {
     if (by_rows)
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE, true, kLastFmt>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
     else
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE, kRows, kLastFmt>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_UPDATE, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   } else if (ps[0].stream_out & kStream256) {
     if (by_rows)
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_STREAM, true, FMT>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_STREAM, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
     else
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_STREAM, kRows, FMT>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_STREAM, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   } else {
     if (by_rows)
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_NONE, true, FMT>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_NONE, true>), dim3((unsigned)grid), dim3(256), 0, s, pm);
     else
-      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_NONE, kRows, FMT>), dim3((unsigned)grid), dim3(256), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_big<EPI_BX, 128, 256, 3, 2, VAR_NONE, false>), dim3((unsigned)grid), dim3(256), 0, s, pm);
   }
   ANC_LAUNCH_CHECK();
   return ANC_OK;
@@ -1241,26 +1230,17 @@ int launch_bx(const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, const N
 
 }  // namespace
 
-#ifdef ANC_NS_F16_UNIT
-int anc_ns_gemm_big_f16(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int fmt, const NsUpdate *upd) {
-  if (epi == EPI_GRAM) return launch_sym<EPI_GRAM, FMT_F16>(ps, Es, n, s);
-  if (epi == EPI_BMAT) return launch_sym<EPI_BMAT, FMT_F16>(ps, Es, n, s);
-  return fmt == FMT_F16 ? launch_bx<FMT_F16>(ps, Es, n, s, upd, true) : launch_bx<FMT_TO_F16>(ps, Es, n, s, upd, true);
-}
-#else
 // Symmetric products run on 256x256 tiles (lower triangle); X = a X + B X runs on 128x256 tiles
 // (the tile counts of the problems are recomputed here).
-int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool by_rows, int fmt,
+int anc_ns_gemm_big_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, bool by_rows,
                           const NsUpdate *upd) {
   ANC_REQUIRE(n >= 1 && n <= kMaxGroups, "anc_ns_gemm_big: 1..%d problems per launch", kMaxGroups);
   for (int k = 0; k < n; ++k)
     ANC_REQUIRE(ps[k].M % 256 == 0 && ps[k].N % 256 == 0 && ps[k].K % 32 == 0,
                 "anc_ns_gemm_big: dims must be multiples of 256");
-  ANC_REQUIRE(fmt == FMT_BF16 || epi != EPI_BX || by_rows, "anc_ns_gemm_big: fp16 reads B by rows k");
-  if (fmt != FMT_BF16) return anc_ns_gemm_big_f16(epi, ps, Es, n, s, fmt, upd);
-  if (epi == EPI_GRAM) return launch_sym<EPI_GRAM, FMT_BF16>(ps, Es, n, s);
-  if (epi == EPI_BMAT) return launch_sym<EPI_BMAT, FMT_BF16>(ps, Es, n, s);
-  return launch_bx<FMT_BF16>(ps, Es, n, s, upd, by_rows);
+  if (epi == EPI_GRAM) return launch_sym<EPI_GRAM>(ps, Es, n, s);
+  if (epi == EPI_BMAT) return launch_sym<EPI_BMAT>(ps, Es, n, s);
+  return launch_bx(ps, Es, n, s, upd, by_rows);
 }
 
 // Bare products C[e] = A[e] B[e] (fp32 out, p.X32), A (M, K) with row pitch p.ldA -- or, with
@@ -1321,4 +1301,3 @@ int anc_ns_gemm_big_plain(const NsGemm *ps, const int64_t *Es, int n, hipStream_
   ANC_LAUNCH_CHECK();
   return ANC_OK;
 }
-#endif

@@ -80,15 +80,14 @@ constexpr int tile_per_cu(int wm, int wn, int ring) { return (wm == 1 ? ring == 
 __host__ __device__ constexpr int anc_sym_tiles(int rows) { return rows * (rows + 1) / 2; }
 
 // SOLO: the launch has one problem, its arguments lie at fixed places.
-// FMT: the 16-bit floats of operands and outputs (FMT_BF16 ..).
 // VAR_STATS (B = b A + c A A of one matrix): the workgroups behind the tiles make the gates' statistics.
 // (by specialisation: an expression in the kernel's signature enters its name, and an unnamed enum has other names there on the host)
 template <int VAR, bool SOLO> struct TileArgs { using type = NsGemmArgs<SOLO ? 1 : kMaxGroups>; };
 template <> struct TileArgs<VAR_STATS, true> { using type = NsStatArgs; };
-template <int EPI, int WM, int WN, int NW, bool AT, int VAR, int kRing, bool SOLO, int FMT = FMT_BF16>
+template <int EPI, int WM, int WN, int NW, bool AT, int VAR, int kRing, bool SOLO>
 __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) * NW / 4) k_ns_gemm_tile(typename TileArgs<VAR, SOLO>::type pm) {
   constexpr int WC = NW / 2, TM = 64 * WM, TN = 32 * WN * WC, KP = WM == 1 ? 2 : 1, TK = 32 * KP;
-  constexpr bool BT = EPI == EPI_BX, PLAINV = VAR == VAR_PLAIN, F16 = FMT == FMT_F16, F16OUT = FMT != FMT_BF16;
+  constexpr bool BT = EPI == EPI_BX, PLAINV = VAR == VAR_PLAIN;
   constexpr int kHalf = TM * TK * 2, kStageBytes = kHalf + TN * TK * 2;      // A's part of a stage, a stage
   constexpr int PA = TM * KP / (16 * NW), PB = TN * KP / (16 * NW), kIps = PA + PB;        // DMA instructions per wavefront and stage
   static_assert(!AT || BT, "A by rows k: X = a X + B X and the plain product only");
@@ -229,13 +228,13 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   const int64_t mm = (int64_t)e * M * M, mn = (int64_t)e * M * N, mv = (int64_t)e * M;
   float *sg = (float *)lds + wave * 32 * kSgPitch;
   float sc = 1.0f;
-  if (EPI != EPI_BMAT && !PLAINV && !F16 && p.scale != nullptr) sc = anc_ld_const(p.scale + e);
-  const float acc_scale = F16 ? kF16Inv * kF16Inv : (EPI == EPI_GRAM) ? sc * sc : sc;
+  if (EPI != EPI_BMAT && !PLAINV && p.scale != nullptr) sc = anc_ld_const(p.scale + e);
+  const float acc_scale = (EPI == EPI_GRAM) ? sc * sc : sc;
   const bool write_lo = (EPI == EPI_GRAM ? p.Fl != nullptr : EPI == EPI_BMAT ? p.Bl != nullptr : false) &&
                         (p.lo_gated == 0 || anc_ns_wide(p, e));
   const bool has_a32 = EPI != EPI_BX && anc_ns_has_a32(p, e);
-  const bool in8 = EPI == EPI_BX && !PLAINV && FMT == FMT_BF16 && anc_ns_low8(p, e, p.l8_in);
-  const bool out8 = EPI == EPI_BX && !PLAINV && FMT == FMT_BF16 && anc_ns_low8(p, e, p.l8_out);
+  const bool in8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_in);
+  const bool out8 = EPI == EPI_BX && !PLAINV && anc_ns_low8(p, e, p.l8_out);
   // This lane's 16 elements of a 32x32 block: NR runs of RUN consecutive columns (reading the block transposed, rows),
   // run r in row lrow + RS r from column c0. 32/RUN neighbouring lanes share a row, so that one instruction covers
   // whole lines.
@@ -331,7 +330,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
     for (int bi = 0; bi < WM; ++bi)
 #pragma unroll
       for (int bj = 0; bj < WN; ++bj)      // operands exchanged: a lane ends with runs of 4 columns of one row
-        acc[bi][bj] = anc_mfma<F16>(b[bj], a[bi], acc[bi][bj]);
+        acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[bj], a[bi], acc[bi][bj], 0, 0, 0);
   };
 
   auto frags = [&](const unsigned char *st, int kk, bf16x8 (&fa)[WM], bf16x8 (&fb)[WN]) {
@@ -658,17 +657,16 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   };
   auto unpack = [&](const uint32_t (&u)[8], float (&x)[16]) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) { x[2 * i] = anc_half_lo<F16>(u[i]); x[2 * i + 1] = anc_half_hi<F16>(u[i]); }
+    for (int i = 0; i < 8; ++i) { x[2 * i] = __uint_as_float(u[i] << 16); x[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u); }
   };
   constexpr bool kStreamX = EPI == EPI_BX && VAR == VAR_STREAM;
-  // 16 floats -> 16-bit runs at out + r * step, and the residuals at lo likewise if not null
-  auto put_16 = [&](auto f16, uint16_t *out, uint16_t *lo, int64_t step) {
-    constexpr bool H = decltype(f16)::value;
+  // 16 floats -> bf16 runs at out + r * step, and the residuals at lo likewise if not null
+  auto put_bf16 = [&](uint16_t *out, uint16_t *lo, int64_t step) {
     uint32_t h[8], l[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      if (lo != nullptr) anc_pk_pair_as<H>(v[2 * i], v[2 * i + 1], h[i], l[i]);
-      else h[i] = anc_pk<H>(v[2 * i], v[2 * i + 1]);
+      if (lo != nullptr) anc_pk_pair(v[2 * i], v[2 * i + 1], h[i], l[i]);
+      else h[i] = anc_pk_bf16(v[2 * i], v[2 * i + 1]);
     }
 #pragma unroll
     for (int r = 0; r < NR; ++r) st_run<RUN * 2, kStreamX>(out + r * step, h + r * (RUN / 2));
@@ -771,13 +769,12 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
           if (dc >= 0) p.dB[mv + gj + dc] = dv;
         }
         uint16_t *oh = EPI == EPI_GRAM ? p.Fh : p.Bh, *ol = EPI == EPI_GRAM ? p.Fl : p.Bl;
-        constexpr std::bool_constant<F16> fmt{};
-        if (!image) put_16(fmt, oh + mm + pan, write_lo ? ol + mm + pan : nullptr, pst);
+        if (!image) put_bf16(oh + mm + pan, write_lo ? ol + mm + pan : nullptr, pst);
         if (mirror) {                        // mirror image: rows gj0 .., 32-column panel gi0/32
           put_rows();
           get_cols();
           const int64_t pt = ((int64_t)(gi0 / 32) * M + gj0 + lrow) * 32 + c0;
-          put_16(fmt, oh + mm + pt, write_lo ? ol + mm + pt : nullptr, pst);
+          put_bf16(oh + mm + pt, write_lo ? ol + mm + pt : nullptr, pst);
           lds_wave_sync();
         }
       } else if constexpr (PLAINV) {
@@ -816,18 +813,12 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
 #pragma unroll
           for (int k = 0; k < 16; ++k) x[k] = x[k] + xl[k];
         }
-        if (!F16 && p.scale != nullptr) {
+        if (p.scale != nullptr) {
 #pragma unroll
           for (int k = 0; k < 16; ++k) v[k] = (p.ca + drow[bi][k / RUN]) * (x[k] * sc) + v[k] * acc_scale;
         } else {
 #pragma unroll
           for (int k = 0; k < 16; ++k) v[k] = (p.ca + drow[bi][k / RUN]) * x[k] + v[k];
-        }
-        // (fp16: the iterate's factor, gone in a result, there in an iterate)
-        constexpr float kOut = F16 ? kF16Inv : kF16Iterate;
-        if (F16 ? VAR == VAR_UPDATE || p.Yh == nullptr : F16OUT) {
-#pragma unroll
-          for (int k = 0; k < 16; ++k) v[k] = v[k] * kOut;
         }
         if constexpr (VAR == VAR_UPDATE) {
           // W -= lr O on the block's 32x32 elements of the weight (transposed where the chain ran on W^T)
@@ -887,7 +878,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
           for (int i = 0; i < 4; ++i)
             *(anc_f32x4 *)(p.X32 + mn + quad(i, N)) = anc_f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
         } else if (p.X16 != nullptr) {
-          put_16(std::false_type{}, p.X16 + mn + (int64_t)gi * N + gj, nullptr, (int64_t)RS * N);
+          put_bf16(p.X16 + mn + (int64_t)gi * N + gj, nullptr, (int64_t)RS * N);
         } else if (out8) {
           uint32_t h[8], q[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -901,7 +892,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
             st_run<RUN, kStreamX>((char *)p.Yl + mn * 2 + pan + r * pst, q + r * (RUN / 4));
           }
         } else {
-          put_16(std::bool_constant<F16OUT>{}, p.Yh + mn + pan, p.Yl + mn + pan, pst);
+          put_bf16(p.Yh + mn + pan, p.Yl + mn + pan, pst);
         }
       }
     }
@@ -914,7 +905,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
 // 640 tokens (1536 tiles 15.6 / 15.7 at 384, 18.7 / 19.0 at 640), but with eight some of the cards took 16 .. 21 there.
 constexpr int kLongPlain = 2048;
 
-template <int EPI, bool AT, int VAR, int FMT>
+template <int EPI, bool AT, int VAR>
 void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm, const NsStatOne *stat = nullptr) {
   if constexpr (VAR == VAR_PLAIN) {
     if (tile == kTile128x64) {
@@ -930,13 +921,13 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm, 
   }
   if constexpr (VAR == VAR_NONE && EPI != EPI_GRAM) {
     if (tile == 128 && (pm.g[0].stream_out & kStream128)) {
-      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, 8, AT, VAR_STREAM, 4, false, FMT>), dim3(grid), dim3(512), 0, s, pm);
+      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, 8, AT, VAR_STREAM, 4, false>), dim3(grid), dim3(512), 0, s, pm);
       return;
     }
   }
-  if (tile == 128)      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, 8, AT, VAR, 4, false, FMT>), dim3(grid), dim3(512), 0, s, pm);
-  else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 3, false, FMT>), dim3(grid), dim3(256), 0, s, pm);
-  else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 4, false, FMT>), dim3(grid), dim3(256), 0, s, pm);
+  if (tile == 128)      hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 2, 1, 8, AT, VAR, 4, false>), dim3(grid), dim3(512), 0, s, pm);
+  else if (grid > 256)  hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 3, false>), dim3(grid), dim3(256), 0, s, pm);
+  else if (pm.n > 1)    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 4, false>), dim3(grid), dim3(256), 0, s, pm);
   else {
     NsStatArgs one;
     one.n = 1;
@@ -946,47 +937,23 @@ void launch_tile(int tile, unsigned grid, hipStream_t s, const NsGemmMulti &pm, 
     one.sr = pm.sr;
     one.seed_base = pm.seed_base;
     one.ctl = pm.ctl;
-    if constexpr (EPI == EPI_BMAT && VAR == VAR_NONE && FMT == FMT_BF16) {
+    if constexpr (EPI == EPI_BMAT && VAR == VAR_NONE) {
       if (stat != nullptr) {
         one.tiles_only = (int)grid;
         one.stat = *stat;
-        hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR_STATS, 4, true, FMT>), dim3(grid + kCondParts + stat->parts), dim3(256), 0, s, one);
+        hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR_STATS, 4, true>), dim3(grid + kCondParts + stat->parts), dim3(256), 0, s, one);
         return;
       }
     }
-    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 4, true, FMT>), dim3(grid), dim3(256), 0, s, (const NsGemmArgs<1> &)one);
+    hipLaunchKernelGGL((k_ns_gemm_tile<EPI, 1, 1, 4, AT, VAR, 4, true>), dim3(grid), dim3(256), 0, s, (const NsGemmArgs<1> &)one);
   }
-}
-
-// X = a X + B X of a chain's iterations but the last (`by_rows` false: bf16 alone)
-template <int FMT>
-void launch_tiles_bx(int tile, unsigned gr, hipStream_t s, const NsGemmMulti &pm, bool by_rows) {
-  if (by_rows) launch_tile<EPI_BX, true, VAR_NONE, FMT>(tile, gr, s, pm);
-  else         launch_tile<EPI_BX, FMT != FMT_BF16, VAR_NONE, FMT>(tile, gr, s, pm);
-}
-// Any product of a chain (`update`: the last with the weight update)
-template <int FMT>
-void launch_tiles(int epi, int tile, unsigned gr, hipStream_t s, const NsGemmMulti &pm, bool by_rows, bool update) {
-  if (epi == EPI_GRAM)      launch_tile<EPI_GRAM, false, VAR_NONE, FMT>(tile, gr, s, pm);
-  else if (epi == EPI_BMAT) launch_tile<EPI_BMAT, false, VAR_NONE, FMT>(tile, gr, s, pm);
-  else if (!update)         launch_tiles_bx<FMT>(tile, gr, s, pm, by_rows);
-  else if (by_rows)         launch_tile<EPI_BX, true, VAR_UPDATE, FMT>(tile, gr, s, pm);
-  else                      launch_tile<EPI_BX, FMT != FMT_BF16, VAR_UPDATE, FMT>(tile, gr, s, pm);
 }
 
 }  // namespace
 
-#ifdef ANC_NS_F16_UNIT
-void anc_ns_gemm_tile_f16(int epi, int tile, unsigned gr, hipStream_t s, const NsGemmMulti &pm, bool update) {
-  launch_tiles<FMT_F16>(epi, tile, gr, s, pm, true, update);
-}
-void anc_ns_gemm_tile_to_f16(int tile, unsigned gr, hipStream_t s, const NsGemmMulti &pm) {
-  launch_tiles_bx<FMT_TO_F16>(tile, gr, s, pm, true);
-}
-#else
 // n <= kMaxGroups problems of the same product in one launch on tiles of 64, 128 or 128x64 (kTile128x64). EPI_BX:
 // `by_rows` as for the 256-wide tiles; `plain`: the bare product, A transposed (by_rows) or not.
-int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int tile, bool by_rows, int fmt,
+int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, hipStream_t s, int tile, bool by_rows,
                            const NsUpdate *upd, bool plain, const NsStatOne *stat) {
   const int TM = tile == 64 ? 64 : 128, TN = tile == 128 ? 128 : 64;
   ANC_REQUIRE(plain || TM == TN, "anc_ns_gemm_tile: tiles of 128x64 are the plain product's");
@@ -1029,23 +996,27 @@ int anc_ns_gemm_tile_multi(int epi, const NsGemm *ps, const int64_t *Es, int n, 
     grid += pm.tiles[k];
   }
   ANC_REQUIRE(grid < (1ll << 31), "anc_ns_gemm_tile: grid out of range");
+  ANC_REQUIRE(stat == nullptr || (n == 1 && epi == EPI_BMAT && tile == 64 && grid <= kStatTiles),
+              "anc_ns_gemm_tile: statistics go with one matrix's B on tiles of 64");
   const unsigned gr = (unsigned)grid;
-  if (upd != nullptr) {
+  if (plain) {
+    if (by_rows) launch_tile<EPI_BX, true, VAR_PLAIN>(tile, gr, s, pm);
+    else         launch_tile<EPI_BX, false, VAR_PLAIN>(tile, gr, s, pm);
+  } else if (epi == EPI_GRAM) {
+    launch_tile<EPI_GRAM, false, VAR_NONE>(tile, gr, s, pm);
+  } else if (epi == EPI_BMAT) {
+    launch_tile<EPI_BMAT, false, VAR_NONE>(tile, gr, s, pm, stat);
+  } else if (upd != nullptr) {
     for (int k = 0; k < ANC_MUON_MAX_SCALES; ++k) pm.lr[k] = upd->lr[k];
     pm.sr = upd->sr;
     pm.seed_base = upd->seed_base;
     pm.ctl = upd->ctl;
+    if (by_rows) launch_tile<EPI_BX, true, VAR_UPDATE>(tile, gr, s, pm);
+    else         launch_tile<EPI_BX, false, VAR_UPDATE>(tile, gr, s, pm);
+  } else {
+    if (by_rows) launch_tile<EPI_BX, true, VAR_NONE>(tile, gr, s, pm);
+    else         launch_tile<EPI_BX, false, VAR_NONE>(tile, gr, s, pm);
   }
-  ANC_REQUIRE(stat == nullptr || (n == 1 && epi == EPI_BMAT && tile == 64 && grid <= kStatTiles && fmt == FMT_BF16),
-              "anc_ns_gemm_tile: statistics go with one matrix's B on tiles of 64");
-  ANC_REQUIRE(fmt == FMT_BF16 || epi != EPI_BX || by_rows, "anc_ns_gemm_tile: fp16 reads B by rows k");
-  if (stat != nullptr)        launch_tile<EPI_BMAT, false, VAR_NONE, FMT_BF16>(tile, gr, s, pm, stat);
-  else if (fmt == FMT_F16)    anc_ns_gemm_tile_f16(epi, tile, gr, s, pm, upd != nullptr);
-  else if (fmt == FMT_TO_F16) anc_ns_gemm_tile_to_f16(tile, gr, s, pm);
-  else if (!plain)            launch_tiles<FMT_BF16>(epi, tile, gr, s, pm, by_rows, upd != nullptr);
-  else if (by_rows)           launch_tile<EPI_BX, true, VAR_PLAIN, FMT_BF16>(tile, gr, s, pm);
-  else                        launch_tile<EPI_BX, false, VAR_PLAIN, FMT_BF16>(tile, gr, s, pm);
   ANC_LAUNCH_CHECK();
   return ANC_OK;
 }
-#endif

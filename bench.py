@@ -169,7 +169,7 @@ def kernel_source_sha16():
     measured on."""
     import hashlib
     h = hashlib.sha256()
-    for f in ("ns_common.h", "lds_dma.h", "ns.hip", "ns_gemm_big.hip", "ns_gemm_tile.hip", "ns_gemm_big_f16.hip", "ns_gemm_tile_f16.hip"):
+    for f in ("ns_common.h", "lds_dma.h", "ns.hip", "ns_gemm_big.hip", "ns_gemm_tile.hip"):
         with open(os.path.join(ROOT, "ancora-cutile_amd", "csrc", f), "rb") as fh:
             h.update(fh.read())
     return h.hexdigest()[:16]

@@ -477,14 +477,9 @@ int anc_quant_mxfp8_w_multi(uint64_t desc_table, int32_t n_weights, int64_t tota
  *   ANC_NS_BF16_LATE3 for coefficients that do not drive the singular values to 1 (Keller's quintic,
  *                     ancora/kernels/muon_ns.py:21, leaves them in 0.7 .. 1.2, so operand rounding
  *                     stays a first-order error to the end: ANC_NS_BF16 reaches 2.8e-3 .. 5e-3 there).
- *                     M < 1024 as ANC_NS_BF16. M >= 1024, every matrix: five steps run on fp16 operands
- *                     and fp16 pairs from iteration 1 on (11 significant bits per operand, 22 per pair), with
- *                     the residual of X in the last iteration (M = 1024), in the last two (up to M = 1280 and
- *                     N = 3M), beyond that all residuals in the last two: 1.1 .. 1.8 times the work of
- *                     ANC_NS_BF16_FAST, 2e-5 .. 6e-4. Other lengths, and coefficients under which the values
- *                     could leave fp16's range, run on bf16 with the residual of X from iteration 2 on, of A
- *                     and B from iteration 3 on (the last three iterations of a chain shorter than 5 steps).
- *                     The wide gate below.
+ *                     Every matrix: residual of X from iteration 2 on, of A and B from iteration 3
+ *                     on (the last three iterations of a chain shorter than 5 steps); the wide gate
+ *                     below; 2.05 times the work of ANC_NS_BF16_FAST; 2e-5 .. 9e-4.
  *   ANC_NS_FP32       every product in fp32 (validation mode, 1e-5).
  *
  * Plan of ANC_NS_BF16 by shape

@@ -19,7 +19,6 @@ Rounding points modelled (same as the kernels):
     Fh Fl + Fl Fh where needed); the entries of A in the fp32 terms are the fp32 F where the chain
     keeps the fp32 copy of A and Fh where it does not; diag(B) in fp32 (dB), Boff -> Bh (, Bl);
   X' = (a + dB) (.) x + Boff X from bf16 operands: Bh Xh (+ Bh Xl) (+ Bl Xh);
-  bf16_late3 chains of five steps, M >= 1024: fp16 in the place of bf16 (F, Boff; both halves of 256 times the iterate) from iteration 1 on;
   where the plan says so (N >= 2M) and no product of the next iteration multiplies it, the low half
     Xl is kept as 8 bits relative to the ulp of Xh instead of a bf16.
 """
@@ -50,7 +49,6 @@ class Plan:
         self.wide_near_diff = 0.0    # > 0: the near range flags on proxy - colc > this instead of the ratio rule
         self.wide_from = 1
         self.drop_a32 = False
-        self.f16 = mode == "bf16_late3" and M >= 1024 and steps == 5       # fp16 operands and iterates from iteration 1 on
         self.low8 = False            # low halves of the iterate as 8 bits where no product multiplies them
         if mode == "bf16_x3":
             self.x_from = self.fb_from = 0
@@ -59,9 +57,6 @@ class Plan:
             self.x_from = self.fb_from = 2 if steps >= 5 else (steps - 3 if steps > 3 else 0)
             if steps >= 5:
                 self.fb_from = self.x_from + 1
-            if self.f16:
-                self.x_from = 4 if M < 1152 else 3
-                self.fb_from = 5 if M < 1152 or (M <= 1280 and N <= 3 * M) else 3
             if self.x_from > 1:
                 self.wide, self.wide_near = True, (TAU_WIDE_NEAR if N < 2 * M else TAU_WIDE_LO)
             return
@@ -136,11 +131,6 @@ def low8(y, Xh):
     return (x - Xh).astype(f32)
 
 
-def f16_round(x, scale=1.0):
-    """What a value kept as fp16 of `scale` times itself reads back as."""
-    return (np.asarray(x, dtype=f32) * f32(scale)).astype(np.float16).astype(f32) / f32(scale)
-
-
 def chain(X, sched, steps=5, mode="bf16", eps=1e-7, info=None, overrides=None):
     """The chain's result for one (M, N) fp32 matrix, M <= N, through the fp32-input entry
     (normalise, then the pair). `info`, if a dict, receives the statistics and decisions.
@@ -160,8 +150,6 @@ def chain(X, sched, steps=5, mode="bf16", eps=1e-7, info=None, overrides=None):
     proxy = colc = bulk = None
     flagged = False
     for k in range(steps):
-        half = f16_round if plan.f16 and k > 0 else bf16_round
-        out_half = (lambda t: f16_round(t, 256.0)) if plan.f16 else bf16_round
         a, b, c = (f32(t) for t in coef_at(sched, k))
         split, split_fb = k >= plan.x_from, k >= plan.fb_from
         over = (not split) and k in plan.gate_tau and proxy is not None and proxy > plan.gate_tau[k]
@@ -178,7 +166,7 @@ def chain(X, sched, steps=5, mode="bf16", eps=1e-7, info=None, overrides=None):
         d = G[idx, idx].copy()
         F = G.copy()
         F[idx, idx] = 0
-        Fh = half(F)
+        Fh = bf16_round(F)
         if k == 0:
             proxy, colc, bulk = statistics(Xh, Fh)
             flagged = wide_flag(plan, proxy, colc, bulk)
@@ -186,7 +174,7 @@ def chain(X, sched, steps=5, mode="bf16", eps=1e-7, info=None, overrides=None):
                 flagged = bool(overrides["wide"]) and plan.wide
         FF = Fh @ Fh
         if f3:
-            Fl = half(F - Fh)
+            Fl = bf16_round(F - Fh)
             P = Fh @ Fl
             FF = FF + P + P.T
         has_a32 = (not plan.drop_a32) or (k > 0 and flagged)
@@ -195,16 +183,16 @@ def chain(X, sched, steps=5, mode="bf16", eps=1e-7, info=None, overrides=None):
         Boff = b * Au + c * a2
         Boff[idx, idx] = 0
         dB = b * d + c * (FF[idx, idx] + d * d)
-        Bh = half(Boff)
+        Bh = bf16_round(Boff)
         Y = Bh @ Xh
         bx_l = (split or (gated_bx and not split_fb) or (wide_k and k < plan.fb_from)
                 or k in ov.get("bx_l", ()))
         if bx_l:
             Y = Y + Bh @ Xl
         if f3:
-            Y = Y + half(Boff - Bh) @ Xh
+            Y = Y + bf16_round(Boff - Bh) @ Xh
         y = (a + dB)[:, None] * (Xh + Xl) + Y
-        Xh = out_half(y)
+        Xh = bf16_round(y)
         # 8-bit low half where no product of the next iteration multiplies it
         nk = k + 1
         if (plan.low8 and nk < steps and plan.gate_tau and not flagged and nk < plan.x_from
@@ -212,7 +200,7 @@ def chain(X, sched, steps=5, mode="bf16", eps=1e-7, info=None, overrides=None):
                 and not any(nk in ov.get(key, ()) for key in ("gram3", "bx_l"))):
             Xl = low8(y, Xh)
         else:
-            Xl = out_half(y - Xh)
+            Xl = bf16_round(y - Xh)
     if info is not None:
         info.update(proxy=proxy, colc=colc, bulk=bulk, wide=flagged, plan=plan)
     return y
