@@ -315,7 +315,7 @@ __global__ void __launch_bounds__(kThreads) k_ns_cond(NsCondArgs a) {
 // once unless the matrix's proxy asks for the statistic. Then the partial sums are added in order and the flag is written that
 // every later product reads: DECIDE, by the matrix's first block where nobody asks and by the last to arrive where it does;
 // otherwise by k_ns_classify_order, for batches that a gated launch takes in another order. (A launch of its own, one wavefront per
-// matrix, was almost all start and end: the step of one (1024,3072) weight 216.7 -> 210.0 us without it.)
+// matrix, was almost all start and end: 6 us less for the step of one (1024,3072) weight.)
 __device__ __forceinline__ int anc_wave_sum_i32(int v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -1029,8 +1029,8 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       if (int rc = anc_ns_gemm_multi(EPI_GRAM, ga, Es, n, force, s)) return rc;
     }
     // One matrix whose B = b A + c A A runs on 64-wide tiles that leave CUs over: the statistics are workgroups of that launch, unless X = a X + B X
-    // of this iteration asks for them (8-bit low halves out). The step of one (1024,3072) weight 215.0 -> 212.0 us,
-    // the default step of a 1024x1024 model 358.6 -> 352.3: a launch's start and end twice less, B's own launch longer by part of that.
+    // of this iteration asks for them (8-bit low halves out). 3 us less for the step of one (1024,3072)
+    // weight, 4 for a 1024x1024 one: a launch's start and end twice less (4.6 and 3.5 us), B's own launch longer by part of that (8.9 -> 11.3).
     NsStatOne beside{};
     const bool with_b = k == 0 && want_cond && n == 1 && Es[0] == 1 && cp[0].scale0 != nullptr && !(gx[0].l8_out > 0.0) &&
                         !ordered(0) && (cp[0].M / 64) * (cp[0].M / 64 + 1) / 2 <= kStatTiles &&
