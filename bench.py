@@ -164,13 +164,28 @@ def measure_gemm_traffic(workload):
                    "write_unit_kib": round(res["WRITE_SIZE"][2], 4)}
 
 
+def kernel_sources():
+    """The Newton-Schulz kernels' sources and every header of this repository that they include."""
+    import re
+    todo = [os.path.join(ROOT, "ancora-cutile_amd", "csrc", f) for f in ("ns.hip", "ns_gemm_big.hip", "ns_gemm_tile.hip")]
+    found = []
+    while todo:
+        f = os.path.normpath(todo.pop(0))
+        if f in found:
+            continue
+        found.append(f)
+        with open(f) as fh:
+            todo += [os.path.join(os.path.dirname(f), h) for h in re.findall(r'^\s*#\s*include\s+"([^"]+)"', fh.read(), re.M)]
+    return found
+
+
 def kernel_source_sha16():
     """Hash of the Newton-Schulz kernel sources: ties a recorded counter figure to the code it was
     measured on."""
     import hashlib
     h = hashlib.sha256()
-    for f in ("ns_common.h", "lds_dma.h", "ns.hip", "ns_gemm_big.hip", "ns_gemm_tile.hip"):
-        with open(os.path.join(ROOT, "ancora-cutile_amd", "csrc", f), "rb") as fh:
+    for f in kernel_sources():
+        with open(f, "rb") as fh:
             h.update(fh.read())
     return h.hexdigest()[:16]
 
