@@ -1028,12 +1028,22 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       AncProfScope prof(ANC_PROF_NS_GRAM, s);
       if (int rc = anc_ns_gemm_multi(EPI_GRAM, ga, Es, n, force, s)) return rc;
     }
-    // One matrix whose B = b A + c A A runs on 64-wide tiles that leave CUs over: the statistics are workgroups of that launch, unless X = a X + B X
-    // of this iteration asks for them (8-bit low halves out). 3 us less for the step of one (1024,3072)
-    // weight, 4 for a 1024x1024 one: a launch's start and end twice less (4.6 and 3.5 us), B's own launch longer by part of that (8.9 -> 11.3).
+    // One matrix whose B = b A + c A A runs on 64-wide tiles that leave CUs over: the statistics are workgroups of that launch. The column
+    // statistic is read there whether the proxy asks for it or not: beyond kStatCols columns matrices that do not lose by it what those
+    // that do gain by the launches.
+    // us per chain, beside B / in launches of their own, plain matrices (with 1 % of the columns x100, which ask for it):
+    //   Keller     (1024,1024) 139.9 / 144.0 (139.4 / 148.9), (1152,1152) 173.9 / 178.2 (173.7 / 182.6), (1280,1280) 190.5 / 194.1 (191.0 / 199.0),
+    //              (1408,1408) 216.8 / 223.3 (217.0 / 228.0), (1024,3072) 236.2 / 239.7 (236.4 / 245.4), (1408,5632) 476.1 / 481.6 (481.3 / 488.1),
+    //              (1024,8192) 430.3 / 430.1 (433.7 / 440.3), (1280,8192) 573.0 / 573.9 (577.1 / 584.3), (1408,8192) 678.1 / 677.2 (680.9 / 691.0),
+    //              (1024,12288) 605.7 / 603.0 (610.2 / 616.6), (1152,12288) 755.4 / 750.8 (759.6 / 764.1), (1408,12288) 991.6 / 990.2 (997.5 /
+    //              1003.8); (1024,14336) 742.1 / 739.1 (749.1 / 753.1), (1024,16384) 827.5 / 820.1 (832.8 / 837.5), (1024,65536) 3117 / 3086
+    //              (3143 / 3141)
+    //   Polar Express  (1024,1024) 126.2 / 130.6 (131.4 / 141.0), (1152,2432) 173.8 / 176.9 (180.5 / 188.6), (1408,1408) 179.5 / 185.4 (203.6 / 214.6)
+    // Matrices whose next iterate has 8-bit low halves (Polar Express, N >= 2M) keep launches of their own, though nothing asks for that:
+    // (1024,3072) 177.0 there, 173.4 beside B, (1024,8192) 303.5, 303.8.
     NsStatOne beside{};
     const bool with_b = k == 0 && want_cond && n == 1 && Es[0] == 1 && cp[0].scale0 != nullptr && !(gx[0].l8_out > 0.0) &&
-                        !ordered(0) && (cp[0].M / 64) * (cp[0].M / 64 + 1) / 2 <= kStatTiles &&
+                        !ordered(0) && (cp[0].M / 64) * (cp[0].M / 64 + 1) / 2 <= kStatTiles && cp[0].N <= kStatCols &&
                         (force != 0 ? force : pick_tile(EPI_BMAT, gb, Es, n)) == 64;
     if (with_b) {
       const Plan &pl = cp[0].pl;

@@ -165,4 +165,4 @@ struct NsStatArgs : NsGemmArgs<1> {
   int tiles_only;            // workgroups before the statistics'
   NsStatOne stat;
 };
-constexpr int64_t kStatTiles = 256;       // tiles of a launch that leaves CUs over
+constexpr int64_t kStatTiles = 256, kStatCols = 12288;       // tiles of a launch that leaves CUs over, columns it reads (measured in ns.hip)

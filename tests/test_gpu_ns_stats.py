@@ -79,3 +79,32 @@ def test_statistics_beside_the_second_product(gpu, M, N, sched):
     t128 = run(low[None], "bf16_t128" if sched == "pe" else "bf16_late3_t128")[0]
     assert bits_equal(t128, run(low[None])[0])
     ws.free()
+
+
+@pytest.mark.parametrize("M,N,beside", [(1024, 1024, True), (1408, 8192, True), (1024, 12288, True), (1024, 12416, False),
+                                        (1152, 16384, False), (1536, 1536, False)])
+def test_long_rows_have_the_statistics_in_launches_of_their_own(gpu, M, N, beside):
+    """Beside B the column statistic is read for every matrix: only up to 12288 columns. Either way the flags and bits are those of
+    the same matrix among two, which always have launches of their own."""
+    from ancora_cutile_amd import DevBuf, _lib, newton_schulz_resident_e
+    from ancora_cutile_amd.muon_ns import NsWorkspace, ns_hard_info
+    from oracle.bf16_ref import bf16_rne_bits
+    ws = NsWorkspace()
+
+    def run(X):
+        g = DevBuf(bf16_rne_bits(X).reshape(-1, N))
+        _lib.profile_enable(True)
+        _lib.profile_read()
+        newton_schulz_resident_e(g, None, None, None, None, None, X.shape[0], M, N, 0, schedule=None, workspace=ws)
+        launches = _lib.profile_read()["ns_fro"][1]
+        _lib.profile_enable(False)
+        out, flags = g.to_numpy().reshape(X.shape), ns_hard_info(ws.buf.ptr, X.shape[0], M, N, 5, "bf16_late3")
+        g.free()
+        return out, flags, launches
+    for kind in ("plain", "cols"):
+        X = _input(M, N, kind, M + N)
+        pair, (n2, _), two = run(np.stack([X, X]))
+        one, (n1, _), alone = run(X[None])
+        assert bits_equal(one[0], pair[0]) and 2 * n1 == n2
+        assert alone == two - (1 if beside else 0)       # (the proxy's and the column statistic's launches share a counter's scope)
+    ws.free()
