@@ -904,6 +904,8 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
   for (int q = 0; q < n; ++q) { curH[q] = cp[q].inH; curL[q] = cp[q].inL; nxt[q] = cp[q].nxt; Es[q] = cp[q].E; }
   bool want_cond = false;      // some later iteration gates a product on the proxy
   for (int q = 0; q < n; ++q) want_cond = want_cond || cp[q].pl.sp.any_gate(steps);
+  for (int q = 0; q < n; ++q)  // (the statistics' buffers come with the wide gate)
+    ANC_REQUIRE(!cp[q].pl.sp.any_gate(steps) || cp[q].pl.sp.wide(), "Newton-Schulz chain: a plan with gates has the wide one");
   // the matrices are dealt over the launches' runs (k_ns_classify_order) where a gate picks some of several
   auto ordered = [&](int q) {
     bool gated = false;
@@ -1057,7 +1059,6 @@ int run_bf16_chain(ChainProb *cp, int n, int steps, const float *coef, int flags
       for (int q = 0; q < n; ++q) any_ordered = any_ordered || (cp[q].pl.sp.any_gate(steps) && ordered(q));
       for (int q = 0; q < n; ++q) {
         if (!cp[q].pl.sp.any_gate(steps)) continue;
-        ANC_REQUIRE(cp[q].pl.sp.wide(), "Newton-Schulz chain: a plan with gates has the wide one");
         ca.arrived[ca.n] = any_ordered ? nullptr : cp[q].pl.order;       // (no order: its place counts arrivals)
         ca.Fh[ca.n] = cp[q].pl.Fh; ca.out[ca.n] = cp[q].pl.condpart; ca.M[ca.n] = (int)cp[q].M;
         ca.blocks[ca.n] = (int)(cp[q].E * kCondParts);

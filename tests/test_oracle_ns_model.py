@@ -203,3 +203,13 @@ def test_known_limit_low_rank_bulk_behind_independent_outlier_columns():
     assert 2e-3 < cheap < 3.5e-3
     assert rel(chain(x, PE_SCHEDULE, 5, "bf16", overrides={"wide": True}), ref) < 1e-4
     assert rel(chain(x, PE_SCHEDULE, 5, "bf16_x3"), ref) < 1e-4
+
+
+def test_every_plan_with_gates_has_the_wide_one():
+    """The chain's check before its first launch (the statistics' buffers come with the wide gate) refuses no plan."""
+    for M, N in ((128, 128), (896, 1024), (1024, 1024), (1024, 1920), (1024, 2048), (1408, 12288), (2048, 4096)):
+        for mode in ("bf16", "bf16_fast", "bf16_x3", "bf16_late3"):
+            for steps in range(1, 65):
+                plan = Plan(M, N, mode, steps)
+                gated = any(k < min(plan.x_from, steps) for k in plan.gate_tau)
+                assert plan.wide or not gated, (M, N, mode, steps)
