@@ -108,3 +108,53 @@ def test_long_rows_have_the_statistics_in_launches_of_their_own(gpu, M, N, besid
         assert bits_equal(one[0], pair[0]) and 2 * n1 == n2
         assert alone == two - (1 if beside else 0)       # (the proxy's and the column statistic's launches share a counter's scope)
     ws.free()
+
+
+@pytest.mark.parametrize("sched,groups", [
+    ("keller", [(3, 1024, 1152, ("lowrank", "cols", "plain")), (2, 1024, 2304, ("cols", "lowrank")), (1, 1408, 1408, ("band",)),
+                (2, 256, 512, ("plain", "plain")), (4, 1152, 1280, ("plain", "band", "cols", "plain"))]),
+    ("pe", [(1, 1024, 1024, ("cols",)), (1, 1024, 1152, ("lowrank",)), (1, 1152, 2432, ("plain",)), (1, 1280, 1280, ("band",))]),
+])
+def test_each_batch_of_a_call_decides_by_its_own_statistic(gpu, sched, groups):
+    """Several batches in one call, none of them in another order: every batch has the flags and bits that it has in a call of
+    its own, in each order of the batches and call after call on the same workspaces."""
+    from ancora_cutile_amd import DevBuf, _lib
+    from ancora_cutile_amd._lib import api
+    from ancora_cutile_amd.muon_ns import MODES, PE_SCHEDULE, coef_array, ns_hard_info, ns_workspace_bytes
+    from oracle.bf16_ref import bf16_rne_bits, bits_to_f32
+    schedule, mode = (PE_SCHEDULE, "bf16") if sched == "pe" else (None, "bf16_late3")
+    coef, rng = coef_array(schedule, 5), np.random.default_rng(3)
+    bufs, probs = [], []
+    for E, M, N, kinds in groups:
+        X = np.stack([_input(M, N, k if k == "cols" else "plain", i + N) for i, k in enumerate(kinds)])
+        for e, k in enumerate(kinds):
+            if k == "lowrank":
+                X[e] = _input(M, 8, "plain", 7) @ _input(8, N, "plain", 8) + 0.01 * X[e]
+            elif k == "band":
+                X[e][:, rng.choice(N, N // 10, replace=False)] *= 10
+        hi = bf16_rne_bits(X).reshape(E, M, N)
+        lo = bf16_rne_bits(X - bits_to_f32(hi).reshape(E, M, N)).reshape(E, M, N)
+        nb = ns_workspace_bytes(E, M, N, mode)
+        b = [DevBuf(hi.reshape(-1, N)), DevBuf(lo.reshape(-1, N)), DevBuf((X.astype(np.float64) ** 2).sum(axis=(1, 2))),
+             DevBuf.empty((E * M, N), np.float32), DevBuf.empty((nb // 4 + 64,), np.float32)]
+        ws = (b[4].ptr + 255) // 256 * 256
+        bufs.append(b)
+        probs.append((_lib.NsProblem(b[0].ptr, b[1].ptr, b[2].ptr, b[3].ptr, ws, 1, E, M, N, nb), ws))
+
+    def call(which, wipe=True):
+        for q in which if wipe else ():                 # (nothing is left of an earlier call)
+            for d in bufs[q][3:]:
+                api.anc_fill_u32(d.ptr, 0x7F7F7F7F, d.size, 0)
+        api.anc_ns_batched_pair_multi((_lib.NsProblem * len(which))(*[probs[q][0] for q in which]), len(which), 5, coef, 1e-7, MODES[mode], 0)
+        return [(bufs[q][3].to_numpy(), ns_hard_info(probs[q][1], *groups[q][:3], 5, mode)) for q in which]
+    alone = [call([q])[0] for q in range(len(groups))]
+    for (E, M, N, kinds), (_, (n, _)) in zip(groups, alone):
+        taken = ("lowrank", "band") if sched == "keller" else ("lowrank", "band", "cols")     # (Polar Express: by the proxy's gates too)
+        assert n == sum(k in taken for k in kinds), (M, N)
+    for which in (list(range(len(groups))), list(range(len(groups)))[::-1], [0, 1], [1, 0], [len(groups) - 1, 0, 1]):
+        for wipe in (True, False):
+            for q, (out, info) in zip(which, call(which, wipe)):
+                assert bits_equal(out, alone[q][0]) and info == alone[q][1], (which, q)
+    for b in bufs:
+        for d in b:
+            d.free()
