@@ -252,7 +252,7 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
   // among them: they are kept in registers as they pass, and X is not read again behind the loop (a launch over the
   // projections of six 640-wide layers reads 295 MB instead of 368, 109 -> 106 us, the last one with the weight update 140 -> 134; chains of
   // 24 x (640,1792) 1016 -> 1010, 24 x (512,512) 309 -> 304, 40 x (256,768) 248 -> 240; the full step of a model of 4 layers, hidden size 512,
-  // 525 -> 520). One workgroup per CU (the ring of four) has them earlier by a request before the loop. Eight wavefronts make room by
+  // 526 -> 524, within what its runs differ by). One workgroup per CU (the ring of four) has them earlier by a request before the loop. Eight wavefronts make room by
   // sharing the registers of a step's low fragments (kShare); four have it, and lose by the sharing (4 x (512,1536) 180 -> 184 us per chain).
   constexpr bool kKeep = EPI == EPI_BX && !PLAINV && (NW == 8 || kRing == 3), kShare = EPI == EPI_BX && NW == 8;
   if constexpr (EPI == EPI_BX && !PLAINV && NW == 4) {
@@ -485,7 +485,8 @@ __global__ void __launch_bounds__(64 * NW, tile_per_cu(WM, WN * NW / 4, kRing) *
       };
       const int np = K / 32;
       // The first fragments of step k are in registers when it begins, the others are read under its matrix
-      // instructions (kShare: the low ones of k 0..15 take the place of those of 16..31, which leaves eight wavefronts the registers for kKeep). Before its last product a wavefront waits for its own DMA of step k + 1 and the workgroup meets:
+      // instructions (kShare: the low ones of k 0..15 take the place of those of 16..31, which leaves eight wavefronts the
+      // registers for kKeep). Before its last product a wavefront waits for its own DMA of step k + 1 and the workgroup meets:
       // everybody has read stage k, which takes the DMA of step k + kPairs, and the next step's first fragments are read
       // under that product. B's fragments of k 0..15 and 16..31 change places from step to step.
 #pragma unroll

@@ -4,7 +4,8 @@
 #include "ns_common.h"
 #include "reduce.h"
 
-// 16-byte loads in flight per lane: a part of a 1024x1024 matrix. (One at a time, behind a test for the end: 5.3 -> 4.6 us for one such
+// 16-byte loads in flight per lane: all that a lane has of a 1024x1024 matrix, M^2 / 2^17. Of a larger one that is no multiple of
+// 1024 the loads behind the last whole eight (two of 1152x1152, seven of 1408x1408) come one at a time. (One at a time, behind a test for the end: 5.3 -> 4.6 us for one such
 // matrix, 19.3 -> 17.3 for 48, 5.8 TB/s; with loads that the caches keep instead of streamed ones 34.9.)
 constexpr int kCondAhead = 8;
 // Part b of the matrices' squares of Fh, for thread 0 of 256.

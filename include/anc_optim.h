@@ -16,7 +16,8 @@
  *   - bf16 travels as uint16 bit patterns, exactly as in the reference
  *     (ancora/optim/adamw.py:63-66);
  *   - results are bitwise reproducible run to run and independent of how tensors are
- *     batched into launches: fixed tiles, no split-K, no atomics, fixed reduction order.
+ *     batched into launches: fixed tiles, no split-K, fixed reduction order (atomics
+ *     count arrivals, they add up no values).
  *
  * Each declaration cites the reference interface (path:line under the reference
  * repository root) that it replaces.
